@@ -13,7 +13,7 @@
 // triangles with atomicAdd, which is a race; here a lattice point's vertices
 // (x, y, z edge in that order) and a cube's triangles get their slots from
 // exclusive prefix sums in lattice order, so the mesh is reproducible.  And the
-// 256-case table is derived on the host instead of being typed in: the cut
+// 256-case table is derived by the compiler instead of being typed in: the cut
 // edges on every cube face are joined into directed segments (an ambiguous face
 // always separates its two inside corners), the segments chain into closed
 // loops, every loop is cut into a fan of triangles from its lowest edge.
@@ -37,27 +37,28 @@ struct McTable {
 };
 
 // ---------------------------------------------------------------------------
-// case table (host)
+// case table: evaluated by the compiler, part of the library's device image
 // ---------------------------------------------------------------------------
 namespace {
 
-const int MC_EDGE_CORNERS[12][2] = {{0, 1}, {1, 2}, {2, 3}, {3, 0}, {4, 5}, {5, 6}, {6, 7}, {7, 4}, {0, 4}, {1, 5}, {2, 6}, {3, 7}};
+constexpr int MC_EDGE_CORNERS[12][2] = {{0, 1}, {1, 2}, {2, 3}, {3, 0}, {4, 5}, {5, 6}, {6, 7}, {7, 4}, {0, 4}, {1, 5}, {2, 6}, {3, 7}};
 // the six faces as corner cycles, counter-clockwise seen from outside: x = 0, x = 1, y = 0, y = 1, z = 0, z = 1
-const int MC_FACES[6][4] = {{4, 7, 3, 0}, {1, 2, 6, 5}, {1, 5, 4, 0}, {3, 7, 6, 2}, {3, 2, 1, 0}, {4, 5, 6, 7}};
+constexpr int MC_FACES[6][4] = {{4, 7, 3, 0}, {1, 2, 6, 5}, {1, 5, 4, 0}, {3, 7, 6, 2}, {3, 2, 1, 0}, {4, 5, 6, 7}};
 
-int mc_edge_between(int a, int b) {
+constexpr int mc_edge_between(int a, int b) {
 	for (int e = 0; e < 12; ++e)
 		if ((MC_EDGE_CORNERS[e][0] == a && MC_EDGE_CORNERS[e][1] == b) || (MC_EDGE_CORNERS[e][0] == b && MC_EDGE_CORNERS[e][1] == a)) return e;
 	return -1;
 }
 
-void mc_build_table(McTable& t) {
-	memset(t.tri, -1, sizeof(t.tri));
+constexpr McTable mc_build_table() {
+	McTable t{};
 	for (int mask = 0; mask < 256; ++mask) {
-		int next[12];
+		int next[12] = {};
 		for (int e = 0; e < 12; ++e) next[e] = -1;
+		for (int k = 0; k < 16; ++k) t.tri[mask][k] = -1;
 		for (const auto& cyc : MC_FACES) {
-			int in[4], n_in = 0;
+			int in[4] = {}, n_in = 0;
 			for (int k = 0; k < 4; ++k) { in[k] = (mask >> cyc[k]) & 1; n_in += in[k]; }
 			if (n_in == 0 || n_in == 4) continue;
 			// every maximal run of inside corners is cut off by one segment, directed from the edge after the run to the
@@ -75,7 +76,7 @@ void mc_build_table(McTable& t) {
 		int n = 0;
 		for (int e = 0; e < 12; ++e) {
 			if (next[e] < 0 || seen[e]) continue;
-			int loop[12], len = 0;
+			int loop[12] = {}, len = 0;
 			for (int c = e; !seen[c]; c = next[c]) { seen[c] = true; loop[len++] = c; }
 			for (int k = 1; k + 1 < len; ++k) {
 				t.tri[mask][n++] = (int8_t)loop[0];
@@ -85,336 +86,401 @@ void mc_build_table(McTable& t) {
 		}
 		t.ntri[mask] = (uint8_t)(n / 3);
 	}
-}
-
-const McTable& mc_table() {
-	static McTable t = [] { McTable x; mc_build_table(x); return x; }();
 	return t;
 }
 
+constexpr McTable MC_TABLE_HOST = mc_build_table();
+
 }  // namespace
+
+__device__ const McTable MC_TABLE = mc_build_table();
 
 // ---------------------------------------------------------------------------
 // kernels
+//
+// The density is read once, for one bit per lattice point (inside or not); everything up to the vertex positions is then
+// worked out from the bits, 64 points of a row at a time:
+//   mc_bits     density -> bits                                                   (bound by HBM: 4 bytes per point)
+//   mc_count    one lane per word: its edge vertices and triangles as bit masks, prefix sums within a block of 256 words
+//   mc_scan     one workgroup: prefix sums over the blocks, the totals the host asks for
+//   mc_emit     one wave per word that owns something: vertices and triangles
+//   mc_normals  one lane per vertex: the sum over the triangles of the four cubes round its edge
+// Rows are padded to whole words, so a word's neighbours in y and z are words too and no mask crosses a row.
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 90 (6.0 TB/s), count 29, scan 9, emit 46, normals 34, with
+// the host's wait for the totals 238 in all.  Deciding every point from the four rows of the density itself took 242 for the
+// count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
 struct McGrid {
 	uint32_t rx, ry, rz;
 	float thresh;
 	float scale[3], offset[3];
+	uint32_t row_words;  // words per row
+	uint32_t n_words;
 };
 
-// A wave looks at 64 consecutive lattice points (a chunk) at a time.  Whether a point is inside is one bit of a ballot, so
-// a chunk costs four coalesced loads (the rows at y, y + 1, z + 1 and both) plus the four values right behind them, however
-// many of the eight cube corners and three edges a point shares with its neighbours; a chunk whose four rows lie entirely
-// on one side of the surface (almost all of them) is decided from the ballots alone.
-constexpr uint32_t MC_CHUNKS = 4;                  // chunks per tile
-constexpr uint32_t MC_WAVE_TILE = 64 * MC_CHUNKS;  // lattice points per tile: the unit the prefix sums are kept for (small, so that
-                                                   // the few tiles the surface crosses spread over many waves when they are emitted)
-constexpr uint32_t MC_COUNT_TILES = 4;             // consecutive tiles per wave of the count kernel
+typedef unsigned long long mc_word;
 
-struct McPoint {
-	uint32_t flags;  // bit a: the edge towards +axis a carries a vertex
-	uint32_t mask;   // corner bits of the point's cube, 0 when it has none
+// What a word of points owns; written for the words that own something, which the `active` bits tell.
+struct alignas(64) McRecord {
+	mc_word edge[3];       // point has a vertex on its edge towards +axis
+	mc_word tri[3];        // bits 0, 1, 2 of the number of triangles of the point's cube
+	uint32_t first_v, first_t;  // vertices and triangles of the words before this one in its block of 256
+	uint32_t pad[2];
 };
 
-// The ballots of MC_GROUP consecutive chunks are formed together, so that a wave has 4 x MC_GROUP loads in flight instead
-// of one round trip per chunk; only the last chunk of a group needs the values right behind its rows, the others take them
-// from the next chunk's ballots.
-constexpr uint32_t MC_GROUP = 4;
-static_assert(MC_CHUNKS % MC_GROUP == 0, "a wave's chunks come in whole groups");
+constexpr uint32_t MC_BITS_WORDS = 16;  // words a wave forms at a time: 16 loads in flight per lane
 
-struct McBallots {
-	unsigned long long m[MC_GROUP][4];  // [chunk][row]: inside bits of 64 consecutive points of the rows at +0, +rx, +rx ry, +rx ry + rx
-	bool next[4];                       // the point right behind the last chunk's rows
-};
-
-__device__ __forceinline__ void mc_load_group(const McGrid& g, const float* __restrict__ density, uint64_t n, uint32_t first, uint32_t lane, McBallots& B) {
-	const uint32_t r1 = g.rx, r2 = g.rx * g.ry;
-	const uint32_t off[4] = {0u, r1, r2, r2 + r1};
-	float v[MC_GROUP][4], e[4];
+__global__ void __launch_bounds__(MC_BLOCK) mc_bits_kernel(McGrid g, const float* __restrict__ density, mc_word* __restrict__ bits) {
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (MC_BLOCK / 64) + (threadIdx.x >> 6));
+	const uint32_t w0 = wave * MC_BITS_WORDS;
+	if (w0 >= g.n_words) return;
+	uint32_t row = w0 / g.row_words, col = w0 - row * g.row_words;
+	float v[MC_BITS_WORDS];
 #pragma unroll
-	for (uint32_t c = 0; c < MC_GROUP; ++c)
+	for (uint32_t k = 0; k < MC_BITS_WORDS; ++k) {
+		const uint32_t x = col * 64u + lane;
+		v[k] = (w0 + k < g.n_words && x < g.rx) ? density[(uint64_t)row * g.rx + x] : -INFINITY;
+		if (++col == g.row_words) { col = 0; ++row; }
+	}
+	mc_word mine = 0;
 #pragma unroll
-		for (int j = 0; j < 4; ++j) {
-			const uint64_t q = (uint64_t)first + c * 64u + off[j] + lane;
-			v[c][j] = q < n ? density[q] : -INFINITY;
+	for (uint32_t k = 0; k < MC_BITS_WORDS; ++k) {
+		const mc_word b = __ballot(v[k] > g.thresh);
+		if (lane == k) mine = b;
+	}
+	if (lane < MC_BITS_WORDS && w0 + lane < g.n_words) bits[w0 + lane] = mine;
+}
+
+// The bits of a word and of its neighbours, in the order of the offsets (y, z) = (0, 0), (1, 0), (0, 1), (1, 1): b the word
+// itself, s the word one point further along x.  ok[0]: points of the word that have a neighbour in x; ok[1], ok[2]: the rows
+// at y + 1, z + 1 exist (their words are zero if not).
+struct McBits {
+	mc_word b[4], s[4], here, xok;
+	bool yok, zok;
+};
+// WAVE: the lanes of the wave hold consecutive words, and take the word behind theirs from the next lane
+template <bool WAVE>
+__device__ __forceinline__ McBits mc_load_bits(const McGrid& g, const mc_word* __restrict__ bits, uint32_t w) {
+	McBits B;
+	const uint32_t row = w / g.row_words, col = w - row * g.row_words;
+	const uint32_t z = row / g.ry, y = row - z * g.ry;
+	B.yok = y + 1u < g.ry;
+	B.zok = z + 1u < g.rz;
+	const uint32_t left = g.rx - col * 64u;  // points from the word's first to the end of the row
+	B.here = left >= 64u ? ~0ull : (1ull << left) - 1ull;
+	B.xok = left > 64u ? ~0ull : (1ull << (left - 1u)) - 1ull;
+#pragma unroll
+	for (uint32_t j = 0; j < 4; ++j) {
+		const bool ok = (!(j & 1u) || B.yok) && (!(j & 2u) || B.zok);
+		const uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u);
+		B.b[j] = ok ? bits[at] : 0ull;
+		mc_word next = 0ull;
+		if (WAVE) next = __shfl_down(B.b[j], 1);
+		if (!WAVE || (threadIdx.x & 63u) == 63u) next = ok && left > 64u ? bits[at + 1u] : 0ull;
+		if (left <= 64u) next = 0ull;
+		B.s[j] = (B.b[j] >> 1) | (next << 63);
+	}
+	return B;
+}
+// corner k of the cubes, as in gen_faces: round the bottom face from the point itself, then the top face
+__device__ __forceinline__ mc_word mc_corner(const McBits& B, uint32_t k) {
+	const mc_word corner[8] = {B.b[0], B.s[0], B.s[1], B.b[1], B.b[2], B.s[2], B.s[3], B.b[3]};
+	return corner[k];
+}
+// corner bits of point `lane`'s cube
+__device__ __forceinline__ uint32_t mc_case(const McBits& B, uint32_t lane) {
+	uint32_t m = 0;
+#pragma unroll
+	for (uint32_t k = 0; k < 8; ++k) m |= (uint32_t)((mc_corner(B, k) >> lane) & 1ull) << k;
+	return m;
+}
+
+// inclusive sum over the lanes of a wave
+__device__ __forceinline__ uint32_t mc_wave_scan(uint32_t v, uint32_t lane) {
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1) {
+		const uint32_t u = __shfl_up(v, o);
+		if ((int)lane >= o) v += u;
+	}
+	return v;
+}
+
+// One lane per word; a lane walks through the cubes of its word that the surface cuts.  (Listing those cubes in LDS and dealing
+// them to the lanes, as the emitting kernel does, takes the same time: the launch is four rounds of load latency.)
+__global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
+                                                            mc_word* __restrict__ active, uint2* __restrict__ blocks) {
+	__shared__ uint8_t ntri[256];
+	__shared__ uint32_t sum_v[MC_BLOCK / 64], sum_t[MC_BLOCK / 64];
+	const uint32_t w = blockIdx.x * MC_BLOCK + threadIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	ntri[threadIdx.x] = MC_TABLE.ntri[threadIdx.x];
+	__syncthreads();
+	McRecord r{};
+	uint32_t nv = 0, nt = 0;
+	mc_word cut = 0;
+	const McBits B = mc_load_bits<true>(g, bits, min(w, g.n_words - 1u));  // every lane takes part in the exchange
+	if (w < g.n_words) {
+		r.edge[0] = (B.b[0] ^ B.s[0]) & B.xok;
+		r.edge[1] = B.yok ? (B.b[0] ^ B.b[1]) & B.here : 0ull;
+		r.edge[2] = B.zok ? (B.b[0] ^ B.b[2]) & B.here : 0ull;
+#pragma unroll
+		for (int a = 0; a < 3; ++a) nv += (uint32_t)__popcll(r.edge[a]);
+		if (B.yok && B.zok) {
+			const mc_word any = B.b[0] | B.b[1] | B.b[2] | B.b[3] | B.s[0] | B.s[1] | B.s[2] | B.s[3];
+			const mc_word all = B.b[0] & B.b[1] & B.b[2] & B.b[3] & B.s[0] & B.s[1] & B.s[2] & B.s[3];
+			cut = any & ~all & B.xok;
+		}
+		for (; cut; cut &= cut - 1ull) {
+			const uint32_t p = (uint32_t)__ffsll(cut) - 1u;
+			const uint32_t t = ntri[mc_case(B, p)];
+			nt += t;
+#pragma unroll
+			for (int a = 0; a < 3; ++a) r.tri[a] |= (mc_word)((t >> a) & 1u) << p;
+		}
+	}
+	const bool owns = nv + nt > 0;
+	const mc_word mask = __ballot(owns);
+	if (lane == 0) active[w >> 6] = mask;
+	if (!__syncthreads_or(owns)) {
+		if (threadIdx.x == 0) blocks[blockIdx.x] = make_uint2(0, 0);
+		return;
+	}
+	const uint32_t iv = mc_wave_scan(nv, lane), it = mc_wave_scan(nt, lane);
+	if (lane == 63) { sum_v[wave] = iv; sum_t[wave] = it; }
+	__syncthreads();
+	uint32_t before_v = 0, before_t = 0, all_v = 0, all_t = 0;
+#pragma unroll
+	for (uint32_t k = 0; k < MC_BLOCK / 64; ++k) {
+		if (k < wave) { before_v += sum_v[k]; before_t += sum_t[k]; }
+		all_v += sum_v[k];
+		all_t += sum_t[k];
+	}
+	if (owns) {
+		r.first_v = before_v + iv - nv;
+		r.first_t = before_t + it - nt;
+		records[w] = r;
+	}
+	if (threadIdx.x == 0) blocks[blockIdx.x] = make_uint2(all_v, all_t);
+}
+
+// Exclusive prefix sums of the blocks' counts in place; element n_blocks receives the totals.
+constexpr uint32_t MC_SCAN_EACH = 8;
+__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks) {
+	__shared__ uint2 wave_sum[16];
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	uint2 carry = make_uint2(0, 0);
+	for (uint32_t c0 = 0; c0 < n_blocks; c0 += 1024u * MC_SCAN_EACH) {
+		const uint32_t i0 = c0 + threadIdx.x * MC_SCAN_EACH;
+		uint2 v[MC_SCAN_EACH], own = make_uint2(0, 0);
+#pragma unroll
+		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) v[k] = i0 + k < n_blocks ? blocks[i0 + k] : make_uint2(0, 0);
+#pragma unroll
+		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) { own.x += v[k].x; own.y += v[k].y; }
+		const uint32_t ix = mc_wave_scan(own.x, lane), iy = mc_wave_scan(own.y, lane);
+		if (lane == 63) wave_sum[wave] = make_uint2(ix, iy);
+		__syncthreads();
+		uint2 run = make_uint2(carry.x + ix - own.x, carry.y + iy - own.y);
+#pragma unroll
+		for (uint32_t k = 0; k < 16; ++k) {
+			const uint2 s = wave_sum[k];
+			if (k < wave) { run.x += s.x; run.y += s.y; }
+			carry.x += s.x;
+			carry.y += s.y;
 		}
 #pragma unroll
-	for (int j = 0; j < 4; ++j) {
-		const uint64_t q = (uint64_t)first + MC_GROUP * 64u + off[j];  // the same address in every lane
-		e[j] = q < n ? density[q] : -INFINITY;
+		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) {
+			if (i0 + k < n_blocks) blocks[i0 + k] = run;
+			run.x += v[k].x;
+			run.y += v[k].y;
+		}
+		__syncthreads();  // the sums have been read
 	}
-#pragma unroll
-	for (uint32_t c = 0; c < MC_GROUP; ++c)
-#pragma unroll
-		for (int j = 0; j < 4; ++j) B.m[c][j] = __ballot(v[c][j] > g.thresh);
-#pragma unroll
-	for (int j = 0; j < 4; ++j) B.next[j] = e[j] > g.thresh;
-}
-
-// (x, y, z) of lattice point first + lane
-__device__ __forceinline__ void mc_point_xyz(const McGrid& g, uint32_t first, uint32_t lane, uint32_t* c) {
-	if (g.rx >= 64u) {  // at most one row ends inside the chunk
-		uint32_t x = first % g.rx + lane;
-		const uint32_t row = first / g.rx + (x >= g.rx ? 1u : 0u);
-		x -= x >= g.rx ? g.rx : 0u;
-		c[0] = x; c[1] = row % g.ry; c[2] = row / g.ry;
-	} else {
-		const uint32_t idx = first + lane;
-		c[0] = idx % g.rx; c[1] = (idx / g.rx) % g.ry; c[2] = idx / (g.rx * g.ry);
-	}
-}
-
-// Chunk c of a group.  False: no point of the chunk has an edge vertex or a triangle (p is then not filled in).
-__device__ __forceinline__ bool mc_chunk(const McGrid& g, uint64_t n, const McBallots& B, uint32_t c, uint32_t first, uint32_t lane, McPoint& p) {
-	unsigned long long m[4];
-	bool next[4];
-	bool all0 = true, all1 = true;
-#pragma unroll
-	for (int j = 0; j < 4; ++j) {
-		m[j] = B.m[c][j];
-		next[j] = c + 1 < MC_GROUP ? (B.m[c + 1 < MC_GROUP ? c + 1 : c][j] & 1ull) != 0ull : B.next[j];
-		all0 = all0 && m[j] == 0ull && !next[j];
-		all1 = all1 && m[j] == ~0ull && next[j];
-	}
-	if (all0 || all1) return false;
-	uint32_t xyz[3];
-	mc_point_xyz(g, first, lane, xyz);
-	const bool here = (uint64_t)first + lane < n;
-	const bool xok = xyz[0] + 1 < g.rx, yok = xyz[1] + 1 < g.ry, zok = xyz[2] + 1 < g.rz;
-	bool in[4], in1[4];
-#pragma unroll
-	for (int j = 0; j < 4; ++j) {
-		in[j] = (m[j] >> lane) & 1ull;
-		in1[j] = lane < 63u ? ((m[j] >> (lane + 1u)) & 1ull) != 0ull : next[j];
-	}
-	p.flags = 0;
-	p.mask = 0;
-	if (here) {
-		if (xok && in[0] != in1[0]) p.flags |= 1u;
-		if (yok && in[0] != in[1]) p.flags |= 2u;
-		if (zok && in[0] != in[2]) p.flags |= 4u;
-		if (xok && yok && zok)  // corner bits as in gen_faces: round the bottom face from the point itself, then the top face
-			p.mask = (in[0] ? 1u : 0u) | (in1[0] ? 2u : 0u) | (in1[1] ? 4u : 0u) | (in[1] ? 8u : 0u) | (in[2] ? 16u : 0u) | (in1[2] ? 32u : 0u) |
-			         (in1[3] ? 64u : 0u) | (in[3] ? 128u : 0u);
-	}
-	return true;
+	if (threadIdx.x == 0) blocks[n_blocks] = carry;
 }
 
 // number of set bits of `b` below this lane
-__device__ __forceinline__ uint32_t mc_below(unsigned long long b, uint32_t lane) { return (uint32_t)__popcll(b & ((1ull << lane) - 1ull)); }
+__device__ __forceinline__ uint32_t mc_below(mc_word b, uint32_t lane) { return (uint32_t)__popcll(b & ((1ull << lane) - 1ull)); }
 
-// Per tile (256 consecutive lattice points): how many edge vertices and triangles its points own.
-__global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const McTable* __restrict__ table, const float* __restrict__ density,
-                                                            uint32_t n_tiles, uint32_t* __restrict__ vsum, uint32_t* __restrict__ tsum,
-                                                            uint8_t* __restrict__ busy) {
-	const uint64_t n = (uint64_t)g.rx * g.ry * g.rz;
-	const uint32_t lane = threadIdx.x & 63u;
-	for (uint32_t tile = (blockIdx.x * (MC_BLOCK / 64) + (threadIdx.x >> 6)) * MC_COUNT_TILES, last = tile + MC_COUNT_TILES; tile < last && tile < n_tiles; ++tile) {
-	uint32_t nv = 0, nt = 0, groups = 0;  // bit k of groups: group k of the tile has a chunk that is not all on one side
-	for (uint32_t c0 = 0; c0 < MC_CHUNKS; c0 += MC_GROUP) {
-		const uint32_t first0 = tile * MC_WAVE_TILE + c0 * 64u;
-		if ((uint64_t)first0 >= n) break;
-		McBallots B;
-		mc_load_group(g, density, n, first0, lane, B);
+// edge masks of a word and its first vertex
+struct McOwned {
+	mc_word e[3];
+	uint32_t first;
+};
+__device__ __forceinline__ McOwned mc_owned(const McRecord* __restrict__ records, const uint2* __restrict__ blocks, uint32_t w) {
+	const McRecord& r = records[w];
+	return McOwned{{r.edge[0], r.edge[1], r.edge[2]}, blocks[w / MC_BLOCK].x + r.first_v};
+}
+// first vertex of the word's point `lane` | its edge flags << 29
+__device__ __forceinline__ uint32_t mc_vertex_slot(const McOwned& o, uint32_t lane) {
+	uint32_t slot = o.first, flags = 0;
 #pragma unroll
-		for (uint32_t c = 0; c < MC_GROUP; ++c) {
-			McPoint p;
-			if (!mc_chunk(g, n, B, c, first0 + c * 64u, lane, p)) continue;
-			groups |= 1u << (c0 / MC_GROUP);
-			nv += (uint32_t)__popc(p.flags);
-			nt += table->ntri[p.mask];
-		}
+	for (uint32_t a = 0; a < 3; ++a) {
+		slot += mc_below(o.e[a], lane);
+		flags |= (uint32_t)((o.e[a] >> lane) & 1ull) << a;
 	}
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) { nv += __shfl_xor(nv, o); nt += __shfl_xor(nt, o); }
-	if (lane == 0) { vsum[tile] = nv; tsum[tile] = nt; busy[tile] = (uint8_t)groups; }
-	}
+	return slot | (flags << 29);
 }
 
-// Exclusive prefix sums of the two per-tile arrays in place, by blocks of 1024 tiles (blockIdx.y 0: vertices, 1: triangles):
-// first the blocks' totals, then every block adds up the totals before it and scans its own elements; element n_tiles
-// receives the grand total.
-__global__ void __launch_bounds__(1024) mc_block_totals_kernel(uint32_t n_tiles, const uint32_t* __restrict__ vsum, const uint32_t* __restrict__ tsum,
-                                                               uint32_t* __restrict__ vblock, uint32_t* __restrict__ tblock) {
-	__shared__ uint32_t wave_sum[16];
-	const uint32_t* data = blockIdx.y == 0 ? vsum : tsum;
-	const uint32_t i = blockIdx.x * 1024u + threadIdx.x;
-	uint32_t v = i < n_tiles ? data[i] : 0u;
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-	if ((threadIdx.x & 63u) == 0) wave_sum[threadIdx.x >> 6] = v;
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		uint32_t all = 0;
-#pragma unroll
-		for (int w = 0; w < 16; ++w) all += wave_sum[w];
-		(blockIdx.y == 0 ? vblock : tblock)[blockIdx.x] = all;
-	}
-}
-__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_tiles, uint32_t* __restrict__ vsum, uint32_t* __restrict__ tsum,
-                                                       const uint32_t* __restrict__ vblock, const uint32_t* __restrict__ tblock) {
-	__shared__ uint32_t wave_before[16], wave_sum[16];
-	uint32_t* data = blockIdx.y == 0 ? vsum : tsum;
-	const uint32_t* block = blockIdx.y == 0 ? vblock : tblock;
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	const uint32_t i = blockIdx.x * 1024u + threadIdx.x;
-	const uint32_t v = i < n_tiles ? data[i] : 0u;
-	uint32_t before = 0;
-	for (uint32_t q = threadIdx.x; q < blockIdx.x; q += 1024u) before += block[q];
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
-	uint32_t incl = v;
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t u = __shfl_up(incl, o);
-		if ((int)lane >= o) incl += u;
-	}
-	if (lane == 63) { wave_before[wave] = before; wave_sum[wave] = incl; }
-	__syncthreads();
-	uint32_t run = incl - v, all = 0;
-#pragma unroll
-	for (uint32_t w = 0; w < 16; ++w) { run += wave_before[w] + (w < wave ? wave_sum[w] : 0u); all += wave_before[w] + wave_sum[w]; }
-	if (i < n_tiles) data[i] = run;
-	if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) data[n_tiles] = all;
-}
+constexpr uint32_t MC_LIST = 2048;
 
-// The emitting kernels run a fixed number of waves that stride over the tiles.  Most tiles own nothing: a wave looks at 64
-// of its tiles at once (one per lane) and then visits those that own something.
-constexpr uint32_t MC_EMIT_BLOCKS = 2048;
-
-// Calls visit(tile, first slot, busy groups) for every tile of this wave whose prefix sum moves.
+// Lists the set bits of every lane's `points` in lane order, as (lane of the workgroup) << 6 | bit, and calls visit(entry)
+// with one entry per lane at a time; all lanes of the workgroup take part.
 template <class Visit>
-__device__ __forceinline__ void mc_for_owning_tiles(uint32_t n_tiles, const uint32_t* __restrict__ sums, const uint8_t* __restrict__ busy, Visit visit) {
-	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t wave = blockIdx.x * (MC_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (MC_BLOCK / 64);
-	// Slot k of the walk deals the tiles k n_waves .. (k + 1) n_waves - 1 to the waves, rotated by 37 k: with a plain stride the
-	// tiles of a wave would sit at one place of the planes they fall into (n_waves is a multiple of a plane's tiles for the
-	// usual resolutions), and the waves that look at the middle of the object would own all the work.
-	for (uint32_t k0 = 0; (uint64_t)k0 * n_waves < n_tiles; k0 += 64u) {
-		const uint32_t k = k0 + lane;
-		const uint64_t mine64 = (uint64_t)k * n_waves + (wave + k * 37u) % n_waves;
-		const uint32_t mine = mine64 < n_tiles ? (uint32_t)mine64 : n_tiles;
-		uint32_t begin = 0, end = 0, groups = 0;
-		if (mine < n_tiles) { begin = sums[mine]; end = sums[mine + 1]; groups = busy[mine]; }
-		unsigned long long owning = __ballot(end != begin);
-		while (owning) {
-			const int l = __ffsll((long long)owning) - 1;
-			owning &= owning - 1ull;
-			visit((uint32_t)__shfl((int)mine, l), (uint32_t)__shfl((int)begin, l), (uint32_t)__shfl((int)groups, l));
-		}
+__device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, uint32_t* wave_sum, Visit visit) {
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	const uint32_t n = (uint32_t)__popcll(points), incl = mc_wave_scan(n, lane);
+	if (lane == 63) wave_sum[wave] = incl;
+	__syncthreads();
+	uint32_t first = incl - n, total = 0;
+#pragma unroll
+	for (uint32_t k = 0; k < MC_BLOCK / 64; ++k) {
+		if (k < wave) first += wave_sum[k];
+		total += wave_sum[k];
+	}
+	for (uint32_t from = 0; from < total; from += MC_LIST) {
+		for (; points && first < from + MC_LIST; points &= points - 1ull, ++first) list[first - from] = (uint16_t)(threadIdx.x << 6 | ((uint32_t)__ffsll(points) - 1u));
+		__syncthreads();
+		const uint32_t count = min(total - from, MC_LIST);
+		for (uint32_t i = threadIdx.x; i < count; i += MC_BLOCK) visit((uint32_t)list[i]);
+		__syncthreads();  // the list has been read
 	}
 }
 
-// Vertices of the tiles that have any, numbered in lattice order (x, y, z edge of a point in that order); voff[point] =
-// first slot | edge flags << 29 is written for the points that own a vertex: the only ones the faces look up.
-__global__ void __launch_bounds__(MC_BLOCK) mc_vertices_kernel(McGrid g, const float* __restrict__ density, uint32_t n_tiles,
-                                                               const uint32_t* __restrict__ vsum, const uint8_t* __restrict__ busy,
-                                                               uint32_t* __restrict__ voff, float* __restrict__ verts) {
-	const uint64_t n = (uint64_t)g.rx * g.ry * g.rz;
-	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t step[3] = {1u, g.rx, g.rx * g.ry};
-	mc_for_owning_tiles(n_tiles, vsum, busy, [&](uint32_t tile, uint32_t run, uint32_t groups) {
-		for (uint32_t c0 = 0; c0 < MC_CHUNKS; c0 += MC_GROUP) {
-			const uint32_t first0 = tile * MC_WAVE_TILE + c0 * 64u;
-			if (!((groups >> (c0 / MC_GROUP)) & 1u)) continue;
-			McBallots B;
-			mc_load_group(g, density, n, first0, lane, B);
+// Workgroup b emits what the words of block b own.  Only one point in ten of such a word owns anything, so the points that do
+// are listed and dealt to the lanes: with a wave per word the launch was a chain of memory round trips at a tenth of the
+// lanes, 240 us.  The vertices that a cube uses belong to its own point and to those one further along x, y and z: their
+// slots come from the records of the (at most eight) words those points are in, and stand in LDS, where a triangle's
+// corners pick theirs.
+// Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
+__global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float* __restrict__ density, const mc_word* __restrict__ bits,
+                                                           const McRecord* __restrict__ records, const mc_word* __restrict__ active,
+                                                           const uint2* __restrict__ blocks, float* __restrict__ verts, uint32_t* __restrict__ indices,
+                                                           uint32_t* __restrict__ origin) {
+	__shared__ uint16_t list[MC_LIST];
+	__shared__ uint32_t slot_of[8][MC_BLOCK];
+	__shared__ uint32_t wave_sum[MC_BLOCK / 64];
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	const uint32_t mine = blockIdx.x * MC_BLOCK + threadIdx.x;
+	const bool owns = (active[blockIdx.x * (MC_BLOCK / 64) + wave] >> lane) & 1ull;
+	if (!__syncthreads_or(owns)) return;
+	mc_word points = 0;
+	if (owns) {
+		const McRecord& r = records[mine];
+		points = r.edge[0] | r.edge[1] | r.edge[2] | r.tri[0] | r.tri[1] | r.tri[2];
+	}
+	mc_for_points(points, list, wave_sum, [&](uint32_t entry) {
+		const uint32_t w = blockIdx.x * MC_BLOCK + (entry >> 6), p = entry & 63u;
+		const McRecord& r = records[w];
+		const McOwned own = mc_owned(records, blocks, w);
+		const mc_word t0 = r.tri[0], t1 = r.tri[1], t2 = r.tri[2];
+		const uint32_t row = w / g.row_words, col = w - row * g.row_words;
+		const uint32_t xyz[3] = {col * 64u + p, row % g.ry, row / g.ry};
+		const uint32_t slot0 = mc_vertex_slot(own, p), flags = slot0 >> 29;
+		if (flags) {
+			const uint64_t idx = (uint64_t)row * g.rx + xyz[0];
+			const uint64_t step[3] = {1u, g.rx, (uint64_t)g.rx * g.ry};
+			const float pos[3] = {(float)xyz[0], (float)xyz[1], (float)xyz[2]};
+			const float f0 = density[idx];
+			float f1[3];
 #pragma unroll
-			for (uint32_t c = 0; c < MC_GROUP; ++c) {
-				const uint32_t first = first0 + c * 64u;
-				McPoint p;
-				if (!mc_chunk(g, n, B, c, first, lane, p)) continue;
-				const unsigned long long b0 = __ballot(p.flags & 1u), b1 = __ballot(p.flags & 2u), b2 = __ballot(p.flags & 4u);
-				uint32_t slot = run + mc_below(b0, lane) + mc_below(b1, lane) + mc_below(b2, lane);
-				run += (uint32_t)(__popcll(b0) + __popcll(b1) + __popcll(b2));
-				if (!p.flags) continue;
-				const uint32_t idx = first + lane;
-				voff[idx] = slot | (p.flags << 29);
-				uint32_t xyz[3];
-				mc_point_xyz(g, first, lane, xyz);
-				const float pos[3] = {(float)xyz[0], (float)xyz[1], (float)xyz[2]};
-				const float f0 = density[idx];
+			for (uint32_t a = 0; a < 3; ++a) f1[a] = ((flags >> a) & 1u) ? density[idx + step[a]] : 0.f;
+			uint32_t slot = slot0 & 0x1FFFFFFFu;
 #pragma unroll
-				for (uint32_t a = 0; a < 3; ++a) {
-					if (!((p.flags >> a) & 1u)) continue;
-					const float f1 = density[idx + step[a]];
-					const float dt = (g.thresh - f0) / (f1 - f0);
-					float* v = verts + (size_t)slot * 3;
+			for (uint32_t a = 0; a < 3; ++a) {
+				if (!((flags >> a) & 1u)) continue;
+				const float dt = (g.thresh - f0) / (f1[a] - f0);
+				float* v = verts + (size_t)slot * 3;
 #pragma unroll
-					for (uint32_t d = 0; d < 3; ++d) v[d] = (d == a ? pos[d] + dt : pos[d]) * g.scale[d] + g.offset[d];
-					++slot;
-				}
+				for (uint32_t d = 0; d < 3; ++d) v[d] = (d == a ? pos[d] + dt : pos[d]) * g.scale[d] + g.offset[d];
+				if (origin) { origin[(size_t)slot * 3] = w; origin[(size_t)slot * 3 + 1] = p | a << 6; }
+				++slot;
+			}
+		}
+		const uint32_t tris = (uint32_t)((t0 >> p) & 1ull) | (uint32_t)((t1 >> p) & 1ull) << 1 | (uint32_t)((t2 >> p) & 1ull) << 2;
+		if (tris == 0) return;  // (the cubes of the last column, row and plane have no triangles: the points below exist)
+#pragma unroll
+		for (uint32_t j = 0; j < 4; ++j) {
+			const uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u);
+			const McOwned o = j == 0 ? own : mc_owned(records, blocks, at);
+			slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, p);
+			slot_of[2 * j + 1][threadIdx.x] = p < 63u ? mc_vertex_slot(o, p + 1u) : mc_vertex_slot(mc_owned(records, blocks, at + 1u), 0u);
+		}
+		const uint32_t first_t = blocks[w / MC_BLOCK].y + r.first_t + mc_below(t0, p) + 2u * mc_below(t1, p) + 4u * mc_below(t2, p);
+		const uint32_t mask = mc_case(mc_load_bits<false>(g, bits, w), p);
+		// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
+		// the owner's offset from this point in x, y, z and the edge's axis.
+		constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
+		                           16ull << 40 | 17ull << 45 | 19ull << 50 | 18ull << 55;
+		const uint4 row4 = *reinterpret_cast<const uint4*>(MC_TABLE.tri[mask]);
+		const uint32_t trow[4] = {row4.x, row4.y, row4.z, row4.w};
+		uint32_t* out = indices + (size_t)first_t * 3;
+#pragma unroll
+		for (uint32_t k = 0; k < 15; ++k) {
+			if (k < 3u * tris) {
+				const uint32_t e = (trow[k >> 2] >> (8u * (k & 3u))) & 0xFu;
+				const uint32_t code = (uint32_t)(OWNER >> (5u * e)) & 31u;
+				const uint32_t at = slot_of[code & 7u][threadIdx.x];
+				// the owner's first slot plus the number of its edges before this one
+				out[k] = (at & 0x1FFFFFFFu) + (uint32_t)__popc((at >> 29) & ((1u << (code >> 3)) - 1u));
 			}
 		}
 	});
 }
 
-// Triangles of the tiles that have any, numbered in lattice order of their cubes.
-__global__ void __launch_bounds__(MC_BLOCK) mc_faces_kernel(McGrid g, const McTable* __restrict__ table, const float* __restrict__ density,
-                                                            uint32_t n_tiles, const uint32_t* __restrict__ tsum, const uint8_t* __restrict__ busy,
-                                                            const uint32_t* __restrict__ voff, uint32_t* __restrict__ indices) {
-	const uint64_t n = (uint64_t)g.rx * g.ry * g.rz;
-	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t r1 = g.rx, r2 = g.rx * g.ry;
-	mc_for_owning_tiles(n_tiles, tsum, busy, [&](uint32_t tile, uint32_t run, uint32_t groups) {
-		for (uint32_t c0 = 0; c0 < MC_CHUNKS; c0 += MC_GROUP) {
-			const uint32_t first0 = tile * MC_WAVE_TILE + c0 * 64u;
-			if (!((groups >> (c0 / MC_GROUP)) & 1u)) continue;
-			McBallots B;
-			mc_load_group(g, density, n, first0, lane, B);
-#pragma unroll
-			for (uint32_t c = 0; c < MC_GROUP; ++c) {
-				const uint32_t first = first0 + c * 64u;
-				McPoint p;
-				if (!mc_chunk(g, n, B, c, first, lane, p)) continue;
-				const uint32_t tris = table->ntri[p.mask];  // 0 .. 5: three bit planes
-				const unsigned long long b0 = __ballot(tris & 1u), b1 = __ballot(tris & 2u), b2 = __ballot(tris & 4u);
-				const uint32_t mine = run + mc_below(b0, lane) + 2u * mc_below(b1, lane) + 4u * mc_below(b2, lane);
-				run += (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2));
-				if (!tris) continue;
-				const uint32_t idx = first + lane;
-				// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
-				// the owner's offset from this point in x, y, z and the edge's axis.  The case's row is one 16-byte load and
-				// all look-ups of a cube are in flight together.
-				constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
-				                           16ull << 40 | 17ull << 45 | 19ull << 50 | 18ull << 55;
-				const uint4 row4 = *reinterpret_cast<const uint4*>(table->tri[p.mask]);
-				const uint32_t row[4] = {row4.x, row4.y, row4.z, row4.w};
-				uint32_t w[15], axis[15];
-#pragma unroll
-				for (uint32_t k = 0; k < 15; ++k) {
-					const uint32_t e = (row[k >> 2] >> (8u * (k & 3u))) & 0xFu;  // rows end with -1: the low four bits of an unused entry name no edge that is read
-					const uint32_t code = (uint32_t)(OWNER >> (5u * (e < 12u ? e : 0u))) & 31u;
-					axis[k] = code >> 3;
-					w[k] = k < 3u * tris ? voff[idx + (code & 1u) + ((code >> 1) & 1u) * r1 + ((code >> 2) & 1u) * r2] : 0u;
-				}
-				uint32_t* out = indices + (size_t)mine * 3;
-#pragma unroll
-				for (uint32_t k = 0; k < 15; ++k)
-					if (k < 3u * tris)  // the owner's first slot plus the number of its edges before this one
-						out[k] = (w[k] & 0x1FFFFFFFu) + (uint32_t)__popc((w[k] >> 29) & ((1u << axis[k]) - 1u));
-			}
-		}
-	});
-}
-
-// accumulate_1ring's normals: per triangle (pb - pa) x (pa - pc), added to its three vertices
-__global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(uint32_t n_tris, const uint32_t* __restrict__ indices, const float* __restrict__ verts,
+// accumulate_1ring's normals: a vertex's is the sum of (pb - pa) x (pa - pc) over the triangles it is a corner of.  They lie in
+// the four cubes round the vertex's edge; the cubes are visited in lattice order and their triangles in theirs, so the sum
+// does not depend on how the work is scheduled.  (Adding every triangle to its corners with float atomics took 276 us for
+// the 512^3 sphere's 1.2 M triangles: 11 M atomics at the part's 40 G/s.)
+__global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const McRecord* __restrict__ records,
+                                                              const mc_word* __restrict__ active, const uint2* __restrict__ blocks,
+                                                              const uint32_t* __restrict__ indices, const float* __restrict__ verts,
                                                               float* __restrict__ normals) {
 	const uint32_t i = blockIdx.x * MC_BLOCK + threadIdx.x;
-	if (i >= n_tris) return;
-	const uint32_t ia = indices[i * 3], ib = indices[i * 3 + 1], ic = indices[i * 3 + 2];
-	const float* pa = verts + (size_t)ia * 3;
-	const float* pb = verts + (size_t)ib * 3;
-	const float* pc = verts + (size_t)ic * 3;
-	const float u[3] = {pb[0] - pa[0], pb[1] - pa[1], pb[2] - pa[2]}, w[3] = {pa[0] - pc[0], pa[1] - pc[1], pa[2] - pc[2]};
-	const float nrm[3] = {u[1] * w[2] - u[2] * w[1], u[2] * w[0] - u[0] * w[2], u[0] * w[1] - u[1] * w[0]};
-	const uint32_t who[3] = {ia, ib, ic};
+	if (i >= n_verts) return;
+	float* mine = normals + (size_t)i * 3;
+	const uint32_t w = __float_as_uint(mine[0]), place = __float_as_uint(mine[1]);
+	const uint32_t lane = place & 63u, axis = place >> 6;
+	const uint32_t row = w / g.row_words, col = w - row * g.row_words;
+	const uint32_t xyz[3] = {col * 64u + lane, row % g.ry, row / g.ry};
+	// the two axes across the edge, the slower one first
+	const uint32_t slow = axis == 2u ? 1u : 2u, fast = axis == 0u ? 1u : 0u;
+	uint32_t first[4], count[4];
 #pragma unroll
-	for (int k = 0; k < 3; ++k)
+	for (uint32_t k = 0; k < 4; ++k) {
+		const uint32_t back_slow = k < 2u ? 1u : 0u, back_fast = (k & 1u) ? 0u : 1u;
+		const uint32_t bx = fast == 0u ? back_fast : 0u, by = (fast == 1u ? back_fast : 0u) + (slow == 1u ? back_slow : 0u), bz = slow == 2u ? back_slow : 0u;
+		count[k] = 0;
+		first[k] = 0;
+		if (bx > xyz[0] || by > xyz[1] || bz > xyz[2]) continue;
+		const uint32_t x = xyz[0] - bx, at = (row - by - bz * g.ry) * g.row_words + (x >> 6), l = x & 63u;
+		if (!((active[at >> 6] >> (at & 63u)) & 1ull)) continue;
+		const McRecord& r = records[at];
+		const mc_word t0 = r.tri[0], t1 = r.tri[1], t2 = r.tri[2];
+		count[k] = (uint32_t)((t0 >> l) & 1ull) | (uint32_t)((t1 >> l) & 1ull) << 1 | (uint32_t)((t2 >> l) & 1ull) << 2;
+		first[k] = blocks[at / MC_BLOCK].y + r.first_t + mc_below(t0, l) + 2u * mc_below(t1, l) + 4u * mc_below(t2, l);
+	}
+	float sum[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-		for (int d = 0; d < 3; ++d) atomicAdd(normals + (size_t)who[k] * 3 + d, nrm[d]);
+	for (uint32_t k = 0; k < 4; ++k) {
+		uint32_t tri[5][3];
+#pragma unroll
+		for (uint32_t t = 0; t < 5; ++t)
+#pragma unroll
+			for (uint32_t c = 0; c < 3; ++c) tri[t][c] = t < count[k] ? indices[(size_t)(first[k] + t) * 3 + c] : 0xFFFFFFFFu;
+#pragma unroll
+		for (uint32_t t = 0; t < 5; ++t) {
+			if (tri[t][0] != i && tri[t][1] != i && tri[t][2] != i) continue;
+			const float* pa = verts + (size_t)tri[t][0] * 3;
+			const float* pb = verts + (size_t)tri[t][1] * 3;
+			const float* pc = verts + (size_t)tri[t][2] * 3;
+			const float u[3] = {pb[0] - pa[0], pb[1] - pa[1], pb[2] - pa[2]}, v[3] = {pa[0] - pc[0], pa[1] - pc[1], pa[2] - pc[2]};
+			sum[0] += u[1] * v[2] - u[2] * v[1];
+			sum[1] += u[2] * v[0] - u[0] * v[2];
+			sum[2] += u[0] * v[1] - u[1] * v[0];
+		}
+	}
+#pragma unroll
+	for (uint32_t d = 0; d < 3; ++d) mine[d] = sum[d];
 }
 
 // ---------------------------------------------------------------------------
@@ -425,7 +491,7 @@ static inline uint64_t m256(uint64_t x) { return (x + 255) / 256 * 256; }
 
 N2_API int n2_marching_cubes_table(int8_t* out_256x16) {
 	N2_REQUIRE(out_256x16 != nullptr, "n2_marching_cubes_table: out is null");
-	memcpy(out_256x16, mc_table().tri, sizeof(mc_table().tri));
+	memcpy(out_256x16, MC_TABLE_HOST.tri, sizeof(MC_TABLE_HOST.tri));
 	return N2_OK;
 }
 
@@ -437,26 +503,23 @@ static int mc_check(const char* fn, const uint32_t res[3], uint64_t& n) {
 	return N2_OK;
 }
 
-// Workspace: voff (one word per lattice point, written only where a point owns a vertex), the two per-tile prefix-sum
-// arrays (one entry more than tiles: the total), the case table.
+// Workspace: the points' bits, one record per word (written only where a word owns something), which words do, and the
+// prefix sums over blocks of 256 words (one entry more than blocks: the totals).
 struct McCarve {
-	uint32_t n_tiles;
-	uint32_t n_blocks;  // blocks of 1024 tiles
-	uint64_t voff, vsum, tsum, busy, vblock, tblock, table, total;
+	uint32_t row_words, n_words, n_blocks;
+	uint64_t bits, records, active, blocks, total;
 };
-static McCarve mc_carve(uint64_t n) {
+static McCarve mc_carve(const uint32_t res[3]) {
 	McCarve c;
-	c.n_tiles = (uint32_t)((n + MC_WAVE_TILE - 1) / MC_WAVE_TILE);
+	c.row_words = (res[0] + 63u) / 64u;
+	c.n_words = c.row_words * res[1] * res[2];  // at most 2^30: rows have at least two points
+	c.n_blocks = (c.n_words + MC_BLOCK - 1) / MC_BLOCK;
 	uint64_t o = 0;
 	auto take = [&](uint64_t bytes) { const uint64_t at = o; o += m256(bytes); return at; };
-	c.voff = take(4 * n);
-	c.vsum = take(4ull * (c.n_tiles + 4));
-	c.tsum = take(4ull * (c.n_tiles + 4));
-	c.busy = take(c.n_tiles);
-	c.n_blocks = (c.n_tiles + 1023u) / 1024u;
-	c.vblock = take(4ull * c.n_blocks);
-	c.tblock = take(4ull * c.n_blocks);
-	c.table = take(sizeof(McTable));
+	c.bits = take(sizeof(mc_word) * (uint64_t)c.n_words);
+	c.records = take(sizeof(McRecord) * (uint64_t)c.n_words);
+	c.active = take(sizeof(mc_word) * (uint64_t)c.n_blocks * (MC_BLOCK / 64));
+	c.blocks = take(sizeof(uint2) * ((uint64_t)c.n_blocks + 1));
 	c.total = o;
 	return c;
 }
@@ -464,17 +527,18 @@ static McCarve mc_carve(uint64_t n) {
 N2_API uint64_t n2_marching_cubes_workspace_bytes(const uint32_t res[3]) {
 	uint64_t n;
 	if (mc_check("n2_marching_cubes_workspace_bytes", res, n) != N2_OK) return 0;
-	return mc_carve(n).total;
+	return mc_carve(res).total;
 }
 
 static McGrid mc_grid(const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh) {
 	McGrid g;
 	g.rx = res[0]; g.ry = res[1]; g.rz = res[2]; g.thresh = thresh;
 	for (int d = 0; d < 3; ++d) { g.scale[d] = (aabb_max[d] - aabb_min[d]) / (float)res[d]; g.offset[d] = aabb_min[d]; }
+	const McCarve c = mc_carve(res);
+	g.row_words = c.row_words;
+	g.n_words = c.n_words;
 	return g;
 }
-static inline dim3 mc_tile_grid(uint32_t n_tiles) { const uint32_t per = MC_BLOCK / 64 * MC_COUNT_TILES; return dim3((n_tiles + per - 1) / per); }
-static inline dim3 mc_emit_grid(uint32_t n_tiles) { const uint32_t b = (n_tiles + MC_BLOCK / 64 - 1) / (MC_BLOCK / 64); return dim3(b < MC_EMIT_BLOCKS ? b : MC_EMIT_BLOCKS); }
 
 N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,
                                    const float* d_density, void* d_workspace, uint64_t workspace_bytes, uint32_t* n_vertices,
@@ -483,27 +547,22 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	if (int rc = mc_check("n2_marching_cubes_count", res, n)) return rc;
 	N2_REQUIRE(d_density && d_workspace && n_vertices && n_triangles && aabb_min && aabb_max, "n2_marching_cubes_count: null argument");
 	N2_REQUIRE(reinterpret_cast<uintptr_t>(d_workspace) % 256 == 0, "n2_marching_cubes_count: workspace must be 256-byte aligned");
-	const McCarve c = mc_carve(n);
+	const McCarve c = mc_carve(res);
 	N2_REQUIRE(workspace_bytes >= c.total, "n2_marching_cubes_count: %llu bytes of workspace given, %llu needed",
 	           (unsigned long long)workspace_bytes, (unsigned long long)c.total);
 	hipStream_t s = n2_stream(stream);
 	unsigned char* b = reinterpret_cast<unsigned char*>(d_workspace);
-	uint32_t* vsum = reinterpret_cast<uint32_t*>(b + c.vsum);
-	uint32_t* tsum = reinterpret_cast<uint32_t*>(b + c.tsum);
-	McTable* table = reinterpret_cast<McTable*>(b + c.table);
-	N2_HIP(hipMemcpyAsync(table, &mc_table(), sizeof(McTable), hipMemcpyHostToDevice, s));
+	mc_word* bits = reinterpret_cast<mc_word*>(b + c.bits);
+	uint2* blocks = reinterpret_cast<uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
-	mc_count_kernel<<<mc_tile_grid(c.n_tiles), dim3(MC_BLOCK), 0, s>>>(g, table, d_density, c.n_tiles, vsum, tsum, b + c.busy);
+	mc_bits_kernel<<<mgrid(((uint64_t)c.n_words + MC_BITS_WORDS - 1) / MC_BITS_WORDS * 64u), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits);
 	N2_LAUNCH_CHECK();
-	uint32_t* vblock = reinterpret_cast<uint32_t*>(b + c.vblock);
-	uint32_t* tblock = reinterpret_cast<uint32_t*>(b + c.tblock);
-	mc_block_totals_kernel<<<dim3(c.n_blocks, 2), dim3(1024), 0, s>>>(c.n_tiles, vsum, tsum, vblock, tblock);
+	mc_count_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
 	N2_LAUNCH_CHECK();
-	mc_scan_kernel<<<dim3(c.n_blocks, 2), dim3(1024), 0, s>>>(c.n_tiles, vsum, tsum, vblock, tblock);
+	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks);
 	N2_LAUNCH_CHECK();
 	uint32_t host[2] = {0, 0};
-	N2_HIP(hipMemcpyAsync(&host[0], vsum + c.n_tiles, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-	N2_HIP(hipMemcpyAsync(&host[1], tsum + c.n_tiles, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+	N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
 	N2_HIP(hipStreamSynchronize(s));
 	N2_REQUIRE(host[0] < (1u << 29), "n2_marching_cubes_count: %u vertices exceed the 2^29 limit", host[0]);
 	*n_vertices = host[0];
@@ -518,29 +577,22 @@ N2_API int n2_marching_cubes_emit(n2_stream_t stream, const uint32_t res[3], con
 	if (int rc = mc_check("n2_marching_cubes_emit", res, n)) return rc;
 	N2_REQUIRE(d_density && d_workspace && aabb_min && aabb_max, "n2_marching_cubes_emit: null argument");
 	N2_REQUIRE((d_vertices || n_vertices == 0) && (d_indices || n_triangles == 0), "n2_marching_cubes_emit: null output");
-	hipStream_t s = n2_stream(stream);
-	const McCarve c = mc_carve(n);
-	unsigned char* b = reinterpret_cast<unsigned char*>(d_workspace);
-	uint32_t* voff = reinterpret_cast<uint32_t*>(b + c.voff);
-	const uint32_t* vsum = reinterpret_cast<const uint32_t*>(b + c.vsum);
-	const uint32_t* tsum = reinterpret_cast<const uint32_t*>(b + c.tsum);
-	const McTable* table = reinterpret_cast<const McTable*>(b + c.table);
 	N2_REQUIRE(d_normals == nullptr || reinterpret_cast<uintptr_t>(d_normals) % 16 == 0, "n2_marching_cubes_emit: d_normals must be 16-byte aligned");
+	if (n_vertices == 0) return N2_OK;  // no cut edge: no triangles either
+	hipStream_t s = n2_stream(stream);
+	const McCarve c = mc_carve(res);
+	unsigned char* b = reinterpret_cast<unsigned char*>(d_workspace);
+	const mc_word* bits = reinterpret_cast<const mc_word*>(b + c.bits);
+	const McRecord* records = reinterpret_cast<const McRecord*>(b + c.records);
+	const mc_word* active = reinterpret_cast<const mc_word*>(b + c.active);
+	const uint2* blocks = reinterpret_cast<const uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
-	if (n_vertices) {
-		mc_vertices_kernel<<<mc_emit_grid(c.n_tiles), dim3(MC_BLOCK), 0, s>>>(g, d_density, c.n_tiles, vsum, b + c.busy, voff, d_vertices);
+	mc_emit_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits, records, active, blocks, d_vertices, d_indices,
+	                                                           reinterpret_cast<uint32_t*>(d_normals));
+	N2_LAUNCH_CHECK();
+	if (d_normals) {
+		mc_normals_kernel<<<mgrid(n_vertices), dim3(MC_BLOCK), 0, s>>>(g, n_vertices, records, active, blocks, d_indices, d_vertices, d_normals);
 		N2_LAUNCH_CHECK();
-	}
-	if (n_triangles) {
-		mc_faces_kernel<<<mc_emit_grid(c.n_tiles), dim3(MC_BLOCK), 0, s>>>(g, table, d_density, c.n_tiles, tsum, b + c.busy, voff, d_indices);
-		N2_LAUNCH_CHECK();
-	}
-	if (d_normals && n_vertices) {
-		if (int rc = n2_fill_zero_u32(s, d_normals, 12ull * n_vertices)) return rc;
-		if (n_triangles) {
-			mc_normals_kernel<<<mgrid(n_triangles), dim3(MC_BLOCK), 0, s>>>(n_triangles, d_indices, d_vertices, d_normals);
-			N2_LAUNCH_CHECK();
-		}
 	}
 	return N2_OK;
 }

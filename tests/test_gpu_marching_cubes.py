@@ -42,6 +42,20 @@ def test_mesh_matches_oracle(res, kind):
         assert check_closed_oriented(host(v), host(t).astype(np.int64)) == 2
 
 
+@pytest.mark.parametrize("res", [(63, 6, 5), (64, 6, 5), (65, 6, 5), (128, 30, 12), (129, 40, 11)])  # one point short of a word of 64, exact, one over; several blocks of words
+def test_rows_of_words(res):
+    """Noise: every word of points owns something, so the points of a block fill the emitting kernel's list several times."""
+    from neus2_amd.mesh import marching_cubes
+    f = np.random.default_rng(res[0] + res[1]).standard_normal((res[2], res[1], res[0])).astype(np.float32)
+    want_v, want_t = omc.marching_cubes(f, res, 0.0, (0, 0, 0), (1, 1, 1))
+    v, t, n = marching_cubes(dev(f), 0.0)
+    np.testing.assert_array_equal(host(v), want_v)
+    np.testing.assert_array_equal(host(t).view(np.uint32), want_t)
+    want_n = omc.vertex_normals(want_v, want_t)
+    np.testing.assert_allclose(host(n), want_n, rtol=1e-4, atol=1e-6 * max(1.0, float(np.abs(want_n).max())))
+    assert marching_cubes(dev(f), 0.0, want_normals=False)[2] is None
+
+
 def test_empty_lattice_and_errors():
     from neus2_amd import capi
     from neus2_amd.mesh import marching_cubes
