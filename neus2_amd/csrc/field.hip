@@ -806,15 +806,14 @@ int n2_field_sdf_row0(n2_field_t* f, n2_stream_t stream, const float* d_xyz, uin
 	return N2_OK;
 }
 
-bool n2_field_sdf_row0_lattice(n2_field_t* f, n2_stream_t stream, const N2Lattice& lattice, uint32_t n, uint32_t n_keep, float* d_row0, int* rc) {
-	*rc = check_field(f, "n2_field_sdf", n);
+bool n2_field_sdf_row0_lattice(n2_field_t* f, n2_stream_t stream, const N2Lattice& lattice, uint32_t chunk, void* d_scratch, void* d_frags, float* d_row0, int* rc) {
+	const uint64_t points = (uint64_t)lattice.res[0] * lattice.res[1] * lattice.res[2];
+	*rc = check_field(f, "n2_field_sdf", points < chunk ? (uint32_t)((points + 7) / 8 * 8) : chunk);
 	if (*rc != N2_OK) return true;
-	if (!(f->fused && fused_ok(f) && n2_grid_lattice_order(f->grid))) return false;
-	if (n == 0) return true;
-	if (d_row0 == nullptr) { n2_set_error("n2_field_sdf: null buffer"); *rc = N2_ERR_INVALID_ARGUMENT; return true; }
+	if (!(f->fused && fused_ok(f)) || chunk < lattice.res[0]) return false;
 	hipStream_t s = n2_stream(stream);
 	N2ProfScope prof(N2_PROF_FIELD_FORWARD, s);
-	*rc = n2_fused_field_sdf(fused_nets(f), s, nullptr, 0, 0, n, nullptr, d_row0, false, nullptr, n_keep, &lattice);
+	*rc = n2_fused_lattice_sdf(fused_nets(f), s, lattice, chunk, d_scratch, d_frags, d_row0);
 	return true;
 }
 

@@ -27,15 +27,16 @@
 
 #include "grid_device.h"
 #include "mlp_device.h"
+#include "sdf_frags.h"
 
 constexpr int FF_BLOCK = 256;  // 4 waves
 constexpr uint32_t FF_LEVELS = 16;  // levels the lane layout covers
 
 // fragment numbers (64 lanes x 16 bytes each)
 enum : int {
-	S_W0 = 0,    // [mt][c]  SDF net W_0 rows 32 mt + n; c = 0, 1: feature rows in chained order, c = 2: centred coordinates
-	S_WO = 6,    // [c]      SDF net W_out rows n < 16, chained K
-	FF_SDF_COUNT = 10,
+	S_W0 = SDF_FRAG_W0,  // the SDF net's forward (sdf_frags.h)
+	S_WO = SDF_FRAG_WO,
+	FF_SDF_COUNT = SDF_FRAG_COUNT,
 	S_W0T = 10,  // [mt][c]  SDF net W_0^T, row = internal input row 32 mt + n, chained K over the neurons
 	S_DH = 18,   // [c]      row 0 of W_out as a chained B operand (every column the same): d sdf / d hidden before the mask
 	C_W0 = 22,   // [mt][c]  colour net W_0 rows 32 mt + n; c = 0 chained (SDF-net outputs), c = 1, 2 natural
@@ -71,9 +72,8 @@ struct FusedArgs {
 	// full field: the weight fragments of the network kernel as one image in global memory (FF_COUNT KiB; null: every
 	// workgroup builds them from the weights).  The gather launch in front of the network kernel writes it.
 	hf* frags;
-	const float* pos;       // coordinate d of sample i at pos[i * ps + d * ds]; null: sample i is point lat.first + i of a lattice
+	const float* pos;       // coordinate d of sample i at pos[i * ps + d * ds]
 	uint32_t ps, ds;
-	N2Lattice lat;
 	const float* coords;    // full field: [N][7] NerfCoordinate (direction at 4..6)
 	// full field: what the backward pass reads, and the output
 	hf* sdf_in;             // [sdf_in_w][N]  rows 0..2 centred coordinates, 3.. features
@@ -89,15 +89,6 @@ struct FusedArgs {
 	int density;            // row 0 becomes the logistic density
 };
 
-__device__ __forceinline__ hf h_or_zero(const hf* W, bool ok, size_t at) { return ok ? W[at] : (hf)0; }
-
-// internal input row of the SDF net -> column of W_0 (or -1): rows 0..31 are features, 32..34 the coordinates
-__device__ __forceinline__ int sdf_col(int row, uint32_t enc_w) {
-	if (row < 32) return (uint32_t)row < enc_w ? 3 + row : -1;
-	return row < 35 ? row - 32 : -1;
-}
-__device__ __forceinline__ int chained_k(int c, int g, int e) { return 16 * c + 4 * g + (e & 3) + ((e >> 2) << 3); }
-
 // lane l's 16 bytes of fragment f
 __device__ __forceinline__ half8 fused_frag_value(const FusedArgs& a, int f, int l) {
 	const hf* W0s = a.sdf_w;
@@ -109,15 +100,8 @@ __device__ __forceinline__ half8 fused_frag_value(const FusedArgs& a, int f, int
 	{
 		const int n = l & 31, g = l >> 5;
 		half8 v = zero8();
-		if (f < S_WO) {
-			const int mt = f / 3, c = f % 3, row = 32 * mt + n;
-#pragma unroll
-			for (int e = 0; e < 8; ++e) {
-				const int col = c < 2 ? sdf_col(chained_k(c, g, e), a.enc_w) : sdf_col(32 + 8 * g + e, a.enc_w);
-				v[e] = h_or_zero(W0s, col >= 0, (size_t)row * ld_s + (col >= 0 ? col : 0));
-			}
-		} else if (f < S_W0T) {
-			if (n < MLP_OUT) v = wfrag_chained(W1s, MLP_WIDTH, n, f - S_WO, g);
+		if (f < S_W0T) {
+			v = sdf_forward_frag(W0s, ld_s, a.enc_w, f, l);
 		} else if (f < S_DH) {
 			const int q = f - S_W0T, mt = q >> 2, c = q & 3, col = sdf_col(32 * mt + n, a.enc_w);
 #pragma unroll
@@ -433,19 +417,9 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 		float p[3], dir[3] = {0.f, 0.f, 0.f};
 		uint4 slope[8];            // FULL: the slopes of the lane's 8 levels as stored
 		if (GATHER) {
-			if (a.pos) {
-				const float* q = a.pos + (size_t)col * a.ps;
+			const float* q = a.pos + (size_t)col * a.ps;
 #pragma unroll
-				for (int d = 0; d < 3; ++d) p[d] = q[(size_t)d * a.ds];
-			} else {
-				// lattice point (x, y, z), x fastest: (c / res) * extent + corner, each step rounded on its own (the positions are
-				// part of a bit-exact contract); points behind the lattice's end sit at the centre
-				const uint32_t idx = a.lat.first + col;
-				const uint32_t c[3] = {idx % a.lat.res[0], (idx / a.lat.res[0]) % a.lat.res[1], idx / (a.lat.res[0] * a.lat.res[1])};
-#pragma unroll
-				for (int d = 0; d < 3; ++d)
-					p[d] = idx < a.lat.total ? __fadd_rn(__fmul_rn(__fmul_rn((float)c[d], a.lat.inv_res[d]), a.lat.extent[d]), a.lat.corner[d]) : 0.5f;
-			}
+			for (int d = 0; d < 3; ++d) p[d] = q[(size_t)d * a.ds];
 			// the lane's 8 levels, the next level's loads in flight while one is finished
 			Item cur, nxt;
 			float unused[2][3];
@@ -730,13 +704,9 @@ int n2_fused_field_forward(const N2FusedNets& nets, hipStream_t s, const float* 
 }
 
 int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
-                       float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n, const N2Lattice* lattice) {
+                       float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n) {
 	FusedArgs a = fused_base(nets, n);
 	a.pos = d_xyz; a.ps = ps; a.ds = ds;
-	if (lattice) {
-		if (d_xyz != nullptr || sdf_in != nullptr) { n2_set_error("n2_fused_field_sdf: lattice points are generated in the one-launch form only"); return N2_ERR_INVALID_ARGUMENT; }
-		a.lat = *lattice;
-	}
 	a.sdf_out = reinterpret_cast<hf*>(d_out_soa);
 	a.row0 = d_row0;
 	a.row0_n = row0_n < n ? row0_n : n;

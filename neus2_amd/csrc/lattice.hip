@@ -1,0 +1,480 @@
+// The field's SDF on a regular lattice (Testbed::get_density_on_grid, src/testbed_nerf.cu:4082-4133): what mesh extraction
+// evaluates, up to 2^31 points at a time.
+//
+// On a lattice everything that a point's place in the encoding depends on is separable: cell and weight along an axis are
+// functions of one index.  A wave takes a run of 64 points along x at one y and walks along z, so y and z quantities are
+// wave-uniform (scalar registers) and a lane keeps only what depends on its x.  Two kinds of levels:
+//  * coarse levels, whose cells are larger than the z step (lattice_walk_kernel): the values of the two z planes of vertices
+//    round the walk's position stay in registers, already interpolated in x and y; a step only interpolates in z, and a
+//    plane is gathered when the walk crosses into it (once per cell, loads issued one step ahead).
+//  * fine levels (lattice_fine_kernel): nothing is shared between steps.  They run level by level over a slab of planes, so
+//    that the 2 MiB table being read stays in every XCD's L2, and leave their features in the caller's scratch; the walk
+//    picks them up.  (Point by point through all levels, 10 MiB of fine tables compete for 4 MiB of L2: 44 % of the requests
+//    missed, 1.4 GB per 2^22 points through the fabric.)
+// The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
+// level" into the operand layout "lane = (point, level group)" without touching LDS.
+// 512^3 lattice: 8.2 -> 5.8 ms, per slab of 7.6e6 points 153 us for six fine levels and 180 us for the walk, which its vector
+// and matrix instructions hold at two waves per SIMD (its plane values take 60 registers, the loads in flight 52).
+#include "n2_common.h"
+
+#include "grid_device.h"
+#include "mlp_device.h"
+#include "sdf_frags.h"
+
+#include <type_traits>
+
+constexpr uint32_t LT_LEVELS = 16;
+constexpr uint32_t LT_BLOCK = 256;
+constexpr uint32_t LT_MAX_FINE = 11;  // feature rows of 4 bytes per point that the scratch holds (n2_density_on_grid_scratch_bytes)
+
+struct LatticeArgs {
+	float scale[LT_LEVELS];
+	uint32_t res[LT_LEVELS], entries[LT_LEVELS], offset[LT_LEVELS];
+	uint32_t hash_mask, active_levels, n_levels;
+	const __half2* table;
+	const hf* frags;          // fragment image of the SDF network
+	float sdf_bias;
+	N2Lattice lat;
+	uint32_t y0, ny, z0, nz;  // the slab: rows y0 .. y0 + ny of planes z0 .. z0 + nz
+	uint32_t x_runs, walk;    // runs of 64 points per row; planes per wave
+	uint32_t first_fine;      // levels first_fine .. n_levels - 1 come from `features`
+	uint32_t* features;       // [n_levels - first_fine][nz ny rx] half2
+	float* out;               // row 0 of point (0, y0, z0)
+};
+
+// coordinate of lattice index c on axis d: each step rounded on its own (positions are part of a bit-exact contract)
+__device__ __forceinline__ float lattice_coord(const N2Lattice& lat, int d, uint32_t c) {
+	return __fadd_rn(__fmul_rn(__fmul_rn((float)c, lat.inv_res[d]), lat.extent[d]), lat.corner[d]);
+}
+__device__ __forceinline__ uint32_t lane_u32(uint32_t v, uint32_t lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane); }
+__device__ __forceinline__ float lane_f32(float v, uint32_t lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)lane)); }
+
+// A vertex's byte offset in its level's table is  xo ^ row  on a hashed level and  xo + row  (minus the table's size if that
+// is past its end) on a dense one, xo the part of x and row the part of (y, z).
+__device__ __forceinline__ uint32_t x_part(bool hashed, uint32_t entries, uint32_t res, uint32_t gx) {
+	return (hashed ? gx & (entries - 1u) : min(gx, res)) << 2;
+}
+__device__ __forceinline__ uint32_t row_part(bool hashed, uint32_t entries, uint32_t res, uint32_t gy, uint32_t gz) {
+	return (hashed ? ((gy * 2654435761u) ^ (gz * 805459861u)) & (entries - 1u) : min(gy, res) * res + min(gz, res) * res * res) << 2;
+}
+__device__ __forceinline__ uint32_t vertex(bool hashed, uint32_t table_bytes, uint32_t xo, uint32_t row) {
+	if (hashed) return xo ^ row;
+	const uint32_t at = xo + row;
+	return min(at, at - table_bytes);  // one conditional subtraction stands in for the modulo (unsigned wrap-around)
+}
+__device__ __forceinline__ float2 lt_h2f(uint32_t raw) {
+	const half2v h = __builtin_bit_cast(half2v, raw);
+	return make_float2((float)h[0], (float)h[1]);
+}
+__device__ __forceinline__ uint32_t lt_pack(float a, float b) {
+	const half2v h = {(hf)a, (hf)b};
+	return __builtin_bit_cast(uint32_t, h);
+}
+
+// The wave's run: x of the lane (clamped into the row), y, first plane.  False: nothing to do.
+__device__ __forceinline__ bool lattice_run(const LatticeArgs& a, uint32_t wave, uint32_t& x, uint32_t& y, uint32_t& z, uint32_t& nz) {
+	const uint32_t xr = wave % a.x_runs, rest = wave / a.x_runs, yy = rest % a.ny, zz = rest / a.ny;
+	if (zz * a.walk >= a.nz) return false;
+	x = xr * 64u + (threadIdx.x & 63u);
+	y = a.y0 + yy;
+	z = a.z0 + zz * a.walk;
+	nz = min(a.walk, a.nz - zz * a.walk);
+	return true;
+}
+
+// Fine levels, level-major workgroup ids.  A run needs eight vertices per point, on four rows (y, z), (y + 1, z), (y, z + 1),
+// (y + 1, z + 1).  On a hashed level a row's neighbours in x stand in one aligned 128-byte line per 32, permuted; a load
+// instruction costs the L1 one clock per group of four lanes at least, and up to four where the lanes' spacing makes their
+// banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks per 4-byte load).  So the wave loads the rows as a
+// whole, 16 bytes per lane, into LDS (FINE_CHUNKS of them per row) and picks the vertices there: for six levels of 2^22 points
+// 153 -> 89 us (L2 fills 52 us of it, LDS 58, measured by counters).  Runs longer than that (coarse lattices) and dense levels gather from memory.
+constexpr uint32_t FINE_CHUNKS = 128;
+
+__global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArgs a, uint32_t blocks_per_level) {
+	__shared__ uint4v staged[LT_BLOCK / 64][4][FINE_CHUNKS];
+	const uint32_t level = a.first_fine + blockIdx.x / blocks_per_level;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x % blocks_per_level) * (LT_BLOCK / 64) + (threadIdx.x >> 6));
+	uint32_t x, y, z, nz;
+	if (!lattice_run(a, wave, x, y, z, nz)) return;
+	const bool inside = x < a.lat.res[0];
+	const uint32_t lane = threadIdx.x & 63u, plane = a.lat.res[0] * a.ny;
+	uint32_t* out = a.features + (size_t)(level - a.first_fine) * plane * a.nz + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.lat.res[0] + x;
+	if (level >= a.active_levels) {
+		for (uint32_t k = 0; k < nz; ++k)
+			if (inside) out[(size_t)k * plane] = 0u;
+		return;
+	}
+	const float scale = a.scale[level];
+	const uint32_t res = a.res[level], entries = a.entries[level], bytes = entries << 2;
+	const bool hashed = (a.hash_mask >> level) & 1u;
+	float wx, wy, wz;
+	uint32_t cx, cy, cz;
+	n2_locate(lattice_coord(a.lat, 0, min(x, a.lat.res[0] - 1u)), scale, wx, cx);
+	n2_locate(lattice_coord(a.lat, 1, y), scale, wy, cy);
+	n2_locate(lattice_coord(a.lat, 2, z + min(lane, nz - 1u)), scale, wz, cz);  // lane k: plane z + k (at most 64 of them)
+	// lane k: the four rows of vertices of plane z + k and their weights
+	uint32_t rows[4];
+	float weights[4];
+#pragma unroll
+	for (uint32_t q = 0; q < 4; ++q) {
+		rows[q] = row_part(hashed, entries, res, cy + (q & 1u), cz + (q >> 1));
+		weights[q] = ((q & 1u) ? wy : 1.f - wy) * ((q >> 1) ? wz : 1.f - wz);
+	}
+	const char* base = reinterpret_cast<const char*>(a.table + a.offset[level]);
+	const float ux = 1.f - wx;
+	auto finish = [&](uint32_t k, const uint32_t (&raw)[8]) {
+		float s[2][2] = {};
+#pragma unroll
+		for (uint32_t q = 0; q < 4; ++q) {
+			const float w = lane_f32(weights[q], k);
+#pragma unroll
+			for (uint32_t b = 0; b < 2; ++b) {
+				const float2 v = lt_h2f(raw[2 * q + b]);
+				s[b][0] = fmaf(w, v.x, s[b][0]);
+				s[b][1] = fmaf(w, v.y, s[b][1]);
+			}
+		}
+		if (inside) *out = lt_pack(fmaf(ux, s[0][0], wx * s[1][0]), fmaf(ux, s[0][1], wx * s[1][1]));
+		out += plane;
+	};
+	// chunks of four entries that the run meets: from c_lo's to the one behind c_hi's
+	const uint32_t c_first = lane_u32(cx, 0), c_last = lane_u32(cx, 63);
+	const bool up = (int32_t)(c_last - c_first) >= 0;
+	const uint32_t c_lo = (up ? c_first : c_last) & ~3u, chunks = (((up ? c_last : c_first) + 1u - c_lo) >> 2) + 1u;
+	if (hashed && chunks <= FINE_CHUNKS) {
+		// (lanes behind the last chunk load it again, into a slot nobody reads)
+		const uint32_t o0 = ((c_lo + 4u * min(lane, chunks - 1u)) & (entries - 1u)) << 2, o1 = ((c_lo + 4u * min(lane + 64u, chunks - 1u)) & (entries - 1u)) << 2;
+		uint4v (&st)[4][FINE_CHUNKS] = staged[threadIdx.x >> 6];
+		const uint32_t at0 = (cx - c_lo) << 2, at1 = at0 + 4u;
+		auto walk = [&](auto halves) {
+			constexpr uint32_t H = decltype(halves)::value;  // 64 chunks per load instruction and row
+			for (uint32_t k = 0; k < nz; ++k) {
+				uint32_t row[4];
+				uint4v v[4][H];
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q) row[q] = lane_u32(rows[q], k);
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q)
+#pragma unroll
+					for (uint32_t h = 0; h < H; ++h) v[q][h] = *reinterpret_cast<const uint4v*>(base + ((h ? o1 : o0) ^ (row[q] & ~15u)));
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q)
+#pragma unroll
+					for (uint32_t h = 0; h < H; ++h) st[q][lane + 64u * h] = v[q][h];
+				__builtin_amdgcn_wave_barrier();
+				uint32_t raw[8];
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q) {
+					const uint32_t flip = row[q] & 12u;  // a chunk's entries are permuted by the row's low bits
+					raw[2 * q] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(&st[q][0]) + (at0 ^ flip));
+					raw[2 * q + 1] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(&st[q][0]) + (at1 ^ flip));
+				}
+				__builtin_amdgcn_wave_barrier();
+				finish(k, raw);
+			}
+		};
+		if (chunks > 64u) walk(std::integral_constant<uint32_t, 2>());
+		else walk(std::integral_constant<uint32_t, 1>());
+		return;
+	}
+	const uint32_t x0 = x_part(hashed, entries, res, cx), x1 = x_part(hashed, entries, res, cx + 1u);
+	for (uint32_t k = 0; k < nz; ++k) {
+		uint32_t raw[8];
+#pragma unroll
+		for (uint32_t q = 0; q < 4; ++q) {
+			const uint32_t row = lane_u32(rows[q], k);
+			raw[2 * q] = *reinterpret_cast<const uint32_t*>(base + vertex(hashed, bytes, x0, row));
+			raw[2 * q + 1] = *reinterpret_cast<const uint32_t*>(base + vertex(hashed, bytes, x1, row));
+		}
+		finish(k, raw);
+	}
+}
+
+// exchange of the upper 32 lanes of `a` with the lower 32 of `b`
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+	const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+	a = r[0];
+	b = r[1];
+}
+
+// The walk.  NM levels are interpolated here, the others come from a.features.
+template <int NM>
+__global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const LatticeArgs a) {
+	__shared__ __align__(16) hf F[SDF_FRAG_COUNT * 512];
+	for (uint32_t i = threadIdx.x; i < SDF_FRAG_COUNT * 64u; i += LT_BLOCK) *reinterpret_cast<half8*>(F + i * 8u) = *reinterpret_cast<const half8*>(a.frags + i * 8u);
+	__syncthreads();
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (LT_BLOCK / 64) + (threadIdx.x >> 6));
+	uint32_t x, y, z, nz;
+	if (!lattice_run(a, wave, x, y, z, nz)) return;
+	const uint32_t lane = threadIdx.x & 63u, rx = a.lat.res[0], plane = rx * a.ny;
+	const bool inside = x < rx;
+	const float px = lattice_coord(a.lat, 0, min(x, rx - 1u)), py = lattice_coord(a.lat, 1, y);
+	const char* base[NM];
+#pragma unroll
+	for (int l = 0; l < NM; ++l) base[l] = reinterpret_cast<const char*>(a.table + a.offset[l]);
+	// lane l: what depends on y and z of level l
+	const uint32_t ll = lane & (LT_LEVELS - 1u);
+	const float my_scale = a.scale[ll];
+	const uint32_t my_res = a.res[ll], my_entries = a.entries[ll];
+	const bool my_hashed = (a.hash_mask >> ll) & 1u;
+	const uint32_t on = a.active_levels >= 32u ? ~0u : (1u << a.active_levels) - 1u;  // levels in use
+	float my_wy, my_wz;
+	uint32_t my_cy, my_cz;
+	n2_locate(py, my_scale, my_wy, my_cy);
+	n2_locate(lattice_coord(a.lat, 2, z), my_scale, my_wz, my_cz);
+	float wy[NM];
+#pragma unroll
+	for (int l = 0; l < NM; ++l) wy[l] = lane_f32(my_wy, l);
+	// the plane of vertices at `row0`, `row1` (byte offsets of its rows y, y + 1): four gathers, and their interpolation in x and y
+	// What depends on x is worked out at each plane, from an opaque copy of the position: kept across the loop, cell and weight of
+	// every level take 40 registers, and the walk needs three waves per SIMD to cover its loads.
+	auto place = [&](int l, float& w, uint32_t& c) {
+		float p = px;
+		asm volatile("" : "+v"(p));
+		n2_locate(p, a.scale[l], w, c);
+	};
+	auto fetch = [&](int l, uint32_t row0, uint32_t row1, uint32_t (&raw)[4]) {
+		const bool hashed = (a.hash_mask >> l) & 1u;
+		const uint32_t bytes = a.entries[l] << 2;
+		float w;
+		uint32_t cx;
+		place(l, w, cx);
+		if (hashed) {
+			const uint32_t x0 = x_part(true, a.entries[l], a.res[l], cx), x1 = x_part(true, a.entries[l], a.res[l], cx + 1u);
+			raw[0] = *reinterpret_cast<const uint32_t*>(base[l] + (x0 ^ row0));
+			raw[1] = *reinterpret_cast<const uint32_t*>(base[l] + (x1 ^ row0));
+			raw[2] = *reinterpret_cast<const uint32_t*>(base[l] + (x0 ^ row1));
+			raw[3] = *reinterpret_cast<const uint32_t*>(base[l] + (x1 ^ row1));
+		} else {
+			const uint32_t x0 = x_part(false, a.entries[l], a.res[l], cx), x1 = x_part(false, a.entries[l], a.res[l], cx + 1u);
+			raw[0] = *reinterpret_cast<const uint32_t*>(base[l] + vertex(false, bytes, x0, row0));
+			raw[1] = *reinterpret_cast<const uint32_t*>(base[l] + vertex(false, bytes, x1, row0));
+			raw[2] = *reinterpret_cast<const uint32_t*>(base[l] + vertex(false, bytes, x0, row1));
+			raw[3] = *reinterpret_cast<const uint32_t*>(base[l] + vertex(false, bytes, x1, row1));
+		}
+	};
+	auto blend = [&](int l, const uint32_t (&raw)[4], float2& p) {
+		const float2 v0 = lt_h2f(raw[0]), v1 = lt_h2f(raw[1]), v2 = lt_h2f(raw[2]), v3 = lt_h2f(raw[3]);
+		float vx, vy = wy[l];
+		uint32_t cx;
+		place(l, vx, cx);
+		asm volatile("" : "+v"(vy));
+		const float uy = 1.f - vy, ux = 1.f - vx, w0 = ux * uy, w1 = vx * uy, w2 = ux * vy, w3 = vx * vy;
+		// (the products too as multiply-adds: those take half-precision operands as they are)
+		p.x = fmaf(w0, v0.x, fmaf(w1, v1.x, fmaf(w2, v2.x, fmaf(w3, v3.x, 0.f))));
+		p.y = fmaf(w0, v0.y, fmaf(w1, v1.y, fmaf(w2, v2.y, fmaf(w3, v3.y, 0.f))));
+	};
+	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) {
+		r0 = row_part(my_hashed, my_entries, my_res, my_cy, cz);
+		r1 = row_part(my_hashed, my_entries, my_res, my_cy + 1u, cz);
+	};
+	float2 lo[NM], hi[NM], rise[NM];  // planes below and above, and their difference
+	auto both_planes = [&](uint32_t which, uint32_t cz) {
+		uint32_t r0, r1, q0, q1;
+		rows_of(cz, r0, r1);
+		rows_of(cz + 1u, q0, q1);
+		uint32_t raw[NM][4];
+		// (all levels' loads of a plane in flight together)
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) blend(l, raw[l], lo[l]);
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) fetch(l, lane_u32(q0, l), lane_u32(q1, l), raw[l]);
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) {
+				blend(l, raw[l], hi[l]);
+				rise[l] = make_float2(hi[l].x - lo[l].x, hi[l].y - lo[l].y);
+			}
+	};
+#pragma unroll
+	for (int l = 0; l < NM; ++l) lo[l] = hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched-off levels
+	both_planes(on, my_cz);
+	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * rx + min(x, rx - 1u);
+	const size_t feat_level = (size_t)plane * a.nz;
+	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + x;
+	const uint32_t g = lane >> 5;  // of the lanes with g = 0 a tile's operands take the coordinates
+	const hf ycoord = (hf)py - (hf)0.5f;
+	// tile 0 works for lanes 0..31, tile 1 for lanes 32..63: the x coordinate of both, for the lanes that need it (g = 0)
+	uint32_t xc0 = lt_pack((float)((hf)px - (hf)0.5f), (float)ycoord), xc1 = xc0;
+	swap_halves(xc0, xc1);
+	xc0 = g == 0u ? xc0 : 0u;
+	xc1 = g == 0u ? xc1 : 0u;
+	// (levels that the table does not have read the last one's row: their weights are zero)
+	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
+	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
+	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) {
+#pragma unroll
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = feat[(size_t)(have_fine ? min(f, a.n_levels - 1u - NM) : 0u) * feat_level + (size_t)k * plane];
+	};
+	load_fine(0, fine);
+	load_fine(min(1u, nz - 1u), ahead);
+	for (uint32_t k = 0; k < nz; ++k) {
+		const float pz = lattice_coord(a.lat, 2, z + k);
+		// features of this step
+		uint32_t enc[LT_LEVELS];
+#pragma unroll
+		for (int l = 0; l < NM; ++l) {
+			const float vz = lane_f32(my_wz, l);
+			enc[l] = lt_pack(fmaf(vz, rise[l].x, lo[l].x), fmaf(vz, rise[l].y, lo[l].y));
+		}
+#pragma unroll
+		for (int f = 0; f < (int)LT_LEVELS - NM; ++f) {
+			enc[NM + f] = fine[f] & have_fine;
+			asm volatile("" : "+v"(enc[NM + f]));  // waited for here, in front of the next step's loads: behind them the wait would include those
+		}
+		// the next step: where it stands, and the loads it needs (the last step looks at its own position again: no loads)
+		const uint32_t next = k + 1u < nz ? k + 1u : k;
+		uint32_t cz;
+		float wz;
+		n2_locate(lattice_coord(a.lat, 2, z + next), my_scale, wz, cz);
+		const uint32_t moved = cz - my_cz;
+		const uint32_t one = (uint32_t)__ballot(moved == 1u) & on, far = (uint32_t)__ballot(moved > 1u) & on;  // lanes 0..15 speak for the levels
+		uint32_t r0, r1;
+		rows_of(cz + 1u, r0, r1);
+		uint32_t raw[NM][4];
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((one >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+		// Behind them the fine features of the step after the next (they come from far away): the planes can then be waited for
+		// without waiting for these.
+#pragma unroll
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
+		load_fine(min(k + 2u, nz - 1u), ahead);
+		// the network on both tiles (the fence keeps its fragments in LDS: hoisted out of the loop they would take 40 registers)
+		tile_fence();
+		half8 xs[2][3];
+#pragma unroll
+		for (int c = 0; c < 2; ++c) {
+			uint4v t[2];
+#pragma unroll
+			for (int q = 0; q < 4; ++q) {
+				constexpr int first[4] = {0, 1, 4, 5};
+				uint32_t p0 = enc[8 * c + first[q]], p1 = enc[8 * c + first[q] + 2];
+				swap_halves(p0, p1);
+				t[0][q] = p0;
+				t[1][q] = p1;
+			}
+			xs[0][c] = __builtin_bit_cast(half8, t[0]);
+			xs[1][c] = __builtin_bit_cast(half8, t[1]);
+		}
+		const half2v zc = {(hf)pz - (hf)0.5f, (hf)0};
+		const uint32_t zcm = g == 0u ? __builtin_bit_cast(uint32_t, zc) : 0u;
+		xs[0][2] = __builtin_bit_cast(half8, uint4v{xc0, zcm, 0u, 0u});
+		xs[1][2] = __builtin_bit_cast(half8, uint4v{xc1, zcm, 0u, 0u});
+		half8 h[2][4];
+#pragma unroll
+		for (int mt = 0; mt < 2; ++mt) {
+			half8 f[3];
+#pragma unroll
+			for (int c = 0; c < 3; ++c) f[c] = frag(F, SDF_FRAG_W0 + mt * 3 + c, lane);
+			float16v acc[2] = {zero16(), zero16()};
+#pragma unroll
+			for (int c = 0; c < 3; ++c)
+#pragma unroll
+				for (int t = 0; t < 2; ++t) acc[t] = N2_MFMA(f[c], xs[t][c], acc[t]);
+#pragma unroll
+			for (int t = 0; t < 2; ++t) relu_pack(acc[t], h[t][2 * mt], h[t][2 * mt + 1]);
+		}
+		// The second layer, of which only row 0 is wanted: a lane holds half of its sample's hidden values (the other group the
+		// other half).  Dot products on the vector unit take a third of the time of four more MFMAs per tile.
+		float dot[2] = {0.f, 0.f};
+#pragma unroll
+		for (int c = 0; c < 4; ++c) {
+			const uint4v wv = __builtin_bit_cast(uint4v, frag(F, SDF_FRAG_WO + c, lane & 32));  // row 0 of W_out in the order of h
+#pragma unroll
+			for (int t = 0; t < 2; ++t) {
+				const uint4v hv = __builtin_bit_cast(uint4v, h[t][c]);
+#pragma unroll
+				for (int q = 0; q < 4; ++q)
+					dot[t] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, (uint32_t)hv[q]), __builtin_bit_cast(half2v, (uint32_t)wv[q]), dot[t], false);
+			}
+		}
+		// tile 0 belongs to lanes 0..31, tile 1 to the upper ones
+		uint32_t s0 = __float_as_uint(dot[0]), s1 = __float_as_uint(dot[1]);
+		swap_halves(s0, s1);
+		const hf sdf = (hf)(__uint_as_float(s0) + __uint_as_float(s1)) + (hf)a.sdf_bias;
+		if (inside) out[0] = (float)sdf;
+		out += (size_t)rx * a.lat.res[1];
+		// the planes the next step has crossed into
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((one >> l) & 1u) {
+				lo[l] = hi[l];
+				blend(l, raw[l], hi[l]);
+				rise[l] = make_float2(hi[l].x - lo[l].x, hi[l].y - lo[l].y);
+			}
+		if (far) both_planes(far, cz);
+		my_cz = cz;
+		my_wz = wz;
+	}
+}
+
+// the SDF network's fragments as one image (SDF_FRAG_COUNT KiB)
+__global__ void __launch_bounds__(64) lattice_frags_kernel(const hf* __restrict__ sdf_w, uint32_t sdf_in_w, uint32_t enc_w, hf* __restrict__ image) {
+	*reinterpret_cast<half8*>(image + (blockIdx.x * 64u + threadIdx.x) * 8u) = sdf_forward_frag(sdf_w, (int)sdf_in_w, enc_w, (int)blockIdx.x, (int)threadIdx.x);
+}
+
+uint64_t n2_lattice_frag_bytes() { return SDF_FRAG_COUNT * 1024ull; }
+
+// Slabs of at most `chunk` points; d_scratch holds LT_MAX_FINE 4-byte rows of `chunk` points, d_frags the fragment image.
+int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice& lat, uint32_t chunk, void* d_scratch, void* d_frags, float* d_out) {
+	const N2LevelTable& tab = *nets.tab;
+	LatticeArgs a{};
+	a.n_levels = tab.n_levels;
+	a.active_levels = tab.active_levels < tab.n_levels ? tab.active_levels : tab.n_levels;
+	for (uint32_t l = 0; l < LT_LEVELS; ++l) {
+		const bool have = l < tab.n_levels;  // levels the table does not have count as switched off
+		a.scale[l] = have ? tab.scale[l] : 1.f;
+		a.res[l] = have ? tab.resolution[l] : 1u;
+		a.entries[l] = have ? tab.entries[l] : 8u;
+		a.offset[l] = have ? tab.offset[l] : 0u;
+		if (have && tab.mode[l] == N2_LEVEL_HASH) a.hash_mask |= 1u << l;
+	}
+	a.table = nets.table;
+	a.frags = reinterpret_cast<const hf*>(d_frags);
+	a.sdf_bias = nets.sdf_bias;
+	a.lat = lat;
+	a.features = reinterpret_cast<uint32_t*>(d_scratch);
+	a.x_runs = (lat.res[0] + 63u) / 64u;
+	// The walk takes the levels whose cells are larger than a step along z: above that, every step meets two new planes and
+	// there is nothing to keep.  (It is right for any level: a step across several cells fetches both planes.)
+	uint32_t coarse = 0;
+	const float step = lat.inv_res[2] * (lat.extent[2] < 0.f ? -lat.extent[2] : lat.extent[2]);
+	while (coarse < LT_LEVELS && a.scale[coarse] * step < 0.95f) ++coarse;
+	const uint32_t nm = coarse >= 10u ? 10u : coarse >= 8u ? 8u : 6u;
+	a.first_fine = nm;
+	const uint32_t n_fine = tab.n_levels > nm ? tab.n_levels - nm : 0u;
+	static_assert(LT_LEVELS - 6u <= LT_MAX_FINE, "the fine levels' features fit the scratch");
+	lattice_frags_kernel<<<dim3(SDF_FRAG_COUNT), dim3(64), 0, s>>>(reinterpret_cast<const hf*>(nets.sdf_w), nets.sdf_in_w, tab.n_levels * 2u, reinterpret_cast<hf*>(d_frags));
+	N2_LAUNCH_CHECK();
+	const uint32_t rx = lat.res[0], ry = lat.res[1], rz = lat.res[2];
+	// rows per slab: what the scratch holds of the fine levels' features, at least one (the caller has checked chunk >= rx)
+	const uint64_t rows = (uint64_t)LT_MAX_FINE * chunk / (n_fine ? n_fine : 1u) / rx;
+	const uint32_t ny = rows < ry ? (uint32_t)rows : ry, nz = rows < ry ? 1u : (rows / ry < rz ? (uint32_t)(rows / ry) : rz);
+	for (uint32_t z0 = 0; z0 < rz; z0 += nz)
+		for (uint32_t y0 = 0; y0 < ry; y0 += ny) {
+			a.y0 = y0; a.ny = ny < ry - y0 ? ny : ry - y0;
+			a.z0 = z0; a.nz = nz < rz - z0 ? nz : rz - z0;
+			a.out = d_out + ((size_t)z0 * ry + y0) * rx;
+			// planes per wave: 16 where that leaves every SIMD several waves (a wave's start costs as much as two steps), fewer on
+			// small lattices; the slab's planes in equal shares
+			const uint64_t runs = (uint64_t)a.x_runs * a.ny * a.nz;
+			const uint32_t most = runs >= 16u * 4096u ? 16u : runs <= 4u * 4096u ? 4u : (uint32_t)(runs / 4096u), parts = (a.nz + most - 1u) / most;
+			a.walk = (a.nz + parts - 1u) / parts;
+			const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk), blocks = (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
+			if (n_fine) {
+				lattice_fine_kernel<<<dim3(blocks * n_fine), dim3(LT_BLOCK), 0, s>>>(a, blocks);
+				N2_LAUNCH_CHECK();
+			}
+			if (nm == 10u) lattice_walk_kernel<10><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+			else if (nm == 8u) lattice_walk_kernel<8><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+			else lattice_walk_kernel<6><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+			N2_LAUNCH_CHECK();
+		}
+	return N2_OK;
+}

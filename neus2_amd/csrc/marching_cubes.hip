@@ -616,7 +616,9 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_lattice_positions_kernel(McGrid g
 #pragma unroll
 	for (int d = 0; d < 3; ++d) p[d] = ((float)c[d] * (1.f / (float)r[d])) * g.scale[d] + g.offset[d];
 }
-N2_API uint64_t n2_density_on_grid_scratch_bytes(uint32_t chunk) { return m256(12ull * chunk) + m256(32ull * chunk); }
+// positions and the network's output for the fields whose points are written out; the fused kernels keep 44 bytes per point
+// there, and their weight fragments behind it
+N2_API uint64_t n2_density_on_grid_scratch_bytes(uint32_t chunk) { return m256(12ull * chunk) + m256(32ull * chunk) + m256(n2_lattice_frag_bytes()); }
 
 N2_API int n2_density_on_grid(n2_field_t* field, n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3],
                               float* d_density, void* d_scratch, uint64_t scratch_bytes, uint32_t chunk) {
@@ -633,16 +635,14 @@ N2_API int n2_density_on_grid(n2_field_t* field, n2_stream_t stream, const uint3
 	g.rx = res[0]; g.ry = res[1]; g.rz = res[2]; g.thresh = 0.f;
 	// here scale is the aabb's extent (the division by the resolution is part of the position formula)
 	for (int d = 0; d < 3; ++d) { g.scale[d] = aabb_max[d] - aabb_min[d]; g.offset[d] = aabb_min[d]; }
+	int rc = N2_OK;
+	N2Lattice lat;
+	for (int d = 0; d < 3; ++d) { lat.res[d] = res[d]; lat.inv_res[d] = 1.f / (float)res[d]; lat.extent[d] = g.scale[d]; lat.corner[d] = g.offset[d]; }
+	if (n2_field_sdf_row0_lattice(field, stream, lat, chunk, d_scratch, reinterpret_cast<unsigned char*>(d_scratch) + m256(12ull * chunk) + m256(32ull * chunk), d_density, &rc)) return rc;
 	// lattice points arrive x fastest: neighbouring lanes in neighbouring cells
 	n2_grid_set_point_order(n2_field_encoding(field), 1);
-	int rc = N2_OK;
 	for (uint64_t first = 0; first < n && rc == N2_OK; first += chunk) {
 		const uint32_t m = (uint32_t)((n - first < chunk) ? n - first : chunk), m8 = (m + 7) / 8 * 8;
-		// the fused kernel forms the lattice points itself; other fields get them written out
-		N2Lattice lat;
-		for (int d = 0; d < 3; ++d) { lat.res[d] = res[d]; lat.inv_res[d] = 1.f / (float)res[d]; lat.extent[d] = g.scale[d]; lat.corner[d] = g.offset[d]; }
-		lat.first = (uint32_t)first; lat.total = (uint32_t)n;
-		if (n < (1ull << 32) && n2_field_sdf_row0_lattice(field, stream, lat, m8, m, d_density + first, &rc)) continue;
 		mc_lattice_positions_kernel<<<mgrid(m8), dim3(MC_BLOCK), 0, s>>>(g, first, m, m8, positions);
 		// the padded tail of the last chunk (m8 - m points at most 7) is evaluated but not kept
 		rc = n2_field_sdf_row0(field, stream, positions, 3, 1, m8, m, d_density + first, reinterpret_cast<n2_half*>(mlp_out));

@@ -126,13 +126,17 @@ int n2_generate_training_samples_rows(n2_stream_t stream, uint32_t n_rays, uint3
 // NerfNetwork::sdf / density: d_out_soa (16 x n, may be null) and / or d_row0 (fp32 copy of row 0, may be null).
 // sdf_in null: one kernel that gathers sample by sample (points in lattice order, whose table lines stay cached);
 // else a level-major gather into the feature rows 3.. of sdf_in (SoA, n columns) followed by the network kernel.
-// lattice (with d_xyz and sdf_in null): sample i is lattice point first + i, x fastest, at (c / res) * extent + corner.
+int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
+                       float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n = 0xFFFFFFFFu);
+// Row 0 of NerfNetwork::sdf as fp32 on a whole lattice, x fastest: point c at (c / res) * extent + corner (lattice.hip).  The
+// lattice is worked off in slabs of at most `chunk` points (at least one row: chunk >= res[0]); d_scratch holds 44 bytes per
+// point of a slab, d_frags n2_lattice_frag_bytes().
 struct N2Lattice {
-	uint32_t res[3], first, total;  // total = res[0] res[1] res[2]
+	uint32_t res[3];
 	float inv_res[3], extent[3], corner[3];
 };
-int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
-                       float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n = 0xFFFFFFFFu, const N2Lattice* lattice = nullptr);
+uint64_t n2_lattice_frag_bytes();
+int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice& lat, uint32_t chunk, void* d_scratch, void* d_frags, float* d_out);
 
 // n2_composite_loss_indexed that also fills the compacted batch up to max_samples_compacted samples (fill = true): slot j
 // behind the n_in = min(*d_compacted_counter, max_samples_compacted) kept samples holds a copy of slot j % n_in (coordinates,
@@ -223,9 +227,9 @@ int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const fl
 // row 0 of n2_field_sdf (density: of n2_field_density) for the first n_keep <= n samples as fp32 (d_scratch16: [16][n] fp16, used when the fused kernels do not serve the field)
 int n2_field_sdf_row0(n2_field_t* field, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n, uint32_t n_keep,
                       float* d_row0, n2_half* d_scratch16, bool density = false);
-// the same on n points of a lattice, generated inside the kernel; false when the field's fused kernels do not serve it (the
-// caller then writes the positions out and uses n2_field_sdf_row0)
-bool n2_field_sdf_row0_lattice(n2_field_t* field, n2_stream_t stream, const N2Lattice& lattice, uint32_t n, uint32_t n_keep, float* d_row0, int* rc);
+// the same over a whole lattice (n2_fused_lattice_sdf); false when the field's fused kernels do not serve it (the caller then
+// writes the positions out and uses n2_field_sdf_row0)
+bool n2_field_sdf_row0_lattice(n2_field_t* field, n2_stream_t stream, const N2Lattice& lattice, uint32_t chunk, void* d_scratch, void* d_frags, float* d_row0, int* rc);
 
 static inline hipStream_t n2_stream(n2_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 

@@ -67,6 +67,34 @@ def test_empty_lattice_and_errors():
         marching_cubes(torch.zeros((8, 8, 8), device="cuda", dtype=torch.float16), 0.0)
 
 
+# rows that end inside a run of 64 points, slabs of part of a plane (and rows longer than a chunk: positions written out), steps
+# of many cells of the fine levels (their rows are then gathered, not staged), several slabs of several planes, a box that
+# sticks out of the unit cube, a grid of 8 levels with dense ones among those the walk does not keep
+@pytest.mark.parametrize("res,chunk,box,levels", [((70, 9, 5), 1 << 14, (0, 1), 16), ((130, 20, 6), 512, (0.2, 0.9), 16), ((96, 4, 3), 64, (0, 1), 16),
+                                                  ((16, 16, 40), 1 << 14, (0, 1), 16), ((320, 12, 33), 1 << 14, (0.4, 0.5), 16), ((40, 33, 21), 4096, (-0.2, 1.1), 16),
+                                                  ((64, 30, 20), 1 << 14, (0, 1), 8)])
+def test_lattice_equals_the_same_points_queried(res, chunk, box, levels):
+    """density_on_grid (rows of lattice points walked along z) against NerfNetwork::sdf on the same positions."""
+    from neus2_amd.mesh import density_on_grid
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork(n_levels=levels)
+    gen = torch.Generator(device="cuda").manual_seed(res[0])
+    o = net.param_offsets()
+    p = torch.randn(o[4], device="cuda", generator=gen) * 0.1
+    net.set_params(p.half(), None)
+    net.reserve(max(1 << 14, (res[0] * res[1] * res[2] + 7) // 8 * 8))
+    lo, hi = (box[0], box[0] + 0.01, box[0]), (box[1], box[1], box[1] - 0.01)
+    d = density_on_grid(net._h, res, lo, hi, chunk=chunk)
+    z, y, x = np.meshgrid(*(np.arange(r, dtype=np.float32) for r in reversed(res)), indexing="ij")
+    ext = np.asarray(hi, np.float32) - np.asarray(lo, np.float32)
+    pos = np.stack([(c * np.float32(np.float32(1.0) / np.float32(r))) * e + np.float32(b) for c, r, e, b in zip((x, y, z), res, ext, lo)]).reshape(3, -1)
+    n = pos.shape[1]
+    padded = np.full((3, (n + 7) // 8 * 8), 0.5, np.float32)
+    padded[:, :n] = pos
+    want = host(net.sdf(dev(padded)))[0, :n].reshape(res[2], res[1], res[0])
+    assert_close(host(d), want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
+
+
 def test_sdf_lattice_and_mesh_of_the_initial_sphere(oracle, tmp_path):
     """get_density_on_grid + marching cubes on the geometric-init network: the zero level set of its SDF is a sphere of
     radius ~0.1 around the cube centre (sdf ~ |x - 0.5| - 0.1)."""
