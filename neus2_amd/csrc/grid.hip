@@ -17,6 +17,7 @@
 
 #include <cmath>
 #include <new>
+#include <type_traits>
 
 struct n2_grid {
 	N2LevelTable tab;
@@ -470,6 +471,8 @@ struct N2BucketPlan {
 	// bucket-major, then group) and the number of split buckets in the levels below
 	uint32_t part_begin[N2_MAX_LEVELS];
 	uint32_t split_begin[N2_MAX_LEVELS + 1];
+	// log2 of the lanes that take one tile's run
+	uint8_t run_lanes[N2_MAX_LEVELS];
 };
 
 template <uint32_t MODE, bool FIRST, bool SECOND, bool WANT_OUT, bool CLAMP_X>
@@ -718,11 +721,7 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 // fp16 values, i.e. multiples of 2^-24 below 2^16, so value * 2^32 is an exact integer below 2^48 and the
 // sum of a whole bucket stays far inside 64 bits.  The accumulation is exact and independent of order.
 constexpr uint32_t RED_BLOCK = 1024;              // 16 waves; two workgroups share a CU
-constexpr uint32_t RED_ITEMS = 2;                 // items a wave has in flight per fetch
-constexpr uint32_t ITEM_SHIFT = 7;                // a run is cut into items of 128 records
-constexpr uint32_t ITEM_RECORDS = 1u << ITEM_SHIFT;
-constexpr uint32_t ITEM_LOADS = ITEM_RECORDS / 64;  // loads per lane and item
-constexpr uint32_t ITEM_CAP = 2048;               // items listed in LDS at a time
+constexpr uint32_t FEW_TILES = 32;                // batches of at most this many tiles: see grid_reduce_kernel
 constexpr float FIX_SCALE = 4294967296.0f;        // 2^32
 
 // x * 2^32 as a two's complement 64-bit integer, for |x| < 2^31 with at most 24 significant bits (any fp16 value):
@@ -735,178 +734,115 @@ __device__ __forceinline__ unsigned long long to_fixed(float x) {
 }
 __device__ __forceinline__ float from_fixed(unsigned long long q) { return (float)((double)(long long)q * (1.0 / 4294967296.0)); }
 
-// Pair levels: an item is 16 pair records and a wave's load covers four items, one per 16 lanes (a bucket's run in a tile
-// is about 32 pair records: whole-wave items would leave half the lanes idle).
-constexpr uint32_t PITEM_SHIFT = 4;
-constexpr uint32_t PITEM_RECORDS = 1u << PITEM_SHIFT;
-constexpr uint32_t PITEM_PER_LOAD = 64 / PITEM_RECORDS;
-constexpr uint32_t P_LOADS = 4;  // loads per lane in flight per register set
+// which (level, bucket, group of tiles) is this workgroup?  (Lane l asks about level l: sixteen scalar loads one after the other
+// were a microsecond of every workgroup.)
+struct N2ReduceItem {
+	uint32_t level, bucket, group, groups, entries;  // entries per bucket: the level's own size (split buckets always have BKT_ENTRIES)
+	bool pair;
+};
+__device__ __forceinline__ N2ReduceItem n2_reduce_item(const N2LevelTable& tab, const N2BucketPlan& plan) {
+	const uint32_t lane = threadIdx.x & 63u;
+	N2ReduceItem it;
+	it.level = __builtin_amdgcn_readfirstlane(__popcll(__ballot(lane < N2_MAX_LEVELS && blockIdx.x >= plan.wg_begin[min(lane, N2_MAX_LEVELS - 1u) + 1u])));
+	const uint32_t local = blockIdx.x - plan.wg_begin[it.level];
+	it.groups = plan.groups[it.level];
+	it.bucket = local / it.groups;
+	it.group = local - it.bucket * it.groups;
+	it.pair = (tab.pair_levels >> it.level) & 1u;
+	it.entries = it.pair ? BKT_ENTRIES : 1u << tab.bucket_shift[it.level];
+	// A tile's runs for neighbouring buckets meet inside a 128-byte line, which both buckets' workgroups fetch.  Workgroup
+	// ids are dealt round-robin over the XCDs: XCD x takes the x-th eighth of the level's buckets, in order, so that both
+	// fetches of such a line go through the same L2 at about the same time.
+	const uint32_t nb = plan.n_buckets[it.level];
+	if (it.groups == 1 && nb % N_XCD == 0) it.bucket = (blockIdx.x % N_XCD) * (nb / N_XCD) + local / N_XCD;
+	return it;
+}
 
-// Every thread owns the bucket's run of one tile.  The runs are cut into items, the items of all runs are numbered
-// consecutively (block scan of the item counts) and listed in LDS (first record, record count), ITEM_CAP at a time:
-// a wave then finds an item's records with one LDS read instead of searching the runs' prefix sums, whose chain of
-// dependent LDS reads was most of this kernel's time.
-template <bool PAIR>
-__device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const uint32_t level, const uint32_t bucket, const uint32_t group,
-                                                 const uint32_t G, const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
-                                                 const uint16_t* __restrict__ offsets, unsigned long long* acc, uint32_t* item_src,
-                                                 uint8_t* item_n, uint32_t* wave_tot, const uint32_t bucket_entries) {
-	constexpr uint32_t SHIFT = PAIR ? PITEM_SHIFT : ITEM_SHIFT, RECS = 1u << SHIFT;
-	constexpr uint32_t TILE_RECS = PAIR ? BIN_RECORDS / 2 : BIN_RECORDS;  // records in a tile's slot of the value array
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	const uint32_t my_tiles = (tiles > group) ? (tiles - group + G - 1) / G : 0;  // tiles group, group + G, ...
-	const size_t level_tile0 = (size_t)level * tiles;
-	const uint32_t* base_val = rec_vals + level_tile0 * BIN_RECORDS;
-	const uint16_t* base_key = rec_keys + level_tile0 * BIN_RECORDS;
-	for (uint32_t c0 = 0; c0 < my_tiles || c0 == 0; c0 += RED_BLOCK) {
-		// this thread's run (the load is in flight while the accumulators are cleared)
-		uint32_t src = 0, len = 0;
-		const uint32_t t = c0 + threadIdx.x;
-		if (t < my_tiles) {
-			const size_t tile = level_tile0 + group + (size_t)t * G;
-			const uint16_t* off = offsets + tile * (BKT_MAX + 1) + bucket;
-			const uint32_t begin = off[0], end = off[1];
-			src = (uint32_t)((tile - level_tile0) * TILE_RECS) + begin;
-			len = end - begin;
-		}
-		if (c0 == 0) {
-			for (uint32_t e = threadIdx.x; e < bucket_entries; e += RED_BLOCK) { acc[e] = 0ull; acc[BKT_ENTRIES + e] = 0ull; }
-		}
-		const uint32_t cnt = (len + RECS - 1u) >> SHIFT;
-		uint32_t incl = cnt;
+// A bucket's runs: 2^run_lanes lanes take a tile's run (as many as hold its records in one step, on average), the workgroup's
+// groups of lanes take the tiles in turn.  A lane has FLIGHT records being added while the next FLIGHT are on their way.
+// (Cutting all runs into items listed in LDS, for an even load, costs a scan, a list and three more barriers in front of the
+// first record: 27 us against 17 for 5e3 points, where a workgroup's time is the chain of round trips, 33 against 25 for
+// 6.5e4, 39 against 33 for 1.2e5, 63 against 62 for 2^18.)
+template <bool PAIR, uint32_t FLIGHT>
+__device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2ReduceItem& it, const uint32_t run_lanes,
+                                                   const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
+                                                   const uint16_t* __restrict__ offsets, unsigned long long* acc) {
+	const uint32_t lanes = 1u << run_lanes, r = threadIdx.x & (lanes - 1u), group = threadIdx.x >> run_lanes, groups = RED_BLOCK >> run_lanes;
+	const size_t level_tile0 = (size_t)it.level * tiles;
+	const uint16_t* off = offsets + level_tile0 * (BKT_MAX + 1) + it.bucket;
+	const uint32_t step = groups * it.groups;  // (a split bucket's workgroup takes the tiles it.group, it.group + it.groups, ...)
+	// where the next step's records are; the bounds of the run behind it are on their way
+	uint32_t tile = group * it.groups + it.group, i = 0, end = 0, next_i = 0, next_end = 0;
+	if (tile < tiles) { i = off[(size_t)tile * (BKT_MAX + 1)] + r; end = off[(size_t)tile * (BKT_MAX + 1) + 1]; }
+	if (tile + step < tiles) { next_i = off[(size_t)(tile + step) * (BKT_MAX + 1)] + r; next_end = off[(size_t)(tile + step) * (BKT_MAX + 1) + 1]; }
+	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
+	struct Step {
+		value v[FLIGHT];
+		uint32_t key[FLIGHT], n;  // n: records of this lane that count
+	};
+	auto load = [&](Step& q) {
+		// (lanes without a record read the level's first one: every load is issued, so the compiler can wait for one step only)
+		const uint32_t left = i < end ? (end - i + lanes - 1u) >> run_lanes : 0u;
+		q.n = left < FLIGHT ? left : FLIGHT;
+		const size_t slot = (level_tile0 + (tile < tiles ? tile : 0u)) * BIN_RECORDS;
 #pragma unroll
-		for (int o = 1; o < 64; o <<= 1) {
-			const uint32_t u = __shfl_up(incl, o);
-			if ((int)lane >= o) incl += u;
+		for (uint32_t u = 0; u < FLIGHT; ++u) {
+			const uint32_t at = u < q.n ? i + u * lanes : 0u;
+			q.key[u] = rec_keys[slot + at];
+			if constexpr (PAIR) q.v[u] = reinterpret_cast<const uint2*>(rec_vals + slot)[at];
+			else q.v[u] = rec_vals[slot + at];
 		}
-		__syncthreads();  // the previous chunk's items are done with wave_tot and the item list
-		if (lane == 63) wave_tot[wave] = incl;
-		__syncthreads();
-		uint32_t first = incl - cnt, n_items = 0;  // number of this thread's first item; items of the chunk
-		for (uint32_t w = 0; w < RED_BLOCK / 64; ++w) {
-			const uint32_t tot = wave_tot[w];
-			if (w < wave) first += tot;
-			n_items += tot;
+		i += FLIGHT * lanes;
+		if (i - r >= end) {  // (the same for all lanes of the run) on to the next run
+			tile += step;
+			i = next_i;
+			end = next_end;
+			const uint32_t t = tile + step;
+			next_i = r;
+			next_end = 0;
+			if (t < tiles) { next_i = off[(size_t)t * (BKT_MAX + 1)] + r; next_end = off[(size_t)t * (BKT_MAX + 1) + 1]; }
 		}
-		for (uint32_t w0 = 0; w0 < n_items; w0 += ITEM_CAP) {
-			if (w0 > 0) __syncthreads();  // the previous window has been read
-			// list this thread's items that fall into the window [w0, w0 + ITEM_CAP)
-			for (uint32_t i = (first < w0) ? w0 - first : 0u; i < cnt && first + i < w0 + ITEM_CAP; ++i) {
-				const uint32_t rest = len - (i << SHIFT);
-				item_src[first + i - w0] = src + (i << SHIFT);
-				item_n[first + i - w0] = (uint8_t)((rest < RECS ? rest : RECS) - 1u);
-			}
-			__syncthreads();
-			const uint32_t n_win = (n_items - w0 < ITEM_CAP) ? n_items - w0 : ITEM_CAP;
+	};
+	auto add = [&](const Step& q) {
+#pragma unroll
+		for (uint32_t u = 0; u < FLIGHT; ++u) {
+			if (u >= q.n) break;
 			if constexpr (PAIR) {
-				const uint2* base_val2 = reinterpret_cast<const uint2*>(base_val);
-				const uint32_t r = lane & (PITEM_RECORDS - 1u), sub = lane >> PITEM_SHIFT;
-				// Lanes past the end of an item read the level's first record instead (and ignore it): with every load issued
-				// unconditionally the compiler can count them, and waits for the CURRENT set only while the next is in flight.
-				auto fetch = [&](uint32_t i0, uint2 (&val)[P_LOADS], uint32_t (&key)[P_LOADS], uint32_t& okmask) {
-					okmask = 0;
-#pragma unroll
-					for (uint32_t h = 0; h < P_LOADS; ++h) {
-						const uint32_t it = i0 + PITEM_PER_LOAD * h + sub;
-						uint32_t s0 = 0, n = 0;
-						if (it < n_win) { s0 = item_src[it]; n = (uint32_t)item_n[it] + 1u; }
-						const bool ok = r < n;
-						okmask |= (ok ? 1u : 0u) << h;
-						const uint32_t at = ok ? s0 + r : 0u;
-						val[h] = base_val2[at];
-						key[h] = base_key[at + (at & ~(TILE_RECS - 1u))];  // a tile's key slot is twice as long as its pair records
-					}
-				};
-				auto accumulate = [&](const uint2 (&val)[P_LOADS], const uint32_t (&key)[P_LOADS], uint32_t okmask) {
-#pragma unroll
-					for (uint32_t q = 0; q < P_LOADS; ++q) {
-						if (okmask & (1u << q)) {
-							const uint32_t a1 = key[q] & (BKT_ENTRIES - 1u);
-							const uint32_t a2 = a1 ^ ((2u << (key[q] >> BKT_SHIFT)) - 1u);  // the x + 1 corner: x ^ (x + 1) = 2^(t+1) - 1
-							const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&val[q].x));
-							const float2 g = __half22float2(*reinterpret_cast<const __half2*>(&val[q].y));
-							atomicAdd(&acc[a1], to_fixed(f.x));  // LDS integer atomics
-							atomicAdd(&acc[BKT_ENTRIES + a1], to_fixed(f.y));
-							atomicAdd(&acc[a2], to_fixed(g.x));
-							atomicAdd(&acc[BKT_ENTRIES + a2], to_fixed(g.y));
-						}
-					}
-				};
-				constexpr uint32_t PER_WAVE = PITEM_PER_LOAD * P_LOADS, STRIDE = (RED_BLOCK / 64) * PER_WAVE;
-				uint2 va[P_LOADS], vb[P_LOADS];
-				uint32_t ka[P_LOADS], kb[P_LOADS], ok_a = 0, ok_b = 0;
-				uint32_t i0 = wave * PER_WAVE;
-				if (i0 < n_win) {
-					fetch(i0, va, ka, ok_a);
-					for (;;) {
-						fetch(i0 + STRIDE, vb, kb, ok_b);
-						accumulate(va, ka, ok_a);
-						i0 += STRIDE;
-						if (i0 >= n_win) break;
-						fetch(i0 + STRIDE, va, ka, ok_a);
-						accumulate(vb, kb, ok_b);
-						i0 += STRIDE;
-						if (i0 >= n_win) break;
-					}
-				}
+				const uint32_t a1 = q.key[u] & (BKT_ENTRIES - 1u), a2 = a1 ^ ((2u << (q.key[u] >> BKT_SHIFT)) - 1u);  // x ^ (x + 1) = 2^(t+1) - 1
+				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&q.v[u].x)), g = __half22float2(*reinterpret_cast<const __half2*>(&q.v[u].y));
+				atomicAdd(&acc[a1], to_fixed(f.x));
+				atomicAdd(&acc[BKT_ENTRIES + a1], to_fixed(f.y));
+				atomicAdd(&acc[a2], to_fixed(g.x));
+				atomicAdd(&acc[BKT_ENTRIES + a2], to_fixed(g.y));
 			} else {
-				// a wave takes RED_ITEMS items at a time
-				auto fetch = [&](uint32_t i0, uint2 (&rec)[ITEM_LOADS * RED_ITEMS], uint32_t& okmask) {
-					okmask = 0;
-#pragma unroll
-					for (uint32_t j = 0; j < RED_ITEMS; ++j) {
-						const uint32_t it = i0 + j;
-						uint32_t s0 = 0, n = 0;
-						if (it < n_win) { s0 = item_src[it]; n = (uint32_t)item_n[it] + 1u; }
-#pragma unroll
-						for (uint32_t h = 0; h < ITEM_LOADS; ++h) {
-							const uint32_t r = h * 64 + lane;
-							const bool ok = r < n;
-							okmask |= (ok ? 1u : 0u) << (ITEM_LOADS * j + h);
-							// lanes past the end of the run read the level's first record instead (and ignore it): with every
-							// load issued unconditionally the compiler can count them, and waits for the CURRENT items only
-							// while the next ones are in flight
-							const size_t at = ok ? (size_t)s0 + r : 0;
-							rec[ITEM_LOADS * j + h] = make_uint2(base_key[at], base_val[at]);
-						}
-					}
-				};
-				constexpr uint32_t STRIDE = (RED_BLOCK / 64) * RED_ITEMS;
-				auto accumulate = [&](const uint2 (&rec)[ITEM_LOADS * RED_ITEMS], uint32_t okmask) {
-#pragma unroll
-					for (uint32_t q = 0; q < ITEM_LOADS * RED_ITEMS; ++q) {
-						if (okmask & (1u << q)) {
-							const __half2 hh = *reinterpret_cast<const __half2*>(&rec[q].y);
-							const float2 f = __half22float2(hh);
-							atomicAdd(&acc[rec[q].x], to_fixed(f.x));  // LDS integer atomics
-							atomicAdd(&acc[BKT_ENTRIES + rec[q].x], to_fixed(f.y));
-						}
-					}
-				};
-				// Two register sets take turns: while one is accumulated the loads of the other are in flight.  Every fetch
-				// issues the same number of loads (items past the end read the first record and are ignored) and no set is
-				// ever copied, so each wait covers exactly the set that is about to be used.
-				uint2 ra[ITEM_LOADS * RED_ITEMS], rb[ITEM_LOADS * RED_ITEMS];
-				uint32_t ok_a = 0, ok_b = 0;
-				uint32_t i0 = wave * RED_ITEMS;
-				if (i0 < n_win) {
-					fetch(i0, ra, ok_a);
-					for (;;) {
-						fetch(i0 + STRIDE, rb, ok_b);
-						accumulate(ra, ok_a);
-						i0 += STRIDE;
-						if (i0 >= n_win) break;
-						fetch(i0 + STRIDE, ra, ok_a);
-						accumulate(rb, ok_b);
-						i0 += STRIDE;
-						if (i0 >= n_win) break;
-					}
-				}
+				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&q.v[u]));
+				atomicAdd(&acc[q.key[u]], to_fixed(f.x));
+				atomicAdd(&acc[BKT_ENTRIES + q.key[u]], to_fixed(f.y));
 			}
 		}
+	};
+	Step qa, qb;
+	ulonglong2* a2 = reinterpret_cast<ulonglong2*>(acc);
+	for (uint32_t e = threadIdx.x; e < it.entries / 2; e += RED_BLOCK) {
+		a2[e] = make_ulonglong2(0ull, 0ull);
+		a2[BKT_ENTRIES / 2 + e] = make_ulonglong2(0ull, 0ull);
+	}
+	load(qa);
+	__syncthreads();
+	while (true) {
+		const bool last_b = tile >= tiles;
+		load(qb);
+		add(qa);
+		if (last_b) break;
+		const bool last_a = tile >= tiles;
+		load(qa);
+		add(qb);
+		if (last_a) break;
 	}
 }
 
+// FLIGHT: 2 for batches of few tiles, whose runs rarely hold more (the loads of absent records cost 2 us at 5e3 points)
+template <uint32_t FLIGHT>
 __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                    const uint16_t* __restrict__ offsets,
@@ -914,49 +850,40 @@ __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable 
                                                                    float2* __restrict__ partials) {
 	// one plane per feature: lanes of a wave's atomic then spread over all bank pairs (entry-major pairs of features would
 	// leave every other pair unused)
-	__shared__ unsigned long long acc[2 * BKT_ENTRIES];
-	__shared__ uint32_t item_src[ITEM_CAP];  // index of the item's first record in the level's records
-	__shared__ uint8_t item_n[ITEM_CAP];     // its record count - 1
-	__shared__ uint32_t wave_tot[RED_BLOCK / 64];
-	// which (level, bucket, group) is this workgroup?
-	uint32_t level = 0;
-	while (blockIdx.x >= plan.wg_begin[level + 1]) ++level;
-	const uint32_t local = blockIdx.x - plan.wg_begin[level];
-	const uint32_t G = plan.groups[level];
-	uint32_t bucket = local / G;
-	const uint32_t group = local - bucket * G;
-	// A tile's runs for neighbouring buckets meet inside a 128-byte line, which both buckets' workgroups fetch.  Workgroup
-	// ids are dealt round-robin over the XCDs: XCD x takes the x-th eighth of the level's buckets, in order, so that both
-	// fetches of such a line go through the same L2 at about the same time.
-	const uint32_t nb = plan.n_buckets[level];
-	// entries per bucket: the level's own size (split buckets always have BKT_ENTRIES)
-	const uint32_t bucket_entries = ((tab.pair_levels >> level) & 1u) ? BKT_ENTRIES : 1u << tab.bucket_shift[level];
-	if (G == 1 && nb % N_XCD == 0) bucket = (blockIdx.x % N_XCD) * (nb / N_XCD) + local / N_XCD;
-	if ((tab.pair_levels >> level) & 1u)
-		grid_reduce_runs<true>(tiles, level, bucket, group, G, rec_vals, rec_keys, offsets, acc, item_src, item_n, wave_tot, BKT_ENTRIES);
-	else
-		grid_reduce_runs<false>(tiles, level, bucket, group, G, rec_vals, rec_keys, offsets, acc, item_src, item_n, wave_tot, bucket_entries);
+	__shared__ __align__(16) unsigned long long acc[2 * BKT_ENTRIES];
+	const N2ReduceItem it = n2_reduce_item(tab, plan);
+	const uint32_t run_lanes = plan.run_lanes[it.level];
+	if (it.pair) grid_reduce_runs<true, FLIGHT>(tiles, it, run_lanes, rec_vals, rec_keys, offsets, acc);
+	else grid_reduce_runs<false, FLIGHT>(tiles, it, run_lanes, rec_vals, rec_keys, offsets, acc);
 	__syncthreads();
-	const uint32_t entries = tab.entries[level];
-	__half2* Gd = grads + tab.offset[level];
-	if (G > 1) {
+	if (it.groups > 1) {
 		// Several workgroups hold parts of this bucket's sums (coarse levels of large batches).  Each leaves its image as
 		// fp32 and grid_combine_kernel adds the G images up in the order of the groups: every entry is the same sum of the
 		// same terms in the same order however the workgroups were scheduled (the images themselves are exact integer sums).
-		float2* mine = partials + ((size_t)plan.part_begin[level] + (size_t)bucket * G + group) * BKT_ENTRIES;
+		float2* mine = partials + ((size_t)plan.part_begin[it.level] + (size_t)it.bucket * it.groups + it.group) * BKT_ENTRIES;
 		for (uint32_t e = threadIdx.x; e < BKT_ENTRIES; e += RED_BLOCK) mine[e] = make_float2(from_fixed(acc[e]), from_fixed(acc[BKT_ENTRIES + e]));
 		return;
 	}
-	for (uint32_t e = threadIdx.x; e < bucket_entries; e += RED_BLOCK) {
-		const uint32_t idx = bucket * bucket_entries + e;
+	// four entries (16 bytes) per lane: a level's table is whole multiples of eight entries and a bucket of 32
+	const uint32_t entries = tab.entries[it.level];
+	__half2* Gd = grads + tab.offset[it.level];
+	for (uint32_t e = threadIdx.x * 4u; e < it.entries; e += RED_BLOCK * 4u) {
+		const uint32_t idx = it.bucket * it.entries + e;
 		if (idx >= entries) break;
-		const float ax = from_fixed(acc[e]), ay = from_fixed(acc[BKT_ENTRIES + e]);
-		if (accumulate) {
-			const float2 old = __half22float2(Gd[idx]);
-			Gd[idx] = __floats2half2_rn(old.x + ax, old.y + ay);
-		} else {
-			Gd[idx] = __floats2half2_rn(ax, ay);
+		typedef uint32_t wide __attribute__((ext_vector_type(4)));
+		wide* at = reinterpret_cast<wide*>(Gd + idx);
+		const wide old = accumulate ? *at : wide(0u);
+		wide out;
+#pragma unroll
+		for (uint32_t q = 0; q < 4; ++q) {
+			const uint32_t o = old[q];
+			float2 f = __half22float2(*reinterpret_cast<const __half2*>(&o));
+			f.x += from_fixed(acc[e + q]);
+			f.y += from_fixed(acc[BKT_ENTRIES + e + q]);
+			const __half2 h = __floats2half2_rn(f.x, f.y);
+			out[q] = *reinterpret_cast<const uint32_t*>(&h);
 		}
+		*at = out;
 	}
 }
 
@@ -1282,18 +1209,22 @@ static uint64_t bucket_ws_bytes(const n2_grid_t* grid, uint32_t max_points) { re
 static bool uses_bucketed(const n2_grid_t* grid, uint32_t n_points) {
 	return grid->grads != nullptr && grid->ws != nullptr && n_points <= grid->ws_max_points && n_points >= 1;
 }
-// workgroups per bucket of a level: aim at <= ~64k records per reduce workgroup (a level holds 8 records per point)
 // Entries per bucket of a level (log2).  Levels that sort pair records keep 4096-entry buckets (a pair's second entry is
 // encoded against that size); the others take the largest size (a power of two, at most 4096 entries and at most BKT_MAX
-// buckets) under which no bucket needs more than one workgroup: small dense levels of large batches get many small buckets
-// instead of few that are split.  When even the smallest size does not get there, the buckets stay large and are split.
+// buckets) under which a bucket holds at most `target` of the level's 8 records per point, or the smallest there is: small
+// dense levels get many small buckets instead of few that outlast the others.  When even the smallest buckets hold more than
+// 65536, they stay large and are split (bucket_groups).
 static uint32_t bucket_shift_for(const n2_grid_t* grid, uint32_t level, uint32_t n_points) {
 	if ((grid->tab.pair_levels >> level) & 1u) return BKT_SHIFT;
 	const uint32_t entries = grid->tab.entries[level];
+	// (8192 and 32768 records: the same within 2 %, 65536: 49 us against 36 at 1.2e5 points, where a dense level's few workgroups
+	// outlast the others)
+	constexpr uint64_t target = 16384u;
 	for (uint32_t shift = BKT_SHIFT; shift >= BKT_MIN_SHIFT; --shift) {
-		const uint32_t nb = (entries + (1u << shift) - 1u) >> shift;
+		const uint32_t nb = (entries + (1u << shift) - 1u) >> shift, finer = (entries + (1u << (shift - 1u)) - 1u) >> (shift - 1u);
 		if (nb > BKT_MAX) break;
-		if ((uint64_t)n_points * 8 / nb <= 65536) return shift;  // (32768: scatter + 1.3 us on the training step, 16384: + 4.7)
+		const uint64_t records = (uint64_t)n_points * 8 / nb;
+		if (records <= target || (records <= 65536u && (shift == BKT_MIN_SHIFT || finer > BKT_MAX))) return shift;
 	}
 	return BKT_SHIFT;
 }
@@ -1361,6 +1292,7 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	N2BucketPlan plan;
 	uint32_t wg = 0, images = 0, split = 0;
 	N2LevelTable tab = grid->tab;  // with this launch's bucket sizes
+	const bool few = tiles <= FEW_TILES;
 	for (uint32_t l = 0; l < L; ++l) {
 		tab.bucket_shift[l] = (uint8_t)bucket_shift_for(grid, l, n_points);
 		const uint32_t nb = level_buckets(grid, l, n_points);
@@ -1368,13 +1300,20 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 		plan.wg_begin[l] = wg;
 		plan.n_buckets[l] = nb;
 		plan.groups[l] = groups;
+		{
+			// lanes per run: with their records in flight, about the records a tile's run holds on average
+			const uint32_t per_run = (((tab.pair_levels >> l) & 1u) ? BIN_RECORDS / 2 : BIN_RECORDS) / nb;
+			uint32_t lanes = 4;
+			while (lanes < 10 && ((few ? 2u : 4u) << lanes) < per_run) ++lanes;
+			plan.run_lanes[l] = (uint8_t)lanes;
+		}
 		plan.part_begin[l] = images;
 		plan.split_begin[l] = split;
 		wg += nb * groups;
 		if (groups > 1) { images += nb * groups; split += nb; }
 	}
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.wg_begin[l] = wg;
-	for (uint32_t l = L; l < N2_MAX_LEVELS; ++l) { plan.n_buckets[l] = 0; plan.groups[l] = 1; plan.part_begin[l] = images; }
+	for (uint32_t l = L; l < N2_MAX_LEVELS; ++l) { plan.n_buckets[l] = 0; plan.groups[l] = 1; plan.part_begin[l] = images; plan.run_lanes[l] = 0; }
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.split_begin[l] = split;
 #define LAUNCH(F, S, O) grid_bin_kernel<F, S, O><<<gd, bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
                                                                    grid->params, dL_ddLdy, rec_vals, rec_keys, offsets, index, n_cols)
@@ -1385,7 +1324,9 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	else LAUNCH(true, false, false);
 #undef LAUNCH
 	N2_LAUNCH_CHECK();
-	grid_reduce_kernel<<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials);
+#define LAUNCH(F) grid_reduce_kernel<F><<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials)
+	if (few) LAUNCH(2); else LAUNCH(4);
+#undef LAUNCH
 	N2_LAUNCH_CHECK();
 	if (split > 0) {
 		N2ImageCombine cmb{};

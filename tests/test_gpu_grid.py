@@ -294,6 +294,28 @@ def test_backward_fused_equals_first_plus_second_order(setup, n):
     assert none is None and rel_l2(host(d_grads), 2 * ref) < 2e-2
 
 
+@pytest.mark.parametrize("n", [1, 1025, (1 << 15) + 1, 70001])  # one record, a second tile, one tile past the few-tiles kernel, tiles taken in several turns
+def test_sorted_scatter_batch_sizes(oracle, n):
+    """The reduce kernel's two forms and its walk over tiles, overwriting and accumulating."""
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
+    og = oracle.Grid(CFG["n_levels"], CFG["log2_hashmap_size"], CFG["base_resolution"], CFG["per_level_scale"])
+    gg = GridEncoding(**CFG)
+    rng = np.random.default_rng(n)
+    dp = dev(q16(rng.uniform(-1, 1, og.n_params)), torch.float16)
+    dg = torch.full_like(dp, 9.0)
+    gg.set_params(dp, dg)
+    assert gg.reserve_scatter_workspace(n)
+    xyz = rng.random((3, n), dtype=np.float32)
+    dy = q16(rng.standard_normal((32, n)))
+    ref, _ = og.backward(host(dp), xyz, dy, want_dx=False)
+    for mode, times in ((GRAD_OVERWRITE, 1), (GRAD_ACCUMULATE, 2)):
+        gg.backward(None, dev(xyz), dev(dy, torch.float16), mode=mode)
+        got = host(dg)
+        for l in range(16):
+            a, b = int(og.offset[l]) * 2, int(og.offset[l + 1]) * 2
+            assert rel_l2(got[a:b], times * ref[a:b]) < RTOL, (mode, l)
+
+
 @pytest.mark.parametrize("kind", ["uniform", "clustered", "rays"])
 def test_sorted_scatter_path(oracle, kind):
     """With a scatter workspace, batches go through the run-length kernel (coarsest levels) and the
