@@ -76,8 +76,8 @@ int n2_grid_level_table(const n2_grid_t* grid, float* scale, uint32_t* resolutio
                         uint32_t* offset);
 
 /* Tuning knob without a counterpart in the reference: the relative cost of one tile of points on each level
- * (n_levels values > 0).  The gather kernels split the levels over the GPU's 8 XCDs in proportion to it so
- * that each XCD's L2 holds only the tables of its own levels.  Defaults: 1 for hashed levels, 0.6 for dense ones.
+ * (n_levels values > 0).  n2_grid_forward then splits the levels over the GPU's 8 XCDs in proportion to it, so
+ * that each XCD's L2 holds only the tables of its own levels.  Without it every XCD gets a fine and a coarse level.
  * Results do not depend on it. */
 int n2_grid_set_level_costs(n2_grid_t* grid, const float* costs);
 

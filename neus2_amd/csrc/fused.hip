@@ -138,6 +138,7 @@ constexpr uint32_t BWD_RGB_FRAGS = FragMap<3, 2>::SEL, BWD_SDF_FRAGS = FragMap<3
 static_assert(FF_COUNT * 1024 == N2_FUSED_FRAG_FORWARD && BWD_RGB_FRAGS * 1024 == N2_FUSED_FRAG_RGB && BWD_SDF_FRAGS * 1024 == N2_FUSED_FRAG_SDF,
               "the image's parts as n2_common.h sizes them");
 constexpr uint32_t FG_BLOCK = 256;  // threads of a gather workgroup (128: the gather 1.8 us shorter, the step 5 us longer; 512: +2 / +5; 1024: +11 / +11)
+constexpr uint32_t FG_PAIRS = FG_BLOCK / 2;
 constexpr uint32_t FRAG_BLOCKS = ((FF_COUNT + BWD_RGB_FRAGS + BWD_SDF_FRAGS) * 64 + FG_BLOCK - 1) / FG_BLOCK;
 __device__ __forceinline__ void write_frag_image(const FusedArgs& a, uint32_t block) {
 	const uint32_t idx = block * FG_BLOCK + threadIdx.x;
@@ -286,19 +287,17 @@ __device__ __forceinline__ void sh4(float x, float y, float z, float* o) {
 // level-major gather: features into the SDF net's input rows, slopes as fp16
 // ----------------------------------------------------------------------------
 
-// FULL: positions from the [N][7] coordinates, slopes and the coordinate rows are written; else positions with the
-// strides (ps, ds) and the feature rows only (inference on points in no particular order).
-// one (sample, level) item: the sample's coordinates are row `src` of the input, what it writes goes to column i
-template <bool FULL>
+// Full field: one (sample, level) item, features and slopes; the sample's coordinates are row `src` of the input (the [N][7]
+// coordinates, or three rows of positions), what it writes goes to column i.
 __device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t src) {
 	const uint32_t N = a.N;
 	// (full field: the positions from the coordinate rows, or from three rows of their own when the caller has them: a wave
 	// then reads two lines per coordinate instead of fourteen)
-	const bool rows = FULL && a.pos == nullptr;
+	const bool rows = a.pos == nullptr;
 	const float* q = rows ? a.coords + (size_t)src * 7 : a.pos + (size_t)src * a.ps;
 	const size_t qs = rows ? 1 : a.ds;
 	const float p[3] = {q[0], q[qs], q[2 * qs]};
-	if (FULL && level == 0) {
+	if (level == 0) {
 #pragma unroll
 		for (int d = 0; d < 3; ++d) {
 			a.sdf_in[(size_t)d * N + i] = (hf)p[d] - (hf)0.5f;
@@ -320,14 +319,47 @@ __device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, 
 		else corner_offsets<0>(L, c, boff);
 #pragma unroll
 		for (int k = 0; k < 8; ++k) it.raw[k] = *reinterpret_cast<const uint32_t*>(base + boff[k]);
-		item_finish<FULL>(it, feat, J);
+		item_finish<true>(it, feat, J);
 	}
 	a.sdf_in[(size_t)(3 + 2 * level) * N + i] = (hf)feat[0];
 	a.sdf_in[(size_t)(4 + 2 * level) * N + i] = (hf)feat[1];
-	if (FULL) {
-		const float six[6] = {J[0][0], J[0][1], J[0][2], J[1][0], J[1][1], J[1][2]};
-		a.slopes[(size_t)level * N + i] = n2_slopes_pack(six);
+	const float six[6] = {J[0][0], J[0][1], J[0][2], J[1][0], J[1][1], J[1][2]};
+	a.slopes[(size_t)level * N + i] = n2_slopes_pack(six);
+}
+
+// Inference on points in no particular order (features only): one (sample, level) item by a PAIR of adjacent lanes.  Lane b
+// gathers the four (y, z) corners of x corner b: the two x corners are neighbours in the table, so the pair reads one line and
+// the L1 looks up half as many as with eight gathers by one lane (2^20 uniform points 330 -> 291 us, 2^21 cells of the
+// occupancy grid 432 -> 407); then lane b finishes feature b.  (The full field's items hold the vector unit as much as the L1: there
+// the pair's doubled index arithmetic costs more than it saves, 80 us against 73 at the training step's batch.)
+__device__ __forceinline__ void gather_pair(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t b) {
+	const float* q = a.pos + (size_t)i * a.ps;
+	const float p[3] = {q[0], q[a.ds], q[2 * (size_t)a.ds]};
+	float feat = 0.f;
+	if (level < a.lv.active_levels) {  // a switched-off level: zero features
+		const uint32_t res = a.lv.res[level], entries = a.lv.entries[level];
+		const bool hashed = (a.lv.hash_mask >> level) & 1u;
+		uint32_t c[3];
+		float w[3];
+#pragma unroll
+		for (int d = 0; d < 3; ++d) n2_locate(p[d], a.lv.scale[level], w[d], c[d]);
+		const __half2* P = a.table + a.lv.offset[level];
+		float2 v[4];
+#pragma unroll
+		for (uint32_t k = 0; k < 4; ++k) {
+			const uint32_t y = c[1] + (k & 1u), z = c[2] + (k >> 1);
+			const uint32_t at = hashed ? n2_entry<N2_LEVEL_HASH>(entries, res, c[0] + b, y, z) : n2_entry<N2_LEVEL_DENSE>(entries, res, c[0] + b, y, z);
+			v[k] = h2f(*reinterpret_cast<const uint32_t*>(P + at));
+		}
+		const float wy = w[1], wz = w[2], uy = 1.f - wy, uz = 1.f - wz;
+		const float w00 = uy * uz, w10 = wy * uz, w01 = uy * wz, w11 = wy * wz;
+		const float s0 = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, w11 * v[3].x)));
+		const float s1 = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, w11 * v[3].y)));
+		// lane b keeps feature b of its own x plane and receives feature b of the partner's
+		const float mine = b ? s1 : s0, other = n2_pair_swap(b ? s0 : s1);
+		feat = fmaf(1.f - w[0], b ? other : mine, w[0] * (b ? mine : other));
 	}
+	a.sdf_in[(size_t)(3 + 2 * level + b) * a.N + i] = (hf)feat;
 }
 
 // first column and number of samples of a listed pass
@@ -337,51 +369,62 @@ __device__ __forceinline__ void listed_range(const FusedArgs& a, uint32_t& begin
 	count = min(a.counts[a.round], a.N - min(begin, a.N));
 }
 
-// The listed pass: the number of samples is known on the device only.  The launch has est_tiles workgroups per level, level-
-// major like the other kernel's; workgroup t of a level takes the tiles t, t + est_tiles, ...: any estimate gives the right
-// result, a good one gives every workgroup one tile.  (A fixed number of workgroups that walk all items by a stride is
-// 1.6 times slower beside the trainer's sample generator: its waves keep some of them from starting until others have
-// finished their whole share.)
+// The listed pass: the number of samples is known on the device only.  The launch has est_tiles workgroups per level, levels dealt
+// to the XCDs as in the other kernel (level-major: the three rounds of a trained field's step 32 us longer); workgroup t of a
+// level takes the tiles t, t + est_tiles, ...: any estimate gives the right result, a good one gives every workgroup one
+// tile.  (A fixed number of workgroups that walk all items by a stride is 1.6 times slower beside the trainer's sample
+// generator: its waves keep some of them from starting until others have finished their whole share.)
 __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const FusedArgs a, uint32_t est_tiles) {
 	__builtin_amdgcn_s_setprio(3);
-	const uint32_t level = blockIdx.x / est_tiles;
-	if (level >= a.n_levels) {  // the network kernel's weight fragments (round 0 only)
-		write_frag_image(a, blockIdx.x - a.n_levels * est_tiles);
+	const uint32_t gather_blocks = n2_xcd_blocks(a.n_levels, est_tiles);
+	if (blockIdx.x >= gather_blocks) {  // the network kernel's weight fragments (round 0 only)
+		write_frag_image(a, blockIdx.x - gather_blocks);
 		return;
 	}
+	uint32_t level, first_tile;
+	if (!n2_xcd_level_tile(a.n_levels, est_tiles, level, first_tile)) return;
 	uint32_t begin, count;
 	listed_range(a, begin, count);
 	const uint32_t tiles = (count + FG_BLOCK - 1) / FG_BLOCK;
-	for (uint32_t tile = blockIdx.x - level * est_tiles; tile < tiles; tile += est_tiles) {
+	for (uint32_t tile = first_tile; tile < tiles; tile += est_tiles) {
 		const uint32_t j = tile * FG_BLOCK + threadIdx.x;
-		if (j < count) gather_item<true>(a, level, begin + j, begin + j);
+		if (j < count) gather_item(a, level, begin + j, begin + j);
 	}
 }
 
 template <bool FULL>
-__global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs a, uint32_t tiles) {
-	// level-major workgroup ids: the workgroups that run at one time work on one or two levels, whose tables stay in every
-	// L2.  The launch is bound by the L2s' request rate: 10 M requests for the training step's 2.6e5 ray-ordered samples
-	// (four lines per sample on every level whose cells are smaller than the marching step), 63 % of them hits.  Measured on
-	// that workload and dropped: whole levels dealt to XCDs by a cost plan (the launch then fetches a third of the 278 MiB,
-	// but takes 9 to 20 us longer with every cost model tried), one 8- or 16-byte load per pair of x neighbours instead of
-	// two 4-byte loads (+12 us), a pair of lanes per sample so that the x neighbours' line is looked up once (+2 us), loads of
-	// the hashed levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then requested twice and
-	// a request is no cheaper) or carry the non-temporal hint (no change).
+__global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs a, uint32_t tiles, int by_xcd) {
+	// by_xcd: whole levels per XCD (n2_xcd_level_tile); else level-major workgroup ids, so that the workgroups that run at one
+	// time work on one or two levels, whose tables stay in every L2.  Level-major reads every table into eight L2s, 200 MB
+	// whatever the batch; by XCD it is 25 MB, but the XCDs are never quite even.  The launch is bound by the lines the L1s fetch
+	// (2.3 clocks of a CU each from the L2; four per sample on every level whose cells are smaller than the marching step)
+	// and, with slopes, by the vector unit: without its gathers it would still take 46 of 73 us.  Measured on the training
+	// step and dropped: one 8- or 16-byte load per pair of x neighbours instead of two 4-byte loads (+12 us), loads of the hashed
+	// levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then requested twice and
+	// a request is no cheaper) or carry the non-temporal hint (no change), the positions read as consecutive words and picked
+	// apart in LDS (+9).
 	// Staging the coarse levels in LDS has nothing to win: with all caches cold, levels 0..2 together add 2 us to the launch
 	// and the five dense levels 4 us, against 5 to 6 us for each of the fine hashed levels and 19 us for reading the
 	// positions and writing 320 bytes of features and slopes per sample.
 	// The trainer's sample generator runs beside this kernel on a second stream: where a wave of each is ready on a SIMD, this
 	// one issues first (the generator has the rest of the step to finish; measured 4 us on the forward, 2 us on the step).
 	__builtin_amdgcn_s_setprio(3);
-	const uint32_t level = blockIdx.x / tiles, tile = blockIdx.x - level * tiles;
-	if (FULL && level >= a.n_levels) {  // the workgroups behind the last level: the network kernel's weight fragments
-		write_frag_image(a, blockIdx.x - a.n_levels * tiles);
+	const uint32_t gather_blocks = by_xcd ? n2_xcd_blocks(a.n_levels, tiles) : a.n_levels * tiles;
+	if (FULL && blockIdx.x >= gather_blocks) {  // the workgroups behind those that gather: the network kernel's weight fragments
+		write_frag_image(a, blockIdx.x - gather_blocks);
 		return;
 	}
-	const uint32_t i = tile * FG_BLOCK + threadIdx.x;
-	if (i >= a.N || (a.live && i >= *a.live)) return;
-	gather_item<FULL>(a, level, i, i);
+	uint32_t level, tile;
+	if (!by_xcd) {
+		level = blockIdx.x / tiles;
+		tile = blockIdx.x - level * tiles;
+	} else if (!n2_xcd_level_tile(a.n_levels, tiles, level, tile)) {
+		return;
+	}
+	const uint32_t i = FULL ? tile * FG_BLOCK + threadIdx.x : tile * FG_PAIRS + (threadIdx.x >> 1);
+	if (i >= a.N || (a.live && i >= *a.live)) return;  // (both lanes of a pair)
+	if (FULL) gather_item(a, level, i, i);
+	else gather_pair(a, level, i, threadIdx.x & 1u);
 }
 
 // ----------------------------------------------------------------------------
@@ -620,10 +663,16 @@ bool n2_fused_supported(const N2LevelTable& tab, uint32_t sdf_hidden_layers, uin
 	return true;
 }
 
+// Up to here a gather's levels are dealt to the XCDs: from there on what the uneven XCDs lose is more than what reading the tables
+// into every L2 costs (field, rays: 2^14 samples 12.4 -> 9.9 us, 5e4 24.8 -> 19, 2.6e5 74.7 -> 73; uniform queries: 2^20 291
+// level-major, 299 by XCD).
+constexpr uint32_t GATHER_XCD_MAX = 1u << 19;
 template <bool FULL>
 static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream_t s) {
-	const uint32_t tiles = (a.N + FG_BLOCK - 1) / FG_BLOCK;
-	field_gather_kernel<FULL><<<dim3(tiles * tab.n_levels + (FULL && a.frags ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, tiles);
+	const uint32_t per = FULL ? FG_BLOCK : FG_PAIRS, tiles = (a.N + per - 1) / per;
+	const bool by_xcd = a.N <= GATHER_XCD_MAX;
+	const uint32_t blocks = by_xcd ? n2_xcd_blocks(tab.n_levels, tiles) : tiles * tab.n_levels;
+	field_gather_kernel<FULL><<<dim3(blocks + (FULL && a.frags ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, tiles, by_xcd ? 1 : 0);
 }
 
 static uint32_t fused_grid(uint32_t n) {
@@ -685,7 +734,7 @@ int n2_fused_field_forward(const N2FusedNets& nets, hipStream_t s, const float* 
 		// est_samples: the caller's estimate of this round's sample count (it only sizes the launches)
 		const uint32_t est = est_samples < 1u ? 1u : (est_samples > n ? n : est_samples);
 		const uint32_t est_tiles = (est + FG_BLOCK - 1) / FG_BLOCK;
-		field_gather_list_kernel<<<dim3(est_tiles * a.n_levels + (a.frags && round == 0 ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, est_tiles);
+		field_gather_list_kernel<<<dim3(n2_xcd_blocks(a.n_levels, est_tiles) + (a.frags && round == 0 ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, est_tiles);
 		N2_LAUNCH_CHECK();
 		// one 32-sample tile per wave where the estimate holds (the weight fragments come as a copy, so small workgroups are cheap)
 		const uint32_t blocks = (est + 127u) / 128u;

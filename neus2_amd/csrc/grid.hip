@@ -3,14 +3,11 @@
 // backward_backward_input, behind the n2_grid_* C ABI.
 //
 // Work decomposition: one workgroup handles a tile of points for ONE level.
-// The gather kernels number their (level, tile) work items level-major and cut
-// that list into 8 contiguous pieces of equal estimated cost, one per XCD: the
-// hardware deals consecutive workgroup ids round-robin over the 8 XCDs, so
-// workgroup id b runs on XCD b % 8 and takes item number b / 8 of that XCD's
-// piece.  Each XCD then streams all points through about two levels, and its
-// private 4 MiB L2 fetches only those levels' tables (<= 2 MiB each at
-// T = 2^19) instead of all 24 MiB.  (With plain level-major ids every XCD
-// walks every level and the table crosses the fabric 8 times per launch.)
+// The gather kernels deal whole levels to the XCDs (n2_xcd_level_tile), each of
+// which then streams all points through about two levels and fetches only those
+// levels' tables (<= 2 MiB each at T = 2^19) into its private 4 MiB L2 instead of
+// all 24 MiB; with costs from n2_grid_set_level_costs they cut the level-major
+// list of items into 8 contiguous pieces of equal estimated cost.
 #include "n2_common.h"
 #include "grid_device.h"
 #include "slab_reduce.h"
@@ -27,6 +24,7 @@ struct n2_grid {
 	__half2* grads;
 	// relative cost of one tile of each level (balances the levels over the XCDs)
 	float level_cost[N2_MAX_LEVELS];
+	bool costs_set;  // by n2_grid_set_level_costs
 	// progressive training (base_training_step 0: off)
 	float base_valid_level_scale, valid_level_scale;
 	uint32_t base_training_step;
@@ -78,7 +76,8 @@ __device__ __forceinline__ float n2_corner_weight(const N2Point& p, uint32_t k) 
 constexpr uint32_t GRID_BLOCK = 256;
 constexpr uint32_t N_XCD = 8;  // gfx950: 8 XCDs, workgroup ids are dealt round-robin
 
-// Piece x of the level-major item list [begin[x], begin[x + 1]) belongs to XCD x.
+// Piece x of the level-major item list [begin[x], begin[x + 1]) belongs to XCD x; begin[N_XCD] = 0: no plan, n2_xcd_level_tile deals
+// the items (2^18 points with dy_dx: 84 us uniform, 60 in ray order; with the plan of the default costs 101 and 74).
 struct N2XcdPlan {
 	uint32_t begin[N_XCD + 1];
 };
@@ -101,11 +100,6 @@ __device__ __forceinline__ bool n2_xcd_item(const N2XcdPlan& plan, uint32_t tile
 // the memory pipeline, which looks up one line per clock, sees half as many lines per point.  The pair then
 // exchanges its partial sums and lane b finishes feature b.
 constexpr uint32_t FWD_POINTS = GRID_BLOCK / 2;  // points per workgroup and level
-
-// value held by the other lane of the pair (lane ^ 1): a quad permute [1, 0, 3, 2] inside the VALU, no LDS crossbar
-__device__ __forceinline__ float n2_pair_swap(float x) {
-	return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, true));
-}
 
 template <uint32_t MODE, bool WANT_DYDX>
 __device__ __forceinline__ void grid_forward_pair(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t b, uint32_t N,
@@ -162,7 +156,7 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable t
                                                                   uint32_t dim_stride, const __half2* __restrict__ params,
                                                                   __half* __restrict__ out, float* __restrict__ dy_dx) {
 	uint32_t level, tile;
-	if (!n2_xcd_item(plan, tiles, level, tile)) return;
+	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_xcd_level_tile(tab.n_levels, tiles, level, tile))) return;
 	const uint32_t i = tile * FWD_POINTS + (threadIdx.x >> 1), b = threadIdx.x & 1u;
 	if (i >= N) return;  // both lanes of a pair share i, so pairs leave together
 #define CALL(M) grid_forward_pair<M, WANT_DYDX>(tab, level, i, b, N, xyz, point_stride, dim_stride, params, out, dy_dx)
@@ -975,6 +969,7 @@ N2_API int n2_grid_create(uint32_t n_levels, uint32_t n_features_per_level, uint
 	g->ws_bytes = 0;
 	g->ws_max_points = 0;
 	g->lattice_order = false;
+	g->costs_set = false;
 	*out = g;
 	return N2_OK;
 }
@@ -1005,6 +1000,7 @@ N2_API int n2_grid_set_level_costs(n2_grid_t* grid, const float* costs) {
 		N2_REQUIRE(costs[l] > 0.f && costs[l] <= 1e6f, "n2_grid_set_level_costs: cost of level %u must be in (0, 1e6]", l);
 	}
 	for (uint32_t l = 0; l < grid->tab.n_levels; ++l) grid->level_cost[l] = costs[l];
+	grid->costs_set = true;
 	return N2_OK;
 }
 
@@ -1138,7 +1134,8 @@ N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_x
 		return N2_OK;
 	}
 	const uint32_t tiles = (n_points + FWD_POINTS - 1) / FWD_POINTS;
-	const dim3 grid_dim(make_xcd_plan(grid, tiles, plan) * N_XCD), block(GRID_BLOCK);
+	plan.begin[N_XCD] = 0;
+	const dim3 grid_dim(grid->costs_set ? make_xcd_plan(grid, tiles, plan) * N_XCD : n2_xcd_blocks(grid->tab.n_levels, tiles)), block(GRID_BLOCK);
 	if (d_dy_dx) {
 		grid_forward_kernel<true><<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride,
 			dim_stride, grid->params, reinterpret_cast<__half*>(d_out), d_dy_dx);

@@ -528,3 +528,22 @@ def test_lattice_order_forward(setup):
         gg.set_max_level(1.0)
     y0, _ = gg.forward(dev(xyz))
     assert rel_l2(host(y1), host(y0)) < 1e-3
+
+
+@pytest.mark.parametrize("levels", [16, 14, 5])  # whole rounds of eight levels over the XCDs, a cut last round, nothing but that
+@pytest.mark.parametrize("n", [1, 129, 3000])
+def test_forward_by_level_costs_equals_the_default_deal(levels, n):
+    """How the levels are dealt to the XCDs never shows in the results."""
+    import ctypes as C
+
+    from neus2_amd import capi
+    from neus2_amd.tcnn_api import GridEncoding
+    g = GridEncoding(levels, 2, 14, 8, 1.5)
+    gen = torch.Generator(device="cuda").manual_seed(levels)
+    p = torch.rand(g.n_params(), device="cuda", generator=gen).half()
+    g.set_params(p, None)
+    x = torch.rand((3, n), device="cuda", generator=gen)
+    a, ja = g.forward(x, prepare_input_gradients=True)
+    capi.check(capi.lib().n2_grid_set_level_costs(g._h, (C.c_float * levels)(*[1.0 + 3 * (l % 3) for l in range(levels)])))
+    b, jb = g.forward(x, prepare_input_gradients=True)
+    assert torch.equal(a, b) and torch.equal(ja, jb) and bool(a.abs().sum() > 0)
