@@ -108,33 +108,79 @@ constexpr uint32_t OCC_WALK_INV = occ_inverse_mod_2_32(OCC_WALK);
 static_assert(OCC_WALK * OCC_WALK_INV == 1u, "inverse of the walk's multiplier");
 static inline uint32_t occ_order_mul(uint32_t n) { return (n >= 2 && (n & (n - 1)) == 0) ? OCC_WALK_INV : 0u; }
 
-__global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uint32_t n_pad, Pcg32 rng, uint32_t step, const float* __restrict__ grid,
+// The generator skips 4 i draws ahead for sample i: state -> mult^(4 i) state + inc (1 + mult + .. + mult^(4 i - 1)).  The skip is
+// composed from the hexadecimal digits of i, whose two factors are a table of constants: a multiply-add per digit instead of
+// a loop over the bits of 4 i with three 64-bit products each (2^21 samples, one cascade: 33 us and 5.6 us for the clearing -> 15.6 us for
+// all of it; 42 us when every workgroup works the factors out itself).
+// The launch also clears tmp (n_tmp floats, a multiple of 4), which the samples' densities are splatted into, and leaves the
+// positions as three rows of n_rows floats beside the [n][3] array (rows: null or these): the encoding's gather reads them.
+constexpr uint32_t OCC_DIGITS = 8;
+struct OccSkips {
+	uint64_t mult[OCC_DIGITS * 16], plus[OCC_DIGITS * 16];  // [digit's place][digit]; plus for an increment of one
+};
+constexpr OccSkips occ_build_skips() {
+	OccSkips t{};
+	uint64_t m = 1, s = 0;  // the skip by one unit of the place: 4 draws at first
+	for (int k = 0; k < 4; ++k) {
+		s = s * PCG32_MULT + 1u;
+		m *= PCG32_MULT;
+	}
+	for (uint32_t p = 0; p < OCC_DIGITS; ++p) {
+		uint64_t cm = 1, cs = 0;
+		for (uint32_t d = 0; d < 16; ++d) {
+			t.mult[p * 16 + d] = cm;
+			t.plus[p * 16 + d] = cs;
+			cs = cs * m + s;
+			cm *= m;
+		}
+		m = cm;
+		s = cs;
+	}
+	return t;
+}
+static __device__ const OccSkips OCC_SKIPS = occ_build_skips();
+
+__global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uint32_t n_pad, Pcg32 rng, uint32_t n_digits, uint32_t step, const float* __restrict__ grid,
                                                                  uint32_t n_cascades, float thresh, uint32_t order_mul,
-                                                                 float* __restrict__ positions, uint32_t* __restrict__ indices) {
+                                                                 float* __restrict__ positions, uint32_t* __restrict__ indices, float* __restrict__ rows, uint32_t n_rows,
+                                                                 float* __restrict__ tmp, uint32_t n_tmp) {
+	__shared__ ulonglong2 skip[OCC_DIGITS][16];
+	if (threadIdx.x < n_digits * 16u) {
+		skip[threadIdx.x >> 4][threadIdx.x & 15u] = make_ulonglong2(OCC_SKIPS.mult[threadIdx.x], OCC_SKIPS.plus[threadIdx.x] * rng.inc);
+	}
 	const uint32_t slot = blockIdx.x * OCC_BLOCK + threadIdx.x;
+	for (uint64_t k = slot; k * 4u < n_tmp; k += (uint64_t)gridDim.x * OCC_BLOCK) reinterpret_cast<float4*>(tmp)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+	__syncthreads();
 	if (slot >= n_pad) return;
-	if (slot >= n) {
-		positions[(size_t)slot * 3] = 0.5f; positions[(size_t)slot * 3 + 1] = 0.5f; positions[(size_t)slot * 3 + 2] = 0.5f;
-		return;
+	float pos[3] = {0.5f, 0.5f, 0.5f};
+	if (slot < n) {
+		const uint32_t i = order_mul ? (slot * order_mul) & (n - 1u) : slot;
+		for (uint32_t p = 0; p < n_digits; ++p) {
+			const ulonglong2 f = skip[p][(i >> (4u * p)) & 15u];
+			rng.state = f.x * rng.state + f.y;
+		}
+		const uint32_t level = (uint32_t)(rng.next_float() * n_cascades) % n_cascades;
+		uint32_t idx = 0;
+		for (uint32_t j = 0; j < 10; ++j) {
+			idx = ((i + step * n) * OCC_WALK + j * 19349663u + 96925573u) % OCC_CELLS;
+			idx += level * OCC_CELLS;
+			if (grid[idx] > thresh) break;
+		}
+		const uint32_t pos_idx = idx % OCC_CELLS;
+		const float scale = scalbnf(1.0f, (int)level);
+#pragma unroll
+		for (int d = 0; d < 3; ++d) {
+			const float c = (float)occ_morton3d_invert(pos_idx >> d);
+			const float u = rng.next_float();
+			pos[d] = ((c + u) / (float)OCC_GRIDSIZE - 0.5f) * scale + 0.5f;
+		}
+		indices[slot] = idx;
 	}
-	const uint32_t i = order_mul ? (slot * order_mul) & (n - 1u) : slot;
-	rng.advance((uint64_t)i * 4);
-	const uint32_t level = (uint32_t)(rng.next_float() * n_cascades) % n_cascades;
-	uint32_t idx = 0;
-	for (uint32_t j = 0; j < 10; ++j) {
-		idx = ((i + step * n) * OCC_WALK + j * 19349663u + 96925573u) % OCC_CELLS;
-		idx += level * OCC_CELLS;
-		if (grid[idx] > thresh) break;
-	}
-	const uint32_t pos_idx = idx % OCC_CELLS;
-	const float scale = scalbnf(1.0f, (int)level);
 #pragma unroll
 	for (int d = 0; d < 3; ++d) {
-		const float c = (float)occ_morton3d_invert(pos_idx >> d);
-		const float u = rng.next_float();
-		positions[(size_t)slot * 3 + d] = ((c + u) / (float)OCC_GRIDSIZE - 0.5f) * scale + 0.5f;
+		positions[(size_t)slot * 3 + d] = pos[d];
+		if (rows) rows[(size_t)d * n_rows + slot] = pos[d];
 	}
-	indices[slot] = idx;
 }
 
 // splat_grid_samples_nerf_max_nearest_neighbor (:662-680): positive floats order like their bit patterns
@@ -154,15 +200,24 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_ema_kernel(uint32_t n_elements,
 	__shared__ float red[OCC_BLOCK / 64];
 	const uint32_t base = blockIdx.x * (OCC_BLOCK * 32);
 	float sum = 0.f;
-	for (uint32_t k = 0; k < 32; ++k) {
-		const uint32_t i = base + k * OCC_BLOCK + threadIdx.x;
-		if (i < n_elements) {
-			float val = grid[i];
+	constexpr uint32_t BATCH = 16;  // cells of a thread in flight (one after the other: 18.5 us for 128^3 cells, in batches 6.7)
+	for (uint32_t k0 = 0; k0 < 32; k0 += BATCH) {
+		float val[BATCH], fresh[BATCH];
+#pragma unroll
+		for (uint32_t k = 0; k < BATCH; ++k) {
+			const uint32_t i = min(base + (k0 + k) * OCC_BLOCK + threadIdx.x, n_elements - 1u);
+			val[k] = grid[i];
+			fresh[k] = MERGE ? tmp[i] : 0.f;
+		}
+#pragma unroll
+		for (uint32_t k = 0; k < BATCH; ++k) {
+			const uint32_t i = base + (k0 + k) * OCC_BLOCK + threadIdx.x;
+			if (i >= n_elements) continue;
 			if (MERGE) {
-				val = (val < 0.f) ? val : fmaxf(val * decay, tmp[i]);
-				grid[i] = val;
+				val[k] = (val[k] < 0.f) ? val[k] : fmaxf(val[k] * decay, fresh[k]);
+				grid[i] = val[k];
 			}
-			sum += fmaxf(val, 0.f);
+			sum += fmaxf(val[k], 0.f);
 		}
 	}
 #pragma unroll
@@ -172,49 +227,92 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_ema_kernel(uint32_t n_elements,
 	if (threadIdx.x == 0 && blockIdx.x < OCC_MEAN_BLOCKS) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ void __launch_bounds__(OCC_MEAN_BLOCKS) occ_mean_kernel(const float* __restrict__ partial, float* __restrict__ mean) {
-	__shared__ float red[OCC_MEAN_BLOCKS / 64];
+// The mean over the first cascade from its partial sums: every workgroup adds them up again, in the same order, instead of
+// waiting for a launch that does.  All OCC_BLOCK lanes take part.
+static_assert(OCC_MEAN_BLOCKS == OCC_BLOCK, "one partial sum per lane");
+__device__ __forceinline__ float occ_mean(const float* __restrict__ partial, float* red) {
 	float sum = partial[threadIdx.x];
 #pragma unroll
 	for (int o = 32; o > 0; o >>= 1) sum += __shfl_down(sum, o);
 	if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
 	__syncthreads();
-	if (threadIdx.x == 0) mean[0] = ((red[0] + red[1]) + (red[2] + red[3])) / (float)OCC_CELLS;
-}
-
-// grid_to_bitfield (:738-764): one byte = 8 consecutive (morton-ordered) cells; levels beyond the scene's cascades are cleared
-__global__ void __launch_bounds__(OCC_BLOCK) occ_bitfield_kernel(uint32_t n_bytes, uint32_t n_nonzero_bytes, const float* __restrict__ grid,
-                                                                 uint8_t* __restrict__ bitfield, const float* __restrict__ mean) {
-	const uint32_t i = blockIdx.x * OCC_BLOCK + threadIdx.x;
-	if (i >= n_bytes) return;
-	if (i >= n_nonzero_bytes) {
-		bitfield[i] = 0;
-		return;
-	}
-	const float thresh = fminf(OCC_MIN_OPTICAL_THICKNESS, mean[0]);
-	const float4 a = reinterpret_cast<const float4*>(grid)[(size_t)i * 2], b = reinterpret_cast<const float4*>(grid)[(size_t)i * 2 + 1];
-	uint32_t bits = 0;
-	bits |= a.x > thresh ? 1u : 0u; bits |= a.y > thresh ? 2u : 0u; bits |= a.z > thresh ? 4u : 0u; bits |= a.w > thresh ? 8u : 0u;
-	bits |= b.x > thresh ? 16u : 0u; bits |= b.y > thresh ? 32u : 0u; bits |= b.z > thresh ? 64u : 0u; bits |= b.w > thresh ? 128u : 0u;
-	bitfield[i] = (uint8_t)bits;
+	return ((red[0] + red[1]) + (red[2] + red[3])) / (float)OCC_CELLS;
 }
 
 // bitfield_max_pool (:766-786): a byte of the next level collects "any bit set" of 8 bytes (8 blocks of 2^3 cells) of
-// the previous one and lands in the central half of the next level's grid.  Distinct i write distinct bytes.
-__global__ void __launch_bounds__(OCC_BLOCK) occ_pool_kernel(const uint8_t* __restrict__ prev, uint8_t* __restrict__ next) {
-	const uint32_t i = blockIdx.x * OCC_BLOCK + threadIdx.x;
-	if (i >= OCC_CELLS / 64) return;
-	const uint2 p = reinterpret_cast<const uint2*>(prev)[i];
+// the previous one ...
+__device__ __forceinline__ uint32_t occ_pool_byte(const uint2 p) {
 	uint32_t bits = 0;
 #pragma unroll
 	for (uint32_t j = 0; j < 4; ++j) {
 		bits |= ((p.x >> (8 * j)) & 0xFFu) ? (1u << j) : 0u;
 		bits |= ((p.y >> (8 * j)) & 0xFFu) ? (16u << j) : 0u;
 	}
-	const uint32_t x = occ_morton3d_invert(i >> 0) + OCC_GRIDSIZE / 8;
-	const uint32_t y = occ_morton3d_invert(i >> 1) + OCC_GRIDSIZE / 8;
-	const uint32_t z = occ_morton3d_invert(i >> 2) + OCC_GRIDSIZE / 8;
-	next[occ_morton3d(x, y, z)] |= (uint8_t)bits;
+	return bits;
+}
+// ... and lands in the central half of the next level's grid: byte i of 8-byte groups -> byte of the next level
+__device__ __forceinline__ uint32_t occ_pool_target(uint32_t i) {
+	return occ_morton3d(occ_morton3d_invert(i >> 0) + OCC_GRIDSIZE / 8, occ_morton3d_invert(i >> 1) + OCC_GRIDSIZE / 8, occ_morton3d_invert(i >> 2) + OCC_GRIDSIZE / 8);
+}
+
+// grid_to_bitfield (:738-764): one byte = 8 consecutive (morton-ordered) cells, a lane works out eight of them and writes them
+// as one store; levels beyond the scene's cascades are cleared.  With one cascade a lane's eight bytes also are all that
+// goes into one byte of level 1: it writes that too, and the lanes that clear level 1 leave the central half alone.
+__global__ void __launch_bounds__(OCC_BLOCK) occ_bitfield_kernel(uint32_t n_cascades, const float* __restrict__ grid, uint8_t* __restrict__ bitfield,
+                                                                 const float* __restrict__ partial, float* __restrict__ mean) {
+	__shared__ float red[OCC_BLOCK / 64];
+	const float m = occ_mean(partial, red);
+	if (blockIdx.x == 0 && threadIdx.x == 0) mean[0] = m;
+	const uint32_t i = blockIdx.x * OCC_BLOCK + threadIdx.x;  // group of eight bytes
+	uint2* out = reinterpret_cast<uint2*>(bitfield) + i;
+	constexpr uint32_t GROUPS = OCC_LEVEL_BYTES / 8;
+	if (i >= n_cascades * GROUPS) {
+		if (n_cascades == 1 && i < 2u * GROUPS) {
+			const uint32_t g = i - GROUPS, x = occ_morton3d_invert(g), y = occ_morton3d_invert(g >> 1), z = occ_morton3d_invert(g >> 2);  // 2^3 bytes each
+			constexpr uint32_t LO = OCC_GRIDSIZE / 16, HI = LO + OCC_GRIDSIZE / 8;
+			if (x >= LO && x < HI && y >= LO && y < HI && z >= LO && z < HI) return;
+		}
+		*out = make_uint2(0u, 0u);
+		return;
+	}
+	const float thresh = fminf(OCC_MIN_OPTICAL_THICKNESS, m);
+	uint32_t bytes[2] = {0u, 0u};
+#pragma unroll
+	for (uint32_t q = 0; q < 16; ++q) {
+		const float4 a = reinterpret_cast<const float4*>(grid)[(size_t)i * 16 + q];
+		const uint32_t bits = (a.x > thresh ? 1u : 0u) | (a.y > thresh ? 2u : 0u) | (a.z > thresh ? 4u : 0u) | (a.w > thresh ? 8u : 0u);
+		bytes[q >> 3] |= bits << (4 * (q & 7u));
+	}
+	*out = make_uint2(bytes[0], bytes[1]);
+	if (n_cascades == 1) bitfield[OCC_LEVEL_BYTES + occ_pool_target(i)] = (uint8_t)occ_pool_byte(make_uint2(bytes[0], bytes[1]));
+}
+
+// One level of pooling, for levels that have cells of their own or lie right above one that has.  Distinct i write distinct bytes.
+__global__ void __launch_bounds__(OCC_BLOCK) occ_pool_kernel(const uint8_t* __restrict__ prev, uint8_t* __restrict__ next) {
+	const uint32_t i = blockIdx.x * OCC_BLOCK + threadIdx.x;
+	if (i >= OCC_CELLS / 64) return;
+	next[occ_pool_target(i)] |= (uint8_t)occ_pool_byte(reinterpret_cast<const uint2*>(prev)[i]);
+}
+
+// The pooling of all levels from `first` on, by one workgroup: level first - 1 has nothing outside its central half, so level
+// `first` has nothing outside its central quarter, and so on: 16^3 groups of bytes for the first level, an eighth for each
+// level after it.  (128^3 cells, one cascade: mean, bitfield and seven
+// launches for the levels 42 us -> 13.3 us in two launches.)
+__global__ void __launch_bounds__(1024) occ_pool_upper_kernel(uint32_t first, uint8_t* __restrict__ bitfield) {
+	uint32_t lo = OCC_GRIDSIZE / 8, hi = 3 * OCC_GRIDSIZE / 8 - 1;  // byte coordinates (64 along a side) of what the level below can hold
+	for (uint32_t level = first; level < OCC_LEVELS; ++level) {
+		const uint8_t* prev = bitfield + (size_t)(level - 1) * OCC_LEVEL_BYTES;
+		uint8_t* next = bitfield + (size_t)level * OCC_LEVEL_BYTES;
+		const uint32_t g = lo / 2, side = hi / 2 - g + 1;
+		for (uint32_t k = threadIdx.x; k < side * side * side; k += 1024) {
+			const uint32_t i = occ_morton3d(g + k % side, g + (k / side) % side, g + k / (side * side));
+			next[occ_pool_target(i)] = (uint8_t)occ_pool_byte(reinterpret_cast<const uint2*>(prev)[i]);
+		}
+		lo = g + OCC_GRIDSIZE / 8;
+		hi = g + side - 1 + OCC_GRIDSIZE / 8;
+		__threadfence_block();
+		__syncthreads();
+	}
 }
 
 // ---------------------------------------------------------------------------
@@ -318,14 +416,17 @@ N2_API int n2_occupancy_update_bitfield(n2_occupancy_t* occ, n2_stream_t stream)
 }
 
 static int occ_bitfield_from_partials(n2_occupancy_t* occ, hipStream_t s) {
-	const uint32_t n_bytes = OCC_LEVELS * OCC_LEVEL_BYTES;
-	occ_mean_kernel<<<dim3(1), dim3(OCC_MEAN_BLOCKS), 0, s>>>(occ->partial, occ->mean);
+	occ_bitfield_kernel<<<ogrid(OCC_LEVELS * OCC_LEVEL_BYTES / 8), dim3(OCC_BLOCK), 0, s>>>(occ->n_cascades, occ->grid, occ->bitfield, occ->partial, occ->mean);
 	N2_LAUNCH_CHECK();
-	occ_bitfield_kernel<<<ogrid(n_bytes), dim3(OCC_BLOCK), 0, s>>>(n_bytes, occ->n_cascades * OCC_LEVEL_BYTES, occ->grid, occ->bitfield, occ->mean);
-	N2_LAUNCH_CHECK();
-	for (uint32_t level = 1; level < OCC_LEVELS; ++level) {
-		occ_pool_kernel<<<ogrid(OCC_CELLS / 64), dim3(OCC_BLOCK), 0, s>>>(occ->bitfield + (size_t)(level - 1) * OCC_LEVEL_BYTES,
-		                                                                  occ->bitfield + (size_t)level * OCC_LEVEL_BYTES);
+	if (occ->n_cascades > 1) {
+		for (uint32_t level = 1; level <= occ->n_cascades && level < OCC_LEVELS; ++level) {
+			occ_pool_kernel<<<ogrid(OCC_CELLS / 64), dim3(OCC_BLOCK), 0, s>>>(occ->bitfield + (size_t)(level - 1) * OCC_LEVEL_BYTES,
+			                                                                  occ->bitfield + (size_t)level * OCC_LEVEL_BYTES);
+			N2_LAUNCH_CHECK();
+		}
+	}
+	if (occ->n_cascades + 1 < OCC_LEVELS) {
+		occ_pool_upper_kernel<<<dim3(1), dim3(1024), 0, s>>>(occ->n_cascades + 1, occ->bitfield);
 		N2_LAUNCH_CHECK();
 	}
 	return N2_OK;
@@ -339,22 +440,30 @@ N2_API int n2_occupancy_update(n2_occupancy_t* occ, n2_field_t* field, n2_stream
 	N2_REQUIRE(n64 <= occ->max_samples, "n2_occupancy_update: %llu samples exceed the workspace's %u", (unsigned long long)n64, occ->max_samples);
 	hipStream_t s = n2_stream(stream);
 	const uint32_t n = (uint32_t)n64, n_elements = occ->n_cascades * OCC_CELLS;
-	if (int rc = n2_fill_zero_u32(s, occ->tmp, 4ull * n_elements)) return rc;
 	Pcg32 rng{occ->rng_state, occ->rng_inc};
+	// when one chunk holds all samples, their positions also go out as rows, into the fp16 scratch (which the unfused field
+	// path writes only after it has read them)
+	const uint32_t n8 = (n + 7) / 8 * 8;
+	float* rows = n8 <= occ->chunk ? reinterpret_cast<float*>(occ->mlp_out) : nullptr;
+	auto generate = [&](uint32_t count, uint32_t pad, uint32_t first, float thresh, bool clear) -> int {
+		uint32_t digits = 1;
+		while (digits < OCC_DIGITS && (count >> (4u * digits)) != 0) ++digits;
+		occ_generate_kernel<<<ogrid(pad), dim3(OCC_BLOCK), 0, s>>>(count, pad, rng, digits, occ->ema_step, occ->grid, occ->n_cascades, thresh, occ_order_mul(count),
+		                                                          occ->positions + (size_t)first * 3, occ->indices + first, rows ? rows + first : nullptr, n8,
+		                                                          occ->tmp, clear ? n_elements : 0u);
+		N2_LAUNCH_CHECK();
+		return N2_OK;
+	};
+	if (n == 0) {
+		if (int rc = n2_fill_zero_u32(s, occ->tmp, 4ull * n_elements)) return rc;
+	}
 	if (n_uniform) {
 		// slots of the second group are written by the second launch; only the last launch pads
-		const uint32_t pad = n_nonuniform ? n_uniform : (n_uniform + 7) / 8 * 8;
-		occ_generate_kernel<<<ogrid(pad), dim3(OCC_BLOCK), 0, s>>>(n_uniform, pad, rng, occ->ema_step, occ->grid, occ->n_cascades, -0.01f,
-		                                                          occ_order_mul(n_uniform), occ->positions, occ->indices);
-		N2_LAUNCH_CHECK();
+		if (int rc = generate(n_uniform, n_nonuniform ? n_uniform : n8, 0, -0.01f, true)) return rc;
 	}
 	rng.advance(1ull << 32);
 	if (n_nonuniform) {
-		const uint32_t pad = (n + 7) / 8 * 8 - n_uniform;
-		occ_generate_kernel<<<ogrid(pad), dim3(OCC_BLOCK), 0, s>>>(n_nonuniform, pad, rng, occ->ema_step, occ->grid, occ->n_cascades,
-		                                                          OCC_MIN_OPTICAL_THICKNESS, occ_order_mul(n_nonuniform),
-		                                                          occ->positions + (size_t)n_uniform * 3, occ->indices + n_uniform);
-		N2_LAUNCH_CHECK();
+		if (int rc = generate(n_nonuniform, n8 - n_uniform, n_uniform, OCC_MIN_OPTICAL_THICKNESS, n_uniform == 0)) return rc;
 	}
 	rng.advance(1ull << 32);
 	occ->rng_state = rng.state;
@@ -363,7 +472,8 @@ N2_API int n2_occupancy_update(n2_occupancy_t* occ, n2_field_t* field, n2_stream
 		const uint32_t m = (n - a < occ->chunk) ? n - a : occ->chunk, m8 = (m + 7) / 8 * 8;
 		// only the density row is kept, as fp32 (the fp16 output widened); the row sits behind the fp16 scratch the unfused path needs
 		float* row0 = reinterpret_cast<float*>(occ->mlp_out + (size_t)16 * occ->chunk);
-		if (int rc = n2_field_sdf_row0(field, stream, occ->positions + (size_t)a * 3, 3, 1, m8, m8, row0, reinterpret_cast<n2_half*>(occ->mlp_out), true)) return rc;
+		if (int rc = n2_field_sdf_row0(field, stream, rows ? rows : occ->positions + (size_t)a * 3, rows ? 1u : 3u, rows ? n8 : 1u, m8, m8, row0,
+		                               reinterpret_cast<n2_half*>(occ->mlp_out), true)) return rc;
 		occ_splat_kernel<<<ogrid(m), dim3(OCC_BLOCK), 0, s>>>(m, occ->indices + a, row0, occ->tmp);
 		N2_LAUNCH_CHECK();
 	}

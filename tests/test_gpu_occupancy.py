@@ -99,6 +99,23 @@ def test_two_cascades_and_mips(oracle, trainer):
     assert_close(host(occ.density_grid_tmp)[cells_in], info["tmp"][cells_in], rtol=RTOL, what="maxima inside the unit cube", outlier_frac=1e-3)
 
 
+@pytest.mark.parametrize("n_cascades", [1, 2, 6, 7, 8])
+def test_bitfield_levels_for_every_cascade_count(oracle, n_cascades):
+    """One cascade pools its own level, one workgroup the levels above the last cascade's next one: all of it exact."""
+    from neus2_amd.training import OccupancyGrid
+    rng = np.random.default_rng(n_cascades)
+    occ = OccupancyGrid(n_cascades, seed=1, max_chunk=1 << 16)
+    grid = np.zeros(n_cascades * CELLS, np.float32)
+    some = rng.choice(grid.size, 4000, replace=False)
+    some[:2] = 0, grid.size - 1  # the corners of the first and of the last cascade
+    grid[some] = rng.uniform(0.0, 0.01, some.size)
+    occ.density_grid.copy_(dev(grid))
+    occ.update_bitfield()
+    want = oracle.grid_to_bitfield(grid, n_cascades, float(host(occ.mean)[0]))
+    np.testing.assert_array_equal(host(occ.bitfield), want)
+    assert want.reshape(8, -1).any(1).sum() >= min(n_cascades + 1, 8)
+
+
 def test_reset_and_restore_state(oracle, trainer):
     from neus2_amd import capi
     from neus2_amd.training import OccupancyGrid
