@@ -332,32 +332,44 @@ __device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, 
 // the L1 looks up half as many as with eight gathers by one lane (2^20 uniform points 330 -> 291 us, 2^21 cells of the
 // occupancy grid 432 -> 407); then lane b finishes feature b.  (The full field's items hold the vector unit as much as the L1: there
 // the pair's doubled index arithmetic costs more than it saves, 80 us against 73 at the training step's batch.)
+struct PairItem {
+	uint32_t raw[4];
+	float w[3];
+};
+__device__ __forceinline__ void pair_fetch(const FusedArgs& a, uint32_t level, const float (&p)[3], uint32_t b, PairItem& it) {
+	const uint32_t res = a.lv.res[level], entries = a.lv.entries[level];
+	const bool hashed = (a.lv.hash_mask >> level) & 1u;
+	uint32_t c[3];
+#pragma unroll
+	for (int d = 0; d < 3; ++d) n2_locate(p[d], a.lv.scale[level], it.w[d], c[d]);
+	const __half2* P = a.table + a.lv.offset[level];
+#pragma unroll
+	for (uint32_t k = 0; k < 4; ++k) {
+		const uint32_t y = c[1] + (k & 1u), z = c[2] + (k >> 1);
+		const uint32_t at = hashed ? n2_entry<N2_LEVEL_HASH>(entries, res, c[0] + b, y, z) : n2_entry<N2_LEVEL_DENSE>(entries, res, c[0] + b, y, z);
+		it.raw[k] = *reinterpret_cast<const uint32_t*>(P + at);
+	}
+}
+__device__ __forceinline__ float pair_finish(const PairItem& it, uint32_t b) {
+	float2 v[4];
+#pragma unroll
+	for (int k = 0; k < 4; ++k) v[k] = h2f(it.raw[k]);
+	const float wy = it.w[1], wz = it.w[2], uy = 1.f - wy, uz = 1.f - wz;
+	const float w00 = uy * uz, w10 = wy * uz, w01 = uy * wz, w11 = wy * wz;
+	const float s0 = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, w11 * v[3].x)));
+	const float s1 = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, w11 * v[3].y)));
+	// lane b keeps feature b of its own x plane and receives feature b of the partner's
+	const float mine = b ? s1 : s0, other = n2_pair_swap(b ? s0 : s1);
+	return fmaf(1.f - it.w[0], b ? other : mine, it.w[0] * (b ? mine : other));
+}
 __device__ __forceinline__ void gather_pair(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t b) {
 	const float* q = a.pos + (size_t)i * a.ps;
 	const float p[3] = {q[0], q[a.ds], q[2 * (size_t)a.ds]};
 	float feat = 0.f;
 	if (level < a.lv.active_levels) {  // a switched-off level: zero features
-		const uint32_t res = a.lv.res[level], entries = a.lv.entries[level];
-		const bool hashed = (a.lv.hash_mask >> level) & 1u;
-		uint32_t c[3];
-		float w[3];
-#pragma unroll
-		for (int d = 0; d < 3; ++d) n2_locate(p[d], a.lv.scale[level], w[d], c[d]);
-		const __half2* P = a.table + a.lv.offset[level];
-		float2 v[4];
-#pragma unroll
-		for (uint32_t k = 0; k < 4; ++k) {
-			const uint32_t y = c[1] + (k & 1u), z = c[2] + (k >> 1);
-			const uint32_t at = hashed ? n2_entry<N2_LEVEL_HASH>(entries, res, c[0] + b, y, z) : n2_entry<N2_LEVEL_DENSE>(entries, res, c[0] + b, y, z);
-			v[k] = h2f(*reinterpret_cast<const uint32_t*>(P + at));
-		}
-		const float wy = w[1], wz = w[2], uy = 1.f - wy, uz = 1.f - wz;
-		const float w00 = uy * uz, w10 = wy * uz, w01 = uy * wz, w11 = wy * wz;
-		const float s0 = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, w11 * v[3].x)));
-		const float s1 = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, w11 * v[3].y)));
-		// lane b keeps feature b of its own x plane and receives feature b of the partner's
-		const float mine = b ? s1 : s0, other = n2_pair_swap(b ? s0 : s1);
-		feat = fmaf(1.f - w[0], b ? other : mine, w[0] * (b ? mine : other));
+		PairItem it;
+		pair_fetch(a, level, p, b, it);
+		feat = pair_finish(it, b);
 	}
 	a.sdf_in[(size_t)(3 + 2 * level + b) * a.N + i] = (hf)feat;
 }
@@ -425,6 +437,105 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 	if (i >= a.N || (a.live && i >= *a.live)) return;  // (both lanes of a pair)
 	if (FULL) gather_item(a, level, i, i);
 	else gather_pair(a, level, i, threadIdx.x & 1u);
+}
+
+// ----------------------------------------------------------------------------
+// the SDF net of 32 samples by one wave: lane (n, g) works for sample n
+// ----------------------------------------------------------------------------
+// h: the hidden layer; the result holds rows 4g .. 4g+3 and 8+4g .. 8+4g+3
+__device__ __forceinline__ half8 sdf_net(const hf* F, int lane, const half8 (&xs)[3], half8 (&h)[4]) {
+#pragma unroll
+	for (int mt = 0; mt < 2; ++mt) {
+		float16v acc = zero16();
+#pragma unroll
+		for (int c = 0; c < 3; ++c) acc = N2_MFMA(frag(F, S_W0 + mt * 3 + c, lane), xs[c], acc);
+		relu_pack(acc, h[2 * mt], h[2 * mt + 1]);
+	}
+	float16v out = zero16();
+#pragma unroll
+	for (int c = 0; c < 4; ++c) out = N2_MFMA(frag(F, S_WO + c, lane), h[c], out);
+	return round8(out, 0);
+}
+
+// inference: bias, density and what the caller wants stored of sample `col` (col_raw: its number before clamping)
+__device__ __forceinline__ void store_sdf(const FusedArgs& a, half8 y, uint32_t col, bool valid, uint32_t col_raw, int g) {
+	if (g == 0) {
+		hf s = y[0] + (hf)a.sdf_bias;
+		if (a.density) {
+			const hf is = (hf)__expf((float)(a.variance[0] * (hf)10.0f));
+			const hf x = s * is;
+			const hf sig = (hf)(1.0f / (1.0f + __expf(-(float)x)));
+			s = is * sig * ((hf)1.0f - sig);
+		}
+		y[0] = s;
+		if (a.row0 && col_raw < a.row0_n) a.row0[col] = (float)s;
+	}
+	if (a.sdf_out && valid) {
+		const size_t off4 = (size_t)4u * g * a.N + col;
+#pragma unroll
+		for (int e = 0; e < 4; ++e) {
+			a.sdf_out[(size_t)e * a.N + off4] = y[e];
+			a.sdf_out[(size_t)(8 + e) * a.N + off4] = y[4 + e];
+		}
+	}
+}
+
+// A small query in one launch: a workgroup takes 32 points, wave w gathers levels w and w + 8 (a lane pair per point, as in
+// gather_pair), the features meet in LDS and wave 0 puts them through the net.  Nothing but latency bounds it: the weights'
+// and the positions' loads are under way together, then the gathers of both levels.
+constexpr uint32_t FQ_BLOCK = 512, FQ_POINTS = 32;
+constexpr uint32_t FQ_PITCH = 36;  // halves per point in LDS: an odd multiple of 8 bytes, so that the net's 8-byte reads spread over the banks
+__global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a) {
+	static_assert(FF_LEVELS == 2 * (FQ_BLOCK / 64), "two levels per wave");
+	__shared__ __align__(16) hf F[FF_SDF_COUNT * 512];
+	__shared__ __align__(16) hf X[FQ_POINTS * FQ_PITCH];
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, b = lane & 1u;
+	const uint32_t first = blockIdx.x * FQ_POINTS;
+	auto position = [&](uint32_t k, float (&p)[3]) {
+		const uint32_t i = min(first + k, a.N - 1u);
+		const float* q = a.pos + (size_t)i * a.ps;
+		p[0] = q[0]; p[1] = q[a.ds]; p[2] = q[2 * (size_t)a.ds];
+	};
+	float p[3];
+	position(lane >> 1, p);
+	constexpr uint32_t VALUES = FF_SDF_COUNT * 64, MORE = VALUES - FQ_BLOCK;
+	static_assert(VALUES > FQ_BLOCK && MORE <= FQ_BLOCK, "one fragment value per thread, and some of the threads a second one");
+	const half8 f0 = fused_frag_value(a, threadIdx.x >> 6, lane);
+	half8 f1 = zero8();
+	if (threadIdx.x < MORE) f1 = fused_frag_value(a, (FQ_BLOCK + threadIdx.x) >> 6, lane);
+	PairItem it[2];
+#pragma unroll
+	for (uint32_t k = 0; k < 2; ++k) {
+		const uint32_t level = wave + 8u * k;
+		pair_fetch(a, level < a.n_levels ? level : 0u, p, b, it[k]);
+	}
+	reinterpret_cast<half8*>(F)[threadIdx.x] = f0;
+	if (threadIdx.x < MORE) reinterpret_cast<half8*>(F)[FQ_BLOCK + threadIdx.x] = f1;
+#pragma unroll
+	for (uint32_t k = 0; k < 2; ++k) {
+		const uint32_t level = wave + 8u * k;
+		const float feat = pair_finish(it[k], b);
+		X[(lane >> 1) * FQ_PITCH + 2u * level + b] = level < a.lv.active_levels ? (hf)feat : (hf)0.f;  // (switched off or not there: zero)
+	}
+	__syncthreads();
+	if (wave != 0) return;
+	const uint32_t n = lane & 31u, g = lane >> 5;
+	position(n, p);
+	half8 xs[3], h[4];
+#pragma unroll
+	for (int c = 0; c < 2; ++c) {
+		const hf* q = X + n * FQ_PITCH + 16 * c + 4u * g;
+		const half4v lo = *reinterpret_cast<const half4v*>(q), hi = *reinterpret_cast<const half4v*>(q + 8);
+		xs[c] = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+	}
+	xs[2] = zero8();
+	if (g == 0) {
+#pragma unroll
+		for (int d = 0; d < 3; ++d) xs[2][d] = (hf)p[d] - (hf)0.5f;
+	}
+	const half8 y = sdf_net(F, (int)lane, xs, h);
+	const bool valid = first + n < a.N;
+	store_sdf(a, y, valid ? first + n : a.N - 1u, valid, first + n, (int)g);
 }
 
 // ----------------------------------------------------------------------------
@@ -504,39 +615,11 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 #pragma unroll
 			for (int d = 0; d < 3; ++d) xs[2][d] = (hf)p[d] - (hf)0.5f;
 		}
-		const size_t off4 = (size_t)4u * g * N + col;
 		// ---- SDF net ----
 		half8 h[4];
-#pragma unroll
-		for (int mt = 0; mt < 2; ++mt) {
-			float16v acc = zero16();
-#pragma unroll
-			for (int c = 0; c < 3; ++c) acc = N2_MFMA(frag(F, S_W0 + mt * 3 + c, lane), xs[c], acc);
-			relu_pack(acc, h[2 * mt], h[2 * mt + 1]);
-		}
-		float16v out = zero16();
-#pragma unroll
-		for (int c = 0; c < 4; ++c) out = N2_MFMA(frag(F, S_WO + c, lane), h[c], out);
-		half8 y = round8(out, 0);  // rows 4g .. 4g+3 and 8+4g .. 8+4g+3
+		half8 y = sdf_net(F, lane, xs, h);
 		if (!FULL) {
-			if (g == 0) {
-				hf s = y[0] + (hf)a.sdf_bias;
-				if (a.density) {
-					const hf is = (hf)__expf((float)(a.variance[0] * (hf)10.0f));
-					const hf x = s * is;
-					const hf sig = (hf)(1.0f / (1.0f + __expf(-(float)x)));
-					s = is * sig * ((hf)1.0f - sig);
-				}
-				y[0] = s;
-				if (a.row0 && col_raw < a.row0_n) a.row0[col] = (float)s;
-			}
-			if (a.sdf_out && valid) {
-#pragma unroll
-				for (int e = 0; e < 4; ++e) {
-					a.sdf_out[(size_t)e * N + off4] = y[e];
-					a.sdf_out[(size_t)(8 + e) * N + off4] = y[4 + e];
-				}
-			}
+			store_sdf(a, y, col, valid, col_raw, g);
 			tile_fence();
 			continue;
 		}
@@ -675,6 +758,11 @@ static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream
 	field_gather_kernel<FULL><<<dim3(blocks + (FULL && a.frags ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, tiles, by_xcd ? 1 : 0);
 }
 
+// Up to here a query is one launch.  Beyond it the fragments that every 32 points rebuild from the weights weigh more than the
+// second launch and its wait (device time in a graph, two launches -> one: 64 points 6.2 -> 4.7 us, 1000 6.9 -> 4.9, 4096 7.8 -> 6.5,
+// 8192 9.4 -> 10.2, 16384 13.0 -> 16.6; a call from Python, bound by the host: 1000 points 9.5 -> 7.3, 8192 the same).
+constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 6144;
+
 static uint32_t fused_grid(uint32_t n) {
 	const uint32_t tiles = (n + 31u) / 32u, blocks = (tiles + 3u) / 4u;
 	return blocks < 512u ? blocks : 512u;
@@ -767,6 +855,11 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 	}
 	// points in no particular order: a sample-major walk would touch all tables at once, so the features are gathered level
 	// by level into the network's input rows first
+	if (n <= QUERY_ONE_LAUNCH_MAX) {
+		field_query_kernel<<<dim3((n + FQ_POINTS - 1) / FQ_POINTS), dim3(FQ_BLOCK), 0, s>>>(a);
+		N2_LAUNCH_CHECK();
+		return N2_OK;
+	}
 	a.sdf_in = reinterpret_cast<hf*>(sdf_in);
 	launch_gather<false>(a, *nets.tab, s);
 	N2_LAUNCH_CHECK();

@@ -8,10 +8,7 @@ import torch
 
 from . import capi
 from .capi import N2Error, check, ptr
-
-
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+from .tcnn_api import _stream
 
 
 def _u3(v):

@@ -16,11 +16,7 @@ import torch
 
 from . import capi
 from .capi import check, ptr
-from .tcnn_api import GRAD_ACCUMULATE, GRAD_IGNORE, GRAD_OVERWRITE, LAYOUT_SOA, FullyFusedMLP, GridEncoding
-
-
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+from .tcnn_api import GRAD_ACCUMULATE, GRAD_IGNORE, GRAD_OVERWRITE, LAYOUT_SOA, FullyFusedMLP, GridEncoding, _stream
 
 
 class SdfNet:

@@ -16,7 +16,8 @@ from .capi import (GRAD_ACCUMULATE, GRAD_IGNORE, GRAD_OVERWRITE, LAYOUT_AOS, LAY
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """torch's current stream as a hipStream_t.  (torch.cuda.current_stream() builds a Stream object: 3 us of a small query's 12.)"""
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _positions(xyz):

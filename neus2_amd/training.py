@@ -9,6 +9,7 @@ import torch
 
 from . import capi
 from .capi import N2Error, check, ptr
+from .tcnn_api import _stream as _current_stream
 
 BATCH_SIZE_GRANULARITY = 128  # tcnn::batch_size_granularity, src/testbed_nerf.cu:3429, 3768
 
@@ -147,7 +148,7 @@ class OccupancyGrid:
 
     @staticmethod
     def _stream():
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _current_stream()
 
     def reset(self):
         check(capi.lib().n2_occupancy_reset(self._h, self._stream()), "n2_occupancy_reset")
@@ -240,7 +241,7 @@ class Trainer:
             pass
 
     def _stream(self):
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _current_stream()
 
     def encoding(self):
         """The field's grid encoding (m_nerf_network->encoding(), src/testbed.cu:2643-2646): set_progressive /
