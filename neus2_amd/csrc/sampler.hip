@@ -1,6 +1,7 @@
 // Training-sample generator: pixel pick, ray / unit-cube intersection and the
-// march through the occupancy bitfield.  One wave per ray (see march_wave); three
-// kernels: march and count, exclusive scan in ray order, emit coordinates.
+// march through the occupancy bitfield.  Kernels: prepare (one lane per ray, and the
+// coarse bitfield), march and count (one wave per ray, see march_wave), exclusive scan
+// in ray order, emit coordinates (one wave per ray).
 //
 // Sample positions are part of the bit-exact contract with the CPU oracle, so
 // floating-point contraction is switched off for this file and every fused
@@ -53,19 +54,22 @@ __device__ __forceinline__ float to_next_voxel(const float* pos, const float* di
 	return fmaxf(__fdiv_rn(t, (float)GRIDSIZE), 0.0f);
 }
 
+// One ray as the prepare kernel leaves it: 64 bytes, which a wave that owns the ray reads with one scalar load.
 struct RaySetup {
-	bool alive;
-	float o[3], dir[3], idir[3], startt, target[3];
-	float tmax;  // where the ray leaves the unit cube (below startt: it misses the cube)
+	float o[3], startt;
+	float dir[3], tmax;  // tmax: where the ray leaves the unit cube (below startt: it misses the cube)
+	float idir[3];
+	uint32_t alive;
+	float target[3], unused;
 };
+static_assert(sizeof(RaySetup) == 64, "one scalar load");
 
 // A coarse, dilated copy of the bitfield's first level, rebuilt by every sample generation: bit x + 32 y + 1024 z is set
 // when any of the 4^3 cells of coarse cell (x, y, z) or of its 26 neighbours is occupied.  The march uses it to leave out,
 // for certain, what cannot hold a sample: rays that pass no occupied cell at all, and the part of a ray behind the last
 // occupied cell it can reach.  (In morton order the 64 cells of an aligned 4^3 block are 64 consecutive bits.)
-constexpr uint32_t COARSE = 32, COARSE_WORDS = COARSE * COARSE * COARSE / 32;
-__global__ void __launch_bounds__(256) sampler_coarse_kernel(const uint8_t* __restrict__ bitfield, uint32_t* __restrict__ coarse) {
-	const uint32_t cell = blockIdx.x * 256u + threadIdx.x;  // x + 32 y + 1024 z
+constexpr uint32_t COARSE = 32, COARSE_WORDS = COARSE * COARSE * COARSE / 32, COARSE_BLOCKS = COARSE * COARSE * COARSE / 256;
+__device__ __forceinline__ void build_coarse(const uint8_t* __restrict__ bitfield, uint32_t* __restrict__ coarse, uint32_t cell) {  // cell: x + 32 y + 1024 z
 	const int x = (int)(cell % COARSE), y = (int)((cell / COARSE) % COARSE), z = (int)(cell / (COARSE * COARSE));
 	const unsigned long long* blocks = reinterpret_cast<const unsigned long long*>(bitfield);
 	bool any = false;
@@ -89,7 +93,7 @@ __global__ void __launch_bounds__(256) sampler_coarse_kernel(const uint8_t* __re
 __device__ __forceinline__ RaySetup setup_ray(uint32_t i, uint32_t n_rays, uint32_t n_rays_total, uint32_t seed,
                                               const n2_camera* __restrict__ cams, uint32_t n_images, const float* __restrict__ rgba,
                                               float bg0, float bg1, float bg2) {
-	RaySetup r;
+	RaySetup r{};
 	const uint32_t img = (((i + n_rays_total) * n_images) / n_rays) % n_images;
 	const n2_camera c = cams[img];
 	const float u0 = rand01(seed, i, 0), u1 = rand01(seed, i, 1);
@@ -99,7 +103,7 @@ __device__ __forceinline__ RaySetup setup_ray(uint32_t i, uint32_t n_rays, uint3
 	const uint64_t off = ((uint64_t)c.pixel_offset_hi << 32) | c.pixel_offset_lo;
 	const float4 pix = *reinterpret_cast<const float4*>(rgba + (off + (uint64_t)px + (uint64_t)py * c.resolution[0]) * 4);
 	if (pix.x <= 0.0f && rand01(seed, i, 2) >= 0.9f) {
-		r.alive = false;
+		r.alive = 0u;
 		return r;
 	}
 	const float bg[3] = {bg0, bg1, bg2};
@@ -131,8 +135,24 @@ __device__ __forceinline__ RaySetup setup_ray(uint32_t i, uint32_t n_rays, uint3
 	r.tmax = hit ? tmax : -1.0f;
 	tmin = fmaxf(tmin, 0.0f);
 	r.startt = __fmaf_rn(STEP, rand01(seed, i, 3), tmin);
-	r.alive = true;
+	r.alive = 1u;
 	return r;
+}
+
+// The coarse bitfield (workgroups 0 .. COARSE_BLOCKS - 1), and every ray's setup by one lane.  A setup is some 400 vector
+// instructions, thirteen divisions among them: done by the wave that marches or emits the ray, the same in all 64 lanes, it
+// was a third of both kernels, which are bound by the vector unit.
+__global__ void __launch_bounds__(256) sampler_prepare_kernel(uint32_t n_rays, uint32_t n_rays_total, uint32_t seed, const n2_camera* __restrict__ cams,
+                                                              uint32_t n_images, const float* __restrict__ rgba, float bg0, float bg1, float bg2,
+                                                              const uint8_t* __restrict__ bitfield, uint32_t* __restrict__ coarse,
+                                                              RaySetup* __restrict__ setups, uint32_t* __restrict__ ray_counter) {
+	if (blockIdx.x == 0 && threadIdx.x == 0) *ray_counter = 0u;  // the scan kernel adds the kept rays up
+	if (blockIdx.x < COARSE_BLOCKS) {
+		build_coarse(bitfield, coarse, blockIdx.x * 256u + threadIdx.x);
+		return;
+	}
+	const uint32_t i = (blockIdx.x - COARSE_BLOCKS) * 256u + threadIdx.x;
+	if (i < n_rays) setups[i] = setup_ray(i, n_rays, n_rays_total, seed, cams, n_images, rgba, bg0, bg1, bg2);
 }
 
 // The march of one ray, as the reference writes it: t_0 = startt, every visited step adds STEP to t; at an occupied
@@ -187,7 +207,19 @@ __device__ __forceinline__ float window_t(float t_first, uint32_t lane) {
 	return window_t(t_first, lane, w);
 }
 
-// Returns the number of samples; mask[2 w], mask[2 w + 1]: which steps of window w emitted; t_first[w]: t of its first step.
+// Returns the number of samples.  With samples, mask[2 w], mask[2 w + 1]: which steps of window w emitted; t_first[w]: t of
+// its first step.
+//
+// Jumps.  Between the places where the coarse bitfield has something the walk only hops from voxel to voxel; those windows
+// are left out (a ray through a thin shell: 4 windows instead of 9).  Two things have to come out as the walk would have
+// left them.  t of the landing step: inside a binade it is t_first + s d_e exactly, so a jump stays below the binade's
+// end.  The skip target that the walk arrives with: it lies at most sqrt(3) / 128, eight steps, behind the last step before
+// the landing, and the walk leaves every group of steps for the first of the next group wherever it entered (below), so two
+// groups further on it no longer matters where it came in.  A jump therefore lands JUMP_LEAD steps before the first step
+// that may be occupied and only counts when the landing window is of that regular kind throughout and inside the cube;
+// else the wave goes back and walks.  (A trained field's step, 36096 rays through a thin shell, kernels beside the forward in
+// us: count 112 -> 95, emit 35 -> 23, the forward's first gather beside them 108 -> 77; the step 601 -> 561.)
+constexpr uint32_t JUMP_LEAD = 20, JUMP_MIN = 24;
 __device__ __forceinline__ uint32_t march_wave(const RaySetup& r, const uint8_t* __restrict__ bitfield, const uint32_t* __restrict__ coarse,
                                                uint32_t* __restrict__ mask, float* __restrict__ t_first_out) {
 	const uint32_t lane = threadIdx.x & 63u;
@@ -200,20 +232,49 @@ __device__ __forceinline__ uint32_t march_wave(const RaySetup& r, const uint8_t*
 	// occupied.  No bit set: the ray has no sample.  Else no step behind the last piece with a set bit is occupied: the
 	// serial march would only walk on to the cube's far side without emitting anything, so it ends there with the same
 	// samples.  (A ray outside these assumptions marches all the way.)
-	float t_stop = 3.4e38f;
-	if (coarse != nullptr && r.tmax > r.startt && r.startt >= 0.f && r.tmax - r.startt < 2.0f) {
-		const float piece = (r.tmax - r.startt) * (1.0f / 64.0f);
+	float t_stop = 3.4e38f, piece = 0.f, jump_from = 3.4e38f;  // no jumps from below jump_from
+	unsigned long long maybe = ~0ull;
+	if (r.tmax > r.startt && r.startt >= 0.f && r.tmax - r.startt < 2.0f) {
+		piece = (r.tmax - r.startt) * (1.0f / 64.0f);
 		const float tm = r.startt + ((float)lane + 0.5f) * piece;
 		uint32_t c[3];
 #pragma unroll
 		for (int k = 0; k < 3; ++k) c[k] = (uint32_t)min(max((int)((tm * r.dir[k] + r.o[k]) * (float)COARSE), 0), (int)COARSE - 1);
 		const uint32_t cell = c[0] + COARSE * c[1] + COARSE * COARSE * c[2];
-		const unsigned long long maybe = __ballot((coarse[cell >> 5] >> (cell & 31u)) & 1u);
+		maybe = __ballot((coarse[cell >> 5] >> (cell & 31u)) & 1u);
 		if (maybe == 0ull) return 0u;
 		t_stop = r.startt + ((float)(64 - (int)__clzll((long long)maybe)) + 0.5f) * piece;
+		// a ray that starts outside the cube by a rounding ends there; from a step inside, all steps up to one inside are inside
+		bool in = true;
+#pragma unroll
+		for (int k = 0; k < 3; ++k) {
+			const float q = __fmaf_rn(r.startt, r.dir[k], r.o[k]);
+			in = in && q >= 0.f && q <= 1.f;
+		}
+		if (in) jump_from = -3.4e38f;
 	}
-	for (uint32_t w = 0; w < WINDOWS; ++w) {
+	uint32_t my_lo = 0, my_hi = 0;  // lane w keeps window w's record
+	float my_t = 0.f;
+	uint32_t w = 0;
+	while (w < WINDOWS) {
 		if (t_first > t_stop) break;  // nothing behind this point can emit
+		bool jumped = false;
+		const float t_before = t_first, pending_before = pending;
+		if (t_first >= jump_from && t_first >= 0.125f) {
+			// (half a piece of room on both sides, far more than the rounding of the pieces' ends)
+			const uint32_t at = (uint32_t)fminf(fmaxf(__fdividef(t_first - r.startt, piece) - 0.5f, 0.f), 63.f);
+			const unsigned long long ahead = maybe >> at;  // (the last set piece is not behind `at`, or t_first > t_stop)
+			if (ahead != 0ull) {
+				const float t_next = r.startt + ((float)(at + (uint32_t)__ffsll((long long)ahead) - 1u) - 0.5f) * piece;
+				const float lo = __uint_as_float(__float_as_uint(t_first) & 0x7F800000u);
+				const float far = fminf((t_next - t_first) * (1.0f / STEP) - (float)JUMP_LEAD, (lo + lo - t_first) * (1.0f / STEP) - 2.f);
+				if (far >= (float)JUMP_MIN) {
+					t_first = __fmaf_rn(floorf(far), (lo + STEP) - lo, t_first);
+					pending = -3.4e38f;
+					jumped = true;
+				}
+			}
+		}
 		WindowShape ws;
 		const float t = window_t(t_first, lane, ws);
 		float pos[3];
@@ -268,6 +329,12 @@ __device__ __forceinline__ uint32_t march_wave(const RaySetup& r, const uint8_t*
 				}
 			}
 		}
+		if (jumped && !walked) {
+			t_first = t_before;
+			pending = pending_before;
+			jump_from = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), 63));
+			continue;
+		}
 		while (!walked && cur < 64u) {
 			if (!((m_inside >> cur) & 1ull)) { done = true; break; }
 			if ((m_occ >> cur) & 1ull) {
@@ -288,27 +355,30 @@ __device__ __forceinline__ uint32_t march_wave(const RaySetup& r, const uint8_t*
 				cur = later ? (uint32_t)__ffsll((long long)later) - 1u : 64u;
 			}
 		}
-		if (lane == 0) {
-			mask[2 * w] = (uint32_t)emit;
-			mask[2 * w + 1] = (uint32_t)(emit >> 32);
-			t_first_out[w] = t_first;
+		if (lane == w) {
+			my_lo = (uint32_t)emit;
+			my_hi = (uint32_t)(emit >> 32);
+			my_t = t_first;
 		}
+		++w;
 		if (done) break;
 		// next window starts one step after this window's last one
 		t_first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), 63)) + STEP;
 	}
+	if (j != 0u && lane < w) {
+		mask[2 * lane] = my_lo;
+		mask[2 * lane + 1] = my_hi;
+		t_first_out[lane] = my_t;
+	}
 	return j;
 }
 
-__global__ void __launch_bounds__(64 * RAYS_PER_BLOCK) sampler_count_kernel(uint32_t n_rays, uint32_t n_rays_total, uint32_t seed, const n2_camera* __restrict__ cams,
-                                                            uint32_t n_images, const float* __restrict__ rgba, float bg0, float bg1, float bg2,
+__global__ void __launch_bounds__(64 * RAYS_PER_BLOCK) sampler_count_kernel(uint32_t n_rays, const RaySetup* __restrict__ setups,
                                                             const uint8_t* __restrict__ bitfield, const uint32_t* __restrict__ coarse,
-                                                            uint32_t* __restrict__ counts, uint32_t* __restrict__ mask, float* __restrict__ t_first,
-                                                            uint32_t* __restrict__ ray_counter) {
-	if (blockIdx.x == 0 && threadIdx.x == 0) *ray_counter = 0u;  // the scan kernel adds the kept rays up
-	const uint32_t i = blockIdx.x * RAYS_PER_BLOCK + (threadIdx.x >> 6);
+                                                            uint32_t* __restrict__ counts, uint32_t* __restrict__ mask, float* __restrict__ t_first) {
+	const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * RAYS_PER_BLOCK + (threadIdx.x >> 6)));
 	if (i >= n_rays) return;
-	const RaySetup r = setup_ray(i, n_rays, n_rays_total, seed, cams, n_images, rgba, bg0, bg1, bg2);
+	const RaySetup r = setups[i];
 	const uint32_t n = r.alive ? march_wave(r, bitfield, coarse, mask + (size_t)i * 2 * WINDOWS, t_first + (size_t)i * WINDOWS) : 0u;
 	if ((threadIdx.x & 63u) == 0) counts[i] = n;
 }
@@ -337,7 +407,7 @@ __global__ void __launch_bounds__(1024) sampler_block_totals_kernel(uint32_t n_r
 // of 1024 consecutive rays: it adds up the totals of the blocks before its own and scans its own counts.  The sums never
 // decrease, so once a ray with samples does not fit, no later one does: if the counts before this block fit the budget,
 // every earlier ray with samples was kept; if they do not, none of this block's rays is.  The number of kept rays is added
-// up over the workgroups with an integer atomic (*ray_counter was cleared by the count kernel).
+// up over the workgroups with an integer atomic (*ray_counter was cleared by the prepare kernel).
 __global__ void __launch_bounds__(1024) sampler_scan_kernel(uint32_t n_rays, uint32_t max_samples, const uint32_t* __restrict__ counts,
                                                             const uint32_t* __restrict__ block_sum, const uint32_t* __restrict__ block_nz,
                                                             uint32_t* __restrict__ base, uint32_t* __restrict__ slot,
@@ -378,19 +448,17 @@ __global__ void __launch_bounds__(1024) sampler_scan_kernel(uint32_t n_rays, uin
 
 // Coordinates of the samples the march marked, one wave per ray: lane l of window w is the step at t_first[w] plus l
 // additions of STEP, formed exactly as in the march.
-__global__ void __launch_bounds__(64 * RAYS_PER_BLOCK) sampler_emit_kernel(uint32_t n_rays, uint32_t n_rays_total, uint32_t seed, const n2_camera* __restrict__ cams,
-                                                           uint32_t n_images, const float* __restrict__ rgba, float bg0, float bg1, float bg2,
-                                                           const uint32_t* __restrict__ mask, const float* __restrict__ t_first,
+__global__ void __launch_bounds__(64 * RAYS_PER_BLOCK) sampler_emit_kernel(uint32_t n_rays, const RaySetup* __restrict__ setups, const uint32_t* __restrict__ mask, const float* __restrict__ t_first,
                                                            const uint32_t* __restrict__ counts,
                                                            const uint32_t* __restrict__ base, const uint32_t* __restrict__ slot,
                                                            uint32_t* __restrict__ ray_indices, uint32_t* __restrict__ numsteps,
                                                            float* __restrict__ rgb_target, float* __restrict__ coords,
                                                            float* __restrict__ xyz_soa, uint32_t soa_pitch) {
-	const uint32_t i = blockIdx.x * RAYS_PER_BLOCK + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+	const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * RAYS_PER_BLOCK + (threadIdx.x >> 6))), lane = threadIdx.x & 63u;
 	if (i >= n_rays) return;
 	const uint32_t s = slot[i];
 	if (s == 0xFFFFFFFFu) return;
-	const RaySetup r = setup_ray(i, n_rays, n_rays_total, seed, cams, n_images, rgba, bg0, bg1, bg2);
+	const RaySetup r = setups[i];
 	const uint32_t n = counts[i], first = base[i];
 	if (lane == 0) {
 		ray_indices[s] = i;
@@ -466,25 +534,26 @@ int n2_generate_training_samples_rows(n2_stream_t stream, uint32_t n_rays, uint3
 	uint32_t* base = reinterpret_cast<uint32_t*>(w + up256(4ull * n_rays));
 	uint32_t* slot = reinterpret_cast<uint32_t*>(w + 2 * up256(4ull * n_rays));
 	uint32_t* mask = reinterpret_cast<uint32_t*>(w + 3 * up256(4ull * n_rays));
-	float* t_first = reinterpret_cast<float*>(w + 3 * up256(4ull * n_rays) + up256(4ull * 2 * WINDOWS * n_rays));
+	RaySetup* setups = reinterpret_cast<RaySetup*>(w + 3 * up256(4ull * n_rays) + up256(4ull * 2 * WINDOWS * n_rays));
+	float* t_first = reinterpret_cast<float*>(setups + n_rays);
+	static_assert(sizeof(RaySetup) + 4 * WINDOWS <= 4 * 2 * WINDOWS, "setups and first steps share one part of the workspace");
 	uint32_t* block_sum = reinterpret_cast<uint32_t*>(w + 3 * up256(4ull * n_rays) + 2 * up256(4ull * 2 * WINDOWS * n_rays));
 	uint32_t* block_nz = block_sum + up256(4ull * scan_blocks(n_rays)) / 4;
 	uint32_t* coarse = block_nz + up256(4ull * scan_blocks(n_rays)) / 4;
 	const dim3 grid((n_rays + RAYS_PER_BLOCK - 1) / RAYS_PER_BLOCK), block(64 * RAYS_PER_BLOCK);
 	N2ProfScope prof(N2_PROF_SAMPLER, s);
 	N2_REQUIRE(reinterpret_cast<uintptr_t>(d_bitfield) % 8 == 0, "n2_generate_training_samples: d_bitfield must be 8-byte aligned");
-	sampler_coarse_kernel<<<dim3(COARSE * COARSE * COARSE / 256), dim3(256), 0, s>>>(d_bitfield, coarse);
+	sampler_prepare_kernel<<<dim3(COARSE_BLOCKS + (n_rays + 255u) / 256u), dim3(256), 0, s>>>(n_rays, n_rays_total, seed, d_cameras, n_images, d_rgba, background[0],
+	                                                background[1], background[2], d_bitfield, coarse, setups, d_ray_counter);
 	N2_LAUNCH_CHECK();
-	sampler_count_kernel<<<grid, block, 0, s>>>(n_rays, n_rays_total, seed, d_cameras, n_images, d_rgba, background[0], background[1],
-	                                            background[2], d_bitfield, coarse, counts, mask, t_first, d_ray_counter);
+	sampler_count_kernel<<<grid, block, 0, s>>>(n_rays, setups, d_bitfield, coarse, counts, mask, t_first);
 	N2_LAUNCH_CHECK();
 	sampler_block_totals_kernel<<<dim3(scan_blocks(n_rays)), dim3(1024), 0, s>>>(n_rays, counts, block_sum, block_nz);
 	N2_LAUNCH_CHECK();
 	sampler_scan_kernel<<<dim3(scan_blocks(n_rays)), dim3(1024), 0, s>>>(n_rays, max_samples, counts, block_sum, block_nz, base, slot, d_ray_counter,
 	                                                                 d_sample_counter);
 	N2_LAUNCH_CHECK();
-	sampler_emit_kernel<<<grid, block, 0, s>>>(n_rays, n_rays_total, seed, d_cameras, n_images, d_rgba, background[0], background[1],
-	                                           background[2], mask, t_first, counts, base, slot, d_ray_indices, d_numsteps, d_rgb_target, d_coords,
+	sampler_emit_kernel<<<grid, block, 0, s>>>(n_rays, setups, mask, t_first, counts, base, slot, d_ray_indices, d_numsteps, d_rgb_target, d_coords,
 	                                           d_xyz_rows, max_samples);
 	N2_LAUNCH_CHECK();
 	return N2_OK;
