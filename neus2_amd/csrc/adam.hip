@@ -73,7 +73,11 @@ __device__ __forceinline__ bool adam_summed(const N2SlabReduce& r, const hf* gra
 	return (g >= r.ga && g < r.ga + r.params_a) || (g >= r.gb && g < r.gb + r.params_b) || (r.extra_n > 0 && g == r.extra_out);
 }
 
-template <typename StepT>
+// STREAM: the moments are read and written past the last-level cache.  The optimiser's state is 176 MB of a step's traffic: with
+// the sample rows and the scatter's records of a large batch it does not fit the cache, and what it pushes out the next step's
+// kernels fetch again.  Kernels of a training step in us, plain | moments streamed | master weights too: batch 2^18 389 | 382 | 384,
+// 2^17 266 | 257, 2^16 193 | 185, 2^15 152 | 152, 2^14 128 | 132 | 134 (there the state stays in the cache from step to step).
+template <typename StepT, bool STREAM>
 __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32_t n, uint32_t n_matrix, float loss_scale, float inv_loss_scale, int saturated,
                                                         uint32_t slot, const uint32_t* __restrict__ gate, float* __restrict__ master, hf* __restrict__ params, const hf* __restrict__ grads,
                                                         float* __restrict__ m1, float* __restrict__ m2, StepT* __restrict__ steps, N2SlabReduce sums,
@@ -140,8 +144,8 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 		const bool all_zero = g[0] == (hf)0 && g[1] == (hf)0 && g[2] == (hf)0 && g[3] == (hf)0;
 		if (all_zero && i0 >= n_matrix) return;  // nothing but the gradient is touched
 		float4 w = *reinterpret_cast<float4*>(master + i0);
-		float4 a = *reinterpret_cast<float4*>(m1 + i0);
-		float4 b = *reinterpret_cast<float4*>(m2 + i0);
+		float4 a = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m1 + i0)) : *reinterpret_cast<const float4*>(m1 + i0);
+		float4 b = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m2 + i0)) : *reinterpret_cast<const float4*>(m2 + i0);
 		uint4 t = step_load4(steps + i0);
 		bool any = false;
 		any |= adam_one(i0 + 0, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[0], w.x, a.x, b.x, t.x);
@@ -150,8 +154,13 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 		any |= adam_one(i0 + 3, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[3], w.w, a.w, b.w, t.w);
 		if (!any) return;
 		*reinterpret_cast<float4*>(master + i0) = w;
-		*reinterpret_cast<float4*>(m1 + i0) = a;
-		*reinterpret_cast<float4*>(m2 + i0) = b;
+		if (STREAM) {
+			n2_stream_store(reinterpret_cast<float4*>(m1 + i0), a);
+			n2_stream_store(reinterpret_cast<float4*>(m2 + i0), b);
+		} else {
+			*reinterpret_cast<float4*>(m1 + i0) = a;
+			*reinterpret_cast<float4*>(m2 + i0) = b;
+		}
 		step_store4(steps + i0, t);
 		*reinterpret_cast<half4*>(params + i0) = half4{(hf)w.x, (hf)w.y, (hf)w.z, (hf)w.w};
 	} else {
@@ -179,7 +188,7 @@ N2_API int n2_adam_step(n2_stream_t stream, const n2_adam_config* config, uint32
 int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_t n_params, uint32_t n_matrix_params,
                        float loss_scale, float* d_master, n2_half* d_params, const n2_half* d_gradients, float* d_m1,
                        float* d_m2, void* d_steps, uint32_t steps_bits, const uint32_t* d_gate, const N2SlabReduce* sums, const N2StepEpilogue* epilogue,
-                       hipEvent_t done_event) {
+                       hipEvent_t done_event, bool stream_moments) {
 	N2_REQUIRE(config != nullptr, "n2_adam_step: config is null");
 	if (n_params == 0) return N2_OK;
 	N2_REQUIRE(d_master && d_params && d_gradients && d_m1 && d_m2 && d_steps, "n2_adam_step: null buffer");
@@ -246,21 +255,26 @@ int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_
 	const dim3 grid((quads + 255) / 256 + plan.units + (epi.values ? 1u : 0u));
 	N2_REQUIRE(steps_bits == 32 || steps_bits == 16, "n2_adam_step: step counters of %u bits", steps_bits);
 	N2_REQUIRE(steps_bits == 32 || saturated, "n2_adam_step: 16-bit step counters need betas whose powers underflow within %u steps", ADAM_TABLE);
-	auto launch = [&](auto* steps) {
+	auto launch = [&](auto* steps, auto stream_tag) {
 		using StepT = std::remove_pointer_t<decltype(steps)>;
+		constexpr bool STREAM = decltype(stream_tag)::value;
 		if (done_event != nullptr) {
 			// the event is tied to this launch's own completion: no packet of its own behind the kernel, where an event record
 			// costs the stream about 5 us before its next kernel starts
-			hipExtLaunchKernelGGL(adam_step_kernel<StepT>, grid, dim3(256), 0, s, nullptr, done_event, 0, *config, n_params, n_matrix_params, loss_scale,
+			hipExtLaunchKernelGGL((adam_step_kernel<StepT, STREAM>), grid, dim3(256), 0, s, nullptr, done_event, 0, *config, n_params, n_matrix_params, loss_scale,
 			                      inv_loss_scale, saturated, slot, d_gate, d_master, reinterpret_cast<hf*>(d_params), reinterpret_cast<const hf*>(d_gradients),
 			                      d_m1, d_m2, steps, plan, epi);
 		} else {
-			adam_step_kernel<StepT><<<grid, dim3(256), 0, s>>>(*config, n_params, n_matrix_params, loss_scale, inv_loss_scale, saturated, slot, d_gate, d_master,
+			adam_step_kernel<StepT, STREAM><<<grid, dim3(256), 0, s>>>(*config, n_params, n_matrix_params, loss_scale, inv_loss_scale, saturated, slot, d_gate, d_master,
 				reinterpret_cast<hf*>(d_params), reinterpret_cast<const hf*>(d_gradients), d_m1, d_m2, steps, plan, epi);
 		}
 	};
-	if (steps_bits == 16) launch(static_cast<uint16_t*>(d_steps));
-	else launch(static_cast<uint32_t*>(d_steps));
+	auto with_steps = [&](auto stream_tag) {
+		if (steps_bits == 16) launch(static_cast<uint16_t*>(d_steps), stream_tag);
+		else launch(static_cast<uint32_t*>(d_steps), stream_tag);
+	};
+	if (stream_moments) with_steps(std::true_type{});
+	else with_steps(std::false_type{});
 	N2_LAUNCH_CHECK();
 	return N2_OK;
 }

@@ -197,10 +197,11 @@ int n2_mlp_backward_and_second_order_indexed(n2_mlp_t* mlp, n2_stream_t stream, 
 // d_steps: uint32_t (steps_bits 32) or uint16_t counters (16)
 // epilogue (or null): one more workgroup of the launch does the caller's bookkeeping (slab_reduce.h), gated or not
 // done_event (or null): recorded by the completion of the launch itself (hipExtLaunchKernel's stop event)
+// stream_moments: the moments pass by the last-level cache (for a caller that moves more than the cache holds between two steps)
 int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_t n_params, uint32_t n_matrix_params,
                        float loss_scale, float* d_master, n2_half* d_params, const n2_half* d_gradients, float* d_m1,
                        float* d_m2, void* d_steps, uint32_t steps_bits, const uint32_t* d_gate, const N2SlabReduce* sums = nullptr,
-                       const N2StepEpilogue* epilogue = nullptr, hipEvent_t done_event = nullptr);
+                       const N2StepEpilogue* epilogue = nullptr, hipEvent_t done_event = nullptr, bool stream_moments = false);
 // true when 1 - beta^t is exactly 1 in fp32 for both betas from the end of the kernel's bias-correction table on: the step
 // counters may then be 16 bits wide (steps_bits 16, saturating at 65535) instead of 32
 bool n2_adam_counters_may_saturate(float beta1, float beta2);
@@ -247,3 +248,25 @@ struct N2ProfScope {
 	N2ProfScope(int id_, hipStream_t s_) : id(id_), s(s_) { n2_prof_begin(id, s); }
 	~N2ProfScope() { n2_prof_end(id, s); }
 };
+
+// Streamed access (the nt bit of a load or store): for data that is passed over once and does not come back before more than
+// the 256 MB last-level cache has gone by, so that it does not push out what does.  Where less is in flight the plain access is
+// the faster one: its reader finds the data in that cache.  Each use states where the line lies.
+typedef uint32_t n2_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 n2_stream_load(const float4* p) { return __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const n2_u32x4*>(p))); }
+__device__ __forceinline__ void n2_stream_store(float4* p, float4 v) { __builtin_nontemporal_store(__builtin_bit_cast(n2_u32x4, v), reinterpret_cast<n2_u32x4*>(p)); }
+// three floats at a 12-byte pitch: a point's row of the encoding's Jacobian
+typedef float n2_float3 __attribute__((ext_vector_type(3), aligned(4)));
+template <bool STREAM>
+__device__ __forceinline__ n2_float3 n2_load3(const float* p) {
+	if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const n2_float3*>(p));
+	else return *reinterpret_cast<const n2_float3*>(p);
+}
+template <bool STREAM>
+__device__ __forceinline__ void n2_store3(float* p, n2_float3 v) {
+	if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<n2_float3*>(p));
+	else *reinterpret_cast<n2_float3*>(p) = v;
+}
+// The encoding's Jacobian (384 bytes per point of sixteen levels) is streamed from 64 MiB on.  Forward, scatter and input gradient
+// in us, plain | streamed: 2^18 points (96 MiB) 241 | 226, 2^17 (48 MiB) 126 | 124, 2^16 80 | 83.
+static inline bool n2_jacobian_streams(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (64ull << 20); }

@@ -14,6 +14,10 @@
 
 typedef _Float16 hf;
 
+// From this batch on the optimiser's moments are streamed: sample rows, scatter records and optimiser state of a step are then
+// more than the last-level cache holds (figures at adam_step_kernel)
+constexpr uint32_t STREAM_MOMENTS_BATCH = 1u << 16;
+
 struct n2_trainer {
 	n2_trainer_config cfg;
 	n2_field_t* field;
@@ -403,7 +407,7 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 	epi.copy_src = set.counters; epi.copy_dst = t->counters; epi.copy_n = 2;
 	if (int rc = n2_adam_step_gated(stream, &t->cfg.adam, t->n_params, t->n_matrix_params, t->cfg.loss_scale, t->master, reinterpret_cast<n2_half*>(t->params),
 	                                reinterpret_cast<const n2_half*>(t->grads), t->m1, t->m2, t->steps, t->steps_bits, compacted_counter, &sums, &epi,
-	                                t->side ? t->ev_main : nullptr)) return rc;
+	                                t->side ? t->ev_main : nullptr, T >= STREAM_MOMENTS_BATCH)) return rc;
 	t->ev_main_from_adam = t->side != nullptr;
 	t->optimizer_steps += 1;
 	t->training_step += 1;
