@@ -101,7 +101,7 @@ __device__ __forceinline__ bool n2_xcd_item(const N2XcdPlan& plan, uint32_t tile
 // exchanges its partial sums and lane b finishes feature b.
 constexpr uint32_t FWD_POINTS = GRID_BLOCK / 2;  // points per workgroup and level
 
-template <uint32_t MODE, bool WANT_DYDX>
+template <uint32_t MODE, bool WANT_DYDX, bool STREAM>
 __device__ __forceinline__ void grid_forward_pair(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t b, uint32_t N,
                                                   const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                                   const __half2* __restrict__ params, __half* __restrict__ out,
@@ -113,8 +113,7 @@ __device__ __forceinline__ void grid_forward_pair(const N2LevelTable& tab, uint3
 	if (n2_level_masked(tab, level, i)) {  // both lanes of a pair share i
 		out[row * N + i] = __float2half_rn(0.f);
 		if (WANT_DYDX) {
-			float* j = dy_dx + (row * N + i) * 3;
-			j[0] = 0.f; j[1] = 0.f; j[2] = 0.f;
+			n2_store3<STREAM>(dy_dx + (row * N + i) * 3, n2_float3{0.f, 0.f, 0.f});
 		}
 		return;
 	}
@@ -143,14 +142,13 @@ __device__ __forceinline__ void grid_forward_pair(const N2LevelTable& tab, uint3
 		const float ty_mine = b ? ty.y : ty.x, ty_other = n2_pair_swap(b ? ty.x : ty.y);
 		const float tz_mine = b ? tz.y : tz.x, tz_other = n2_pair_swap(b ? tz.x : tz.y);
 		const float w_mine = b ? wx : ux, w_other = b ? ux : wx;
-		float* j = dy_dx + (row * N + i) * 3;
-		j[0] = (s_hi - s_lo) * scale;
-		j[1] = fmaf(w_mine, ty_mine, w_other * ty_other) * scale;
-		j[2] = fmaf(w_mine, tz_mine, w_other * tz_other) * scale;
+		n2_store3<STREAM>(dy_dx + (row * N + i) * 3, n2_float3{(s_hi - s_lo) * scale, fmaf(w_mine, ty_mine, w_other * ty_other) * scale,
+		                                                       fmaf(w_mine, tz_mine, w_other * tz_other) * scale});
 	}
 }
 
-template <bool WANT_DYDX>
+// STREAM: dy_dx is written past the last-level cache (n2_jacobian_streams)
+template <bool WANT_DYDX, bool STREAM>
 __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable tab, N2XcdPlan plan, uint32_t N, uint32_t tiles,
                                                                   const float* __restrict__ xyz, uint32_t point_stride,
                                                                   uint32_t dim_stride, const __half2* __restrict__ params,
@@ -159,7 +157,7 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable t
 	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_xcd_level_tile(tab.n_levels, tiles, level, tile))) return;
 	const uint32_t i = tile * FWD_POINTS + (threadIdx.x >> 1), b = threadIdx.x & 1u;
 	if (i >= N) return;  // both lanes of a pair share i, so pairs leave together
-#define CALL(M) grid_forward_pair<M, WANT_DYDX>(tab, level, i, b, N, xyz, point_stride, dim_stride, params, out, dy_dx)
+#define CALL(M) grid_forward_pair<M, WANT_DYDX, STREAM>(tab, level, i, b, N, xyz, point_stride, dim_stride, params, out, dy_dx)
 	N2_DISPATCH_MODE(tab.mode[level], CALL)
 #undef CALL
 }
@@ -327,7 +325,10 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_scatter_kernel(N2LevelTable t
 #undef CALL
 }
 
-// ... and input gradient dL_dx[d][i] = sum_k dL_dy[k][i] * dy_dx[k][i][d]
+// ... and input gradient dL_dx[d][i] = sum_k dL_dy[k][i] * dy_dx[k][i][d].  Bound by HBM on large batches and by latency on small
+// ones: eight rows' loads are under way together (one row at a time: 10.5 us for 5003 points, 23.5 for 2^18; now 4.4 and 20.3).
+constexpr uint32_t BWD_IN_ROWS = 8;
+template <bool STREAM>
 __global__ void __launch_bounds__(GRID_BLOCK) grid_backward_input_kernel(uint32_t N, uint32_t n_out,
                                                                          const __half* __restrict__ dL_dy,
                                                                          const float* __restrict__ dy_dx,
@@ -335,12 +336,25 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_backward_input_kernel(uint32_
 	const uint32_t i = blockIdx.x * GRID_BLOCK + threadIdx.x;
 	if (i >= N) return;
 	float r0 = 0.f, r1 = 0.f, r2 = 0.f;
-	for (uint32_t k = 0; k < n_out; ++k) {
-		const float g = __half2float(dL_dy[(size_t)k * N + i]);
-		const float* j = dy_dx + ((size_t)k * N + i) * 3;
-		r0 = fmaf(g, j[0], r0);
-		r1 = fmaf(g, j[1], r1);
-		r2 = fmaf(g, j[2], r2);
+	for (uint32_t k0 = 0; k0 < n_out; k0 += BWD_IN_ROWS) {
+		__half g[BWD_IN_ROWS];
+		n2_float3 j[BWD_IN_ROWS];
+#pragma unroll
+		for (uint32_t u = 0; u < BWD_IN_ROWS; ++u) {
+			const size_t at = (size_t)min(k0 + u, n_out - 1u) * N + i;
+			g[u] = dL_dy[at];
+			j[u] = n2_load3<STREAM>(dy_dx + at * 3);
+		}
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (uint32_t u = 0; u < BWD_IN_ROWS; ++u) {
+			if (k0 + u < n_out) {
+				const float f = __half2float(g[u]);
+				r0 = fmaf(f, j[u].x, r0);
+				r1 = fmaf(f, j[u].y, r1);
+				r2 = fmaf(f, j[u].z, r2);
+			}
+		}
 	}
 	dL_dx[i] = r0;
 	dL_dx[(size_t)N + i] = r1;
@@ -1136,13 +1150,10 @@ N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_x
 	const uint32_t tiles = (n_points + FWD_POINTS - 1) / FWD_POINTS;
 	plan.begin[N_XCD] = 0;
 	const dim3 grid_dim(grid->costs_set ? make_xcd_plan(grid, tiles, plan) * N_XCD : n2_xcd_blocks(grid->tab.n_levels, tiles)), block(GRID_BLOCK);
-	if (d_dy_dx) {
-		grid_forward_kernel<true><<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride,
-			dim_stride, grid->params, reinterpret_cast<__half*>(d_out), d_dy_dx);
-	} else {
-		grid_forward_kernel<false><<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride,
-			dim_stride, grid->params, reinterpret_cast<__half*>(d_out), nullptr);
-	}
+	const bool streams = n2_jacobian_streams(n_points, grid->tab.n_levels * grid->n_features);
+	auto* const kernel = !d_dy_dx ? grid_forward_kernel<false, false> : streams ? grid_forward_kernel<true, true> : grid_forward_kernel<true, false>;
+	kernel<<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride, dim_stride, grid->params,
+	                                                  reinterpret_cast<__half*>(d_out), d_dy_dx);
 	N2_LAUNCH_CHECK();
 	return N2_OK;
 }
@@ -1384,8 +1395,9 @@ N2_API int n2_grid_backward(n2_grid_t* grid, n2_stream_t stream, const float* d_
 		                            nullptr, grid->grads, nullptr, mode == N2_GRAD_ACCUMULATE)) return rc;
 	}
 	if (d_dL_dx) {
-		grid_backward_input_kernel<<<dim3(n_tiles(n_points)), dim3(GRID_BLOCK), 0, s>>>(
-			n_points, grid->tab.n_levels * grid->n_features, reinterpret_cast<const __half*>(d_dL_dy), d_dy_dx, d_dL_dx);
+		const uint32_t rows = grid->tab.n_levels * grid->n_features;
+		auto* const kernel = n2_jacobian_streams(n_points, rows) ? grid_backward_input_kernel<true> : grid_backward_input_kernel<false>;
+		kernel<<<dim3(n_tiles(n_points)), dim3(GRID_BLOCK), 0, s>>>(n_points, rows, reinterpret_cast<const __half*>(d_dL_dy), d_dy_dx, d_dL_dx);
 		N2_LAUNCH_CHECK();
 	}
 	return N2_OK;
