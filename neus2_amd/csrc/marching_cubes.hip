@@ -106,8 +106,8 @@ __device__ const McTable MC_TABLE = mc_build_table();
 //   mc_emit     one wave per word that owns something: vertices and triangles
 //   mc_normals  one lane per vertex: the sum over the triangles of the four cubes round its edge
 // Rows are padded to whole words, so a word's neighbours in y and z are words too and no mask crosses a row.
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 90 (6.0 TB/s), count 29, scan 9, emit 46, normals 34, with
-// the host's wait for the totals 238 in all.  Deciding every point from the four rows of the density itself took 242 for the
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 29, scan 9, emit 46, normals 34, with
+// the host's wait for the totals 227 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
 struct McGrid {
@@ -130,6 +130,10 @@ struct alignas(64) McRecord {
 
 constexpr uint32_t MC_BITS_WORDS = 16;  // words a wave forms at a time: 16 loads in flight per lane
 
+// STREAM: the density is read past the last-level cache; the lattice is larger than that and would only push itself out (512^3,
+// 512 MiB: 92 -> 80 us; 384^3, 216 MiB, which stays there for the emitting kernel: 32 -> 34).
+constexpr uint64_t MC_STREAM_BYTES = 256ull << 20;
+template <bool STREAM>
 __global__ void __launch_bounds__(MC_BLOCK) mc_bits_kernel(McGrid g, const float* __restrict__ density, mc_word* __restrict__ bits) {
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (MC_BLOCK / 64) + (threadIdx.x >> 6));
@@ -140,7 +144,8 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_bits_kernel(McGrid g, const float
 #pragma unroll
 	for (uint32_t k = 0; k < MC_BITS_WORDS; ++k) {
 		const uint32_t x = col * 64u + lane;
-		v[k] = (w0 + k < g.n_words && x < g.rx) ? density[(uint64_t)row * g.rx + x] : -INFINITY;
+		const float* at = density + (uint64_t)row * g.rx + x;
+		v[k] = (w0 + k < g.n_words && x < g.rx) ? (STREAM ? __builtin_nontemporal_load(at) : *at) : -INFINITY;
 		if (++col == g.row_words) { col = 0; ++row; }
 	}
 	mc_word mine = 0;
@@ -555,7 +560,8 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	mc_word* bits = reinterpret_cast<mc_word*>(b + c.bits);
 	uint2* blocks = reinterpret_cast<uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
-	mc_bits_kernel<<<mgrid(((uint64_t)c.n_words + MC_BITS_WORDS - 1) / MC_BITS_WORDS * 64u), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits);
+	auto* const bits_kernel = 4 * n >= MC_STREAM_BYTES ? mc_bits_kernel<true> : mc_bits_kernel<false>;
+	bits_kernel<<<mgrid(((uint64_t)c.n_words + MC_BITS_WORDS - 1) / MC_BITS_WORDS * 64u), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits);
 	N2_LAUNCH_CHECK();
 	mc_count_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
 	N2_LAUNCH_CHECK();

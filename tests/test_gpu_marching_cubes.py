@@ -133,3 +133,15 @@ def test_sdf_lattice_and_mesh_of_the_initial_sphere(oracle, tmp_path):
         else:
             assert text[0] == "ply" and f"element vertex {len(vv)}" in text and f"element face {len(tt)}" in text
             assert len(text) == text.index("end_header") + 1 + len(vv) + len(tt)
+
+
+def test_lattice_larger_than_the_last_level_cache():
+    """A lattice whose density is streamed (512 x 512 x 256 points) holds the mesh of the smaller lattice it contains."""
+    from neus2_amd.mesh import marching_cubes
+    x, y, z = ((torch.arange(r, device="cuda") - c) / 512 for r, c in ((512, 250.3), (512, 260.1), (256, 62.4)))
+    d = 0.1 - (x[None, None, :] ** 2 + y[None, :, None] ** 2 + z[:, None, None] ** 2).sqrt()  # all of it below plane 128
+    big = marching_cubes(d.contiguous(), 0.0, (0, 0, 0), (1, 1, 0.5))
+    small = marching_cubes(d[:128].contiguous(), 0.0, (0, 0, 0), (1, 1, 0.25))
+    assert big[0].shape[0] > 10000
+    for a, b in zip(big, small):
+        assert torch.equal(a, b)
