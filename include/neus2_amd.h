@@ -418,6 +418,11 @@ int n2_sdf_eikonal_loss(n2_stream_t stream, uint32_t n, uint32_t encoding_width,
                         const n2_half* d_dsdf_dinput, const float* d_normal_encoding, float* d_normal, float ek_weight, float loss_scale, n2_half* d_dL_doutput,
                         float* d_dL_dnormal, n2_half* d_second_order_input, float* d_loss, void* d_workspace, uint64_t workspace_bytes,
                         const float* d_dy_dx);
+/* n2_grid_backward for d_normal_encoding (mode IGNORE) followed by n2_sdf_eikonal_loss with d_dy_dx, in one pass over the Jacobian */
+int n2_sdf_normals_and_eikonal_loss(n2_stream_t stream, uint32_t n, uint32_t encoding_width, uint32_t input_width, const n2_half* d_sdf_output,
+                                    const n2_half* d_dsdf_dinput, const float* d_dy_dx, float* d_normal, float ek_weight, float loss_scale,
+                                    n2_half* d_dL_doutput, float* d_dL_dnormal, n2_half* d_second_order_input, float* d_loss, void* d_workspace,
+                                    uint64_t workspace_bytes);
 
 /* ------------------------------------------------------------------------
  * Adam on fp32 master weights with an fp16 working copy: tcnn's Adam as the

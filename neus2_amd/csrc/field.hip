@@ -636,6 +636,41 @@ __global__ void __launch_bounds__(FB) sdf_pack_input_kernel(const float* __restr
 	for (uint32_t r = first_pad; r < in_w; ++r) input[(size_t)r * N + i] = (hf)0;
 }
 
+// One point: its normal from the encoding's part `enc`, its term of the loss, and what the backward takes but for the
+// encoding's rows; x: d loss / d normal.
+__device__ __forceinline__ float eikonal_point(uint32_t N, uint32_t i, uint32_t first_pad, uint32_t in_w, const hf* __restrict__ sdf_out, const hf* __restrict__ g,
+                                               const float (&enc)[3], float* __restrict__ normal, float ek_weight, float scale, hf* __restrict__ dL_dy,
+                                               float* __restrict__ v, hf* __restrict__ v_in, float (&x)[3]) {
+	const float sdf = (float)sdf_out[i];
+	float nrm[3], len2 = 0.f;
+#pragma unroll
+	for (int d = 0; d < 3; ++d) {
+		nrm[d] = enc[d] + (float)g[(size_t)d * N + i];  // add_positions_view: the direct coordinate rows
+		normal[(size_t)d * N + i] = nrm[d];
+		len2 = fmaf(nrm[d], nrm[d], len2);
+	}
+	const float len = fmaxf(sqrtf(len2), 1e-12f);
+	dL_dy[i] = (hf)((sdf > 0.f ? 1.f : sdf < 0.f ? -1.f : 0.f) * scale);
+	for (uint32_t r = 1; r < 16; ++r) dL_dy[(size_t)r * N + i] = (hf)0;
+	const float k = 2.f * ek_weight * (len - 1.f) / len * scale;
+#pragma unroll
+	for (int d = 0; d < 3; ++d) {
+		x[d] = nrm[d] * k;
+		v[(size_t)d * N + i] = x[d];
+		v_in[(size_t)d * N + i] = (hf)x[d];
+	}
+	for (uint32_t r = first_pad; r < in_w; ++r) v_in[(size_t)r * N + i] = (hf)0;
+	return fabsf(sdf) + ek_weight * (len - 1.f) * (len - 1.f);
+}
+// the workgroup's part of the loss
+__device__ __forceinline__ void eikonal_part(float term, float* part, float* __restrict__ parts) {
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) term += __shfl_xor(term, o);
+	if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = term;
+	__syncthreads();
+	if (threadIdx.x == 0) parts[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 __global__ void __launch_bounds__(FB) sdf_eikonal_loss_kernel(uint32_t N, uint32_t first_pad, uint32_t in_w, const hf* __restrict__ sdf_out,
                                                               const hf* __restrict__ g, const float* __restrict__ normal_enc, float* __restrict__ normal, float ek_weight, float scale,
                                                               hf* __restrict__ dL_dy, float* __restrict__ v, hf* __restrict__ v_in,
@@ -644,26 +679,9 @@ __global__ void __launch_bounds__(FB) sdf_eikonal_loss_kernel(uint32_t N, uint32
 	const uint32_t i = blockIdx.x * FB + threadIdx.x;
 	float term = 0.f;
 	if (i < N) {
-		const float sdf = (float)sdf_out[i];
-		float nrm[3], len2 = 0.f;
-#pragma unroll
-		for (int d = 0; d < 3; ++d) {
-			nrm[d] = normal_enc[(size_t)d * N + i] + (float)g[(size_t)d * N + i];  // add_positions_view: the direct coordinate rows
-			normal[(size_t)d * N + i] = nrm[d];
-			len2 = fmaf(nrm[d], nrm[d], len2);
-		}
-		const float len = fmaxf(sqrtf(len2), 1e-12f);
-		term = fabsf(sdf) + ek_weight * (len - 1.f) * (len - 1.f);
-		dL_dy[i] = (hf)((sdf > 0.f ? 1.f : sdf < 0.f ? -1.f : 0.f) * scale);
-		for (uint32_t r = 1; r < 16; ++r) dL_dy[(size_t)r * N + i] = (hf)0;
-		const float k = 2.f * ek_weight * (len - 1.f) / len * scale;
+		const float enc[3] = {normal_enc[i], normal_enc[(size_t)N + i], normal_enc[(size_t)2 * N + i]};
 		float x[3];
-#pragma unroll
-		for (int d = 0; d < 3; ++d) {
-			x[d] = nrm[d] * k;  // d loss / d normal
-			v[(size_t)d * N + i] = x[d];
-			v_in[(size_t)d * N + i] = (hf)x[d];
-		}
+		term = eikonal_point(N, i, first_pad, in_w, sdf_out, g, enc, normal, ek_weight, scale, dL_dy, v, v_in, x);
 		if (dy_dx) {
 			// the encoding's dL_ddLdoutput = J v from the Jacobian the forward saved ([row][N][3]), eight rows' loads in flight
 			const uint32_t enc_w = first_pad - 3;
@@ -679,13 +697,61 @@ __global__ void __launch_bounds__(FB) sdf_eikonal_loss_kernel(uint32_t N, uint32
 					if (r0 + u < enc_w) v_in[(size_t)(3 + r0 + u) * N + i] = (hf)fmaf(j[u][0], x[0], fmaf(j[u][1], x[1], j[u][2] * x[2]));
 			}
 		}
-		for (uint32_t r = first_pad; r < in_w; ++r) v_in[(size_t)r * N + i] = (hf)0;
 	}
+	eikonal_part(term, part, parts);
+}
+
+// The same with the normals' encoding part formed here, J^T g from the Jacobian, whose rows a lane holds in registers for
+// J v: the Jacobian (384 bytes per point) is read once instead of twice.  Bound by that read, so all of it is under way at once:
+// 2^18 points 40.5 us (input gradient 17.6, loss 22.9) -> 32 us (46 where the compiler was left to spread the loads).
+// FITS: the encoding has at most EIK_ROWS rows; else they are read eight at a time, twice.
+constexpr uint32_t EIK_ROWS = 32;
+template <bool STREAM, uint32_t ROWS>
+__device__ __forceinline__ void eikonal_rows(n2_float3 (&j)[ROWS], const float* __restrict__ dy_dx, uint32_t r0, uint32_t enc_w, uint32_t N, uint32_t i) {
 #pragma unroll
-	for (int o = 32; o > 0; o >>= 1) term += __shfl_xor(term, o);
-	if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = term;
-	__syncthreads();
-	if (threadIdx.x == 0) parts[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+	for (uint32_t u = 0; u < ROWS; ++u) j[u] = n2_load3<STREAM>(dy_dx + ((size_t)min(r0 + u, enc_w - 1u) * N + i) * 3);
+}
+template <bool STREAM, bool FITS>
+__global__ void __launch_bounds__(FB, 3) sdf_normals_eikonal_kernel(uint32_t N, uint32_t first_pad, uint32_t in_w, const hf* __restrict__ sdf_out,
+                                                                    const hf* __restrict__ g, float* __restrict__ normal, float ek_weight, float scale,
+                                                                    hf* __restrict__ dL_dy, float* __restrict__ v, hf* __restrict__ v_in,
+                                                                    float* __restrict__ parts, const float* __restrict__ dy_dx) {
+	constexpr uint32_t ROWS = FITS ? EIK_ROWS : 8;
+	__shared__ float part[FB / 64];
+	const uint32_t i = blockIdx.x * FB + threadIdx.x, enc_w = first_pad - 3;
+	float term = 0.f;
+	if (i < N) {
+		n2_float3 j[ROWS];
+		float enc[3] = {0.f, 0.f, 0.f}, x[3];
+		uint32_t r0 = 0;
+		do {
+			hf f[ROWS];
+			eikonal_rows<STREAM>(j, dy_dx, r0, enc_w, N, i);
+#pragma unroll
+			for (uint32_t u = 0; u < ROWS; ++u) f[u] = g[(size_t)(3 + min(r0 + u, enc_w - 1u)) * N + i];
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (uint32_t u = 0; u < ROWS; ++u) {
+				if (r0 + u < enc_w) {
+					enc[0] = fmaf((float)f[u], j[u].x, enc[0]);
+					enc[1] = fmaf((float)f[u], j[u].y, enc[1]);
+					enc[2] = fmaf((float)f[u], j[u].z, enc[2]);
+				}
+			}
+			r0 += ROWS;
+		} while (!FITS && r0 < enc_w);
+		term = eikonal_point(N, i, first_pad, in_w, sdf_out, g, enc, normal, ek_weight, scale, dL_dy, v, v_in, x);
+		r0 = 0;
+		do {
+			if (!FITS) eikonal_rows<STREAM>(j, dy_dx, r0, enc_w, N, i);
+#pragma unroll
+			for (uint32_t u = 0; u < ROWS; ++u) {
+				if (r0 + u < enc_w) v_in[(size_t)(3 + r0 + u) * N + i] = (hf)fmaf(j[u].x, x[0], fmaf(j[u].y, x[1], j[u].z * x[2]));
+			}
+			r0 += ROWS;
+		} while (!FITS && r0 < enc_w);
+	}
+	eikonal_part(term, part, parts);
 }
 
 // loss = sum of the workgroups' partial sums / N, in a fixed order
@@ -730,6 +796,30 @@ N2_API int n2_sdf_eikonal_loss(n2_stream_t stream, uint32_t n, uint32_t encoding
 	                                                      reinterpret_cast<const hf*>(d_dsdf_dinput), d_normal_encoding, d_normal, ek_weight, loss_scale / (float)n,
 	                                                      reinterpret_cast<hf*>(d_dL_doutput), d_dL_dnormal, reinterpret_cast<hf*>(d_second_order_input), parts,
 	                                                      d_dy_dx);
+	N2_LAUNCH_CHECK();
+	sdf_loss_sum_kernel<<<dim3(1), dim3(256), 0, s>>>(parts, fgrid(n).x, 1.f / (float)n, d_loss);
+	N2_LAUNCH_CHECK();
+	return N2_OK;
+}
+
+N2_API int n2_sdf_normals_and_eikonal_loss(n2_stream_t stream, uint32_t n, uint32_t encoding_width, uint32_t input_width, const n2_half* d_sdf_output,
+                                           const n2_half* d_dsdf_dinput, const float* d_dy_dx, float* d_normal, float ek_weight, float loss_scale,
+                                           n2_half* d_dL_doutput, float* d_dL_dnormal, n2_half* d_second_order_input, float* d_loss, void* d_workspace,
+                                           uint64_t workspace_bytes) {
+	const char* fn = "n2_sdf_normals_and_eikonal_loss";
+	N2_REQUIRE(n > 0, "%s: empty batch", fn);
+	N2_REQUIRE(d_sdf_output && d_dsdf_dinput && d_dy_dx && d_normal && d_dL_doutput && d_dL_dnormal && d_second_order_input && d_loss && d_workspace,
+	           "%s: null buffer", fn);
+	N2_REQUIRE(encoding_width >= 1 && input_width >= 3 + encoding_width && input_width <= 64, "%s: input width %u does not hold 3 + %u rows", fn, input_width, encoding_width);
+	N2_REQUIRE(workspace_bytes >= n2_sdf_eikonal_workspace_bytes(n), "%s: workspace of %llu bytes, %llu needed", fn, (unsigned long long)workspace_bytes,
+	           (unsigned long long)n2_sdf_eikonal_workspace_bytes(n));
+	hipStream_t s = n2_stream(stream);
+	float* parts = reinterpret_cast<float*>(d_workspace);
+	auto* const kernel = encoding_width > EIK_ROWS ? sdf_normals_eikonal_kernel<false, false>
+	                     : n2_jacobian_streams(n, encoding_width) ? sdf_normals_eikonal_kernel<true, true> : sdf_normals_eikonal_kernel<false, true>;
+	kernel<<<fgrid(n), dim3(FB), 0, s>>>(n, 3 + encoding_width, input_width, reinterpret_cast<const hf*>(d_sdf_output), reinterpret_cast<const hf*>(d_dsdf_dinput),
+	                                     d_normal, ek_weight, loss_scale / (float)n, reinterpret_cast<hf*>(d_dL_doutput), d_dL_dnormal,
+	                                     reinterpret_cast<hf*>(d_second_order_input), parts, d_dy_dx);
 	N2_LAUNCH_CHECK();
 	sdf_loss_sum_kernel<<<dim3(1), dim3(256), 0, s>>>(parts, fgrid(n).x, 1.f / (float)n, d_loss);
 	N2_LAUNCH_CHECK();

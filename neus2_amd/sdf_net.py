@@ -16,7 +16,7 @@ import torch
 
 from . import capi
 from .capi import check, ptr
-from .tcnn_api import GRAD_ACCUMULATE, GRAD_IGNORE, GRAD_OVERWRITE, LAYOUT_SOA, FullyFusedMLP, GridEncoding, _stream
+from .tcnn_api import GRAD_OVERWRITE, LAYOUT_SOA, FullyFusedMLP, GridEncoding, _stream
 
 
 class SdfNet:
@@ -38,7 +38,7 @@ class SdfNet:
             f = lambda rows: torch.empty((rows, n), dtype=torch.float32, device=device)
             self._inp, self._g, self._y, self._dL_dy, self._v_in, self._d_inp = h(self.in_w), h(self.in_w), h(16), h(16), h(self.in_w), h(self.in_w)
             self._dy_dx = torch.empty((self.enc_w, n, 3), dtype=torch.float32, device=device)
-            self._normal_enc, self._normal, self._v = f(3), f(3), f(3)
+            self._normal, self._v = f(3), f(3)
             self._loss = torch.empty(1, dtype=torch.float32, device=device)
             nb = int(capi.lib().n2_sdf_eikonal_workspace_bytes(C.c_uint32(n)))
             self._ws = torch.empty(nb, dtype=torch.uint8, device=device)
@@ -59,20 +59,18 @@ class SdfNet:
         check(L.n2_grid_forward(self.grid._h, s, ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), ptr(enc), ptr(self._dy_dx)), "n2_grid_forward")
         check(L.n2_mlp_forward_and_input_gradient(self.mlp._h, s, C.c_uint32(0), ptr(inp), C.c_uint32(n), ptr(y), C.c_int(LAYOUT_SOA), ptr(g)),
               "n2_mlp_forward_and_input_gradient")
-        # encoding backward of d sdf / d encoding without parameter gradients: J^T g (nerf_network.h:230-234)
-        check(L.n2_grid_backward(self.grid._h, s, ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), ptr(g[3:3 + self.enc_w]), ptr(self._dy_dx),
-                                 ptr(self._normal_enc), C.c_int(GRAD_IGNORE)), "n2_grid_backward")
         ctx = dict(x=x, inp=inp, dy_dx=self._dy_dx, y=y, g=g, sdf=y[0], normal=self._normal, loss=self._loss)
         self._eikonal(ctx, ek_weight, loss_scale)
         return ctx
 
     def _eikonal(self, ctx, ek_weight, loss_scale):
         n = ctx["x"].shape[1]
-        check(capi.lib().n2_sdf_eikonal_loss(_stream(), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), ptr(ctx["y"]), ptr(ctx["g"]),
-                                             ptr(self._normal_enc), ptr(self._normal), C.c_float(ek_weight), C.c_float(loss_scale), ptr(self._dL_dy),
-                                             ptr(self._v), ptr(self._v_in), ptr(self._loss), ptr(self._ws), C.c_uint64(self._ws_bytes),
-                                             ptr(ctx["dy_dx"])),
-              "n2_sdf_eikonal_loss")
+        # normals: encoding backward of d sdf / d encoding without parameter gradients, J^T g (nerf_network.h:230-234)
+        check(capi.lib().n2_sdf_normals_and_eikonal_loss(_stream(), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), ptr(ctx["y"]),
+                                                         ptr(ctx["g"]), ptr(ctx["dy_dx"]), ptr(self._normal), C.c_float(ek_weight),
+                                                         C.c_float(loss_scale), ptr(self._dL_dy), ptr(self._v), ptr(self._v_in), ptr(self._loss),
+                                                         ptr(self._ws), C.c_uint64(self._ws_bytes)),
+              "n2_sdf_normals_and_eikonal_loss")
         ctx["weights"] = (ek_weight, loss_scale)
 
     def loss_backward(self, ctx, ek_weight=0.1, loss_scale=128.0):
@@ -81,14 +79,13 @@ class SdfNet:
         x, inp, g, n = ctx["x"], ctx["inp"], ctx["g"], ctx["x"].shape[1]
         if ctx["weights"] != (ek_weight, loss_scale):
             self._eikonal(ctx, ek_weight, loss_scale)
-        # first order through the MLP, then both orders through the grid in one pass; the grid's dL_ddLdoutput (rows 3.. of
-        # the MLP's second-order input) was already formed from the saved Jacobian by n2_sdf_eikonal_loss
-        check(L.n2_mlp_backward(self.mlp._h, s, ptr(inp), C.c_uint32(n), ptr(self._dL_dy), C.c_int(LAYOUT_SOA), ptr(self._d_inp), C.c_int(GRAD_OVERWRITE)),
-              "n2_mlp_backward")
+        # both orders through the MLP in one pass (the second's first-order output gradient was e_0), then both through the grid;
+        # the grid's dL_ddLdoutput (rows 3.. of the MLP's second-order input) was already formed from the saved Jacobian with
+        # the loss
+        check(L.n2_mlp_backward_and_second_order(self.mlp._h, s, ptr(inp), C.c_uint32(n), ptr(self._dL_dy), C.c_int(LAYOUT_SOA), ptr(self._d_inp),
+                                                 ptr(self._v_in), None, C.c_int(GRAD_OVERWRITE)),
+              "n2_mlp_backward_and_second_order")
         check(L.n2_grid_backward_fused(self.grid._h, s, ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), ptr(self._d_inp[3:3 + self.enc_w]),
                                        ptr(self._v), ptr(g[3:3 + self.enc_w]), None, C.c_int(GRAD_OVERWRITE)),
               "n2_grid_backward_fused")
-        # second order through the MLP: its first-order output gradient was e_0
-        check(L.n2_mlp_backward_backward_input(self.mlp._h, s, ptr(inp), C.c_uint32(n), ptr(self._v_in), None, None, C.c_int(GRAD_ACCUMULATE)),
-              "n2_mlp_backward_backward_input")
         return self._loss

@@ -42,3 +42,42 @@ def test_sdf_eikonal_step_matches_oracle(oracle, kind):
     for l in range(16):
         a, b = int(ref["offset"][l]) * 2, int(ref["offset"][l + 1]) * 2
         assert rel_l2(got[a:b], ref["grid_grad"][a:b]) < 5e-3, (l, rel_l2(got[a:b], ref["grid_grad"][a:b]))
+
+
+@pytest.mark.parametrize("n_levels,n", [(16, 1), (16, 255), (16, 5003), (3, 257), (13, 1000), (20, 777), (16, 180000)])
+def test_normals_and_loss_in_one_pass_equal_the_two_calls(n_levels, n):
+    """n2_sdf_normals_and_eikonal_loss against n2_grid_backward and n2_sdf_eikonal_loss, bit for bit: fewer rows than a lane
+    holds at once, more (20 levels), and a Jacobian that is streamed (180000 points)."""
+    import ctypes as C
+    from neus2_amd import capi
+    from neus2_amd.capi import check, ptr
+    from neus2_amd.tcnn_api import GRAD_IGNORE, GridEncoding, _stream
+    L = capi.lib()
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    enc = GridEncoding(n_levels, 2, 14, 16, 1.3)
+    P = (torch.randn(enc.n_params(), device="cuda", generator=gen) * 0.01).half()
+    enc.set_params(P, None)
+    x = torch.rand((3, n), device="cuda", generator=gen)
+    rows, in_w = 2 * n_levels, (3 + 2 * n_levels + 15) // 16 * 16
+    _, dy_dx = enc.forward(x, prepare_input_gradients=True)
+    g = torch.randn((in_w, n), device="cuda", generator=gen).half()
+    y = torch.randn((16, n), device="cuda", generator=gen).half()
+    ws = torch.empty(int(L.n2_sdf_eikonal_workspace_bytes(C.c_uint32(n))), dtype=torch.uint8, device="cuda")
+    outs = []
+    for one in (False, True):
+        normal, v = (torch.full((3, n), 7.0, device="cuda") for _ in range(2))
+        dL_dy, v_in = torch.full((16, n), 7.0, device="cuda").half(), torch.full((in_w, n), 7.0, device="cuda").half()
+        loss = torch.zeros(1, device="cuda")
+        head = (_stream(), C.c_uint32(n), C.c_uint32(rows), C.c_uint32(in_w), ptr(y), ptr(g))
+        tail = (ptr(normal), C.c_float(0.1), C.c_float(128.0), ptr(dL_dy), ptr(v), ptr(v_in), ptr(loss), ptr(ws), C.c_uint64(ws.numel()))
+        if one:
+            check(L.n2_sdf_normals_and_eikonal_loss(*head, ptr(dy_dx), *tail), "n2_sdf_normals_and_eikonal_loss")
+        else:
+            normal_enc = enc.backward(dy_dx, x, g[3:3 + rows].contiguous(), want_input_grad=True, mode=GRAD_IGNORE)
+            # (in 64 bits first: the input gradient is a sum of 32-bit products of `rows` terms)
+            ref = (g[3:3 + rows].double()[:, :, None] * dy_dx.double()).sum(0).t()
+            assert float((normal_enc.double() - ref).norm() / ref.norm()) < 1e-6
+            check(L.n2_sdf_eikonal_loss(*head, ptr(normal_enc), *tail, ptr(dy_dx)), "n2_sdf_eikonal_loss")
+        outs.append((normal, v, dL_dy, v_in, loss))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
