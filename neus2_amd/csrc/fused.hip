@@ -763,9 +763,9 @@ static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream
 // 8192 9.4 -> 10.2, 16384 13.0 -> 16.6; a call from Python, bound by the host: 1000 points 9.5 -> 7.3, 8192 the same).
 constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 6144;
 
-static uint32_t fused_grid(uint32_t n) {
+static uint32_t fused_grid(uint32_t n, uint32_t most = 512u) {
 	const uint32_t tiles = (n + 31u) / 32u, blocks = (tiles + 3u) / 4u;
-	return blocks < 512u ? blocks : 512u;
+	return blocks < most ? blocks : most;
 }
 static size_t fused_lds(int n_frags, bool staged = false) {
 	return (size_t)n_frags * 1024 + FF_LEVELS * sizeof(uint4) + (staged ? (size_t)(FF_BLOCK / 64) * 32 * 2 * N2_RGB_IN_PITCH : 0);
@@ -824,9 +824,9 @@ int n2_fused_field_forward(const N2FusedNets& nets, hipStream_t s, const float* 
 		const uint32_t est_tiles = (est + FG_BLOCK - 1) / FG_BLOCK;
 		field_gather_list_kernel<<<dim3(n2_xcd_blocks(a.n_levels, est_tiles) + (a.frags && round == 0 ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, est_tiles);
 		N2_LAUNCH_CHECK();
-		// one 32-sample tile per wave where the estimate holds (the weight fragments come as a copy, so small workgroups are cheap)
-		const uint32_t blocks = (est + 127u) / 128u;
-		field_fused_forward_kernel<true, false><<<dim3(blocks < 2048u ? blocks : 2048u), dim3(FF_BLOCK), fused_lds(FF_COUNT, true), s>>>(a);
+		// (two workgroups per CU, as many as run at a time: a workgroup's start copies 40 KiB of fragments.  Up to 2048 of one tile per
+		// wave: the first round of a trained step 47 us instead of 38, the step 544 instead of 533; 768 and 1024: 541)
+		field_fused_forward_kernel<true, false><<<dim3(fused_grid(est)), dim3(FF_BLOCK), fused_lds(FF_COUNT, true), s>>>(a);
 		N2_LAUNCH_CHECK();
 		return N2_OK;
 	}
@@ -863,7 +863,10 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 	a.sdf_in = reinterpret_cast<hf*>(sdf_in);
 	launch_gather<false>(a, *nets.tab, s);
 	N2_LAUNCH_CHECK();
-	field_fused_forward_kernel<false, false><<<dim3(fused_grid(n)), dim3(FF_BLOCK), fused_lds(FF_SDF_COUNT), s>>>(a);
+	// (bound by the latency of its loads at few registers: four workgroups per CU for large batches, where 512 | 1024 | 2048 of them
+	// take 28.8 | 26.8 | 31 us for 2^20 points and 45.8 | 38.2 | 41.6 for 2^21; every workgroup builds the fragments, which
+	// costs smaller batches more than it gains: 2^17 to 2^19 points 0.5 to 1.4 us)
+	field_fused_forward_kernel<false, false><<<dim3(fused_grid(n, n >= (1u << 20) ? 1024u : 512u)), dim3(FF_BLOCK), fused_lds(FF_SDF_COUNT), s>>>(a);
 	N2_LAUNCH_CHECK();
 	return N2_OK;
 }
