@@ -2,16 +2,17 @@
 // NerfNetwork::sdf / density, :643-726).
 //
 // Training forward = two kernels.
-//  * field_gather_kernel walks the grid LEVEL-MAJOR (one workgroup = one level x 256 samples, all workgroups of a
-//    level next to each other in time), so that the level being read (<= 2 MiB) stays resident in every L2; a
-//    sample-major walk touches all 24 MiB of tables at once and three of five L2 requests miss.  It writes the
-//    features into the SDF net's input rows and the level's slopes (the Jacobian of the encoding without the level's
-//    scale factor) as a 16-byte block-float per sample and level (n2_slopes_pack), against 24 bytes of fp32.
+//  * field_gather_kernel walks the grid level by level (one workgroup = one level x 256 samples; every XCD takes whole
+//    levels, or all take the same one at a time: launch_gather), so that the tables being read (2 MiB at most each) stay
+//    resident in the L2s; a sample-major walk touches all 24 MiB of tables at once and three of five L2 requests miss.  It
+//    writes the features into the SDF net's input rows and the level's slopes (the Jacobian of the encoding without the
+//    level's scale factor) as a 16-byte block-float per sample and level (n2_slopes_pack), against 24 bytes of fp32.
 //  * field_fused_forward_kernel then takes 32 samples per wave through everything else without touching memory in
 //    between: SDF net forward, the gradient of its first output w.r.t. its input, the normal (that gradient contracted
 //    with the slopes), the direction encoding, the colour net and the 16 output rows.
-// Inference (sdf / density) is the second kernel alone with the gather inside it: positions that arrive in lattice or
-// near-lattice order hit cached lines whatever the order of the levels.
+// Inference (sdf / density) of points in no order is a gather of features alone and the second kernel without its second half,
+// or one launch for a few thousand points; positions that arrive in lattice or near-lattice order hit cached lines whatever
+// the order of the levels, and take the second kernel alone with the gather inside it.
 //
 // Layout of the network kernel.  Lane (n, g), n = lane % 32, g = lane / 32, works for sample b0 + n.  In the MFMA
 // layouts (see mlp_device.h) lane (n, g)
