@@ -148,3 +148,20 @@ def test_progressive_levels_tables_of_the_shipped_configs(oracle):
     for k in range(0, 41):
         exact = min(14, int(fractions.Fraction(14, 5) + fractions.Fraction(7, 25) * k))
         assert oracle.progressive_levels(14, 0.2, 0.02, 100, 100 * k) == exact, k
+
+
+@pytest.mark.parametrize("marched,kept,before,after", [
+    (720_000, 260_000, 0, 3), (720_000, 500_000, 0, 0), (400_000, 130_000, 0, 3), (399_999, 130_000, 0, 0),  # on: by ratio and by size
+    (390_000, 130_000, 3, 3), (330_000, 130_000, 3, 0), (46_000, 16_000, 3, 0), (700_000, 600_000, 3, 0)])   # off: by either
+def test_depth_rounds_are_for_large_steps(marched, kept, before, after):
+    from types import SimpleNamespace
+    from neus2_amd.training import Trainer
+    tr = Trainer.__new__(Trainer)
+    tr.cfg = SimpleNamespace(recompute_training_forward=0, target_batch_size=1 << 20)
+    tr.budget = SimpleNamespace(update=lambda *a: True)
+    tr.auto_depth_chunks, tr.depth_chunks, tr._h = True, (16, before) if before else (0, 0), None
+    tr.read_counters = lambda: dict(rays=1000, samples=marched, compacted=kept, loss=0.0)
+    tr._update_chunk_estimates = lambda: None
+    tr.set_depth_chunks = lambda size, rounds: setattr(tr, "depth_chunks", (size, rounds))
+    tr.update_budget()
+    assert tr.depth_chunks[1] == after
