@@ -900,7 +900,7 @@ bool n2_field_sdf_row0_lattice(n2_field_t* f, n2_stream_t stream, const N2Lattic
 	const uint64_t points = (uint64_t)lattice.res[0] * lattice.res[1] * lattice.res[2];
 	*rc = check_field(f, "n2_field_sdf", points < chunk ? (uint32_t)((points + 7) / 8 * 8) : chunk);
 	if (*rc != N2_OK) return true;
-	if (!(f->fused && fused_ok(f)) || chunk < lattice.res[0]) return false;
+	if (!(f->fused && fused_ok(f))) return false;
 	hipStream_t s = n2_stream(stream);
 	N2ProfScope prof(N2_PROF_FIELD_FORWARD, s);
 	*rc = n2_fused_lattice_sdf(fused_nets(f), s, lattice, chunk, d_scratch, d_frags, d_row0);

@@ -18,6 +18,7 @@
 #include "n2_common.h"
 
 #include "grid_device.h"
+#include "launch_rules.h"
 #include "mlp_device.h"
 #include "sdf_frags.h"
 
@@ -35,11 +36,11 @@ struct LatticeArgs {
 	const hf* frags;          // fragment image of the SDF network
 	float sdf_bias;
 	N2Lattice lat;
-	uint32_t y0, ny, z0, nz;  // the slab: rows y0 .. y0 + ny of planes z0 .. z0 + nz
-	uint32_t x_runs, walk;    // runs of 64 points per row; planes per wave
+	uint32_t x0, nx, y0, ny, z0, nz;  // the slab: columns x0 .. x0 + nx of rows y0 .. y0 + ny of planes z0 .. z0 + nz
+	uint32_t x_runs, walk;    // runs of 64 points per row of the slab; planes per wave
 	uint32_t first_fine;      // levels first_fine .. n_levels - 1 come from `features`
-	uint32_t* features;       // [n_levels - first_fine][nz ny rx] half2
-	float* out;               // row 0 of point (0, y0, z0)
+	uint32_t* features;       // [n_levels - first_fine][nz ny nx] half2
+	float* out;               // row 0 of point (x0, y0, z0)
 };
 
 // coordinate of lattice index c on axis d: each step rounded on its own (positions are part of a bit-exact contract)
@@ -71,11 +72,11 @@ __device__ __forceinline__ uint32_t lt_pack(float a, float b) {
 	return __builtin_bit_cast(uint32_t, h);
 }
 
-// The wave's run: x of the lane (clamped into the row), y, first plane.  False: nothing to do.
+// The wave's run: x of the lane (past the slab's last column in a run that is not full), y, first plane.  False: nothing to do.
 __device__ __forceinline__ bool lattice_run(const LatticeArgs& a, uint32_t wave, uint32_t& x, uint32_t& y, uint32_t& z, uint32_t& nz) {
 	const uint32_t xr = wave % a.x_runs, rest = wave / a.x_runs, yy = rest % a.ny, zz = rest / a.ny;
 	if (zz * a.walk >= a.nz) return false;
-	x = xr * 64u + (threadIdx.x & 63u);
+	x = a.x0 + xr * 64u + (threadIdx.x & 63u);
 	y = a.y0 + yy;
 	z = a.z0 + zz * a.walk;
 	nz = min(a.walk, a.nz - zz * a.walk);
@@ -96,9 +97,10 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x % blocks_per_level) * (LT_BLOCK / 64) + (threadIdx.x >> 6));
 	uint32_t x, y, z, nz;
 	if (!lattice_run(a, wave, x, y, z, nz)) return;
-	const bool inside = x < a.lat.res[0];
-	const uint32_t lane = threadIdx.x & 63u, plane = a.lat.res[0] * a.ny;
-	uint32_t* out = a.features + (size_t)(level - a.first_fine) * plane * a.nz + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.lat.res[0] + x;
+	const uint32_t x_last = a.x0 + a.nx - 1u;
+	const bool inside = x <= x_last;
+	const uint32_t lane = threadIdx.x & 63u, plane = a.nx * a.ny;
+	uint32_t* out = a.features + (size_t)(level - a.first_fine) * plane * a.nz + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + (x - a.x0);
 	if (level >= a.active_levels) {
 		for (uint32_t k = 0; k < nz; ++k)
 			if (inside) out[(size_t)k * plane] = 0u;
@@ -109,7 +111,7 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	const bool hashed = (a.hash_mask >> level) & 1u;
 	float wx, wy, wz;
 	uint32_t cx, cy, cz;
-	n2_locate(lattice_coord(a.lat, 0, min(x, a.lat.res[0] - 1u)), scale, wx, cx);
+	n2_locate(lattice_coord(a.lat, 0, min(x, x_last)), scale, wx, cx);
 	n2_locate(lattice_coord(a.lat, 1, y), scale, wy, cy);
 	n2_locate(lattice_coord(a.lat, 2, z + min(lane, nz - 1u)), scale, wz, cz);  // lane k: plane z + k (at most 64 of them)
 	// lane k: the four rows of vertices of plane z + k and their weights
@@ -206,9 +208,9 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (LT_BLOCK / 64) + (threadIdx.x >> 6));
 	uint32_t x, y, z, nz;
 	if (!lattice_run(a, wave, x, y, z, nz)) return;
-	const uint32_t lane = threadIdx.x & 63u, rx = a.lat.res[0], plane = rx * a.ny;
-	const bool inside = x < rx;
-	const float px = lattice_coord(a.lat, 0, min(x, rx - 1u)), py = lattice_coord(a.lat, 1, y);
+	const uint32_t lane = threadIdx.x & 63u, rx = a.lat.res[0], plane = a.nx * a.ny, x_last = a.x0 + a.nx - 1u;
+	const bool inside = x <= x_last;
+	const float px = lattice_coord(a.lat, 0, min(x, x_last)), py = lattice_coord(a.lat, 1, y);
 	const char* base[NM];
 #pragma unroll
 	for (int l = 0; l < NM; ++l) base[l] = reinterpret_cast<const char*>(a.table + a.offset[l]);
@@ -294,9 +296,9 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 #pragma unroll
 	for (int l = 0; l < NM; ++l) lo[l] = hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched-off levels
 	both_planes(on, my_cz);
-	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * rx + min(x, rx - 1u);
+	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + (min(x, x_last) - a.x0);
 	const size_t feat_level = (size_t)plane * a.nz;
-	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + x;
+	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + (x - a.x0);
 	const uint32_t g = lane >> 5;  // of the lanes with g = 0 a tile's operands take the coordinates
 	const hf ycoord = (hf)py - (hf)0.5f;
 	// tile 0 works for lanes 0..31, tile 1 for lanes 32..63: the x coordinate of both, for the lanes that need it (g = 0)
@@ -440,7 +442,6 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 	a.sdf_bias = nets.sdf_bias;
 	a.lat = lat;
 	a.features = reinterpret_cast<uint32_t*>(d_scratch);
-	a.x_runs = (lat.res[0] + 63u) / 64u;
 	// The walk takes the levels whose cells are larger than a step along z: above that, every step meets two new planes and
 	// there is nothing to keep.  (It is right for any level: a step across several cells fetches both planes.)
 	uint32_t coarse = 0;
@@ -452,29 +453,31 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 	static_assert(LT_LEVELS - 6u <= LT_MAX_FINE, "the fine levels' features fit the scratch");
 	lattice_frags_kernel<<<dim3(SDF_FRAG_COUNT), dim3(64), 0, s>>>(reinterpret_cast<const hf*>(nets.sdf_w), nets.sdf_in_w, tab.n_levels * 2u, reinterpret_cast<hf*>(d_frags));
 	N2_LAUNCH_CHECK();
+	// a slab holds as many points as the scratch has room for the fine levels' features of
 	const uint32_t rx = lat.res[0], ry = lat.res[1], rz = lat.res[2];
-	// rows per slab: what the scratch holds of the fine levels' features, at least one (the caller has checked chunk >= rx)
-	const uint64_t rows = (uint64_t)LT_MAX_FINE * chunk / (n_fine ? n_fine : 1u) / rx;
-	const uint32_t ny = rows < ry ? (uint32_t)rows : ry, nz = rows < ry ? 1u : (rows / ry < rz ? (uint32_t)(rows / ry) : rz);
-	for (uint32_t z0 = 0; z0 < rz; z0 += nz)
-		for (uint32_t y0 = 0; y0 < ry; y0 += ny) {
-			a.y0 = y0; a.ny = ny < ry - y0 ? ny : ry - y0;
-			a.z0 = z0; a.nz = nz < rz - z0 ? nz : rz - z0;
-			a.out = d_out + ((size_t)z0 * ry + y0) * rx;
-			// planes per wave: 16 where that leaves every SIMD several waves (a wave's start costs as much as two steps), fewer on
-			// small lattices; the slab's planes in equal shares
-			const uint64_t runs = (uint64_t)a.x_runs * a.ny * a.nz;
-			const uint32_t most = runs >= 16u * 4096u ? 16u : runs <= 4u * 4096u ? 4u : (uint32_t)(runs / 4096u), parts = (a.nz + most - 1u) / most;
-			a.walk = (a.nz + parts - 1u) / parts;
-			const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk), blocks = (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
-			if (n_fine) {
-				lattice_fine_kernel<<<dim3(blocks * n_fine), dim3(LT_BLOCK), 0, s>>>(a, blocks);
+	const N2LatticeSlab slab = n2_lattice_slab(lat.res, (uint64_t)LT_MAX_FINE * chunk / (n_fine ? n_fine : 1u));
+	for (uint32_t z0 = 0; z0 < rz; z0 += slab.nz)
+		for (uint32_t y0 = 0; y0 < ry; y0 += slab.ny)
+			for (uint32_t x0 = 0; x0 < rx; x0 += slab.nx) {
+				a.x0 = x0; a.nx = slab.nx < rx - x0 ? slab.nx : rx - x0;
+				a.y0 = y0; a.ny = slab.ny < ry - y0 ? slab.ny : ry - y0;
+				a.z0 = z0; a.nz = slab.nz < rz - z0 ? slab.nz : rz - z0;
+				a.out = d_out + ((size_t)z0 * ry + y0) * rx + x0;
+				a.x_runs = (a.nx + 63u) / 64u;
+				// planes per wave: 16 where that leaves every SIMD several waves (a wave's start costs as much as two steps), fewer on
+				// small lattices; the slab's planes in equal shares
+				const uint64_t runs = (uint64_t)a.x_runs * a.ny * a.nz;
+				const uint32_t most = runs >= 16u * 4096u ? 16u : runs <= 4u * 4096u ? 4u : (uint32_t)(runs / 4096u), parts = (a.nz + most - 1u) / most;
+				a.walk = (a.nz + parts - 1u) / parts;
+				const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk), blocks = (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
+				if (n_fine) {
+					lattice_fine_kernel<<<dim3(blocks * n_fine), dim3(LT_BLOCK), 0, s>>>(a, blocks);
+					N2_LAUNCH_CHECK();
+				}
+				if (nm == 10u) lattice_walk_kernel<10><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+				else if (nm == 8u) lattice_walk_kernel<8><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+				else lattice_walk_kernel<6><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
 				N2_LAUNCH_CHECK();
 			}
-			if (nm == 10u) lattice_walk_kernel<10><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
-			else if (nm == 8u) lattice_walk_kernel<8><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
-			else lattice_walk_kernel<6><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
-			N2_LAUNCH_CHECK();
-		}
 	return N2_OK;
 }

@@ -129,8 +129,8 @@ int n2_generate_training_samples_rows(n2_stream_t stream, uint32_t n_rays, uint3
 int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
                        float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n = 0xFFFFFFFFu);
 // Row 0 of NerfNetwork::sdf as fp32 on a whole lattice, x fastest: point c at (c / res) * extent + corner (lattice.hip).  The
-// lattice is worked off in slabs of at most `chunk` points (at least one row: chunk >= res[0]); d_scratch holds 44 bytes per
-// point of a slab, d_frags n2_lattice_frag_bytes().
+// lattice is worked off in slabs, whose size follows from d_scratch: 44 bytes for each of `chunk` points.  d_frags holds
+// n2_lattice_frag_bytes().  The values do not depend on where the slabs are cut.
 struct N2Lattice {
 	uint32_t res[3];
 	float inv_res[3], extent[3], corner[3];

@@ -67,7 +67,7 @@ def test_empty_lattice_and_errors():
         marching_cubes(torch.zeros((8, 8, 8), device="cuda", dtype=torch.float16), 0.0)
 
 
-# rows that end inside a run of 64 points, slabs of part of a plane (and rows longer than a chunk: positions written out), steps
+# rows that end inside a run of 64 points, slabs of part of a plane (and of part of a row), steps
 # of many cells of the fine levels (their rows are then gathered, not staged), several slabs of several planes, a box that
 # sticks out of the unit cube, a grid of 8 levels with dense ones among those the walk does not keep
 @pytest.mark.parametrize("res,chunk,box,levels", [((70, 9, 5), 1 << 14, (0, 1), 16), ((130, 20, 6), 512, (0.2, 0.9), 16), ((96, 4, 3), 64, (0, 1), 16),
@@ -93,6 +93,20 @@ def test_lattice_equals_the_same_points_queried(res, chunk, box, levels):
     padded[:, :n] = pos
     want = host(net.sdf(dev(padded)))[0, :n].reshape(res[2], res[1], res[0])
     assert_close(host(d), want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
+
+
+# rows longer than the chunk, down to the smallest one: slabs of a few runs, and of less than one
+@pytest.mark.parametrize("res,chunk", [((513, 3, 5), 64), ((200, 4, 3), 8)])
+def test_lattice_of_rows_longer_than_the_chunk(res, chunk):
+    """The values do not depend on where the lattice is cut, also where a row does not fit a slab."""
+    from neus2_amd.mesh import density_on_grid
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork()
+    p = torch.randn(net.param_offsets()[4], device="cuda", generator=torch.Generator(device="cuda").manual_seed(res[0])) * 0.1
+    net.set_params(p.half(), None)
+    net.reserve(1 << 14)
+    whole = density_on_grid(net._h, res, chunk=1 << 14)
+    assert torch.equal(whole, density_on_grid(net._h, res, chunk=chunk))
 
 
 def test_sdf_lattice_and_mesh_of_the_initial_sphere(oracle, tmp_path):

@@ -1,0 +1,50 @@
+"""The sizes of launches (neus2_amd/csrc/launch_rules.h), compiled with the host compiler: no GPU needed."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+WRAPPERS = """
+#include "launch_rules.h"
+extern "C" void lattice_slab(const uint32_t* res, uint64_t points, uint32_t* out) {
+	const N2LatticeSlab s = n2_lattice_slab(res, points);
+	out[0] = s.nx; out[1] = s.ny; out[2] = s.nz;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, so = d / "rules.cpp", d / "rules.so"
+    src.write_text(WRAPPERS)
+    subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "neus2_amd", "csrc"),
+                    str(src), "-o", str(so)], check=True, timeout=60)
+    return C.CDLL(str(so))
+
+
+# the smallest scratch, rows longer than it (with and without a whole run in it), rows of two points, the largest lattices,
+# a row that alone has more runs than a launch takes
+@pytest.mark.parametrize("res", [(2, 2, 2), (512, 512, 512), (96, 4, 3), (1000, 7, 2), (2, 1 << 23, 2), (2, 1 << 15, 1 << 15), (1 << 29, 2, 2), (3, 5, 1 << 27)])
+@pytest.mark.parametrize("chunk", [8, 64, 1 << 14, 1 << 22, 1 << 31])
+@pytest.mark.parametrize("n_fine", [1, 6, 10])
+def test_lattice_slabs_fit_the_scratch_and_the_launch(rules, res, chunk, n_fine):
+    points = 11 * chunk // n_fine
+    out = (C.c_uint32 * 3)()
+    rules.lattice_slab((C.c_uint32 * 3)(*res), C.c_uint64(points), out)
+    nx, ny, nz = out
+    assert 1 <= nx <= res[0] and 1 <= ny <= res[1] and 1 <= nz <= res[2]
+    assert nx * ny * nz <= points
+    assert (ny == 1 or nx == res[0]) and (nz == 1 or ny == res[1])  # the slab is one piece of the scratch's rows
+    # a launch counts its threads in 32 bits: 64 lanes per run of 64 points and level, in workgroups of four
+    assert ((nx + 63) // 64 * ny * nz + 3) // 4 * 256 * n_fine < 1 << 32
+    # nothing is given away: the slab is the lattice, or another column, row or plane would not fit one of the two
+    runs = (nx + 63) // 64
+    if nx < res[0]:
+        assert nx == points or nx == points // 64 * 64 or runs == 1 << 22
+    elif ny < res[1]:
+        assert nx * (ny + 1) > points or runs * (ny + 1) > 1 << 22
+    elif nz < res[2]:
+        assert nx * ny * (nz + 1) > points or runs * ny * (nz + 1) > 1 << 22
