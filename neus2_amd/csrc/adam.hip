@@ -73,10 +73,8 @@ __device__ __forceinline__ bool adam_summed(const N2SlabReduce& r, const hf* gra
 	return (g >= r.ga && g < r.ga + r.params_a) || (g >= r.gb && g < r.gb + r.params_b) || (r.extra_n > 0 && g == r.extra_out);
 }
 
-// STREAM: the moments are read and written past the last-level cache.  The optimiser's state is 176 MB of a step's traffic: with
-// the sample rows and the scatter's records of a large batch it does not fit the cache, and what it pushes out the next step's
-// kernels fetch again.  Kernels of a training step in us, plain | moments streamed | master weights too: batch 2^18 389 | 382 | 384,
-// 2^17 266 | 257, 2^16 193 | 185, 2^15 152 | 152, 2^14 128 | 132 | 134 (there the state stays in the cache from step to step).
+// STREAM: the moments are read and written past the last-level cache, for a caller whose state and samples do not fit it (the
+// trainer: n2_moments_stream, launch_rules.h).  Master weights streamed too: the training step at 2^18 382 -> 384 us, at 2^14 132 -> 134.
 template <typename StepT, bool STREAM>
 __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32_t n, uint32_t n_matrix, float loss_scale, float inv_loss_scale, int saturated,
                                                         uint32_t slot, const uint32_t* __restrict__ gate, float* __restrict__ master, hf* __restrict__ params, const hf* __restrict__ grads,

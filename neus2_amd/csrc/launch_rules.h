@@ -2,6 +2,18 @@
 #pragma once
 #include <cstdint>
 
+// Whether a training step streams its optimiser's moments past the last-level cache (n2_adam_step_gated): when what the step
+// passes over between two uses of a moment is more than the cache holds, the moments do not stay there and only push out
+// what the next kernels read.  That is the optimiser's state and, for each sample of the batch, about 1600 bytes of coordinates,
+// network rows, slopes and scatter records.  Steps in us, plain | streamed:
+//   state 227 MB (table of 2^19 entries a level): batch 4096 113 | 120, 20 480 140 | 142, 24 576 147 | 146, 28 672 154 | 152, 2^16 198 | 187, 2^18 381 | 373
+//   434 MB (2^20): 4096 149 | 148, 8192 187 | 180, 2^15 349 | 335        1.5 GB (2^22): 4096 236 | 234, 2^14 385 | 379
+//   63 MB (2^17): 2^14 100 | 102, 2^16 141 | 143, 2^17 201 | 199, 2^18 325 | 323        9 MB (2^14): 2^17 184 | 184, 2^18 305 | 304
+constexpr uint64_t N2_LAST_LEVEL_CACHE_BYTES = 256ull << 20, N2_STEP_BYTES_PER_SAMPLE = 1600;
+static inline bool n2_moments_stream(uint64_t state_bytes, uint64_t batch) {
+	return state_bytes + N2_STEP_BYTES_PER_SAMPLE * batch > N2_LAST_LEVEL_CACHE_BYTES;
+}
+
 // The part of a lattice that one launch of its kernels takes: columns, rows and planes (lattice.hip).
 struct N2LatticeSlab {
 	uint32_t nx, ny, nz;

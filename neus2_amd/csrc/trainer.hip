@@ -6,17 +6,13 @@
 // the scene and the seed) may run ahead on a stream the trainer owns, into the
 // other of two sample sets, while this step's field kernels occupy the GPU.
 #include "n2_common.h"
+#include "launch_rules.h"
 #include "slab_reduce.h"
-
 
 #include <cstring>
 #include <new>
 
 typedef _Float16 hf;
-
-// From this batch on the optimiser's moments are streamed: sample rows, scatter records and optimiser state of a step are then
-// more than the last-level cache holds (figures at adam_step_kernel)
-constexpr uint32_t STREAM_MOMENTS_BATCH = 1u << 16;
 
 struct n2_trainer {
 	n2_trainer_config cfg;
@@ -405,9 +401,11 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 	N2StepEpilogue epi{};
 	epi.values = t->ray_loss; epi.n_ptr = ray_counter; epi.n_max = n_rays; epi.sum_out = reinterpret_cast<float*>(t->counters) + 4;
 	epi.copy_src = set.counters; epi.copy_dst = t->counters; epi.copy_n = 2;
+	// master, moments, counters, fp16 parameters and gradients, and the average's two copies
+	const uint64_t state_bytes = (uint64_t)t->n_params * (16u + t->steps_bits / 8u + (t->ema ? 6u : 0u));
 	if (int rc = n2_adam_step_gated(stream, &t->cfg.adam, t->n_params, t->n_matrix_params, t->cfg.loss_scale, t->master, reinterpret_cast<n2_half*>(t->params),
 	                                reinterpret_cast<const n2_half*>(t->grads), t->m1, t->m2, t->steps, t->steps_bits, compacted_counter, &sums, &epi,
-	                                t->side ? t->ev_main : nullptr, T >= STREAM_MOMENTS_BATCH)) return rc;
+	                                t->side ? t->ev_main : nullptr, n2_moments_stream(state_bytes, T))) return rc;
 	t->ev_main_from_adam = t->side != nullptr;
 	t->optimizer_steps += 1;
 	t->training_step += 1;

@@ -12,6 +12,7 @@ extern "C" void lattice_slab(const uint32_t* res, uint64_t points, uint32_t* out
 	const N2LatticeSlab s = n2_lattice_slab(res, points);
 	out[0] = s.nx; out[1] = s.ny; out[2] = s.nz;
 }
+extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
 
 
@@ -48,3 +49,11 @@ def test_lattice_slabs_fit_the_scratch_and_the_launch(rules, res, chunk, n_fine)
         assert nx * (ny + 1) > points or runs * (ny + 1) > 1 << 22
     elif nz < res[2]:
         assert nx * ny * (nz + 1) > points or runs * ny * (nz + 1) > 1 << 22
+
+
+# parameters of the field with tables of 2^14 to 2^22 entries a level (18 bytes of optimiser state each), batch, streamed
+@pytest.mark.parametrize("n_params,batch,streams", [
+    (506884, 1 << 14, 0), (506884, 1 << 16, 0), (506884, 1 << 18, 1), (3507780, 1 << 16, 0), (3507780, 1 << 18, 1), (12612212, 1 << 12, 0),
+    (12612212, 20480, 0), (12612212, 28672, 1), (12612212, 1 << 18, 1), (24146548, 1 << 12, 1), (85050820, 1 << 12, 1), (1 << 31, 1 << 31, 1)])
+def test_moments_are_streamed_where_state_and_samples_exceed_the_cache(rules, n_params, batch, streams):
+    assert rules.moments_stream(C.c_uint64(18 * n_params), C.c_uint64(batch)) == streams
