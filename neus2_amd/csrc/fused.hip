@@ -383,7 +383,7 @@ __device__ __forceinline__ void listed_range(const FusedArgs& a, uint32_t& begin
 }
 
 // The listed pass: the number of samples is known on the device only.  The launch has est_tiles workgroups per level, levels dealt
-// to the XCDs as in the other kernel (level-major: the three rounds of a trained field's step 32 us longer); workgroup t of a
+// to the XCDs (figures at n2_gather_grid); workgroup t of a
 // level takes the tiles t, t + est_tiles, ...: any estimate gives the right result, a good one gives every workgroup one
 // tile.  (A fixed number of workgroups that walk all items by a stride is 1.6 times slower beside the trainer's sample
 // generator: its waves keep some of them from starting until others have finished their whole share.)
@@ -395,7 +395,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const Fused
 		return;
 	}
 	uint32_t level, first_tile;
-	if (!n2_xcd_level_tile(a.n_levels, est_tiles, level, first_tile)) return;
+	if (!n2_xcd_level_tile(blockIdx.x, a.n_levels, est_tiles, level, first_tile)) return;
 	uint32_t begin, count;
 	listed_range(a, begin, count);
 	const uint32_t tiles = (count + FG_BLOCK - 1) / FG_BLOCK;
@@ -407,10 +407,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const Fused
 
 template <bool FULL>
 __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs a, uint32_t tiles, int by_xcd) {
-	// by_xcd: whole levels per XCD (n2_xcd_level_tile); else level-major workgroup ids, so that the workgroups that run at one
-	// time work on one or two levels, whose tables stay in every L2.  Level-major reads every table into eight L2s, 200 MB
-	// whatever the batch; by XCD it is 25 MB, but the XCDs are never quite even.  The launch is bound by the lines the L1s fetch
-	// (2.3 clocks of a CU each from the L2; four per sample on every level whose cells are smaller than the marching step)
+	// Bound by the lines the L1s fetch (four per sample on every level whose cells are smaller than the marching step)
 	// and, with slopes, by the vector unit: without its gathers it would still take 46 of 73 us.  Measured on the training
 	// step and dropped: one 8- or 16-byte load per pair of x neighbours instead of two 4-byte loads (+12 us), loads of the hashed
 	// levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then requested twice and
@@ -428,12 +425,9 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 		return;
 	}
 	uint32_t level, tile;
-	if (!by_xcd) {
-		level = blockIdx.x / tiles;
-		tile = blockIdx.x - level * tiles;
-	} else if (!n2_xcd_level_tile(a.n_levels, tiles, level, tile)) {
-		return;
-	}
+	// (the full field's workgroups are counted along x alone)
+	const uint32_t y = FULL && !by_xcd ? blockIdx.x / tiles : blockIdx.y, x = FULL ? blockIdx.x - y * tiles : blockIdx.x;
+	if (!n2_gather_item(x, y, by_xcd ? 1u : a.n_levels, a.n_levels, tiles, level, tile)) return;
 	const uint32_t i = FULL ? tile * FG_BLOCK + threadIdx.x : tile * FG_PAIRS + (threadIdx.x >> 1);
 	if (i >= a.N || (a.live && i >= *a.live)) return;  // (both lanes of a pair)
 	if (FULL) gather_item(a, level, i, i);
@@ -747,16 +741,12 @@ bool n2_fused_supported(const N2LevelTable& tab, uint32_t sdf_hidden_layers, uin
 	return true;
 }
 
-// Up to here a gather's levels are dealt to the XCDs: from there on what the uneven XCDs lose is more than what reading the tables
-// into every L2 costs (field, rays: 2^14 samples 12.4 -> 9.9 us, 5e4 24.8 -> 19, 2.6e5 74.7 -> 73; uniform queries: 2^20 291
-// level-major, 299 by XCD).
-constexpr uint32_t GATHER_XCD_MAX = 1u << 19;
 template <bool FULL>
 static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream_t s) {
 	const uint32_t per = FULL ? FG_BLOCK : FG_PAIRS, tiles = (a.N + per - 1) / per;
-	const bool by_xcd = a.N <= GATHER_XCD_MAX;
-	const uint32_t blocks = by_xcd ? n2_xcd_blocks(tab.n_levels, tiles) : tiles * tab.n_levels;
-	field_gather_kernel<FULL><<<dim3(blocks + (FULL && a.frags ? FRAG_BLOCKS : 0u)), dim3(FG_BLOCK), 0, s>>>(a, tiles, by_xcd ? 1 : 0);
+	const N2GatherGrid g = n2_gather_grid(FULL ? N2_FIELD_XCD_MAX : N2_QUERY_XCD_MAX, a.N, tab.n_levels, per);
+	const dim3 grid = FULL ? dim3(g.x * g.y + (a.frags ? FRAG_BLOCKS : 0u)) : dim3(g.x, g.y);
+	field_gather_kernel<FULL><<<grid, dim3(FG_BLOCK), 0, s>>>(a, tiles, g.y == 1u ? 1 : 0);
 }
 
 // Up to here a query is one launch.  Beyond it the fragments that every 32 points rebuild from the weights weigh more than the

@@ -3,7 +3,7 @@
 // backward_backward_input, behind the n2_grid_* C ABI.
 //
 // Work decomposition: one workgroup handles a tile of points for ONE level.
-// The gather kernels deal whole levels to the XCDs (n2_xcd_level_tile), each of
+// The gather kernels deal whole levels to the XCDs (n2_gather_item), each of
 // which then streams all points through about two levels and fetches only those
 // levels' tables (<= 2 MiB each at T = 2^19) into its private 4 MiB L2 instead of
 // all 24 MiB; with costs from n2_grid_set_level_costs they cut the level-major
@@ -74,9 +74,9 @@ __device__ __forceinline__ float n2_corner_weight(const N2Point& p, uint32_t k) 
 	}
 
 constexpr uint32_t GRID_BLOCK = 256;
-constexpr uint32_t N_XCD = 8;  // gfx950: 8 XCDs, workgroup ids are dealt round-robin
+constexpr uint32_t N_XCD = N2_XCDS;
 
-// Piece x of the level-major item list [begin[x], begin[x + 1]) belongs to XCD x; begin[N_XCD] = 0: no plan, n2_xcd_level_tile deals
+// Piece x of the level-major item list [begin[x], begin[x + 1]) belongs to XCD x; begin[N_XCD] = 0: no plan, n2_gather_item deals
 // the items (2^18 points with dy_dx: 84 us uniform, 60 in ray order; with the plan of the default costs 101 and 74).
 struct N2XcdPlan {
 	uint32_t begin[N_XCD + 1];
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable t
                                                                   uint32_t dim_stride, const __half2* __restrict__ params,
                                                                   __half* __restrict__ out, float* __restrict__ dy_dx) {
 	uint32_t level, tile;
-	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_xcd_level_tile(tab.n_levels, tiles, level, tile))) return;
+	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_gather_item(blockIdx.x, blockIdx.y, gridDim.y, tab.n_levels, tiles, level, tile))) return;
 	const uint32_t i = tile * FWD_POINTS + (threadIdx.x >> 1), b = threadIdx.x & 1u;
 	if (i >= N) return;  // both lanes of a pair share i, so pairs leave together
 #define CALL(M) grid_forward_pair<M, WANT_DYDX, STREAM>(tab, level, i, b, N, xyz, point_stride, dim_stride, params, out, dy_dx)
@@ -1149,7 +1149,8 @@ N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_x
 	}
 	const uint32_t tiles = (n_points + FWD_POINTS - 1) / FWD_POINTS;
 	plan.begin[N_XCD] = 0;
-	const dim3 grid_dim(grid->costs_set ? make_xcd_plan(grid, tiles, plan) * N_XCD : n2_xcd_blocks(grid->tab.n_levels, tiles)), block(GRID_BLOCK);
+	const N2GatherGrid dealt = n2_gather_grid(N2_ENCODING_XCD_MAX, n_points, grid->tab.n_levels, FWD_POINTS);
+	const dim3 grid_dim = grid->costs_set ? dim3(make_xcd_plan(grid, tiles, plan) * N_XCD) : dim3(dealt.x, dealt.y), block(GRID_BLOCK);
 	const bool streams = n2_jacobian_streams(n_points, grid->tab.n_levels * grid->n_features);
 	auto* const kernel = !d_dy_dx ? grid_forward_kernel<false, false> : streams ? grid_forward_kernel<true, true> : grid_forward_kernel<true, false>;
 	kernel<<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride, dim_stride, grid->params,

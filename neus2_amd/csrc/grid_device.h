@@ -2,6 +2,7 @@
 // fused field kernels: cell location, level mask and the entry index of a grid vertex.
 #pragma once
 #include "n2_common.h"
+#include "launch_rules.h"
 
 // ----------------------------------------------------------------------------
 // device helpers
@@ -23,32 +24,6 @@ __device__ __forceinline__ bool n2_level_masked(const N2LevelTable& tab, uint32_
 	if (tab.max_level_gpu == nullptr) return level >= tab.active_levels;  // uniform: the host has applied both rules
 	const float limit = (tab.max_level_gpu[i] * (float)(tab.n_levels * tab.n_features)) / (float)tab.n_features;
 	return (float)level >= limit + 1e-3f || level >= tab.valid_levels;
-}
-
-// ----------------------------------------------------------------------------
-// Which (level, tile of points) is this workgroup?  The hardware deals consecutive workgroup ids round-robin over the XCDs,
-// each with an L2 of its own: id b runs on XCD b % 8.  Every XCD gets whole levels, so that its L2 fetches only those levels'
-// tables and not all of them (24 MiB, eight times over).  Their cost per point differs by how the points lie (on points in
-// ray order a fine level costs two and a half times a coarse one, on scattered ones about the same), so no plan by fixed costs is
-// even on both; dealing the levels out in rounds of eight, forwards and backwards in turn from the finest down (XCD 0: 15 and
-// 0, XCD 1: 14 and 1, ...), is within a tenth on both.  A last round of fewer than eight levels, the coarsest, is cut evenly.
-// ----------------------------------------------------------------------------
-constexpr uint32_t N2_XCDS = 8;
-__host__ __device__ __forceinline__ uint32_t n2_xcd_blocks(uint32_t n_levels, uint32_t tiles) {
-	return N2_XCDS * ((n_levels / N2_XCDS) * tiles + ((n_levels % N2_XCDS) * tiles + N2_XCDS - 1u) / N2_XCDS);
-}
-__device__ __forceinline__ bool n2_xcd_level_tile(uint32_t n_levels, uint32_t tiles, uint32_t& level, uint32_t& tile) {
-	const uint32_t xcd = blockIdx.x % N2_XCDS, j = blockIdx.x / N2_XCDS, round = j / tiles, rest = n_levels % N2_XCDS;
-	if (round < n_levels / N2_XCDS) {
-		tile = j - round * tiles;
-		level = n_levels - N2_XCDS * (round + 1u) + ((round & 1u) ? xcd : N2_XCDS - 1u - xcd);
-		return true;
-	}
-	const uint32_t share = (rest * tiles + N2_XCDS - 1u) / N2_XCDS, k = j - (n_levels / N2_XCDS) * tiles, item = xcd * share + k;
-	if (k >= share || item >= rest * tiles) return false;
-	level = item / tiles;
-	tile = item - level * tiles;
-	return true;
 }
 
 template <uint32_t MODE>

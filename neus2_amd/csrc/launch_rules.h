@@ -1,6 +1,13 @@
-// Sizes of launches that depend on nothing but numbers: host code without HIP, so that they can be checked on their own.
+// Sizes of launches, and how their workgroups share the work, as functions of nothing but numbers: they also compile without
+// HIP, so that they can be checked on their own.
 #pragma once
 #include <cstdint>
+
+#ifdef __HIPCC__
+#define N2_HD __host__ __device__
+#else
+#define N2_HD
+#endif
 
 // Whether a training step streams its optimiser's moments past the last-level cache (n2_adam_step_gated): when what the step
 // passes over between two uses of a moment is more than the cache holds, the moments do not stay there and only push out
@@ -30,4 +37,57 @@ static inline N2LatticeSlab n2_lattice_slab(const uint32_t res[3], uint64_t poin
 	if (nx < res[0]) return {nx, 1u, 1u};
 	if (rows < res[1]) return {nx, rows, 1u};
 	return {nx, res[1], rows / res[1] < res[2] ? rows / res[1] : res[2]};
+}
+
+// ----------------------------------------------------------------------------
+// Which (level, tile of points) is this workgroup?  The hardware deals consecutive workgroup ids round-robin over the XCDs,
+// each with an L2 of its own: id b runs on XCD b % 8.  Every XCD gets whole levels, so that its L2 fetches only those levels'
+// tables and not all of them (24 MiB, eight times over).  Their cost per point differs by how the points lie (on points in
+// ray order a fine level costs two and a half times a coarse one, on scattered ones about the same), so no plan by fixed costs is
+// even on both; dealing the levels out in rounds of eight, forwards and backwards in turn from the finest down (XCD 0: 15 and
+// 0, XCD 1: 14 and 1, ...), is within a tenth on both.  A last round of fewer than eight levels, the coarsest, is cut evenly.
+// ----------------------------------------------------------------------------
+constexpr uint32_t N2_XCDS = 8;
+N2_HD inline uint32_t n2_xcd_blocks(uint32_t n_levels, uint32_t tiles) {
+	return N2_XCDS * ((n_levels / N2_XCDS) * tiles + ((n_levels % N2_XCDS) * tiles + N2_XCDS - 1u) / N2_XCDS);
+}
+N2_HD inline bool n2_xcd_level_tile(uint32_t block, uint32_t n_levels, uint32_t tiles, uint32_t& level, uint32_t& tile) {
+	const uint32_t xcd = block % N2_XCDS, j = block / N2_XCDS, round = j / tiles, rest = n_levels % N2_XCDS;
+	if (round < n_levels / N2_XCDS) {
+		tile = j - round * tiles;
+		level = n_levels - N2_XCDS * (round + 1u) + ((round & 1u) ? xcd : N2_XCDS - 1u - xcd);
+		return true;
+	}
+	const uint32_t share = (rest * tiles + N2_XCDS - 1u) / N2_XCDS, k = j - (n_levels / N2_XCDS) * tiles, item = xcd * share + k;
+	if (k >= share || item >= rest * tiles) return false;
+	level = item / tiles;
+	tile = item - level * tiles;
+	return true;
+}
+
+// The launch of a kernel that takes (level, tile of points) items: workgroups in x and y.  Up to `by_xcd_max` points the levels are
+// dealt to the XCDs (y is 1); beyond, y counts the levels: the workgroups that run at one time then work on one or two
+// levels, whose tables stay in every L2, and what reading the tables into every L2 costs is less than what the uneven XCDs
+// lose.  (y, because a launch has at most 2^32 - 1 threads along x: 2^27 points of sixteen levels with two lanes each.)
+// Call in us, level-major | by XCD:
+//   field, points along rays: 2^14 12.4 | 9.9 and 52 000 24.8 | 19 (gather alone), 2^18 279 | 271, 2^19 507 | 502, 3 * 2^18 734 | 735, 2^20 961 | 969, 2^21 1917 | 1954
+//   query, uniform points: 2^17 52.8 | 47.9, 2^18 87.8 | 86.6, 5 * 2^16 105.4 | 105.6, 3 * 2^17 123.4 | 125.3, 2^19 159 | 164, 2^20 301 | 314, 2^21 594 | 617
+//   encoding alone, with the Jacobian and the backward: uniform 2^18 202 | 196, 2^19 421 | 422, 3 * 2^18 618 | 627, 2^20 819 | 834, 2^21 1708 | 1743;
+//   rays 2^18 165 | 158, 2^19 334 | 329, 2^20 654 | 655, 2^21 1333 | 1349
+// A listed pass of the field is dealt to the XCDs at any size (trained training step: 2^17 364 | 363, 2^18 559 | 530, 2^19 947 | 929, 2^20 1749 | 1726).
+constexpr uint32_t N2_FIELD_XCD_MAX = 1u << 19, N2_QUERY_XCD_MAX = 5u << 16, N2_ENCODING_XCD_MAX = 1u << 19;
+struct N2GatherGrid {
+	uint32_t x, y;
+};
+static inline N2GatherGrid n2_gather_grid(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels, uint32_t points_per_block) {
+	const uint32_t tiles = n / points_per_block + (n % points_per_block != 0u);
+	if (n <= by_xcd_max || n_levels == 1u) return {n2_xcd_blocks(n_levels, tiles), 1u};
+	return {tiles, n_levels};
+}
+// the item of workgroup (x, y) of such a launch of `height` workgroups in y; false: none
+N2_HD inline bool n2_gather_item(uint32_t x, uint32_t y, uint32_t height, uint32_t n_levels, uint32_t tiles, uint32_t& level, uint32_t& tile) {
+	if (height == 1u) return n2_xcd_level_tile(x, n_levels, tiles, level, tile);
+	level = y;
+	tile = x;
+	return true;
 }

@@ -149,6 +149,27 @@ def test_small_queries_equal_the_same_points_in_a_large_one(n, levels, active):
         assert torch.equal(query(few.T.contiguous()).view(torch.int16), want.contiguous().view(torch.int16))
 
 
+# one tile past the line at which a query's and a forward's levels are no longer dealt to the XCDs
+@pytest.mark.parametrize("levels", [16, 14, 1])
+def test_batches_past_the_deal_by_xcd_equal_their_parts(levels):
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork(n_levels=levels)
+    gen = torch.Generator(device="cuda").manual_seed(levels)
+    net.set_params((torch.randn(net.param_offsets()[4], device="cuda", generator=gen) * 0.1).half(), None)
+    n, part = (1 << 19) + 8, 1 << 17
+    net.reserve(n)
+    x = torch.rand((3, n), device="cuda", generator=gen)
+    whole = net.sdf(x[:, :(5 << 16) + 8].contiguous()).clone()
+    pieces = [net.sdf(x[:, a:a + part].contiguous()).clone() for a in range(0, (5 << 16) + 8, part)]
+    assert torch.equal(whole, torch.cat(pieces, 1)[:, :whole.shape[1]])
+    coords = torch.rand((n, 7), device="cuda", generator=gen)
+    out = net.forward(coords).clone()
+    assert torch.equal(out, torch.cat([net.forward(coords[a:a + part].contiguous()).clone() for a in range(0, n, part)]))
+    enc = net.encoding()
+    y, _ = enc.forward(x)
+    assert torch.equal(y, torch.cat([enc.forward(x[:, a:a + part].contiguous())[0] for a in range(0, n, part)], 1))
+
+
 def test_field_errors(oracle):
     from neus2_amd.tcnn_api import N2Error, NerfNetwork
     gf = NerfNetwork()

@@ -3,6 +3,7 @@ import ctypes as C
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -11,6 +12,20 @@ WRAPPERS = """
 extern "C" void lattice_slab(const uint32_t* res, uint64_t points, uint32_t* out) {
 	const N2LatticeSlab s = n2_lattice_slab(res, points);
 	out[0] = s.nx; out[1] = s.ny; out[2] = s.nz;
+}
+extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels, uint32_t points_per_block, uint32_t* visits, uint32_t* grid) {
+	const N2GatherGrid g = n2_gather_grid(by_xcd_max, n, n_levels, points_per_block);
+	grid[0] = g.x; grid[1] = g.y;
+	const uint32_t tiles = n / points_per_block + (n % points_per_block != 0u);
+	if (visits == nullptr) return 0;
+	for (uint32_t y = 0; y < g.y; ++y)
+		for (uint32_t x = 0; x < g.x; ++x) {
+			uint32_t level = 0, tile = 0;
+			if (!n2_gather_item(x, y, g.y, n_levels, tiles, level, tile)) continue;
+			if (level >= n_levels || tile >= tiles) return 1;
+			++visits[level * tiles + tile];
+		}
+	return 0;
 }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
@@ -57,3 +72,22 @@ def test_lattice_slabs_fit_the_scratch_and_the_launch(rules, res, chunk, n_fine)
     (12612212, 20480, 0), (12612212, 28672, 1), (12612212, 1 << 18, 1), (24146548, 1 << 12, 1), (85050820, 1 << 12, 1), (1 << 31, 1 << 31, 1)])
 def test_moments_are_streamed_where_state_and_samples_exceed_the_cache(rules, n_params, batch, streams):
     assert rules.moments_stream(C.c_uint64(18 * n_params), C.c_uint64(batch)) == streams
+
+
+# one level, fewer levels than XCDs, a last round that is not full, the most levels; one tile, tiles that the XCDs cannot share
+# evenly; either side of the line
+@pytest.mark.parametrize("n_levels", [1, 3, 8, 11, 16, 32])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1999, 2000, 2001, 5003])
+def test_gather_workgroups_meet_every_level_and_tile_once(rules, n_levels, n):
+    tiles = -(-n // 128)
+    visits, grid = np.zeros(n_levels * tiles, np.uint32), np.zeros(2, np.uint32)
+    assert rules.gather_visits(2000, n, n_levels, 128, visits.ctypes.data_as(C.c_void_p), grid.ctypes.data_as(C.c_void_p)) == 0
+    assert (visits == 1).all()
+    assert (grid[1] > 1) == (n > 2000 and n_levels > 1)
+
+
+@pytest.mark.parametrize("n", [1 << 18, (1 << 27) - 8, 1 << 27, 1 << 28, 1 << 30])
+def test_gather_launch_of_two_lanes_a_point_stays_below_the_thread_limit(rules, n):
+    grid = np.zeros(2, np.uint32)
+    rules.gather_visits(1 << 19, n, 16, 128, None, grid.ctypes.data_as(C.c_void_p))
+    assert int(grid[0]) * 256 < 1 << 32 and int(grid[1]) < 1 << 16
