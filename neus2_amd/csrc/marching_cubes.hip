@@ -32,9 +32,10 @@
 constexpr uint32_t MC_BLOCK = 256;
 
 struct McTable {
-	int8_t tri[256][16];
+	alignas(16) int8_t tri[256][16];  // a case's row is read as one uint4
 	uint8_t ntri[256];  // triangles of each case
 };
+static_assert(alignof(McTable) >= alignof(uint4) && sizeof(McTable::tri[0]) == sizeof(uint4), "rows can be read as uint4");
 
 // ---------------------------------------------------------------------------
 // case table: evaluated by the compiler, part of the library's device image
