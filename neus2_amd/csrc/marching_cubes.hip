@@ -107,6 +107,10 @@ __device__ const McTable MC_TABLE = mc_build_table();
 //   mc_emit     one wave per word that owns something: vertices and triangles
 //   mc_normals  one lane per vertex: the sum over the triangles of the four cubes round its edge
 // Rows are padded to whole words, so a word's neighbours in y and z are words too and no mask crosses a row.
+// Lattices whose rows have fewer than 16 points (SHORT) put several rows of a plane into the lower half of a word, each padded to
+// a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
+// word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
+// twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
 // 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 29, scan 9, emit 46, normals 34, with
 // the host's wait for the totals 227 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
@@ -117,9 +121,27 @@ struct McGrid {
 	float scale[3], offset[3];
 	uint32_t row_words;  // words per row
 	uint32_t n_words;
+	// SHORT: log2 of the pitch and of the rows of a word; words per plane; a full word's points, and those with a neighbour in x
+	uint32_t pitch_log, rows_log, plane_words, here, xok;
 };
+constexpr uint32_t MC_SHORT_ROW = 16, MC_SHORT_BITS_LOG = 5;
 
 typedef unsigned long long mc_word;
+
+// where a word's bit is in the lattice
+struct McPlace {
+	uint32_t x, y, z;
+};
+template <bool SHORT>
+__device__ __forceinline__ McPlace mc_place(const McGrid& g, uint32_t w, uint32_t bit) {
+	if constexpr (SHORT) {
+		const uint32_t z = w / g.plane_words, yw = w - z * g.plane_words;
+		return {bit & ((1u << g.pitch_log) - 1u), (yw << g.rows_log) + (bit >> g.pitch_log), z};
+	} else {
+		const uint32_t row = w / g.row_words, col = w - row * g.row_words;
+		return {col * 64u + bit, row % g.ry, row / g.ry};
+	}
+}
 
 // What a word of points owns; written for the words that own something, which the `active` bits tell.
 struct alignas(64) McRecord {
@@ -134,7 +156,7 @@ constexpr uint32_t MC_BITS_WORDS = 16;  // words a wave forms at a time: 16 load
 // STREAM: the density is read past the last-level cache; the lattice is larger than that and would only push itself out (512^3,
 // 512 MiB: 92 -> 80 us; 384^3, 216 MiB, which stays there for the emitting kernel: 32 -> 34).
 constexpr uint64_t MC_STREAM_BYTES = 256ull << 20;
-template <bool STREAM>
+template <bool STREAM, bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_bits_kernel(McGrid g, const float* __restrict__ density, mc_word* __restrict__ bits) {
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (MC_BLOCK / 64) + (threadIdx.x >> 6));
@@ -146,7 +168,13 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_bits_kernel(McGrid g, const float
 	for (uint32_t k = 0; k < MC_BITS_WORDS; ++k) {
 		const uint32_t x = col * 64u + lane;
 		const float* at = density + (uint64_t)row * g.rx + x;
-		v[k] = (w0 + k < g.n_words && x < g.rx) ? (STREAM ? __builtin_nontemporal_load(at) : *at) : -INFINITY;
+		bool inside = x < g.rx;
+		if (SHORT) {
+			const McPlace p = mc_place<true>(g, w0 + k, lane);
+			at = density + ((uint64_t)p.z * g.ry + p.y) * g.rx + p.x;
+			inside = lane >> MC_SHORT_BITS_LOG == 0u && p.x < g.rx && p.y < g.ry;
+		}
+		v[k] = (w0 + k < g.n_words && inside) ? (STREAM ? __builtin_nontemporal_load(at) : *at) : -INFINITY;
 		if (++col == g.row_words) { col = 0; ++row; }
 	}
 	mc_word mine = 0;
@@ -159,26 +187,51 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_bits_kernel(McGrid g, const float
 }
 
 // The bits of a word and of its neighbours, in the order of the offsets (y, z) = (0, 0), (1, 0), (0, 1), (1, 1): b the word
-// itself, s the word one point further along x.  ok[0]: points of the word that have a neighbour in x; ok[1], ok[2]: the rows
-// at y + 1, z + 1 exist (their words are zero if not).
+// itself, s the word one point further along x.  here: the word's points; xok, yok: those that have a neighbour in x, in y; zok: the
+// plane at z + 1 exists (words of rows and planes that do not are zero).
 struct McBits {
-	mc_word b[4], s[4], here, xok;
-	bool yok, zok;
+	mc_word b[4], s[4], here, xok, yok;
+	bool zok;
 };
+// SHORT: the points of the first n rows of a word
+__device__ __forceinline__ mc_word mc_first_rows(const McGrid& g, uint32_t n) {
+	return n >> g.rows_log ? (1ull << (1u << MC_SHORT_BITS_LOG)) - 1ull : (1ull << (n << g.pitch_log)) - 1ull;
+}
 // WAVE: the lanes of the wave hold consecutive words, and take the word behind theirs from the next lane
-template <bool WAVE>
+template <bool WAVE, bool SHORT>
 __device__ __forceinline__ McBits mc_load_bits(const McGrid& g, const mc_word* __restrict__ bits, uint32_t w) {
 	McBits B;
+	if constexpr (SHORT) {
+		const McPlace first = mc_place<true>(g, w, 0u);
+		const uint32_t rows = g.ry - first.y, pitch = 1u << g.pitch_log;  // rows from the word's first on
+		B.here = g.here & mc_first_rows(g, rows);
+		B.xok = g.xok & mc_first_rows(g, rows);
+		B.yok = mc_first_rows(g, rows - 1u);
+		B.zok = first.z + 1u < g.rz;
+#pragma unroll
+		for (uint32_t j = 0; j < 4; j += 2) {
+			const uint32_t at = w + (j ? g.plane_words : 0u);
+			const bool ok = j == 0u || B.zok;
+			B.b[j] = ok ? bits[at] : 0ull;
+			const mc_word next = ok && (rows - 1u) >> g.rows_log ? bits[at + 1u] : 0ull;  // the plane has rows behind the word's
+			// (what the last points of a row get as their neighbours in x, and what stands above the lower half, is not used: xok, here)
+			B.b[j + 1] = (B.b[j] >> pitch) | (next << ((1u << MC_SHORT_BITS_LOG) - pitch));
+			B.s[j] = B.b[j] >> 1;
+			B.s[j + 1] = B.b[j + 1] >> 1;
+		}
+		return B;
+	}
 	const uint32_t row = w / g.row_words, col = w - row * g.row_words;
 	const uint32_t z = row / g.ry, y = row - z * g.ry;
-	B.yok = y + 1u < g.ry;
+	const bool yok = y + 1u < g.ry;
+	B.yok = yok ? ~0ull : 0ull;
 	B.zok = z + 1u < g.rz;
 	const uint32_t left = g.rx - col * 64u;  // points from the word's first to the end of the row
 	B.here = left >= 64u ? ~0ull : (1ull << left) - 1ull;
 	B.xok = left > 64u ? ~0ull : (1ull << (left - 1u)) - 1ull;
 #pragma unroll
 	for (uint32_t j = 0; j < 4; ++j) {
-		const bool ok = (!(j & 1u) || B.yok) && (!(j & 2u) || B.zok);
+		const bool ok = (!(j & 1u) || yok) && (!(j & 2u) || B.zok);
 		const uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u);
 		B.b[j] = ok ? bits[at] : 0ull;
 		mc_word next = 0ull;
@@ -214,6 +267,7 @@ __device__ __forceinline__ uint32_t mc_wave_scan(uint32_t v, uint32_t lane) {
 
 // One lane per word; a lane walks through the cubes of its word that the surface cuts.  (Listing those cubes in LDS and dealing
 // them to the lanes, as the emitting kernel does, takes the same time: the launch is four rounds of load latency.)
+template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
                                                             mc_word* __restrict__ active, uint2* __restrict__ blocks) {
 	__shared__ uint8_t ntri[256];
@@ -224,17 +278,17 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const mc_w
 	McRecord r{};
 	uint32_t nv = 0, nt = 0;
 	mc_word cut = 0;
-	const McBits B = mc_load_bits<true>(g, bits, min(w, g.n_words - 1u));  // every lane takes part in the exchange
+	const McBits B = mc_load_bits<true, SHORT>(g, bits, min(w, g.n_words - 1u));  // every lane takes part in the exchange
 	if (w < g.n_words) {
 		r.edge[0] = (B.b[0] ^ B.s[0]) & B.xok;
-		r.edge[1] = B.yok ? (B.b[0] ^ B.b[1]) & B.here : 0ull;
+		r.edge[1] = (B.b[0] ^ B.b[1]) & B.here & B.yok;
 		r.edge[2] = B.zok ? (B.b[0] ^ B.b[2]) & B.here : 0ull;
 #pragma unroll
 		for (int a = 0; a < 3; ++a) nv += (uint32_t)__popcll(r.edge[a]);
 		if (B.yok && B.zok) {
 			const mc_word any = B.b[0] | B.b[1] | B.b[2] | B.b[3] | B.s[0] | B.s[1] | B.s[2] | B.s[3];
 			const mc_word all = B.b[0] & B.b[1] & B.b[2] & B.b[3] & B.s[0] & B.s[1] & B.s[2] & B.s[3];
-			cut = any & ~all & B.xok;
+			cut = any & ~all & B.xok & B.yok;
 		}
 		for (; cut; cut &= cut - 1ull) {
 			const uint32_t p = (uint32_t)__ffsll(cut) - 1u;
@@ -358,6 +412,7 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // slots come from the records of the (at most eight) words those points are in, and stand in LDS, where a triangle's
 // corners pick theirs.
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
+template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float* __restrict__ density, const mc_word* __restrict__ bits,
                                                            const McRecord* __restrict__ records, const mc_word* __restrict__ active,
                                                            const uint2* __restrict__ blocks, float* __restrict__ verts, uint32_t* __restrict__ indices,
@@ -379,11 +434,11 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 		const McRecord& r = records[w];
 		const McOwned own = mc_owned(records, blocks, w);
 		const mc_word t0 = r.tri[0], t1 = r.tri[1], t2 = r.tri[2];
-		const uint32_t row = w / g.row_words, col = w - row * g.row_words;
-		const uint32_t xyz[3] = {col * 64u + p, row % g.ry, row / g.ry};
+		const McPlace place = mc_place<SHORT>(g, w, p);
+		const uint32_t xyz[3] = {place.x, place.y, place.z};
 		const uint32_t slot0 = mc_vertex_slot(own, p), flags = slot0 >> 29;
 		if (flags) {
-			const uint64_t idx = (uint64_t)row * g.rx + xyz[0];
+			const uint64_t idx = ((uint64_t)xyz[2] * g.ry + xyz[1]) * g.rx + xyz[0];
 			const uint64_t step[3] = {1u, g.rx, (uint64_t)g.rx * g.ry};
 			const float pos[3] = {(float)xyz[0], (float)xyz[1], (float)xyz[2]};
 			const float f0 = density[idx];
@@ -406,13 +461,18 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 		if (tris == 0) return;  // (the cubes of the last column, row and plane have no triangles: the points below exist)
 #pragma unroll
 		for (uint32_t j = 0; j < 4; ++j) {
-			const uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u);
+			uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u), bit = p;
+			if (SHORT) {
+				bit = (j & 1u) ? p + (1u << g.pitch_log) : p;
+				at = w + (bit >> MC_SHORT_BITS_LOG) + ((j & 2u) ? g.plane_words : 0u);
+				bit &= (1u << MC_SHORT_BITS_LOG) - 1u;
+			}
 			const McOwned o = j == 0 ? own : mc_owned(records, blocks, at);
-			slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, p);
-			slot_of[2 * j + 1][threadIdx.x] = p < 63u ? mc_vertex_slot(o, p + 1u) : mc_vertex_slot(mc_owned(records, blocks, at + 1u), 0u);
+			slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, bit);
+			slot_of[2 * j + 1][threadIdx.x] = bit < 63u ? mc_vertex_slot(o, bit + 1u) : mc_vertex_slot(mc_owned(records, blocks, at + 1u), 0u);
 		}
 		const uint32_t first_t = blocks[w / MC_BLOCK].y + r.first_t + mc_below(t0, p) + 2u * mc_below(t1, p) + 4u * mc_below(t2, p);
-		const uint32_t mask = mc_case(mc_load_bits<false>(g, bits, w), p);
+		const uint32_t mask = mc_case(mc_load_bits<false, SHORT>(g, bits, w), p);
 		// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
 		// the owner's offset from this point in x, y, z and the edge's axis.
 		constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
@@ -437,6 +497,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 // the four cubes round the vertex's edge; the cubes are visited in lattice order and their triangles in theirs, so the sum
 // does not depend on how the work is scheduled.  (Adding every triangle to its corners with float atomics took 276 us for
 // the 512^3 sphere's 1.2 M triangles: 11 M atomics at the part's 40 G/s.)
+template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const McRecord* __restrict__ records,
                                                               const mc_word* __restrict__ active, const uint2* __restrict__ blocks,
                                                               const uint32_t* __restrict__ indices, const float* __restrict__ verts,
@@ -446,8 +507,8 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t
 	float* mine = normals + (size_t)i * 3;
 	const uint32_t w = __float_as_uint(mine[0]), place = __float_as_uint(mine[1]);
 	const uint32_t lane = place & 63u, axis = place >> 6;
-	const uint32_t row = w / g.row_words, col = w - row * g.row_words;
-	const uint32_t xyz[3] = {col * 64u + lane, row % g.ry, row / g.ry};
+	const McPlace p = mc_place<SHORT>(g, w, lane);
+	const uint32_t xyz[3] = {p.x, p.y, p.z};
 	// the two axes across the edge, the slower one first
 	const uint32_t slow = axis == 2u ? 1u : 2u, fast = axis == 0u ? 1u : 0u;
 	uint32_t first[4], count[4];
@@ -458,7 +519,12 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t
 		count[k] = 0;
 		first[k] = 0;
 		if (bx > xyz[0] || by > xyz[1] || bz > xyz[2]) continue;
-		const uint32_t x = xyz[0] - bx, at = (row - by - bz * g.ry) * g.row_words + (x >> 6), l = x & 63u;
+		const uint32_t x = xyz[0] - bx, y = xyz[1] - by, z = xyz[2] - bz;
+		uint32_t at = (z * g.ry + y) * g.row_words + (x >> 6), l = x & 63u;
+		if (SHORT) {
+			at = z * g.plane_words + (y >> g.rows_log);
+			l = (y & ((1u << g.rows_log) - 1u)) << g.pitch_log | x;
+		}
 		if (!((active[at >> 6] >> (at & 63u)) & 1ull)) continue;
 		const McRecord& r = records[at];
 		const mc_word t0 = r.tri[0], t1 = r.tri[1], t2 = r.tri[2];
@@ -512,13 +578,19 @@ static int mc_check(const char* fn, const uint32_t res[3], uint64_t& n) {
 // Workspace: the points' bits, one record per word (written only where a word owns something), which words do, and the
 // prefix sums over blocks of 256 words (one entry more than blocks: the totals).
 struct McCarve {
-	uint32_t row_words, n_words, n_blocks;
+	uint32_t row_words, pitch_log, rows_log, plane_words, n_words, n_blocks;
+	bool short_rows;
 	uint64_t bits, records, active, blocks, total;
 };
 static McCarve mc_carve(const uint32_t res[3]) {
 	McCarve c;
 	c.row_words = (res[0] + 63u) / 64u;
-	c.n_words = c.row_words * res[1] * res[2];  // at most 2^30: rows have at least two points
+	c.short_rows = res[0] < MC_SHORT_ROW;
+	c.pitch_log = 1;
+	while ((1u << c.pitch_log) < res[0] && c.short_rows) ++c.pitch_log;
+	c.rows_log = MC_SHORT_BITS_LOG - c.pitch_log;
+	c.plane_words = c.short_rows ? (res[1] + (1u << c.rows_log) - 1u) >> c.rows_log : c.row_words * res[1];
+	c.n_words = c.plane_words * res[2];  // at most 2^29: planes have at least four points
 	c.n_blocks = (c.n_words + MC_BLOCK - 1) / MC_BLOCK;
 	uint64_t o = 0;
 	auto take = [&](uint64_t bytes) { const uint64_t at = o; o += m256(bytes); return at; };
@@ -543,6 +615,14 @@ static McGrid mc_grid(const uint32_t res[3], const float aabb_min[3], const floa
 	const McCarve c = mc_carve(res);
 	g.row_words = c.row_words;
 	g.n_words = c.n_words;
+	g.pitch_log = c.pitch_log;
+	g.rows_log = c.rows_log;
+	g.plane_words = c.plane_words;
+	g.here = g.xok = 0;
+	for (uint32_t at = 0; c.short_rows && at < 1u << MC_SHORT_BITS_LOG; at += 1u << c.pitch_log) {
+		g.here |= ((1u << res[0]) - 1u) << at;
+		g.xok |= ((1u << (res[0] - 1u)) - 1u) << at;
+	}
 	return g;
 }
 
@@ -561,10 +641,13 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	mc_word* bits = reinterpret_cast<mc_word*>(b + c.bits);
 	uint2* blocks = reinterpret_cast<uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
-	auto* const bits_kernel = 4 * n >= MC_STREAM_BYTES ? mc_bits_kernel<true> : mc_bits_kernel<false>;
+	const bool stream_density = 4 * n >= MC_STREAM_BYTES;
+	auto* const bits_kernel = c.short_rows ? (stream_density ? mc_bits_kernel<true, true> : mc_bits_kernel<false, true>)
+	                                       : (stream_density ? mc_bits_kernel<true, false> : mc_bits_kernel<false, false>);
 	bits_kernel<<<mgrid(((uint64_t)c.n_words + MC_BITS_WORDS - 1) / MC_BITS_WORDS * 64u), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits);
 	N2_LAUNCH_CHECK();
-	mc_count_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
+	auto* const count_kernel = c.short_rows ? mc_count_kernel<true> : mc_count_kernel<false>;
+	count_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
 	N2_LAUNCH_CHECK();
 	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks);
 	N2_LAUNCH_CHECK();
@@ -594,11 +677,13 @@ N2_API int n2_marching_cubes_emit(n2_stream_t stream, const uint32_t res[3], con
 	const mc_word* active = reinterpret_cast<const mc_word*>(b + c.active);
 	const uint2* blocks = reinterpret_cast<const uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
-	mc_emit_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits, records, active, blocks, d_vertices, d_indices,
-	                                                           reinterpret_cast<uint32_t*>(d_normals));
+	auto* const emit_kernel = c.short_rows ? mc_emit_kernel<true> : mc_emit_kernel<false>;
+	emit_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits, records, active, blocks, d_vertices, d_indices,
+	                                                        reinterpret_cast<uint32_t*>(d_normals));
 	N2_LAUNCH_CHECK();
 	if (d_normals) {
-		mc_normals_kernel<<<mgrid(n_vertices), dim3(MC_BLOCK), 0, s>>>(g, n_vertices, records, active, blocks, d_indices, d_vertices, d_normals);
+		auto* const normals_kernel = c.short_rows ? mc_normals_kernel<true> : mc_normals_kernel<false>;
+		normals_kernel<<<mgrid(n_vertices), dim3(MC_BLOCK), 0, s>>>(g, n_vertices, records, active, blocks, d_indices, d_vertices, d_normals);
 		N2_LAUNCH_CHECK();
 	}
 	return N2_OK;

@@ -65,6 +65,16 @@ def test_level_table_matches_oracle(oracle):
         L.n2_grid_destroy(h)
 
 
+@pytest.mark.parametrize("res", [(2, 32, 64), (2, 1 << 15, 1 << 15), (3, 6, 1000), (16, 16, 16), (16, 512, 512), (17, 9, 33), (33, 5, 7), (63, 512, 512), (65, 64, 64), (512, 512, 512)])
+def test_marching_cubes_workspace_of_short_rows(res):
+    """A word of bits takes 72 bytes and has at least sixteen points where a plane has them; 4 KiB for what is per block."""
+    from neus2_amd import capi
+    L = capi.lib()
+    L.n2_marching_cubes_workspace_bytes.restype = ctypes.c_uint64
+    n = res[0] * res[1] * res[2]
+    assert 0 < L.n2_marching_cubes_workspace_bytes((ctypes.c_uint32 * 3)(*res)) <= 4.6 * n + 4096
+
+
 def test_cpp_shim_host_checks():
     """The header-only C++ shim (tcnn method names over the C ABI) compiles with the host compiler and its
     host-only behaviour holds: shapes, parameter counts, matrix views, errors as std::runtime_error."""

@@ -42,7 +42,10 @@ def test_mesh_matches_oracle(res, kind):
         assert check_closed_oriented(host(v), host(t).astype(np.int64)) == 2
 
 
-@pytest.mark.parametrize("res", [(63, 6, 5), (64, 6, 5), (65, 6, 5), (128, 30, 12), (129, 40, 11)])  # one point short of a word of 64, exact, one over; several blocks of words
+@pytest.mark.parametrize("res", [(63, 6, 5), (64, 6, 5), (65, 6, 5), (128, 30, 12), (129, 40, 11),  # one point short of a word of 64, exact, one over; several blocks of words
+                                 # several rows to a word: every pitch, rows that fill it and do not, planes of part of a word, of whole ones, of one row more
+                                 (2, 2, 5), (2, 32, 7), (2, 33, 7), (3, 17, 9), (4, 15, 6), (5, 8, 6), (8, 9, 70), (9, 4, 5), (9, 3, 5), (15, 7, 40), (15, 6, 300),
+                                 (16, 7, 5), (17, 65, 4)])
 def test_rows_of_words(res):
     """Noise: every word of points owns something, so the points of a block fill the emitting kernel's list several times."""
     from neus2_amd.mesh import marching_cubes
