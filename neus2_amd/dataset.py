@@ -164,7 +164,7 @@ def load_images(ds, device="cuda"):
     from PIL import Image
     from . import capi
     from .capi import check, ptr
-    from .tcnn_api import pack_cameras
+    from .tcnn_api import _stream, pack_cameras
     arrays, cams, offset = [], [], 0
     for fr in ds["frames"]:
         if not os.path.exists(fr["file"]):
@@ -198,7 +198,7 @@ def load_images(ds, device="cuda"):
         offset += w * h
     bytes_dev = torch.from_numpy(np.concatenate(arrays)).to(device)
     rgba = torch.empty((offset, 4), dtype=torch.float32, device=device)
-    check(capi.lib().n2_convert_rgba8(C.c_void_p(torch.cuda.current_stream().cuda_stream), C.c_uint64(offset), ptr(bytes_dev), ptr(rgba),
+    check(capi.lib().n2_convert_rgba8(_stream(), C.c_uint64(offset), ptr(bytes_dev), ptr(rgba),
                                       C.c_int(int(ds["white_transparent"])), C.c_int(int(ds["black_transparent"])), C.c_uint32(0)),
           "n2_convert_rgba8")
     return pack_cameras(cams, device=device), len(cams), rgba, cams

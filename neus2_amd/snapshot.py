@@ -8,6 +8,7 @@ import torch
 
 from . import capi
 from .capi import N2Error, check, ptr
+from .tcnn_api import _stream
 
 
 class SnapshotDesc(C.Structure):
@@ -122,10 +123,6 @@ def pack_config(obj):
 
     put(obj)
     return bytes(out)
-
-
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def save_snapshot(path, trainer, occupancy=None, config=None, include_optimizer_state=False, loss=0.0, aabb_scale=1):

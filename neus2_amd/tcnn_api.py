@@ -15,9 +15,15 @@ from .capi import (GRAD_ACCUMULATE, GRAD_IGNORE, GRAD_OVERWRITE, LAYOUT_AOS, LAY
                    ptr)
 
 
+# not part of torch's public interface: where a torch does without it, the public call serves
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
     """torch's current stream as a hipStream_t.  (torch.cuda.current_stream() builds a Stream object: 3 us of a small query's 12.)"""
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    if _raw_stream is None:
+        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 def _positions(xyz):

@@ -170,6 +170,14 @@ def test_batches_past_the_deal_by_xcd_equal_their_parts(levels):
     assert torch.equal(y, torch.cat([enc.forward(x[:, a:a + part].contiguous())[0] for a in range(0, n, part)], 1))
 
 
+def test_stream_lookup_follows_the_current_stream():
+    from neus2_amd.tcnn_api import _stream
+    side = torch.cuda.Stream()
+    for s in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(s):
+            assert (_stream().value or 0) == s.cuda_stream == torch.cuda.current_stream().cuda_stream
+
+
 def test_field_errors(oracle):
     from neus2_amd.tcnn_api import N2Error, NerfNetwork
     gf = NerfNetwork()

@@ -165,3 +165,14 @@ def test_depth_rounds_are_for_large_steps(marched, kept, before, after):
     tr.set_depth_chunks = lambda size, rounds: setattr(tr, "depth_chunks", (size, rounds))
     tr.update_budget()
     assert tr.depth_chunks[1] == after
+
+
+def test_stream_lookup_without_torchs_private_call(monkeypatch):
+    """The modules share one lookup, which does without the private call where torch has none."""
+    from types import SimpleNamespace
+
+    from neus2_amd import mesh, sdf_net, snapshot, tcnn_api
+    assert mesh._stream is sdf_net._stream is snapshot._stream is tcnn_api._stream
+    monkeypatch.setattr(tcnn_api, "_raw_stream", None)
+    monkeypatch.setattr(tcnn_api.torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=4711))
+    assert tcnn_api._stream().value == 4711
