@@ -442,12 +442,7 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 	a.sdf_bias = nets.sdf_bias;
 	a.lat = lat;
 	a.features = reinterpret_cast<uint32_t*>(d_scratch);
-	// The walk takes the levels whose cells are larger than a step along z: above that, every step meets two new planes and
-	// there is nothing to keep.  (It is right for any level: a step across several cells fetches both planes.)
-	uint32_t coarse = 0;
-	const float step = lat.inv_res[2] * (lat.extent[2] < 0.f ? -lat.extent[2] : lat.extent[2]);
-	while (coarse < LT_LEVELS && a.scale[coarse] * step < 0.95f) ++coarse;
-	const uint32_t nm = coarse >= 10u ? 10u : coarse >= 8u ? 8u : 6u;
+	const uint32_t nm = n2_lattice_walked_levels(a.scale, lat.inv_res[2] * (lat.extent[2] < 0.f ? -lat.extent[2] : lat.extent[2]));
 	a.first_fine = nm;
 	const uint32_t n_fine = tab.n_levels > nm ? tab.n_levels - nm : 0u;
 	static_assert(LT_LEVELS - 6u <= LT_MAX_FINE, "the fine levels' features fit the scratch");

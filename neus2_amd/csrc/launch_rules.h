@@ -39,6 +39,16 @@ static inline N2LatticeSlab n2_lattice_slab(const uint32_t res[3], uint64_t poin
 	return {nx, res[1], rows / res[1] < res[2] ? rows / res[1] : res[2]};
 }
 
+// Levels that the lattice's walk keeps planes of, by the step along z (it is right for any level and step).  A level whose cells are
+// larger than a step crosses into a new plane less than once per step; of one whose cells are smaller every step meets two
+// planes and nothing is kept, but up to about 1.15 cells per step that costs less than its features' way through memory.
+// Call in us with 6 | 8 | 10 levels walked, the default table: 64^3 59 | 61 | 60, 128^3 187 | 190 | 197, 176^3 438 | 407 | 427, 208^3 647 | 679 | 675,
+// 224^3 792 | 767 | 776, 256^3 1056 | 1001 | 1010, 272^3 1335 | 1273 | 1257, 320^3 1918 | 1856 | 1742, 384^3 3097 | 2858 | 2706, 464^3 5812 | 5485 | 5107,
+// 512^3 6783 | 6220 | 5745; 512 x 512 x 128 1777 | 1726 | 1789, 320 x 320 x 128 791 | 830 | 827, 128 x 128 x 512 692 | 668 | 664.
+static inline uint32_t n2_lattice_walked_levels(const float scale[16], float step) {
+	return scale[8] * step < 1.15f ? 10u : scale[7] * step < 0.95f ? 8u : 6u;
+}
+
 // ----------------------------------------------------------------------------
 // Which (level, tile of points) is this workgroup?  The hardware deals consecutive workgroup ids round-robin over the XCDs,
 // each with an L2 of its own: id b runs on XCD b % 8.  Every XCD gets whole levels, so that its L2 fetches only those levels'

@@ -72,10 +72,10 @@ def test_empty_lattice_and_errors():
 
 # rows that end inside a run of 64 points, slabs of part of a plane (and of part of a row), steps
 # of many cells of the fine levels (their rows are then gathered, not staged), several slabs of several planes, a box that
-# sticks out of the unit cube, a grid of 8 levels with dense ones among those the walk does not keep
+# sticks out of the unit cube, a grid of 8 levels with dense ones among those the walk does not keep, eight and ten levels walked
 @pytest.mark.parametrize("res,chunk,box,levels", [((70, 9, 5), 1 << 14, (0, 1), 16), ((130, 20, 6), 512, (0.2, 0.9), 16), ((96, 4, 3), 64, (0, 1), 16),
                                                   ((16, 16, 40), 1 << 14, (0, 1), 16), ((320, 12, 33), 1 << 14, (0.4, 0.5), 16), ((40, 33, 21), 4096, (-0.2, 1.1), 16),
-                                                  ((64, 30, 20), 1 << 14, (0, 1), 8)])
+                                                  ((64, 30, 20), 1 << 14, (0, 1), 8), ((70, 5, 256), 1 << 14, (0, 1), 16), ((66, 4, 300), 4096, (0, 1), 16)])
 def test_lattice_equals_the_same_points_queried(res, chunk, box, levels):
     """density_on_grid (rows of lattice points walked along z) against NerfNetwork::sdf on the same positions."""
     from neus2_amd.mesh import density_on_grid

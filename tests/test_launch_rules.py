@@ -27,6 +27,7 @@ extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels,
 		}
 	return 0;
 }
+extern "C" uint32_t walked_levels(const float* scale, float step) { return n2_lattice_walked_levels(scale, step); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
 
@@ -91,3 +92,11 @@ def test_gather_launch_of_two_lanes_a_point_stays_below_the_thread_limit(rules, 
     grid = np.zeros(2, np.uint32)
     rules.gather_visits(1 << 19, n, 16, 128, None, grid.ctypes.data_as(C.c_void_p))
     assert int(grid[0]) * 256 < 1 << 32 and int(grid[1]) < 1 << 16
+
+
+# lattices over the unit cube with 64 to 512 planes (the default table), a box of a tenth of it, a table of eight levels (the rest have scale 1)
+@pytest.mark.parametrize("planes,extent,levels,walked", [(64, 1, 16, 6), (128, 1, 16, 6), (208, 1, 16, 6), (224, 1, 16, 8), (256, 1, 16, 8), (272, 1, 16, 10), (384, 1, 16, 10),
+                                                         (512, 1, 16, 10), (64, 0.1, 16, 10), (64, 1, 8, 10), (1 << 20, 1, 16, 10), (2, 1, 16, 6)])
+def test_levels_the_lattice_walks(rules, planes, extent, levels, walked):
+    scale = [16 * 1.447 ** l - 1 if l < levels else 1.0 for l in range(16)]
+    assert rules.walked_levels((C.c_float * 16)(*scale), C.c_float(extent / planes)) == walked
