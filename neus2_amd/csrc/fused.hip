@@ -407,8 +407,10 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const Fused
 
 template <bool FULL>
 __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs a, uint32_t tiles, int by_xcd) {
-	// Bound by the lines the L1s fetch (four per sample on every level whose cells are smaller than the marching step)
-	// and, with slopes, by the vector unit: without its gathers it would still take 46 of 73 us.  Measured on the training
+	// Bound by the L1s: a query of 2^20 uniform points looks a line up in 87 % of a CU's clocks and fetches one of 128 bytes every 2.7
+	// (four per point on every level above the coarsest); the samples of a training step share lines along their rays (67 %,
+	// one every 5.1) but also hold the vector unit in 41 % of the cycles for their slopes: without its gathers the launch
+	// would still take 46 of 73 us.  Measured on the training
 	// step and dropped: one 8- or 16-byte load per pair of x neighbours instead of two 4-byte loads (+12 us), loads of the hashed
 	// levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then requested twice and
 	// a request is no cheaper) or carry the non-temporal hint (no change), the positions read as consecutive words and picked

@@ -77,7 +77,8 @@ constexpr uint32_t GRID_BLOCK = 256;
 constexpr uint32_t N_XCD = N2_XCDS;
 
 // Piece x of the level-major item list [begin[x], begin[x + 1]) belongs to XCD x; begin[N_XCD] = 0: no plan, n2_gather_item deals
-// the items (2^18 points with dy_dx: 84 us uniform, 60 in ray order; with the plan of the default costs 101 and 74).
+// the items (2^18 points with dy_dx, plain stores: 84 us uniform, 60 in ray order; with the plan of the default costs 101 and 74.  Streamed
+// stores lengthen the uniform launch to 91 and shorten what follows it: n2_jacobian_streams).
 struct N2XcdPlan {
 	uint32_t begin[N_XCD + 1];
 };

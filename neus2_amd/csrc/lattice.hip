@@ -13,8 +13,11 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice: 8.2 -> 5.8 ms, per slab of 7.6e6 points 153 us for six fine levels and 180 us for the walk, which its vector
-// and matrix instructions hold at two waves per SIMD (its plane values take 60 registers, the loads in flight 52).
+// 512^3 lattice: 8.2 -> 5.8 ms, per slab of 7.6e6 points 156 us for six fine levels and 182 us for the walk.  The walk runs two waves
+// per SIMD (its plane values take 60 registers, the loads in flight 52); it issues vector instructions in half of the
+// cycles, and its waves wait for memory in 43 % of theirs.
+// Rows that are no multiple of 64 leave lanes idle in their last run; against one gather per point and level: 80^3 124 -> 86 us, 144^3
+// 478 -> 280, 208^3 1088 -> 645, 272^3 1876 -> 1259, 464^3 6123 -> 5121, 80 x 512 x 400 3591 -> 1687 (64^3 71 -> 59, 128^3 342 -> 187, 256^3 1525 -> 1003).
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -88,7 +91,8 @@ __device__ __forceinline__ bool lattice_run(const LatticeArgs& a, uint32_t wave,
 // instruction costs the L1 one clock per group of four lanes at least, and up to four where the lanes' spacing makes their
 // banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks per 4-byte load).  So the wave loads the rows as a
 // whole, 16 bytes per lane, into LDS (FINE_CHUNKS of them per row) and picks the vertices there: for six levels of 2^22 points
-// 153 -> 89 us (L2 fills 52 us of it, LDS 58, measured by counters).  Runs longer than that (coarse lattices) and dense levels gather from memory.
+// 153 -> 89 us.  LDS is active in 73 % of the launch's cycles then, a third of that bank conflicts; of the lines it asks the L2s for
+// 91 % are there.  Runs longer than that (coarse lattices) and dense levels gather from memory.
 constexpr uint32_t FINE_CHUNKS = 128;
 
 __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArgs a, uint32_t blocks_per_level) {
@@ -229,7 +233,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 	for (int l = 0; l < NM; ++l) wy[l] = lane_f32(my_wy, l);
 	// the plane of vertices at `row0`, `row1` (byte offsets of its rows y, y + 1): four gathers, and their interpolation in x and y
 	// What depends on x is worked out at each plane, from an opaque copy of the position: kept across the loop, cell and weight of
-	// every level take 40 registers, and the walk needs three waves per SIMD to cover its loads.
+	// every level take 40 registers more than the 225 that two waves per SIMD leave room for.
 	auto place = [&](int l, float& w, uint32_t& c) {
 		float p = px;
 		asm volatile("" : "+v"(p));
@@ -423,7 +427,7 @@ __global__ void __launch_bounds__(64) lattice_frags_kernel(const hf* __restrict_
 
 uint64_t n2_lattice_frag_bytes() { return SDF_FRAG_COUNT * 1024ull; }
 
-// Slabs of at most `chunk` points; d_scratch holds LT_MAX_FINE 4-byte rows of `chunk` points, d_frags the fragment image.
+// d_scratch holds LT_MAX_FINE 4-byte rows of `chunk` points, d_frags the fragment image.
 int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice& lat, uint32_t chunk, void* d_scratch, void* d_frags, float* d_out) {
 	const N2LevelTable& tab = *nets.tab;
 	LatticeArgs a{};

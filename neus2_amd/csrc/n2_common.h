@@ -267,6 +267,8 @@ __device__ __forceinline__ void n2_store3(float* p, n2_float3 v) {
 	if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<n2_float3*>(p));
 	else *reinterpret_cast<n2_float3*>(p) = v;
 }
-// The encoding's Jacobian (384 bytes per point of sixteen levels) is streamed from 64 MiB on.  Forward, scatter and input gradient
-// in us, plain | streamed: 2^18 points (96 MiB) 241 | 226, 2^17 (48 MiB) 126 | 124, 2^16 80 | 83.
+// The encoding's Jacobian (384 bytes per point of sixteen levels) is streamed from 64 MiB on.  Forward, scatter and input gradient in
+// us with nothing | the loads | the stores | both streamed: 2^18 uniform points (96 MiB) 219 | 203 | 204 | 195, along rays 169 | 165 | 163 | 157;
+// 2^19 434 | 430 | 430 | 423; 2^17 (48 MiB) 108 in all four, along rays 92.  The SDF network with the eikonal term, 2^18: uniform 283 | 285 | 288 | 287,
+// along rays 244 | 236 | 241 | 235; 2^17 155 | 154 | 155 | 153.
 static inline bool n2_jacobian_streams(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (64ull << 20); }
