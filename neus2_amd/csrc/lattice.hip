@@ -144,9 +144,8 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 		out += plane;
 	};
 	// chunks of four entries that the run meets: from c_lo's to the one behind c_hi's
-	const uint32_t c_first = lane_u32(cx, 0), c_last = lane_u32(cx, 63);
-	const bool up = (int32_t)(c_last - c_first) >= 0;
-	const uint32_t c_lo = (up ? c_first : c_last) & ~3u, chunks = (((up ? c_last : c_first) + 1u - c_lo) >> 2) + 1u;
+	uint32_t c_lo, chunks;
+	n2_lattice_chunks(lane_u32(cx, 0), lane_u32(cx, 63), c_lo, chunks);
 	if (hashed && chunks <= FINE_CHUNKS) {
 		// (lanes behind the last chunk load it again, into a slot nobody reads)
 		const uint32_t o0 = ((c_lo + 4u * min(lane, chunks - 1u)) & (entries - 1u)) << 2, o1 = ((c_lo + 4u * min(lane + 64u, chunks - 1u)) & (entries - 1u)) << 2;

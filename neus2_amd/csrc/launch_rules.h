@@ -39,6 +39,15 @@ static inline N2LatticeSlab n2_lattice_slab(const uint32_t res[3], uint64_t poin
 	return {nx, res[1], rows / res[1] < res[2] ? rows / res[1] : res[2]};
 }
 
+// The chunks of four entries along x that the cells c_first .. c_last of a run and their neighbours at +1 lie in (either end may be
+// the larger one): `chunks` of them from cell c_lo on.  Cells are signed: a box far outside the unit cube has them saturated at
+// the ends of the 32-bit range, 2^32 apart.
+N2_HD inline void n2_lattice_chunks(uint32_t c_first, uint32_t c_last, uint32_t& c_lo, uint32_t& chunks) {
+	const int64_t a = (int32_t)c_first, b = (int32_t)c_last, lo = (a < b ? a : b) & ~(int64_t)3, hi = (a < b ? b : a) + 1;
+	c_lo = (uint32_t)lo;
+	chunks = (uint32_t)((hi - lo) >> 2) + 1u;
+}
+
 // Levels that the lattice's walk keeps planes of, by the step along z (it is right for any level and step).  A level whose cells are
 // larger than a step crosses into a new plane less than once per step; of one whose cells are smaller every step meets two
 // planes and nothing is kept, but up to about 1.15 cells per step that costs less than its features' way through memory.

@@ -27,6 +27,7 @@ extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels,
 		}
 	return 0;
 }
+extern "C" void lattice_chunks(uint32_t first, uint32_t last, uint32_t* out) { n2_lattice_chunks(first, last, out[0], out[1]); }
 extern "C" uint32_t walked_levels(const float* scale, float step) { return n2_lattice_walked_levels(scale, step); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
@@ -100,3 +101,14 @@ def test_gather_launch_of_two_lanes_a_point_stays_below_the_thread_limit(rules, 
 def test_levels_the_lattice_walks(rules, planes, extent, levels, walked):
     scale = [16 * 1.447 ** l - 1 if l < levels else 1.0 for l in range(16)]
     assert rules.walked_levels((C.c_float * 16)(*scale), C.c_float(extent / planes)) == walked
+
+
+# cells of a run's ends: rising, falling, one cell, negative, and the ends of the 32-bit range (boxes far outside the unit cube)
+@pytest.mark.parametrize("first,last", [(0, 0), (3, 4), (8, 519), (519, 8), (-1, 2), (-517, -3), (-2 ** 31, 2 ** 31 - 1), (2 ** 31 - 1, -2 ** 31), (-2 ** 31, 5), (0, 2 ** 31 - 1),
+                                        (2 ** 31 - 1, 2 ** 31 - 1), (-2 ** 31, -2 ** 31)])
+def test_lattice_chunks_hold_every_cell_of_the_run(rules, first, last):
+    out = (C.c_uint32 * 2)()
+    rules.lattice_chunks(C.c_uint32(first % 2 ** 32), C.c_uint32(last % 2 ** 32), out)
+    lo, chunks = C.c_int32(out[0]).value, out[1]
+    a, b = min(first, last), max(first, last)
+    assert lo % 4 == 0 and lo <= a < lo + 4 and lo + 4 * (chunks - 1) <= b + 1 < lo + 4 * chunks
