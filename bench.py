@@ -3,7 +3,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload step|grid|sdf|lattice|occupancy|mesh] [--no-cpu-baseline]
 
-A step is one full static NeuS2 training step (configuration 4 of BASELINE.json) on a synthetic scene: an analytic sphere of
+A step is one full static NeuS2 training step on a synthetic scene: an analytic sphere of
 radius 0.3, Lambertian-textured, seen by 64 cameras at 512x512 on a sphere of radius 2; rays are marched through a
 128^3 occupancy bitfield and compacted to 2^18 samples; hash grid + SDF MLP + colour MLP forward, first- and
 second-order backward, compositing and Adam, all on the GPU.  Prints ONE JSON line.
@@ -84,14 +84,14 @@ def summarize_traffic(fetch_csv, write_csv, copy_mib):
         return {k: statistics.median(v[len(v) // 2:]) * 1024.0 * factor for k, v in per.items()}, factor
     fetch, ff = load(fetch_csv, "FETCH_SIZE")
     write, wf = load(write_csv, "WRITE_SIZE")
-    cmd = ("rocprofv3 --pmc {c} --kernel-trace --output-format csv -d gpurun_out/pp/{d} -o f -- python3 bench.py --no-cpu-baseline "
+    cmd = ("rocprofv3 --pmc {c} --kernel-trace --output-format csv -d /tmp/pp/{d} -o f -- python3 bench.py --no-cpu-baseline "
            "--trained-steps 0 --extra-regions 0 --calibrate-copy %d --steps 20 --warmup 5" % copy_mib)
     kernels = {k: {"fetch_bytes": int(fetch.get(k, 0.0)), "write_bytes": int(write.get(k, 0.0))}
                for k in sorted(set(fetch) | set(write)) if "_kernel" in k and not k.startswith("at::")}
     return {"workload": "default benchmark: full training step, 2^18 batch", "command_fetch": cmd.format(c="FETCH_SIZE", d="fetch"),
             "command_write": cmd.format(c="WRITE_SIZE", d="write"),
-            "then": "python3 bench.py --calibrate-copy %d --summarize-traffic gpurun_out/pp/fetch/f_counter_collection.csv "
-                    "gpurun_out/pp/write/f_counter_collection.csv > profiles/training_step_2p18_hbm_traffic.json" % copy_mib,
+            "then": "python3 bench.py --calibrate-copy %d --summarize-traffic /tmp/pp/fetch/f_counter_collection.csv "
+                    "/tmp/pp/write/f_counter_collection.csv > profiles/training_step_2p18_hbm_traffic.json" % copy_mib,
             "calibration": {"copy_mib": copy_mib, "fetch_factor": ff, "write_factor": wf,
                             "note": "factor = known bytes of the calibration copy / what the counter read for it"},
             "unit": "bytes per launch (median of the steady-state launches)", "kernels": kernels}
@@ -248,7 +248,7 @@ def run_step_workload(args):
         "ms_per_step": elapsed / args.steps * 1e3,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16", "data": "synthetic",
-        "config": {"workload": "full NeuS2 static training step (BASELINE configs[3]): analytic sphere r=0.3, 64 cameras 512x512 "
+        "config": {"workload": "full NeuS2 static training step: analytic sphere r=0.3, 64 cameras 512x512 "
                                "on a radius-2 sphere, 128^3 occupancy bitfield, rays compacted to 2^18 samples; hash grid "
                                "L=16 F=2 T=2^19 + SDF MLP 48-64-16 + colour MLP 48-64-64-16, first and second order backward, "
                                "compositing, Adam",
@@ -345,7 +345,7 @@ def timed_best(fn, budget_s=15.0, min_runs=2, max_runs=8):
 
 
 def run_grid_workload(args):
-    """Configuration 2 of BASELINE.json: hash-grid encoding only, forward + backward on 2^18 uniform points."""
+    """Hash-grid encoding only, forward + backward on 2^18 uniform points."""
     import torch
     from neus2_amd import capi
     from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
@@ -383,7 +383,7 @@ def run_grid_workload(args):
     result = {"metric": "hash-grid fwd+bwd samples/sec @2^18 batch (1 GPU)", "value": args.steps * TARGET / elapsed, "unit": "samples/s",
               "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": elapsed / args.steps * 1e3,
               "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f16", "data": "synthetic",
-              "config": {"workload": "hash-grid encoding only, forward + backward (BASELINE configs[1])", "batch": TARGET},
+              "config": {"workload": "hash-grid encoding only, forward + backward", "batch": TARGET},
               "roofline": {"kernel": dom, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                            "frac": achieved / HBM_PEAK_GBS, "traffic": None, "algorithmic_bytes_per_sample": ALGO_BYTES[dom],
                            "samples_per_launch": TARGET, "avg_launch_us": kernels[dom]["avg_us"]},
@@ -405,7 +405,7 @@ def run_grid_workload(args):
 
 
 def run_sdf_workload(args):
-    """Configuration 3 of BASELINE.json: grid + SDF MLP with the eikonal second-order path on 2^18 uniform points: forward,
+    """Grid + SDF MLP with the eikonal second-order path on 2^18 uniform points: forward,
     normals, backward of mean|sdf| + 0.1 mean(|grad sdf| - 1)^2 through the encoding and the MLP weights."""
     import numpy as np
     import torch
@@ -448,7 +448,7 @@ def run_sdf_workload(args):
               "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": elapsed / args.steps * 1e3,
               "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f16", "data": "synthetic",
               "config": {"workload": "hash grid + SDF MLP 48-64-16, forward, normals, first and second order backward of "
-                                     "mean|sdf| + 0.1 mean(|grad sdf| - 1)^2 (BASELINE configs[2]); 2^18 uniform points",
+                                     "mean|sdf| + 0.1 mean(|grad sdf| - 1)^2; 2^18 uniform points",
                          "batch": TARGET, "loss": float(loss), "kernel_ms_per_step": total},
               "roofline": {"kernel": "grid_backward_params (merged first+second order scatter)", "bound": "hbm", "achieved": achieved,
                            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": None,
@@ -467,7 +467,7 @@ def run_sdf_workload(args):
 
 
 def run_lattice_workload(args):
-    """Configuration 5 of BASELINE.json: SDF inference for mesh extraction (hash grid + SDF MLP forward, fp16) over the 512^3
+    """SDF inference for mesh extraction (hash grid + SDF MLP forward, fp16) over the 512^3
     lattice p = (i, j, k) / 512, in chunks of 2^22 points; a step is one chunk, chunks are visited in order, each as one
     n2_field_sdf on points in lattice order (one gather per point and level, all 16 output rows).  n2_density_on_grid, which walks
     the lattice instead, is timed after it (density_on_grid)."""
@@ -516,7 +516,7 @@ def run_lattice_workload(args):
     result = {"metric": "SDF inference points/sec over a 512^3 lattice in 2^22-point chunks (1 GPU)", "value": args.steps * CH / elapsed,
               "unit": "points/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": elapsed / args.steps * 1e3,
               "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f16", "data": "synthetic",
-              "config": {"workload": "hash grid + SDF MLP forward over the 512^3 lattice (BASELINE configs[4]), geometric-init SDF MLP, "
+              "config": {"workload": "hash grid + SDF MLP forward over the 512^3 lattice, geometric-init SDF MLP, "
                                      "grid U(-1e-4, 1e-4) seed 1; n2_field_sdf on points in lattice order (n2_density_on_grid beside it: density_on_grid)", "chunk": CH, "chunks_in_lattice": n_chunks,
                          "sdf_mean_abs": float(out[0].float().abs().mean())},
               "roofline": {"kernel": dom, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -624,8 +624,8 @@ def run_occupancy_workload(args):
 
 
 def run_mesh_workload(args):
-    """The consumer of configuration 5 of BASELINE.json: marching cubes over the 512^3 SDF lattice (count per tile, prefix sums over
-    the tiles, vertices, faces, normals).  The lattice is evaluated once, untimed (that part is `--workload lattice`); a step is one full extraction."""
+    """The consumer of the SDF lattice: marching cubes over the 512^3 SDF lattice (one bit per point, counts and prefix
+    sums over words of 64 points, vertices, faces, normals).  The lattice is evaluated once, untimed (that part is `--workload lattice`); a step is one full extraction."""
     import numpy as np
     import torch
     from neus2_amd.mesh import density_on_grid, marching_cubes

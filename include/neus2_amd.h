@@ -397,7 +397,7 @@ int n2_field_density(n2_field_t* field, n2_stream_t stream, const float* d_xyz, 
 /* ------------------------------------------------------------------------
  * The SDF network trained on its own with the eikonal term (no colour branch): the element-wise steps that
  * NerfNetwork performs between the encoding's and the network's calls, for a caller that composes
- * n2_grid_* and n2_mlp_* itself (this repository's neus2_amd/sdf_net.py, BASELINE configuration 3):
+ * n2_grid_* and n2_mlp_* itself (this repository's neus2_amd/sdf_net.py):
  *   n2_sdf_pack_input     rows 0..2 of the network input = (T)x - (T)0.5 and zero padding rows behind the encoding
  *                         (fill_positions_view_with_fixed_offset, nerf_network.h:193-195, common_operation.cuh:186-199)
  *   n2_sdf_eikonal_loss   d_normal_encoding holds the encoding's backward of rows 3.. of d sdf / d input (n2_grid_backward

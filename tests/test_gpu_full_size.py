@@ -152,9 +152,9 @@ def test_lattice_512_chunks_and_subsample(oracle):
 
 
 def test_sdf_eikonal_step_2p18_against_oracle(oracle):
-    """BASELINE configuration 3 at its full size, through the entry points that configuration's benchmark times
-    (n2_sdf_pack_input, n2_grid_forward with the Jacobian, n2_mlp_forward_and_input_gradient, n2_sdf_eikonal_loss,
-    n2_mlp_backward, n2_grid_backward_fused, n2_mlp_backward_backward_input): 2^18 points uniform in the unit cube, the
+    """The SDF network with the eikonal term at its full size, through the entry points that its benchmark times
+    (n2_sdf_pack_input, n2_grid_forward with the Jacobian, n2_mlp_forward_and_input_gradient, n2_sdf_normals_and_eikonal_loss,
+    n2_mlp_backward_and_second_order, n2_grid_backward_fused): 2^18 points uniform in the unit cube, the
     SDF, the normals, the loss, the MLP's weight gradients and the encoding's gradients level by level against the oracle's
     composition, at the tolerances of the small test (nerf_network.h:184-238, 402-429, 534-571)."""
     from neus2_amd.sdf_net import SdfNet

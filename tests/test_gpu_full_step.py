@@ -1,4 +1,4 @@
-"""The training step at the benchmark's shape (BASELINE configuration 4: 64 cameras at 512 x 512, 2^18-sample batch,
+"""The training step at the benchmark's shape (64 cameras at 512 x 512, 2^18-sample batch,
 capacity 16 x 2^18, sample generation running ahead), checked stage by stage against the oracle
 (Testbed::train_nerf_step, src/testbed_nerf.cu:3717-3987)."""
 import os
