@@ -218,7 +218,8 @@ __device__ __forceinline__ float window_t(float t_first, uint32_t lane) {
 // groups further on it no longer matters where it came in.  A jump therefore lands JUMP_LEAD steps before the first step
 // that may be occupied and only counts when the landing window is of that regular kind throughout and inside the cube;
 // else the wave goes back and walks.  (A trained field's step, 36096 rays through a thin shell, kernels beside the forward in
-// us: count 112 -> 95, emit 35 -> 23, the forward's first gather beside them 108 -> 77; the step 601 -> 561.)
+// us, jumps alone: count 108 -> 98, emit 22 -> 19, the forward's first gather beside them 82 -> 76; the step 542 -> 532.  With the
+// setups by one lane: 112 -> 95, 35 -> 23, 108 -> 77; 601 -> 561.)
 constexpr uint32_t JUMP_LEAD = 20, JUMP_MIN = 24;
 __device__ __forceinline__ uint32_t march_wave(const RaySetup& r, const uint8_t* __restrict__ bitfield, const uint32_t* __restrict__ coarse,
                                                uint32_t* __restrict__ mask, float* __restrict__ t_first_out) {
