@@ -39,11 +39,12 @@ struct LatticeArgs {
 	const hf* frags;          // fragment image of the SDF network
 	float sdf_bias;
 	N2Lattice lat;
-	uint32_t x0, nx, y0, ny, z0, nz;  // the slab: columns x0 .. x0 + nx of rows y0 .. y0 + ny of planes z0 .. z0 + nz
+	uint32_t y0, ny, z0, nz;  // the slab: rows y0 .. y0 + ny of planes z0 .. z0 + nz,
 	uint32_t x_runs, walk;    // runs of 64 points per row of the slab; planes per wave
 	uint32_t first_fine;      // levels first_fine .. n_levels - 1 come from `features`
 	uint32_t* features;       // [n_levels - first_fine][nz ny nx] half2
 	float* out;               // row 0 of point (x0, y0, z0)
+	uint32_t x0, nx;          // columns x0 .. x0 + nx of the slab
 };
 
 // coordinate of lattice index c on axis d: each step rounded on its own (positions are part of a bit-exact contract)
@@ -75,11 +76,11 @@ __device__ __forceinline__ uint32_t lt_pack(float a, float b) {
 	return __builtin_bit_cast(uint32_t, h);
 }
 
-// The wave's run: x of the lane (past the slab's last column in a run that is not full), y, first plane.  False: nothing to do.
+// The wave's run: the lane's column of the slab (past the last one in a run that is not full), y, first plane.  False: nothing to do.
 __device__ __forceinline__ bool lattice_run(const LatticeArgs& a, uint32_t wave, uint32_t& x, uint32_t& y, uint32_t& z, uint32_t& nz) {
 	const uint32_t xr = wave % a.x_runs, rest = wave / a.x_runs, yy = rest % a.ny, zz = rest / a.ny;
 	if (zz * a.walk >= a.nz) return false;
-	x = a.x0 + xr * 64u + (threadIdx.x & 63u);
+	x = xr * 64u + (threadIdx.x & 63u);
 	y = a.y0 + yy;
 	z = a.z0 + zz * a.walk;
 	nz = min(a.walk, a.nz - zz * a.walk);
@@ -101,10 +102,9 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x % blocks_per_level) * (LT_BLOCK / 64) + (threadIdx.x >> 6));
 	uint32_t x, y, z, nz;
 	if (!lattice_run(a, wave, x, y, z, nz)) return;
-	const uint32_t x_last = a.x0 + a.nx - 1u;
-	const bool inside = x <= x_last;
+	const bool inside = x < a.nx;
 	const uint32_t lane = threadIdx.x & 63u, plane = a.nx * a.ny;
-	uint32_t* out = a.features + (size_t)(level - a.first_fine) * plane * a.nz + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + (x - a.x0);
+	uint32_t* out = a.features + (size_t)(level - a.first_fine) * plane * a.nz + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + x;
 	if (level >= a.active_levels) {
 		for (uint32_t k = 0; k < nz; ++k)
 			if (inside) out[(size_t)k * plane] = 0u;
@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	const bool hashed = (a.hash_mask >> level) & 1u;
 	float wx, wy, wz;
 	uint32_t cx, cy, cz;
-	n2_locate(lattice_coord(a.lat, 0, min(x, x_last)), scale, wx, cx);
+	n2_locate(lattice_coord(a.lat, 0, a.x0 + min(x, a.nx - 1u)), scale, wx, cx);
 	n2_locate(lattice_coord(a.lat, 1, y), scale, wy, cy);
 	n2_locate(lattice_coord(a.lat, 2, z + min(lane, nz - 1u)), scale, wz, cz);  // lane k: plane z + k (at most 64 of them)
 	// lane k: the four rows of vertices of plane z + k and their weights
@@ -211,9 +211,9 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (LT_BLOCK / 64) + (threadIdx.x >> 6));
 	uint32_t x, y, z, nz;
 	if (!lattice_run(a, wave, x, y, z, nz)) return;
-	const uint32_t lane = threadIdx.x & 63u, rx = a.lat.res[0], plane = a.nx * a.ny, x_last = a.x0 + a.nx - 1u;
-	const bool inside = x <= x_last;
-	const float px = lattice_coord(a.lat, 0, min(x, x_last)), py = lattice_coord(a.lat, 1, y);
+	const uint32_t lane = threadIdx.x & 63u, rx = a.lat.res[0], plane = a.nx * a.ny;
+	const bool inside = x < a.nx;
+	const float px = lattice_coord(a.lat, 0, a.x0 + min(x, a.nx - 1u)), py = lattice_coord(a.lat, 1, y);
 	const char* base[NM];
 #pragma unroll
 	for (int l = 0; l < NM; ++l) base[l] = reinterpret_cast<const char*>(a.table + a.offset[l]);
@@ -299,9 +299,9 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 #pragma unroll
 	for (int l = 0; l < NM; ++l) lo[l] = hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched-off levels
 	both_planes(on, my_cz);
-	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + (min(x, x_last) - a.x0);
+	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + min(x, a.nx - 1u);
 	const size_t feat_level = (size_t)plane * a.nz;
-	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + (x - a.x0);
+	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + x;
 	const uint32_t g = lane >> 5;  // of the lanes with g = 0 a tile's operands take the coordinates
 	const hf ycoord = (hf)py - (hf)0.5f;
 	// tile 0 works for lanes 0..31, tile 1 for lanes 32..63: the x coordinate of both, for the lanes that need it (g = 0)
