@@ -81,6 +81,7 @@ constexpr uint32_t N_XCD = N2_XCDS;
 // stores lengthen the uniform launch to 91 and shorten what follows it: n2_jacobian_streams).
 struct N2XcdPlan {
 	uint32_t begin[N_XCD + 1];
+	uint32_t height;  // of a launch without a plan: its workgroups in y
 };
 
 // The (level, tile) item of this workgroup, or false if its XCD's piece is shorter than the longest one.
@@ -155,7 +156,7 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable t
                                                                   uint32_t dim_stride, const __half2* __restrict__ params,
                                                                   __half* __restrict__ out, float* __restrict__ dy_dx) {
 	uint32_t level, tile;
-	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_gather_item(blockIdx.x, blockIdx.y, gridDim.y, tab.n_levels, tiles, level, tile))) return;
+	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_gather_item(blockIdx.x, blockIdx.y, plan.height, tab.n_levels, tiles, level, tile))) return;
 	const uint32_t i = tile * FWD_POINTS + (threadIdx.x >> 1), b = threadIdx.x & 1u;
 	if (i >= N) return;  // both lanes of a pair share i, so pairs leave together
 #define CALL(M) grid_forward_pair<M, WANT_DYDX, STREAM>(tab, level, i, b, N, xyz, point_stride, dim_stride, params, out, dy_dx)
@@ -1149,8 +1150,9 @@ N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_x
 		return N2_OK;
 	}
 	const uint32_t tiles = (n_points + FWD_POINTS - 1) / FWD_POINTS;
-	plan.begin[N_XCD] = 0;
 	const N2GatherGrid dealt = n2_gather_grid(N2_ENCODING_XCD_MAX, n_points, grid->tab.n_levels, FWD_POINTS);
+	plan.begin[N_XCD] = 0;
+	plan.height = dealt.y;
 	const dim3 grid_dim = grid->costs_set ? dim3(make_xcd_plan(grid, tiles, plan) * N_XCD) : dim3(dealt.x, dealt.y), block(GRID_BLOCK);
 	const bool streams = n2_jacobian_streams(n_points, grid->tab.n_levels * grid->n_features);
 	auto* const kernel = !d_dy_dx ? grid_forward_kernel<false, false> : streams ? grid_forward_kernel<true, true> : grid_forward_kernel<true, false>;
