@@ -139,7 +139,6 @@ constexpr uint32_t BWD_RGB_FRAGS = FragMap<3, 2>::SEL, BWD_SDF_FRAGS = FragMap<3
 static_assert(FF_COUNT * 1024 == N2_FUSED_FRAG_FORWARD && BWD_RGB_FRAGS * 1024 == N2_FUSED_FRAG_RGB && BWD_SDF_FRAGS * 1024 == N2_FUSED_FRAG_SDF,
               "the image's parts as n2_common.h sizes them");
 constexpr uint32_t FG_BLOCK = 256;  // threads of a gather workgroup (128: the gather 1.8 us shorter, the step 5 us longer; 512: +2 / +5; 1024: +11 / +11)
-constexpr uint32_t FG_PAIRS = FG_BLOCK / 2;
 constexpr uint32_t FRAG_BLOCKS = ((FF_COUNT + BWD_RGB_FRAGS + BWD_SDF_FRAGS) * 64 + FG_BLOCK - 1) / FG_BLOCK;
 __device__ __forceinline__ void write_frag_image(const FusedArgs& a, uint32_t block) {
 	const uint32_t idx = block * FG_BLOCK + threadIdx.x;
@@ -288,14 +287,16 @@ __device__ __forceinline__ void sh4(float x, float y, float z, float* o) {
 // level-major gather: features into the SDF net's input rows, slopes as fp16
 // ----------------------------------------------------------------------------
 
-// Full field: one (sample, level) item, features and slopes; the sample's coordinates are row `src` of the input (the [N][7]
-// coordinates, or three rows of positions), what it writes goes to column i.
-__device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t src) {
+// Full field: one (sample, level) item, features and slopes; the item is column i of the matrices, and its
+// coordinates are row i of the input (the [N][7] coordinates, or three rows of positions).  (With the pairs of n2_encode_level a step of
+// 2^18 samples takes 390 us instead of 383, 52344 samples forward and backward 110 instead of 106: these items hold the vector unit as
+// much as the L1.)
+__device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, uint32_t i) {
 	const uint32_t N = a.N;
 	// (full field: the positions from the coordinate rows, or from three rows of their own when the caller has them: a wave
 	// then reads two lines per coordinate instead of fourteen)
 	const bool rows = a.pos == nullptr;
-	const float* q = rows ? a.coords + (size_t)src * 7 : a.pos + (size_t)src * a.ps;
+	const float* q = rows ? a.coords + (size_t)i * 7 : a.pos + (size_t)i * a.ps;
 	const size_t qs = rows ? 1 : a.ds;
 	const float p[3] = {q[0], q[qs], q[2 * qs]};
 	if (level == 0) {
@@ -328,28 +329,24 @@ __device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, 
 	a.slopes[(size_t)level * N + i] = n2_slopes_pack(six);
 }
 
-// Inference on points in no particular order (features only): one (sample, level) item by a PAIR of adjacent lanes.  Lane b
-// gathers the four (y, z) corners of x corner b: the two x corners are neighbours in the table, so the pair reads one line and
-// the L1 looks up half as many as with eight gathers by one lane (2^20 uniform points 330 -> 291 us, 2^21 cells of the
-// occupancy grid 432 -> 407); then lane b finishes feature b.  (The full field's items hold the vector unit as much as the L1: there
-// the pair's doubled index arithmetic costs more than it saves, 80 us against 73 at the training step's batch.)
+// Small queries: one (sample, level) item by a PAIR of adjacent lanes.  Lane b gathers the four (y, z) corners of x corner b, and
+// finishes feature b.
 struct PairItem {
 	uint32_t raw[4];
 	float w[3];
 };
 __device__ __forceinline__ void pair_fetch(const FusedArgs& a, uint32_t level, const float (&p)[3], uint32_t b, PairItem& it) {
 	const uint32_t res = a.lv.res[level], entries = a.lv.entries[level];
-	const bool hashed = (a.lv.hash_mask >> level) & 1u;
-	uint32_t c[3];
+	uint32_t c[3], at[4];
 #pragma unroll
 	for (int d = 0; d < 3; ++d) n2_locate(p[d], a.lv.scale[level], it.w[d], c[d]);
-	const __half2* P = a.table + a.lv.offset[level];
+	if ((a.lv.hash_mask >> level) & 1u) {
+		n2_hash_terms(c);
+		n2_corner_bytes<N2_LEVEL_HASH>(entries, res, c[0] + b, c[1], c[2], at);
+	} else n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, c[0] + b, c[1], c[2], at);
+	const char* base = reinterpret_cast<const char*>(a.table + a.lv.offset[level]);
 #pragma unroll
-	for (uint32_t k = 0; k < 4; ++k) {
-		const uint32_t y = c[1] + (k & 1u), z = c[2] + (k >> 1);
-		const uint32_t at = hashed ? n2_entry<N2_LEVEL_HASH>(entries, res, c[0] + b, y, z) : n2_entry<N2_LEVEL_DENSE>(entries, res, c[0] + b, y, z);
-		it.raw[k] = *reinterpret_cast<const uint32_t*>(P + at);
-	}
+	for (uint32_t k = 0; k < 4; ++k) it.raw[k] = *reinterpret_cast<const uint32_t*>(base + at[k]);
 }
 __device__ __forceinline__ float pair_finish(const PairItem& it, uint32_t b) {
 	float2 v[4];
@@ -357,22 +354,29 @@ __device__ __forceinline__ float pair_finish(const PairItem& it, uint32_t b) {
 	for (int k = 0; k < 4; ++k) v[k] = h2f(it.raw[k]);
 	const float wy = it.w[1], wz = it.w[2], uy = 1.f - wy, uz = 1.f - wz;
 	const float w00 = uy * uz, w10 = wy * uz, w01 = uy * wz, w11 = wy * wz;
-	const float s0 = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, w11 * v[3].x)));
-	const float s1 = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, w11 * v[3].y)));
+	// (the first products as multiply-adds too: those take half-precision operands as they are)
+	const float s0 = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, fmaf(w11, v[3].x, 0.f))));
+	const float s1 = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, fmaf(w11, v[3].y, 0.f))));
 	// lane b keeps feature b of its own x plane and receives feature b of the partner's
 	const float mine = b ? s1 : s0, other = n2_pair_swap(b ? s0 : s1);
-	return fmaf(1.f - it.w[0], b ? other : mine, it.w[0] * (b ? mine : other));
+	float feat = fmaf(1.f - it.w[0], b ? other : mine, it.w[0] * (b ? mine : other));
+	asm volatile("" : "+v"(feat));  // rounded to fp32 before fp16, as in the gather kernels: one instruction could do both and round once
+	return feat;
 }
-__device__ __forceinline__ void gather_pair(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t b) {
-	const float* q = a.pos + (size_t)i * a.ps;
-	const float p[3] = {q[0], q[a.ds], q[2 * (size_t)a.ds]};
-	float feat = 0.f;
+// Inference on points in no particular order: the features of one (point, level) item per lane
+__device__ __forceinline__ void gather_features(const FusedArgs& a, uint32_t level, uint32_t i, bool store) {
+	float feat[2] = {0.f, 0.f}, unused[2][3];
 	if (level < a.lv.active_levels) {  // a switched-off level: zero features
-		PairItem it;
-		pair_fetch(a, level, p, b, it);
-		feat = pair_finish(it, b);
+		const float* q = a.pos + (size_t)i * a.ps;
+		const float p[3] = {q[0], q[a.ds], q[2 * (size_t)a.ds]};
+		const uint32_t entries = a.lv.entries[level], res = a.lv.res[level];
+		const char* base = reinterpret_cast<const char*>(a.table + a.lv.offset[level]);
+		if ((a.lv.hash_mask >> level) & 1u) n2_encode_level<N2_LEVEL_HASH, false>(base, entries, res, a.lv.scale[level], p, 1.f, feat, unused);
+		else n2_encode_level<N2_LEVEL_DENSE, false>(base, entries, res, a.lv.scale[level], p, 1.f, feat, unused);
 	}
-	a.sdf_in[(size_t)(3 + 2 * level + b) * a.N + i] = (hf)feat;
+	if (!store) return;
+	a.sdf_in[(size_t)(3 + 2 * level) * a.N + i] = (hf)feat[0];
+	a.sdf_in[(size_t)(4 + 2 * level) * a.N + i] = (hf)feat[1];
 }
 
 // first column and number of samples of a listed pass
@@ -401,20 +405,19 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const Fused
 	const uint32_t tiles = (count + FG_BLOCK - 1) / FG_BLOCK;
 	for (uint32_t tile = first_tile; tile < tiles; tile += est_tiles) {
 		const uint32_t j = tile * FG_BLOCK + threadIdx.x;
-		if (j < count) gather_item(a, level, begin + j, begin + j);
+		if (j < count) gather_item(a, level, begin + j);
 	}
 }
 
 template <bool FULL>
 __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs a, uint32_t tiles, int by_xcd) {
-	// Bound by the L1s: a query of 2^20 uniform points looks a line up in 87 % of a CU's clocks and fetches one of 128 bytes every 2.7
-	// (four per point on every level above the coarsest); the samples of a training step share lines along their rays (67 %,
-	// one every 5.1) but also hold the vector unit in 41 % of the cycles for their slopes: without its gathers the launch
-	// would still take 46 of 73 us.  Measured on the training
-	// step and dropped: one 8- or 16-byte load per pair of x neighbours instead of two 4-byte loads (+12 us), loads of the hashed
-	// levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then requested twice and
-	// a request is no cheaper) or carry the non-temporal hint (no change), the positions read as consecutive words and picked
-	// apart in LDS (+9).
+	// Bound by lines on their way from the L2s to the L1s (n2_encode_level): a query of 2^20 uniform points takes one in every 2.6 clocks of
+	// a CU, four per point on every level above the coarsest, and the address units are busy in 95 % of the clocks; the samples of a
+	// training step share lines along their rays (one every 4.7, address units busy in 76 %) but also hold the vector unit in 41 % of the
+	// cycles for their slopes: without its gathers the launch would still take 46 of 71 us.  Measured on the training
+	// step and dropped: loads of the hashed levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then
+	// requested twice and a request is no cheaper) or carry the non-temporal hint (no change), the positions read as consecutive words
+	// and picked apart in LDS (+9).
 	// Staging the coarse levels in LDS has nothing to win: with all caches cold, levels 0..2 together add 2 us to the launch
 	// and the five dense levels 4 us, against 5 to 6 us for each of the fine hashed levels and 19 us for reading the
 	// positions and writing 320 bytes of features and slopes per sample.
@@ -430,10 +433,14 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 	// (the full field's workgroups are counted along x alone)
 	const uint32_t y = FULL && !by_xcd ? blockIdx.x / tiles : blockIdx.y, x = FULL ? blockIdx.x - y * tiles : blockIdx.x;
 	if (!n2_gather_item(x, y, by_xcd ? 1u : a.n_levels, a.n_levels, tiles, level, tile)) return;
-	const uint32_t i = FULL ? tile * FG_BLOCK + threadIdx.x : tile * FG_PAIRS + (threadIdx.x >> 1);
-	if (i >= a.N || (a.live && i >= *a.live)) return;  // (both lanes of a pair)
-	if (FULL) gather_item(a, level, i, i);
-	else gather_pair(a, level, i, threadIdx.x & 1u);
+	const uint32_t n_live = a.live ? min(*a.live, a.N) : a.N;
+	const uint32_t i = tile * FG_BLOCK + threadIdx.x;
+	if (FULL) {
+		if (i < n_live) gather_item(a, level, i);
+	} else {
+		if (tile * FG_BLOCK >= n_live) return;
+		gather_features(a, level, min(i, n_live - 1u), i < n_live);  // (lanes behind the last point take part in its pair's exchange)
+	}
 }
 
 // ----------------------------------------------------------------------------
@@ -745,8 +752,8 @@ bool n2_fused_supported(const N2LevelTable& tab, uint32_t sdf_hidden_layers, uin
 
 template <bool FULL>
 static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream_t s) {
-	const uint32_t per = FULL ? FG_BLOCK : FG_PAIRS, tiles = (a.N + per - 1) / per;
-	const N2GatherGrid g = n2_gather_grid(FULL ? N2_FIELD_XCD_MAX : N2_QUERY_XCD_MAX, a.N, tab.n_levels, per);
+	const uint32_t tiles = (a.N + FG_BLOCK - 1) / FG_BLOCK;
+	const N2GatherGrid g = n2_gather_grid(FULL ? N2_FIELD_XCD_MAX : N2_QUERY_XCD_MAX, a.N, tab.n_levels, FG_BLOCK);
 	const dim3 grid = FULL ? dim3(g.x * g.y + (a.frags ? FRAG_BLOCKS : 0u)) : dim3(g.x, g.y);
 	field_gather_kernel<FULL><<<grid, dim3(FG_BLOCK), 0, s>>>(a, tiles, g.y == 1u ? 1 : 0);
 }

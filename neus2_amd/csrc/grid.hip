@@ -96,56 +96,27 @@ __device__ __forceinline__ bool n2_xcd_item(const N2XcdPlan& plan, uint32_t tile
 // ----------------------------------------------------------------------------
 // forward
 // ----------------------------------------------------------------------------
-// A point is handled by a PAIR of adjacent lanes: lane bit 0 selects the x corner, each lane gathers the four
-// (y, z) corners of its x.  The two x corners are neighbours in the table (dense levels: index + 1; hashed
-// levels: x enters the hash with prime 1), so the two lanes of a pair read the same cache line almost always and
-// the memory pipeline, which looks up one line per clock, sees half as many lines per point.  The pair then
-// exchanges its partial sums and lane b finishes feature b.
-constexpr uint32_t FWD_POINTS = GRID_BLOCK / 2;  // points per workgroup and level
+constexpr uint32_t FWD_POINTS = GRID_BLOCK;  // points per workgroup and level
 
 template <uint32_t MODE, bool WANT_DYDX, bool STREAM>
-__device__ __forceinline__ void grid_forward_pair(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t b, uint32_t N,
+__device__ __forceinline__ void grid_forward_item(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t N,
                                                   const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                                   const __half2* __restrict__ params, __half* __restrict__ out,
                                                   float* __restrict__ dy_dx) {
-	const float scale = tab.scale[level];
-	const uint32_t entries = tab.entries[level], res = tab.resolution[level];
-	const __half2* P = params + tab.offset[level];
-	const size_t row = (size_t)level * 2 + b;
-	if (n2_level_masked(tab, level, i)) {  // both lanes of a pair share i
-		out[row * N + i] = __float2half_rn(0.f);
-		if (WANT_DYDX) {
-			n2_store3<STREAM>(dy_dx + (row * N + i) * 3, n2_float3{0.f, 0.f, 0.f});
-		}
-		return;
+	const uint32_t at = min(i, N - 1u);  // (lanes behind the last point take part in its pair's exchange)
+	const bool off = n2_level_masked(tab, level, at);
+	float feat[2] = {0.f, 0.f}, J[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+	if (!__all(off)) {
+		const float* q = xyz + (size_t)at * point_stride;
+		const float p[3] = {q[0], q[dim_stride], q[2 * (size_t)dim_stride]}, scale = tab.scale[level];
+		n2_encode_level<MODE, WANT_DYDX>(reinterpret_cast<const char*>(params + tab.offset[level]), tab.entries[level], tab.resolution[level], scale, p, scale, feat, J);
 	}
-	const N2Point p = n2_load_point(xyz, point_stride, dim_stride, i, scale);
-	const uint32_t gx = p.c[0] + b;
-	float2 v[4];
+	if (i >= N) return;
 #pragma unroll
-	for (uint32_t k = 0; k < 4; ++k) v[k] = __half22float2(P[n2_entry<MODE>(entries, res, gx, p.c[1] + (k & 1u), p.c[2] + (k >> 1))]);
-	const float wy = p.w[1], wz = p.w[2], uy = 1.f - wy, uz = 1.f - wz;
-	// this lane's x plane: bilinear value s, and its y and z differences ty, tz (k = y + 2 z)
-	float2 s, ty, tz;
-	s.x = fmaf(uy * uz, v[0].x, fmaf(wy * uz, v[1].x, fmaf(uy * wz, v[2].x, wy * wz * v[3].x)));
-	s.y = fmaf(uy * uz, v[0].y, fmaf(wy * uz, v[1].y, fmaf(uy * wz, v[2].y, wy * wz * v[3].y)));
-	if (WANT_DYDX) {
-		ty.x = fmaf(uz, v[1].x - v[0].x, wz * (v[3].x - v[2].x));
-		ty.y = fmaf(uz, v[1].y - v[0].y, wz * (v[3].y - v[2].y));
-		tz.x = fmaf(uy, v[2].x - v[0].x, wy * (v[3].x - v[1].x));
-		tz.y = fmaf(uy, v[2].y - v[0].y, wy * (v[3].y - v[1].y));
-	}
-	// lane b keeps feature b of its own plane and receives feature b of the partner's plane
-	const float s_mine = b ? s.y : s.x, s_other = n2_pair_swap(b ? s.x : s.y);
-	const float s_lo = b ? s_other : s_mine, s_hi = b ? s_mine : s_other;  // x corner 0 / 1
-	const float wx = p.w[0], ux = 1.f - wx;
-	out[row * N + i] = __float2half_rn(fmaf(ux, s_lo, wx * s_hi));
-	if (WANT_DYDX) {
-		const float ty_mine = b ? ty.y : ty.x, ty_other = n2_pair_swap(b ? ty.x : ty.y);
-		const float tz_mine = b ? tz.y : tz.x, tz_other = n2_pair_swap(b ? tz.x : tz.y);
-		const float w_mine = b ? wx : ux, w_other = b ? ux : wx;
-		n2_store3<STREAM>(dy_dx + (row * N + i) * 3, n2_float3{(s_hi - s_lo) * scale, fmaf(w_mine, ty_mine, w_other * ty_other) * scale,
-		                                                       fmaf(w_mine, tz_mine, w_other * tz_other) * scale});
+	for (uint32_t f = 0; f < 2; ++f) {
+		const size_t row = (size_t)level * 2 + f;
+		out[row * N + i] = __float2half_rn(off ? 0.f : feat[f]);
+		if (WANT_DYDX) n2_store3<STREAM>(dy_dx + (row * N + i) * 3, off ? n2_float3{0.f, 0.f, 0.f} : n2_float3{J[f][0], J[f][1], J[f][2]});
 	}
 }
 
@@ -157,9 +128,8 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable t
                                                                   __half* __restrict__ out, float* __restrict__ dy_dx) {
 	uint32_t level, tile;
 	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_gather_item(blockIdx.x, blockIdx.y, plan.height, tab.n_levels, tiles, level, tile))) return;
-	const uint32_t i = tile * FWD_POINTS + (threadIdx.x >> 1), b = threadIdx.x & 1u;
-	if (i >= N) return;  // both lanes of a pair share i, so pairs leave together
-#define CALL(M) grid_forward_pair<M, WANT_DYDX, STREAM>(tab, level, i, b, N, xyz, point_stride, dim_stride, params, out, dy_dx)
+	const uint32_t i = tile * FWD_POINTS + threadIdx.x;
+#define CALL(M) grid_forward_item<M, WANT_DYDX, STREAM>(tab, level, i, N, xyz, point_stride, dim_stride, params, out, dy_dx)
 	N2_DISPATCH_MODE(tab.mode[level], CALL)
 #undef CALL
 }

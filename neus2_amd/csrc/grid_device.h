@@ -44,6 +44,110 @@ __device__ __forceinline__ uint32_t n2_entry(uint32_t entries, uint32_t res, uin
 	}
 }
 
+// Byte offsets in the level's table of the four (y, z) corners k = y + 2 z of a cell at x corner gx: what n2_entry gives, times four.
+// On power-of-two tables y and z come as the hash's terms (n2_hash_terms; a multiplication by a constant and one by four commute
+// modulo 2^32), which two x corners share.
+__device__ __forceinline__ void n2_hash_terms(uint32_t (&c)[3]) {
+	c[1] *= 2654435761u * 4u;
+	c[2] *= 805459861u * 4u;
+}
+template <uint32_t MODE>
+__device__ __forceinline__ void n2_corner_bytes(uint32_t entries, uint32_t res, uint32_t gx, uint32_t cy, uint32_t cz, uint32_t (&at)[4]) {
+	if (MODE == N2_LEVEL_HASH) {
+		const uint32_t mask = (entries - 1u) << 2, x = gx << 2, z1 = cz + 805459861u * 4u, xy0 = x ^ cy, xy1 = x ^ (cy + 2654435761u * 4u);
+		at[0] = (xy0 ^ cz) & mask;
+		at[1] = (xy1 ^ cz) & mask;
+		at[2] = (xy0 ^ z1) & mask;
+		at[3] = (xy1 ^ z1) & mask;
+	} else if (MODE == N2_LEVEL_DENSE) {
+		const uint32_t bytes = entries << 2, row = res << 2, plane = row * res;
+		const uint32_t x = min(gx, res) << 2, y0 = x + min(cy, res) * row, y1 = x + min(cy + 1u, res) * row, z0 = min(cz, res) * plane, z1 = min(cz + 1u, res) * plane;
+		const uint32_t sum[4] = {y0 + z0, y1 + z0, y0 + z1, y1 + z1};
+#pragma unroll
+		for (uint32_t k = 0; k < 4; ++k) at[k] = min(sum[k], sum[k] - bytes);  // one conditional subtraction is the modulo (unsigned wrap-around)
+	} else {
+#pragma unroll
+		for (uint32_t k = 0; k < 4; ++k) at[k] = n2_entry<MODE>(entries, res, gx, cy + (k & 1u), cz + (k >> 1)) << 2;
+	}
+}
+
+// value held by the other lane of the pair (lane ^ 1), and by the pair's lane M: quad permutes inside the VALU, no LDS crossbar
+__device__ __forceinline__ uint32_t n2_pair_swap(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, true); }
+__device__ __forceinline__ float n2_pair_swap(float x) { return __uint_as_float(n2_pair_swap(__float_as_uint(x))); }
+template <int M>
+__device__ __forceinline__ uint32_t n2_pair_lane(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, M ? 0xF5 : 0xA0, 0xF, 0xF, true); }
+template <int M>
+__device__ __forceinline__ float n2_pair_lane(float x) { return __uint_as_float(n2_pair_lane<M>(__float_as_uint(x))); }
+
+// The encoding of one level at the lane's own point: both features and, with WANT_J, their derivatives along the axes (times jscale).
+// Two adjacent lanes share the work on their two points: for either point lane b gathers the four (y, z) corners of x corner b, whose
+// other x corner stands beside it (dense levels: index + 1; hashed levels: x enters the hash with prime 1), nearly always in the same
+// line of 128 bytes.  What bounds the gathers is lines: an L1 takes one in from the L2 every 2.3 clocks (measured with loads of 4, 8 and
+// 16 bytes alike), and a wave's load of 64 words it has takes 40 clocks.  So a pair's load meets 32 lines and not 64, and because
+// every lane keeps a point of its own, positions come in and results go out as whole lines (8 clocks a load), where two lanes to a point
+// took 16 clocks for each of three coordinates.  Call in us, two lanes per point -> this: 2^21 cells of the occupancy grid 503 -> 467, 2^20
+// uniform points 304 -> 297, the encoding forward and backward on 2^18 points 214 -> 211.  Two or four points per lane with their loads under
+// way together are no faster, and neither are loads of the 8 or 16 bytes round a corner, which an L1 serves in less time when the lanes
+// of a pair share them.  All lanes of the wave take part.
+template <uint32_t MODE, bool WANT_J>
+__device__ __forceinline__ void n2_encode_level(const char* __restrict__ base, uint32_t entries, uint32_t res, float scale, const float (&p)[3], float jscale,
+                                                float (&feat)[2], float (&J)[2][3]) {
+	const uint32_t b = threadIdx.x & 1u;
+	float w[3];
+	uint32_t c[3], at[2][4], raw[2][4];
+#pragma unroll
+	for (int d = 0; d < 3; ++d) n2_locate(p[d], scale, w[d], c[d]);
+	if (MODE == N2_LEVEL_HASH) n2_hash_terms(c);
+	n2_corner_bytes<MODE>(entries, res, n2_pair_lane<0>(c[0]) + b, n2_pair_lane<0>(c[1]), n2_pair_lane<0>(c[2]), at[0]);
+	n2_corner_bytes<MODE>(entries, res, n2_pair_lane<1>(c[0]) + b, n2_pair_lane<1>(c[1]), n2_pair_lane<1>(c[2]), at[1]);
+#pragma unroll
+	for (int m = 0; m < 2; ++m)
+#pragma unroll
+		for (int k = 0; k < 4; ++k) raw[m][k] = *reinterpret_cast<const uint32_t*>(base + at[m][k]);
+	const float wy[2] = {n2_pair_lane<0>(w[1]), n2_pair_lane<1>(w[1])}, wz[2] = {n2_pair_lane<0>(w[2]), n2_pair_lane<1>(w[2])};
+	// of point m's x corner b: the bilinear value s, and its y and z differences ty, tz
+	float s[2][2], ty[2][2], tz[2][2];  // [point][feature]
+#pragma unroll
+	for (int m = 0; m < 2; ++m) {
+		float v[4][2];
+#pragma unroll
+		for (int k = 0; k < 4; ++k) {
+			const float2 h = __half22float2(*reinterpret_cast<const __half2*>(&raw[m][k]));
+			v[k][0] = h.x;
+			v[k][1] = h.y;
+		}
+		const float uy = 1.f - wy[m], uz = 1.f - wz[m], w00 = uy * uz, w10 = wy[m] * uz, w01 = uy * wz[m], w11 = wy[m] * wz[m];
+#pragma unroll
+		for (int f = 0; f < 2; ++f) {
+			// (the last product as a multiply-add too: those take half-precision operands as they are)
+			s[m][f] = fmaf(w00, v[0][f], fmaf(w10, v[1][f], fmaf(w01, v[2][f], fmaf(w11, v[3][f], 0.f))));
+			if (WANT_J) {
+				ty[m][f] = fmaf(uz, v[1][f] - v[0][f], wz[m] * (v[3][f] - v[2][f]));
+				tz[m][f] = fmaf(uy, v[2][f] - v[0][f], wy[m] * (v[3][f] - v[1][f]));
+			}
+		}
+	}
+	// of the lane's own point, x corner b is its own and the other one its partner's
+	const float wx = w[0], ux = 1.f - wx;
+	auto corners = [&](const float q0, const float q1, float& lo, float& hi) {
+		const float from0 = n2_pair_swap(q0), from1 = n2_pair_swap(q1);
+		lo = b ? from1 : q0;
+		hi = b ? q1 : from0;
+	};
+#pragma unroll
+	for (int f = 0; f < 2; ++f) {
+		float lo, hi;
+		corners(s[0][f], s[1][f], lo, hi);
+		feat[f] = fmaf(ux, lo, wx * hi);
+		if (WANT_J) {
+			J[f][0] = (hi - lo) * jscale;
+			corners(ty[0][f], ty[1][f], lo, hi);
+			J[f][1] = fmaf(ux, lo, wx * hi) * jscale;
+			corners(tz[0][f], tz[1][f], lo, hi);
+			J[f][2] = fmaf(ux, lo, wx * hi) * jscale;
+		}
+	}
+}
 
 // ----------------------------------------------------------------------------
 // Slopes of one (sample, level): the six values d feature_f / d x_d (before the level's scale factor) as one 16-byte
@@ -76,9 +180,6 @@ __device__ __forceinline__ uint4 n2_slopes_pack(const float (&v)[6]) {
 	w.w = (q[4] >> 16) | (q[5] << 4) | ((uint32_t)e << 24);
 	return w;
 }
-// value held by the other lane of the pair (lane ^ 1): a quad permute [1, 0, 3, 2] inside the VALU, no LDS crossbar
-__device__ __forceinline__ uint32_t n2_pair_swap(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, true); }
-__device__ __forceinline__ float n2_pair_swap(float x) { return __uint_as_float(n2_pair_swap(__float_as_uint(x))); }
 
 // mantissas as floats and the factor 2^(e - 19) they share
 __device__ __forceinline__ float n2_slopes_unpack(const uint4 w, float (&q)[6]) {

@@ -87,7 +87,7 @@ N2_HD inline bool n2_xcd_level_tile(uint32_t block, uint32_t n_levels, uint32_t 
 // The launch of a kernel that takes (level, tile of points) items: workgroups in x and y.  Up to `by_xcd_max` points the levels are
 // dealt to the XCDs (y is 1); beyond, y counts the levels: the workgroups that run at one time then work on one or two
 // levels, whose tables stay in every L2, and what reading the tables into every L2 costs is less than what the uneven XCDs
-// lose.  (y, because a launch has at most 2^32 - 1 threads along x: 2^27 points of sixteen levels with two lanes each.)
+// lose.  (y, because a launch has at most 2^32 - 1 threads along x: 2^28 points of sixteen levels.)
 // Call in us, level-major | by XCD:
 //   field, points along rays: 2^14 12.4 | 9.9 and 52 000 24.8 | 19 (gather alone), 2^18 279 | 271, 2^19 507 | 502, 3 * 2^18 734 | 735, 2^20 961 | 969, 2^21 1917 | 1954
 //   query, uniform points: 2^17 52.8 | 47.9, 2^18 87.8 | 86.6, 5 * 2^16 105.4 | 105.6, 3 * 2^17 123.4 | 125.3, 2^19 159 | 164, 2^20 301 | 314, 2^21 594 | 617

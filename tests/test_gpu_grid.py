@@ -547,3 +547,26 @@ def test_forward_by_level_costs_equals_the_default_deal(levels, n):
     capi.check(capi.lib().n2_grid_set_level_costs(g._h, (C.c_float * levels)(*[1.0 + 3 * (l % 3) for l in range(levels)])))
     b, jb = g.forward(x, prepare_input_gradients=True)
     assert torch.equal(a, b) and torch.equal(ja, jb) and bool(a.abs().sum() > 0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 257])
+@pytest.mark.parametrize("masked", [False, True])
+def test_a_point_is_encoded_the_same_beside_any_neighbour(setup, n, masked):
+    """Two adjacent lanes share the gathers of their points: bit for bit the same with another partner, one that is not a
+    number or whose levels are switched off among them, and with none."""
+    og, gg, params, *_ = setup
+    rng = np.random.default_rng(n)
+    xyz = (rng.random((3, n + 1)) * 1.1 - 0.05).astype(np.float32)
+    xyz[:, 0] = np.nan
+    frac = (rng.random(n + 1) * 2).astype(np.float32)
+    keep = [dev(frac), dev(np.ascontiguousarray(frac[1:]))]
+    try:
+        outs = []
+        for x, f in ((xyz, keep[0]), (np.ascontiguousarray(xyz[:, 1:]), keep[1])):
+            if masked:
+                gg.set_max_level_gpu(f)
+            outs.append(gg.forward(dev(x), prepare_input_gradients=True))
+    finally:
+        gg.set_max_level_gpu(None)
+    (a, ja), (b, jb) = outs
+    assert torch.equal(a[:, 1:], b) and torch.equal(ja[:, 1:], jb) and bool(b.abs().sum() > 0)
