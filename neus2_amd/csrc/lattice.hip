@@ -4,20 +4,21 @@
 // On a lattice everything that a point's place in the encoding depends on is separable: cell and weight along an axis are
 // functions of one index.  A wave takes a run of 64 points along x at one y and walks along z, so y and z quantities are
 // wave-uniform (scalar registers) and a lane keeps only what depends on its x.  Two kinds of levels:
-//  * coarse levels, whose cells are larger than the z step (lattice_walk_kernel): the values of the two z planes of vertices
+//  * coarse levels, whose cells are larger than the steps (lattice_walk_kernel): the values of the two z planes of vertices
 //    round the walk's position stay in registers, already interpolated in x and y; a step only interpolates in z, and a
-//    plane is gathered when the walk crosses into it (once per cell, loads issued one step ahead).
+//    plane is loaded when the walk crosses into it (once per cell, loads issued one step ahead).
 //  * fine levels (lattice_fine_kernel): nothing is shared between steps.  They run level by level over a slab of planes, so
 //    that the 2 MiB table being read stays in every XCD's L2, and leave their features in the caller's scratch; the walk
 //    picks them up.  (Point by point through all levels, 10 MiB of fine tables compete for 4 MiB of L2: 44 % of the requests
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice: 8.2 -> 5.8 ms, per slab of 7.6e6 points 156 us for six fine levels and 182 us for the walk.  The walk runs two waves
-// per SIMD (its plane values take 60 registers, the loads in flight 52); it issues vector instructions in half of the
-// cycles, and its waves wait for memory in 43 % of theirs.
-// Rows that are no multiple of 64 leave lanes idle in their last run; against one gather per point and level: 80^3 124 -> 86 us, 144^3
-// 478 -> 280, 208^3 1088 -> 645, 272^3 1876 -> 1259, 464^3 6123 -> 5121, 80 x 512 x 400 3591 -> 1687 (64^3 71 -> 59, 128^3 342 -> 187, 256^3 1525 -> 1003).
+// 512^3 lattice 4.8 ms, per slab of 7.6e6 points 142 us for six fine levels and 135 us for the walk.  Before: 5.76, 154 and 180, with
+// vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  The fine levels are held by the L1's
+// data return (busy in 89 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (58 %) and by
+// the features, which come from beyond the L2.
+// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before | now: 80^3 86 | 81 us, 128^3 187 | 176, 208^3 654 | 595,
+// 256^3 1008 | 890, 320^3 1750 | 1605, 400^3 3410 | 2925, 464^3 5130 | 4550, 512 x 64 x 512 752 | 625, 64 x 512 x 512 1672 | 1624.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -29,14 +30,16 @@
 
 constexpr uint32_t LT_LEVELS = 16;
 constexpr uint32_t LT_BLOCK = 256;
-constexpr uint32_t LT_MAX_FINE = 11;  // feature rows of 4 bytes per point that the scratch holds (n2_density_on_grid_scratch_bytes)
+constexpr uint32_t LT_MAX_FINE = 11;  // feature rows of 4 bytes per point of a chunk that the scratch holds (n2_density_on_grid_scratch_bytes)
 
 struct LatticeArgs {
 	float scale[LT_LEVELS];
 	uint32_t res[LT_LEVELS], entries[LT_LEVELS], offset[LT_LEVELS];
 	uint32_t hash_mask, active_levels, n_levels;
 	const __half2* table;
-	const hf* frags;          // fragment image of the SDF network
+	hf* frags;                // fragment image of the SDF network, and what it is made of
+	const hf* sdf_w;
+	uint32_t sdf_in_w;
 	float sdf_bias;
 	N2Lattice lat;
 	uint32_t y0, ny, z0, nz;  // the slab: rows y0 .. y0 + ny of planes z0 .. z0 + nz,
@@ -87,17 +90,75 @@ __device__ __forceinline__ bool lattice_run(const LatticeArgs& a, uint32_t wave,
 	return true;
 }
 
-// Fine levels, level-major workgroup ids.  A run needs eight vertices per point, on four rows (y, z), (y + 1, z), (y, z + 1),
+// The SDF network's fragments as one image (SDF_FRAG_COUNT KiB): workgroup `block` of FRAG_BLOCKS
+constexpr uint32_t FRAG_BLOCKS = SDF_FRAG_COUNT * 64u / LT_BLOCK + (SDF_FRAG_COUNT * 64u % LT_BLOCK != 0u);
+__device__ __forceinline__ void lattice_write_frags(const LatticeArgs& a, uint32_t block) {
+	const uint32_t i = block * LT_BLOCK + threadIdx.x;
+	if (i < SDF_FRAG_COUNT * 64u) *reinterpret_cast<half8*>(a.frags + i * 8u) = sdf_forward_frag(a.sdf_w, (int)a.sdf_in_w, a.n_levels * 2u, (int)(i >> 6), (int)(i & 63u));
+}
+__global__ void __launch_bounds__(LT_BLOCK) lattice_frags_kernel(const LatticeArgs a) { lattice_write_frags(a, blockIdx.x); }
+
+// Fine levels, level-major workgroup ids; the workgroups behind those write the fragments (a launch for them alone was 5 us of the 60
+// that a lattice of 64^3 takes).  A run needs eight vertices per point, on four rows (y, z), (y + 1, z), (y, z + 1),
 // (y + 1, z + 1).  On a hashed level a row's neighbours in x stand in one aligned 128-byte line per 32, permuted; a load
 // instruction costs the L1 one clock per group of four lanes at least, and up to four where the lanes' spacing makes their
 // banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks per 4-byte load).  So the wave loads the rows as a
-// whole, 16 bytes per lane, into LDS (FINE_CHUNKS of them per row) and picks the vertices there: for six levels of 2^22 points
-// 153 -> 89 us.  LDS is active in 73 % of the launch's cycles then, a third of that bank conflicts; of the lines it asks the L2s for
-// 91 % are there.  Runs longer than that (coarse lattices) and dense levels gather from memory.
-constexpr uint32_t FINE_CHUNKS = 128;
+// whole, 2, 4 or 8 entries per lane as the run's length asks for, and weighs the four rows against each other where they are, in
+// registers; what remains is one row, which goes through LDS (in fp32, a slot left out after every 32 entries so that lanes any
+// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 25 % of the
+// clocks; 73 % when the eight vertices were picked there).  Runs longer than that (coarse lattices) and dense levels gather from memory.
+constexpr uint32_t FINE_CHUNKS = 128;  // chunks of four entries a row may have
+constexpr uint32_t FINE_SLOTS = FINE_CHUNKS * 4u + FINE_CHUNKS / 8u;
+__device__ __forceinline__ uint32_t fine_slot(uint32_t entry) { return entry + (entry >> 5); }
+
+// EACH entries per lane: of the rows at byte offsets row[q] (on a hashed level: entry x is at x's bytes ^ row[q]), weighed by
+// weight[q], the sum.  off: the lane's places in a row, of up to four entries each; have: whether there is one.
+template <uint32_t EACH>
+__device__ __forceinline__ void fine_sum_rows(const char* __restrict__ base, const uint32_t (&off)[2], const bool (&have)[2], const uint32_t (&row)[4],
+                                              const float (&weight)[4], float2 (&sum)[EACH]) {
+	constexpr uint32_t W = EACH < 4u ? EACH : 4u, H = EACH / W;  // entries per load, loads per row
+	typedef uint32_t words __attribute__((ext_vector_type(W)));
+	words v[4][H];  // (a lane without a place holds anything: its slots are not read)
+#pragma unroll
+	for (uint32_t h = 0; h < H; ++h)
+		if (have[h]) {
+#pragma unroll
+			for (uint32_t q = 0; q < 4; ++q) v[q][h] = *reinterpret_cast<const words*>(base + (off[h] ^ (row[q] & ~(4u * W - 1u))));
+		}
+#pragma unroll
+	for (uint32_t e = 0; e < EACH; ++e) sum[e] = make_float2(0.f, 0.f);
+#pragma unroll
+	for (uint32_t q = 0; q < 4; ++q) {
+		// the entries of a load are permuted by the row's low bits, the same for the whole wave
+		auto add = [&](auto flip) __attribute__((always_inline)) {
+			constexpr uint32_t F = decltype(flip)::value;
+#pragma unroll
+			for (uint32_t e = 0; e < EACH; ++e) {
+				const float2 f = lt_h2f(v[q][e / W][(e % W) ^ F]);
+				sum[e].x = fmaf(weight[q], f.x, sum[e].x);
+				sum[e].y = fmaf(weight[q], f.y, sum[e].y);
+				asm volatile("; permutation %2" : "+v"(sum[e].x), "+v"(sum[e].y) : "n"(F));  // (the cases stay apart: merged, each entry is picked by selects)
+			}
+		};
+		if (W > 2u && (row[q] & 8u)) {
+			if (row[q] & 4u) add(std::integral_constant<uint32_t, 3 % W>());
+			else add(std::integral_constant<uint32_t, 2 % W>());
+		} else {
+			if (row[q] & 4u) add(std::integral_constant<uint32_t, 1>());
+			else add(std::integral_constant<uint32_t, 0>());
+		}
+		// (here every load of the row has arrived, whichever case was taken; without saying so the next plane's loads wait for the store)
+#pragma unroll
+		for (uint32_t h = 0; h < H; ++h) asm volatile("" ::"v"(v[q][h]));
+	}
+}
 
 __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArgs a, uint32_t blocks_per_level) {
-	__shared__ uint4v staged[LT_BLOCK / 64][4][FINE_CHUNKS];
+	if (blockIdx.x >= blocks_per_level * (a.n_levels - a.first_fine)) {
+		lattice_write_frags(a, blockIdx.x - blocks_per_level * (a.n_levels - a.first_fine));
+		return;
+	}
+	__shared__ float2 staged[LT_BLOCK / 64][FINE_SLOTS];
 	const uint32_t level = a.first_fine + blockIdx.x / blocks_per_level;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x % blocks_per_level) * (LT_BLOCK / 64) + (threadIdx.x >> 6));
 	uint32_t x, y, z, nz;
@@ -147,39 +208,43 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	uint32_t c_lo, chunks;
 	n2_lattice_chunks(lane_u32(cx, 0), lane_u32(cx, 63), c_lo, chunks);
 	if (hashed && chunks <= FINE_CHUNKS) {
-		// (lanes behind the last chunk load it again, into a slot nobody reads)
-		const uint32_t o0 = ((c_lo + 4u * min(lane, chunks - 1u)) & (entries - 1u)) << 2, o1 = ((c_lo + 4u * min(lane + 64u, chunks - 1u)) & (entries - 1u)) << 2;
-		uint4v (&st)[4][FINE_CHUNKS] = staged[threadIdx.x >> 6];
-		const uint32_t at0 = (cx - c_lo) << 2, at1 = at0 + 4u;
-		auto walk = [&](auto halves) {
-			constexpr uint32_t H = decltype(halves)::value;  // 64 chunks per load instruction and row
+		float2* st = staged[threadIdx.x >> 6];
+		const uint32_t at0 = fine_slot(cx - c_lo), at1 = fine_slot(cx - c_lo + 1u);
+		auto walk = [&](auto each) __attribute__((always_inline)) {
+			constexpr uint32_t EACH = decltype(each)::value, W = EACH < 4u ? EACH : 4u, H = EACH / W;
+			// The run's places, of W entries each, start anywhere in 64 bytes.  The lanes are turned so that those of a group meet one
+			// aligned 64 bytes (permuted), which the address unit takes at once; a group across two of them costs twice the time.
+			uint32_t off[2], slot[2];
+			bool have[2];
+#pragma unroll
+			for (uint32_t h = 0; h < H; ++h) {
+				const uint32_t at = (lane + 64u * h - c_lo / W % (16u / W)) % (64u * H);
+				have[h] = at < chunks * (4u / W);
+				off[h] = ((c_lo + W * at) & (entries - 1u)) << 2;
+				slot[h] = fine_slot(W * at);
+			}
 			for (uint32_t k = 0; k < nz; ++k) {
 				uint32_t row[4];
-				uint4v v[4][H];
-#pragma unroll
-				for (uint32_t q = 0; q < 4; ++q) row[q] = lane_u32(rows[q], k);
-#pragma unroll
-				for (uint32_t q = 0; q < 4; ++q)
-#pragma unroll
-					for (uint32_t h = 0; h < H; ++h) v[q][h] = *reinterpret_cast<const uint4v*>(base + ((h ? o1 : o0) ^ (row[q] & ~15u)));
-#pragma unroll
-				for (uint32_t q = 0; q < 4; ++q)
-#pragma unroll
-					for (uint32_t h = 0; h < H; ++h) st[q][lane + 64u * h] = v[q][h];
-				__builtin_amdgcn_wave_barrier();
-				uint32_t raw[8];
+				float weight[4];
 #pragma unroll
 				for (uint32_t q = 0; q < 4; ++q) {
-					const uint32_t flip = row[q] & 12u;  // a chunk's entries are permuted by the row's low bits
-					raw[2 * q] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(&st[q][0]) + (at0 ^ flip));
-					raw[2 * q + 1] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(&st[q][0]) + (at1 ^ flip));
+					row[q] = lane_u32(rows[q], k);
+					weight[q] = lane_f32(weights[q], k);
 				}
+				float2 sum[EACH];
+				fine_sum_rows<EACH>(base, off, have, row, weight, sum);
 				__builtin_amdgcn_wave_barrier();
-				finish(k, raw);
+#pragma unroll
+				for (uint32_t e = 0; e < EACH; ++e) st[slot[e / W] + e % W] = sum[e];
+				__builtin_amdgcn_wave_barrier();
+				const float2 lo = st[at0], hi = st[at1];
+				if (inside) *out = lt_pack(fmaf(ux, lo.x, wx * hi.x), fmaf(ux, lo.y, wx * hi.y));
+				out += plane;
 			}
 		};
-		if (chunks > 64u) walk(std::integral_constant<uint32_t, 2>());
-		else walk(std::integral_constant<uint32_t, 1>());
+		if (chunks > 64u) walk(std::integral_constant<uint32_t, 8>());
+		else if (chunks > 32u) walk(std::integral_constant<uint32_t, 4>());
+		else walk(std::integral_constant<uint32_t, 2>());
 		return;
 	}
 	const uint32_t x0 = x_part(hashed, entries, res, cx), x1 = x_part(hashed, entries, res, cx + 1u);
@@ -202,9 +267,231 @@ __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
 	b = r[1];
 }
 
-// The walk.  NM levels are interpolated here, the others come from a.features.
+// The SDF of the wave's 64 points from their features (enc: one word per level), two tiles of the network.  Tile 0 works for lanes
+// 0..31, tile 1 for lanes 32..63; xc0, xc1: the x and y coordinate for either, in the lanes that need them (the lower half).
+__device__ __forceinline__ void lattice_xy(float px, float py, uint32_t g, uint32_t& xc0, uint32_t& xc1) {
+	xc0 = xc1 = lt_pack((float)((hf)px - (hf)0.5f), (float)((hf)py - (hf)0.5f));
+	swap_halves(xc0, xc1);
+	xc0 = g == 0u ? xc0 : 0u;
+	xc1 = g == 0u ? xc1 : 0u;
+}
+__device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32_t (&enc)[LT_LEVELS], uint32_t xc0, uint32_t xc1, float pz, float bias) {
+	// (the fence keeps the network's fragments in LDS: hoisted out of the walk's loop they would take 40 registers)
+	tile_fence();
+	half8 xs[2][3];
+#pragma unroll
+	for (int c = 0; c < 2; ++c) {
+		uint4v t[2];
+#pragma unroll
+		for (int q = 0; q < 4; ++q) {
+			constexpr int first[4] = {0, 1, 4, 5};
+			uint32_t p0 = enc[8 * c + first[q]], p1 = enc[8 * c + first[q] + 2];
+			swap_halves(p0, p1);
+			t[0][q] = p0;
+			t[1][q] = p1;
+		}
+		xs[0][c] = __builtin_bit_cast(half8, t[0]);
+		xs[1][c] = __builtin_bit_cast(half8, t[1]);
+	}
+	const half2v zc = {(hf)pz - (hf)0.5f, (hf)0};
+	const uint32_t zcm = lane < 32u ? __builtin_bit_cast(uint32_t, zc) : 0u;
+	xs[0][2] = __builtin_bit_cast(half8, uint4v{xc0, zcm, 0u, 0u});
+	xs[1][2] = __builtin_bit_cast(half8, uint4v{xc1, zcm, 0u, 0u});
+	// The second layer, of which only row 0 is wanted: a lane holds half of its sample's hidden values (the other group the
+	// other half).  Dot products on the vector unit take a third of the time of four more MFMAs per tile.
+	// (one tile after the other: side by side they take 32 registers more, and a third wave has no room)
+	float dot[2] = {0.f, 0.f};
+#pragma unroll
+	for (int t = 0; t < 2; ++t)
+#pragma unroll
+		for (int mt = 0; mt < 2; ++mt) {
+			float16v acc = zero16();
+#pragma unroll
+			for (int c = 0; c < 3; ++c) acc = N2_MFMA(frag(F, SDF_FRAG_W0 + mt * 3 + c, lane), xs[t][c], acc);
+			half8 h[2];
+			relu_pack(acc, h[0], h[1]);
+#pragma unroll
+			for (int c = 0; c < 2; ++c) {
+				const uint4v wv = __builtin_bit_cast(uint4v, frag(F, SDF_FRAG_WO + 2 * mt + c, lane & 32)), hv = __builtin_bit_cast(uint4v, h[c]);  // row 0 of W_out in the order of h
+#pragma unroll
+				for (int q = 0; q < 4; ++q)
+					dot[t] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, (uint32_t)hv[q]), __builtin_bit_cast(half2v, (uint32_t)wv[q]), dot[t], false);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	// tile 0 belongs to lanes 0..31, tile 1 to the upper ones
+	uint32_t s0 = __float_as_uint(dot[0]), s1 = __float_as_uint(dot[1]);
+	swap_halves(s0, s1);
+	return (hf)(__uint_as_float(s0) + __uint_as_float(s1)) + (hf)bias;
+}
+
+// The walk.  NM levels are interpolated here, the others come from a.features.  A row of a walked level's vertices that a run of 64
+// points meets fits the wave's lanes (n2_lattice_walked_levels): lane v holds vertex v of the run, the two rows of a plane are loaded
+// as consecutive words and interpolated in y there, and the points pick their two neighbours through LDS.
 template <int NM>
-__global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const LatticeArgs a) {
+__global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const LatticeArgs a) {
+	__shared__ __align__(16) hf F[SDF_FRAG_COUNT * 512];
+	__shared__ float2 line[LT_BLOCK / 64][NM][64];
+	for (uint32_t i = threadIdx.x; i < SDF_FRAG_COUNT * 64u; i += LT_BLOCK) *reinterpret_cast<half8*>(F + i * 8u) = *reinterpret_cast<const half8*>(a.frags + i * 8u);
+	__syncthreads();
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (LT_BLOCK / 64) + (threadIdx.x >> 6));
+	uint32_t x, y, z, nz;
+	if (!lattice_run(a, wave, x, y, z, nz)) return;
+	const uint32_t lane = threadIdx.x & 63u, plane = a.nx * a.ny;
+	const bool inside = x < a.nx;
+	const float px = lattice_coord(a.lat, 0, a.x0 + min(x, a.nx - 1u)), py = lattice_coord(a.lat, 1, y);
+	float2 (&mine)[NM][64] = line[threadIdx.x >> 6];
+	// lane l: what depends on y and z of level l, and its lowest cell along x
+	const uint32_t ll = lane & (LT_LEVELS - 1u);
+	const float my_scale = a.scale[ll];
+	const uint32_t my_res = a.res[ll], my_entries = a.entries[ll];
+	const bool my_hashed = (a.hash_mask >> ll) & 1u;
+	const uint32_t on = (1u << min(a.active_levels, (uint32_t)NM)) - 1u;  // levels in use here
+	float my_wy, my_back, unused;  // my_back: from the plane above to the walk's position
+	uint32_t my_cy, my_cz, my_first, my_last;
+	n2_locate(py, my_scale, my_wy, my_cy);
+	n2_locate(lane_f32(px, 0), my_scale, unused, my_first);
+	n2_locate(lane_f32(px, 63), my_scale, unused, my_last);
+	my_first = (uint32_t)min((int32_t)my_first, (int32_t)my_last);
+	// the plane of vertices whose rows y, y + 1 are at byte offsets row0, row1
+	auto fetch = [&](int l, uint32_t row0, uint32_t row1, uint32_t (&raw)[2]) __attribute__((always_inline)) {
+		const char* base = reinterpret_cast<const char*>(a.table + a.offset[l]);
+		const uint32_t entries = lane_u32(my_entries, l), v = lane_u32(my_first, l) + lane;
+		if ((a.hash_mask >> l) & 1u) {
+			const uint32_t xo = x_part(true, entries, 0u, v);
+			raw[0] = *reinterpret_cast<const uint32_t*>(base + (xo ^ row0));
+			raw[1] = *reinterpret_cast<const uint32_t*>(base + (xo ^ row1));
+		} else {
+			const uint32_t xo = x_part(false, entries, lane_u32(my_res, l), v);
+			raw[0] = *reinterpret_cast<const uint32_t*>(base + vertex(false, entries << 2, xo, row0));
+			raw[1] = *reinterpret_cast<const uint32_t*>(base + vertex(false, entries << 2, xo, row1));
+		}
+	};
+	auto blend_y = [&](int l, const uint32_t (&raw)[2]) __attribute__((always_inline)) {
+		const float2 v0 = lt_h2f(raw[0]), v1 = lt_h2f(raw[1]);
+		const float wy = lane_f32(my_wy, l);
+		// (the differences as multiply-adds: those take half-precision operands as they are)
+		mine[l][lane] = make_float2(fmaf(wy, fmaf(1.f, v1.x, -v0.x), v0.x), fmaf(wy, fmaf(1.f, v1.y, -v0.y), v0.y));
+	};
+	// What depends on x is worked out at each plane, from an opaque copy of the position: kept across the loop, cell and weight of
+	// every level take 20 registers.
+	auto blend_x = [&](int l, float2& to) __attribute__((always_inline)) {
+		float p = px, w;
+		uint32_t cx;
+		asm volatile("" : "+v"(p));
+		n2_locate(p, lane_f32(my_scale, l), w, cx);
+		const float2* at = &mine[l][min(cx - lane_u32(my_first, l), 62u)];
+		const float2 lo = at[0], hi = at[1];
+		to = make_float2(fmaf(w, hi.x - lo.x, lo.x), fmaf(w, hi.y - lo.y, lo.y));
+	};
+	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) __attribute__((always_inline)) {
+		r0 = row_part(my_hashed, my_entries, my_res, my_cy, cz);
+		r1 = row_part(my_hashed, my_entries, my_res, my_cy + 1u, cz);
+	};
+	float2 hi[NM], rise[NM];  // the plane above, and by how much it is above the one below
+	auto one_plane = [&](uint32_t which, uint32_t cz, float2 (&to)[NM]) __attribute__((always_inline)) {
+		uint32_t r0, r1, raw[NM][2];
+		rows_of(cz, r0, r1);
+		// (all levels' loads in flight together)
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) blend_y(l, raw[l]);
+		__builtin_amdgcn_wave_barrier();
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((which >> l) & 1u) blend_x(l, to[l]);
+		__builtin_amdgcn_wave_barrier();
+	};
+	const uint64_t feat_level = (uint64_t)plane * a.nz;
+	const uint32_t* feat = a.features + (uint64_t)(z - a.z0) * plane + (uint64_t)(y - a.y0) * a.nx;  // (the same for the wave, like out)
+	const uint32_t feat_x = min(x, a.nx - 1u);
+	float* out = a.out + (uint64_t)(z - a.z0) * ((uint64_t)a.lat.res[0] * a.lat.res[1]) + (uint64_t)(y - a.y0) * a.lat.res[0];
+	uint32_t xc0, xc1;
+	lattice_xy(px, py, lane >> 5, xc0, xc1);
+	// (levels that the table does not have read the last one's row: their weights are zero)
+	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
+	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
+	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) __attribute__((always_inline)) {
+#pragma unroll
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = (feat + (have_fine ? min(f, a.n_levels - 1u - NM) : 0u) * feat_level + (uint64_t)k * plane)[feat_x];
+	};
+	// Steps one after the other from plane k on, until the end or to where some level's next plane is not the one above (a box upside down;
+	// steps of more than a cell): there the walk starts anew.  (With that case inside the loop, where it is hardly ever met, its
+	// loads cost all others their overlap: whether they are under way is then not known, and everything is waited for; 131 -> 190 us.)
+	uint32_t k = 0;
+	while (true) {
+	n2_locate(lattice_coord(a.lat, 2, z + k), my_scale, my_back, my_cz);
+	my_back -= 1.f;
+#pragma unroll
+	for (int l = 0; l < NM; ++l) hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched-off levels
+	one_plane(on, my_cz, rise);
+	one_plane(on, my_cz + 1u, hi);
+#pragma unroll
+	for (int l = 0; l < NM; ++l) rise[l] = make_float2(hi[l].x - rise[l].x, hi[l].y - rise[l].y);
+	load_fine(k, fine);
+	load_fine(min(k + 1u, nz - 1u), ahead);
+	while (true) {
+		const float pz = lattice_coord(a.lat, 2, z + k);
+		// features of this step
+		uint32_t enc[LT_LEVELS];
+#pragma unroll
+		for (int l = 0; l < NM; ++l) {
+			const float back = lane_f32(my_back, l);
+			enc[l] = lt_pack(fmaf(back, rise[l].x, hi[l].x), fmaf(back, rise[l].y, hi[l].y));
+		}
+#pragma unroll
+		for (int f = 0; f < (int)LT_LEVELS - NM; ++f) {
+			enc[NM + f] = fine[f] & have_fine;
+			asm volatile("" : "+v"(enc[NM + f]));  // waited for here, in front of the next step's loads: behind them the wait would include those
+		}
+		// the next step: where it stands, and the loads it needs (the last step looks at its own position again: no loads)
+		const uint32_t next = k + 1u < nz ? k + 1u : k;
+		uint32_t cz;
+		float wz;
+		n2_locate(lattice_coord(a.lat, 2, z + next), my_scale, wz, cz);
+		const uint32_t moved = cz - my_cz;
+		const uint32_t one = (uint32_t)__ballot(moved == 1u) & on, far = (uint32_t)__ballot(moved > 1u) & on;  // lanes 0..15 speak for the levels
+		uint32_t r0, r1;
+		rows_of(cz + 1u, r0, r1);
+		uint32_t raw[NM][2];
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((one >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+		// Behind them the fine features of the step after the next (they come from far away): the planes can then be waited for
+		// without waiting for these.
+#pragma unroll
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
+		load_fine(min(k + 2u, nz - 1u), ahead);
+		const hf sdf = lattice_network(F, lane, enc, xc0, xc1, pz, a.sdf_bias);
+		if (inside) out[x] = (float)sdf;
+		out += (uint64_t)a.lat.res[0] * a.lat.res[1];
+		if (++k == nz) return;
+		if (far) break;
+		// the planes the next step has crossed into
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((one >> l) & 1u) blend_y(l, raw[l]);
+		__builtin_amdgcn_wave_barrier();
+#pragma unroll
+		for (int l = 0; l < NM; ++l)
+			if ((one >> l) & 1u) {
+				const float2 below = hi[l];
+				blend_x(l, hi[l]);
+				rise[l] = make_float2(hi[l].x - below.x, hi[l].y - below.y);
+			}
+		my_cz = cz;
+		my_back = wz - 1.f;
+	}
+	}
+}
+
+// The walk for lattices of a few dozen points along x, or with steps along z of more than a walked level's cell: every point gathers
+// its own vertices, and a step meets any planes.
+template <int NM>
+__global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const LatticeArgs a) {
 	__shared__ __align__(16) hf F[SDF_FRAG_COUNT * 512];
 	for (uint32_t i = threadIdx.x; i < SDF_FRAG_COUNT * 64u; i += LT_BLOCK) *reinterpret_cast<half8*>(F + i * 8u) = *reinterpret_cast<const half8*>(a.frags + i * 8u);
 	__syncthreads();
@@ -222,7 +509,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 	const float my_scale = a.scale[ll];
 	const uint32_t my_res = a.res[ll], my_entries = a.entries[ll];
 	const bool my_hashed = (a.hash_mask >> ll) & 1u;
-	const uint32_t on = a.active_levels >= 32u ? ~0u : (1u << a.active_levels) - 1u;  // levels in use
+	const uint32_t on = (1u << min(a.active_levels, (uint32_t)NM)) - 1u;  // levels in use here
 	float my_wy, my_wz;
 	uint32_t my_cy, my_cz;
 	n2_locate(py, my_scale, my_wy, my_cy);
@@ -302,13 +589,8 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + min(x, a.nx - 1u);
 	const size_t feat_level = (size_t)plane * a.nz;
 	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + x;
-	const uint32_t g = lane >> 5;  // of the lanes with g = 0 a tile's operands take the coordinates
-	const hf ycoord = (hf)py - (hf)0.5f;
-	// tile 0 works for lanes 0..31, tile 1 for lanes 32..63: the x coordinate of both, for the lanes that need it (g = 0)
-	uint32_t xc0 = lt_pack((float)((hf)px - (hf)0.5f), (float)ycoord), xc1 = xc0;
-	swap_halves(xc0, xc1);
-	xc0 = g == 0u ? xc0 : 0u;
-	xc1 = g == 0u ? xc1 : 0u;
+	uint32_t xc0, xc1;
+	lattice_xy(px, py, lane >> 5, xc0, xc1);
 	// (levels that the table does not have read the last one's row: their weights are zero)
 	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
 	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
@@ -350,59 +632,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 #pragma unroll
 		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
 		load_fine(min(k + 2u, nz - 1u), ahead);
-		// the network on both tiles (the fence keeps its fragments in LDS: hoisted out of the loop they would take 40 registers)
-		tile_fence();
-		half8 xs[2][3];
-#pragma unroll
-		for (int c = 0; c < 2; ++c) {
-			uint4v t[2];
-#pragma unroll
-			for (int q = 0; q < 4; ++q) {
-				constexpr int first[4] = {0, 1, 4, 5};
-				uint32_t p0 = enc[8 * c + first[q]], p1 = enc[8 * c + first[q] + 2];
-				swap_halves(p0, p1);
-				t[0][q] = p0;
-				t[1][q] = p1;
-			}
-			xs[0][c] = __builtin_bit_cast(half8, t[0]);
-			xs[1][c] = __builtin_bit_cast(half8, t[1]);
-		}
-		const half2v zc = {(hf)pz - (hf)0.5f, (hf)0};
-		const uint32_t zcm = g == 0u ? __builtin_bit_cast(uint32_t, zc) : 0u;
-		xs[0][2] = __builtin_bit_cast(half8, uint4v{xc0, zcm, 0u, 0u});
-		xs[1][2] = __builtin_bit_cast(half8, uint4v{xc1, zcm, 0u, 0u});
-		half8 h[2][4];
-#pragma unroll
-		for (int mt = 0; mt < 2; ++mt) {
-			half8 f[3];
-#pragma unroll
-			for (int c = 0; c < 3; ++c) f[c] = frag(F, SDF_FRAG_W0 + mt * 3 + c, lane);
-			float16v acc[2] = {zero16(), zero16()};
-#pragma unroll
-			for (int c = 0; c < 3; ++c)
-#pragma unroll
-				for (int t = 0; t < 2; ++t) acc[t] = N2_MFMA(f[c], xs[t][c], acc[t]);
-#pragma unroll
-			for (int t = 0; t < 2; ++t) relu_pack(acc[t], h[t][2 * mt], h[t][2 * mt + 1]);
-		}
-		// The second layer, of which only row 0 is wanted: a lane holds half of its sample's hidden values (the other group the
-		// other half).  Dot products on the vector unit take a third of the time of four more MFMAs per tile.
-		float dot[2] = {0.f, 0.f};
-#pragma unroll
-		for (int c = 0; c < 4; ++c) {
-			const uint4v wv = __builtin_bit_cast(uint4v, frag(F, SDF_FRAG_WO + c, lane & 32));  // row 0 of W_out in the order of h
-#pragma unroll
-			for (int t = 0; t < 2; ++t) {
-				const uint4v hv = __builtin_bit_cast(uint4v, h[t][c]);
-#pragma unroll
-				for (int q = 0; q < 4; ++q)
-					dot[t] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, (uint32_t)hv[q]), __builtin_bit_cast(half2v, (uint32_t)wv[q]), dot[t], false);
-			}
-		}
-		// tile 0 belongs to lanes 0..31, tile 1 to the upper ones
-		uint32_t s0 = __float_as_uint(dot[0]), s1 = __float_as_uint(dot[1]);
-		swap_halves(s0, s1);
-		const hf sdf = (hf)(__uint_as_float(s0) + __uint_as_float(s1)) + (hf)a.sdf_bias;
+		const hf sdf = lattice_network(F, lane, enc, xc0, xc1, pz, a.sdf_bias);
 		if (inside) out[0] = (float)sdf;
 		out += (size_t)rx * a.lat.res[1];
 		// the planes the next step has crossed into
@@ -417,11 +647,6 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_walk_kernel(const Lattice
 		my_cz = cz;
 		my_wz = wz;
 	}
-}
-
-// the SDF network's fragments as one image (SDF_FRAG_COUNT KiB)
-__global__ void __launch_bounds__(64) lattice_frags_kernel(const hf* __restrict__ sdf_w, uint32_t sdf_in_w, uint32_t enc_w, hf* __restrict__ image) {
-	*reinterpret_cast<half8*>(image + (blockIdx.x * 64u + threadIdx.x) * 8u) = sdf_forward_frag(sdf_w, (int)sdf_in_w, enc_w, (int)blockIdx.x, (int)threadIdx.x);
 }
 
 uint64_t n2_lattice_frag_bytes() { return SDF_FRAG_COUNT * 1024ull; }
@@ -441,16 +666,26 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 		if (have && tab.mode[l] == N2_LEVEL_HASH) a.hash_mask |= 1u << l;
 	}
 	a.table = nets.table;
-	a.frags = reinterpret_cast<const hf*>(d_frags);
+	a.frags = reinterpret_cast<hf*>(d_frags);
+	a.sdf_w = reinterpret_cast<const hf*>(nets.sdf_w);
+	a.sdf_in_w = nets.sdf_in_w;
 	a.sdf_bias = nets.sdf_bias;
 	a.lat = lat;
 	a.features = reinterpret_cast<uint32_t*>(d_scratch);
-	const uint32_t nm = n2_lattice_walked_levels(a.scale, lat.inv_res[2] * (lat.extent[2] < 0.f ? -lat.extent[2] : lat.extent[2]));
+	const float step_z = lat.inv_res[2] * lat.extent[2], end_x = lat.corner[0] + lat.extent[0];
+	const uint32_t rows = n2_lattice_row_levels(a.scale, lat.res[0], fabsf(lat.inv_res[0] * lat.extent[0]), fmaxf(fabsf(lat.corner[0]), fabsf(end_x)), step_z);
+	const uint32_t walked = n2_lattice_walked_levels(a.scale, fabsf(step_z));
+	const bool by_rows = n2_lattice_by_rows(rows, walked, (uint64_t)lat.res[0] * lat.res[1] * lat.res[2]);
+	const uint32_t nm = by_rows ? rows : walked;
 	a.first_fine = nm;
 	const uint32_t n_fine = tab.n_levels > nm ? tab.n_levels - nm : 0u;
-	static_assert(LT_LEVELS - 6u <= LT_MAX_FINE, "the fine levels' features fit the scratch");
-	lattice_frags_kernel<<<dim3(SDF_FRAG_COUNT), dim3(64), 0, s>>>(reinterpret_cast<const hf*>(nets.sdf_w), nets.sdf_in_w, tab.n_levels * 2u, reinterpret_cast<hf*>(d_frags));
-	N2_LAUNCH_CHECK();
+	void (*const kernels[7])(LatticeArgs) = {lattice_walk_kernel<4>, lattice_walk_kernel<5>, lattice_walk_kernel<6>, lattice_walk_kernel<7>, lattice_walk_kernel<8>, lattice_walk_kernel<9>,
+	                                         lattice_walk_kernel<10>};
+	auto* const walk_kernel = by_rows ? kernels[nm - 4u] : nm == 10u ? lattice_gather_walk_kernel<10> : nm == 8u ? lattice_gather_walk_kernel<8> : lattice_gather_walk_kernel<6>;
+	if (n_fine == 0) {
+		lattice_frags_kernel<<<dim3(FRAG_BLOCKS), dim3(LT_BLOCK), 0, s>>>(a);
+		N2_LAUNCH_CHECK();
+	}
 	// a slab holds as many points as the scratch has room for the fine levels' features of
 	const uint32_t rx = lat.res[0], ry = lat.res[1], rz = lat.res[2];
 	const N2LatticeSlab slab = n2_lattice_slab(lat.res, (uint64_t)LT_MAX_FINE * chunk / (n_fine ? n_fine : 1u));
@@ -469,12 +704,11 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 				a.walk = (a.nz + parts - 1u) / parts;
 				const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk), blocks = (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
 				if (n_fine) {
-					lattice_fine_kernel<<<dim3(blocks * n_fine), dim3(LT_BLOCK), 0, s>>>(a, blocks);
+					const bool first = x0 == 0 && y0 == 0 && z0 == 0;
+					lattice_fine_kernel<<<dim3(blocks * n_fine + (first ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks);
 					N2_LAUNCH_CHECK();
 				}
-				if (nm == 10u) lattice_walk_kernel<10><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
-				else if (nm == 8u) lattice_walk_kernel<8><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
-				else lattice_walk_kernel<6><<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+				walk_kernel<<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
 				N2_LAUNCH_CHECK();
 			}
 	return N2_OK;

@@ -48,14 +48,32 @@ N2_HD inline void n2_lattice_chunks(uint32_t c_first, uint32_t c_last, uint32_t&
 	chunks = (uint32_t)((hi - lo) >> 2) + 1u;
 }
 
-// Levels that the lattice's walk keeps planes of, by the step along z (it is right for any level and step).  A level whose cells are
-// larger than a step crosses into a new plane less than once per step; of one whose cells are smaller every step meets two
-// planes and nothing is kept, but up to about 1.15 cells per step that costs less than its features' way through memory.
-// Call in us with 6 | 8 | 10 levels walked, the default table: 64^3 59 | 61 | 60, 128^3 187 | 190 | 197, 176^3 438 | 407 | 427, 208^3 647 | 679 | 675,
-// 224^3 792 | 767 | 776, 256^3 1056 | 1001 | 1010, 272^3 1335 | 1273 | 1257, 320^3 1918 | 1856 | 1742, 384^3 3097 | 2858 | 2706, 464^3 5812 | 5485 | 5107,
-// 512^3 6783 | 6220 | 5745; 512 x 512 x 128 1777 | 1726 | 1789, 320 x 320 x 128 791 | 830 | 827, 128 x 128 x 512 692 | 668 | 664.
+// Levels that the lattice's walk keeps planes of where its points gather for themselves (lattice_gather_walk_kernel), by the step along z.
+// It is right for any level and step.  A level whose cells are larger than a step crosses into a new plane less than once per step; of one
+// whose cells are smaller every step meets two planes and nothing is kept, but up to about 1.15 cells per step that costs less than its
+// features' way through memory.  (Call in us with 6 | 8 | 10 levels walked, the default table, when every lattice took this kernel and it was a
+// tenth slower: 128^3 187 | 190 | 197, 176^3 438 | 407 | 427, 208^3 647 | 679 | 675, 256^3 1056 | 1001 | 1010, 272^3 1335 | 1273 | 1257, 384^3 3097 | 2858 | 2706,
+// 512^3 6783 | 6220 | 5745; 512 x 512 x 128 1777 | 1726 | 1789, 128 x 128 x 512 692 | 668 | 664.)
 static inline uint32_t n2_lattice_walked_levels(const float scale[16], float step) {
 	return scale[8] * step < 1.15f ? 10u : scale[7] * step < 0.95f ? 8u : 6u;
+}
+// The levels that lattice_walk_kernel can take, by where their vertices lie: a run of up to 64 points that are `step_x` apart meets at most
+// 62 vertices of a row, which stand in the wave's lanes then, and a step along z (step_z >= 0) never leaves out a plane.  reach: the
+// largest coordinate along x; where it is too large for a cell's number to be exact in fp32 nothing is known about a run's vertices.
+// At most ten: a wave has registers for no more.
+static inline uint32_t n2_lattice_row_levels(const float scale[16], uint32_t nx, float step_x, float reach, float step_z) {
+	const float points = (float)(nx < 64u ? nx : 64u) - 1.f;
+	uint32_t l = 0;
+	while (l < 10u && points * scale[l] * step_x <= 60.f && scale[l] * reach < 4194304.f && step_z >= 0.f && scale[l] * step_z < 0.95f) ++l;
+	return l;
+}
+// Which of the two.  A plane costs lattice_walk_kernel half the loads, but it walks fewer levels where the points are further apart along x
+// than along z.  Call in us, gathering | by rows, (levels): 64^3 60 (6) | 81 (4), 80^3 83 (6) | 81 (5), 512 x 64 x 64 121 (6) | 128 (4),
+// 512 x 512 x 64 913 (6) | 840 (4), 512 x 512 x 128 1604 (6) | 1495 (6), 256 x 256 x 512 1782 (10) | 1725 (8), 96 x 304 x 304 859 (10) | 852 (5),
+// 128 x 512 x 512 2420 (10) | 2536 (6), 80 x 512 x 400 1638 (10) | 1703 (5), 64 x 512 x 512 1624 (10) | 1799 (4), 512^3 5219 (10) | 4802 (10).
+// (With four levels walked, the other twelve levels' features of a small lattice do not fit the scratch at once.)
+static inline bool n2_lattice_by_rows(uint32_t rows, uint32_t walked, uint64_t points) {
+	return rows + 2u >= walked && (rows >= 5u || (rows == 4u && points >= 1u << 23));
 }
 
 // ----------------------------------------------------------------------------

@@ -98,6 +98,39 @@ def test_lattice_equals_the_same_points_queried(res, chunk, box, levels):
     assert_close(host(d), want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
 
 
+# Steps of 1 / side and planes of 1 / side: every number of levels that is walked by rows (sides 80 to 512; four only on large lattices), rows that
+# end inside a run, several slabs, all three widths of the fine levels' rows; more levels walked along z than along x, boxes upside
+# down along z and x, and one far from the unit cube (four vertices gathered per point and plane).  `part` of the box that is evaluated.
+@pytest.mark.parametrize("side,res,part,chunk", [(80, (80, 6, 80), 1, 1 << 14), (112, (112, 4, 56), 0.5, 1 << 14), (150, (75, 5, 40), (0.5, 40 / 150), 1 << 11), (210, (70, 9, 66), (70 / 210, 66 / 210), 1 << 14),
+                                                 (304, (152, 4, 38), (0.5, 0.125), 1 << 12), (416, (104, 5, 52), (0.25, 0.125), 1 << 14), (512, (130, 6, 64), (130 / 512, 0.125), 1 << 14),
+                                                 (64, (512, 512, 64), (1, 1), 1 << 22), (512, (64, 6, 128), (1, 0.25), 1 << 14), (512, (130, 6, 64), (130 / 512, -0.125), 1 << 14),
+                                                 (512, (130, 6, 64), (-130 / 512, 0.125), 1 << 14), (512, (66, 4, 64), (66 / 512, 0.125, 3e4), 1 << 14)])
+def test_lattices_walked_by_rows_equal_the_same_points_queried(side, res, part, chunk):
+    from neus2_amd.mesh import density_on_grid
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork()
+    p = torch.randn(net.param_offsets()[4], device="cuda", generator=torch.Generator(device="cuda").manual_seed(side)) * 0.1
+    net.set_params(p.half(), None)
+    net.reserve(max(1 << 16, chunk))
+    part = part if isinstance(part, tuple) else (part, part)
+    at = part[2] if len(part) == 3 else 0.0
+    f = np.float32
+    lo = np.array([at + (0.3 if part[0] < 1 else 0), 0.2, 0.4 if abs(part[1]) < 1 else 0], f)
+    hi = lo + np.array([part[0], res[1] / 300, part[1]], f)
+    d = density_on_grid(net._h, res, tuple(lo), tuple(hi), chunk=chunk)
+    keep = [np.arange(r) if r < 300 else np.unique(np.linspace(0, r - 1, 23).astype(int)) for r in res]  # of a large lattice some rows
+    z, y, x = np.meshgrid(*(k.astype(f) for k in reversed(keep)), indexing="ij")
+    ext = hi - lo
+    pos = np.stack([(c * f(f(1.0) / f(r))) * e + b for c, r, e, b in zip((x, y, z), res, ext, lo)]).reshape(3, -1)
+    n = pos.shape[1]
+    padded = np.full((3, (n + 7) // 8 * 8), 0.5, f)
+    padded[:, :n] = pos
+    net.reserve(max(1 << 16, chunk, padded.shape[1]))
+    want = host(net.sdf(dev(padded)))[0, :n].reshape(z.shape)
+    got = host(d)[np.ix_(*reversed(keep))]
+    assert_close(got, want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
+
+
 # rows longer than the chunk, down to the smallest one: slabs of a few runs, and of less than one
 @pytest.mark.parametrize("res,chunk", [((513, 3, 5), 64), ((200, 4, 3), 8)])
 def test_lattice_of_rows_longer_than_the_chunk(res, chunk):

@@ -29,6 +29,8 @@ extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels,
 }
 extern "C" void lattice_chunks(uint32_t first, uint32_t last, uint32_t* out) { n2_lattice_chunks(first, last, out[0], out[1]); }
 extern "C" uint32_t walked_levels(const float* scale, float step) { return n2_lattice_walked_levels(scale, step); }
+extern "C" uint32_t row_levels(const float* scale, uint32_t nx, float step_x, float reach, float step_z) { return n2_lattice_row_levels(scale, nx, step_x, reach, step_z); }
+extern "C" int by_rows(uint32_t rows, uint32_t walked, uint64_t points) { return n2_lattice_by_rows(rows, walked, points); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
 
@@ -112,3 +114,33 @@ def test_lattice_chunks_hold_every_cell_of_the_run(rules, first, last):
     lo, chunks = C.c_int32(out[0]).value, out[1]
     a, b = min(first, last), max(first, last)
     assert lo % 4 == 0 and lo <= a < lo + 4 and lo + 4 * (chunks - 1) <= b + 1 < lo + 4 * chunks
+
+
+# the unit cube at several sizes, part of a run, a box upside down along x and along z, one as large as its cells' numbers are exact, no box
+@pytest.mark.parametrize("nx,lo,hi,planes,down", [(512, 0, 1, 512, 1), (400, 0, 1, 400, 1), (64, 0, 1, 64, 1), (2, 0, 1, 512, 1), (33, 0, 1, 300, 1), (200, 1, 0, 200, 1), (200, 0, 1, 200, -1),
+                                                  (512, -1.5, 2.5, 512, 1), (512, 4e3, 4e3 + 1, 512, 1), (512, 3e5, 3e5 + 1, 512, 1), (512, 0, float("nan"), 512, 1), (512, -2.0 ** 40, 2.0 ** 40, 8, 1)])
+def test_runs_of_the_levels_walked_by_rows_fit_a_wave(rules, nx, lo, hi, planes, down):
+    """The vertices that any 64 points of such a level meet, cells as the kernels round them, are 64 at most; no plane is left out."""
+    f = np.float32
+    scale = [float(f(16 * 1.447 ** l - 1)) for l in range(16)]
+    inv, ext = f(1) / f(nx), f(hi) - f(lo)
+    step_z = f(down) / f(planes)
+    reach = max(abs(f(lo)), abs(f(lo) + ext))
+    n = rules.row_levels((C.c_float * 16)(*scale), C.c_uint32(nx), C.c_float(abs(float(inv * ext))), C.c_float(float(reach)), C.c_float(float(step_z)))
+    assert n <= 10 and (n == 0 or (np.isfinite(hi) and down > 0))
+    x = (np.arange(nx).astype(f) * inv * ext + f(lo)).astype(f)
+    z = (np.arange(planes).astype(f) * abs(step_z)).astype(f)
+    for s in scale[:n]:
+        cell, plane = (np.floor((v.astype(np.float64) * f(s) + 0.5).astype(f)) for v in (x, z))  # one fused multiply-add
+        for at in range(0, nx, 64):
+            run = cell[at:at + 64]
+            assert run.max() + 1 - run.min() < 64
+        assert np.diff(plane).max(initial=0) <= 1
+    if (lo, hi, down) == (0, 1, 1):
+        assert n >= {512: 10, 400: 9, 64: 4}.get(nx, 0)
+
+
+@pytest.mark.parametrize("rows,walked,points,want", [(4, 6, 64 ** 3, 0), (5, 6, 80 ** 3, 1), (4, 6, 512 * 512 * 64, 1), (4, 10, 64 * 512 * 512, 0), (5, 10, 80 * 512 * 400, 0),
+                                                     (8, 10, 256 * 256 * 512, 1), (10, 10, 512 ** 3, 1), (0, 6, 1 << 31, 0), (3, 6, 1 << 31, 0)])
+def test_which_lattices_are_walked_by_rows(rules, rows, walked, points, want):
+    assert rules.by_rows(C.c_uint32(rows), C.c_uint32(walked), C.c_uint64(points)) == want
