@@ -92,9 +92,55 @@ constexpr McTable mc_build_table() {
 
 constexpr McTable MC_TABLE_HOST = mc_build_table();
 
+// The triangles round a cut edge, as mc_normals_kernel wants them.  `axis` is the edge's; along, fast and slow are the axis and the two across
+// it (mc_ring_axes); cube q of the four round the edge starts one step back along slow for q < 2 and along fast for even q.  In the
+// frame (along, fast, slow) an edge of a cube is its first corner, one bit per axis, and its direction << 3.  A triangle that the edge is part of
+// takes twelve bits: the other two edges in the triangle's order, and << 10 the edge's place in it; their number stands in bits 60..62.
+struct McRing {
+	uint64_t fan[3][4][256];  // [axis][cube][corner bits in the frame]
+};
+constexpr int MC_RING_AXES[3][3] = {{0, 1, 2}, {1, 0, 2}, {2, 0, 1}};
+constexpr McRing mc_build_ring() {
+	McRing r{};
+	for (int axis = 0; axis < 3; ++axis) {
+		int corner[8] = {}, local[8] = {}, edge[12] = {};  // corner of the frame -> of the cube and back; the cube's edges in the frame
+		for (int c = 0; c < 8; ++c) {
+			int d[3] = {};
+			for (int k = 0; k < 3; ++k) d[MC_RING_AXES[axis][k]] = (c >> k) & 1;
+			corner[c] = (d[1] ? (d[0] ? 2 : 3) : (d[0] ? 1 : 0)) + 4 * d[2];
+			local[corner[c]] = c;
+		}
+		for (int e = 0; e < 12; ++e) {
+			const int p = local[MC_EDGE_CORNERS[e][0]], q = local[MC_EDGE_CORNERS[e][1]], diff = p ^ q;
+			edge[e] = (p & q) | (diff == 1 ? 0 : diff == 2 ? 8 : 16);
+		}
+		for (int mask = 0; mask < 256; ++mask) {
+			int cube = 0;
+			for (int c = 0; c < 8; ++c) cube |= ((mask >> c) & 1) << corner[c];
+			for (int q = 0; q < 4; ++q) {
+				const int self = ((q & 1) ? 0 : 2) | (q < 2 ? 4 : 0);
+				uint64_t fan = 0, n = 0;
+				for (int t = 0; t < MC_TABLE_HOST.ntri[cube]; ++t) {
+					int at = -1;
+					uint64_t others = 0;
+					for (int k = 2; k >= 0; --k) {
+						const int e = edge[MC_TABLE_HOST.tri[cube][3 * t + k]];
+						if (e == self) at = k;
+						else others = others << 5 | (uint64_t)e;
+					}
+					if (at >= 0) fan |= (others | (uint64_t)at << 10) << (12 * n++);
+				}
+				r.fan[axis][q][mask] = fan | n << 60;
+			}
+		}
+	}
+	return r;
+}
+
 }  // namespace
 
 __device__ const McTable MC_TABLE = mc_build_table();
+__device__ const McRing MC_RING = mc_build_ring();
 
 // ---------------------------------------------------------------------------
 // kernels
@@ -146,10 +192,16 @@ __device__ __forceinline__ McPlace mc_place(const McGrid& g, uint32_t w, uint32_
 // What a word of points owns; written for the words that own something, which the `active` bits tell.
 struct alignas(64) McRecord {
 	mc_word edge[3];       // point has a vertex on its edge towards +axis
-	mc_word tri[3];        // bits 0, 1, 2 of the number of triangles of the point's cube
 	uint32_t first_v, first_t;  // vertices and triangles of the words before this one in its block of 256
+	mc_word tri[3];        // bits 0, 1, 2 of the number of triangles of the point's cube
 	uint32_t pad[2];
 };
+// Which words of a block own something: four words of bits per block.
+template <bool SHORT>
+__device__ __forceinline__ bool mc_owns(const mc_word* __restrict__ active, uint32_t block, uint32_t word) {
+	// (mc_count_kernel has four consecutive words per lane, mc_count_short_kernel one)
+	return SHORT ? (active[block * 4u + (word >> 6)] >> (word & 63u)) & 1ull : (active[block * 4u + (word & 3u)] >> (word >> 2)) & 1ull;
+}
 
 constexpr uint32_t MC_BITS_WORDS = 16;  // words a wave forms at a time: 16 loads in flight per lane
 
@@ -197,8 +249,7 @@ struct McBits {
 __device__ __forceinline__ mc_word mc_first_rows(const McGrid& g, uint32_t n) {
 	return n >> g.rows_log ? (1ull << (1u << MC_SHORT_BITS_LOG)) - 1ull : (1ull << (n << g.pitch_log)) - 1ull;
 }
-// WAVE: the lanes of the wave hold consecutive words, and take the word behind theirs from the next lane
-template <bool WAVE, bool SHORT>
+template <bool SHORT>
 __device__ __forceinline__ McBits mc_load_bits(const McGrid& g, const mc_word* __restrict__ bits, uint32_t w) {
 	McBits B;
 	if constexpr (SHORT) {
@@ -234,10 +285,7 @@ __device__ __forceinline__ McBits mc_load_bits(const McGrid& g, const mc_word* _
 		const bool ok = (!(j & 1u) || yok) && (!(j & 2u) || B.zok);
 		const uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u);
 		B.b[j] = ok ? bits[at] : 0ull;
-		mc_word next = 0ull;
-		if (WAVE) next = __shfl_down(B.b[j], 1);
-		if (!WAVE || (threadIdx.x & 63u) == 63u) next = ok && left > 64u ? bits[at + 1u] : 0ull;
-		if (left <= 64u) next = 0ull;
+		const mc_word next = ok && left > 64u ? bits[at + 1u] : 0ull;
 		B.s[j] = (B.b[j] >> 1) | (next << 63);
 	}
 	return B;
@@ -265,10 +313,164 @@ __device__ __forceinline__ uint32_t mc_wave_scan(uint32_t v, uint32_t lane) {
 	return v;
 }
 
-// One lane per word; a lane walks through the cubes of its word that the surface cuts.  (Listing those cubes in LDS and dealing
-// them to the lanes, as the emitting kernel does, takes the same time: the launch is four rounds of load latency.)
-template <bool SHORT>
-__global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
+// The number of triangles of 64 cubes at a time.  A cube that the surface crosses in one piece has two triangles fewer than cut edges; bits
+// 0, 1, 2 of that number follow from a carry-save addition of the twelve edges' words.  `several`: the cubes that it may cross in several
+// pieces, namely those with a face whose four edges are cut, and those with two opposite corners (inside or outside) alone; their numbers
+// come from the table.
+struct McTriBits {
+	mc_word tri[3], several;
+};
+template <class Word>
+constexpr __host__ __device__ __forceinline__ void mc_add(Word a, Word b, Word c, Word& sum, Word& carry) {
+	sum = a ^ b ^ c;
+	carry = (a & b) | (c & (a | b));
+}
+template <class Word, class Bits>
+constexpr __host__ __device__ __forceinline__ void mc_triangle_bits(const Word (&c)[8], Bits& out) {
+	const Word x[4] = {(Word)(c[0] ^ c[1]), (Word)(c[3] ^ c[2]), (Word)(c[4] ^ c[5]), (Word)(c[7] ^ c[6])};  // edges along x: (y, z) = (0, 0), (1, 0), (0, 1), (1, 1)
+	const Word y[4] = {(Word)(c[0] ^ c[3]), (Word)(c[1] ^ c[2]), (Word)(c[4] ^ c[7]), (Word)(c[5] ^ c[6])};  // along y: (x, z)
+	const Word z[4] = {(Word)(c[0] ^ c[4]), (Word)(c[1] ^ c[5]), (Word)(c[3] ^ c[7]), (Word)(c[2] ^ c[6])};  // along z: (x, y)
+	Word s0 = 0, s1 = 0, s2 = 0, s3 = 0, c0 = 0, c1 = 0, c2 = 0, c3 = 0, c4 = 0, c5 = 0, t0 = 0, t1 = 0, d0 = 0, d1 = 0, d2 = 0, e0 = 0, e1 = 0, e2 = 0, unused = 0;
+	mc_add(x[0], x[1], x[2], s0, c0);
+	mc_add(x[3], y[0], y[1], s1, c1);
+	mc_add(y[2], y[3], z[0], s2, c2);
+	mc_add(z[1], z[2], z[3], s3, c3);
+	mc_add(s0, s1, s2, t0, c4);
+	mc_add(t0, s3, (Word)0, e0, c5);
+	mc_add(c0, c1, c2, t0, d0);
+	mc_add(c3, c4, c5, t1, d1);
+	mc_add(t0, t1, (Word)0, e1, d2);
+	mc_add(d0, d1, d2, e2, unused);
+	const Word faces = (x[0] & x[1] & y[0]) | (x[2] & x[3] & y[2]) | (x[0] & x[2] & z[0]) | (x[1] & x[3] & z[2]) | (y[0] & y[2] & z[0]) | (y[1] & y[3] & z[1]);
+	const Word odd_z = x[0] ^ c[2] ^ c[3] ^ (Word)0, odd_y = x[0] ^ c[4] ^ c[5], odd_x = y[0] ^ c[4] ^ c[7], all = odd_z ^ c[4] ^ c[5] ^ c[6] ^ c[7];
+	out.several = faces | (odd_x & odd_y & odd_z & ~all);
+	out.tri[0] = e0;
+	out.tri[1] = ~e1;
+	out.tri[2] = e2 & e1;
+}
+struct McCaseBits {
+	uint32_t tri[3], several;
+};
+constexpr bool mc_triangle_bits_hold() {
+	for (uint32_t mask = 1; mask < 255; ++mask) {
+		uint32_t c[8] = {};
+		for (uint32_t k = 0; k < 8; ++k) c[k] = (mask >> k) & 1u;
+		McCaseBits b{};
+		mc_triangle_bits(c, b);
+		if (!(b.several & 1u) && (b.tri[0] & 1u) + 2u * (b.tri[1] & 1u) + 4u * (b.tri[2] & 1u) != MC_TABLE_HOST.ntri[mask]) return false;
+	}
+	return true;
+}
+static_assert(mc_triangle_bits_hold(), "the cubes left to the formula have as many triangles as the table says");
+
+// edges, triangles and their numbers of one word (B: its bits and its neighbours')
+__device__ __forceinline__ void mc_own(const McBits& B, McRecord& r, uint32_t& nv, uint32_t& nt) {
+	r.edge[0] = (B.b[0] ^ B.s[0]) & B.xok;
+	r.edge[1] = (B.b[0] ^ B.b[1]) & B.here & B.yok;
+	r.edge[2] = B.zok ? (B.b[0] ^ B.b[2]) & B.here : 0ull;
+	const mc_word corner[8] = {B.b[0], B.s[0], B.s[1], B.b[1], B.b[2], B.s[2], B.s[3], B.b[3]};
+	mc_word any = corner[0], all = corner[0];
+#pragma unroll
+	for (uint32_t k = 1; k < 8; ++k) { any |= corner[k]; all &= corner[k]; }
+	const mc_word cut = B.zok ? any & ~all & B.xok & B.yok : 0ull;
+	r.tri[0] = r.tri[1] = r.tri[2] = 0ull;
+	if (__any(cut != 0ull)) {
+		McTriBits t;
+		mc_triangle_bits(corner, t);
+		const mc_word simple = cut & ~t.several;
+#pragma unroll
+		for (int a = 0; a < 3; ++a) r.tri[a] = t.tri[a] & simple;
+		for (mc_word rest = cut & t.several; rest; rest &= rest - 1ull) {
+			const uint32_t p = (uint32_t)__ffsll(rest) - 1u, n = MC_TABLE.ntri[mc_case(B, p)];
+#pragma unroll
+			for (int a = 0; a < 3; ++a) r.tri[a] |= (mc_word)((n >> a) & 1u) << p;
+		}
+	}
+	nv = (uint32_t)(__popcll(r.edge[0]) + __popcll(r.edge[1]) + __popcll(r.edge[2]));
+	nt = (uint32_t)(__popcll(r.tri[0]) + 2 * __popcll(r.tri[1]) + 4 * __popcll(r.tri[2]));
+}
+
+// One wave per block of 256 words, four consecutive words per lane: with their neighbours in y and z four loads of 32 bytes, and nothing to
+// wait for but these.  (A lane per word in workgroups of four waves, with a table of triangle numbers in LDS: four rounds of workgroups that
+// each waited for the table, the bits and each other, 30 us for 512^3, of which walking through the cut cubes took 3.)
+constexpr uint32_t MC_EACH = 4;
+static_assert(MC_BLOCK == 64u * MC_EACH, "a wave takes a block");
+__global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
+                                                      mc_word* __restrict__ active, uint2* __restrict__ blocks) {
+	typedef mc_word two __attribute__((ext_vector_type(2), aligned(8)));
+	const uint32_t lane = threadIdx.x, w0 = blockIdx.x * MC_BLOCK + lane * MC_EACH;
+	const uint32_t plane = g.row_words * g.ry;
+	// (the same for the wave: all of its loads, and the word behind its last one, are inside the array)
+	const bool inner = (uint64_t)blockIdx.x * MC_BLOCK + MC_BLOCK + 1u + plane + g.row_words <= g.n_words;
+	mc_word b[4][MC_EACH + 1];
+	if (inner) {
+#pragma unroll
+		for (uint32_t j = 0; j < 4; ++j) {
+			const mc_word* at = bits + w0 + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? plane : 0u);
+#pragma unroll
+			for (uint32_t q = 0; q < MC_EACH; q += 2u) {
+				const two v = *reinterpret_cast<const two*>(at + q);
+				b[j][q] = v.x;
+				b[j][q + 1u] = v.y;
+			}
+			b[j][MC_EACH] = lane == 63u ? at[MC_EACH] : 0ull;
+		}
+#pragma unroll
+		for (uint32_t j = 0; j < 4; ++j) {
+			const mc_word next = __shfl_down(b[j][0], 1);
+			if (lane != 63u) b[j][MC_EACH] = next;
+		}
+	}
+	McRecord r[MC_EACH];
+	uint32_t nv[MC_EACH], nt[MC_EACH], sum_v = 0, sum_t = 0;
+	const uint32_t row0 = w0 / g.row_words, col0 = w0 - row0 * g.row_words, z0 = row0 / g.ry;
+	uint32_t col = col0, y = row0 - z0 * g.ry, z = z0;
+#pragma unroll
+	for (uint32_t q = 0; q < MC_EACH; ++q) {
+		nv[q] = nt[q] = 0;
+		McBits B;
+		if (inner) {
+			const uint32_t left = g.rx - col * 64u;  // points from the word's first to the end of the row
+			B.here = left >= 64u ? ~0ull : (1ull << left) - 1ull;
+			B.xok = left > 64u ? ~0ull : (1ull << (left - 1u)) - 1ull;
+			B.yok = y + 1u < g.ry ? ~0ull : 0ull;
+			B.zok = true;  // (a plane lies behind all that the wave loads)
+#pragma unroll
+			for (uint32_t j = 0; j < 4; ++j) {
+				// (rows that are not there meet yok)
+				B.b[j] = b[j][q];
+				B.s[j] = (B.b[j] >> 1) | (left > 64u ? b[j][q + 1u] << 63 : 0ull);
+			}
+			if (++col == g.row_words) {
+				col = 0;
+				if (++y == g.ry) { y = 0; ++z; }
+			}
+		} else if (w0 + q < g.n_words) {
+			B = mc_load_bits<false>(g, bits, w0 + q);
+		}
+		if (inner || w0 + q < g.n_words) mc_own(B, r[q], nv[q], nt[q]);
+		sum_v += nv[q];
+		sum_t += nt[q];
+		const mc_word mask = __ballot(nv[q] + nt[q] > 0u);
+		if (lane == 0) active[blockIdx.x * MC_EACH + q] = mask;
+	}
+	const uint32_t iv = mc_wave_scan(sum_v, lane), it = mc_wave_scan(sum_t, lane);
+	uint32_t first_v = iv - sum_v, first_t = it - sum_t;
+#pragma unroll
+	for (uint32_t q = 0; q < MC_EACH; ++q) {
+		if (nv[q] + nt[q] > 0u) {
+			r[q].first_v = first_v;
+			r[q].first_t = first_t;
+			records[w0 + q] = r[q];
+		}
+		first_v += nv[q];
+		first_t += nt[q];
+	}
+	if (lane == 63) blocks[blockIdx.x] = make_uint2(iv, it);
+}
+
+// Short rows: one lane per word; a lane walks through the cubes of its word that the surface cuts.
+__global__ void __launch_bounds__(MC_BLOCK) mc_count_short_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
                                                             mc_word* __restrict__ active, uint2* __restrict__ blocks) {
 	__shared__ uint8_t ntri[256];
 	__shared__ uint32_t sum_v[MC_BLOCK / 64], sum_t[MC_BLOCK / 64];
@@ -278,7 +480,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const mc_w
 	McRecord r{};
 	uint32_t nv = 0, nt = 0;
 	mc_word cut = 0;
-	const McBits B = mc_load_bits<true, SHORT>(g, bits, min(w, g.n_words - 1u));  // every lane takes part in the exchange
+	const McBits B = mc_load_bits<true>(g, bits, min(w, g.n_words - 1u));
 	if (w < g.n_words) {
 		r.edge[0] = (B.b[0] ^ B.s[0]) & B.xok;
 		r.edge[1] = (B.b[0] ^ B.b[1]) & B.here & B.yok;
@@ -323,39 +525,50 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_kernel(McGrid g, const mc_w
 	if (threadIdx.x == 0) blocks[blockIdx.x] = make_uint2(all_v, all_t);
 }
 
-// Exclusive prefix sums of the blocks' counts in place; element n_blocks receives the totals.
+// Exclusive prefix sums of the blocks' counts in place; element n_blocks receives the totals.  The blocks that own something are listed, their
+// number goes behind the totals.
 constexpr uint32_t MC_SCAN_EACH = 8;
-__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks) {
+__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks, uint32_t* __restrict__ listed) {
 	__shared__ uint2 wave_sum[16];
+	__shared__ uint32_t wave_n[16];
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 	uint2 carry = make_uint2(0, 0);
+	uint32_t carry_n = 0;
 	for (uint32_t c0 = 0; c0 < n_blocks; c0 += 1024u * MC_SCAN_EACH) {
 		const uint32_t i0 = c0 + threadIdx.x * MC_SCAN_EACH;
 		uint2 v[MC_SCAN_EACH], own = make_uint2(0, 0);
+		uint32_t n = 0;
 #pragma unroll
 		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) v[k] = i0 + k < n_blocks ? blocks[i0 + k] : make_uint2(0, 0);
 #pragma unroll
-		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) { own.x += v[k].x; own.y += v[k].y; }
-		const uint32_t ix = mc_wave_scan(own.x, lane), iy = mc_wave_scan(own.y, lane);
-		if (lane == 63) wave_sum[wave] = make_uint2(ix, iy);
+		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) { own.x += v[k].x; own.y += v[k].y; n += (v[k].x | v[k].y) ? 1u : 0u; }
+		const uint32_t ix = mc_wave_scan(own.x, lane), iy = mc_wave_scan(own.y, lane), in = mc_wave_scan(n, lane);
+		if (lane == 63) { wave_sum[wave] = make_uint2(ix, iy); wave_n[wave] = in; }
 		__syncthreads();
 		uint2 run = make_uint2(carry.x + ix - own.x, carry.y + iy - own.y);
+		uint32_t run_n = carry_n + in - n;
 #pragma unroll
 		for (uint32_t k = 0; k < 16; ++k) {
 			const uint2 s = wave_sum[k];
-			if (k < wave) { run.x += s.x; run.y += s.y; }
+			const uint32_t m = wave_n[k];
+			if (k < wave) { run.x += s.x; run.y += s.y; run_n += m; }
 			carry.x += s.x;
 			carry.y += s.y;
+			carry_n += m;
 		}
 #pragma unroll
 		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) {
 			if (i0 + k < n_blocks) blocks[i0 + k] = run;
+			if (v[k].x | v[k].y) listed[run_n++] = i0 + k;
 			run.x += v[k].x;
 			run.y += v[k].y;
 		}
 		__syncthreads();  // the sums have been read
 	}
-	if (threadIdx.x == 0) blocks[n_blocks] = carry;
+	if (threadIdx.x == 0) {
+		blocks[n_blocks] = carry;
+		blocks[n_blocks + 1u] = make_uint2(carry_n, 0u);
+	}
 }
 
 // number of set bits of `b` below this lane
@@ -366,10 +579,6 @@ struct McOwned {
 	mc_word e[3];
 	uint32_t first;
 };
-__device__ __forceinline__ McOwned mc_owned(const McRecord* __restrict__ records, const uint2* __restrict__ blocks, uint32_t w) {
-	const McRecord& r = records[w];
-	return McOwned{{r.edge[0], r.edge[1], r.edge[2]}, blocks[w / MC_BLOCK].x + r.first_v};
-}
 // first vertex of the word's point `lane` | its edge flags << 29
 __device__ __forceinline__ uint32_t mc_vertex_slot(const McOwned& o, uint32_t lane) {
 	uint32_t slot = o.first, flags = 0;
@@ -406,153 +615,212 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 	}
 }
 
-// Workgroup b emits what the words of block b own.  Only one point in ten of such a word owns anything, so the points that do
+// A workgroup emits what the words of a listed block own, and goes on to another one.  Only one point in ten of such a word owns anything, so the points that do
 // are listed and dealt to the lanes: with a wave per word the launch was a chain of memory round trips at a tenth of the
 // lanes, 240 us.  The vertices that a cube uses belong to its own point and to those one further along x, y and z: their
 // slots come from the records of the (at most eight) words those points are in, and stand in LDS, where a triangle's
-// corners pick theirs.
+// corners pick theirs.  What bounds the launch is the chain of round trips: which words own something, their records (they stay in LDS, for
+// their neighbours in y too), then all that a point needs at once; a cube's case comes from the densities that its vertices need.
+// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now EMIT_NOW.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
+constexpr uint32_t MC_EMIT_GRID = 1536;  // as many as run at a time: six per CU, by their LDS
+typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t mc_words3 __attribute__((ext_vector_type(3), aligned(4)));
+typedef float mc_float2 __attribute__((ext_vector_type(2), aligned(4)));
 template <bool SHORT>
-__global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float* __restrict__ density, const mc_word* __restrict__ bits,
+__global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float* __restrict__ density,
                                                            const McRecord* __restrict__ records, const mc_word* __restrict__ active,
-                                                           const uint2* __restrict__ blocks, float* __restrict__ verts, uint32_t* __restrict__ indices,
-                                                           uint32_t* __restrict__ origin) {
+                                                           const uint2* __restrict__ blocks, uint32_t n_blocks, const uint32_t* __restrict__ listed,
+                                                           float* __restrict__ verts, uint32_t* __restrict__ indices, uint32_t* __restrict__ origin) {
 	__shared__ uint16_t list[MC_LIST];
 	__shared__ uint32_t slot_of[8][MC_BLOCK];
 	__shared__ uint32_t wave_sum[MC_BLOCK / 64];
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	const uint32_t mine = blockIdx.x * MC_BLOCK + threadIdx.x;
-	const bool owns = (active[blockIdx.x * (MC_BLOCK / 64) + wave] >> lane) & 1ull;
-	if (!__syncthreads_or(owns)) return;
-	mc_word points = 0;
-	if (owns) {
-		const McRecord& r = records[mine];
-		points = r.edge[0] | r.edge[1] | r.edge[2] | r.tri[0] | r.tri[1] | r.tri[2];
-	}
-	mc_for_points(points, list, wave_sum, [&](uint32_t entry) {
-		const uint32_t w = blockIdx.x * MC_BLOCK + (entry >> 6), p = entry & 63u;
-		const McRecord& r = records[w];
-		const McOwned own = mc_owned(records, blocks, w);
-		const mc_word t0 = r.tri[0], t1 = r.tri[1], t2 = r.tri[2];
-		const McPlace place = mc_place<SHORT>(g, w, p);
-		const uint32_t xyz[3] = {place.x, place.y, place.z};
-		const uint32_t slot0 = mc_vertex_slot(own, p), flags = slot0 >> 29;
-		if (flags) {
-			const uint64_t idx = ((uint64_t)xyz[2] * g.ry + xyz[1]) * g.rx + xyz[0];
-			const uint64_t step[3] = {1u, g.rx, (uint64_t)g.rx * g.ry};
-			const float pos[3] = {(float)xyz[0], (float)xyz[1], (float)xyz[2]};
-			const float f0 = density[idx];
-			float f1[3];
-#pragma unroll
-			for (uint32_t a = 0; a < 3; ++a) f1[a] = ((flags >> a) & 1u) ? density[idx + step[a]] : 0.f;
-			uint32_t slot = slot0 & 0x1FFFFFFFu;
+	__shared__ mc_word edges[3][MC_BLOCK], tri[3][MC_BLOCK];
+	__shared__ uint2 first[MC_BLOCK];
+	const uint32_t n_listed = blocks[n_blocks + 1u].x;
+	for (uint32_t at_block = blockIdx.x; at_block < n_listed; at_block += gridDim.x) {
+		const uint32_t block = listed[at_block], block0 = block * MC_BLOCK;
+		const bool owns = mc_owns<SHORT>(active, block, threadIdx.x);
+		const uint2 before = blocks[block];
+		mc_word points = 0;
+		if (owns) {
+			const McRecord& r = records[block0 + threadIdx.x];
 #pragma unroll
 			for (uint32_t a = 0; a < 3; ++a) {
-				if (!((flags >> a) & 1u)) continue;
-				const float dt = (g.thresh - f0) / (f1[a] - f0);
-				float* v = verts + (size_t)slot * 3;
-#pragma unroll
-				for (uint32_t d = 0; d < 3; ++d) v[d] = (d == a ? pos[d] + dt : pos[d]) * g.scale[d] + g.offset[d];
-				if (origin) { origin[(size_t)slot * 3] = w; origin[(size_t)slot * 3 + 1] = p | a << 6; }
-				++slot;
+				edges[a][threadIdx.x] = r.edge[a];
+				tri[a][threadIdx.x] = r.tri[a];
+				points |= r.edge[a] | r.tri[a];
 			}
+			first[threadIdx.x] = make_uint2(before.x + r.first_v, before.y + r.first_t);
 		}
-		const uint32_t tris = (uint32_t)((t0 >> p) & 1ull) | (uint32_t)((t1 >> p) & 1ull) << 1 | (uint32_t)((t2 >> p) & 1ull) << 2;
-		if (tris == 0) return;  // (the cubes of the last column, row and plane have no triangles: the points below exist)
-#pragma unroll
-		for (uint32_t j = 0; j < 4; ++j) {
-			uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u), bit = p;
-			if (SHORT) {
-				bit = (j & 1u) ? p + (1u << g.pitch_log) : p;
-				at = w + (bit >> MC_SHORT_BITS_LOG) + ((j & 2u) ? g.plane_words : 0u);
-				bit &= (1u << MC_SHORT_BITS_LOG) - 1u;
+		// (mc_for_points' first barrier stands between these stores and their readers)
+		auto owned = [&](uint32_t w) {
+			McOwned o;
+			if (w - block0 < MC_BLOCK) {
+				o = McOwned{{edges[0][w - block0], edges[1][w - block0], edges[2][w - block0]}, first[w - block0].x};
+			} else {
+				const McRecord& r = records[w];
+				o = McOwned{{r.edge[0], r.edge[1], r.edge[2]}, blocks[w / MC_BLOCK].x + r.first_v};
 			}
-			const McOwned o = j == 0 ? own : mc_owned(records, blocks, at);
-			slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, bit);
-			slot_of[2 * j + 1][threadIdx.x] = bit < 63u ? mc_vertex_slot(o, bit + 1u) : mc_vertex_slot(mc_owned(records, blocks, at + 1u), 0u);
-		}
-		const uint32_t first_t = blocks[w / MC_BLOCK].y + r.first_t + mc_below(t0, p) + 2u * mc_below(t1, p) + 4u * mc_below(t2, p);
-		const uint32_t mask = mc_case(mc_load_bits<false, SHORT>(g, bits, w), p);
-		// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
-		// the owner's offset from this point in x, y, z and the edge's axis.
-		constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
-		                           16ull << 40 | 17ull << 45 | 19ull << 50 | 18ull << 55;
-		const uint4 row4 = *reinterpret_cast<const uint4*>(MC_TABLE.tri[mask]);
-		const uint32_t trow[4] = {row4.x, row4.y, row4.z, row4.w};
-		uint32_t* out = indices + (size_t)first_t * 3;
+			return o;
+		};
+		mc_for_points(points, list, wave_sum, [&](uint32_t entry) {
+			const uint32_t at0 = entry >> 6, w = block0 + at0, p = entry & 63u;
+			const McOwned own{{edges[0][at0], edges[1][at0], edges[2][at0]}, first[at0].x};
+			const mc_word t0 = tri[0][at0], t1 = tri[1][at0], t2 = tri[2][at0];
+			const McPlace place = mc_place<SHORT>(g, w, p);
+			const uint32_t tris = (uint32_t)((t0 >> p) & 1ull) | (uint32_t)((t1 >> p) & 1ull) << 1 | (uint32_t)((t2 >> p) & 1ull) << 2;
+			// the point's density and those at +1 along x, in the four rows of its cube (where they are not there, those of the last row or plane)
+			const uint32_t x0 = min(place.x, g.rx - 2u);
+			float low[4], high[4];
 #pragma unroll
-		for (uint32_t k = 0; k < 15; ++k) {
-			if (k < 3u * tris) {
-				const uint32_t e = (trow[k >> 2] >> (8u * (k & 3u))) & 0xFu;
-				const uint32_t code = (uint32_t)(OWNER >> (5u * e)) & 31u;
-				const uint32_t at = slot_of[code & 7u][threadIdx.x];
-				// the owner's first slot plus the number of its edges before this one
-				out[k] = (at & 0x1FFFFFFFu) + (uint32_t)__popc((at >> 29) & ((1u << (code >> 3)) - 1u));
+			for (uint32_t j = 0; j < 4; ++j) {
+				const uint32_t y = min(place.y + (j & 1u), g.ry - 1u), z = min(place.z + (j >> 1), g.rz - 1u);
+				const mc_float2 v = *reinterpret_cast<const mc_float2*>(density + ((uint64_t)z * g.ry + y) * g.rx + x0);
+				low[j] = place.x == x0 ? v.x : v.y;
+				high[j] = v.y;
 			}
-		}
-	});
+			if (tris) {  // (the cubes of the last column, row and plane have no triangles: the points below exist)
+#pragma unroll
+				for (uint32_t j = 0; j < 4; ++j) {
+					uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u), bit = p;
+					if (SHORT) {
+						bit = (j & 1u) ? p + (1u << g.pitch_log) : p;
+						at = w + (bit >> MC_SHORT_BITS_LOG) + ((j & 2u) ? g.plane_words : 0u);
+						bit &= (1u << MC_SHORT_BITS_LOG) - 1u;
+					}
+					const McOwned o = j == 0 ? own : owned(at);
+					slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, bit);
+					slot_of[2 * j + 1][threadIdx.x] = bit < 63u ? mc_vertex_slot(o, bit + 1u) : mc_vertex_slot(owned(at + 1u), 0u);
+				}
+			}
+			const uint32_t slot0 = mc_vertex_slot(own, p), flags = slot0 >> 29;
+			if (flags) {
+				const float pos[3] = {(float)place.x, (float)place.y, (float)place.z}, f1[3] = {high[0], low[1], low[2]};
+				uint32_t slot = slot0 & 0x1FFFFFFFu;
+#pragma unroll
+				for (uint32_t a = 0; a < 3; ++a) {
+					if (!((flags >> a) & 1u)) continue;
+					const float dt = (g.thresh - low[0]) / (f1[a] - low[0]);
+					n2_float3 v;
+#pragma unroll
+					for (uint32_t d = 0; d < 3; ++d) v[d] = (d == a ? pos[d] + dt : pos[d]) * g.scale[d] + g.offset[d];
+					n2_store3<false>(verts + (size_t)slot * 3, v);
+					if (origin) *reinterpret_cast<mc_words2*>(origin + (size_t)slot * 3) = mc_words2{w, p | a << 6};
+					++slot;
+				}
+			}
+			if (tris == 0) return;
+			const uint32_t first_t = first[at0].y + mc_below(t0, p) + 2u * mc_below(t1, p) + 4u * mc_below(t2, p);
+			const float corner[8] = {low[0], high[0], high[1], low[1], low[2], high[2], high[3], low[3]};
+			uint32_t mask = 0;
+#pragma unroll
+			for (uint32_t k = 0; k < 8; ++k) mask |= corner[k] > g.thresh ? 1u << k : 0u;
+			// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
+			// the owner's offset from this point in x, y, z and the edge's axis.
+			constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
+			                           16ull << 40 | 17ull << 45 | 19ull << 50 | 18ull << 55;
+			const uint4 row4 = *reinterpret_cast<const uint4*>(MC_TABLE.tri[mask]);
+			const uint32_t trow[4] = {row4.x, row4.y, row4.z, row4.w};
+			uint32_t* out = indices + (size_t)first_t * 3;
+#pragma unroll
+			for (uint32_t t = 0; t < 5; ++t) {
+				if (t < tris) {
+					mc_words3 v;
+#pragma unroll
+					for (uint32_t c = 0; c < 3; ++c) {
+						const uint32_t k = 3 * t + c, e = (trow[k >> 2] >> (8u * (k & 3u))) & 0xFu;
+						const uint32_t code = (uint32_t)(OWNER >> (5u * e)) & 31u;
+						const uint32_t at = slot_of[code & 7u][threadIdx.x];
+						// the owner's first slot plus the number of its edges before this one
+						v[c] = (at & 0x1FFFFFFFu) + (uint32_t)__popc((at >> 29) & ((1u << (code >> 3)) - 1u));
+					}
+					*reinterpret_cast<mc_words3*>(out + 3 * t) = v;
+				}
+			}
+		});
+	}
 }
 
 // accumulate_1ring's normals: a vertex's is the sum of (pb - pa) x (pa - pc) over the triangles it is a corner of.  They lie in
 // the four cubes round the vertex's edge; the cubes are visited in lattice order and their triangles in theirs, so the sum
 // does not depend on how the work is scheduled.  (Adding every triangle to its corners with float atomics took 276 us for
 // the 512^3 sphere's 1.2 M triangles: 11 M atomics at the part's 40 G/s.)
+// The triangles' other corners are worked out again from the density, by the arithmetic that placed them: the eighteen values of the four
+// cubes tell which triangles there are (MC_RING) and where their corners lie.  That is 18 loads a vertex and vector instructions; going
+// through the words' records to the triangles and from those to the vertices was some 45 loads, most of them lines of their own, one a
+// clock and CU: 34 us for 512^3, now NORMALS_NOW.
 template <bool SHORT>
-__global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const McRecord* __restrict__ records,
-                                                              const mc_word* __restrict__ active, const uint2* __restrict__ blocks,
-                                                              const uint32_t* __restrict__ indices, const float* __restrict__ verts,
-                                                              float* __restrict__ normals) {
+__global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const float* __restrict__ density, float* __restrict__ normals) {
+	__shared__ float values[18][MC_BLOCK];  // [slow -1 .. 1][fast -1 .. 1][along 0, 1]
 	const uint32_t i = blockIdx.x * MC_BLOCK + threadIdx.x;
 	if (i >= n_verts) return;
 	float* mine = normals + (size_t)i * 3;
 	const uint32_t w = __float_as_uint(mine[0]), place = __float_as_uint(mine[1]);
-	const uint32_t lane = place & 63u, axis = place >> 6;
-	const McPlace p = mc_place<SHORT>(g, w, lane);
-	const uint32_t xyz[3] = {p.x, p.y, p.z};
-	// the two axes across the edge, the slower one first
-	const uint32_t slow = axis == 2u ? 1u : 2u, fast = axis == 0u ? 1u : 0u;
-	uint32_t first[4], count[4];
+	const uint32_t axis = place >> 6;
+	const McPlace p = mc_place<SHORT>(g, w, place & 63u);
+	// in the frame (along, fast, slow): the point, the lattice and its strides
+	const uint64_t row = g.rx, plane = (uint64_t)g.rx * g.ry;
+	const uint32_t at[3] = {axis == 0u ? p.x : axis == 1u ? p.y : p.z, axis == 0u ? p.y : p.x, axis == 2u ? p.y : p.z};
+	const uint32_t size[3] = {0u, axis == 0u ? g.ry : g.rx, axis == 2u ? g.ry : g.rz};
+	const uint64_t step[3] = {axis == 0u ? 1u : axis == 1u ? row : plane, axis == 0u ? row : 1u, axis == 2u ? row : plane};
+	const float scale[3] = {axis == 0u ? g.scale[0] : axis == 1u ? g.scale[1] : g.scale[2], axis == 0u ? g.scale[1] : g.scale[0], axis == 2u ? g.scale[1] : g.scale[2]};
+	const float offset[3] = {axis == 0u ? g.offset[0] : axis == 1u ? g.offset[1] : g.offset[2], axis == 0u ? g.offset[1] : g.offset[0], axis == 2u ? g.offset[1] : g.offset[2]};
+	const bool below[3] = {false, at[1] > 0u, at[2] > 0u}, above[3] = {false, at[1] + 1u < size[1], at[2] + 1u < size[2]};
+	const float* here = density + (p.z * plane + p.y * row + p.x);
+	uint32_t inside = 0;
 #pragma unroll
-	for (uint32_t k = 0; k < 4; ++k) {
-		const uint32_t back_slow = k < 2u ? 1u : 0u, back_fast = (k & 1u) ? 0u : 1u;
-		const uint32_t bx = fast == 0u ? back_fast : 0u, by = (fast == 1u ? back_fast : 0u) + (slow == 1u ? back_slow : 0u), bz = slow == 2u ? back_slow : 0u;
-		count[k] = 0;
-		first[k] = 0;
-		if (bx > xyz[0] || by > xyz[1] || bz > xyz[2]) continue;
-		const uint32_t x = xyz[0] - bx, y = xyz[1] - by, z = xyz[2] - bz;
-		uint32_t at = (z * g.ry + y) * g.row_words + (x >> 6), l = x & 63u;
-		if (SHORT) {
-			at = z * g.plane_words + (y >> g.rows_log);
-			l = (y & ((1u << g.rows_log) - 1u)) << g.pitch_log | x;
+	for (uint32_t k = 0; k < 3; ++k) {
+		// (where there is nothing beyond the point, its own row or plane again: the cubes that would use it are left out)
+		const float* in_k = k == 0u ? (below[2] ? here - step[2] : here) : k == 2u ? (above[2] ? here + step[2] : here) : here;
+#pragma unroll
+		for (uint32_t j = 0; j < 3; ++j) {
+			const float* in_j = j == 0u ? (below[1] ? in_k - step[1] : in_k) : j == 2u ? (above[1] ? in_k + step[1] : in_k) : in_k;
+#pragma unroll
+			for (uint32_t o = 0; o < 2; ++o) {
+				const float v = in_j[o ? step[0] : 0u];
+				values[6 * k + 2 * j + o][threadIdx.x] = v;
+				inside |= v > g.thresh ? 1u << (6 * k + 2 * j + o) : 0u;
+			}
 		}
-		if (!((active[at >> 6] >> (at & 63u)) & 1ull)) continue;
-		const McRecord& r = records[at];
-		const mc_word t0 = r.tri[0], t1 = r.tri[1], t2 = r.tri[2];
-		count[k] = (uint32_t)((t0 >> l) & 1ull) | (uint32_t)((t1 >> l) & 1ull) << 1 | (uint32_t)((t2 >> l) & 1ull) << 2;
-		first[k] = blocks[at / MC_BLOCK].y + r.first_t + mc_below(t0, l) + 2u * mc_below(t1, l) + 4u * mc_below(t2, l);
 	}
-	float sum[3] = {0.f, 0.f, 0.f};
+	// position of the vertex on the edge that starts at `corner` of the cube whose first corner is (0, j, k) - 1 of the values, as mc_emit_kernel gives it
+	auto vertex = [&](uint32_t j, uint32_t k, uint32_t edge, float (&to)[3]) {
+		const uint32_t dir = edge >> 3, n = (edge & 1u) + 2u * (j + ((edge >> 1) & 1u)) + 6u * (k + ((edge >> 2) & 1u)), next = n + (dir == 0u ? 1u : dir == 1u ? 2u : 6u);
+		const float f0 = values[n][threadIdx.x], f1 = values[next][threadIdx.x], dt = (g.thresh - f0) / (f1 - f0);
+		const float from[3] = {(float)(at[0] + (edge & 1u)), (float)(at[1] + j - 1u + ((edge >> 1) & 1u)), (float)(at[2] + k - 1u + ((edge >> 2) & 1u))};
 #pragma unroll
-	for (uint32_t k = 0; k < 4; ++k) {
-		uint32_t tri[5][3];
+		for (uint32_t d = 0; d < 3; ++d) to[d] = (from[d] + (dir == d ? dt : 0.f)) * scale[d] + offset[d];
+	};
+	float self[3], sum[3] = {0.f, 0.f, 0.f};
+	vertex(1u, 1u, 0u, self);
 #pragma unroll
-		for (uint32_t t = 0; t < 5; ++t)
+	for (uint32_t q = 0; q < 4; ++q) {
+		const uint32_t j = q & 1u, k = q >> 1;  // the cube's first corner among the values
+		if (!(j ? above[1] : below[1]) || !(k ? above[2] : below[2])) continue;
+		const uint32_t corners = ((inside >> (6u * k + 2u * j)) & 15u) | ((inside >> (6u * k + 6u + 2u * j)) & 15u) << 4;
+		uint64_t fan = MC_RING.fan[axis][q][corners];
+		for (uint32_t n = (uint32_t)(fan >> 60); n; --n, fan >>= 12) {
+			float p1[3], p2[3];
+			vertex(j, k, (uint32_t)fan & 31u, p1);
+			vertex(j, k, (uint32_t)(fan >> 5) & 31u, p2);
+			const uint32_t me = (uint32_t)(fan >> 10) & 3u;
+			float u[3], v[3];
 #pragma unroll
-			for (uint32_t c = 0; c < 3; ++c) tri[t][c] = t < count[k] ? indices[(size_t)(first[k] + t) * 3 + c] : 0xFFFFFFFFu;
-#pragma unroll
-		for (uint32_t t = 0; t < 5; ++t) {
-			if (tri[t][0] != i && tri[t][1] != i && tri[t][2] != i) continue;
-			const float* pa = verts + (size_t)tri[t][0] * 3;
-			const float* pb = verts + (size_t)tri[t][1] * 3;
-			const float* pc = verts + (size_t)tri[t][2] * 3;
-			const float u[3] = {pb[0] - pa[0], pb[1] - pa[1], pb[2] - pa[2]}, v[3] = {pa[0] - pc[0], pa[1] - pc[1], pa[2] - pc[2]};
+			for (uint32_t d = 0; d < 3; ++d) {
+				const float pa = me == 0u ? self[d] : p1[d], pb = me == 0u ? p1[d] : me == 1u ? self[d] : p2[d], pc = me == 2u ? self[d] : p2[d];
+				u[d] = pb - pa;
+				v[d] = pa - pc;
+			}
 			sum[0] += u[1] * v[2] - u[2] * v[1];
 			sum[1] += u[2] * v[0] - u[0] * v[2];
 			sum[2] += u[0] * v[1] - u[1] * v[0];
 		}
 	}
-#pragma unroll
-	for (uint32_t d = 0; d < 3; ++d) mine[d] = sum[d];
+	// (along y the frame is left-handed)
+	mine[0] = axis == 0u ? sum[0] : axis == 1u ? 0.f - sum[1] : sum[1];
+	mine[1] = axis == 0u ? sum[1] : axis == 1u ? 0.f - sum[0] : sum[2];
+	mine[2] = axis == 0u ? sum[2] : axis == 1u ? 0.f - sum[2] : sum[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -576,11 +844,11 @@ static int mc_check(const char* fn, const uint32_t res[3], uint64_t& n) {
 }
 
 // Workspace: the points' bits, one record per word (written only where a word owns something), which words do, and the
-// prefix sums over blocks of 256 words (one entry more than blocks: the totals).
+// prefix sums over blocks of 256 words (behind them the totals and the number of blocks that own something), and a list of those blocks.
 struct McCarve {
 	uint32_t row_words, pitch_log, rows_log, plane_words, n_words, n_blocks;
 	bool short_rows;
-	uint64_t bits, records, active, blocks, total;
+	uint64_t bits, records, active, blocks, listed, total;
 };
 static McCarve mc_carve(const uint32_t res[3]) {
 	McCarve c;
@@ -597,7 +865,8 @@ static McCarve mc_carve(const uint32_t res[3]) {
 	c.bits = take(sizeof(mc_word) * (uint64_t)c.n_words);
 	c.records = take(sizeof(McRecord) * (uint64_t)c.n_words);
 	c.active = take(sizeof(mc_word) * (uint64_t)c.n_blocks * (MC_BLOCK / 64));
-	c.blocks = take(sizeof(uint2) * ((uint64_t)c.n_blocks + 1));
+	c.blocks = take(sizeof(uint2) * ((uint64_t)c.n_blocks + 2));
+	c.listed = take(sizeof(uint32_t) * (uint64_t)c.n_blocks);
 	c.total = o;
 	return c;
 }
@@ -646,10 +915,10 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	                                       : (stream_density ? mc_bits_kernel<true, false> : mc_bits_kernel<false, false>);
 	bits_kernel<<<mgrid(((uint64_t)c.n_words + MC_BITS_WORDS - 1) / MC_BITS_WORDS * 64u), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits);
 	N2_LAUNCH_CHECK();
-	auto* const count_kernel = c.short_rows ? mc_count_kernel<true> : mc_count_kernel<false>;
-	count_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
+	auto* const count_kernel = c.short_rows ? mc_count_short_kernel : mc_count_kernel;
+	count_kernel<<<dim3(c.n_blocks), dim3(c.short_rows ? MC_BLOCK : 64u), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
 	N2_LAUNCH_CHECK();
-	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks);
+	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks, reinterpret_cast<uint32_t*>(b + c.listed));
 	N2_LAUNCH_CHECK();
 	uint32_t host[2] = {0, 0};
 	N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
@@ -672,18 +941,17 @@ N2_API int n2_marching_cubes_emit(n2_stream_t stream, const uint32_t res[3], con
 	hipStream_t s = n2_stream(stream);
 	const McCarve c = mc_carve(res);
 	unsigned char* b = reinterpret_cast<unsigned char*>(d_workspace);
-	const mc_word* bits = reinterpret_cast<const mc_word*>(b + c.bits);
 	const McRecord* records = reinterpret_cast<const McRecord*>(b + c.records);
 	const mc_word* active = reinterpret_cast<const mc_word*>(b + c.active);
 	const uint2* blocks = reinterpret_cast<const uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
 	auto* const emit_kernel = c.short_rows ? mc_emit_kernel<true> : mc_emit_kernel<false>;
-	emit_kernel<<<dim3(c.n_blocks), dim3(MC_BLOCK), 0, s>>>(g, d_density, bits, records, active, blocks, d_vertices, d_indices,
+	emit_kernel<<<dim3(c.n_blocks < MC_EMIT_GRID ? c.n_blocks : MC_EMIT_GRID), dim3(MC_BLOCK), 0, s>>>(g, d_density, records, active, blocks, c.n_blocks, reinterpret_cast<const uint32_t*>(b + c.listed), d_vertices, d_indices,
 	                                                        reinterpret_cast<uint32_t*>(d_normals));
 	N2_LAUNCH_CHECK();
 	if (d_normals) {
 		auto* const normals_kernel = c.short_rows ? mc_normals_kernel<true> : mc_normals_kernel<false>;
-		normals_kernel<<<mgrid(n_vertices), dim3(MC_BLOCK), 0, s>>>(g, n_vertices, records, active, blocks, d_indices, d_vertices, d_normals);
+		normals_kernel<<<mgrid(n_vertices), dim3(MC_BLOCK), 0, s>>>(g, n_vertices, d_density, d_normals);
 		N2_LAUNCH_CHECK();
 	}
 	return N2_OK;
