@@ -26,6 +26,7 @@
 #include "n2_common.h"
 
 #include <cstring>
+#include <mutex>
 
 #pragma clang fp contract(off)
 
@@ -148,17 +149,17 @@ __device__ const McRing MC_RING = mc_build_ring();
 // The density is read once, for one bit per lattice point (inside or not); everything up to the vertex positions is then
 // worked out from the bits, 64 points of a row at a time:
 //   mc_bits     density -> bits                                                   (bound by HBM: 4 bytes per point)
-//   mc_count    one lane per word: its edge vertices and triangles as bit masks, prefix sums within a block of 256 words
-//   mc_scan     one workgroup: prefix sums over the blocks, the totals the host asks for
-//   mc_emit     one wave per word that owns something: vertices and triangles
+//   mc_count    four words per lane: their edge vertices and triangles as bit masks, prefix sums within a block of 256 words
+//   mc_scan     one workgroup: prefix sums over the blocks, the list of the blocks that own something, the totals
+//   mc_emit     a workgroup per listed block: its vertices and triangles
 //   mc_normals  one lane per vertex: the sum over the triangles of the four cubes round its edge
 // Rows are padded to whole words, so a word's neighbours in y and z are words too and no mask crosses a row.
 // Lattices whose rows have fewer than 16 points (SHORT) put several rows of a plane into the lower half of a word, each padded to
 // a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 29, scan 9, emit 46, normals 34, with
-// the host's wait for the totals 227 in all.  Deciding every point from the four rows of the density itself took 242 for the
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 17, scan 9, emit 33, normals 24, with
+// the host's wait for the totals 182 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
 struct McGrid {
@@ -528,7 +529,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_short_kernel(McGrid g, cons
 // Exclusive prefix sums of the blocks' counts in place; element n_blocks receives the totals.  The blocks that own something are listed, their
 // number goes behind the totals.
 constexpr uint32_t MC_SCAN_EACH = 8;
-__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks, uint32_t* __restrict__ listed) {
+__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks, uint32_t* __restrict__ listed, uint32_t* __restrict__ totals) {
 	__shared__ uint2 wave_sum[16];
 	__shared__ uint32_t wave_n[16];
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -568,6 +569,7 @@ __global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2*
 	if (threadIdx.x == 0) {
 		blocks[n_blocks] = carry;
 		blocks[n_blocks + 1u] = make_uint2(carry_n, 0u);
+		if (totals) { totals[0] = carry.x; totals[1] = carry.y; }
 	}
 }
 
@@ -621,7 +623,7 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // slots come from the records of the (at most eight) words those points are in, and stand in LDS, where a triangle's
 // corners pick theirs.  What bounds the launch is the chain of round trips: which words own something, their records (they stay in LDS, for
 // their neighbours in y too), then all that a point needs at once; a cube's case comes from the densities that its vertices need.
-// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now EMIT_NOW.)
+// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 33.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
 constexpr uint32_t MC_EMIT_GRID = 1536;  // as many as run at a time: six per CU, by their LDS
 typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -749,7 +751,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 // The triangles' other corners are worked out again from the density, by the arithmetic that placed them: the eighteen values of the four
 // cubes tell which triangles there are (MC_RING) and where their corners lie.  That is 18 loads a vertex and vector instructions; going
 // through the words' records to the triangles and from those to the vertices was some 45 loads, most of them lines of their own, one a
-// clock and CU: 34 us for 512^3, now NORMALS_NOW.
+// clock and CU: 34 us for 512^3, now 24.
 template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const float* __restrict__ density, float* __restrict__ normals) {
 	__shared__ float values[18][MC_BLOCK];  // [slow -1 .. 1][fast -1 .. 1][along 0, 1]
@@ -895,6 +897,48 @@ static McGrid mc_grid(const uint32_t res[3], const float aabb_min[3], const floa
 	return g;
 }
 
+// Where the scan leaves the totals for the host: slots of one page of pinned memory, each held by a call while it waits.  (Copied to the call's own
+// variables they cost a copy kernel and its staging: 512^3 191 -> 182 us, 64^3 61 -> 53.)  The page stays for the process; where there is none, or
+// every slot is held, the totals are copied.
+class McTotalsSlot {
+public:
+	McTotalsSlot() {
+		std::lock_guard<std::mutex> lock(mutex_);
+		if (!asked_) {
+			asked_ = true;
+			hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (another thread may be capturing: an allocation is no part of that)
+			(void)hipThreadExchangeStreamCaptureMode(&mode);
+			if (hipHostMalloc(reinterpret_cast<void**>(&page_), SLOTS * STRIDE * sizeof(uint32_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+				(void)hipGetLastError();
+				page_ = nullptr;
+			}
+			(void)hipThreadExchangeStreamCaptureMode(&mode);
+		}
+		for (uint32_t k = 0; page_ && k < SLOTS && !at_; ++k)
+			if (!((held_ >> k) & 1u)) {
+				held_ |= 1u << k;
+				slot_ = k;
+				at_ = page_ + k * STRIDE;
+			}
+	}
+	~McTotalsSlot() {
+		std::lock_guard<std::mutex> lock(mutex_);
+		if (at_) held_ &= ~(1u << slot_);
+	}
+	McTotalsSlot(const McTotalsSlot&) = delete;
+	McTotalsSlot& operator=(const McTotalsSlot&) = delete;
+	uint32_t* get() const { return at_; }
+
+private:
+	static constexpr uint32_t SLOTS = 32, STRIDE = 32;  // a cache line each
+	static inline std::mutex mutex_;
+	static inline uint32_t* page_ = nullptr;
+	static inline uint32_t held_ = 0;
+	static inline bool asked_ = false;
+	uint32_t* at_ = nullptr;
+	uint32_t slot_ = 0;
+};
+
 N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,
                                    const float* d_density, void* d_workspace, uint64_t workspace_bytes, uint32_t* n_vertices,
                                    uint32_t* n_triangles) {
@@ -918,11 +962,13 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	auto* const count_kernel = c.short_rows ? mc_count_short_kernel : mc_count_kernel;
 	count_kernel<<<dim3(c.n_blocks), dim3(c.short_rows ? MC_BLOCK : 64u), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
 	N2_LAUNCH_CHECK();
-	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks, reinterpret_cast<uint32_t*>(b + c.listed));
+	const McTotalsSlot slot;
+	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks, reinterpret_cast<uint32_t*>(b + c.listed), slot.get());
 	N2_LAUNCH_CHECK();
 	uint32_t host[2] = {0, 0};
-	N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
+	if (!slot.get()) N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
 	N2_HIP(hipStreamSynchronize(s));
+	if (slot.get()) memcpy(host, slot.get(), sizeof(host));
 	N2_REQUIRE(host[0] < (1u << 29), "n2_marching_cubes_count: %u vertices exceed the 2^29 limit", host[0]);
 	*n_vertices = host[0];
 	*n_triangles = host[1];

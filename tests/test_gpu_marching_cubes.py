@@ -59,6 +59,43 @@ def test_rows_of_words(res):
     assert marching_cubes(dev(f), 0.0, want_normals=False)[2] is None
 
 
+@pytest.mark.parametrize("res", [(512, 512, 128), (320, 64, 16)])
+def test_a_plane_through_every_block_of_words(res):
+    """More blocks that own something than workgroups emit at a time, and waves that count whole blocks: one vertex per row, two triangles per square."""
+    from neus2_amd.mesh import marching_cubes
+    rx, ry, rz = res
+    f = (torch.arange(rx, device="cuda") - 200.25).expand(rz, ry, rx).contiguous()
+    v, t, n = marching_cubes(f, 0.0, (0, 0, 0), res)  # (one unit per cell)
+    assert v.shape == (ry * rz, 3) and t.shape == (2 * (ry - 1) * (rz - 1), 3)
+    v, t, n = (a.cpu().view(*s, 3) for a, s in ((v, (rz, ry)), (t, (rz - 1, ry - 1, 2)), (n, (rz, ry))))
+    assert bool((v[..., 0] == 200.25).all())
+    assert torch.equal(v[..., 1], torch.arange(ry).float().expand(rz, ry)) and torch.equal(v[..., 2], torch.arange(rz).float().view(-1, 1).expand(rz, ry))
+    z, y = torch.meshgrid(torch.arange(rz - 1), torch.arange(ry - 1), indexing="ij")
+    corner = (z * ry + y).int()
+    assert torch.equal(t.reshape(rz - 1, ry - 1, 6).amin(-1), corner) and torch.equal(t.reshape(rz - 1, ry - 1, 6).amax(-1), corner + ry + 1)
+    assert bool((n[..., 1:] == 0).all()) and bool((n[1:-1, 1:-1, 0].abs() == 6).all())  # six triangles of twice the area one
+
+
+def test_meshes_counted_by_several_threads_at_once():
+    """Each call waits for totals of its own; more calls than there are slots for them."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from neus2_amd.mesh import marching_cubes
+    fields = [dev(np.random.default_rng(k).standard_normal((6 + k % 5, 9 + k % 7, 20 + k)).astype(np.float32)) for k in range(40)]
+    want = [tuple(host(a) for a in marching_cubes(f, 0.0)) for f in fields]
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            out = [marching_cubes(fields[(k + q) % 40], 0.0) for q in range(4)]
+            torch.cuda.current_stream().synchronize()
+            return [tuple(host(a) for a in o) for o in out]
+    with ThreadPoolExecutor(40) as pool:
+        for k, got in enumerate(pool.map(work, range(40))):
+            for q, o in enumerate(got):
+                for a, b in zip(o, want[(k + q) % 40]):
+                    np.testing.assert_array_equal(a, b)
+
+
 def test_empty_lattice_and_errors():
     from neus2_amd import capi
     from neus2_amd.mesh import marching_cubes
