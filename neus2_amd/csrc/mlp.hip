@@ -439,10 +439,13 @@ static inline uint32_t stream_grid(uint32_t n, uint32_t waves_per_tile) {
 	return blocks < (uint32_t)MLP_MAX_SLABS ? blocks : (uint32_t)MLP_MAX_SLABS;
 }
 static inline size_t frag_bytes(int n_frags) { return (size_t)n_frags * 64 * 16; }
-// workgroups of the weight-gradient kernels: rounds of 128 samples in a grid-stride loop, two workgroups per CU
+// Waves of a weight-gradient workgroup, and workgroups of a launch: rounds of 32 samples per wave in a grid-stride loop, eight
+// waves per CU.  One workgroup of eight leaves half as many slabs as two of four; up to one workgroup of four per CU, the batch
+// spreads over more CUs that way.
+static inline uint32_t wgrad_waves(uint32_t n) { return n > 32u * 4u * 256u ? 8u : 4u; }
 static inline uint32_t wgrad_grid(uint32_t n) {
-	const uint32_t rounds = (n + WG_SAMPLES - 1) / WG_SAMPLES;
-	return rounds < (uint32_t)MLP_MAX_SLABS ? rounds : (uint32_t)MLP_MAX_SLABS;
+	const uint32_t per_round = 32u * wgrad_waves(n), rounds = (n + per_round - 1) / per_round;
+	return rounds < 256u ? rounds : 256u;
 }
 uint32_t n2_mlp_wgrad_blocks(uint32_t n) { return wgrad_grid(n); }
 
@@ -599,6 +602,25 @@ static int allow_lds(K kernel, size_t bytes) {
 	return N2_OK;
 }
 
+template <int IC, int NH, int WANT_DX, bool SECOND, class Tail, class... Args>
+static int launch_wgrad(hipStream_t s, uint32_t n, bool dy_aos, const Args&... args) {
+	auto with_waves = [&](auto waves) -> int {
+		constexpr int WAVES = decltype(waves)::value;
+		auto launch = [&](auto* kernel) -> int {
+			constexpr size_t lds = mlp_wgrad_lds<WAVES, IC, NH>();
+			if (int rc = allow_lds(kernel, lds)) return rc;
+			kernel<<<dim3(wgrad_grid(n)), dim3(64 * WAVES), lds, s>>>(args...);
+			N2_LAUNCH_CHECK();
+			return N2_OK;
+		};
+		if constexpr (!Tail::active)
+			if (!dy_aos) return launch(mlp_wgrad_kernel<WAVES, IC, NH, WANT_DX, SECOND, false, Tail>);
+		return launch(mlp_wgrad_kernel<WAVES, IC, NH, WANT_DX, SECOND, true, Tail>);
+	};
+	if (wgrad_waves(n) == 8u) return with_waves(std::integral_constant<int, 8>{});
+	return with_waves(std::integral_constant<int, 4>{});
+}
+
 // unit_row >= 0: dL_doutput is the constant e_{unit_row} and d_dL_doutput is not read
 static int mlp_backward_impl(n2_mlp_t* mlp, n2_stream_t stream, const n2_half* d_input, uint32_t n,
                              const n2_half* d_dL_doutput, n2_layout dL_layout, int unit_row, n2_half* d_dL_dinput, n2_grad_mode mode,
@@ -635,21 +657,16 @@ static int mlp_backward_impl(n2_mlp_t* mlp, n2_stream_t stream, const n2_half* d
 	} while (0)
 #define LAUNCH_W(IC, NH, DX)                                                                                        \
 	do {                                                                                                            \
-		const size_t lds = mlp_wgrad_lds<IC, NH, false>();                                                          \
-		if (int rc = allow_lds(mlp_wgrad_kernel<IC, NH, DX, false>, lds)) return rc;                                \
-		mlp_wgrad_kernel<IC, NH, DX, false><<<dim3(blocks), dim3(MLP_BLOCK), lds, s>>>(mlp->params, X, n, dY, aos & 1, (int)dy_rows, dX, \
-			next_slabs(mlp), nullptr, nullptr, -1, x_index, x_cols, dy_gain, dy_gain_inv, mlp->frag_image);                            \
+		if (int rc = launch_wgrad<IC, NH, DX, false, WgNoTail>(s, n, aos & 1, mlp->params, X, n, dY, (int)dy_rows, dX, next_slabs(mlp), nullptr, nullptr, -1, \
+			x_index, x_cols, dy_gain, dy_gain_inv, mlp->frag_image, WgNoTail())) return rc;                             \
 	} while (0)
 	// the field's colour net (48 inputs, two hidden layers): only the rows the field reads are stored
 	N2_REQUIRE(tail == nullptr || (want_dx && want_dw && dx_out_and_normal_only && mlp->in_w == 48 && mlp->n_hidden == 2 && (aos & 1) && dy_rows <= 8),
 	           "n2_mlp_backward: the field's tail goes with the colour net's launch (48 inputs, two hidden layers, AoS output gradient)");
 	if (want_dx && want_dw && dx_out_and_normal_only && mlp->in_w == 48 && mlp->n_hidden == 2) {
 		if (tail) {
-			WgFieldPrepTail t{*tail};
-			const size_t lds = mlp_wgrad_lds<3, 2, false>();
-			if (int rc = allow_lds(mlp_wgrad_kernel<3, 2, WG_DX_OUT_AND_NORMAL, false, WgFieldPrepTail>, lds)) return rc;
-			mlp_wgrad_kernel<3, 2, WG_DX_OUT_AND_NORMAL, false, WgFieldPrepTail><<<dim3(blocks), dim3(MLP_BLOCK), lds, s>>>(mlp->params, X, n, dY, aos & 1,
-				(int)dy_rows, dX, next_slabs(mlp), nullptr, nullptr, -1, x_index, x_cols, dy_gain, dy_gain_inv, mlp->frag_image, t);
+			if (int rc = launch_wgrad<3, 2, WG_DX_OUT_AND_NORMAL, false, WgFieldPrepTail>(s, n, true, mlp->params, X, n, dY, (int)dy_rows, dX, next_slabs(mlp), nullptr,
+				nullptr, -1, x_index, x_cols, dy_gain, dy_gain_inv, mlp->frag_image, WgFieldPrepTail{*tail})) return rc;
 		} else {
 			LAUNCH_W(3, 2, WG_DX_OUT_AND_NORMAL);
 		}
@@ -752,33 +769,26 @@ int n2_mlp_backward_and_second_order_indexed(n2_mlp_t* mlp, n2_stream_t stream, 
 	const int aos = dL_layout == N2_LAYOUT_AOS ? 1 : 0;
 	const int unit_row2 = d_second_dL_doutput == nullptr ? 0 : -1;
 	N2ProfScope prof(N2_PROF_MLP_BACKWARD, s);
+	auto launch = [&](auto ic, auto want_dx) {
+		return launch_wgrad<decltype(ic)::value, 1, decltype(want_dx)::value, true, WgNoTail>(s, n, aos != 0, mlp->params, reinterpret_cast<const hf*>(d_input), n,
+			reinterpret_cast<const hf*>(d_dL_doutput), MLP_OUT, reinterpret_cast<hf*>(d_dL_dinput), next_slabs(mlp), reinterpret_cast<const hf*>(d_dL_ddLdinput),
+			reinterpret_cast<const hf*>(d_second_dL_doutput), unit_row2, d_index, n_cols, 1.f, 1.f, mlp->frag_image, WgNoTail());
+	};
+	using std::integral_constant;
+	int rc;
 	if (dx_encoding_only && mlp->in_w == 48) {
 		// the field's SDF net: only the encoding's rows of dL/dinput are stored
-		const size_t lds = mlp_wgrad_lds<3, 1, true>();
-		if (int rc = allow_lds(mlp_wgrad_kernel<3, 1, WG_DX_ENCODING, true>, lds)) return rc;
-		mlp_wgrad_kernel<3, 1, WG_DX_ENCODING, true><<<dim3(blocks), dim3(MLP_BLOCK), lds, s>>>(mlp->params,
-			reinterpret_cast<const hf*>(d_input), n, reinterpret_cast<const hf*>(d_dL_doutput), aos, MLP_OUT,
-			reinterpret_cast<hf*>(d_dL_dinput), next_slabs(mlp), reinterpret_cast<const hf*>(d_dL_ddLdinput),
-			reinterpret_cast<const hf*>(d_second_dL_doutput), unit_row2, d_index, n_cols, 1.f, 1.f, mlp->frag_image);
-		N2_LAUNCH_CHECK();
-		return reduce_partials(mlp, s, blocks, mode);
+		rc = launch(integral_constant<int, 3>{}, integral_constant<int, WG_DX_ENCODING>{});
+	} else {
+		switch (mlp->in_w / 16) {
+			case 1: rc = launch(integral_constant<int, 1>{}, integral_constant<int, WG_DX_ALL>{}); break;
+			case 2: rc = launch(integral_constant<int, 2>{}, integral_constant<int, WG_DX_ALL>{}); break;
+			case 3: rc = launch(integral_constant<int, 3>{}, integral_constant<int, WG_DX_ALL>{}); break;
+			case 4: rc = launch(integral_constant<int, 4>{}, integral_constant<int, WG_DX_ALL>{}); break;
+			default: n2_set_error("mlp: unsupported shape"); return N2_ERR_UNSUPPORTED;
+		}
 	}
-	switch (mlp->in_w / 16) {
-#define CASE(IC)                                                                                                           \
-	case IC: {                                                                                                             \
-		const size_t lds = mlp_wgrad_lds<IC, 1, true>();                                                                   \
-		if (int rc = allow_lds(mlp_wgrad_kernel<IC, 1, WG_DX_ALL, true>, lds)) return rc;                                  \
-		mlp_wgrad_kernel<IC, 1, WG_DX_ALL, true><<<dim3(blocks), dim3(MLP_BLOCK), lds, s>>>(mlp->params,                   \
-			reinterpret_cast<const hf*>(d_input), n, reinterpret_cast<const hf*>(d_dL_doutput), aos, MLP_OUT,              \
-			reinterpret_cast<hf*>(d_dL_dinput), next_slabs(mlp), reinterpret_cast<const hf*>(d_dL_ddLdinput),              \
-			reinterpret_cast<const hf*>(d_second_dL_doutput), unit_row2, d_index, n_cols, 1.f, 1.f, mlp->frag_image);                       \
-		break;                                                                                                             \
-	}
-		CASE(1) CASE(2) CASE(3) CASE(4)
-#undef CASE
-		default: n2_set_error("mlp: unsupported shape"); return N2_ERR_UNSUPPORTED;
-	}
-	N2_LAUNCH_CHECK();
+	if (rc) return rc;
 	return reduce_partials(mlp, s, blocks, mode);
 }
 

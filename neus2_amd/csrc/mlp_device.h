@@ -241,14 +241,15 @@ __device__ __forceinline__ half8 mlp_frag_value(const hf* __restrict__ W, int f,
 		return v;
 	}
 }
-template <int IC, int NH>
+template <int IC, int NH, int BLOCK = MLP_BLOCK>
 __device__ __forceinline__ void build_frags(hf* F, const hf* __restrict__ W, int count) {
-	for (int idx = threadIdx.x; idx < count * 64; idx += MLP_BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = mlp_frag_value<IC, NH>(W, idx >> 6, idx & 63);
+	for (int idx = threadIdx.x; idx < count * 64; idx += BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = mlp_frag_value<IC, NH>(W, idx >> 6, idx & 63);
 	__syncthreads();
 }
 // the same fragments from an image that another launch has built in global memory (count KiB)
+template <int BLOCK = MLP_BLOCK>
 __device__ __forceinline__ void load_frags(hf* F, const hf* __restrict__ image, int count) {
-	for (int idx = threadIdx.x; idx < count * 64; idx += MLP_BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = *reinterpret_cast<const half8*>(image + (size_t)idx * 8);
+	for (int idx = threadIdx.x; idx < count * 64; idx += BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = *reinterpret_cast<const half8*>(image + (size_t)idx * 8);
 	__syncthreads();
 }
 

@@ -1,29 +1,35 @@
 // Backward pass of the fully fused 64-wide MLP WITH weight gradients (and, for one hidden layer, the second-order pass
-// riding along): every wave runs the forward and the data-gradient chain for its OWN 32 samples only, and the batch
-// reductions dW = dh h^T take their operands from LDS, where the four waves of a workgroup leave the activations and
-// their gradients of 128 samples.
+// riding along): every wave runs the forward and the data-gradient chain for tiles of 32 samples of its own and adds the
+// tile's part of the batch reductions dW = dh h^T to accumulators of its own; the waves meet once, at the end, to add up.
 //
 // The chain produces matrices in sample-lane form (lane = sample, registers = rows); a product over samples needs
-// them in row-lane form (lane = row, registers = 8 consecutive samples), for both operands.  The staging buffer is laid
-// out as quads, S[quad q][sample s] = rows 4q .. 4q+3 of sample s (8 bytes): a lane writes the rows it holds with 8-byte
-// stores, and ds_read_b64_tr_b16 hands a row-lane its samples: in every group of 16 lanes, lane i receives as element j
-// the (i % 4)-th 16-bit value of what lane i / 4 + 4 j of the group addressed.  With lane a + 4 j' of a group addressing
-// quad qb + a of sample k + j', lane i gets row 4 qb + i for the samples k .. k+3: two such reads are one MFMA operand
-// (32 rows x 16 samples).  A quad row is 128 x 8 + 32 bytes, so the four quads of a read fall on different banks.
+// them in row-lane form (lane = row, registers = 8 samples), for both operands.  They change form through a staging
+// buffer of the wave's own in LDS, laid out as quads, S[quad q][sample s] = rows 4q .. 4q+3 of sample s (8 bytes): a lane
+// writes the rows it holds with 8-byte stores, and ds_read_b64_tr_b16 hands a row-lane its samples: in every group of 16
+// lanes, lane i receives as element j the (i % 4)-th 16-bit value of what lane i / 4 + 4 j of the group addressed.  With
+// lane a + 4 j' of a group addressing quad qb + a of sample k + j', lane i gets row 4 qb + i for the samples k .. k+3: two
+// such reads are one operand of v_mfma_f32_16x16x32_f16 (16 rows x 32 samples).  Which samples a lane holds where does not
+// matter as long as both operands agree: group G takes samples 16 (G & 1) + 4 (G >> 1) + {0..3, 8..11}, so that with quad
+// rows of 32 x 8 + 32 bytes the four quads of two groups fall on different banks.
 //
-// Stages of a round (a stage = write, barrier, products, barrier), two hidden layers:  {dy, h1} -> dW_out,
-// {dh1, h0} -> dW_1, {dh0, x} -> dW_0; one hidden layer with the second-order pass:  {dy, h, g, a} -> dW_out,
-// {dh, x} -> dW_0, {b, v} -> dW_0.  The weight-gradient tiles (32 x 32) of a matrix are dealt to the four waves; where a
-// matrix has two tiles only, the waves split the samples or the two products.  Each wave then holds 48 accumulator
-// registers instead of 128, and no activation is computed twice.
+// Stages (a stage = write, read back, products; the LDS runs a wave's accesses in their order, so no barrier and no second
+// buffer), two hidden layers:  {dy, h1} -> dW_out, {dh1, h0} -> dW_1, {dh0, x} -> dW_0; one hidden layer with the second-order
+// pass:  {dy, h} -> dW_out, {g, a} -> dW_out, {dh, x} -> dW_0, {b, v} -> dW_0.
+// A wave holds all tiles of the weight gradients: 16 x 16 tiles have no padding, 128 accumulator registers for 48 -> 64 -> 64 -> 16,
+// which leaves the chain 128 at two waves per SIMD.  (The tiles dealt to the four waves of a workgroup, 48 accumulator
+// registers, takes eight barriers for every 128 samples: at 2^18 samples 40 us for that network and 33 for 48 -> 64 -> 16 with the
+// second-order pass, now 37 and 28; both at 52344 samples 28 -> 26, at 16 384 21 -> 20.)
 #pragma once
 #include "grid_device.h"
 #include "mlp_device.h"
 
-constexpr int WG_SAMPLES = 128;              // samples per workgroup round (4 waves x 32)
-constexpr int WG_QP = WG_SAMPLES * 8 + 32;   // bytes per quad row of the staging buffer
+#include <type_traits>
+
+constexpr int WG_QP = 32 * 8 + 32;      // bytes per quad row of a wave's staging buffer
+constexpr int WG_STAGE = 32 * WG_QP;    // a wave's staging buffer: two matrices of 64 rows
 
 typedef short short4v __attribute__((ext_vector_type(4)));
+typedef float float4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4v* lds_short4_ptr;
 
 // staging writes: v holds 8 rows of the lane's sample; `at` = S + quad offset of the rows' block + the lane's part
@@ -39,20 +45,34 @@ __device__ __forceinline__ void stage_chained(unsigned char* at, const half8& v)
 	*reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
 	*reinterpret_cast<uint2*>(at + 2 * WG_QP) = make_uint2(w[2], w[3]);
 }
-// row-lane MFMA operand: rows 4 qb .. 4 qb + 31, samples 16 kc .. 16 kc + 15 of the round; tr = S + the lane's part
-// ((4 (G & 1) + (l & 3)) * WG_QP + (8 (G >> 1) + ((l & 15) >> 2)) * 8, G = l / 16)
-__device__ __forceinline__ half8 row_operand(const unsigned char* tr, int qb, int kc) {
-	const unsigned char* p = tr + qb * WG_QP + kc * 128;
+// row-lane MFMA operand: rows 16 c .. 16 c + 15, the 32 samples; tr = S + the lane's part
+// (l & 3) * WG_QP + (16 (G & 1) + 4 (G >> 1) + ((l & 15) >> 2)) * 8, G = l / 16
+__device__ __forceinline__ half8 row_operand(const unsigned char* tr, int c) {
+	const unsigned char* p = tr + 4 * c * WG_QP;
 	const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(p));
-	const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(p + 32));
+	const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(p + 64));
 	const short8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 	return __builtin_bit_cast(half8, v);
 }
-// acc += A B^T over the sample chunks [kc0, kc0 + NK): A = rows of quad base qa, B = rows of quad base qb
-template <int NK>
-__device__ __forceinline__ void wgrad_tile(const unsigned char* tr, int qa, int qb, int kc0, float16v& acc) {
+// Between a wave's writes to its staging buffer and its reads, and the reads and the next writes: the LDS keeps them in
+// order, this keeps the compiler from changing it.
+__device__ __forceinline__ void stage_order() {
+	asm volatile("" ::: "memory");
+	__builtin_amdgcn_sched_barrier(0);
+}
+// acc[AT + i * NB + j] += A_i B_j^T: A = the 16 NA rows from chunk ca of the staging buffer, B = the 16 NB rows from chunk cb
+template <int AT, int NA, int NB, int T>
+__device__ __forceinline__ void wgrad_tiles(const unsigned char* tr, int ca, int cb, float4v (&acc)[T]) {
+	static_assert(AT + NA * NB <= T, "tiles of the network");
+	half8 b[NB];
 #pragma unroll
-	for (int k = 0; k < NK; ++k) acc = N2_MFMA(row_operand(tr, qa, kc0 + k), row_operand(tr, qb, kc0 + k), acc);
+	for (int j = 0; j < NB; ++j) b[j] = row_operand(tr, cb + j);
+#pragma unroll
+	for (int i = 0; i < NA; ++i) {
+		const half8 a = row_operand(tr, ca + i);
+#pragma unroll
+		for (int j = 0; j < NB; ++j) acc[AT + i * NB + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[j], acc[AT + i * NB + j], 0, 0, 0);
+	}
 }
 
 // input operands (natural K order) of one 32-sample tile; column `col` of a matrix with n_cols columns
@@ -93,14 +113,38 @@ struct WgFieldPrepTail {
 	N2FieldPrepTail a;
 };
 
-template <int IC, int NH, int WANT_DX, bool SECOND, class Tail = WgNoTail>
-__global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __restrict__ W, const hf* __restrict__ X, uint32_t N, const hf* __restrict__ dY,
-                                                                 int dy_aos, int dy_rows, hf* __restrict__ dX, float* __restrict__ partials,
+// the 16 x 16 tiles of the weight gradients: W_0 (4 x IC), W_1 (4 x 4, two hidden layers), W_out (1 x 4), row by row
+template <int IC, int NH>
+struct WgTiles {
+	static constexpr int WH = 4 * IC, WO = WH + (NH - 1) * 16, COUNT = WO + 4;
+};
+// dynamic LDS of the kernel: fragments, then the waves' staging buffers
+template <int WAVES, int IC, int NH>
+constexpr size_t mlp_wgrad_lds() {
+	return (size_t)FragMap<IC, NH>::SEL * 1024 + (size_t)WAVES * WG_STAGE;
+}
+// At the end the waves exchange their tiles through LDS in columns of four (a column of 16 of W_0 or W_1, the whole of W_out), as many at a
+// time as fit it (a column of every wave: WAVES * 4 KiB), and wave w adds up tile w % 4 of every column (of every second one, where there are eight).
+template <int WAVES, int IC, int NH>
+struct WgFold {
+	static constexpr int COLS = WgTiles<IC, NH>::COUNT / 4, FIT = (int)(mlp_wgrad_lds<WAVES, IC, NH>() - 64) / (WAVES * 4096);
+	static constexpr int PASSES = (COLS + FIT - 1) / FIT, PER = (COLS + PASSES - 1) / PASSES;
+	static_assert(FIT >= 1 && WAVES * PER * 4096 + 64 <= mlp_wgrad_lds<WAVES, IC, NH>(), "a pass, and a value of every wave behind it, fit");
+	// place of tile t of column c among the accumulators
+	static constexpr int tile(int c, int t) {
+		using T = WgTiles<IC, NH>;
+		return c < IC ? t * IC + c : c < COLS - 1 ? T::WH + t * 4 + (c - IC) : T::WO + t;
+	}
+};
+
+template <int WAVES, int IC, int NH, int WANT_DX, bool SECOND, bool DY_AOS, class Tail = WgNoTail>
+__global__ void __launch_bounds__(64 * WAVES, 8 / WAVES) mlp_wgrad_kernel(const hf* __restrict__ W, const hf* __restrict__ X, uint32_t N, const hf* __restrict__ dY,
+                                                                 int dy_rows, hf* __restrict__ dX, float* __restrict__ partials,
                                                                  const hf* __restrict__ V, const hf* __restrict__ G2, int unit_row2,
                                                                  const uint32_t* __restrict__ x_index, uint32_t x_cols, float dy_gain, float dy_gain_inv,
                                                                  const hf* __restrict__ frag_image, const Tail tail = Tail()) {
 	static_assert(!SECOND || NH == 1, "the second-order pass needs one hidden layer");
-	static_assert(!Tail::active || (IC == 3 && NH == 2 && WANT_DX == WG_DX_OUT_AND_NORMAL), "the field's tail goes with the colour net");
+	static_assert(!Tail::active || (IC == 3 && NH == 2 && WANT_DX == WG_DX_OUT_AND_NORMAL && DY_AOS), "the field's tail goes with the colour net");
 	// dy_gain = 2^k, dy_gain_inv = 2^-k (first-order launches only).  The output gradient is multiplied by 2^k when it is
 	// loaded and everything the launch hands on (dL/dinput, the weight-gradient slab) by 2^-k in fp32, so the chain between
 	// them, whose matrices are rounded to fp16 for the matrix cores, works on values 2^k larger: an output gradient in the
@@ -108,45 +152,78 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __res
 	// near 2e-6) then loses nothing, the products with a power of two being exact.  2^0 leaves every value as it is.
 	const float gain_inv = SECOND ? 1.f : dy_gain_inv;
 	using M = FragMap<IC, NH>;
+	using T = WgTiles<IC, NH>;
+	using Fold = WgFold<WAVES, IC, NH>;
+	constexpr uint32_t ROUND = 32 * WAVES;  // samples of a workgroup's round
 	constexpr int IN_W = 16 * IC, IN_MT = M::IN_MT;
 	constexpr int N_PARAMS = MLP_WIDTH * IN_W + (NH - 1) * MLP_WIDTH * MLP_WIDTH + MLP_OUT * MLP_WIDTH;
 	extern __shared__ __align__(16) unsigned char smem[];
 	hf* F = reinterpret_cast<hf*>(smem);
-	unsigned char* S = smem + (size_t)M::SEL * 1024;  // staging buffer behind the fragments
-	// (frag_image: the fragments as a launch in front of this one has left them in global memory, M::SEL KiB; null: built here)
-	if (frag_image) load_frags(F, frag_image, M::SEL);
-	else build_frags<IC, NH>(F, W, M::SEL);
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, g = lane >> 5;
-	const int mt = __builtin_amdgcn_readfirstlane(wave >> 1), nt = __builtin_amdgcn_readfirstlane(wave & 1);
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31;
 	const uint32_t s_local = 32u * wave + n;
-	unsigned char* const st_nat = S + s_local * 8u + 2u * g * WG_QP;
-	unsigned char* const st_ch = S + s_local * 8u + (uint32_t)g * WG_QP;
+	unsigned char* const S = smem + (size_t)M::SEL * 1024 + wave * WG_STAGE;  // the wave's staging buffer behind the fragments
+	unsigned char* const st_nat = S + n * 8 + 2 * (lane >> 5) * WG_QP;
+	unsigned char* const st_ch = S + n * 8 + (lane >> 5) * WG_QP;
 	const int G = lane >> 4;
-	const unsigned char* const tr = S + (4 * (G & 1) + (lane & 3)) * WG_QP + (8 * (G >> 1) + ((lane & 15) >> 2)) * 8;
-	float16v gW0 = zero16(), gWh = zero16(), gWo = zero16();
+	const unsigned char* const tr = S + (lane & 3) * WG_QP + (16 * (G & 1) + 4 * (G >> 1) + ((lane & 15) >> 2)) * 8;
+	float4v acc[T::COUNT];
+#pragma unroll
+	for (auto& t : acc) t = float4v{0.f, 0.f, 0.f, 0.f};
 	float var_acc = 0.f;  // tail: this lane's part of the variance gradient
-	const uint32_t n_rounds = (N + WG_SAMPLES - 1) / WG_SAMPLES;
-	for (uint32_t round = blockIdx.x; round < n_rounds; round += gridDim.x) {
-		const uint32_t col_raw = round * WG_SAMPLES + s_local;
-		const bool valid = col_raw < N;
-		const uint32_t col = valid ? col_raw : N - 1u;
-		// ---- the chain of this wave's 32 samples ----
-		half8 x[IC], dy, h[NH][4];
-		const uint32_t col_src = x_index ? min(x_index[col], x_cols - 1u) : col;  // the sample's column in X
+	const uint32_t n_rounds = (N + ROUND - 1) / ROUND;
+	// A round's operands are loaded while the round before it works: x and dy once its own are staged, the index they go by (a
+	// sample's column in X) before that.  A round has the arithmetic of 6 k cycles and two waves share a SIMD: waiting for
+	// three loads one behind the other, it took 21 k.
+	// (Nothing here may sit in a branch: its join would wait for all loads.  Without an index its load takes a word of X, which has one for each column.)
+	const uint32_t* const index = x_index ? x_index : reinterpret_cast<const uint32_t*>(X);
+	auto column = [&](uint32_t round) { return min(round * ROUND + s_local, N - 1u); };
+	half8 x[IC], dy;
+	auto load = [&](uint32_t col, uint32_t src, int g) __attribute__((always_inline)) {
+		const uint32_t col_src = x_index ? min(src, x_cols - 1u) : col;
 		if constexpr (Tail::active) {
 			// the field keeps the colour net's input sample-major (N2_RGB_IN_PITCH values per column, the rows behind them
 			// are the padding's zeros): an operand is one 16-byte load
+			const hf* const at = X + (size_t)col_src * N2_RGB_IN_PITCH;
 #pragma unroll
-			for (int c = 0; c < IC; ++c)
-				x[c] = 16 * c + 8 * g < (int)N2_RGB_IN_PITCH ? *reinterpret_cast<const half8*>(X + (size_t)col_src * N2_RGB_IN_PITCH + 16 * c + 8 * g) : zero8();
+			for (int c = 0; c < IC; ++c) x[c] = *reinterpret_cast<const half8*>(at + (16 * c + 8 * g < (int)N2_RGB_IN_PITCH ? 16 * c + 8 * g : 0));
 		} else {
 			load_tile_rows<IC>(X, x_index ? x_cols : N, col_src, g, x);
 		}
-		if (dy_aos) {
+		if constexpr (DY_AOS) {
 			dy = *reinterpret_cast<const half8*>(dY + (size_t)col * MLP_OUT + 8 * g);
 		} else {
 #pragma unroll
 			for (int e = 0; e < 8; ++e) dy[e] = dY[(size_t)(8 * g + e) * N + col];
+		}
+		return col_src;
+	};
+	// Awaits the next round's operands (and all loads before them) in front of a round's stores: behind a branch round a store,
+	// a wait for a load becomes one for the store as well.
+	auto arrived = [&]() __attribute__((always_inline)) {
+#pragma unroll
+		for (int c = 0; c < IC; ++c) asm volatile("" : "+v"(x[c]));
+		asm volatile("" : "+v"(dy));
+	};
+	const uint32_t col0 = column(blockIdx.x);
+	uint32_t col_src = load(col0, index[col0], lane >> 5);
+	// (frag_image: the fragments as a launch in front of this one has left them in global memory, M::SEL KiB; null: built here)
+	if (frag_image) load_frags<64 * WAVES>(F, frag_image, M::SEL);
+	else build_frags<IC, NH, 64 * WAVES>(F, W, M::SEL);
+	for (uint32_t round = blockIdx.x; round < n_rounds; round += gridDim.x) {
+		int g = lane >> 5;
+		asm volatile("" : "+v"(g));  // addresses that depend on it are formed anew in every round: kept, they take 40 registers
+		const bool valid = round * ROUND + s_local < N, more = round + gridDim.x < n_rounds;
+		const uint32_t col = column(round), next_col = column(min(round + gridDim.x, n_rounds - 1u));
+		const uint32_t off4 = (4u * g * N + col) * 2u;  // of the column's value in row 4 g (N <= 2^28)
+		const uint32_t next_src = index[next_col];
+		half8 v[SECOND ? IC : 1];
+		if constexpr (SECOND) load_tile_rows<IC>(V, N, col, g, v);
+		// ---- the chain of this wave's 32 samples ----
+		half8 h[NH][4];
+		if constexpr (Tail::active) {
+#pragma unroll
+			for (int c = 0; c < IC; ++c)
+				if (16 * c + 8 * g >= (int)N2_RGB_IN_PITCH) x[c] = zero8();
 		}
 		const half8 dy_all = dy;  // tail: all 16 rows of the output gradient
 #pragma unroll
@@ -158,19 +235,97 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __res
 			for (int e = 0; e < 8; ++e) dy[e] = dy[e] * gain;
 		}
 		hidden_S<IC, NH>(F, lane, x, h);
+		// ---- dW_out = dy h_last^T: chunks dy 0 | h_last 1..4 ----
+		stage_order();
+		stage_natural(st_nat, dy);
+#pragma unroll
+		for (int c = 0; c < 4; ++c) stage_chained(st_ch + 4 * (1 + c) * WG_QP, h[NH - 1][c]);
+		stage_order();
+		wgrad_tiles<T::WO, 1, 4>(tr, 0, 1, acc);
 		half8 dh[NH][4];
 #pragma unroll
 		for (int t = 0; t < 2; ++t)
 			mask_pack(N2_MFMA(frag(F, M::WOT + t, lane), dy, zero16()), h[NH - 1][2 * t], h[NH - 1][2 * t + 1], dh[NH - 1][2 * t], dh[NH - 1][2 * t + 1]);
+		// ---- hidden matrix: dW_1 = dh_1 h_0^T: chunks dh_1 0..3 | h_0 4..7 ----
+		if constexpr (NH > 1) {
+			static_assert(NH <= 2, "one hidden matrix");
+			stage_order();
 #pragma unroll
-		for (int k = NH - 1; k >= 1; --k)
+			for (int c = 0; c < 4; ++c) {
+				stage_chained(st_ch + 4 * c * WG_QP, dh[1][c]);
+				stage_chained(st_ch + 4 * (4 + c) * WG_QP, h[0][c]);
+			}
+			stage_order();
+			wgrad_tiles<T::WH, 4, 4>(tr, 0, 4, acc);
 #pragma unroll
 			for (int t = 0; t < 2; ++t) {
 				float16v a = zero16();
 #pragma unroll
-				for (int c = 0; c < 4; ++c) a = N2_MFMA(frag(F, M::WHT + (k - 1) * 8 + t * 4 + c, lane), dh[k][c], a);
-				mask_pack(a, h[k - 1][2 * t], h[k - 1][2 * t + 1], dh[k - 1][2 * t], dh[k - 1][2 * t + 1]);
+				for (int c = 0; c < 4; ++c) a = N2_MFMA(frag(F, M::WHT + t * 4 + c, lane), dh[1][c], a);
+				mask_pack(a, h[0][2 * t], h[0][2 * t + 1], dh[0][2 * t], dh[0][2 * t + 1]);
 			}
+		}
+		// ---- first matrix: dW_0 = dh_0 x^T: chunks dh_0 0..3 | x 4.. ----
+		stage_order();
+#pragma unroll
+		for (int c = 0; c < 4; ++c) stage_chained(st_ch + 4 * c * WG_QP, dh[0][c]);
+#pragma unroll
+		for (int c = 0; c < IC; ++c) stage_natural(st_nat + 4 * (4 + c) * WG_QP, x[c]);
+		stage_order();
+		uint4 sl[Tail::active ? 8 : 1];
+		if constexpr (Tail::active) {
+			// the slopes of this lane's 8 levels (level 4 (j / 2) + 2 g + j % 2)
+			const uint4* const at = reinterpret_cast<const uint4*>(tail.a.slopes) + (size_t)(4u * g < tail.a.enc_w ? 2u * g : 0u) * tail.a.n_src + col_src;
+#pragma unroll
+			for (int j = 0; j < 8; ++j) {
+				const uint32_t level = 4u * (j >> 1) + (j & 1);  // + 2 g
+				sl[j] = at[(size_t)(2u * (level + 2u * g) < tail.a.enc_w ? level : 0u) * tail.a.n_src];
+			}
+		}
+		const uint32_t next_col_src = load(next_col, next_src, g);
+		wgrad_tiles<0, 4, IC>(tr, 0, 4, acc);
+		if constexpr (SECOND) {
+			if (!valid) {
+#pragma unroll
+				for (int c = 0; c < IC; ++c) v[c] = zero8();
+			}
+			// a = m * (W_0 v),  b = m * (W_out^T g); m = the sign of the hidden layer.  dW_out += g a^T, dW_0 += b v^T
+			half8 s2[4];
+#pragma unroll
+			for (int t = 0; t < 2; ++t) {
+				float16v a = zero16();
+#pragma unroll
+				for (int c = 0; c < IC; ++c) a = N2_MFMA(frag(F, M::W0 + t * IC + c, lane), v[c], a);
+				mask_pack(a, h[0][2 * t], h[0][2 * t + 1], s2[2 * t], s2[2 * t + 1]);
+			}
+			half8 gg;
+			if (unit_row2 >= 0) {
+#pragma unroll
+				for (int e = 0; e < 8; ++e) gg[e] = (8 * g + e == unit_row2) ? (hf)1 : (hf)0;
+			} else {
+#pragma unroll
+				for (int e = 0; e < 8; ++e) gg[e] = G2[(size_t)(8 * g + e) * N + col];
+			}
+			if (!valid) gg = zero8();
+			stage_order();
+			stage_natural(st_nat, gg);
+#pragma unroll
+			for (int c = 0; c < 4; ++c) stage_chained(st_ch + 4 * (1 + c) * WG_QP, s2[c]);
+			stage_order();
+			wgrad_tiles<T::WO, 1, 4>(tr, 0, 1, acc);
+#pragma unroll
+			for (int t = 0; t < 2; ++t)
+				mask_pack(N2_MFMA(frag(F, M::WOT + t, lane), gg, zero16()), h[0][2 * t], h[0][2 * t + 1], s2[2 * t], s2[2 * t + 1]);
+			stage_order();
+#pragma unroll
+			for (int c = 0; c < 4; ++c) stage_chained(st_ch + 4 * c * WG_QP, s2[c]);
+#pragma unroll
+			for (int c = 0; c < IC; ++c) stage_natural(st_nat + 4 * (4 + c) * WG_QP, v[c]);
+			stage_order();
+			wgrad_tiles<0, 4, IC>(tr, 0, 4, acc);
+		}
+		stage_order();
+		half4v out_lo, out_hi;
 		hf dn[2] = {(hf)0, (hf)0};  // tail: g = 0: row 35; g = 1: rows 36, 37 of dL/dinput
 		if (WANT_DX != WG_DX_NONE) {
 #pragma unroll
@@ -186,101 +341,26 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __res
 					if (t == 1) { dn[0] = (hf)(g == 0 ? d[3] : d[0]); dn[1] = (hf)d[1]; }
 					// rows 0..15 go out sample-major (16 values per column, the SDF net's output gradient): the lane holds
 					// rows 4 g .. 4 g + 3 and 8 + 4 g .. 8 + 4 g + 3; rows 35..37 stay in registers (dn)
-					if (t == 0 && valid) {
-						const half4v lo = {(hf)d[0], (hf)d[1], (hf)d[2], (hf)d[3]}, hi = {(hf)d[4], (hf)d[5], (hf)d[6], (hf)d[7]};
-						hf* o = dX + (size_t)col * MLP_OUT + 4 * g;
-						*reinterpret_cast<half4v*>(o) = lo;
-						*reinterpret_cast<half4v*>(o + 8) = hi;
+					if (t == 0) {
+						out_lo = half4v{(hf)d[0], (hf)d[1], (hf)d[2], (hf)d[3]};
+						out_hi = half4v{(hf)d[4], (hf)d[5], (hf)d[6], (hf)d[7]};
 					}
 				}
+				if (t == 0 && !Tail::active && more) arrived();
 				if (!Tail::active && valid) {
 #pragma unroll
 					for (int r = 0; r < 16; ++r) {
 						const int row = 32 * t + 8 * (r >> 2) + (r & 3);  // + 4 g
 						const bool lo = wg_dx_row(WANT_DX, row, IN_W), hi = wg_dx_row(WANT_DX, row + 4, IN_W);
-						if (lo && hi) dX[(size_t)(row + 4 * g) * N + col] = (hf)d[r];
-						else if (lo) { if (g == 0) dX[(size_t)row * N + col] = (hf)d[r]; }
-						else if (hi) { if (g == 1) dX[(size_t)(row + 4) * N + col] = (hf)d[r]; }
+						// (row + 4 g; a uniform base and the lane's offset, whose 64-bit sums would be kept for all rows from round to round)
+						hf* const o = reinterpret_cast<hf*>(reinterpret_cast<char*>(dX + (size_t)row * N) + off4);
+						if (lo && hi) *o = (hf)d[r];
+						else if (lo) { if (g == 0) *o = (hf)d[r]; }
+						else if (hi) { if (g == 1) *o = (hf)d[r]; }
 					}
 				}
 			}
 		}
-		half8 v[IC], gg, sa[4], sb[4];
-		if constexpr (SECOND) {
-			load_tile_rows<IC>(V, N, col, g, v);
-			if (unit_row2 >= 0) {
-#pragma unroll
-				for (int e = 0; e < 8; ++e) gg[e] = (8 * g + e == unit_row2) ? (hf)1 : (hf)0;
-			} else {
-#pragma unroll
-				for (int e = 0; e < 8; ++e) gg[e] = G2[(size_t)(8 * g + e) * N + col];
-			}
-			if (!valid) {
-				gg = zero8();
-#pragma unroll
-				for (int c = 0; c < IC; ++c) v[c] = zero8();
-			}
-			// a = m * (W_0 v),  b = m * (W_out^T g); m = the sign of the hidden layer
-#pragma unroll
-			for (int t = 0; t < 2; ++t) {
-				float16v a = zero16();
-#pragma unroll
-				for (int c = 0; c < IC; ++c) a = N2_MFMA(frag(F, M::W0 + t * IC + c, lane), v[c], a);
-				mask_pack(a, h[0][2 * t], h[0][2 * t + 1], sa[2 * t], sa[2 * t + 1]);
-				mask_pack(N2_MFMA(frag(F, M::WOT + t, lane), gg, zero16()), h[0][2 * t], h[0][2 * t + 1], sb[2 * t], sb[2 * t + 1]);
-			}
-		}
-		// ---- stage 1: dW_out = dy h_last^T (+ g a^T) ----
-		// quads: dy 0..3 | h_last 4..19 | g 20..23 | a 24..39
-		stage_natural(st_nat, dy);
-#pragma unroll
-		for (int c = 0; c < 4; ++c) stage_chained(st_ch + (4 + 4 * c) * WG_QP, h[NH - 1][c]);
-		if constexpr (SECOND) {
-			stage_natural(st_nat + 20 * WG_QP, gg);
-#pragma unroll
-			for (int c = 0; c < 4; ++c) stage_chained(st_ch + (24 + 4 * c) * WG_QP, sa[c]);
-		}
-		__syncthreads();
-		if constexpr (SECOND) {
-			// waves 0, 1: dy h^T; waves 2, 3: g a^T; column tile nt, all samples
-			if (mt == 0) wgrad_tile<8>(tr, 0, 4 + 8 * nt, 0, gWo);
-			else wgrad_tile<8>(tr, 20, 24 + 8 * nt, 0, gWo);
-		} else {
-			// column tile nt, samples of half mt
-			wgrad_tile<4>(tr, 0, 4 + 8 * nt, 4 * mt, gWo);
-		}
-		__syncthreads();
-		// ---- hidden matrices: dW_k = dh_k h_{k-1}^T ----
-#pragma unroll
-		for (int k = NH - 1; k >= 1; --k) {
-#pragma unroll
-			for (int c = 0; c < 4; ++c) {
-				stage_chained(st_ch + (4 * c) * WG_QP, dh[k][c]);
-				stage_chained(st_ch + (16 + 4 * c) * WG_QP, h[k - 1][c]);
-			}
-			__syncthreads();
-			wgrad_tile<8>(tr, 8 * mt, 16 + 8 * nt, 0, gWh);
-			__syncthreads();
-		}
-		// ---- first matrix: dW_0 = dh_0 x^T (+ b v^T) ----
-		// quads: dh_0 (b) 0..15 | x (v) 16..16+4 IC-1; a column tile that the input does not fill reads what lies behind
-		// (stale values of an earlier stage), which only reaches accumulator columns that are never written out
-#pragma unroll
-		for (int c = 0; c < 4; ++c) stage_chained(st_ch + (4 * c) * WG_QP, dh[0][c]);
-#pragma unroll
-		for (int c = 0; c < IC; ++c) stage_natural(st_nat + (16 + 4 * c) * WG_QP, x[c]);
-		uint4 sl[Tail::active ? 8 : 1];
-		if constexpr (Tail::active) {
-			// the slopes of this lane's 8 levels (level 4 (j / 2) + 2 g + j % 2), in flight during the last products
-#pragma unroll
-			for (int j = 0; j < 8; ++j) {
-				const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
-				sl[j] = reinterpret_cast<const uint4*>(tail.a.slopes)[(size_t)(2u * level < tail.a.enc_w ? level : 0u) * tail.a.n_src + col_src];
-			}
-		}
-		__syncthreads();
-		if (nt < IN_MT) wgrad_tile<8>(tr, 8 * mt, 16 + 8 * nt, 0, gW0);
-		__syncthreads();
 		if constexpr (Tail::active) {
 			// dL/dnormal = row 35..37 of dL/dinput + rows 4..6 of dL/doutput / ek_batch + rows 8..10 of dL/doutput; its pieces
 			// sit in the two halves of the wave: g = 0 holds dn[0] and rows 4..6, g = 1 holds dn[0..1] (rows 36, 37) and rows 8..10
@@ -293,6 +373,9 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __res
 			const uint32_t o0 = (uint32_t)__shfl_xor((int)m0, 32), o1 = (uint32_t)__shfl_xor((int)m1, 32), o2 = (uint32_t)__shfl_xor((int)m2, 32);
 			const uint32_t a0 = g == 0 ? m0 : o0, a1 = g == 0 ? m1 : o1;             // what the lower half holds
 			const uint32_t b0 = g == 0 ? o0 : m0, b1 = g == 0 ? o1 : m1, b2 = g == 0 ? o2 : m2;  // what the upper half holds
+#pragma unroll
+			for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(sl[j].x), "+v"(sl[j].y), "+v"(sl[j].z), "+v"(sl[j].w));
+			if (more) arrived();
 			float vv[3] = {lo16(a0), lo16(b0), hi16(b0)};
 			const float r4[3] = {hi16(a0), lo16(a1), hi16(a1)}, r8[3] = {lo16(b1), hi16(b1), lo16(b2)};
 #pragma unroll
@@ -301,6 +384,9 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __res
 				vv[d] += r8[d];
 			}
 			if (valid) {
+				hf* const o = dX + (size_t)col * MLP_OUT + 4 * g;
+				*reinterpret_cast<half4v*>(o) = out_lo;
+				*reinterpret_cast<half4v*>(o + 8) = out_hi;
 				if (g == 0) {
 					var_acc += (float)dy_all[7];
 #pragma unroll
@@ -312,67 +398,62 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) mlp_wgrad_kernel(const hf* __res
 				// rows 3.. of the SDF net's second-order input: the encoding's dL_ddLdoutput = J v
 #pragma unroll
 				for (int j = 0; j < 8; ++j) {
-					const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
-					if (2u * level < tail.a.enc_w) {
-						float m[6];
-						const float unit = n2_slopes_unpack(sl[j], m) * tail.a.scale[level];
-						hf* o = reinterpret_cast<hf*>(tail.a.d_density_in) + (size_t)(3 + 2 * level) * N + col;
-						o[0] = (hf)((m[0] * vv[0] + m[1] * vv[1] + m[2] * vv[2]) * unit);
-						o[N] = (hf)((m[3] * vv[0] + m[4] * vv[1] + m[5] * vv[2]) * unit);
+					const uint32_t level = 4u * (j >> 1) + (j & 1);  // + 2 g
+					float m[6];
+					float scale0 = tail.a.scale[level], scale2 = tail.a.scale[level + 2u];
+					asm("" : "+s"(scale0), "+s"(scale2));  // (the compiler would choose the address and load per lane)
+					const float unit = n2_slopes_unpack(sl[j], m) * (g == 0 ? scale0 : scale2);
+					hf f0 = (hf)((m[0] * vv[0] + m[1] * vv[1] + m[2] * vv[2]) * unit), f1 = (hf)((m[3] * vv[0] + m[4] * vv[1] + m[5] * vv[2]) * unit);
+					asm volatile("" : "+v"(f0), "+v"(f1));  // (formed outside the condition, which then takes no branch)
+					char* const rows = reinterpret_cast<char*>(reinterpret_cast<hf*>(tail.a.d_density_in) + (size_t)(3 + 2 * level) * N);
+					if (2u * (level + 2u * g) < tail.a.enc_w) {
+						*reinterpret_cast<hf*>(rows + off4) = f0;
+						*reinterpret_cast<hf*>(rows + 2 * (size_t)N + off4) = f1;
 					}
 				}
 			}
 		}
-		if constexpr (SECOND) {
-#pragma unroll
-			for (int c = 0; c < 4; ++c) stage_chained(st_ch + (4 * c) * WG_QP, sb[c]);
-#pragma unroll
-			for (int c = 0; c < IC; ++c) stage_natural(st_nat + (16 + 4 * c) * WG_QP, v[c]);
-			__syncthreads();
-			if (nt < IN_MT) wgrad_tile<8>(tr, 8 * mt, 16 + 8 * nt, 0, gW0);
-			__syncthreads();
-		}
+		col_src = next_col_src;
 	}
-	// ---- the workgroup's slab: an fp32 image of the parameters in LDS, summed over the waves that share a tile ----
-	float* Wl = reinterpret_cast<float*>(smem);
-	__syncthreads();  // every wave is done with the fragments the image overlays
-	if (nt < IN_MT) {
-#pragma unroll
-		for (int r = 0; r < 16; ++r)
-			if (32 * nt + n < IN_W) Wl[(32 * mt + drow(r, g)) * IN_W + 32 * nt + n] = gW0[r] * gain_inv;
-	}
-	if (NH > 1) {
-#pragma unroll
-		for (int r = 0; r < 16; ++r) Wl[MLP_WIDTH * IN_W + (32 * mt + drow(r, g)) * MLP_WIDTH + 32 * nt + n] = gWh[r] * gain_inv;
-	}
-	constexpr int OFF_O = MLP_WIDTH * IN_W + (NH - 1) * MLP_WIDTH * MLP_WIDTH;
-	if (mt == 0) {
-#pragma unroll
-		for (int r = 0; r < 16; ++r)
-			if (drow(r, g) < MLP_OUT) Wl[OFF_O + drow(r, g) * MLP_WIDTH + 32 * nt + n] = gWo[r] * gain_inv;
-	}
-	__syncthreads();
-	if (mt == 1) {
-#pragma unroll
-		for (int r = 0; r < 16; ++r)
-			if (drow(r, g) < MLP_OUT) Wl[OFF_O + drow(r, g) * MLP_WIDTH + 32 * nt + n] += gWo[r] * gain_inv;
-	}
-	__syncthreads();
-	float* slab = partials + (size_t)blockIdx.x * N_PARAMS;
-	for (int i = threadIdx.x; i < N_PARAMS; i += MLP_BLOCK) slab[i] = Wl[i];
+	// ---- the workgroup's slab: the sum over its waves, a share of the tiles by each ----
+	constexpr int OFF_H = MLP_WIDTH * IN_W, OFF_O = OFF_H + (NH - 1) * MLP_WIDTH * MLP_WIDTH;
+	float4v* const Wl = reinterpret_cast<float4v*>(smem);
+	float* const slab = partials + (size_t)blockIdx.x * N_PARAMS;
+	const int w_fold = __builtin_amdgcn_readfirstlane(wave), t_fold = w_fold & 3, row = 4 * (lane >> 4), col = lane & 15;
+	float* const at_0 = slab + (16 * t_fold + row) * IN_W + col;
+	float* const at_h = slab + OFF_H + (16 * t_fold + row) * MLP_WIDTH + col;
+	float* const at_o = slab + OFF_O + row * MLP_WIDTH + 16 * t_fold + col;
+	float* const var = reinterpret_cast<float*>(smem + WAVES * Fold::PER * 4096);
 	if constexpr (Tail::active) {
 		// the workgroup's part of the variance gradient (row 7 of dL/doutput), summed in a fixed order
 #pragma unroll
 		for (int o = 32; o > 0; o >>= 1) var_acc += __shfl_xor(var_acc, o);
-		__syncthreads();
-		if (lane == 0) Wl[wave] = var_acc;
-		__syncthreads();
-		if (threadIdx.x == 0) tail.a.var_part[blockIdx.x] = (Wl[0] + Wl[1]) + (Wl[2] + Wl[3]);
 	}
-}
-
-// dynamic LDS of the kernel: fragments, then the staging buffer (40 quad rows with the second-order pass, else 32)
-template <int IC, int NH, bool SECOND>
-constexpr size_t mlp_wgrad_lds() {
-	return (size_t)FragMap<IC, NH>::SEL * 1024 + (size_t)(SECOND ? 40 : 32) * WG_QP;
+#pragma unroll
+	for (int c0 = 0; c0 < Fold::COLS; c0 += Fold::PER) {
+		__syncthreads();  // every wave is done with the fragments and staging buffers, or the tiles, that these overlay
+#pragma unroll
+		for (int c = c0; c < c0 + Fold::PER && c < Fold::COLS; ++c)
+#pragma unroll
+			for (int t = 0; t < 4; ++t) Wl[((wave * Fold::PER + c - c0) * 4 + t) * 64 + lane] = acc[Fold::tile(c, t)];
+		if (Tail::active && c0 == 0 && lane == 0) var[wave] = var_acc;
+		__syncthreads();
+#pragma unroll
+		for (int c = c0; c < c0 + Fold::PER && c < Fold::COLS; ++c) {
+			if (WAVES == 8 && (c & 1) != (w_fold >> 2)) continue;
+			const float4v* const tiles = Wl + ((c - c0) * 4 + t_fold) * 64 + lane;
+			float4v s = tiles[0];
+#pragma unroll
+			for (int w = 1; w < WAVES; ++w) s += tiles[w * Fold::PER * 256];
+			float* const o = c < IC ? at_0 + 16 * c : c < Fold::COLS - 1 ? at_h + 16 * (c - IC) : at_o;
+#pragma unroll
+			for (int r = 0; r < 4; ++r) o[r * (c < IC ? IN_W : MLP_WIDTH)] = s[r] * gain_inv;
+		}
+		if constexpr (Tail::active) if (c0 == 0 && threadIdx.x == 0) {
+			float sum = var[0];
+#pragma unroll
+			for (int w = 1; w < WAVES; ++w) sum += var[w];
+			tail.a.var_part[blockIdx.x] = sum;
+		}
+	}
 }

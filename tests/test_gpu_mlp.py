@@ -319,6 +319,32 @@ def test_backward_and_second_order_equals_the_two_calls(oracle, in_w, unit):
     assert_grad_close(host(dG), base + ref1 + ref2, what="accumulated first + second order weight gradients")
 
 
+@pytest.mark.parametrize("in_w,n_hidden,second", [(48, 2, False), (48, 1, True), (64, 2, False), (16, 1, True)])
+@pytest.mark.parametrize("n", [32768, 32776, 65536 + 264, 131072 + 40])  # workgroups of four waves, of eight, a second and a third round that is not full
+def test_large_batches_equal_the_sum_of_small_ones(oracle, in_w, n_hidden, second, n):
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, LAYOUT_AOS, LAYOUT_SOA
+    _, gm, _, _, dG, _ = make(oracle, in_w, n_hidden, 41)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x, dy, v = (torch.randn((w, n), device="cuda", generator=gen).half() for w in (in_w, 16, in_w))
+
+    def call(a, b, layout):
+        xs, dys = x[:, a:b].contiguous(), dy[:, a:b].contiguous()
+        dys = dys.t().contiguous() if layout == LAYOUT_AOS else dys
+        dG.fill_(3.0)
+        if second:
+            dx = gm.backward_and_second_order(xs, dys, v[:, a:b].contiguous(), None, dL_layout=layout, mode=GRAD_OVERWRITE)
+        else:
+            dx = gm.backward(xs, dys, layout, want_input_grad=True, mode=GRAD_OVERWRITE)
+        return dx, dG.double()
+    parts = [call(a, min(a + 4096, n), LAYOUT_SOA) for a in range(0, n, 4096)]
+    want_dx, want = torch.cat([p[0] for p in parts], 1), sum(p[1] for p in parts)
+    for layout in (LAYOUT_SOA, LAYOUT_AOS):
+        dx, got = call(0, n, layout)
+        assert torch.equal(dx, want_dx)
+        # every part and the whole are rounded to fp16 once: 2^-11 of an entry each, the parts' errors independent of each other
+        assert float((got - want).norm() / want.norm()) < 2 ** -10
+
+
 def test_backward_and_second_order_errors(oracle):
     from neus2_amd.tcnn_api import GRAD_IGNORE, FullyFusedMLP, N2Error
     om, gm, W, dW, dG, rng = make(oracle, 48, 1, 32)
