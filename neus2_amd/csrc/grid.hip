@@ -455,15 +455,38 @@ struct N2BucketPlan {
 	uint8_t run_lanes[N2_MAX_LEVELS];
 };
 
+// what a point brings along: its position, dL/dy of the level's two features, g2 of them and v
+struct N2BinInput {
+	float p[3], v[3];
+	__half dy[2], g2[2];
+};
+template <bool FIRST, bool SECOND>
+__device__ __forceinline__ N2BinInput grid_bin_load(uint32_t level, uint32_t i, uint32_t N, const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
+                                                    const __half* __restrict__ dL_dy, const float* __restrict__ v, const __half* __restrict__ g2, uint32_t xi, uint32_t Ng) {
+	N2BinInput in;
+	const float* q = xyz + (size_t)xi * point_stride;
+	const size_t row = (size_t)level * 2;
+#pragma unroll
+	for (int d = 0; d < 3; ++d) in.p[d] = q[(size_t)d * dim_stride];
+#pragma unroll
+	for (int f = 0; f < 2; ++f) {
+		if (FIRST) in.dy[f] = dL_dy[(row + f) * N + i];
+		if (SECOND) in.g2[f] = g2[(row + f) * Ng + xi];
+	}
+#pragma unroll
+	for (int d = 0; d < 3; ++d)
+		if (SECOND) in.v[d] = v[(size_t)d * N + i];
+	return in;
+}
+
 template <uint32_t MODE, bool FIRST, bool SECOND, bool WANT_OUT, bool CLAMP_X>
-__device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t N,
-                                               const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
-                                               const __half* __restrict__ dL_dy, const float* __restrict__ v,
-                                               const __half* __restrict__ g2, const __half2* __restrict__ params,
-                                               __half* __restrict__ dL_ddLdy, uint32_t* e_out, float* r0_out, float* r1_out,
-                                               uint32_t* cell, uint32_t xi, uint32_t Ng) {
+__device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t N, const N2BinInput& in,
+                                               const __half2* __restrict__ params, __half* __restrict__ dL_ddLdy, uint32_t* e_out, float* r0_out, float* r1_out,
+                                               uint32_t* cell) {
 	const float scale = tab.scale[level];
-	N2Point p = n2_load_point(xyz, point_stride, dim_stride, xi, scale);
+	N2Point p;
+#pragma unroll
+	for (int d = 0; d < 3; ++d) n2_locate(in.p[d], scale, p.w[d], p.c[d]);
 	if (CLAMP_X) p.c[0] = min(p.c[0], PAIR_MAX_CELL);  // pair records: x + 1 stays inside the bucket's index bits
 	cell[0] = p.c[0]; cell[1] = p.c[1]; cell[2] = p.c[2];
 	uint32_t e[8];
@@ -471,13 +494,13 @@ __device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t
 	const size_t row = (size_t)level * 2;
 	float a0 = 0.f, a1 = 0.f, c0 = 0.f, c1 = 0.f, v0 = 0.f, v1 = 0.f, v2 = 0.f;
 	if (FIRST) {
-		a0 = __half2float(dL_dy[row * N + i]);
-		a1 = __half2float(dL_dy[(row + 1) * N + i]);
+		a0 = __half2float(in.dy[0]);
+		a1 = __half2float(in.dy[1]);
 	}
 	if (SECOND) {
-		c0 = __half2float(g2[row * Ng + xi]);
-		c1 = __half2float(g2[(row + 1) * Ng + xi]);
-		v0 = v[i] * scale; v1 = v[(size_t)N + i] * scale; v2 = v[(size_t)2 * N + i] * scale;
+		c0 = __half2float(in.g2[0]);
+		c1 = __half2float(in.g2[1]);
+		v0 = in.v[0] * scale; v1 = in.v[1] * scale; v2 = in.v[2] * scale;
 	}
 	const __half2* P = params + tab.offset[level];
 	float o0 = 0.f, o1 = 0.f;
@@ -533,10 +556,27 @@ __device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t
 constexpr uint32_t MERGE_MAX_HEADS = 52;  // measured on the training step: 16: +16 us for the scatter pair, 24: +6, 32: +1, 40: +2 against 48 .. 58
 constexpr unsigned long long ROW_HEADS = 0x0001000100010001ull;  // first lane of each 16-lane row
 
-// value of the lane D places below in the same 16-lane row (0 if that leaves the row)
+// r += take * (r of the lane D places below in the same 16-lane row; 0 if that leaves the row), for the sixteen values of a point.
+// (Written out: the compiler makes a move with the lane shift, a wait state and a multiply-add of each.  s_nop: a lane shift must not
+// read what one of the two instructions before it wrote.)
 template <int D>
-__device__ __forceinline__ float n2_row_shr(float x) {
-	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x110 + D, 0xf, 0xf, true));  // lanes without a source read 0
+__device__ __forceinline__ void n2_row_add(float (&a)[8], float (&b)[8], const float take) {
+#define N2_ROW_ADD(K) "v_fmac_f32_dpp %" #K ", %" #K ", %16 row_shr:%17 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+	asm("s_nop 1\n\t" N2_ROW_ADD(0) N2_ROW_ADD(1) N2_ROW_ADD(2) N2_ROW_ADD(3) N2_ROW_ADD(4) N2_ROW_ADD(5) N2_ROW_ADD(6) N2_ROW_ADD(7)
+	    N2_ROW_ADD(8) N2_ROW_ADD(9) N2_ROW_ADD(10) N2_ROW_ADD(11) N2_ROW_ADD(12) N2_ROW_ADD(13) N2_ROW_ADD(14) N2_ROW_ADD(15) "s_nop 0"
+	    : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),
+	      "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4]), "+v"(b[5]), "+v"(b[6]), "+v"(b[7]) : "v"(take), "n"(D));
+#undef N2_ROW_ADD
+}
+// sum over the lanes up to this one (all 64 lanes active): lane shifts inside the rows of 16, then the rows' totals
+__device__ __forceinline__ uint32_t n2_wave_prefix(uint32_t x) {
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // a row's last lane to the next row, rows 1 and 3
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2 and 3
+	return x;
 }
 constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 
@@ -548,6 +588,10 @@ constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 // stores here, half the key traffic and decoding in the reduce kernel.  Points outside the unit cube could carry an x
 // beyond that range: their cell is clamped for the records (the dense levels clamp such points too).
 
+// What a workgroup takes is its chain of waits (three share a CU, and the vector units are busy two thirds of the time): loads, counter
+// updates and prefix look-ups are therefore issued together, and nothing waits in a branch.  With each of them awaited where it was used,
+// and the second point's loads behind the first one's counters: training step at 2^18 samples 57 us, now 48; 2^18 uniform points 47, now 43;
+// 52344 samples 15.2, now 12.6.
 template <bool FIRST, bool SECOND, bool WANT_OUT, bool PAIR>
 __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uint32_t level, const uint32_t tile, uint32_t N, uint32_t tiles,
                                               const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
@@ -561,9 +605,28 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	const uint32_t shift = PAIR ? BKT_SHIFT : (uint32_t)tab.bucket_shift[level], in_bucket = (1u << shift) - 1u;
 	// records of this thread: entry | rank << 19 after the counting step (REC_SKIP: merged into a later lane)
 	uint32_t re[BIN_PER_THREAD * R], rv[BIN_PER_THREAD * 8], tcode[BIN_PER_THREAD];
+	// The second point's inputs are under way while the first one's records are merged and counted, the index it reads some of them by before
+	// that.  (The
+	// position and g2's columns may be read through an index: n2_grid_backward_fused_indexed.)
+	const uint32_t Ng = index ? n_cols : N;
+	uint32_t src[BIN_PER_THREAD];
+#pragma unroll
+	for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) src[j] = min(tile * BIN_POINTS + j * BIN_BLOCK + threadIdx.x, N - 1u);
+	if (index) {
+#pragma unroll
+		for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) src[j] = index[src[j]];
+#pragma unroll
+		for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) src[j] = min(src[j], n_cols - 1u);
+	}
+	auto load = [&](uint32_t j) __attribute__((always_inline)) {
+		const uint32_t i = min(tile * BIN_POINTS + j * BIN_BLOCK + threadIdx.x, N - 1u);
+		return grid_bin_load<FIRST, SECOND>(level, i, N, xyz, point_stride, dim_stride, dL_dy, v, g2, src[j], Ng);
+	};
+	N2BinInput next = load(0);
 #pragma unroll
 	for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) {
 		const uint32_t i = tile * BIN_POINTS + j * BIN_BLOCK + threadIdx.x;
+		const N2BinInput in = next;
 		bool valid = i < N;
 		if (valid && n2_level_masked(tab, level, i)) {  // a switched-off level: no records, zero second-order output
 			valid = false;
@@ -577,16 +640,15 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 #pragma unroll
 		for (uint32_t k = 0; k < 8; ++k) { e[k] = 0; r0[k] = 0.f; r1[k] = 0.f; }
 		if (valid) {
-			// positions and g2 columns may be read through an index (see n2_grid_backward_fused_indexed)
-			const uint32_t xi = index ? min(index[i], n_cols - 1u) : i, Ng = index ? n_cols : N;
 			if (PAIR) {
-				grid_bin_point<N2_LEVEL_HASH, FIRST, SECOND, WANT_OUT, true>(tab, level, i, N, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, e, r0, r1, cell, xi, Ng);
+				grid_bin_point<N2_LEVEL_HASH, FIRST, SECOND, WANT_OUT, true>(tab, level, i, N, in, params, dL_ddLdy, e, r0, r1, cell);
 			} else {
-#define CALL(M) grid_bin_point<M, FIRST, SECOND, WANT_OUT, false>(tab, level, i, N, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, e, r0, r1, cell, xi, Ng)
+#define CALL(M) grid_bin_point<M, FIRST, SECOND, WANT_OUT, false>(tab, level, i, N, in, params, dL_ddLdy, e, r0, r1, cell)
 				N2_DISPATCH_MODE(tab.mode[level], CALL)
 #undef CALL
 			}
 		}
+		if (j + 1 < BIN_PER_THREAD) next = load(j + 1);
 		// runs of equal cells among the wave's 64 consecutive points
 		const uint32_t up_x = __shfl_up(cell[0], 1), up_y = __shfl_up(cell[1], 1), up_z = __shfl_up(cell[2], 1);
 		const int up_valid = __shfl_up((int)valid, 1);
@@ -598,30 +660,26 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 			const uint32_t start = 63u - (uint32_t)__clzll(heads & (~0ull >> (63u - lane)));
 			emit = valid && (lane == 63u || ((heads >> (lane + 1u)) & 1ull));
 			const uint32_t depth = lane - start;  // lanes of the run below this one
-#define N2_SCAN_STEP(D)                                               \
-			{                                                         \
-				const float take = depth >= D ? 1.f : 0.f;            \
-				_Pragma("unroll") for (uint32_t k = 0; k < 8; ++k) {  \
-					r0[k] = fmaf(n2_row_shr<D>(r0[k]), take, r0[k]);  \
-					r1[k] = fmaf(n2_row_shr<D>(r1[k]), take, r1[k]);  \
-				}                                                     \
-			}
-			N2_SCAN_STEP(1) N2_SCAN_STEP(2) N2_SCAN_STEP(4) N2_SCAN_STEP(8)
-#undef N2_SCAN_STEP
+			// (a step that no run of the wave is long enough for adds nothing)
+			n2_row_add<1>(r0, r1, depth >= 1u ? 1.f : 0.f);
+			if (__ballot(depth >= 2u)) n2_row_add<2>(r0, r1, depth >= 2u ? 1.f : 0.f);
+			if (__ballot(depth >= 4u)) n2_row_add<4>(r0, r1, depth >= 4u ? 1.f : 0.f);
+			if (__ballot(depth >= 8u)) n2_row_add<8>(r0, r1, depth >= 8u ? 1.f : 0.f);
 		}
 		if (PAIR) tcode[j] = ((uint32_t)__popc((e[0] ^ e[1]) & (BKT_ENTRIES - 1u)) - 1u) << BKT_SHIFT;
 #pragma unroll
 		for (uint32_t k = 0; k < 8; ++k) {
-			if (!PAIR || (k & 1u) == 0) {
-				uint32_t rec = REC_SKIP;
-				if (emit) {
-					const uint32_t rank = atomicAdd(&hist[e[k] >> shift], 1u);
-					rec = e[k] | (rank << 19);
-				}
-				re[R * j + (PAIR ? k >> 1 : k)] = rec;
-			}
 			const __half2 h = __floats2half2_rn(r0[k], r1[k]);
 			rv[8 * j + k] = *reinterpret_cast<const uint32_t*>(&h);
+		}
+#pragma unroll
+		for (uint32_t q = 0; q < R; ++q) re[R * j + q] = REC_SKIP;
+		if (emit) {
+			uint32_t rank[R];
+#pragma unroll
+			for (uint32_t q = 0; q < R; ++q) rank[q] = atomicAdd(&hist[e[PAIR ? 2 * q : q] >> shift], 1u);
+#pragma unroll
+			for (uint32_t q = 0; q < R; ++q) re[R * j + q] = e[PAIR ? 2 * q : q] | (rank[q] << 19);
 		}
 	}
 	__syncthreads();
@@ -631,11 +689,7 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 #pragma unroll
 		for (uint32_t q = 0; q < PER; ++q) { c[q] = hist[threadIdx.x * PER + q]; s += c[q]; }
 		const uint32_t own = s;
-#pragma unroll
-		for (int o = 1; o < 64; o <<= 1) {
-			const uint32_t u = __shfl_up(s, o);
-			if ((int)threadIdx.x >= o) s += u;
-		}
+		s = n2_wave_prefix(s);
 		uint32_t run = s - own;
 #pragma unroll
 		for (uint32_t q = 0; q < PER; ++q) { prefix[threadIdx.x * PER + q] = run; run += c[q]; }
@@ -644,18 +698,19 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	__syncthreads();
 #pragma unroll
 	for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) {
+		if (re[R * j] == REC_SKIP) continue;  // (a point's records go in together or not at all)
+		uint32_t pos[R];
+#pragma unroll
+		for (uint32_t k = 0; k < R; ++k) pos[k] = prefix[(re[R * j + k] & 0x7FFFFu) >> shift] + (re[R * j + k] >> 19);
 #pragma unroll
 		for (uint32_t k = 0; k < R; ++k) {
-			if (re[R * j + k] != REC_SKIP) {
-				const uint32_t e = re[R * j + k] & 0x7FFFFu, rank = re[R * j + k] >> 19;
-				const uint32_t pos = prefix[e >> shift] + rank;
-				if (PAIR) {
-					reinterpret_cast<uint2*>(stage_val)[pos] = make_uint2(rv[8 * j + 2 * k], rv[8 * j + 2 * k + 1]);
-					stage_key[pos] = (uint16_t)((e & (BKT_ENTRIES - 1u)) | tcode[j]);
-				} else {
-					stage_val[pos] = rv[8 * j + k];
-					stage_key[pos] = (uint16_t)(e & in_bucket);
-				}
+			const uint32_t e = re[R * j + k] & 0x7FFFFu;
+			if (PAIR) {
+				reinterpret_cast<uint2*>(stage_val)[pos[k]] = make_uint2(rv[8 * j + 2 * k], rv[8 * j + 2 * k + 1]);
+				stage_key[pos[k]] = (uint16_t)((e & (BKT_ENTRIES - 1u)) | tcode[j]);
+			} else {
+				stage_val[pos[k]] = rv[8 * j + k];
+				stage_key[pos[k]] = (uint16_t)(e & in_bucket);
 			}
 		}
 	}

@@ -378,6 +378,31 @@ def test_sorted_scatter_path(oracle, kind):
     assert (got[ref1 == 0] == 0).all()
 
 
+@pytest.mark.parametrize("run", [1, 2, 3, 5, 8, 9, 16, 40])  # around the steps of the sum over a run, and longer than a row of 16 lanes
+def test_sorted_scatter_merges_runs_of_one_length(oracle, run):
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
+    og = oracle.Grid(CFG["n_levels"], CFG["log2_hashmap_size"], CFG["base_resolution"], CFG["per_level_scale"])
+    gg = GridEncoding(**CFG)
+    rng = np.random.default_rng(run)
+    params = q16(rng.uniform(-1, 1, og.n_params))
+    dp = dev(params, torch.float16)
+    dg = torch.full_like(dp, 9.0)
+    gg.set_params(dp, dg)
+    n = 1500  # a second tile, and in it a second point of some threads
+    assert gg.reserve_scatter_workspace(n)
+    xyz = np.repeat(rng.random((3, (n + 4) // run + 1), dtype=np.float32), run, axis=1)[:, :n + 4][:, 4:].copy()  # (runs start off the rows)
+    dy, g2 = q16(rng.standard_normal((32, n))), q16(rng.standard_normal((32, n)) * 0.1)
+    v = (rng.standard_normal((3, n)) * 1e-3).astype(np.float32)
+    ref1, _ = og.backward(params, xyz, dy, want_dx=False)
+    ref, _, _ = og.backward_backward_input(params, xyz, v, g2, grad=ref1.copy(), want_dinput=False)
+    gg.backward(None, dev(xyz), dev(dy, torch.float16), mode=GRAD_OVERWRITE)
+    first = host(dg).copy()
+    gg.backward_fused(dev(xyz), dev(dy, torch.float16), dev(v), dev(g2, torch.float16), want_dL_ddLdy=False, mode=GRAD_OVERWRITE)
+    for l in range(16):
+        a, b = int(og.offset[l]) * 2, int(og.offset[l + 1]) * 2
+        assert rel_l2(first[a:b], ref1[a:b]) < RTOL and rel_l2(host(dg)[a:b], ref[a:b]) < RTOL, l
+
+
 def test_sorted_scatter_pair_records_edge_cells(oracle):
     """Hashed levels sort one record per pair of x-neighbour corners; the second corner's place in the bucket is the
     first one's xor 2^(t+1) - 1, t = trailing one bits of the cell's x.  Cells whose x ends in 0 .. 11 one bits (the
