@@ -806,16 +806,24 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2R
 	const size_t level_tile0 = (size_t)it.level * tiles;
 	const uint16_t* off = offsets + level_tile0 * (BKT_MAX + 1) + it.bucket;
 	const uint32_t step = groups * it.groups;  // (a split bucket's workgroup takes the tiles it.group, it.group + it.groups, ...)
-	// where the next step's records are; the bounds of the run behind it are on their way
-	uint32_t tile = group * it.groups + it.group, i = 0, end = 0, next_i = 0, next_end = 0;
-	if (tile < tiles) { i = off[(size_t)tile * (BKT_MAX + 1)] + r; end = off[(size_t)tile * (BKT_MAX + 1) + 1]; }
-	if (tile + step < tiles) { next_i = off[(size_t)(tile + step) * (BKT_MAX + 1)] + r; next_end = off[(size_t)(tile + step) * (BKT_MAX + 1) + 1]; }
+	// Where the next step's records are; the bounds of the run behind it are on their way, two 16-bit offsets as they lie in memory: taken apart
+	// where they are loaded, they were waited for there, and with them all records under way (2^18 samples: 51.6 -> 50.2 us, 2^18 uniform points 58 -> 55.5).
+	uint32_t tile = group * it.groups + it.group, i, end;
+	auto bounds = [&](uint32_t t) {
+		uint32_t two;
+		__builtin_memcpy(&two, off + (size_t)min(t, tiles - 1u) * (BKT_MAX + 1), sizeof(two));
+		return two;
+	};
+	const uint32_t first = bounds(tile);
+	i = (first & 0xFFFFu) + r;
+	end = tile < tiles ? first >> 16 : 0u;
 	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
 	struct Step {
 		value v[FLIGHT];
 		uint32_t key[FLIGHT], n;  // n: records of this lane that count
+		uint32_t next;            // bounds of the run behind the one the next step begins with
 	};
-	auto load = [&](Step& q) {
+	auto load = [&](Step& q, uint32_t& next) {
 		// (lanes without a record read the level's first one: every load is issued, so the compiler can wait for one step only)
 		const uint32_t left = i < end ? (end - i + lanes - 1u) >> run_lanes : 0u;
 		q.n = left < FLIGHT ? left : FLIGHT;
@@ -827,16 +835,14 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2R
 			if constexpr (PAIR) q.v[u] = reinterpret_cast<const uint2*>(rec_vals + slot)[at];
 			else q.v[u] = rec_vals[slot + at];
 		}
+		asm volatile("" : "+v"(next) : : "memory");  // (awaited behind the records' loads, not in front of them)
 		i += FLIGHT * lanes;
 		if (i - r >= end) {  // (the same for all lanes of the run) on to the next run
 			tile += step;
-			i = next_i;
-			end = next_end;
-			const uint32_t t = tile + step;
-			next_i = r;
-			next_end = 0;
-			if (t < tiles) { next_i = off[(size_t)t * (BKT_MAX + 1)] + r; next_end = off[(size_t)t * (BKT_MAX + 1) + 1]; }
+			i = (next & 0xFFFFu) + r;
+			end = tile < tiles ? next >> 16 : 0u;
 		}
+		q.next = bounds(tile + step);
 	};
 	auto add = [&](const Step& q) {
 #pragma unroll
@@ -857,20 +863,22 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2R
 		}
 	};
 	Step qa, qb;
+	qb.next = bounds(tile + step);
 	ulonglong2* a2 = reinterpret_cast<ulonglong2*>(acc);
 	for (uint32_t e = threadIdx.x; e < it.entries / 2; e += RED_BLOCK) {
 		a2[e] = make_ulonglong2(0ull, 0ull);
 		a2[BKT_ENTRIES / 2 + e] = make_ulonglong2(0ull, 0ull);
 	}
-	load(qa);
+	const bool any = __any(tile < tiles);  // (of a small batch's waves some have no tile)
+	if (any) load(qa, qb.next);
 	__syncthreads();
-	while (true) {
+	while (any) {
 		const bool last_b = tile >= tiles;
-		load(qb);
+		load(qb, qa.next);
 		add(qa);
 		if (last_b) break;
 		const bool last_a = tile >= tiles;
-		load(qa);
+		load(qa, qb.next);
 		add(qb);
 		if (last_a) break;
 	}
