@@ -127,12 +127,6 @@ __device__ __forceinline__ void build_fused_frags(hf* F, const FusedArgs& a, int
 	for (int idx = threadIdx.x; idx < count * 64; idx += FF_BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = fused_frag_value(a, idx >> 6, idx & 63);
 	__syncthreads();
 }
-// the same fragments copied from the image a gather launch left in global memory: 16 consecutive bytes per lane instead
-// of two-byte picks all over the weight matrices (5 to 7 us of a network launch went into those)
-__device__ __forceinline__ void load_fused_frags(hf* F, const hf* __restrict__ image, int count) {
-	for (int idx = threadIdx.x; idx < count * 64; idx += FF_BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = *reinterpret_cast<const half8*>(image + (size_t)idx * 8);
-	__syncthreads();
-}
 // Workgroups FRAG_BLOCKS .. of a gather launch (behind those that gather) write the image: the network kernel's fragments,
 // then those of the backward's weight-gradient kernels (colour net: FragMap<3, 2>; SDF net with 48 inputs: FragMap<3, 1>).
 constexpr uint32_t BWD_RGB_FRAGS = FragMap<3, 2>::SEL, BWD_SDF_FRAGS = FragMap<3, 1>::SEL;
@@ -556,7 +550,8 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 	unsigned char* const stage = smem + (size_t)(FULL ? FF_COUNT : FF_SDF_COUNT) * 1024 + FF_LEVELS * sizeof(uint4) + (threadIdx.x >> 6) * (32 * 2 * N2_RGB_IN_PITCH);
 	if (threadIdx.x < FF_LEVELS)
 		LV[threadIdx.x] = make_uint4(__float_as_uint(a.lv.scale[threadIdx.x]), a.lv.res[threadIdx.x], a.lv.entries[threadIdx.x], a.lv.offset[threadIdx.x]);
-	if (FULL && a.frags) load_fused_frags(F, a.frags, FF_COUNT);
+	// (a.frags: copied from the image a gather launch left in global memory, instead of two-byte picks all over the weight matrices: 5 to 7 us of a launch)
+	if (FULL && a.frags) load_frags<FF_COUNT, FF_BLOCK>(F, a.frags);
 	else build_fused_frags(F, a, FULL ? FF_COUNT : FF_SDF_COUNT);
 	const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
 	const uint32_t N = a.N, hash_mask = a.lv.hash_mask, active = a.lv.active_levels;

@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(MLP_BLOCK, 2) __attribute__((amdgpu_num_vgpr(1
 	constexpr int IN_W = 16 * IC, IN_MT = M::IN_MT;
 	extern __shared__ __align__(16) unsigned char smem[];
 	hf* F = reinterpret_cast<hf*>(smem);
-	build_frags<IC, NH>(F, W, M::SEL);
+	build_frags_staged<IC, NH>(F, F + M::SEL * 512, W, M::SEL);
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, g = lane >> 5;
 	const uint32_t n_tiles = (N + MLP_TILE - 1) / MLP_TILE;
 	const uint32_t slot = blockIdx.x * (MLP_BLOCK / 64) + wave, n_slots = gridDim.x * (MLP_BLOCK / 64);
@@ -651,7 +651,7 @@ static int mlp_backward_impl(n2_mlp_t* mlp, n2_stream_t stream, const n2_half* d
 	N2ProfScope prof(N2_PROF_MLP_BACKWARD, s);
 #define LAUNCH(IC, NH)                                                                                              \
 	do {                                                                                                            \
-		const size_t lds = frag_bytes(FragMap<IC, NH>::SEL);                                                        \
+		const size_t lds = frag_bytes(FragMap<IC, NH>::SEL) + sizeof(hf) * mlp_n_params<IC, NH>();                  \
 		if (int rc = allow_lds(mlp_backward_kernel<IC, NH>, lds)) return rc;                                        \
 		mlp_backward_kernel<IC, NH><<<dim3(blocks), dim3(MLP_BLOCK), lds, s>>>(mlp->params, X, n, dY, aos, unit_row, dX, nullptr, 0, x_index, x_cols); \
 	} while (0)
@@ -675,7 +675,7 @@ static int mlp_backward_impl(n2_mlp_t* mlp, n2_stream_t stream, const n2_half* d
 	}
 #define LAUNCH_Y(IC, NH)                                                                                            \
 	do {                                                                                                            \
-		const size_t lds = frag_bytes(FragMap<IC, NH>::SEL);                                                        \
+		const size_t lds = frag_bytes(FragMap<IC, NH>::SEL) + sizeof(hf) * mlp_n_params<IC, NH>();                  \
 		if (int rc = allow_lds(mlp_backward_kernel<IC, NH, true>, lds)) return rc;                                  \
 		mlp_backward_kernel<IC, NH, true><<<dim3(blocks), dim3(MLP_BLOCK), lds, s>>>(mlp->params, X, n, dY, aos, unit_row, dX, \
 			reinterpret_cast<hf*>(d_output), out_layout == N2_LAYOUT_AOS ? 1 : 0);                                  \

@@ -241,15 +241,37 @@ __device__ __forceinline__ half8 mlp_frag_value(const hf* __restrict__ W, int f,
 		return v;
 	}
 }
+// 16-byte pieces of global memory into LDS, PIECES of them by the BLOCK threads of a workgroup: all loads under way together.  (A loop that
+// stores each piece before it loads the next takes a trip to the L2 for each: 10 of them for 40 KiB by 256 threads.)
+template <int BLOCK, int PIECES>
+__device__ __forceinline__ void copy_to_lds(hf* to, const hf* __restrict__ from) {
+	constexpr int PER = (PIECES + BLOCK - 1) / BLOCK;
+	half8 v[PER];
+#pragma unroll
+	for (int k = 0; k < PER; ++k) v[k] = reinterpret_cast<const half8*>(from)[min((int)threadIdx.x + k * BLOCK, PIECES - 1)];
+#pragma unroll
+	for (int k = 0; k < PER; ++k)
+		if (PIECES % BLOCK == 0 || (int)threadIdx.x + k * BLOCK < PIECES) reinterpret_cast<half8*>(to)[threadIdx.x + k * BLOCK] = v[k];
+}
+template <int IC, int NH>
+constexpr int mlp_n_params() { return MLP_WIDTH * 16 * IC + (NH - 1) * MLP_WIDTH * MLP_WIDTH + MLP_OUT * MLP_WIDTH; }
 template <int IC, int NH, int BLOCK = MLP_BLOCK>
 __device__ __forceinline__ void build_frags(hf* F, const hf* __restrict__ W, int count) {
 	for (int idx = threadIdx.x; idx < count * 64; idx += BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = mlp_frag_value<IC, NH>(W, idx >> 6, idx & 63);
 	__syncthreads();
 }
-// the same fragments from an image that another launch has built in global memory (count KiB)
-template <int BLOCK = MLP_BLOCK>
-__device__ __forceinline__ void load_frags(hf* F, const hf* __restrict__ image, int count) {
-	for (int idx = threadIdx.x; idx < count * 64; idx += BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = *reinterpret_cast<const half8*>(image + (size_t)idx * 8);
+// the same by way of the weights themselves, copied to `raw` in LDS (mlp_n_params halves): their pieces are picked from all over the matrices
+template <int IC, int NH, int BLOCK = MLP_BLOCK>
+__device__ __forceinline__ void build_frags_staged(hf* F, hf* raw, const hf* __restrict__ W, int count) {
+	copy_to_lds<BLOCK, mlp_n_params<IC, NH>() / 8>(raw, W);
+	__syncthreads();
+	for (int idx = threadIdx.x; idx < count * 64; idx += BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = mlp_frag_value<IC, NH>(raw, idx >> 6, idx & 63);
+	__syncthreads();
+}
+// the same fragments from an image that another launch has built in global memory (COUNT KiB)
+template <int COUNT, int BLOCK>
+__device__ __forceinline__ void load_frags(hf* F, const hf* __restrict__ image) {
+	copy_to_lds<BLOCK, COUNT * 64>(F, image);
 	__syncthreads();
 }
 

@@ -156,7 +156,8 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES) mlp_wgrad_kernel(const 
 	using Fold = WgFold<WAVES, IC, NH>;
 	constexpr uint32_t ROUND = 32 * WAVES;  // samples of a workgroup's round
 	constexpr int IN_W = 16 * IC, IN_MT = M::IN_MT;
-	constexpr int N_PARAMS = MLP_WIDTH * IN_W + (NH - 1) * MLP_WIDTH * MLP_WIDTH + MLP_OUT * MLP_WIDTH;
+	constexpr int N_PARAMS = mlp_n_params<IC, NH>();
+	static_assert(2 * N_PARAMS <= WAVES * WG_STAGE, "the weights fit where the staging buffers are");
 	extern __shared__ __align__(16) unsigned char smem[];
 	hf* F = reinterpret_cast<hf*>(smem);
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31;
@@ -207,8 +208,8 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES) mlp_wgrad_kernel(const 
 	const uint32_t col0 = column(blockIdx.x);
 	uint32_t col_src = load(col0, index[col0], lane >> 5);
 	// (frag_image: the fragments as a launch in front of this one has left them in global memory, M::SEL KiB; null: built here)
-	if (frag_image) load_frags<64 * WAVES>(F, frag_image, M::SEL);
-	else build_frags<IC, NH, 64 * WAVES>(F, W, M::SEL);
+	if (frag_image) load_frags<M::SEL, 64 * WAVES>(F, frag_image);
+	else build_frags_staged<IC, NH, 64 * WAVES>(F, F + M::SEL * 512, W, M::SEL);
 	for (uint32_t round = blockIdx.x; round < n_rounds; round += gridDim.x) {
 		int g = lane >> 5;
 		asm volatile("" : "+v"(g));  // addresses that depend on it are formed anew in every round: kept, they take 40 registers
