@@ -29,13 +29,6 @@ struct Sample {
 
 __device__ __forceinline__ float logistic(float x) { return 1.f / (1.f + __expf(-x)); }
 
-__device__ __forceinline__ void load_out(const hf* __restrict__ net_out, size_t s, float* o) {
-	const half8 a = *reinterpret_cast<const half8*>(net_out + s * 16);
-	const half8 b = *reinterpret_cast<const half8*>(net_out + s * 16 + 8);
-#pragma unroll
-	for (int k = 0; k < 8; ++k) { o[k] = (float)a[k]; o[8 + k] = (float)b[k]; }
-}
-
 __device__ __forceinline__ Sample eval_sample(const float* o, hf var_h, float warped_dt, const float* dir, const CompParams& c) {
 	Sample s;
 	s.dt = warped_dt * (c.max_step - c.min_step) + c.min_step;
@@ -69,24 +62,44 @@ __device__ __forceinline__ float wave_sum(float v) {
 	v += dpp(v, std::integral_constant<int, 0xB1>());   // quad_perm [1, 0, 3, 2]
 	return v;
 }
-// exclusive product scan over the 64 lanes
-__device__ __forceinline__ float wave_excl_prod(float v, int lane) {
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const float u = __shfl_up(v, o);
-		if (lane >= o) v *= u;
-	}
-	const float e = __shfl_up(v, 1);
-	return lane == 0 ? 1.f : e;
+// x of the lane the data-parallel control names, `none` where there is no such lane or the lane's row is not in ROWS
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float lane_of(float none, float x) {
+	return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(none), __float_as_int(x), CTRL, ROWS, 0xF, false));
 }
-__device__ __forceinline__ float wave_incl_sum(float v, int lane) {
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const float u = __shfl_up(v, o);
-		if (lane >= o) v += u;
-	}
+// Scans over the 64 lanes: inside the rows of 16 by lane shifts, then a row's last lane on to the next row (rows 1 and 3), then lane 31's
+// on to rows 2 and 3.  (By the LDS crossbar every step was a trip of a hundred cycles: forward and backward 11.0 and 16.2 us for 5000 rays,
+// now 10.6 and 14.6, and 6.6 and 9.6 for 300, now 5.9 and 7.8.)
+template <class Op>
+__device__ __forceinline__ float wave_scan(float v, float none, Op op) {
+	v = op(v, lane_of<0x111>(none, v));
+	v = op(v, lane_of<0x112>(none, v));
+	v = op(v, lane_of<0x114>(none, v));
+	v = op(v, lane_of<0x118>(none, v));
+	v = op(v, lane_of<0x142, 0xA>(none, v));
+	v = op(v, lane_of<0x143, 0xC>(none, v));
 	return v;
 }
+// exclusive product scan
+__device__ __forceinline__ float wave_excl_prod(float v) {
+	return lane_of<0x138>(1.f, wave_scan(v, 1.f, [](float a, float b) { return a * b; }));  // (one lane on, across the rows)
+}
+__device__ __forceinline__ float wave_incl_sum(float v) {
+	return wave_scan(v, 0.f, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v) {
+	auto step = [&](auto ctrl, auto rows) { v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false); };
+	using std::integral_constant;
+	step(integral_constant<int, 0x111>(), integral_constant<int, 0xF>());
+	step(integral_constant<int, 0x112>(), integral_constant<int, 0xF>());
+	step(integral_constant<int, 0x114>(), integral_constant<int, 0xF>());
+	step(integral_constant<int, 0x118>(), integral_constant<int, 0xF>());
+	step(integral_constant<int, 0x142>(), integral_constant<int, 0xA>());
+	step(integral_constant<int, 0x143>(), integral_constant<int, 0xC>());
+	return v;
+}
+__device__ __forceinline__ uint32_t of_lane(uint32_t x, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)x, lane); }
+__device__ __forceinline__ float of_lane(float x, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane)); }
 
 // One sample's outputs as they stand in memory
 struct OutRow {
@@ -106,12 +119,7 @@ __device__ __forceinline__ void unit_dir(hf dx, hf dy, hf dz, float* dir) {
 	const float len = sqrtf(x * x + y * y + z * z);
 	dir[0] = x / len; dir[1] = y / len; dir[2] = z / len;
 }
-// direction of the ray: rows 8..10 of its first sample, unwarped and normalised
-__device__ __forceinline__ void ray_dir(const hf* __restrict__ net_out, size_t base, float* dir) {
-	const hf* o = net_out + base * 16;
-	unit_dir(o[8], o[9], o[10], dir);
-}
-// ... from the row that lane 0 holds
+// direction of the ray (rows 8..10 of its first sample, unwarped and normalised) from the row that lane 0 holds
 __device__ __forceinline__ void ray_dir_lane0(const OutRow& row, float* dir) {
 	typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 	typedef _Float16 half2c __attribute__((ext_vector_type(2)));
@@ -170,7 +178,7 @@ __global__ void __launch_bounds__(CB) composite_forward_kernel(CompParams c, uin
 				const Sample sm = eval_row(row, dt, dir, c);
 				alpha = sm.alpha; rgb[0] = sm.rgb[0]; rgb[1] = sm.rgb[1]; rgb[2] = sm.rgb[2];
 			}
-			const float Tb = T * wave_excl_prod(1.f - alpha, lane);
+			const float Tb = T * wave_excl_prod(1.f - alpha);
 			// samples are consumed while the transmittance before them is >= 1e-4
 			const unsigned long long stop = __ballot(!valid || Tb < T_EPS);
 			const int n_proc = stop ? (int)__ffsll((long long)stop) - 1 : 64;
@@ -182,7 +190,7 @@ __global__ void __launch_bounds__(CB) composite_forward_kernel(CompParams c, uin
 			r1 += wave_sum(in ? w * rgb[1] : 0.f);
 			r2 += wave_sum(in ? w * rgb[2] : 0.f);
 			kept += n_proc;
-			if (n_proc > 0) T = __shfl(Tb * (1.f - alpha), n_proc - 1);
+			if (n_proc > 0) T = of_lane(Tb * (1.f - alpha), n_proc - 1);
 			if (n_proc < 64) break;
 		}
 		if (kept == n) { r0 += T * c.bg[0]; r1 += T * c.bg[1]; r2 += T * c.bg[2]; }
@@ -224,14 +232,8 @@ __global__ void __launch_bounds__(OFFSETS_BLOCK) composite_offsets_kernel(uint32
 #pragma unroll
 		for (uint32_t u = 0; u < 16; ++u) before += v[u];
 	}
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
-	uint32_t incl = own;
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t up = __shfl_up(incl, o);
-		if ((int)lane >= o) incl += up;
-	}
+	before = wave_incl_sum(before);
+	const uint32_t incl = wave_incl_sum(own);
 	if (lane == 63u) { wave_before[wave] = before; wave_total[wave] = incl; }
 	__syncthreads();
 	uint32_t base = 0;
@@ -286,9 +288,9 @@ __global__ void __launch_bounds__(CB) composite_backward_kernel(CompParams c, ui
 			before += r0 + u * CB + threadIdx.x < blockIdx.x ? v[u] : 0u;
 		}
 	}
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) { before += __shfl_xor(before, o); all += __shfl_xor(all, o); }
-	if (lane == 0) { part[wave] = before; part_all[wave] = all; part_kept[wave] = kept; }
+	before = wave_incl_sum(before);
+	all = wave_incl_sum(all);
+	if (lane == 63) { part[wave] = before; part_all[wave] = all; part_kept[wave] = kept; }
 	// the first 64 samples
 	OutRow row{};
 	float ci[7] = {};
@@ -341,12 +343,12 @@ __global__ void __launch_bounds__(CB) composite_backward_kernel(CompParams c, ui
 		if (c0 > 0 && valid) load_sample(s);
 		if (valid) sm = eval_row(row, ci[3], dir, c);
 		const float alpha = valid ? sm.alpha : 0.f;
-		const float Tb = T * wave_excl_prod(1.f - alpha, lane);
+		const float Tb = T * wave_excl_prod(1.f - alpha);
 		const float w = valid ? alpha * Tb : 0.f;
 		const float Ta = Tb * (1.f - alpha);
-		const float q0 = p0 + wave_incl_sum(valid ? w * sm.rgb[0] : 0.f, lane);
-		const float q1 = p1 + wave_incl_sum(valid ? w * sm.rgb[1] : 0.f, lane);
-		const float q2 = p2 + wave_incl_sum(valid ? w * sm.rgb[2] : 0.f, lane);
+		const float q0 = p0 + wave_incl_sum(valid ? w * sm.rgb[0] : 0.f);
+		const float q1 = p1 + wave_incl_sum(valid ? w * sm.rgb[1] : 0.f);
+		const float q2 = p2 + wave_incl_sum(valid ? w * sm.rgb[2] : 0.f);
 		if (valid) {
 			const float dot = grad[0] * (Ta * sm.rgb[0] - (rs.rgb[0] - q0)) + grad[1] * (Ta * sm.rgb[1] - (rs.rgb[1] - q1)) +
 			                  grad[2] * (Ta * sm.rgb[2] - (rs.rgb[2] - q2));
@@ -413,8 +415,8 @@ __global__ void __launch_bounds__(CB) composite_backward_kernel(CompParams c, ui
 				}
 			}
 		}
-		T = __shfl(Ta, 63);
-		p0 = __shfl(q0, 63); p1 = __shfl(q1, 63); p2 = __shfl(q2, 63);
+		T = of_lane(Ta, 63);
+		p0 = of_lane(q0, 63); p1 = of_lane(q1, 63); p2 = of_lane(q2, 63);
 	}
 }
 
@@ -440,6 +442,8 @@ constexpr float CHUNK_T_EPS = 0.5f * T_EPS;
 // counter, and those atomics, all on one address, run one after the other (16 rays per workgroup: 2500 of them, 20 us)
 constexpr uint32_t CHUNK_BLOCK = 1024, CHUNK_LANES = 16, CHUNK_RAYS = CHUNK_BLOCK / CHUNK_LANES;
 
+// The launch is a chain of round trips: what goes by the ray's number is fetched together, then its direction with its first samples, and a listed sample's
+// ray is searched once, not again for each of its seven coordinates (15.0 -> 10.8 us for 36 000 rays, three times a step).
 // One ray per sixteen lanes (a row of the data-parallel lane operations): the lanes take the ray's samples sixteen at a
 // time.  coords_listed receives the coordinate rows of the listed samples in list order, so that the field's kernels read
 // their input without going through the list.
@@ -449,44 +453,51 @@ __global__ void __launch_bounds__(CHUNK_BLOCK) composite_chunk_kernel(CompParams
                                                                       ChunkRay* __restrict__ state, uint32_t* __restrict__ counts,
                                                                       uint32_t* __restrict__ counts_other, uint32_t* __restrict__ list,
                                                                       uint32_t* __restrict__ column_of, float* __restrict__ coords_listed) {
-	__shared__ uint32_t takes[CHUNK_RAYS], firsts[CHUNK_RAYS], before[CHUNK_RAYS + 1], wg_at;
+	__shared__ uint32_t takes[CHUNK_RAYS], firsts[CHUNK_RAYS], before[CHUNK_RAYS + 1], wg_at, ids[CHUNK_BLOCK];
 	const uint32_t l = threadIdx.x % CHUNK_LANES, slot = threadIdx.x / CHUNK_LANES;
 	const uint32_t ray = blockIdx.x * CHUNK_RAYS + slot;
 	const uint32_t live_rays = ray_counter ? min(*ray_counter, n_rays) : n_rays;
 	// the counters that the following step uses start from zero
 	if (round == 0 && blockIdx.x == 0 && threadIdx.x < N2_CHUNK_MAX_ROUNDS) counts_other[threadIdx.x] = 0u;
+	// (what is fetched by the ray's number alone, whether it counts or not, goes out together; so do the ray's direction and its first samples)
 	uint32_t begin = 0;  // samples listed by the rounds before this one
-	for (uint32_t q = 0; q < round; ++q) begin += counts[q];
-	ChunkRay st = {0u, 0u, 1.f, 0u};
-	uint32_t n = 0, base = 0;
-	if (ray < live_rays) {
-		n = numsteps[2 * ray];
-		base = numsteps[2 * ray + 1];
-		if (round == 0) {
-			st.live = n > 0 ? 1u : 0u;
-		} else {
-			st = state[ray];
-			if (st.live) {
-				float dir[3];
-				ray_dir(net_out, base, dir);
-				float T = st.T;
-				for (uint32_t s0 = st.prev; s0 < st.done; s0 += CHUNK_LANES) {
-					const uint32_t s = s0 + l;
-					float keep = 1.f;
-					if (s < st.done) {
-						float o[16];
-						load_out(net_out, (size_t)base + s, o);
-						const Sample sm = eval_sample(o, net_out[((size_t)base + s) * 16 + 7], coords[((size_t)base + s) * 7 + 3], dir, c);
-						keep = 1.f - sm.alpha;
-					}
 #pragma unroll
-					for (int o = 1; o < (int)CHUNK_LANES; o <<= 1) keep *= __shfl_xor(keep, o);  // stays inside the sixteen lanes
-					T *= keep;
-				}
-				st.T = T;
-				if (!(T >= CHUNK_T_EPS) || st.done >= n) st.live = 0u;  // (a transmittance that is not a number retires the ray too)
+	for (uint32_t q = 0; q < N2_CHUNK_MAX_ROUNDS; ++q) {
+		const uint32_t listed = counts[q];
+		begin += q < round ? listed : 0u;
+	}
+	const uint32_t at = min(ray, n_rays - 1u);
+	uint32_t n = numsteps[2 * at];
+	const uint32_t base = numsteps[2 * at + 1];
+	ChunkRay st = {0u, 0u, 1.f, 0u};
+	if (round > 0) st = state[at];
+	if (ray >= live_rays) {
+		n = 0;
+		st.live = 0u;
+	} else if (round == 0) {
+		st.live = n > 0 ? 1u : 0u;
+	} else if (st.live) {
+		const hf* const first = net_out + (size_t)base * 16 + 8;
+		const hf dx = first[0], dy = first[1], dz = first[2];
+		float dir[3], T = st.T;
+		for (uint32_t s0 = st.prev; s0 < st.done; s0 += CHUNK_LANES) {
+			const uint32_t s = s0 + l;
+			OutRow row{};
+			float dt = 0.f, keep = 1.f;
+			if (s < st.done) {
+				row = load_row(net_out, (size_t)base + s);
+				dt = coords[((size_t)base + s) * 7 + 3];
 			}
+			unit_dir(dx, dy, dz, dir);
+			if (s < st.done) keep = 1.f - eval_row(row, dt, dir, c).alpha;
+			keep *= lane_of<0x128>(1.f, keep);  // the product over the sixteen lanes, as a butterfly over distances 8, 4, 2, 1 (see wave_sum)
+			keep *= lane_of<0x124>(1.f, keep);
+			keep *= lane_of<0x4E>(1.f, keep);
+			keep *= lane_of<0xB1>(1.f, keep);
+			T *= keep;
 		}
+		st.T = T;
+		if (!(T >= CHUNK_T_EPS) || st.done >= n) st.live = 0u;  // (a transmittance that is not a number retires the ray too)
 	}
 	const uint32_t take = st.live ? min(n - st.done, chunk) : 0u;
 	// places in the list: the workgroup's 64 rays in order, one atomic per workgroup for its block of places
@@ -495,18 +506,12 @@ __global__ void __launch_bounds__(CHUNK_BLOCK) composite_chunk_kernel(CompParams
 	if (threadIdx.x < 64) {  // one wave scans the 64 counts
 		static_assert(CHUNK_RAYS == 64, "one count per lane");
 		const uint32_t own = takes[threadIdx.x];
-		uint32_t incl = own;
-#pragma unroll
-		for (int o = 1; o < 64; o <<= 1) {
-			const uint32_t up = __shfl_up(incl, o);
-			if ((int)threadIdx.x >= o) incl += up;
-		}
-		const uint32_t total = __shfl(incl, 63);
-		uint32_t at = 0;
-		if (threadIdx.x == 0 && total) at = atomicAdd(&counts[round], total);
+		const uint32_t incl = wave_incl_sum(own), total = of_lane(incl, 63);
+		uint32_t place = 0;
+		if (threadIdx.x == 0 && total) place = atomicAdd(&counts[round], total);
 		before[threadIdx.x] = incl - own;
 		if (threadIdx.x == 63) before[CHUNK_RAYS] = total;
-		if (threadIdx.x == 0) wg_at = at;
+		if (threadIdx.x == 0) wg_at = place;
 	}
 	__syncthreads();
 	// The workgroup's listed samples, all threads together (a ray that lists hundreds of samples in the last round would
@@ -520,15 +525,26 @@ __global__ void __launch_bounds__(CHUNK_BLOCK) composite_chunk_kernel(CompParams
 			if (before[r + step] <= e) r += step;
 		return r;
 	};
-	for (uint32_t e = threadIdx.x; e < total; e += CHUNK_BLOCK) {
-		const uint32_t r = ray_of(e), id = firsts[r] + (e - before[r]);
-		list[at0 + e] = id;
-		column_of[id] = at0 + e;
-	}
-	float* to = coords_listed + (size_t)at0 * 7;
-	for (uint32_t f = threadIdx.x; f < total * 7u; f += CHUNK_BLOCK) {
-		const uint32_t e = f / 7u, r = ray_of(e);
-		to[f] = coords[(size_t)(firsts[r] + (e - before[r])) * 7 + (f - e * 7u)];
+	for (uint32_t e0 = 0; e0 < total; e0 += CHUNK_BLOCK) {
+		const uint32_t e = e0 + threadIdx.x, here = min(total - e0, CHUNK_BLOCK) * 7u;
+		if (e < total) {
+			const uint32_t r = ray_of(e), id = firsts[r] + (e - before[r]);
+			ids[threadIdx.x] = id;
+			list[at0 + e] = id;
+			column_of[id] = at0 + e;
+		}
+		__syncthreads();
+		float v[7];
+#pragma unroll
+		for (uint32_t k = 0; k < 7; ++k) {
+			const uint32_t f = min(threadIdx.x + k * CHUNK_BLOCK, here - 1u), q = f / 7u;
+			v[k] = coords[(size_t)ids[q] * 7 + (f - q * 7u)];
+		}
+		float* const to = coords_listed + (size_t)(at0 + e0) * 7;
+#pragma unroll
+		for (uint32_t k = 0; k < 7; ++k)
+			if (threadIdx.x + k * CHUNK_BLOCK < here) to[threadIdx.x + k * CHUNK_BLOCK] = v[k];
+		__syncthreads();
 	}
 	if (ray < live_rays && l == 0) {
 		st.prev = st.done;
