@@ -375,9 +375,16 @@ __device__ __forceinline__ void gather_features(const FusedArgs& a, uint32_t lev
 
 // first column and number of samples of a listed pass
 __device__ __forceinline__ void listed_range(const FusedArgs& a, uint32_t& begin, uint32_t& count) {
-	begin = 0;
-	for (uint32_t q = 0; q < a.round; ++q) begin += a.counts[q];
-	count = min(a.counts[a.round], a.N - min(begin, a.N));
+	uint32_t listed[N2_CHUNK_MAX_ROUNDS];
+#pragma unroll
+	for (uint32_t q = 0; q < N2_CHUNK_MAX_ROUNDS; ++q) listed[q] = a.counts[min(q, a.round)];  // (all of them under way together)
+	begin = count = 0;
+#pragma unroll
+	for (uint32_t q = 0; q < N2_CHUNK_MAX_ROUNDS; ++q) {
+		begin += q < a.round ? listed[q] : 0u;
+		count = q == a.round ? listed[q] : count;
+	}
+	count = min(count, a.N - min(begin, a.N));
 }
 
 // The listed pass: the number of samples is known on the device only.  The launch has est_tiles workgroups per level, levels dealt
@@ -548,24 +555,54 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 	uint4* LV = reinterpret_cast<uint4*>(smem + (size_t)(FULL ? FF_COUNT : FF_SDF_COUNT) * 1024);
 	// FULL: each wave's staging area for the colour net's input (32 samples)
 	unsigned char* const stage = smem + (size_t)(FULL ? FF_COUNT : FF_SDF_COUNT) * 1024 + FF_LEVELS * sizeof(uint4) + (threadIdx.x >> 6) * (32 * 2 * N2_RGB_IN_PITCH);
-	if (threadIdx.x < FF_LEVELS)
-		LV[threadIdx.x] = make_uint4(__float_as_uint(a.lv.scale[threadIdx.x]), a.lv.res[threadIdx.x], a.lv.entries[threadIdx.x], a.lv.offset[threadIdx.x]);
-	// (a.frags: copied from the image a gather launch left in global memory, instead of two-byte picks all over the weight matrices: 5 to 7 us of a launch)
-	if (FULL && a.frags) load_frags<FF_COUNT, FF_BLOCK>(F, a.frags);
-	else build_fused_frags(F, a, FULL ? FF_COUNT : FF_SDF_COUNT);
 	const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
 	const uint32_t N = a.N, hash_mask = a.lv.hash_mask, active = a.lv.active_levels;
 	uint32_t n_live = a.live ? min(*a.live, N) : N, col0 = 0;
 	if (FULL && a.list) listed_range(a, col0, n_live);  // a listed pass: columns col0 .. col0 + n_live
 	const uint32_t n_tiles = (n_live + 31u) / 32u;
 	const uint32_t wave_gid = blockIdx.x * (FF_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (FF_BLOCK / 64);
-	// (Loading a wave's next tile while the current one is computed, into the registers the current operands have left, was
-	// measured on the full forward: no change; neither did three workgroups per CU at 168 registers, which spills.)
+	// FULL: what a tile starts with (features, coordinates, place in the output); the next tile's is under way while the current one is computed, the
+	// first one's beside the weights.  (2^18 samples 35.7 -> 33 us, a round of the depth rounds 17 -> 14.6: two waves a SIMD hide little, and the loads of a tile also waited for the
+	// stores of the last one.  Three workgroups per CU at 168 registers spill.)
+	struct Start {
+		hf feat[16];
+		float p[3], dir[3];
+		uint32_t dst;
+	};
+	const uint32_t* const places = a.list ? a.list : reinterpret_cast<const uint32_t*>(a.coords);  // (no branch round the load; without a list its value is not used)
+	auto start = [&](uint32_t tile) __attribute__((always_inline)) {
+		Start t;
+		const uint32_t col = col0 + min(tile * 32u + n, n_live - 1u);
+		const float* q = a.coords + (size_t)col * 7;
+#pragma unroll
+		for (int d = 0; d < 3; ++d) { t.p[d] = q[d]; t.dir[d] = q[4 + d]; }
+#pragma unroll
+		for (int j = 0; j < 8; ++j) {
+			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
+			// levels the grid does not have read level 0's rows and are ignored (their weights are zero)
+			const uint32_t lr = 2u * level < a.enc_w ? level : 0u;
+			t.feat[2 * j] = a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
+			t.feat[2 * j + 1] = a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
+		}
+		t.dst = places[col];
+		return t;
+	};
+	Start next;
+	hf variance = (hf)0;
+	if constexpr (FULL) {
+		if (n_tiles > 0) next = start(min(wave_gid, n_tiles - 1u));
+		variance = a.variance[0];
+	}
+	if (threadIdx.x < FF_LEVELS)
+		LV[threadIdx.x] = make_uint4(__float_as_uint(a.lv.scale[threadIdx.x]), a.lv.res[threadIdx.x], a.lv.entries[threadIdx.x], a.lv.offset[threadIdx.x]);
+	// (a.frags: copied from the image a gather launch left in global memory, instead of two-byte picks all over the weight matrices: 5 to 7 us of a launch)
+	if (FULL && a.frags) load_frags<FF_COUNT, FF_BLOCK>(F, a.frags);
+	else build_fused_frags(F, a, FULL ? FF_COUNT : FF_SDF_COUNT);
 	for (uint32_t tile = wave_gid; tile < n_tiles; tile += n_waves) {
 		const uint32_t col_raw = tile * 32u + n;
 		const bool valid = col_raw < n_live;
 		const uint32_t col = col0 + (valid ? col_raw : n_live - 1u);
-		const uint32_t dst = (FULL && a.list) ? a.list[col] : col;  // the sample's row in the output
+		uint32_t dst = col;  // the sample's row in the output
 		half8 xs[3];               // SDF net input, B operands
 		float p[3], dir[3] = {0.f, 0.f, 0.f};
 		uint4 slope[8];            // FULL: the slopes of the lane's 8 levels as stored
@@ -591,9 +628,9 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 #undef FF_STEP
 		} else {
 			if (FULL) {
-				const float* q = a.coords + (size_t)col * 7;
+				if (a.list) dst = next.dst;
 #pragma unroll
-				for (int d = 0; d < 3; ++d) { p[d] = q[d]; dir[d] = q[4 + d]; }
+				for (int d = 0; d < 3; ++d) { p[d] = next.p[d]; dir[d] = next.dir[d]; }
 			} else {
 				const float* q = a.pos + (size_t)col * a.ps;
 #pragma unroll
@@ -604,8 +641,8 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 				const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
 				// levels the grid does not have read level 0's rows and are ignored (their weights are zero)
 				const uint32_t lr = 2u * level < a.enc_w ? level : 0u;
-				xs[j >> 2][2 * (j & 3)] = a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
-				xs[j >> 2][2 * (j & 3) + 1] = a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
+				xs[j >> 2][2 * (j & 3)] = FULL ? next.feat[2 * j] : a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
+				xs[j >> 2][2 * (j & 3) + 1] = FULL ? next.feat[2 * j + 1] : a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
 				if (FULL) slope[j] = a.slopes[(size_t)lr * N + col];
 			}
 		}
@@ -622,6 +659,8 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 			tile_fence();
 			continue;
 		}
+		const uint32_t next_tile = tile + n_waves;
+		if constexpr (FULL) next = start(next_tile < n_tiles ? next_tile : tile);
 		// ---- d sdf / d input: dh = mask * W_out[0, :], dX = W_0^T dh ----
 		half8 dh[4];
 #pragma unroll
@@ -683,6 +722,13 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 			__builtin_amdgcn_wave_barrier();
 			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+			// (The next tile's start has arrived before this one's stores are issued: a load behind a store in a branch is awaited
+			// with the store.)
+#pragma unroll
+			for (int k = 0; k < 16; ++k) asm volatile("" : "+v"(next.feat[k]));
+#pragma unroll
+			for (int d = 0; d < 3; ++d) asm volatile("" : "+v"(next.p[d]), "+v"(next.dir[d]));
+			asm volatile("" : "+v"(next.dst));
 			const uint32_t chunks = 5u * min(32u, n_live - tile * 32u);  // 16-byte chunks of the tile's samples
 			unsigned char* out = reinterpret_cast<unsigned char*>(a.rgb_in) + ((size_t)col0 + (size_t)tile * 32u) * (2u * N2_RGB_IN_PITCH);
 #pragma unroll
@@ -723,7 +769,7 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 			lo[3] = y[0] + (hf)a.sdf_bias;
 			hi[0] = (hf)dir[0]; hi[1] = (hf)dir[1]; hi[2] = (hf)dir[2];
 		} else {
-			lo[0] = hn[0]; lo[1] = hn[1]; lo[2] = hn[2]; lo[3] = a.variance[0];
+			lo[0] = hn[0]; lo[1] = hn[1]; lo[2] = hn[2]; lo[3] = variance;
 		}
 		if (valid) {
 			hf* o = a.output + (size_t)dst * MLP_OUT;
