@@ -152,6 +152,36 @@ def test_samples_generated_ahead_give_the_same_steps():
     np.testing.assert_array_equal(m_a, m_b)
 
 
+def test_steps_on_changing_streams_wait_for_the_samples_generated_ahead():
+    """A step leaves the wait for the following step's samples on its own stream: a following step on another stream waits for itself, and so does one
+    after a step that was refused."""
+    from neus2_amd.capi import N2Error
+    from neus2_amd.tcnn_api import pack_cameras
+    from neus2_amd.training import Trainer, default_config
+    cams = scene.cameras_on_sphere(6, 64)
+    d_cams, d_rgba, d_bits = pack_cameras(cams), dev(scene.render_sphere_images(cams)), dev(scene.sphere_bitfield())
+    T = 2048
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    runs = []
+    for order in ([0] * 8, [0, 0, 1, 1, 2, 0, 2, 1]):
+        tr = Trainer(default_config(target_batch_size=T, max_rays_per_batch=512, max_samples=16 * T, prefetch_samples=True))
+        tr.set_scene(d_cams, len(cams), d_rgba, d_bits)
+        tr.initialize_params(seed=5, sdf_mlp_weights=None)
+        torch.cuda.synchronize()
+        for k, which in enumerate(order):
+            streams[which].wait_stream(streams[order[k - 1]] if k else streams[0])
+            with torch.cuda.stream(streams[which]):
+                if k == 5:
+                    with pytest.raises(N2Error, match="n_rays"):
+                        tr.step(n_rays=10 ** 6, n_inference=16 * T, seed=k)
+                tr.step(n_rays=200, n_inference=16 * T, seed=k)
+        torch.cuda.synchronize()
+        runs.append((tr.read_counters(), host(tr.master).copy()))
+        del tr
+    assert runs[0][0] == runs[1][0] and runs[0][0]["rays"] > 0
+    np.testing.assert_array_equal(runs[0][1], runs[1][1])
+
+
 def test_a_step_is_bit_reproducible_at_the_benchmark_batch():
     """Two trainers run the same steps at the 2^18 batch (the encoding's coarsest levels then split their buckets over
     several workgroups, whose partial sums meet in a fixed order): gradients, counters, loss and parameters agree bit for
