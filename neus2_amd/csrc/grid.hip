@@ -12,6 +12,7 @@
 #include "grid_device.h"
 #include "slab_reduce.h"
 
+#include <algorithm>
 #include <cmath>
 #include <new>
 #include <type_traits>
@@ -438,10 +439,14 @@ constexpr uint32_t BKT_MAX = (1u << 19) >> BKT_SHIFT;  // buckets per level (ent
 constexpr uint32_t BKT_MIN_SHIFT = 5;                  // smallest bucket of a level that chooses its own size (N2LevelTable::bucket_shift)
 constexpr uint32_t PAIR_MAX_CELL = BKT_ENTRIES - 2u;  // pair records (grid_bin_kernel): x + 1 <= BKT_ENTRIES - 1
 static_assert(BKT_SHIFT <= 12, "a pair record's 16-bit key holds the entry within the bucket and four bits of carry length");
-constexpr uint32_t BIN_POINTS = 1024;    // points per bin workgroup
-constexpr uint32_t BIN_RECORDS = BIN_POINTS * 8;
 constexpr uint32_t BIN_BLOCK = 512;       // 8 waves: three workgroups (3 x 49 KiB of LDS) keep 6 waves on every SIMD, at 80 registers (with 96 or 128: pair +10 us)
-constexpr uint32_t BIN_PER_THREAD = BIN_POINTS / BIN_BLOCK;  // 2
+// Points per thread of a bin workgroup (a tile: BIN_BLOCK * per points, eight records each).  Two, and one for batches whose tiles of two would not
+// give every CU a workgroup: those wait for one workgroup's chain of round trips, which is shorter for one point (5003 points: first order
+// 7.1 -> 5.5 us, second order with its output 14.5 -> 9.7; 12000 uniform points 9 -> 8; 16384 samples 7.9 -> 6.1, and the summing kernel, which has twice the runs, 16.6 -> 17.5).
+constexpr uint32_t BIN_HALF_POINTS = 16384;
+__host__ __device__ constexpr uint32_t bin_per_thread(uint32_t n_points) { return n_points <= BIN_HALF_POINTS ? 1u : 2u; }
+__host__ __device__ constexpr uint32_t bin_points(uint32_t per) { return BIN_BLOCK * per; }
+__host__ __device__ constexpr uint32_t bin_records(uint32_t per) { return bin_points(per) * 8u; }
 
 struct N2BucketPlan {
 	uint32_t wg_begin[N2_MAX_LEVELS + 1];  // first reduce workgroup of each level
@@ -592,7 +597,7 @@ constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 // updates and prefix look-ups are therefore issued together, and nothing waits in a branch.  With each of them awaited where it was used,
 // and the second point's loads behind the first one's counters: training step at 2^18 samples 57 us, now 48; 2^18 uniform points 47, now 43;
 // 52344 samples 15.2, now 12.6.
-template <bool FIRST, bool SECOND, bool WANT_OUT, bool PAIR>
+template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT, bool PAIR>
 __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uint32_t level, const uint32_t tile, uint32_t N, uint32_t tiles,
                                               const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                               const __half* __restrict__ dL_dy, const float* __restrict__ v, const __half* __restrict__ g2,
@@ -604,28 +609,28 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t shift = PAIR ? BKT_SHIFT : (uint32_t)tab.bucket_shift[level], in_bucket = (1u << shift) - 1u;
 	// records of this thread: entry | rank << 19 after the counting step (REC_SKIP: merged into a later lane)
-	uint32_t re[BIN_PER_THREAD * R], rv[BIN_PER_THREAD * 8], tcode[BIN_PER_THREAD];
+	uint32_t re[PER * R], rv[PER * 8], tcode[PER];
 	// The second point's inputs are under way while the first one's records are merged and counted, the index it reads some of them by before
 	// that.  (The
 	// position and g2's columns may be read through an index: n2_grid_backward_fused_indexed.)
 	const uint32_t Ng = index ? n_cols : N;
-	uint32_t src[BIN_PER_THREAD];
+	uint32_t src[PER];
 #pragma unroll
-	for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) src[j] = min(tile * BIN_POINTS + j * BIN_BLOCK + threadIdx.x, N - 1u);
+	for (uint32_t j = 0; j < PER; ++j) src[j] = min(tile * bin_points(PER) + j * BIN_BLOCK + threadIdx.x, N - 1u);
 	if (index) {
 #pragma unroll
-		for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) src[j] = index[src[j]];
+		for (uint32_t j = 0; j < PER; ++j) src[j] = index[src[j]];
 #pragma unroll
-		for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) src[j] = min(src[j], n_cols - 1u);
+		for (uint32_t j = 0; j < PER; ++j) src[j] = min(src[j], n_cols - 1u);
 	}
 	auto load = [&](uint32_t j) __attribute__((always_inline)) {
-		const uint32_t i = min(tile * BIN_POINTS + j * BIN_BLOCK + threadIdx.x, N - 1u);
+		const uint32_t i = min(tile * bin_points(PER) + j * BIN_BLOCK + threadIdx.x, N - 1u);
 		return grid_bin_load<FIRST, SECOND>(level, i, N, xyz, point_stride, dim_stride, dL_dy, v, g2, src[j], Ng);
 	};
 	N2BinInput next = load(0);
 #pragma unroll
-	for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) {
-		const uint32_t i = tile * BIN_POINTS + j * BIN_BLOCK + threadIdx.x;
+	for (uint32_t j = 0; j < PER; ++j) {
+		const uint32_t i = tile * bin_points(PER) + j * BIN_BLOCK + threadIdx.x;
 		const N2BinInput in = next;
 		bool valid = i < N;
 		if (valid && n2_level_masked(tab, level, i)) {  // a switched-off level: no records, zero second-order output
@@ -648,7 +653,7 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 #undef CALL
 			}
 		}
-		if (j + 1 < BIN_PER_THREAD) next = load(j + 1);
+		if (j + 1 < PER) next = load(j + 1);
 		// runs of equal cells among the wave's 64 consecutive points
 		const uint32_t up_x = __shfl_up(cell[0], 1), up_y = __shfl_up(cell[1], 1), up_z = __shfl_up(cell[2], 1);
 		const int up_valid = __shfl_up((int)valid, 1);
@@ -684,20 +689,20 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	}
 	__syncthreads();
 	if (threadIdx.x < 64) {  // one wave scans the counters, BKT_MAX / 64 consecutive ones per lane
-		constexpr uint32_t PER = BKT_MAX / 64;
-		uint32_t c[PER], s = 0;
+		constexpr uint32_t EACH = BKT_MAX / 64;
+		uint32_t c[EACH], s = 0;
 #pragma unroll
-		for (uint32_t q = 0; q < PER; ++q) { c[q] = hist[threadIdx.x * PER + q]; s += c[q]; }
+		for (uint32_t q = 0; q < EACH; ++q) { c[q] = hist[threadIdx.x * EACH + q]; s += c[q]; }
 		const uint32_t own = s;
 		s = n2_wave_prefix(s);
 		uint32_t run = s - own;
 #pragma unroll
-		for (uint32_t q = 0; q < PER; ++q) { prefix[threadIdx.x * PER + q] = run; run += c[q]; }
+		for (uint32_t q = 0; q < EACH; ++q) { prefix[threadIdx.x * EACH + q] = run; run += c[q]; }
 		if (threadIdx.x == 63) prefix[BKT_MAX] = s;
 	}
 	__syncthreads();
 #pragma unroll
-	for (uint32_t j = 0; j < BIN_PER_THREAD; ++j) {
+	for (uint32_t j = 0; j < PER; ++j) {
 		if (re[R * j] == REC_SKIP) continue;  // (a point's records go in together or not at all)
 		uint32_t pos[R];
 #pragma unroll
@@ -717,7 +722,7 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	__syncthreads();
 	const uint32_t total = prefix[BKT_MAX];
 	// 16 bytes per lane; the last store of each array may run past `total` inside the tile's own slot, which nobody reads
-	const size_t slot = ((size_t)level * tiles + tile) * BIN_RECORDS;
+	const size_t slot = ((size_t)level * tiles + tile) * bin_records(PER);
 	uint4* out_val = reinterpret_cast<uint4*>(rec_vals + slot);
 	uint4* out_key = reinterpret_cast<uint4*>(rec_keys + slot);
 	const uint4* sv = reinterpret_cast<const uint4*>(stage_val);
@@ -727,7 +732,7 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	if (threadIdx.x <= BKT_MAX) offsets[((size_t)level * tiles + tile) * (BKT_MAX + 1) + threadIdx.x] = (uint16_t)prefix[threadIdx.x];
 }
 
-template <bool FIRST, bool SECOND, bool WANT_OUT>
+template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT>
 __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab, uint32_t first_level, uint32_t N, uint32_t tiles,
                                                               const float* __restrict__ xyz, uint32_t point_stride,
                                                               uint32_t dim_stride, const __half* __restrict__ dL_dy,
@@ -738,16 +743,16 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
                                                               const uint32_t* __restrict__ index, uint32_t n_cols) {
 	__shared__ uint32_t hist[BKT_MAX];
 	__shared__ uint32_t prefix[BKT_MAX + 1];
-	__shared__ __align__(16) uint32_t stage_val[BIN_RECORDS];  // sorted records: packed half2 value (a pair of them on pair levels) ...
-	__shared__ __align__(16) uint16_t stage_key[BIN_RECORDS];  // ... and entry within its bucket
+	__shared__ __align__(16) uint32_t stage_val[bin_records(PER)];  // sorted records: packed half2 value (a pair of them on pair levels) ...
+	__shared__ __align__(16) uint16_t stage_key[bin_records(PER)];  // ... and entry within its bucket
 	const uint32_t level = first_level + blockIdx.x / tiles, tile = blockIdx.x % tiles;
 	if (threadIdx.x < BKT_MAX) hist[threadIdx.x] = 0;
 	__syncthreads();
 	if ((tab.pair_levels >> level) & 1u)
-		grid_bin_tile<FIRST, SECOND, WANT_OUT, true>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, rec_vals,
+		grid_bin_tile<PER, FIRST, SECOND, WANT_OUT, true>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, rec_vals,
 		                                             rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
 	else
-		grid_bin_tile<FIRST, SECOND, WANT_OUT, false>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, rec_vals,
+		grid_bin_tile<PER, FIRST, SECOND, WANT_OUT, false>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, rec_vals,
 		                                              rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
 }
 
@@ -799,7 +804,7 @@ __device__ __forceinline__ N2ReduceItem n2_reduce_item(const N2LevelTable& tab, 
 // first record: 27 us against 17 for 5e3 points, where a workgroup's time is the chain of round trips, 33 against 25 for
 // 6.5e4, 39 against 33 for 1.2e5, 63 against 62 for 2^18.)
 template <bool PAIR, uint32_t FLIGHT>
-__device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2ReduceItem& it, const uint32_t run_lanes,
+__device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const uint32_t slot_records, const N2ReduceItem& it, const uint32_t run_lanes,
                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                    const uint16_t* __restrict__ offsets, unsigned long long* acc) {
 	const uint32_t lanes = 1u << run_lanes, r = threadIdx.x & (lanes - 1u), group = threadIdx.x >> run_lanes, groups = RED_BLOCK >> run_lanes;
@@ -827,7 +832,7 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2R
 		// (lanes without a record read the level's first one: every load is issued, so the compiler can wait for one step only)
 		const uint32_t left = i < end ? (end - i + lanes - 1u) >> run_lanes : 0u;
 		q.n = left < FLIGHT ? left : FLIGHT;
-		const size_t slot = (level_tile0 + (tile < tiles ? tile : 0u)) * BIN_RECORDS;
+		const size_t slot = (level_tile0 + (tile < tiles ? tile : 0u)) * slot_records;
 #pragma unroll
 		for (uint32_t u = 0; u < FLIGHT; ++u) {
 			const uint32_t at = u < q.n ? i + u * lanes : 0u;
@@ -886,7 +891,7 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const N2R
 
 // FLIGHT: 2 for batches of few tiles, whose runs rarely hold more (the loads of absent records cost 2 us at 5e3 points)
 template <uint32_t FLIGHT>
-__global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles,
+__global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                    const uint16_t* __restrict__ offsets,
                                                                    __half2* __restrict__ grads, int accumulate,
@@ -896,8 +901,8 @@ __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable 
 	__shared__ __align__(16) unsigned long long acc[2 * BKT_ENTRIES];
 	const N2ReduceItem it = n2_reduce_item(tab, plan);
 	const uint32_t run_lanes = plan.run_lanes[it.level];
-	if (it.pair) grid_reduce_runs<true, FLIGHT>(tiles, it, run_lanes, rec_vals, rec_keys, offsets, acc);
-	else grid_reduce_runs<false, FLIGHT>(tiles, it, run_lanes, rec_vals, rec_keys, offsets, acc);
+	if (it.pair) grid_reduce_runs<true, FLIGHT>(tiles, slot_records, it, run_lanes, rec_vals, rec_keys, offsets, acc);
+	else grid_reduce_runs<false, FLIGHT>(tiles, slot_records, it, run_lanes, rec_vals, rec_keys, offsets, acc);
 	__syncthreads();
 	if (it.groups > 1) {
 		// Several workgroups hold parts of this bucket's sums (coarse levels of large batches).  Each leaves its image as
@@ -1222,7 +1227,10 @@ static int prepare_grads(n2_grid_t* grid, const char* fn, hipStream_t stream, n2
 }
 
 static inline uint32_t n_pair_tiles(uint32_t n_points) { return (n_points + PAIR_POINTS - 1) / PAIR_POINTS; }
-static inline uint32_t n_bin_tiles(uint32_t n_points) { return (n_points + BIN_POINTS - 1) / BIN_POINTS; }
+static inline uint32_t n_bin_tiles(uint32_t n_points) {
+	const uint32_t points = bin_points(bin_per_thread(n_points));
+	return (n_points + points - 1) / points;
+}
 
 static bool bucket_supported(const n2_grid_t* grid) {
 	for (uint32_t l = 0; l < grid->tab.n_levels; ++l)
@@ -1237,13 +1245,15 @@ struct BucketCarve {
 static uint32_t split_images(const n2_grid_t* grid, uint32_t n_points);
 static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points) {
 	const uint64_t tiles = n_bin_tiles(max_points), L = grid->tab.n_levels;
-	const uint64_t n_rec = L * tiles * BIN_RECORDS;
+	const uint64_t n_rec = L * tiles * bin_records(bin_per_thread(max_points));
 	auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
 	BucketCarve c{};
 	c.vals = 0;
 	c.keys = c.vals + n_rec * sizeof(uint32_t);
 	c.offsets = c.keys + n_rec * sizeof(uint16_t);
 	c.partials = up(c.offsets + L * tiles * (BKT_MAX + 1) * sizeof(uint16_t));
+	// (a batch of half as many points per tile has twice the tiles and bucket offsets: the images of a larger one stand behind those, too)
+	if (max_points > BIN_HALF_POINTS) c.partials = std::max(c.partials, bucket_carve(grid, BIN_HALF_POINTS).partials);
 	c.total = up(c.partials + (uint64_t)split_images(grid, max_points) * BKT_ENTRIES * sizeof(float2));
 	return c;
 }
@@ -1323,7 +1333,7 @@ N2_API int n2_grid_set_workspace(n2_grid_t* grid, void* d_workspace, uint64_t n_
 static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
                            const __half* dL_dy, const float* v, const __half* g2, __half* dL_ddLdy, bool accumulate,
                            const uint32_t* index, uint32_t n_cols) {
-	const uint32_t tiles = n_bin_tiles(n_points), L = grid->tab.n_levels;
+	const uint32_t tiles = n_bin_tiles(n_points), per = bin_per_thread(n_points), L = grid->tab.n_levels;
 	const bool first = dL_dy != nullptr, second = v != nullptr, out = dL_ddLdy != nullptr;
 	const dim3 bd(BIN_BLOCK);
 	// The records of this batch are packed as for a workspace of exactly this size (values, keys, offsets one behind the
@@ -1347,8 +1357,8 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 		plan.groups[l] = groups;
 		{
 			// lanes per run: with their records in flight, about the records a tile's run holds on average
-			const uint32_t per_run = (((tab.pair_levels >> l) & 1u) ? BIN_RECORDS / 2 : BIN_RECORDS) / nb;
-			uint32_t lanes = 4;
+			const uint32_t per_run = (((tab.pair_levels >> l) & 1u) ? bin_records(per) / 2 : bin_records(per)) / nb;
+			uint32_t lanes = 4;  // (3 for tiles of one point per thread: 16.0 -> 16.8 us at 5003 points)
 			while (lanes < 10 && ((few ? 2u : 4u) << lanes) < per_run) ++lanes;
 			plan.run_lanes[l] = (uint8_t)lanes;
 		}
@@ -1360,16 +1370,21 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.wg_begin[l] = wg;
 	for (uint32_t l = L; l < N2_MAX_LEVELS; ++l) { plan.n_buckets[l] = 0; plan.groups[l] = 1; plan.part_begin[l] = images; plan.run_lanes[l] = 0; }
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.split_begin[l] = split;
-#define LAUNCH(F, S, O) grid_bin_kernel<F, S, O><<<gd, bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
-                                                                   grid->params, dL_ddLdy, rec_vals, rec_keys, offsets, index, n_cols)
-	if (first && second && out) LAUNCH(true, true, true);
-	else if (first && second) LAUNCH(true, true, false);
-	else if (second && out) LAUNCH(false, true, true);
-	else if (second) LAUNCH(false, true, false);
-	else LAUNCH(true, false, false);
+	auto bin = [&](auto per_thread) {
+		constexpr uint32_t PER = decltype(per_thread)::value;
+#define LAUNCH(F, S, O) grid_bin_kernel<PER, F, S, O><<<gd, bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
+                                                                        grid->params, dL_ddLdy, rec_vals, rec_keys, offsets, index, n_cols)
+		if (first && second && out) LAUNCH(true, true, true);
+		else if (first && second) LAUNCH(true, true, false);
+		else if (second && out) LAUNCH(false, true, true);
+		else if (second) LAUNCH(false, true, false);
+		else LAUNCH(true, false, false);
 #undef LAUNCH
+	};
+	if (per == 1u) bin(std::integral_constant<uint32_t, 1>());
+	else bin(std::integral_constant<uint32_t, 2>());
 	N2_LAUNCH_CHECK();
-#define LAUNCH(F) grid_reduce_kernel<F><<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials)
+#define LAUNCH(F) grid_reduce_kernel<F><<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials)
 	if (few) LAUNCH(2); else LAUNCH(4);
 #undef LAUNCH
 	N2_LAUNCH_CHECK();

@@ -316,6 +316,31 @@ def test_sorted_scatter_batch_sizes(oracle, n):
             assert rel_l2(got[a:b], times * ref[a:b]) < RTOL, (mode, l)
 
 
+@pytest.mark.parametrize("n,room", [(512, 512), (513, 513), (513, 70000), (16384, 16384), (16384, 16385)])
+def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
+    """The sums are exact, so the size of a tile leaves no trace: a batch equals the one that has points without a gradient behind it, up to where
+    tiles are larger; in a workspace that is just large enough and in a larger one."""
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(**CFG)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = (torch.rand(gg.n_params(), device="cuda", generator=gen) * 2 - 1).half()
+    dg = torch.zeros_like(dp)
+    gg.set_params(dp, dg)
+    large = 16384 + 1024
+    x = torch.rand((3, large), device="cuda", generator=gen)
+    dy, g2, v = (torch.randn((w, large), device="cuda", generator=gen) for w in (32, 32, 3))
+    dy[:, n:] = 0
+    g2[:, n:] = 0
+    got = []
+    for points, space in ((n, room), (large, large)):
+        gg.set_params(dp, dg)
+        assert gg.reserve_scatter_workspace(space)
+        dg.fill_(9.0)
+        out = gg.backward_fused(x[:, :points].contiguous(), dy[:, :points].half().contiguous(), v[:, :points].contiguous(), g2[:, :points].half().contiguous(), mode=GRAD_OVERWRITE)
+        got.append((dg.clone(), out[:, :n].clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and bool((got[0][0] != 0).any())
+
+
 @pytest.mark.parametrize("kind", ["uniform", "clustered", "rays"])
 def test_sorted_scatter_path(oracle, kind):
     """With a scatter workspace, batches go through the run-length kernel (coarsest levels) and the
