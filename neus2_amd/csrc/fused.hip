@@ -358,19 +358,24 @@ __device__ __forceinline__ float pair_finish(const PairItem& it, uint32_t b) {
 	return feat;
 }
 // Inference on points in no particular order: the features of one (point, level) item per lane
-__device__ __forceinline__ void gather_features(const FusedArgs& a, uint32_t level, uint32_t i, bool store) {
-	float feat[2] = {0.f, 0.f}, unused[2][3];
+__device__ __forceinline__ void gather_features(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t n_live) {
+	uint32_t both = 0u;
 	if (level < a.lv.active_levels) {  // a switched-off level: zero features
-		const float* q = a.pos + (size_t)i * a.ps;
-		const float p[3] = {q[0], q[a.ds], q[2 * (size_t)a.ds]};
+		float feat[2], unused[2][3];
+		// (lanes behind the last point take part in its pair's exchange)
+		const float* q = a.pos + (size_t)min(i, n_live - 1u) * a.ps;
+		const float p[3] = {n2_to_pairs(q[0]), n2_to_pairs(q[a.ds]), n2_to_pairs(q[2 * (size_t)a.ds])};
 		const uint32_t entries = a.lv.entries[level], res = a.lv.res[level];
 		const char* base = reinterpret_cast<const char*>(a.table + a.lv.offset[level]);
 		if ((a.lv.hash_mask >> level) & 1u) n2_encode_level<N2_LEVEL_HASH, false>(base, entries, res, a.lv.scale[level], p, 1.f, feat, unused);
 		else n2_encode_level<N2_LEVEL_DENSE, false>(base, entries, res, a.lv.scale[level], p, 1.f, feat, unused);
+		const half2v packed = {(hf)feat[0], (hf)feat[1]};
+		both = n2_from_pairs(__builtin_bit_cast(uint32_t, packed));
 	}
-	if (!store) return;
-	a.sdf_in[(size_t)(3 + 2 * level) * a.N + i] = (hf)feat[0];
-	a.sdf_in[(size_t)(4 + 2 * level) * a.N + i] = (hf)feat[1];
+	if (i >= n_live) return;
+	const half2v feat = __builtin_bit_cast(half2v, both);
+	a.sdf_in[(size_t)(3 + 2 * level) * a.N + i] = feat[0];
+	a.sdf_in[(size_t)(4 + 2 * level) * a.N + i] = feat[1];
 }
 
 // first column and number of samples of a listed pass
@@ -440,7 +445,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 		if (i < n_live) gather_item(a, level, i);
 	} else {
 		if (tile * FG_BLOCK >= n_live) return;
-		gather_features(a, level, min(i, n_live - 1u), i < n_live);  // (lanes behind the last point take part in its pair's exchange)
+		gather_features(a, level, i, n_live);
 	}
 }
 

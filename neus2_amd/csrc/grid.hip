@@ -104,13 +104,20 @@ __device__ __forceinline__ void grid_forward_item(const N2LevelTable& tab, uint3
                                                   const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                                   const __half2* __restrict__ params, __half* __restrict__ out,
                                                   float* __restrict__ dy_dx) {
-	const uint32_t at = min(i, N - 1u);  // (lanes behind the last point take part in its pair's exchange)
-	const bool off = n2_level_masked(tab, level, at);
+	const bool off = n2_level_masked(tab, level, min(i, N - 1u));
 	float feat[2] = {0.f, 0.f}, J[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
 	if (!__all(off)) {
-		const float* q = xyz + (size_t)at * point_stride;
-		const float p[3] = {q[0], q[dim_stride], q[2 * (size_t)dim_stride]}, scale = tab.scale[level];
+		// (lanes behind the last point take part in its pair's exchange)
+		const float* q = xyz + (size_t)min(i, N - 1u) * point_stride;
+		const float p[3] = {n2_to_pairs(q[0]), n2_to_pairs(q[dim_stride]), n2_to_pairs(q[2 * (size_t)dim_stride])}, scale = tab.scale[level];
 		n2_encode_level<MODE, WANT_DYDX>(reinterpret_cast<const char*>(params + tab.offset[level]), tab.entries[level], tab.resolution[level], scale, p, scale, feat, J);
+#pragma unroll
+		for (uint32_t f = 0; f < 2; ++f) {
+			feat[f] = n2_from_pairs(feat[f]);
+#pragma unroll
+			for (uint32_t d = 0; d < 3; ++d)
+				if (WANT_DYDX) J[f][d] = n2_from_pairs(J[f][d]);
+		}
 	}
 	if (i >= N) return;
 #pragma unroll
