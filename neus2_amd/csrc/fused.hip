@@ -224,36 +224,22 @@ __device__ __forceinline__ float2 h2f(uint32_t raw) {
 }
 
 // trilinear value and (with WANT_J) Jacobian of both features of one level
-template <bool WANT_J>
-__device__ __forceinline__ void item_finish(const Item& it, float (&feat)[2], float (&J)[2][3]) {
+__device__ __forceinline__ void item_finish(const Item& it, float (&feat)[2]) {
 	float2 v[8];
 #pragma unroll
 	for (int k = 0; k < 8; ++k) v[k] = h2f(it.raw[k]);
 	const float wx = it.w[0], wy = it.w[1], wz = it.w[2], ux = 1.f - wx, uy = 1.f - wy, uz = 1.f - wz;
 	const float w00 = uy * uz, w10 = wy * uz, w01 = uy * wz, w11 = wy * wz;
-	float s[2][2], ty[2][2], tz[2][2];  // [x plane][feature]
+	float s[2][2];  // [x plane][feature]
 #pragma unroll
 	for (int b = 0; b < 2; ++b) {
 		const float2 a0 = v[b], a1 = v[b + 2], a2 = v[b + 4], a3 = v[b + 6];
 		s[b][0] = fmaf(w00, a0.x, fmaf(w10, a1.x, fmaf(w01, a2.x, w11 * a3.x)));
 		s[b][1] = fmaf(w00, a0.y, fmaf(w10, a1.y, fmaf(w01, a2.y, w11 * a3.y)));
-		if (WANT_J) {
-			ty[b][0] = fmaf(uz, a1.x - a0.x, wz * (a3.x - a2.x));
-			ty[b][1] = fmaf(uz, a1.y - a0.y, wz * (a3.y - a2.y));
-			tz[b][0] = fmaf(uy, a2.x - a0.x, wy * (a3.x - a1.x));
-			tz[b][1] = fmaf(uy, a2.y - a0.y, wy * (a3.y - a1.y));
-		}
 	}
-	const float sc = it.scale, on = it.scale != 0.f ? 1.f : 0.f;
+	const float on = it.scale != 0.f ? 1.f : 0.f;
 #pragma unroll
-	for (int f = 0; f < 2; ++f) {
-		feat[f] = fmaf(ux, s[0][f], wx * s[1][f]) * on;
-		if (WANT_J) {
-			J[f][0] = (s[1][f] - s[0][f]) * sc;
-			J[f][1] = fmaf(ux, ty[0][f], wx * ty[1][f]) * sc;
-			J[f][2] = fmaf(ux, tz[0][f], wx * tz[1][f]) * sc;
-		}
-	}
+	for (int f = 0; f < 2; ++f) feat[f] = fmaf(ux, s[0][f], wx * s[1][f]) * on;
 }
 
 // degree-4 real spherical harmonics of the direction 2 d - 1 (tcnn's SphericalHarmonics encoding, nerf_network.h:251-257)
@@ -282,45 +268,44 @@ __device__ __forceinline__ void sh4(float x, float y, float z, float* o) {
 // ----------------------------------------------------------------------------
 
 // Full field: one (sample, level) item, features and slopes; the item is column i of the matrices, and its
-// coordinates are row i of the input (the [N][7] coordinates, or three rows of positions).  (With the pairs of n2_encode_level a step of
-// 2^18 samples takes 390 us instead of 383, 52344 samples forward and backward 110 instead of 106: these items hold the vector unit as
-// much as the L1.)
-__device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, uint32_t i) {
-	const uint32_t N = a.N;
+// coordinates are row i of the input (the [N][7] coordinates, or three rows of positions).  (2^18 samples of a training step: one lane per sample
+// with eight gathers 68.9 us, lane pairs with adjacent samples 72, with samples 32 apart 66.3; a trained state's step 509.5 -> 504.2.)
+__device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t end) {
+	const uint32_t N = a.N, at = min(i, end - 1u);  // (lanes behind the last sample take part in its pair's exchange)
 	// (full field: the positions from the coordinate rows, or from three rows of their own when the caller has them: a wave
 	// then reads two lines per coordinate instead of fourteen)
 	const bool rows = a.pos == nullptr;
-	const float* q = rows ? a.coords + (size_t)i * 7 : a.pos + (size_t)i * a.ps;
+	const float* q = rows ? a.coords + (size_t)at * 7 : a.pos + (size_t)at * a.ps;
 	const size_t qs = rows ? 1 : a.ds;
 	const float p[3] = {q[0], q[qs], q[2 * qs]};
-	if (level == 0) {
+	if (level == 0 && i < end) {
 #pragma unroll
 		for (int d = 0; d < 3; ++d) {
 			a.sdf_in[(size_t)d * N + i] = (hf)p[d] - (hf)0.5f;
 			a.xyz_rows[(size_t)d * N + i] = p[d];
 		}
 	}
-	float feat[2] = {0.f, 0.f}, J[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+	uint32_t both = 0u;
+	uint4 slopes = make_uint4(0u, 0u, 0u, 0u);
 	if (level < a.lv.active_levels) {  // a switched-off level: zero features, zero slopes
-		LaneLevel L;
-		L.scale = a.lv.scale[level]; L.res = a.lv.res[level]; L.entries = a.lv.entries[level]; L.offset = a.lv.offset[level];
-		L.hashed = (a.lv.hash_mask >> level) & 1u;
-		Item it;
-		uint32_t c[3], boff[8];
-#pragma unroll
-		for (int d = 0; d < 3; ++d) n2_locate(p[d], L.scale, it.w[d], c[d]);
-		it.scale = 1.f;  // slopes are stored without the level's scale factor
-		const char* base = reinterpret_cast<const char*>(a.table);
-		if (L.hashed) corner_offsets<1>(L, c, boff);
-		else corner_offsets<0>(L, c, boff);
-#pragma unroll
-		for (int k = 0; k < 8; ++k) it.raw[k] = *reinterpret_cast<const uint32_t*>(base + boff[k]);
-		item_finish<true>(it, feat, J);
+		float feat[2], J[2][3];
+		const float own[3] = {n2_to_pairs(p[0]), n2_to_pairs(p[1]), n2_to_pairs(p[2])};
+		const uint32_t entries = a.lv.entries[level], res = a.lv.res[level];
+		const char* base = reinterpret_cast<const char*>(a.table + a.lv.offset[level]);
+		// (slopes are stored without the level's scale factor)
+		if ((a.lv.hash_mask >> level) & 1u) n2_encode_level<N2_LEVEL_HASH, true>(base, entries, res, a.lv.scale[level], own, 1.f, feat, J);
+		else n2_encode_level<N2_LEVEL_DENSE, true>(base, entries, res, a.lv.scale[level], own, 1.f, feat, J);
+		const half2v packed = {(hf)feat[0], (hf)feat[1]};
+		both = n2_from_pairs(__builtin_bit_cast(uint32_t, packed));
+		const float six[6] = {J[0][0], J[0][1], J[0][2], J[1][0], J[1][1], J[1][2]};
+		const uint4 w = n2_slopes_pack(six);
+		slopes = make_uint4(n2_from_pairs(w.x), n2_from_pairs(w.y), n2_from_pairs(w.z), n2_from_pairs(w.w));
 	}
-	a.sdf_in[(size_t)(3 + 2 * level) * N + i] = (hf)feat[0];
-	a.sdf_in[(size_t)(4 + 2 * level) * N + i] = (hf)feat[1];
-	const float six[6] = {J[0][0], J[0][1], J[0][2], J[1][0], J[1][1], J[1][2]};
-	a.slopes[(size_t)level * N + i] = n2_slopes_pack(six);
+	if (i >= end) return;
+	const half2v feat = __builtin_bit_cast(half2v, both);
+	a.sdf_in[(size_t)(3 + 2 * level) * N + i] = feat[0];
+	a.sdf_in[(size_t)(4 + 2 * level) * N + i] = feat[1];
+	a.slopes[(size_t)level * N + i] = slopes;
 }
 
 // Small queries: one (sample, level) item by a PAIR of adjacent lanes.  Lane b gathers the four (y, z) corners of x corner b, and
@@ -411,7 +396,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const Fused
 	const uint32_t tiles = (count + FG_BLOCK - 1) / FG_BLOCK;
 	for (uint32_t tile = first_tile; tile < tiles; tile += est_tiles) {
 		const uint32_t j = tile * FG_BLOCK + threadIdx.x;
-		if (j < count) gather_item(a, level, begin + j);
+		if (j - (threadIdx.x & 63u) < count) gather_item(a, level, begin + j, begin + count);  // (whole waves)
 	}
 }
 
@@ -420,7 +405,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 	// Bound by lines on their way from the L2s to the L1s (n2_encode_level): a query of 2^20 uniform points takes one in every 2.6 clocks of
 	// a CU, four per point on every level above the coarsest, and the address units are busy in 95 % of the clocks; the samples of a
 	// training step share lines along their rays (one every 4.7, address units busy in 76 %) but also hold the vector unit in 41 % of the
-	// cycles for their slopes: without its gathers the launch would still take 46 of 71 us.  Measured on the training
+	// cycles for their slopes: without its gathers the launch would still take 46 of 66 us.  Measured on the training
 	// step and dropped: loads of the hashed levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then
 	// requested twice and a request is no cheaper) or carry the non-temporal hint (no change), the positions read as consecutive words
 	// and picked apart in LDS (+9).
@@ -442,7 +427,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 	const uint32_t n_live = a.live ? min(*a.live, a.N) : a.N;
 	const uint32_t i = tile * FG_BLOCK + threadIdx.x;
 	if (FULL) {
-		if (i < n_live) gather_item(a, level, i);
+		if (i - (threadIdx.x & 63u) < n_live) gather_item(a, level, i, n_live);  // (whole waves)
 	} else {
 		if (tile * FG_BLOCK >= n_live) return;
 		gather_features(a, level, i, n_live);
@@ -617,13 +602,12 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 			for (int d = 0; d < 3; ++d) p[d] = q[(size_t)d * a.ds];
 			// the lane's 8 levels, the next level's loads in flight while one is finished
 			Item cur, nxt;
-			float unused[2][3];
 			item_fetch<0>(LV, hash_mask, active, a.table, g, p, cur);
 #define FF_STEP(J)                                                                           \
 			if (J < 7) item_fetch<(J < 7 ? J + 1 : 0)>(LV, hash_mask, active, a.table, g, p, nxt); \
 			{                                                                                \
 				float feat[2];                                                               \
-				item_finish<false>(cur, feat, unused);                                       \
+				item_finish(cur, feat);                                                      \
 				xs[J >> 2][2 * (J & 3)] = (hf)feat[0];                                       \
 				xs[J >> 2][2 * (J & 3) + 1] = (hf)feat[1];                                   \
 			}                                                                                \
