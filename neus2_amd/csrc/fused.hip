@@ -316,13 +316,17 @@ struct PairItem {
 };
 __device__ __forceinline__ void pair_fetch(const FusedArgs& a, uint32_t level, const float (&p)[3], uint32_t b, PairItem& it) {
 	const uint32_t res = a.lv.res[level], entries = a.lv.entries[level];
-	uint32_t c[3], at[4];
+	const bool hashed = (a.lv.hash_mask >> level) & 1u;
+	uint32_t c[3], h[3], at[4], dense[4];
 #pragma unroll
 	for (int d = 0; d < 3; ++d) n2_locate(p[d], a.lv.scale[level], it.w[d], c[d]);
-	if ((a.lv.hash_mask >> level) & 1u) {
-		n2_hash_terms(c);
-		n2_corner_bytes<N2_LEVEL_HASH>(entries, res, c[0] + b, c[1], c[2], at);
-	} else n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, c[0] + b, c[1], c[2], at);
+#pragma unroll
+	for (int d = 0; d < 3; ++d) h[d] = c[d];
+	n2_hash_terms(h);
+	n2_corner_bytes<N2_LEVEL_HASH>(entries, res, h[0] + b, h[1], h[2], at);
+	n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, c[0] + b, c[1], c[2], dense);
+#pragma unroll
+	for (uint32_t k = 0; k < 4; ++k) at[k] = hashed ? at[k] : dense[k];  // (both, and no branch)
 	const char* base = reinterpret_cast<const char*>(a.table + a.lv.offset[level]);
 #pragma unroll
 	for (uint32_t k = 0; k < 4; ++k) it.raw[k] = *reinterpret_cast<const uint32_t*>(base + at[k]);
@@ -476,36 +480,49 @@ __device__ __forceinline__ void store_sdf(const FusedArgs& a, half8 y, uint32_t 
 }
 
 // A small query in one launch: a workgroup takes 32 points, wave w gathers levels w and w + 8 (a lane pair per point, as in
-// gather_pair), the features meet in LDS and wave 0 puts them through the net.  Nothing but latency bounds it: the weights'
-// and the positions' loads are under way together, then the gathers of both levels.
+// PairItem), the features meet in LDS and wave 0 puts them through the net.  Nothing but latency bounds it: the positions' and the
+// weights' loads are under way together, then the gathers of both levels.  No load stands in a branch, which would end in a wait of its
+// own, and the wave's number is made a scalar: what depends on it alone, levels and fragments, then comes through the scalar cache.
+// (1000 points, with branches on the kind of level and the kind of fragment -> so: 7.4 -> 6.9 us; the call takes 7.5, the host's part.)
 constexpr uint32_t FQ_BLOCK = 512, FQ_POINTS = 32;
 constexpr uint32_t FQ_PITCH = 36;  // halves per point in LDS: an odd multiple of 8 bytes, so that the net's 8-byte reads spread over the banks
 __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a) {
 	static_assert(FF_LEVELS == 2 * (FQ_BLOCK / 64), "two levels per wave");
 	__shared__ __align__(16) hf F[FF_SDF_COUNT * 512];
 	__shared__ __align__(16) hf X[FQ_POINTS * FQ_PITCH];
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, b = lane & 1u;
-	const uint32_t first = blockIdx.x * FQ_POINTS;
+	const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), b = lane & 1u;
+	const uint32_t first = blockIdx.x * FQ_POINTS, n = lane & 31u, g = lane >> 5;
 	auto position = [&](uint32_t k, float (&p)[3]) {
 		const uint32_t i = min(first + k, a.N - 1u);
 		const float* q = a.pos + (size_t)i * a.ps;
 		p[0] = q[0]; p[1] = q[a.ds]; p[2] = q[2 * (size_t)a.ds];
 	};
-	float p[3];
+	float p[3], net_p[3];
 	position(lane >> 1, p);
-	constexpr uint32_t VALUES = FF_SDF_COUNT * 64, MORE = VALUES - FQ_BLOCK;
-	static_assert(VALUES > FQ_BLOCK && MORE <= FQ_BLOCK, "one fragment value per thread, and some of the threads a second one");
-	const half8 f0 = fused_frag_value(a, threadIdx.x >> 6, lane);
-	half8 f1 = zero8();
-	if (threadIdx.x < MORE) f1 = fused_frag_value(a, (FQ_BLOCK + threadIdx.x) >> 6, lane);
+	position(n, net_p);
+	// the wave's fragment of the weights, and for two waves a second one: what sdf_forward_frag gives, without a branch round any load
+	constexpr uint32_t WAVES = FQ_BLOCK / 64, MORE = SDF_FRAG_COUNT - WAVES;
+	static_assert(FF_SDF_COUNT == SDF_FRAG_COUNT && SDF_FRAG_WO < WAVES && MORE <= WAVES, "one fragment per wave, and some of the waves a second one");
+	const bool out = wave >= SDF_FRAG_WO;
+	const uint32_t c = out ? wave - SDF_FRAG_WO : wave % 3u, row_n = min(n, MLP_OUT - 1u);
+	const hf* const W1 = a.sdf_w + MLP_WIDTH * a.sdf_in_w;
+	const hf* const row = out ? W1 + row_n * MLP_WIDTH : a.sdf_w + (32u * (wave / 3u) + n) * a.sdf_in_w;
+	hf f0[8];
+#pragma unroll
+	for (int e = 0; e < 8; ++e) {
+		const int k = chained_k((int)c, (int)g, e), col = out ? k : sdf_col(c < 2u ? k : (int)(32u + 8u * g) + e, a.enc_w);
+		f0[e] = h_or_zero(row, out ? n < MLP_OUT : col >= 0, (size_t)max(col, 0));
+	}
+	half8 f1 = wfrag_chained(W1, MLP_WIDTH, (int)row_n, (int)(WAVES - SDF_FRAG_WO + wave % MORE), (int)g);
 	PairItem it[2];
 #pragma unroll
 	for (uint32_t k = 0; k < 2; ++k) {
 		const uint32_t level = wave + 8u * k;
 		pair_fetch(a, level < a.n_levels ? level : 0u, p, b, it[k]);
 	}
-	reinterpret_cast<half8*>(F)[threadIdx.x] = f0;
-	if (threadIdx.x < MORE) reinterpret_cast<half8*>(F)[FQ_BLOCK + threadIdx.x] = f1;
+	reinterpret_cast<half8*>(F)[threadIdx.x] = half8{f0[0], f0[1], f0[2], f0[3], f0[4], f0[5], f0[6], f0[7]};
+	if (n >= MLP_OUT) f1 = zero8();
+	if (wave < MORE) reinterpret_cast<half8*>(F)[FQ_BLOCK + threadIdx.x] = f1;
 #pragma unroll
 	for (uint32_t k = 0; k < 2; ++k) {
 		const uint32_t level = wave + 8u * k;
@@ -514,8 +531,6 @@ __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a
 	}
 	__syncthreads();
 	if (wave != 0) return;
-	const uint32_t n = lane & 31u, g = lane >> 5;
-	position(n, p);
 	half8 xs[3], h[4];
 #pragma unroll
 	for (int c = 0; c < 2; ++c) {
@@ -526,7 +541,7 @@ __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a
 	xs[2] = zero8();
 	if (g == 0) {
 #pragma unroll
-		for (int d = 0; d < 3; ++d) xs[2][d] = (hf)p[d] - (hf)0.5f;
+		for (int d = 0; d < 3; ++d) xs[2][d] = (hf)net_p[d] - (hf)0.5f;
 	}
 	const half8 y = sdf_net(F, (int)lane, xs, h);
 	const bool valid = first + n < a.N;

@@ -25,7 +25,7 @@ constexpr int MLP_WIDTH = 64;
 constexpr int MLP_OUT = 16;
 constexpr int MLP_BLOCK = 256;      // 4 waves
 constexpr int MLP_TILE = 64;        // samples per wave iteration
-constexpr int MLP_MAX_SLABS = 512;  // workgroups of the weight-gradient kernels (two per CU)
+constexpr int MLP_MAX_SLABS = 512;  // slabs of one backward pass that the workspace holds (mlp_bbi_kernel: two workgroups per CU)
 
 // ----------------------------------------------------------------------------
 // fragment loaders (weights live in global memory, a few KB, L1/L2 resident)
