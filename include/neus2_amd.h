@@ -689,7 +689,9 @@ int n2_trainer_set_depth_chunk_estimates(n2_trainer_t* trainer, const uint32_t* 
  *  seed         seed of this step's random draws
  * A step whose rays kept no sample leaves parameters and optimiser state alone (the reference stops training there,
  * src/testbed_nerf.cu:3536-3542), but the host-side counts (optimizer_steps, the training step, the Ema's step count)
- * advance with every call: they count calls, the device decides about the update. */
+ * advance with every call: they count calls, the device decides about the update.
+ * With prefetch_samples a stream that is being captured is refused, before anything is enqueued or noted: the samples generated
+ * ahead cross from one step to the next on a stream of the trainer's own, which a capture of one step cannot hold. */
 int n2_trainer_step(n2_trainer_t* trainer, n2_stream_t stream, uint32_t n_rays, uint32_t n_inference, uint32_t seed);
 
 /* Device buffers of the last step, for inspection and tests (the reference keeps the same data in its arena allocation,

@@ -292,6 +292,13 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 	N2_REQUIRE(n_inference % 8 == 0 && n_inference <= t->cfg.max_samples, "n2_trainer_step: n_inference %u must be a multiple of 8 and <= %u",
 	           n_inference, t->cfg.max_samples);
 	hipStream_t s = n2_stream(stream);
+	// Samples generated ahead cross from one step to the next by events, and what this step notes about them on the host holds only
+	// when its launches run: a captured step would leave the next one to read samples that nothing has written.
+	if (t->side) {
+		hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+		N2_HIP(hipStreamIsCapturing(s, &capture));
+		N2_REQUIRE(capture == hipStreamCaptureStatusNone, "n2_trainer_step: the stream is being captured, which a trainer with prefetch_samples does not allow");
+	}
 	const uint32_t T = t->cfg.target_batch_size;
 	uint32_t* compacted_counter = t->counters + 2;
 	// progressive level mask: the encoding is told the number of training steps taken so far before every step
@@ -334,10 +341,8 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 			// ev_main stands for the last step's Adam launch: enough unless the caller may have put readers of that step's
 			// buffers on the stream since (it asked for the view), or this step runs on another stream
 			main_event_is_last_step = t->ev_main_from_adam && !t->view_taken && s == t->last_stream;
-			// (the last step has left the wait in front of its Adam launch; a stream that is being captured must not go past it)
-			hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-			N2_HIP(hipStreamIsCapturing(s, &capture));
-			if (!t->ready_awaited || s != t->last_stream || capture != hipStreamCaptureStatusNone) N2_HIP(hipStreamWaitEvent(s, t->ev_ready, 0));
+			// (the last step has left the wait in front of its Adam launch)
+			if (!t->ready_awaited || s != t->last_stream) N2_HIP(hipStreamWaitEvent(s, t->ev_ready, 0));
 		} else {
 			// a generation that ran ahead with other arguments is abandoned (it stays ordered on the side stream)
 			cur = t->pf_valid ? 1u - t->pf_set : 1u - t->last_set;

@@ -182,6 +182,43 @@ def test_steps_on_changing_streams_wait_for_the_samples_generated_ahead():
     np.testing.assert_array_equal(runs[0][1], runs[1][1])
 
 
+def test_a_step_under_capture_is_refused_and_leaves_no_trace():
+    """Samples generated ahead do not fit into a captured step: it is refused, whether it would find them (the next seed) or not, and the
+    steps around it are those of a run without it."""
+    from neus2_amd.capi import N2Error
+    from neus2_amd.tcnn_api import pack_cameras
+    from neus2_amd.training import Trainer, default_config
+    cams = scene.cameras_on_sphere(6, 64)
+    d_cams, d_rgba, d_bits = pack_cameras(cams), dev(scene.render_sphere_images(cams)), dev(scene.sphere_bitfield())
+    T = 2048
+    stream = torch.cuda.Stream()
+    runs = []
+    for captures in ({}, {0: 0, 2: 2, 4: 9}):  # before step k a capture with this seed: the first step, a hit, a miss
+        tr = Trainer(default_config(target_batch_size=T, max_rays_per_batch=512, max_samples=16 * T, prefetch_samples=True))
+        tr.set_scene(d_cams, len(cams), d_rgba, d_bits)
+        tr.initialize_params(seed=5, sdf_mlp_weights=None)
+        torch.cuda.synchronize()
+        log = []
+        for k in range(6):
+            if k in captures:
+                x, graph = torch.zeros(8, device="cuda"), torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=stream):
+                    x.add_(1)
+                    with pytest.raises(N2Error, match="captured"):
+                        tr.step(n_rays=200, n_inference=16 * T, seed=captures[k])
+                graph.replay()
+                torch.cuda.synchronize()
+                assert bool((x == 1).all())
+            with torch.cuda.stream(stream):
+                tr.step(n_rays=200, n_inference=16 * T, seed=k)
+                log.append(tr.read_counters())
+        torch.cuda.synchronize()
+        runs.append((log, host(tr.master).copy()))
+        del tr
+    assert runs[0][0] == runs[1][0] and all(c["rays"] > 0 for c in runs[0][0])
+    np.testing.assert_array_equal(runs[0][1], runs[1][1])
+
+
 def test_a_step_is_bit_reproducible_at_the_benchmark_batch():
     """Two trainers run the same steps at the 2^18 batch (the encoding's coarsest levels then split their buckets over
     several workgroups, whose partial sums meet in a fixed order): gradients, counters, loss and parameters agree bit for
