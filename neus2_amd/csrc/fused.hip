@@ -314,20 +314,23 @@ struct PairItem {
 	uint32_t raw[4];
 	float w[3];
 };
-__device__ __forceinline__ void pair_fetch(const FusedArgs& a, uint32_t level, const float (&p)[3], uint32_t b, PairItem& it) {
-	const uint32_t res = a.lv.res[level], entries = a.lv.entries[level];
-	const bool hashed = (a.lv.hash_mask >> level) & 1u;
-	uint32_t c[3], h[3], at[4], dense[4];
+// a level of the wave's own, all of it in scalar registers
+struct WaveLevel {
+	float scale;
+	uint32_t res, entries, offset;
+	bool hashed;
+};
+__device__ __forceinline__ void pair_fetch(const __half2* __restrict__ table, const WaveLevel& L, const float (&p)[3], uint32_t b, PairItem& it) {
+	uint32_t c[3], at[4];
 #pragma unroll
-	for (int d = 0; d < 3; ++d) n2_locate(p[d], a.lv.scale[level], it.w[d], c[d]);
-#pragma unroll
-	for (int d = 0; d < 3; ++d) h[d] = c[d];
-	n2_hash_terms(h);
-	n2_corner_bytes<N2_LEVEL_HASH>(entries, res, h[0] + b, h[1], h[2], at);
-	n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, c[0] + b, c[1], c[2], dense);
-#pragma unroll
-	for (uint32_t k = 0; k < 4; ++k) at[k] = hashed ? at[k] : dense[k];  // (both, and no branch)
-	const char* base = reinterpret_cast<const char*>(a.table + a.lv.offset[level]);
+	for (int d = 0; d < 3; ++d) n2_locate(p[d], L.scale, it.w[d], c[d]);
+	if (L.hashed) {  // (the same for the wave)
+		n2_hash_terms(c);
+		n2_corner_bytes<N2_LEVEL_HASH>(L.entries, L.res, c[0] + b, c[1], c[2], at);
+	} else {
+		n2_corner_bytes<N2_LEVEL_DENSE>(L.entries, L.res, c[0] + b, c[1], c[2], at);
+	}
+	const char* base = reinterpret_cast<const char*>(table + L.offset);
 #pragma unroll
 	for (uint32_t k = 0; k < 4; ++k) it.raw[k] = *reinterpret_cast<const uint32_t*>(base + at[k]);
 }
@@ -457,7 +460,8 @@ __device__ __forceinline__ half8 sdf_net(const hf* F, int lane, const half8 (&xs
 }
 
 // inference: bias, density and what the caller wants stored of sample `col` (col_raw: its number before clamping)
-__device__ __forceinline__ void store_sdf(const FusedArgs& a, half8 y, uint32_t col, bool valid, uint32_t col_raw, int g) {
+template <class Args>
+__device__ __forceinline__ void store_sdf(const Args& a, half8 y, uint32_t col, bool valid, uint32_t col_raw, int g) {
 	if (g == 0) {
 		hf s = y[0] + (hf)a.sdf_bias;
 		if (a.density) {
@@ -480,10 +484,11 @@ __device__ __forceinline__ void store_sdf(const FusedArgs& a, half8 y, uint32_t 
 }
 
 // A small query in one launch: a workgroup takes 32 points, wave w gathers levels w and w + 8 (a lane pair per point, as in
-// PairItem), the features meet in LDS and wave 0 puts them through the net.  Nothing but latency bounds it: the positions' and the
-// weights' loads are under way together, then the gathers of both levels.  No load stands in a branch, which would end in a wait of its
-// own, and the wave's number is made a scalar: what depends on it alone, levels and fragments, then comes through the scalar cache.
-// (1000 points, with branches on the kind of level and the kind of fragment -> so: 7.4 -> 6.9 us; the call takes 7.5, the host's part.)
+// PairItem), the features meet in LDS and wave 0 puts them through the net.  Latency bounds it, and the lines that the weights' loads
+// ask the L1 for: the arguments, then the positions and the weights together, then the gathers of both levels, are a trip each.
+// The weights come four elements a load: with one element a load every lane asked for a line of its own, eight times.  (1000 points, in us: one
+// element a load and branches round those of zero elements 6.6, without the branches 7.1, so 5.6; arguments where they are used 5.8.  The launch
+// alone takes 1.6, without the gathers 5.4 of the 7.1.  The call takes 7.4 and so does one of 8 points: the host's part.)
 constexpr uint32_t FQ_BLOCK = 512, FQ_POINTS = 32;
 constexpr uint32_t FQ_PITCH = 36;  // halves per point in LDS: an odd multiple of 8 bytes, so that the net's 8-byte reads spread over the banks
 __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a) {
@@ -492,60 +497,85 @@ __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a
 	__shared__ __align__(16) hf X[FQ_POINTS * FQ_PITCH];
 	const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), b = lane & 1u;
 	const uint32_t first = blockIdx.x * FQ_POINTS, n = lane & 31u, g = lane >> 5;
-	auto position = [&](uint32_t k, float (&p)[3]) {
-		const uint32_t i = min(first + k, a.N - 1u);
-		const float* q = a.pos + (size_t)i * a.ps;
-		p[0] = q[0]; p[1] = q[a.ds]; p[2] = q[2 * (size_t)a.ds];
-	};
-	float p[3], net_p[3];
-	position(lane >> 1, p);
-	position(n, net_p);
-	// the wave's fragment of the weights, and for two waves a second one: what sdf_forward_frag gives, without a branch round any load
-	constexpr uint32_t WAVES = FQ_BLOCK / 64, MORE = SDF_FRAG_COUNT - WAVES;
-	static_assert(FF_SDF_COUNT == SDF_FRAG_COUNT && SDF_FRAG_WO < WAVES && MORE <= WAVES, "one fragment per wave, and some of the waves a second one");
-	const bool out = wave >= SDF_FRAG_WO;
-	const uint32_t c = out ? wave - SDF_FRAG_WO : wave % 3u, row_n = min(n, MLP_OUT - 1u);
-	const hf* const W1 = a.sdf_w + MLP_WIDTH * a.sdf_in_w;
-	const hf* const row = out ? W1 + row_n * MLP_WIDTH : a.sdf_w + (32u * (wave / 3u) + n) * a.sdf_in_w;
-	hf f0[8];
-#pragma unroll
-	for (int e = 0; e < 8; ++e) {
-		const int k = chained_k((int)c, (int)g, e), col = out ? k : sdf_col(c < 2u ? k : (int)(32u + 8u * g) + e, a.enc_w);
-		f0[e] = h_or_zero(row, out ? n < MLP_OUT : col >= 0, (size_t)max(col, 0));
-	}
-	half8 f1 = wfrag_chained(W1, MLP_WIDTH, (int)row_n, (int)(WAVES - SDF_FRAG_WO + wave % MORE), (int)g);
-	PairItem it[2];
+	// Every argument but the variance in one trip to the scalar cache, the wave's levels among them; left to the compiler each comes where it is used.
+	struct {
+		const __half2* table;
+		const hf *sdf_w, *variance;
+		const float* pos;
+		uint32_t sdf_in_w, enc_w, N, ps, ds, hash_mask, active, row0_n;
+		hf* sdf_out;
+		float *row0, sdf_bias;
+		int density;
+	} q{a.table, a.sdf_w, a.variance, a.pos, a.sdf_in_w, a.enc_w, a.N, a.ps, a.ds, a.lv.hash_mask, a.lv.active_levels, a.row0_n, a.sdf_out, a.row0, a.sdf_bias, a.density};
+	// (levels that the table does not have: n2_fused_field_sdf gives them eight entries, which any table has)
+	uint32_t v[2][3];
+	float scale[2];
 #pragma unroll
 	for (uint32_t k = 0; k < 2; ++k) {
-		const uint32_t level = wave + 8u * k;
-		pair_fetch(a, level < a.n_levels ? level : 0u, p, b, it[k]);
+		const uint32_t l = wave + 8u * k;
+		scale[k] = a.lv.scale[l];
+		v[k][0] = a.lv.res[l]; v[k][1] = a.lv.entries[l]; v[k][2] = a.lv.offset[l];
 	}
-	reinterpret_cast<half8*>(F)[threadIdx.x] = half8{f0[0], f0[1], f0[2], f0[3], f0[4], f0[5], f0[6], f0[7]};
+	asm volatile("" : "+s"(q.N), "+s"(q.row0_n), "+s"(q.sdf_bias), "+s"(q.density)
+	             : "s"(q.table), "s"(q.sdf_w), "s"(q.pos), "s"(q.sdf_in_w), "s"(q.enc_w), "s"(q.ps), "s"(q.ds), "s"(q.hash_mask), "s"(q.active), "s"(q.sdf_out), "s"(q.row0),
+	               "s"(v[0][0]), "s"(v[0][1]), "s"(v[0][2]), "s"(scale[0]), "s"(v[1][0]), "s"(v[1][1]), "s"(v[1][2]), "s"(scale[1]));
+	auto position = [&](uint32_t k, float (&p)[3]) {
+		const uint32_t i = min(first + k, q.N - 1u);
+		const float* at = q.pos + (size_t)i * q.ps;
+		p[0] = at[0]; p[1] = at[q.ds]; p[2] = at[2 * (size_t)q.ds];
+	};
+	float p[3];
+	position(lane >> 1, p);
+	// The wave's fragment of the weights, and for two waves a second one: what sdf_forward_frag gives, four elements a load and without a branch
+	// round any.  Element e is column x + (e & 3) + step (e >> 2) + shift of its row where x + .. is below `columns`, else zero; the four columns
+	// a load takes may reach past the row, but not past the weights, where W_out follows W_0.
+	constexpr uint32_t WAVES = FQ_BLOCK / 64, MORE = SDF_FRAG_COUNT - WAVES;
+	static_assert(FF_SDF_COUNT == SDF_FRAG_COUNT && SDF_FRAG_WO < WAVES && MORE <= WAVES, "one fragment per wave, and some of the waves a second one");
+	typedef hf four __attribute__((ext_vector_type(4), aligned(2)));
+	const bool out = wave >= SDF_FRAG_WO, features = !out && wave % 3u < 2u;
+	const uint32_t c = out ? wave - SDF_FRAG_WO : wave % 3u, row_n = min(n, MLP_OUT - 1u);
+	const hf* const W1 = q.sdf_w + MLP_WIDTH * q.sdf_in_w;
+	const hf* const row = out ? W1 + row_n * MLP_WIDTH : q.sdf_w + (32u * (wave / 3u) + n) * q.sdf_in_w;
+	const uint32_t x = out || features ? 16u * c + 4u * g : 8u * g, step = out || features ? 8u : 4u, shift = features ? 3u : 0u;
+	const uint32_t columns = out ? (n < MLP_OUT ? (uint32_t)MLP_WIDTH : 0u) : features ? q.enc_w : 3u;
+	const four f_lo = *reinterpret_cast<const four*>(row + x + shift), f_hi = *reinterpret_cast<const four*>(row + x + step + shift);
+	half8 f1 = wfrag_chained(W1, MLP_WIDTH, wave < MORE ? (int)row_n : 0, (int)(WAVES - SDF_FRAG_WO + wave % MORE), (int)g);
+	PairItem it[2];
+#pragma unroll
+	for (uint32_t k = 0; k < 2; ++k) pair_fetch(q.table, WaveLevel{scale[k], v[k][0], v[k][1], v[k][2], ((q.hash_mask >> (wave + 8u * k)) & 1u) != 0u}, p, b, it[k]);
+	asm volatile("" : "+v"(f1));  // (not loaded in the branch below)
+	half8 f0;
+#pragma unroll
+	for (uint32_t e = 0; e < 4; ++e) {
+		f0[e] = x + e < columns ? f_lo[e] : (hf)0;
+		f0[4 + e] = x + step + e < columns ? f_hi[e] : (hf)0;
+	}
+	reinterpret_cast<half8*>(F)[threadIdx.x] = f0;
 	if (n >= MLP_OUT) f1 = zero8();
 	if (wave < MORE) reinterpret_cast<half8*>(F)[FQ_BLOCK + threadIdx.x] = f1;
 #pragma unroll
 	for (uint32_t k = 0; k < 2; ++k) {
-		const uint32_t level = wave + 8u * k;
 		const float feat = pair_finish(it[k], b);
-		X[(lane >> 1) * FQ_PITCH + 2u * level + b] = level < a.lv.active_levels ? (hf)feat : (hf)0.f;  // (switched off or not there: zero)
+		X[(lane >> 1) * FQ_PITCH + 2u * (wave + 8u * k) + b] = wave + 8u * k < q.active ? (hf)feat : (hf)0.f;  // (switched off or not there: zero)
 	}
 	__syncthreads();
 	if (wave != 0) return;
 	half8 xs[3], h[4];
 #pragma unroll
 	for (int c = 0; c < 2; ++c) {
-		const hf* q = X + n * FQ_PITCH + 16 * c + 4u * g;
-		const half4v lo = *reinterpret_cast<const half4v*>(q), hi = *reinterpret_cast<const half4v*>(q + 8);
+		const hf* at = X + n * FQ_PITCH + 16 * c + 4u * g;
+		const half4v lo = *reinterpret_cast<const half4v*>(at), hi = *reinterpret_cast<const half4v*>(at + 8);
 		xs[c] = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 	}
 	xs[2] = zero8();
-	if (g == 0) {
 #pragma unroll
-		for (int d = 0; d < 3; ++d) xs[2][d] = (hf)net_p[d] - (hf)0.5f;
+	for (int d = 0; d < 3; ++d) {
+		const float at = __shfl(p[d], 2 * (int)n);  // the point's position, from the pair that gathered for it
+		xs[2][d] = g == 0 ? (hf)at - (hf)0.5f : (hf)0.f;
 	}
 	const half8 y = sdf_net(F, (int)lane, xs, h);
-	const bool valid = first + n < a.N;
-	store_sdf(a, y, valid ? first + n : a.N - 1u, valid, first + n, (int)g);
+	const bool valid = first + n < q.N;
+	store_sdf(q, y, valid ? first + n : q.N - 1u, valid, first + n, (int)g);
 }
 
 // ----------------------------------------------------------------------------

@@ -15,11 +15,7 @@ __device__ __forceinline__ int sdf_col(int row, uint32_t enc_w) {
 	return row < 35 ? row - 32 : -1;
 }
 __device__ __forceinline__ int chained_k(int c, int g, int e) { return 16 * c + 4 * g + (e & 3) + ((e >> 2) << 3); }
-// W[at], or zero (`at` is in bounds all the same: a load without a branch, which would end in a wait of its own)
-__device__ __forceinline__ hf h_or_zero(const hf* W, bool ok, size_t at) {
-	const hf v = W[at];
-	return ok ? v : (hf)0;
-}
+__device__ __forceinline__ hf h_or_zero(const hf* W, bool ok, size_t at) { return ok ? W[at] : (hf)0; }
 
 // lane l's 16 bytes of fragment f < SDF_FRAG_COUNT; ld: columns of W_0
 __device__ __forceinline__ half8 sdf_forward_frag(const hf* W, int ld, uint32_t enc_w, int f, int l) {

@@ -149,6 +149,11 @@ def test_small_queries_equal_the_same_points_in_a_large_one(n, levels, active):
         assert torch.equal(query(few.T.contiguous()).view(torch.int16), want.contiguous().view(torch.int16))
 
 
+@pytest.mark.parametrize("levels", [1, 6])  # input rows of 16 columns: four elements a load reach into the next row, and of the last one into W_out
+def test_small_queries_of_narrow_networks_equal_the_same_points_in_a_large_one(levels):
+    test_small_queries_equal_the_same_points_in_a_large_one(72, levels, 1.0)
+
+
 # one tile past the line at which a query's and a forward's levels are no longer dealt to the XCDs
 @pytest.mark.parametrize("n", [8, 32, 40, 64, 72, 264])  # pairs across a wave's halves: no second half, a part of it, all, a wave more, a workgroup more
 @pytest.mark.parametrize("active", [1.0, 0.5])
