@@ -782,7 +782,9 @@ int n2_occupancy_set_state(n2_occupancy_t* occupancy, uint32_t ema_step, uint64_
  * triangle_table, src/marching_cubes.cu:400-657). */
 int n2_marching_cubes_table(int8_t* out_256x16);
 uint64_t n2_marching_cubes_workspace_bytes(const uint32_t res[3]);
-/* First pass: counts (the reference's "count only" launches, :807-811).  Synchronises with the stream. */
+/* First pass: counts (the reference's "count only" launches, :807-811).  Synchronises with the stream.  n_vertices and n_triangles are
+ * host variables; when both lie in pinned host memory (hipHostMalloc on the current device), a kernel leaves the totals there itself,
+ * which saves a copy's 9 us. */
 int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3],
                             float thresh, const float* d_density, void* d_workspace, uint64_t workspace_bytes,
                             uint32_t* n_vertices, uint32_t* n_triangles);

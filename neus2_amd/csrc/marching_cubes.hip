@@ -26,7 +26,6 @@
 #include "n2_common.h"
 
 #include <cstring>
-#include <mutex>
 
 #pragma clang fp contract(off)
 
@@ -425,7 +424,7 @@ __global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* _
 	McRecord r[MC_EACH];
 	uint32_t nv[MC_EACH], nt[MC_EACH], sum_v = 0, sum_t = 0;
 	const uint32_t row0 = w0 / g.row_words, col0 = w0 - row0 * g.row_words, z0 = row0 / g.ry;
-	uint32_t col = col0, y = row0 - z0 * g.ry, z = z0;
+	uint32_t col = col0, y = row0 - z0 * g.ry;
 #pragma unroll
 	for (uint32_t q = 0; q < MC_EACH; ++q) {
 		nv[q] = nt[q] = 0;
@@ -444,7 +443,7 @@ __global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* _
 			}
 			if (++col == g.row_words) {
 				col = 0;
-				if (++y == g.ry) { y = 0; ++z; }
+				if (++y == g.ry) y = 0;
 			}
 		} else if (w0 + q < g.n_words) {
 			B = mc_load_bits<false>(g, bits, w0 + q);
@@ -529,7 +528,8 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_short_kernel(McGrid g, cons
 // Exclusive prefix sums of the blocks' counts in place; element n_blocks receives the totals.  The blocks that own something are listed, their
 // number goes behind the totals.
 constexpr uint32_t MC_SCAN_EACH = 8;
-__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks, uint32_t* __restrict__ listed, uint32_t* __restrict__ totals) {
+__global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks, uint32_t* __restrict__ listed,
+                                                       uint32_t* to_v, uint32_t* to_t) {
 	__shared__ uint2 wave_sum[16];
 	__shared__ uint32_t wave_n[16];
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -569,7 +569,7 @@ __global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2*
 	if (threadIdx.x == 0) {
 		blocks[n_blocks] = carry;
 		blocks[n_blocks + 1u] = make_uint2(carry_n, 0u);
-		if (totals) { totals[0] = carry.x; totals[1] = carry.y; }
+		if (to_v) { *to_v = carry.x; *to_t = carry.y; }
 	}
 }
 
@@ -897,47 +897,25 @@ static McGrid mc_grid(const uint32_t res[3], const float aabb_min[3], const floa
 	return g;
 }
 
-// Where the scan leaves the totals for the host: slots of one page of pinned memory, each held by a call while it waits.  (Copied to the call's own
-// variables they cost a copy kernel and its staging: 512^3 191 -> 182 us, 64^3 61 -> 53.)  The page stays for the process; where there is none, or
-// every slot is held, the totals are copied.
-class McTotalsSlot {
-public:
-	McTotalsSlot() {
-		std::lock_guard<std::mutex> lock(mutex_);
-		if (!asked_) {
-			asked_ = true;
-			hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (another thread may be capturing: an allocation is no part of that)
-			(void)hipThreadExchangeStreamCaptureMode(&mode);
-			if (hipHostMalloc(reinterpret_cast<void**>(&page_), SLOTS * STRIDE * sizeof(uint32_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-				(void)hipGetLastError();
-				page_ = nullptr;
-			}
-			(void)hipThreadExchangeStreamCaptureMode(&mode);
+// Where the scan can leave the totals by itself: the addresses that a kernel of this device has for the caller's variables when both lie in pinned
+// host memory, else null.
+static void mc_totals_of(uint32_t* n_vertices, uint32_t* n_triangles, uint32_t*& to_v, uint32_t*& to_t) {
+	int device = -1;
+	auto mapped = [&](uint32_t* p) -> uint32_t* {
+		hipPointerAttribute_t attr{};
+		if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+			(void)hipGetLastError();  // (memory that HIP does not know)
+			return nullptr;
 		}
-		for (uint32_t k = 0; page_ && k < SLOTS && !at_; ++k)
-			if (!((held_ >> k) & 1u)) {
-				held_ |= 1u << k;
-				slot_ = k;
-				at_ = page_ + k * STRIDE;
-			}
-	}
-	~McTotalsSlot() {
-		std::lock_guard<std::mutex> lock(mutex_);
-		if (at_) held_ &= ~(1u << slot_);
-	}
-	McTotalsSlot(const McTotalsSlot&) = delete;
-	McTotalsSlot& operator=(const McTotalsSlot&) = delete;
-	uint32_t* get() const { return at_; }
-
-private:
-	static constexpr uint32_t SLOTS = 32, STRIDE = 32;  // a cache line each
-	static inline std::mutex mutex_;
-	static inline uint32_t* page_ = nullptr;
-	static inline uint32_t held_ = 0;
-	static inline bool asked_ = false;
-	uint32_t* at_ = nullptr;
-	uint32_t slot_ = 0;
-};
+		const bool ours = attr.type == hipMemoryTypeHost && attr.device == device && !(attr.allocationFlags & hipHostRegisterReadOnly);
+		return ours ? static_cast<uint32_t*>(attr.devicePointer) : nullptr;
+	};
+	to_v = to_t = nullptr;
+	if (hipGetDevice(&device) != hipSuccess) return;
+	uint32_t* const v = mapped(n_vertices);
+	uint32_t* const t = v ? mapped(n_triangles) : nullptr;
+	if (t) { to_v = v; to_t = t; }
+}
 
 N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,
                                    const float* d_density, void* d_workspace, uint64_t workspace_bytes, uint32_t* n_vertices,
@@ -962,13 +940,15 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	auto* const count_kernel = c.short_rows ? mc_count_short_kernel : mc_count_kernel;
 	count_kernel<<<dim3(c.n_blocks), dim3(c.short_rows ? MC_BLOCK : 64u), 0, s>>>(g, bits, reinterpret_cast<McRecord*>(b + c.records), reinterpret_cast<mc_word*>(b + c.active), blocks);
 	N2_LAUNCH_CHECK();
-	const McTotalsSlot slot;
-	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks, reinterpret_cast<uint32_t*>(b + c.listed), slot.get());
+	// (left there by the scan: 512^3 182 us, 64^3 53; copied, with a copy kernel and its staging, 191 and 61)
+	uint32_t *to_v, *to_t;
+	mc_totals_of(n_vertices, n_triangles, to_v, to_t);
+	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks, reinterpret_cast<uint32_t*>(b + c.listed), to_v, to_t);
 	N2_LAUNCH_CHECK();
 	uint32_t host[2] = {0, 0};
-	if (!slot.get()) N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
+	if (!to_v) N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
 	N2_HIP(hipStreamSynchronize(s));
-	if (slot.get()) memcpy(host, slot.get(), sizeof(host));
+	if (to_v) { host[0] = *n_vertices; host[1] = *n_triangles; }
 	N2_REQUIRE(host[0] < (1u << 29), "n2_marching_cubes_count: %u vertices exceed the 2^29 limit", host[0]);
 	*n_vertices = host[0];
 	*n_triangles = host[1];

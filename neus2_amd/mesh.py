@@ -60,7 +60,8 @@ def marching_cubes(density, thresh, aabb_min=(0, 0, 0), aabb_max=(1, 1, 1), want
     if nbytes == 0:
         raise N2Error("n2_marching_cubes_workspace_bytes: " + L.n2_last_error().decode())
     ws = torch.empty(nbytes, dtype=torch.uint8, device=density.device)
-    nv, nt = C.c_uint32(), C.c_uint32()
+    totals = torch.empty(2, dtype=torch.int32, pin_memory=True)  # pinned: a kernel leaves the totals there by itself, without a copy
+    nv, nt = (C.c_uint32.from_address(totals.data_ptr() + 4 * k) for k in range(2))
     check(L.n2_marching_cubes_count(_stream(), _u3(res), _f3(aabb_min), _f3(aabb_max), C.c_float(thresh), ptr(density), ptr(ws),
                                     C.c_uint64(nbytes), C.byref(nv), C.byref(nt)), "n2_marching_cubes_count")
     verts = torch.empty((nv.value, 3), dtype=torch.float32, device=density.device)

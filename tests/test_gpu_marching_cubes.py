@@ -77,7 +77,7 @@ def test_a_plane_through_every_block_of_words(res):
 
 
 def test_meshes_counted_by_several_threads_at_once():
-    """Each call waits for totals of its own; more calls than there are slots for them."""
+    """Each call waits for totals of its own."""
     from concurrent.futures import ThreadPoolExecutor
 
     from neus2_amd.mesh import marching_cubes
@@ -94,6 +94,31 @@ def test_meshes_counted_by_several_threads_at_once():
             for q, o in enumerate(got):
                 for a, b in zip(o, want[(k + q) % 40]):
                     np.testing.assert_array_equal(a, b)
+
+
+def test_totals_in_pinned_and_in_other_host_memory():
+    """A kernel writes them where both variables are pinned; else they are copied, and nothing beside them is written."""
+    import ctypes as C
+
+    from neus2_amd import capi
+    from neus2_amd.mesh import _f3, _stream, _u3, marching_cubes
+    L = capi.lib()
+    L.n2_marching_cubes_workspace_bytes.restype = C.c_uint64
+    pinned, pageable = torch.empty(24, dtype=torch.int32, pin_memory=True), torch.empty(24, dtype=torch.int32)
+    for k in range(6):
+        f = dev(np.random.default_rng(k).standard_normal((9 + k, 8, 21 + k)).astype(np.float32))
+        v, t, _ = marching_cubes(f, 0.0)
+        res = _u3(f.shape[::-1])
+        nbytes = int(L.n2_marching_cubes_workspace_bytes(res))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        for a, b in ((pinned, pinned), (pageable, pageable), (pinned, pageable), (pageable, pinned)):
+            pinned.fill_(-1)
+            pageable.fill_(-1)
+            at = [C.c_uint32.from_address(a.data_ptr() + 4 * 5), C.c_uint32.from_address(b.data_ptr() + 4 * (11 + k))]
+            capi.check(L.n2_marching_cubes_count(_stream(), res, _f3((0, 0, 0)), _f3((1, 1, 1)), C.c_float(0), capi.ptr(f), capi.ptr(ws),
+                                                 C.c_uint64(nbytes), C.byref(at[0]), C.byref(at[1])), "n2_marching_cubes_count")
+            assert (at[0].value, at[1].value) == (len(v), len(t))
+            assert int((pinned == -1).sum() + (pageable == -1).sum()) == 46
 
 
 def test_empty_lattice_and_errors():
