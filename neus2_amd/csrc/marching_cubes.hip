@@ -157,7 +157,7 @@ __device__ const McRing MC_RING = mc_build_ring();
 // a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 17, scan 9, emit 33, normals 24, with
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 17, scan 8, emit 35, normals 26, with
 // the host's wait for the totals 182 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
@@ -622,15 +622,16 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // lanes, 240 us.  The vertices that a cube uses belong to its own point and to those one further along x, y and z: their
 // slots come from the records of the (at most eight) words those points are in, and stand in LDS, where a triangle's
 // corners pick theirs.  What bounds the launch is the chain of round trips: which words own something, their records (they stay in LDS, for
-// their neighbours in y too), then all that a point needs at once; a cube's case comes from the densities that its vertices need.
-// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 33.)
+// their neighbours in y too), then all that a point needs at once.  A cube's case comes from the bits, as its number of triangles did: whatever
+// the density is by now, a triangle's corners are vertices that this pass writes.
+// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 35; with the case from the density 34.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
 constexpr uint32_t MC_EMIT_GRID = 1536;  // as many as run at a time: six per CU, by their LDS
 typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t mc_words3 __attribute__((ext_vector_type(3), aligned(4)));
 typedef float mc_float2 __attribute__((ext_vector_type(2), aligned(4)));
 template <bool SHORT>
-__global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float* __restrict__ density,
+__global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float* __restrict__ density, const mc_word* __restrict__ bits,
                                                            const McRecord* __restrict__ records, const mc_word* __restrict__ active,
                                                            const uint2* __restrict__ blocks, uint32_t n_blocks, const uint32_t* __restrict__ listed,
                                                            float* __restrict__ verts, uint32_t* __restrict__ indices, uint32_t* __restrict__ origin) {
@@ -672,38 +673,42 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 			const mc_word t0 = tri[0][at0], t1 = tri[1][at0], t2 = tri[2][at0];
 			const McPlace place = mc_place<SHORT>(g, w, p);
 			const uint32_t tris = (uint32_t)((t0 >> p) & 1ull) | (uint32_t)((t1 >> p) & 1ull) << 1 | (uint32_t)((t2 >> p) & 1ull) << 2;
-			// the point's density and those at +1 along x, in the four rows of its cube (where they are not there, those of the last row or plane)
-			const uint32_t x0 = min(place.x, g.rx - 2u);
-			float low[4], high[4];
+			// The point's density and its neighbours' (where there is none, another one), and the bits of the point and of the next along x in the
+			// four rows of its cube (the cubes of the last column, row and plane have no triangles: any bits).
+			const uint32_t x0 = min(place.x, g.rx - 2u), y1 = min(place.y + 1u, g.ry - 1u), z1 = min(place.z + 1u, g.rz - 1u);
+			const mc_float2 along = *reinterpret_cast<const mc_float2*>(density + ((uint64_t)place.z * g.ry + place.y) * g.rx + x0);
+			const float f0 = place.x == x0 ? along.x : along.y;
+			const float f1[3] = {along.y, density[((uint64_t)place.z * g.ry + y1) * g.rx + place.x], density[((uint64_t)z1 * g.ry + place.y) * g.rx + place.x]};
+			uint32_t at[4], bit[4], pair[4];
 #pragma unroll
 			for (uint32_t j = 0; j < 4; ++j) {
-				const uint32_t y = min(place.y + (j & 1u), g.ry - 1u), z = min(place.z + (j >> 1), g.rz - 1u);
-				const mc_float2 v = *reinterpret_cast<const mc_float2*>(density + ((uint64_t)z * g.ry + y) * g.rx + x0);
-				low[j] = place.x == x0 ? v.x : v.y;
-				high[j] = v.y;
+				at[j] = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u);
+				bit[j] = p;
+				if (SHORT) {
+					bit[j] = (j & 1u) ? p + (1u << g.pitch_log) : p;
+					at[j] = w + (bit[j] >> MC_SHORT_BITS_LOG) + ((j & 2u) ? g.plane_words : 0u);
+					bit[j] &= (1u << MC_SHORT_BITS_LOG) - 1u;
+				}
+				// (eight bytes from the 32 bits that the point is in; behind the last word the records follow)
+				const mc_words2 two = *reinterpret_cast<const mc_words2*>(reinterpret_cast<const uint32_t*>(bits) + 2u * min(at[j], g.n_words - 1u) + (bit[j] >> 5));
+				pair[j] = (uint32_t)(((uint64_t)two.y << 32 | two.x) >> (bit[j] & 31u)) & 3u;
 			}
-			if (tris) {  // (the cubes of the last column, row and plane have no triangles: the points below exist)
+			if (tris) {  // (the points one further along x, y and z exist)
 #pragma unroll
 				for (uint32_t j = 0; j < 4; ++j) {
-					uint32_t at = w + ((j & 1u) ? g.row_words : 0u) + ((j & 2u) ? g.row_words * g.ry : 0u), bit = p;
-					if (SHORT) {
-						bit = (j & 1u) ? p + (1u << g.pitch_log) : p;
-						at = w + (bit >> MC_SHORT_BITS_LOG) + ((j & 2u) ? g.plane_words : 0u);
-						bit &= (1u << MC_SHORT_BITS_LOG) - 1u;
-					}
-					const McOwned o = j == 0 ? own : owned(at);
-					slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, bit);
-					slot_of[2 * j + 1][threadIdx.x] = bit < 63u ? mc_vertex_slot(o, bit + 1u) : mc_vertex_slot(owned(at + 1u), 0u);
+					const McOwned o = j == 0 ? own : owned(at[j]);
+					slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, bit[j]);
+					slot_of[2 * j + 1][threadIdx.x] = bit[j] < 63u ? mc_vertex_slot(o, bit[j] + 1u) : mc_vertex_slot(owned(at[j] + 1u), 0u);
 				}
 			}
 			const uint32_t slot0 = mc_vertex_slot(own, p), flags = slot0 >> 29;
 			if (flags) {
-				const float pos[3] = {(float)place.x, (float)place.y, (float)place.z}, f1[3] = {high[0], low[1], low[2]};
+				const float pos[3] = {(float)place.x, (float)place.y, (float)place.z};
 				uint32_t slot = slot0 & 0x1FFFFFFFu;
 #pragma unroll
 				for (uint32_t a = 0; a < 3; ++a) {
 					if (!((flags >> a) & 1u)) continue;
-					const float dt = (g.thresh - low[0]) / (f1[a] - low[0]);
+					const float dt = (g.thresh - f0) / (f1[a] - f0);
 					n2_float3 v;
 #pragma unroll
 					for (uint32_t d = 0; d < 3; ++d) v[d] = (d == a ? pos[d] + dt : pos[d]) * g.scale[d] + g.offset[d];
@@ -714,10 +719,8 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 			}
 			if (tris == 0) return;
 			const uint32_t first_t = first[at0].y + mc_below(t0, p) + 2u * mc_below(t1, p) + 4u * mc_below(t2, p);
-			const float corner[8] = {low[0], high[0], high[1], low[1], low[2], high[2], high[3], low[3]};
-			uint32_t mask = 0;
-#pragma unroll
-			for (uint32_t k = 0; k < 8; ++k) mask |= corner[k] > g.thresh ? 1u << k : 0u;
+			auto turned = [](uint32_t two) { return two >> 1 | (two & 1u) << 1; };  // (corners run round a face)
+			const uint32_t mask = pair[0] | turned(pair[1]) << 2 | pair[2] << 4 | turned(pair[3]) << 6;
 			// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
 			// the owner's offset from this point in x, y, z and the edge's axis.
 			constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
@@ -751,7 +754,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 // The triangles' other corners are worked out again from the density, by the arithmetic that placed them: the eighteen values of the four
 // cubes tell which triangles there are (MC_RING) and where their corners lie.  That is 18 loads a vertex and vector instructions; going
 // through the words' records to the triangles and from those to the vertices was some 45 loads, most of them lines of their own, one a
-// clock and CU: 34 us for 512^3, now 24.
+// clock and CU: 34 us for 512^3, now 26.
 template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const float* __restrict__ density, float* __restrict__ normals) {
 	__shared__ float values[18][MC_BLOCK];  // [slow -1 .. 1][fast -1 .. 1][along 0, 1]
@@ -972,7 +975,7 @@ N2_API int n2_marching_cubes_emit(n2_stream_t stream, const uint32_t res[3], con
 	const uint2* blocks = reinterpret_cast<const uint2*>(b + c.blocks);
 	const McGrid g = mc_grid(res, aabb_min, aabb_max, thresh);
 	auto* const emit_kernel = c.short_rows ? mc_emit_kernel<true> : mc_emit_kernel<false>;
-	emit_kernel<<<dim3(c.n_blocks < MC_EMIT_GRID ? c.n_blocks : MC_EMIT_GRID), dim3(MC_BLOCK), 0, s>>>(g, d_density, records, active, blocks, c.n_blocks, reinterpret_cast<const uint32_t*>(b + c.listed), d_vertices, d_indices,
+	emit_kernel<<<dim3(c.n_blocks < MC_EMIT_GRID ? c.n_blocks : MC_EMIT_GRID), dim3(MC_BLOCK), 0, s>>>(g, d_density, reinterpret_cast<const mc_word*>(b + c.bits), records, active, blocks, c.n_blocks, reinterpret_cast<const uint32_t*>(b + c.listed), d_vertices, d_indices,
 	                                                        reinterpret_cast<uint32_t*>(d_normals));
 	N2_LAUNCH_CHECK();
 	if (d_normals) {

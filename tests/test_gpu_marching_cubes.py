@@ -96,6 +96,32 @@ def test_meshes_counted_by_several_threads_at_once():
                     np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("res", [(70, 9, 11), (192, 5, 4), (64, 3, 2), (7, 9, 11), (15, 6, 5)])  # rows that end inside a word and with one, shared words
+def test_triangles_are_those_of_the_counted_density(res):
+    """The second pass with another density and threshold moves vertices; its triangles stay those that the first pass counted."""
+    import ctypes as C
+
+    from neus2_amd import capi
+    from neus2_amd.mesh import _f3, _stream, _u3, marching_cubes
+    L = capi.lib()
+    L.n2_marching_cubes_workspace_bytes.restype = C.c_uint64
+    rng = np.random.default_rng(sum(res))
+    f, other = (dev(rng.standard_normal(res[::-1]).astype(np.float32)) for _ in range(2))
+    v, t, _ = marching_cubes(f, 0.1)
+    assert 0 <= int(t.min()) and int(t.max()) < len(v)
+    nbytes = int(L.n2_marching_cubes_workspace_bytes(_u3(res)))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    box = _u3(res), _f3((0, 0, 0)), _f3((1, 1, 1))
+    for density, thresh in ((f, 0.1), (f, 0.7), (other, 0.1), (torch.zeros_like(f), 0.0)):
+        nv, nt = C.c_uint32(), C.c_uint32()
+        capi.check(L.n2_marching_cubes_count(_stream(), *box, C.c_float(0.1), capi.ptr(f), capi.ptr(ws), C.c_uint64(nbytes), C.byref(nv), C.byref(nt)), "count")
+        verts, normals = (torch.empty((nv.value, 3), device="cuda") for _ in range(2))
+        idx = torch.full((nt.value, 3), -1, dtype=torch.int32, device="cuda")
+        capi.check(L.n2_marching_cubes_emit(_stream(), *box, C.c_float(thresh), capi.ptr(density), capi.ptr(ws), capi.ptr(verts), capi.ptr(idx), capi.ptr(normals), nv, nt), "emit")
+        assert torch.equal(idx, t)
+        assert torch.equal(verts, v) == (density is f and thresh == 0.1)
+
+
 def test_totals_in_pinned_and_in_other_host_memory():
     """A kernel writes them where both variables are pinned; else they are copied, and nothing beside them is written."""
     import ctypes as C
