@@ -570,14 +570,14 @@ constexpr unsigned long long ROW_HEADS = 0x0001000100010001ull;  // first lane o
 
 // r += take * (r of the lane D places below in the same 16-lane row; 0 if that leaves the row), for the sixteen values of a point.
 // (Written out: the compiler makes a move with the lane shift, a wait state and a multiply-add of each.  s_nop: a lane shift must not
-// read what one of the two instructions before it wrote.)
+// read what one of the two instructions before it wrote.  &: `take` is read after the first values are written, so no value may share its register.)
 template <int D>
 __device__ __forceinline__ void n2_row_add(float (&a)[8], float (&b)[8], const float take) {
 #define N2_ROW_ADD(K) "v_fmac_f32_dpp %" #K ", %" #K ", %16 row_shr:%17 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
 	asm("s_nop 1\n\t" N2_ROW_ADD(0) N2_ROW_ADD(1) N2_ROW_ADD(2) N2_ROW_ADD(3) N2_ROW_ADD(4) N2_ROW_ADD(5) N2_ROW_ADD(6) N2_ROW_ADD(7)
 	    N2_ROW_ADD(8) N2_ROW_ADD(9) N2_ROW_ADD(10) N2_ROW_ADD(11) N2_ROW_ADD(12) N2_ROW_ADD(13) N2_ROW_ADD(14) N2_ROW_ADD(15) "s_nop 0"
-	    : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),
-	      "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4]), "+v"(b[5]), "+v"(b[6]), "+v"(b[7]) : "v"(take), "n"(D));
+	    : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]),
+	      "+&v"(b[0]), "+&v"(b[1]), "+&v"(b[2]), "+&v"(b[3]), "+&v"(b[4]), "+&v"(b[5]), "+&v"(b[6]), "+&v"(b[7]) : "v"(take), "n"(D));
 #undef N2_ROW_ADD
 }
 // sum over the lanes up to this one (all 64 lanes active): lane shifts inside the rows of 16, then the rows' totals
