@@ -447,11 +447,7 @@ constexpr uint32_t BKT_MIN_SHIFT = 5;                  // smallest bucket of a l
 constexpr uint32_t PAIR_MAX_CELL = BKT_ENTRIES - 2u;  // pair records (grid_bin_kernel): x + 1 <= BKT_ENTRIES - 1
 static_assert(BKT_SHIFT <= 12, "a pair record's 16-bit key holds the entry within the bucket and four bits of carry length");
 constexpr uint32_t BIN_BLOCK = 512;       // 8 waves: three workgroups (3 x 49 KiB of LDS) keep 6 waves on every SIMD, at 80 registers (with 96 or 128: pair +10 us)
-// Points per thread of a bin workgroup (a tile: BIN_BLOCK * per points, eight records each).  Two, and one for batches whose tiles of two would not
-// give every CU a workgroup: those wait for one workgroup's chain of round trips, which is shorter for one point (5003 points: first order
-// 7.1 -> 5.5 us, second order with its output 14.5 -> 9.7; 12000 uniform points 9 -> 8; 16384 samples 7.9 -> 6.1, and the summing kernel, which has twice the runs, 16.6 -> 17.5).
-constexpr uint32_t BIN_HALF_POINTS = 16384;
-__host__ __device__ constexpr uint32_t bin_per_thread(uint32_t n_points) { return n_points <= BIN_HALF_POINTS ? 1u : 2u; }
+// Points per thread of a bin workgroup (a tile: BIN_BLOCK * per points, eight records each): n2_bin_points_per_thread.
 __host__ __device__ constexpr uint32_t bin_points(uint32_t per) { return BIN_BLOCK * per; }
 __host__ __device__ constexpr uint32_t bin_records(uint32_t per) { return bin_points(per) * 8u; }
 
@@ -1234,8 +1230,9 @@ static int prepare_grads(n2_grid_t* grid, const char* fn, hipStream_t stream, n2
 }
 
 static inline uint32_t n_pair_tiles(uint32_t n_points) { return (n_points + PAIR_POINTS - 1) / PAIR_POINTS; }
-static inline uint32_t n_bin_tiles(uint32_t n_points) {
-	const uint32_t points = bin_points(bin_per_thread(n_points));
+static inline uint32_t bin_per_thread(const n2_grid_t* grid, uint32_t n_points) { return n2_bin_points_per_thread(grid->tab.n_levels, n_points, BIN_BLOCK); }
+static inline uint32_t n_bin_tiles(const n2_grid_t* grid, uint32_t n_points) {
+	const uint32_t points = bin_points(bin_per_thread(grid, n_points));
 	return (n_points + points - 1) / points;
 }
 
@@ -1251,8 +1248,8 @@ struct BucketCarve {
 };
 static uint32_t split_images(const n2_grid_t* grid, uint32_t n_points);
 static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points) {
-	const uint64_t tiles = n_bin_tiles(max_points), L = grid->tab.n_levels;
-	const uint64_t n_rec = L * tiles * bin_records(bin_per_thread(max_points));
+	const uint64_t tiles = n_bin_tiles(grid, max_points), L = grid->tab.n_levels;
+	const uint64_t n_rec = L * tiles * bin_records(bin_per_thread(grid, max_points));
 	auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
 	BucketCarve c{};
 	c.vals = 0;
@@ -1260,7 +1257,8 @@ static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points) {
 	c.offsets = c.keys + n_rec * sizeof(uint16_t);
 	c.partials = up(c.offsets + L * tiles * (BKT_MAX + 1) * sizeof(uint16_t));
 	// (a batch of half as many points per tile has twice the tiles and bucket offsets: the images of a larger one stand behind those, too)
-	if (max_points > BIN_HALF_POINTS) c.partials = std::max(c.partials, bucket_carve(grid, BIN_HALF_POINTS).partials);
+	const uint32_t largest = n2_bin_single_points(grid->tab.n_levels, BIN_BLOCK);
+	if (max_points > largest) c.partials = std::max(c.partials, bucket_carve(grid, largest).partials);
 	c.total = up(c.partials + (uint64_t)split_images(grid, max_points) * BKT_ENTRIES * sizeof(float2));
 	return c;
 }
@@ -1307,7 +1305,7 @@ static uint32_t bucket_groups(const n2_grid_t* grid, uint32_t level, uint32_t n_
 
 // fp32 images of all split buckets of a batch (never more for a smaller batch: the groups per bucket grow with the batch)
 static uint32_t split_images(const n2_grid_t* grid, uint32_t n_points) {
-	const uint32_t tiles = n_bin_tiles(n_points);
+	const uint32_t tiles = n_bin_tiles(grid, n_points);
 	uint32_t n = 0;
 	for (uint32_t l = 0; l < grid->tab.n_levels; ++l) {
 		const uint32_t nb = level_buckets(grid, l, n_points), groups = bucket_groups(grid, l, n_points, tiles);
@@ -1340,7 +1338,7 @@ N2_API int n2_grid_set_workspace(n2_grid_t* grid, void* d_workspace, uint64_t n_
 static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
                            const __half* dL_dy, const float* v, const __half* g2, __half* dL_ddLdy, bool accumulate,
                            const uint32_t* index, uint32_t n_cols) {
-	const uint32_t tiles = n_bin_tiles(n_points), per = bin_per_thread(n_points), L = grid->tab.n_levels;
+	const uint32_t tiles = n_bin_tiles(grid, n_points), per = bin_per_thread(grid, n_points), L = grid->tab.n_levels;
 	const bool first = dL_dy != nullptr, second = v != nullptr, out = dL_ddLdy != nullptr;
 	const dim3 bd(BIN_BLOCK);
 	// The records of this batch are packed as for a workspace of exactly this size (values, keys, offsets one behind the

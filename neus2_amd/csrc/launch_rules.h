@@ -21,6 +21,19 @@ static inline bool n2_moments_stream(uint64_t state_bytes, uint64_t batch) {
 	return state_bytes + N2_STEP_BYTES_PER_SAMPLE * batch > N2_LAST_LEVEL_CACHE_BYTES;
 }
 
+// Points per thread of the scatter's sorting kernel.  Three of its workgroups share a CU, 768 run at a time.  One point per thread where all workgroups
+// (levels x tiles) then start together: the launch takes one workgroup's chain of round trips, which is shorter for one point.  Beyond, a
+// workgroup of two points per thread takes less than two of one, and the summing kernel finds half as many runs.  Both kernels in us, one | two:
+//   16 levels (768: 24 576 points): uniform 8192 21.7 | 25.2, 16 384 25.1 | 26.8, 20 480 28.7 | 28.9, 24 576 30.0 | 30.0, 32 768 33.4 | 31.8, 52 344 40.4 | 38.0, 2^17 63 | 56
+//     rays 8192 20.3 | 22.2, 16 384 23.3 | 23.5, 20 480 25.8 | 25.4, 24 576 27.2 | 26.8, 32 768 31.7 | 29.0; training step 16 384 134.7 | 135.9, 24 576 154.0 | 153.7,
+//     32 768 153.7 | 151.6; field 16 384 55.8 | 57.2, 24 576 62.5 | 62.8, 32 768 68.4 | 67.6, 49 152 85.8 | 82.9
+//   8 levels (49 152): uniform 32 768 21.4 | 22.2, 49 152 25.3 | 24.9, 52 344 26.5 | 25.5, 2^17 40 | 37; rays 24 576 15.0 | 15.7, 32 768 16.7 | 16.2, 49 152 18.9 | 17.8
+//   4 levels (98 304): uniform 65 536 20.3 | 20.9, 98 304 24.4 | 24.8, 2^17 28.7 | 28.6; rays 65 536 12.6 | 12.9, 98 304 14.8 | 15.9, 2^17 18.2 | 18.0
+constexpr uint32_t N2_BIN_AT_A_TIME = 768;
+// the largest batch that takes one
+static inline uint32_t n2_bin_single_points(uint32_t n_levels, uint32_t block) { return N2_BIN_AT_A_TIME / n_levels * block; }
+static inline uint32_t n2_bin_points_per_thread(uint32_t n_levels, uint32_t n_points, uint32_t block) { return n_points <= n2_bin_single_points(n_levels, block) ? 1u : 2u; }
+
 // The part of a lattice that one launch of its kernels takes: columns, rows and planes (lattice.hip).
 struct N2LatticeSlab {
 	uint32_t nx, ny, nz;

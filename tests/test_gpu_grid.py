@@ -341,6 +341,32 @@ def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and bool((got[0][0] != 0).any())
 
 
+# the last batch of one point per thread and the next one, workspaces that are just large enough and larger; buckets of up to 65536 records are whole
+@pytest.mark.parametrize("levels,log2_size,line,whole", [(16, 19, 24576, True), (7, 16, 55808, True), (7, 14, 55808, False), (2, 6, 196608, False)])
+def test_sorted_scatter_at_the_line_between_the_tiles(levels, log2_size, line, whole):
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(**{**CFG, "n_levels": levels, "log2_hashmap_size": log2_size})
+    gen = torch.Generator(device="cuda").manual_seed(levels)
+    dp = (torch.rand(gg.n_params(), device="cuda", generator=gen) * 2 - 1).half()
+    dg = torch.zeros_like(dp)
+    gg.set_params(dp, dg)
+    x = torch.rand((3, line + 1), device="cuda", generator=gen)
+    dy, g2, v = (torch.randn((w, line + 1), device="cuda", generator=gen) for w in (2 * levels, 2 * levels, 3))
+    dy[:, line:] = 0
+    g2[:, line:] = 0
+    got = []
+    for points, space in ((line, line), (line, line + 1), (line + 1, line + 1)):
+        assert gg.reserve_scatter_workspace(space)
+        dg.fill_(9.0)
+        gg.backward_fused(x[:, :points].contiguous(), dy[:, :points].half().contiguous(), v[:, :points].contiguous(), g2[:, :points].half().contiguous(), want_dL_ddLdy=False, mode=GRAD_OVERWRITE)
+        got.append(dg.clone())
+    assert torch.equal(got[0], got[1]) and bool((got[0] != 0).any()) and bool(torch.isfinite(got[0].float()).all())
+    if whole:
+        assert torch.equal(got[0], got[2])
+    else:  # fp32 images of a bucket's parts, and other tiles make other parts: some entries round to the next fp16 number, 2^-10 of the entry away
+        assert float((got[0].float() - got[2].float()).norm() / got[2].float().norm()) < 2 ** -10
+
+
 @pytest.mark.parametrize("kind", ["uniform", "clustered", "rays"])
 def test_sorted_scatter_path(oracle, kind):
     """With a scatter workspace, batches go through the run-length kernel (coarsest levels) and the

@@ -31,6 +31,8 @@ extern "C" void lattice_chunks(uint32_t first, uint32_t last, uint32_t* out) { n
 extern "C" uint32_t walked_levels(const float* scale, float step) { return n2_lattice_walked_levels(scale, step); }
 extern "C" uint32_t row_levels(const float* scale, uint32_t nx, float step_x, float reach, float step_z) { return n2_lattice_row_levels(scale, nx, step_x, reach, step_z); }
 extern "C" int by_rows(uint32_t rows, uint32_t walked, uint64_t points) { return n2_lattice_by_rows(rows, walked, points); }
+extern "C" uint32_t bin_points_per_thread(uint32_t levels, uint32_t n) { return n2_bin_points_per_thread(levels, n, 512); }
+extern "C" uint32_t bin_single_points(uint32_t levels) { return n2_bin_single_points(levels, 512); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
 
@@ -144,3 +146,10 @@ def test_runs_of_the_levels_walked_by_rows_fit_a_wave(rules, nx, lo, hi, planes,
                                                      (8, 10, 256 * 256 * 512, 1), (10, 10, 512 ** 3, 1), (0, 6, 1 << 31, 0), (3, 6, 1 << 31, 0)])
 def test_which_lattices_are_walked_by_rows(rules, rows, walked, points, want):
     assert rules.by_rows(C.c_uint32(rows), C.c_uint32(walked), C.c_uint64(points)) == want
+
+
+@pytest.mark.parametrize("levels", [1, 4, 5, 8, 16, 32])
+def test_one_point_per_thread_while_all_sorting_workgroups_run_at_once(rules, levels):
+    line = rules.bin_single_points(C.c_uint32(levels))
+    assert levels * (line // 512) <= 768 < levels * (line // 512 + 1) and line % 512 == 0
+    assert [rules.bin_points_per_thread(C.c_uint32(levels), C.c_uint32(n)) for n in (1, line, line + 1, 1 << 31)] == [1, 1, 2, 2]
