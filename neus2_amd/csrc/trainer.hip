@@ -318,6 +318,9 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 		                                         t->cfg.composite.background, t->bitfield, n_inference, set.counters, set.counters + 1, set.ray_indices,
 		                                         set.numsteps, set.rgb_target, set.coords, set.ws_sampler, t->ws_sampler_bytes, want_rows ? set.xyz_rows : nullptr);
 	};
+	// (ev_main stands for a step's end from its Adam launch on: a step that fails before it has put kernels on the stream behind the event)
+	const bool main_event_from_adam = t->ev_main_from_adam;
+	t->ev_main_from_adam = false;
 	// the following step's samples on the side stream, assuming the same ray count and the next seed
 	bool main_event_is_last_step = false;
 	auto prefetch = [&](uint32_t cur_set) -> int {
@@ -340,7 +343,7 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 			cur = t->pf_set;
 			// ev_main stands for the last step's Adam launch: enough unless the caller may have put readers of that step's
 			// buffers on the stream since (it asked for the view), or this step runs on another stream
-			main_event_is_last_step = t->ev_main_from_adam && !t->view_taken && s == t->last_stream;
+			main_event_is_last_step = main_event_from_adam && !t->view_taken && s == t->last_stream;
 			// (the last step has left the wait in front of its Adam launch)
 			if (!t->ready_awaited || s != t->last_stream) N2_HIP(hipStreamWaitEvent(s, t->ev_ready, 0));
 		} else {

@@ -182,6 +182,41 @@ def test_steps_on_changing_streams_wait_for_the_samples_generated_ahead():
     np.testing.assert_array_equal(runs[0][1], runs[1][1])
 
 
+def test_steps_after_one_that_failed_halfway():
+    """Depth rounds need the fused kernels: without them a step fails behind the start of the generation that runs ahead, and behind kernels of its
+    own that read the sample set which the following step's generation overwrites."""
+    import ctypes as C
+
+    from neus2_amd import capi
+    from neus2_amd.capi import N2Error
+    from neus2_amd.tcnn_api import pack_cameras
+    from neus2_amd.training import Trainer, default_config
+    cams = scene.cameras_on_sphere(6, 64)
+    d_cams, d_rgba, d_bits = pack_cameras(cams), dev(scene.render_sphere_images(cams)), dev(scene.sphere_bitfield())
+    T = 2048
+    runs = []
+    for ahead in (False, True):
+        tr = Trainer(default_config(target_batch_size=T, max_rays_per_batch=512, max_samples=16 * T, prefetch_samples=ahead))
+        tr.set_scene(d_cams, len(cams), d_rgba, d_bits)
+        tr.initialize_params(seed=5, sdf_mlp_weights=None)
+        log = []
+        for seed in range(8):
+            if seed in (3, 4):
+                capi.check(capi.lib().n2_field_set_fused(tr._field, C.c_int(0)))
+                tr.set_depth_chunks(8, 3)
+                with pytest.raises(N2Error, match="fused"):
+                    tr.step(n_rays=200, n_inference=16 * T, seed=seed)
+                tr.set_depth_chunks(0, 0)
+                capi.check(capi.lib().n2_field_set_fused(tr._field, C.c_int(1)))
+            else:
+                tr.step(n_rays=200, n_inference=16 * T, seed=seed)
+                log.append(tr.read_counters())
+        runs.append((log, host(tr.master).copy()))
+        del tr
+    assert runs[0][0] == runs[1][0] and all(c["rays"] > 0 for c in runs[0][0])
+    np.testing.assert_array_equal(runs[0][1], runs[1][1])
+
+
 def test_a_step_under_capture_is_refused_and_leaves_no_trace():
     """Samples generated ahead do not fit into a captured step: it is refused, whether it would find them (the next seed) or not, and the
     steps around it are those of a run without it."""
