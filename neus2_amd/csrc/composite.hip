@@ -68,8 +68,8 @@ __device__ __forceinline__ float lane_of(float none, float x) {
 	return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(none), __float_as_int(x), CTRL, ROWS, 0xF, false));
 }
 // Scans over the 64 lanes: inside the rows of 16 by lane shifts, then a row's last lane on to the next row (rows 1 and 3), then lane 31's
-// on to rows 2 and 3.  (By the LDS crossbar every step was a trip of a hundred cycles: forward and backward 11.0 and 16.2 us for 5000 rays,
-// now 10.6 and 14.6, and 6.6 and 9.6 for 300, now 5.9 and 7.8.)
+// on to rows 2 and 3.  (By the LDS crossbar every step was a trip of a hundred cycles: forward and backward 8.5 and 15.4 us for 5000 rays,
+// now 8.1 and 13.9, and 6.3 and 9.7 for 300, now 5.6 and 7.8.)
 template <class Op>
 __device__ __forceinline__ float wave_scan(float v, float none, Op op) {
 	v = op(v, lane_of<0x111>(none, v));
@@ -443,7 +443,7 @@ constexpr float CHUNK_T_EPS = 0.5f * T_EPS;
 constexpr uint32_t CHUNK_BLOCK = 1024, CHUNK_LANES = 16, CHUNK_RAYS = CHUNK_BLOCK / CHUNK_LANES;
 
 // The launch is a chain of round trips: what goes by the ray's number is fetched together, then its direction with its first samples, and a listed sample's
-// ray is searched once, not again for each of its seven coordinates (15.0 -> 10.8 us for 36 000 rays, three times a step).
+// ray is searched once, not again for each of its seven coordinates (13.0 -> 10.1 us for 36 000 rays, three times a step).
 // One ray per sixteen lanes (a row of the data-parallel lane operations): the lanes take the ray's samples sixteen at a
 // time.  coords_listed receives the coordinate rows of the listed samples in list order, so that the field's kernels read
 // their input without going through the list.

@@ -269,7 +269,7 @@ __device__ __forceinline__ void sh4(float x, float y, float z, float* o) {
 
 // Full field: one (sample, level) item, features and slopes; the item is column i of the matrices, and its
 // coordinates are row i of the input (the [N][7] coordinates, or three rows of positions).  (2^18 samples of a training step: one lane per sample
-// with eight gathers 68.9 us, lane pairs with adjacent samples 72, with samples 32 apart 66.3; a trained state's step 509.5 -> 504.2.)
+// with eight gathers 66.0 us, lane pairs with samples 32 apart 63.8, with adjacent samples slower than either; a trained state's step 509.5 -> 504.2.)
 __device__ __forceinline__ void gather_item(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t end) {
 	const uint32_t N = a.N, at = min(i, end - 1u);  // (lanes behind the last sample take part in its pair's exchange)
 	// (full field: the positions from the coordinate rows, or from three rows of their own when the caller has them: a wave
@@ -409,10 +409,11 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_list_kernel(const Fused
 
 template <bool FULL>
 __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs a, uint32_t tiles, int by_xcd) {
-	// Bound by lines on their way from the L2s to the L1s (n2_encode_level): a query of 2^20 uniform points takes one in every 2.6 clocks of
-	// a CU, four per point on every level above the coarsest, and the address units are busy in 95 % of the clocks; the samples of a
-	// training step share lines along their rays (one every 4.7, address units busy in 76 %) but also hold the vector unit in 41 % of the
-	// cycles for their slopes: without its gathers the launch would still take 46 of 66 us.  Measured on the training
+	// Bound by the L1s (n2_encode_level): a query of 2^20 uniform points takes a line in from the L2 in every 2.7 clocks of a CU, four per
+	// point on every level above the coarsest, with the address units busy in 93 % of the clocks; points in the order of the occupancy grid's
+	// cells share lines on the coarse levels (35 a point, one every 3.2 clocks) and look one up in every clock.  The samples of a
+	// training step share lines along their rays (one every 5.2, a lookup every 1.65, address units busy in 66 %) but also hold the vector unit
+	// in 54 % of the cycles for their slopes: without its gathers the launch would still take 46 of 66 us.  Measured on the training
 	// step and dropped: loads of the hashed levels that bypass the L1 (agent- or system-scope: +27 us, the x neighbour's line is then
 	// requested twice and a request is no cheaper) or carry the non-temporal hint (no change), the positions read as consecutive words
 	// and picked apart in LDS (+9).
@@ -597,7 +598,7 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 	const uint32_t n_tiles = (n_live + 31u) / 32u;
 	const uint32_t wave_gid = blockIdx.x * (FF_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (FF_BLOCK / 64);
 	// FULL: what a tile starts with (features, coordinates, place in the output); the next tile's is under way while the current one is computed, the
-	// first one's beside the weights.  (2^18 samples 35.7 -> 33 us, a round of the depth rounds 17 -> 14.6: two waves a SIMD hide little, and the loads of a tile also waited for the
+	// first one's beside the weights.  (2^18 samples 37.1 -> 33.0 us, the weights' copies included, a depth round 16.0 -> 13.4: two waves a SIMD hide little, and the loads of a tile also waited for the
 	// stores of the last one.  Three workgroups per CU at 168 registers spill.)
 	struct Start {
 		hf feat[16];

@@ -598,8 +598,8 @@ constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 
 // What a workgroup takes is its chain of waits (three share a CU, and the vector units are busy two thirds of the time): loads, counter
 // updates and prefix look-ups are therefore issued together, and nothing waits in a branch.  With each of them awaited where it was used,
-// and the second point's loads behind the first one's counters: training step at 2^18 samples 57 us, now 48; 2^18 uniform points 47, now 43;
-// 52344 samples 15.2, now 12.6.
+// and the second point's loads behind the first one's counters: training step at 2^18 samples 69 us, now 59 (57 and 47 on another card); trained 58, now 51; 2^18 uniform points
+// 51.5, now 47.8; 52344 samples 15.1, now 12.7.
 template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT, bool PAIR>
 __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uint32_t level, const uint32_t tile, uint32_t N, uint32_t tiles,
                                               const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
@@ -815,7 +815,8 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const uin
 	const uint16_t* off = offsets + level_tile0 * (BKT_MAX + 1) + it.bucket;
 	const uint32_t step = groups * it.groups;  // (a split bucket's workgroup takes the tiles it.group, it.group + it.groups, ...)
 	// Where the next step's records are; the bounds of the run behind it are on their way, two 16-bit offsets as they lie in memory: taken apart
-	// where they are loaded, they were waited for there, and with them all records under way (2^18 samples: 51.6 -> 50.2 us, 2^18 uniform points 58 -> 55.5).
+	// where they are loaded, they were waited for there, and with them all records under way (2^18 uniform points 52.2 -> 50.5 us,
+	// a trained step 47 -> 44.6, 5003 points 17.1 -> 15.5; a training step in its initial state 55 before and after, the SDF network's 64.6).
 	uint32_t tile = group * it.groups + it.group, i, end;
 	auto bounds = [&](uint32_t t) {
 		uint32_t two;

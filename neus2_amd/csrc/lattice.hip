@@ -13,10 +13,10 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.8 ms, per slab of 7.6e6 points 142 us for six fine levels and 135 us for the walk.  Before: 5.76, 154 and 180, with
+// 512^3 lattice 4.8 ms, per slab of 7.6e6 points 140 us for six fine levels and 130 us for the walk.  Before: 5.76, 148 and 176, with
 // vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  The fine levels are held by the L1's
-// data return (busy in 89 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (58 %) and by
-// the features, which come from beyond the L2.
+// data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and by
+// the features, which come from beyond the L2 (28 % hits).
 // Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before | now: 80^3 86 | 81 us, 128^3 187 | 176, 208^3 654 | 595,
 // 256^3 1008 | 890, 320^3 1750 | 1605, 400^3 3410 | 2925, 464^3 5130 | 4550, 512 x 64 x 512 752 | 625, 64 x 512 x 512 1672 | 1624.
 #include "n2_common.h"
@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_frags_kernel(const LatticeAr
 // banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks per 4-byte load).  So the wave loads the rows as a
 // whole, 2, 4 or 8 entries per lane as the run's length asks for, and weighs the four rows against each other where they are, in
 // registers; what remains is one row, which goes through LDS (in fp32, a slot left out after every 32 entries so that lanes any
-// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 25 % of the
+// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 39 % of the
 // clocks; 73 % when the eight vertices were picked there).  Runs longer than that (coarse lattices) and dense levels gather from memory.
 constexpr uint32_t FINE_CHUNKS = 128;  // chunks of four entries a row may have
 constexpr uint32_t FINE_SLOTS = FINE_CHUNKS * 4u + FINE_CHUNKS / 8u;
@@ -326,7 +326,7 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 }
 
 // The walk.  NM levels are interpolated here, the others come from a.features.  A row of a walked level's vertices that a run of 64
-// points meets fits the wave's lanes (n2_lattice_walked_levels): lane v holds vertex v of the run, the two rows of a plane are loaded
+// points meets fits the wave's lanes (n2_lattice_row_levels): lane v holds vertex v of the run, the two rows of a plane are loaded
 // as consecutive words and interpolated in y there, and the points pick their two neighbours through LDS.
 template <int NM>
 __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const LatticeArgs a) {

@@ -157,7 +157,7 @@ __device__ const McRing MC_RING = mc_build_ring();
 // a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 80 (6.7 TB/s), count 17, scan 8, emit 35, normals 26, with
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 81 (6.6 TB/s), count 16, scan 8, emit 34, normals 26, with
 // the host's wait for the totals 182 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
@@ -392,7 +392,7 @@ __device__ __forceinline__ void mc_own(const McBits& B, McRecord& r, uint32_t& n
 
 // One wave per block of 256 words, four consecutive words per lane: with their neighbours in y and z four loads of 32 bytes, and nothing to
 // wait for but these.  (A lane per word in workgroups of four waves, with a table of triangle numbers in LDS: four rounds of workgroups that
-// each waited for the table, the bits and each other, 30 us for 512^3, of which walking through the cut cubes took 3.)
+// each waited for the table, the bits and each other, 28 us for 512^3, of which walking through the cut cubes took 3; now 16.)
 constexpr uint32_t MC_EACH = 4;
 static_assert(MC_BLOCK == 64u * MC_EACH, "a wave takes a block");
 __global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
@@ -624,7 +624,7 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // corners pick theirs.  What bounds the launch is the chain of round trips: which words own something, their records (they stay in LDS, for
 // their neighbours in y too), then all that a point needs at once.  A cube's case comes from the bits, as its number of triangles did: whatever
 // the density is by now, a triangle's corners are vertices that this pass writes.
-// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 35; with the case from the density 34.)
+// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 34; with the case from the density 33.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
 constexpr uint32_t MC_EMIT_GRID = 1536;  // as many as run at a time: six per CU, by their LDS
 typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -754,7 +754,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 // The triangles' other corners are worked out again from the density, by the arithmetic that placed them: the eighteen values of the four
 // cubes tell which triangles there are (MC_RING) and where their corners lie.  That is 18 loads a vertex and vector instructions; going
 // through the words' records to the triangles and from those to the vertices was some 45 loads, most of them lines of their own, one a
-// clock and CU: 34 us for 512^3, now 26.
+// clock and CU: 32.5 us for 512^3, now 25.6.
 template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const float* __restrict__ density, float* __restrict__ normals) {
 	__shared__ float values[18][MC_BLOCK];  // [slow -1 .. 1][fast -1 .. 1][along 0, 1]

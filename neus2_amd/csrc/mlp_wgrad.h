@@ -17,8 +17,9 @@
 // pass:  {dy, h} -> dW_out, {g, a} -> dW_out, {dh, x} -> dW_0, {b, v} -> dW_0.
 // A wave holds all tiles of the weight gradients: 16 x 16 tiles have no padding, 128 accumulator registers for 48 -> 64 -> 64 -> 16,
 // which leaves the chain 128 at two waves per SIMD.  (The tiles dealt to the four waves of a workgroup, 48 accumulator
-// registers, takes eight barriers for every 128 samples: at 2^18 samples 40 us for that network and 33 for 48 -> 64 -> 16 with the
-// second-order pass, now 37 and 28; both at 52344 samples 28 -> 26, at 16 384 21 -> 20.)
+// registers, takes eight barriers for every 128 samples: at 2^18 samples 36.5 us for that network and 32.8 for 48 -> 64 -> 16 with the
+// second-order pass, now 35.4 and 27.5; a trained step's 44.5 and 36.6, now 40.7 and 32.7; both at 52344 samples 28 -> 25.5, and at 16 384, with the
+// weights' copies under way together, 22 -> 18.)
 #pragma once
 #include "grid_device.h"
 #include "mlp_device.h"

@@ -154,7 +154,6 @@ def test_small_queries_of_narrow_networks_equal_the_same_points_in_a_large_one(l
     test_small_queries_equal_the_same_points_in_a_large_one(72, levels, 1.0)
 
 
-# one tile past the line at which a query's and a forward's levels are no longer dealt to the XCDs
 @pytest.mark.parametrize("n", [8, 32, 40, 64, 72, 264])  # pairs across a wave's halves: no second half, a part of it, all, a wave more, a workgroup more
 @pytest.mark.parametrize("active", [1.0, 0.5])
 def test_small_batches_equal_the_same_samples_in_a_large_one(n, active):
@@ -169,6 +168,7 @@ def test_small_batches_equal_the_same_samples_in_a_large_one(n, active):
     assert torch.equal(net.forward(coords[:n].contiguous()), large[:n]) and bool(torch.isfinite(large.float()).all())
 
 
+# one tile past the line at which a query's and a forward's levels are no longer dealt to the XCDs
 @pytest.mark.parametrize("levels", [16, 14, 1])
 def test_batches_past_the_deal_by_xcd_equal_their_parts(levels):
     from neus2_amd.tcnn_api import NerfNetwork
