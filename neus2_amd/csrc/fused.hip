@@ -834,10 +834,11 @@ static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream
 	field_gather_kernel<FULL><<<grid, dim3(FG_BLOCK), 0, s>>>(a, tiles, g.y == 1u ? 1 : 0);
 }
 
-// Up to here a query is one launch.  Beyond it the fragments that every 32 points rebuild from the weights weigh more than the
-// second launch and its wait (device time in a graph, two launches -> one: 64 points 6.2 -> 4.7 us, 1000 6.9 -> 4.9, 4096 7.8 -> 6.5,
-// 8192 9.4 -> 10.2, 16384 13.0 -> 16.6; a call from Python, bound by the host: 1000 points 9.5 -> 7.3, 8192 the same).
-constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 6144;
+// Up to here a query is one launch: 256 workgroups of FQ_POINTS, one for each CU.  Beyond, some CUs run two, and the fragments that every 32 points
+// rebuild from the weights weigh more than the second launch and its wait.  (Device time in a graph, two launches | one: 64 points 6.3 | 3.5 us, 1000 8.1 | 5.0,
+// 4096 10.3 | 6.9, 6144 11.5 | 8.4, 8192 11.7 | 9.7, 10 240 12.85 | 12.7, 12 288 12.8 | 13.4, 16 384 14.1 | 16.3; a call from Python, bound by the host below
+// 5000 points: 1000 9.4 | 7.2, 8192 11.7 | 9.7.)
+constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 256 * FQ_POINTS;
 
 static uint32_t fused_grid(uint32_t n, uint32_t most = 512u) {
 	const uint32_t tiles = (n + 31u) / 32u, blocks = (tiles + 3u) / 4u;

@@ -131,17 +131,17 @@ def test_sdf_and_density(oracle):
     assert torch.equal(gf.sdf(dev(rows)), gf.sdf(dev(xyz)))
 
 
-@pytest.mark.parametrize("n", [8, 32, 40, 1000, 6144, 6152])
+@pytest.mark.parametrize("n", [8, 32, 40, 1000, 6144, 6152, 8192, 8200])
 @pytest.mark.parametrize("levels,active", [(16, 1.0), (14, 1.0), (16, 0.5), (9, 1.0)])
 def test_small_queries_equal_the_same_points_in_a_large_one(n, levels, active):
-    """Queries of up to 6144 points are one launch: bit for bit what the gather and network launches give."""
+    """Queries of up to 8192 points are one launch: bit for bit what the gather and network launches give."""
     from neus2_amd.tcnn_api import NerfNetwork
     net = NerfNetwork(n_levels=levels)
     gen = torch.Generator(device="cuda").manual_seed(n + levels)
     net.set_params((torch.randn(net.param_offsets()[4], device="cuda", generator=gen) * 0.1).half(), None)
     if active < 1.0:
         net.encoding().set_max_level(active)
-    many = torch.rand((8192, 3), device="cuda", generator=gen) * 1.2 - 0.1
+    many = torch.rand((16384, 3), device="cuda", generator=gen) * 1.2 - 0.1
     few = many[:n].contiguous()
     for query in (net.sdf, net.density):
         want = query(many)[:, :n]
