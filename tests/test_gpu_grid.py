@@ -326,7 +326,7 @@ def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     dp = (torch.rand(gg.n_params(), device="cuda", generator=gen) * 2 - 1).half()
     dg = torch.zeros_like(dp)
     gg.set_params(dp, dg)
-    large = 16384 + 1024
+    large = 24576 + 1024  # (two points per thread, the batches one)
     x = torch.rand((3, large), device="cuda", generator=gen)
     dy, g2, v = (torch.randn((w, large), device="cuda", generator=gen) for w in (32, 32, 3))
     dy[:, n:] = 0
