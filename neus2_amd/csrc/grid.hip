@@ -764,7 +764,7 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 // fp16 values, i.e. multiples of 2^-24 below 2^16, so value * 2^32 is an exact integer below 2^48 and the
 // sum of a whole bucket stays far inside 64 bits.  The accumulation is exact and independent of order.
 constexpr uint32_t RED_BLOCK = 1024;              // 16 waves; two workgroups share a CU
-constexpr uint32_t FEW_TILES = 32;                // batches of at most this many tiles: see grid_reduce_kernel
+constexpr uint32_t FLIGHT_TILES = 32;             // batches of at most this many tiles: see grid_reduce_kernel
 constexpr float FIX_SCALE = 4294967296.0f;        // 2^32
 
 // x * 2^32 as a two's complement 64-bit integer, for |x| < 2^31 with at most 24 significant bits (any fp16 value):
@@ -893,7 +893,7 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const uin
 	}
 }
 
-// FLIGHT: 2 for batches of few tiles, whose runs rarely hold more (the loads of absent records cost 2 us at 5e3 points)
+// FLIGHT: 2 for batches of few tiles, whose runs rarely hold more (30 000 points: forward and backward 41.6 -> 41.3 us)
 template <uint32_t FLIGHT>
 __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
@@ -937,6 +937,174 @@ __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable 
 		}
 		*at = out;
 	}
+}
+
+// Small batches: the gradient of a bucket with few records.
+// grid_reduce_kernel keeps a sum for each of a bucket's 4096 entries: 64 KiB of LDS to clear and to read again, at two workgroups per CU, for a bucket that
+// holds 160 records when the batch has 5000 points.  Here a record claims a sum: every record writes its own number to the 16-bit place of its entry, and
+// whichever number stands there afterwards is the entry's sum (64-bit fixed point as above, so the result is the same whoever wins).  Nothing is cleared but
+// the sums that exist; the other entries' zeros go out while the first loads are under way (an accumulating launch leaves them alone), and a workgroup's
+// 32 KiB let four of 512 threads share a CU.  Every thread finds its records by their number among the bucket's, so no lane has to
+// match a tile's run.  Levels of few entries keep an image, as does (range by range) a bucket with more records than
+// there are sums to claim.  What bounds it is the chain level -> bounds -> records -> sums and the 25 MB the gradient's zeros take.
+// Launch in us, image -> claims: 600 uniform points 15 -> 10.1, 5003 along rays 15.1 -> 10.6 (accumulating 15.6 -> 9.5), training step of 2^14 samples 17.5 -> 14.8.
+// (256 threads: the same up to 5000 points, 16 384 uniform points +4; 1024: +4; 128: +0.5)
+constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 4096;
+constexpr uint32_t FEW_TILES = 64;                                  // a lane of every wave looks up one tile's run
+constexpr uint32_t FEW_CLAIMS = (FEW_WORDS - BKT_ENTRIES / 4) / 2;  // sums of both features, beside the table of 16-bit claims
+constexpr uint32_t FEW_RANGE = FEW_WORDS / 2;                       // entries of an image
+
+// A bucket's records, numbered through its tiles' runs.
+struct N2FewRuns {
+	uint32_t first, upto, total;  // lane t: where tile t's run starts in its slot, records in the tiles up to t; all records
+	// the tile of record r < total and its place in the tile's slot (by all lanes of the wave)
+	__device__ __forceinline__ void find(uint32_t r, uint32_t& tile, uint32_t& at) const {
+		uint32_t t = 0;
+#pragma unroll
+		for (uint32_t s = FEW_TILES / 2; s > 0; s >>= 1) t += r >= n2_lane_value(upto, t + s - 1u) ? s : 0u;
+		// (every lane takes part in the exchanges: a lane that a branch had left out would pass nothing on)
+		const uint32_t begin = n2_lane_value(first, t), below = n2_lane_value(upto, t - 1u);
+		tile = t;
+		at = begin + r - (t > 0u ? below : 0u);
+	}
+};
+
+template <bool PAIR>
+__device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_records, const uint32_t tiles, const N2ReduceItem& it, const uint32_t entries,
+                                                       const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
+                                                       const uint16_t* __restrict__ offsets, __half2* __restrict__ Gd, const bool accumulate, unsigned long long* mem) {
+	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
+	constexpr uint32_t EACH = PAIR ? 2u : 1u;                                               // entries of a record
+	constexpr uint32_t K = (FEW_CLAIMS / EACH + FEW_BLOCK - 1u) / FEW_BLOCK;  // records of a thread that may claim
+	const size_t level_tile0 = (size_t)it.level * tiles;
+	const uint32_t lane = threadIdx.x & 63u;
+	uint32_t two;
+	__builtin_memcpy(&two, offsets + (level_tile0 + min(lane, tiles - 1u)) * (BKT_MAX + 1) + it.bucket, sizeof(two));
+	const uint32_t left = min(it.entries, entries - it.bucket * it.entries);  // entries of the bucket (a level's are a multiple of eight)
+	__half2* G = Gd + it.bucket * it.entries;
+	const bool claims = it.entries > FEW_RANGE;
+	typedef uint32_t wide __attribute__((ext_vector_type(4)));
+	if (claims && !accumulate)
+		for (uint32_t e = threadIdx.x * 4u; e < left; e += FEW_BLOCK * 4u) *reinterpret_cast<wide*>(G + e) = wide(0u);
+	N2FewRuns runs;
+	runs.first = two & 0xFFFFu;
+	const uint32_t own = lane < tiles ? (two >> 16) - runs.first : 0u;
+	runs.upto = n2_wave_prefix(own);
+	runs.total = __builtin_amdgcn_readlane(runs.upto, 63);
+	auto load = [&](uint32_t r, uint32_t& key, value& v) {
+		uint32_t tile, at;
+		runs.find(r, tile, at);
+		const size_t slot = (level_tile0 + tile) * slot_records + at;
+		key = rec_keys[slot];
+		v = reinterpret_cast<const value*>(rec_vals + (level_tile0 + tile) * slot_records)[at];
+	};
+	auto places = [&](uint32_t key, uint32_t (&e)[EACH]) {
+		if constexpr (PAIR) {
+			e[0] = key & (BKT_ENTRIES - 1u);
+			e[1] = e[0] ^ ((2u << (key >> BKT_SHIFT)) - 1u);  // x ^ (x + 1) = 2^(t+1) - 1
+		} else e[0] = key;
+	};
+	auto word = [](const value& v, uint32_t q) {
+		if constexpr (sizeof(value) == 8) return q ? v.y : v.x;
+		else return v;
+	};
+	auto sum_of = [&](uint32_t old, unsigned long long a, unsigned long long b) {
+		float2 f = accumulate ? __half22float2(*reinterpret_cast<const __half2*>(&old)) : make_float2(0.f, 0.f);
+		return __floats2half2_rn(f.x + from_fixed(a), f.y + from_fixed(b));
+	};
+	if (claims && runs.total * EACH <= FEW_CLAIMS) {
+		uint16_t* claim = reinterpret_cast<uint16_t*>(mem);
+		unsigned long long* acc = mem + BKT_ENTRIES / 4;
+		uint32_t key[K], e[K][EACH], by[K][EACH], old[K][EACH];
+		value v[K];
+#pragma unroll
+		for (uint32_t k = 0; k < K; ++k) {
+			const uint32_t r = threadIdx.x + k * FEW_BLOCK;
+			if (k * FEW_BLOCK < runs.total) load(min(r, runs.total - 1u), key[k], v[k]);
+		}
+#pragma unroll
+		for (uint32_t k = 0; k < K; ++k) {
+			const uint32_t r = threadIdx.x + k * FEW_BLOCK;
+			if (r >= runs.total) break;
+			places(key[k], e[k]);
+#pragma unroll
+			for (uint32_t q = 0; q < EACH; ++q) {
+				claim[e[k][q]] = (uint16_t)(r * EACH + q);
+				acc[r * EACH + q] = 0ull;
+				acc[FEW_CLAIMS + r * EACH + q] = 0ull;
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (uint32_t k = 0; k < K; ++k) {
+			if (threadIdx.x + k * FEW_BLOCK >= runs.total) break;
+#pragma unroll
+			for (uint32_t q = 0; q < EACH; ++q) {
+				by[k][q] = claim[e[k][q]];
+				const uint32_t raw = word(v[k], q);
+				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
+				atomicAdd(&acc[by[k][q]], to_fixed(f.x));
+				atomicAdd(&acc[FEW_CLAIMS + by[k][q]], to_fixed(f.y));
+				old[k][q] = accumulate && by[k][q] == (threadIdx.x + k * FEW_BLOCK) * EACH + q && e[k][q] < left ? *reinterpret_cast<const uint32_t*>(G + e[k][q]) : 0u;
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (uint32_t k = 0; k < K; ++k) {
+			const uint32_t r = threadIdx.x + k * FEW_BLOCK;
+			if (r >= runs.total) break;
+#pragma unroll
+			for (uint32_t q = 0; q < EACH; ++q) {
+				const uint32_t id = r * EACH + q;
+				if (by[k][q] != id || e[k][q] >= left) continue;
+				G[e[k][q]] = sum_of(old[k][q], acc[id], acc[FEW_CLAIMS + id]);
+			}
+		}
+		return;
+	}
+	for (uint32_t from = 0; from < left; from += FEW_RANGE) {
+		const uint32_t n = min(FEW_RANGE, left - from);
+		for (uint32_t e = threadIdx.x; e < n; e += FEW_BLOCK) { mem[e] = 0ull; mem[FEW_RANGE + e] = 0ull; }
+		__syncthreads();
+		for (uint32_t r = threadIdx.x; __any(r < runs.total); r += FEW_BLOCK) {
+			uint32_t key, e[EACH];
+			value v;
+			load(min(r, runs.total - 1u), key, v);
+			places(key, e);
+#pragma unroll
+			for (uint32_t q = 0; q < EACH; ++q) {
+				const uint32_t at = e[q] - from, raw = word(v, q);
+				if (r >= runs.total || at >= n) continue;
+				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
+				atomicAdd(&mem[at], to_fixed(f.x));
+				atomicAdd(&mem[FEW_RANGE + at], to_fixed(f.y));
+			}
+		}
+		__syncthreads();
+		for (uint32_t e = threadIdx.x * 4u; e < n; e += FEW_BLOCK * 4u) {
+			wide* at = reinterpret_cast<wide*>(G + from + e);
+			const wide old = accumulate ? *at : wide(0u);
+			wide out;
+#pragma unroll
+			for (uint32_t q = 0; q < 4; ++q) {
+				const __half2 h = sum_of(old[q], mem[e + q], mem[FEW_RANGE + e + q]);
+				out[q] = *reinterpret_cast<const uint32_t*>(&h);
+			}
+			*at = out;
+		}
+		__syncthreads();
+	}
+}
+
+__global__ void __launch_bounds__(FEW_BLOCK, 8) grid_reduce_few_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
+                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
+                                                                    const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, int accumulate) {
+	__shared__ __align__(16) unsigned long long mem[FEW_WORDS];
+	const N2ReduceItem it = n2_reduce_item(tab, plan);
+	__half2* Gd = grads + tab.offset[it.level];
+	const uint32_t entries = tab.entries[it.level];
+	if (it.pair) grid_reduce_few_bucket<true>(slot_records, tiles, it, entries, rec_vals, rec_keys, offsets, Gd, accumulate != 0, mem);
+	else grid_reduce_few_bucket<false>(slot_records, tiles, it, entries, rec_vals, rec_keys, offsets, Gd, accumulate != 0, mem);
 }
 
 // Split buckets: the sum of a bucket's G partial images in a fixed order (n2_image_combine_unit, slab_reduce.h: with the
@@ -1275,12 +1443,11 @@ static bool uses_bucketed(const n2_grid_t* grid, uint32_t n_points) {
 // buckets) under which a bucket holds at most `target` of the level's 8 records per point, or the smallest there is: small
 // dense levels get many small buckets instead of few that outlast the others.  When even the smallest buckets hold more than
 // 65536, they stay large and are split (bucket_groups).
-static uint32_t bucket_shift_for(const n2_grid_t* grid, uint32_t level, uint32_t n_points) {
+// The target is 16384 for grid_reduce_kernel (8192 and 32768: the same within 2 %, 65536: 49 us against 36 at 1.2e5 points, where a dense
+// level's few workgroups outlast the others) and 512, a record per thread, for grid_reduce_few_kernel.
+static uint32_t bucket_shift(const n2_grid_t* grid, uint32_t level, uint32_t n_points, uint64_t target) {
 	if ((grid->tab.pair_levels >> level) & 1u) return BKT_SHIFT;
 	const uint32_t entries = grid->tab.entries[level];
-	// (8192 and 32768 records: the same within 2 %, 65536: 49 us against 36 at 1.2e5 points, where a dense level's few workgroups
-	// outlast the others)
-	constexpr uint64_t target = 16384u;
 	for (uint32_t shift = BKT_SHIFT; shift >= BKT_MIN_SHIFT; --shift) {
 		const uint32_t nb = (entries + (1u << shift) - 1u) >> shift, finer = (entries + (1u << (shift - 1u)) - 1u) >> (shift - 1u);
 		if (nb > BKT_MAX) break;
@@ -1288,6 +1455,22 @@ static uint32_t bucket_shift_for(const n2_grid_t* grid, uint32_t level, uint32_t
 		if (records <= target || (records <= 65536u && (shift == BKT_MIN_SHIFT || finer > BKT_MAX))) return shift;
 	}
 	return BKT_SHIFT;
+}
+// Whether a batch takes grid_reduce_few_kernel: on average its buckets hold no more records than threads on levels of pair records, which is two thirds of
+// the claims there are, and 2048 on the others, whose buckets are the smallest there can be.  With the default table that is up to 16 384 points.
+// Encoding forward and backward in us, grid_reduce_kernel | this one: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5, 8192 33.5 | 29.1, 12 288 35.5 | 32.7,
+// 16 384 37.7 | 37.0; along rays 3000 28.7 | 25.2, 16 384 34.9 | 31.1, 32 768 41.8 | 43.2.
+static bool few_records(const n2_grid_t* grid, uint32_t n_points) {
+	if (n_bin_tiles(grid, n_points) > FEW_TILES) return false;
+	for (uint32_t l = 0; l < grid->tab.n_levels; ++l) {
+		const bool pair = (grid->tab.pair_levels >> l) & 1u;
+		const uint32_t shift = bucket_shift(grid, l, n_points, FEW_BLOCK), nb = (grid->tab.entries[l] + (1u << shift) - 1u) >> shift;
+		if ((uint64_t)n_points * (pair ? 4u : 8u) > (uint64_t)nb * (pair ? FEW_BLOCK : 4u * FEW_BLOCK)) return false;
+	}
+	return true;
+}
+static uint32_t bucket_shift_for(const n2_grid_t* grid, uint32_t level, uint32_t n_points) {
+	return bucket_shift(grid, level, n_points, few_records(grid, n_points) ? FEW_BLOCK : 16384u);
 }
 static inline uint32_t level_buckets(const n2_grid_t* grid, uint32_t level, uint32_t n_points) {
 	const uint32_t shift = bucket_shift_for(grid, level, n_points);
@@ -1353,7 +1536,7 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	N2BucketPlan plan;
 	uint32_t wg = 0, images = 0, split = 0;
 	N2LevelTable tab = grid->tab;  // with this launch's bucket sizes
-	const bool few = tiles <= FEW_TILES;
+	const bool few = tiles <= FLIGHT_TILES;
 	for (uint32_t l = 0; l < L; ++l) {
 		tab.bucket_shift[l] = (uint8_t)bucket_shift_for(grid, l, n_points);
 		const uint32_t nb = level_buckets(grid, l, n_points);
@@ -1391,7 +1574,10 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	else bin(std::integral_constant<uint32_t, 2>());
 	N2_LAUNCH_CHECK();
 #define LAUNCH(F) grid_reduce_kernel<F><<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials)
-	if (few) LAUNCH(2); else LAUNCH(4);
+	if (few_records(grid, n_points))
+		grid_reduce_few_kernel<<<dim3(wg), dim3(FEW_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
+	else if (few) LAUNCH(2);
+	else LAUNCH(4);
 #undef LAUNCH
 	N2_LAUNCH_CHECK();
 	if (split > 0) {

@@ -341,6 +341,46 @@ def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and bool((got[0][0] != 0).any())
 
 
+# batches whose buckets hold few records, up to the last one and the next; points that all fall into a few cells, in turn (no runs to merge), so that
+# single buckets hold more records than sums can be claimed for; tables of few and of small buckets
+@pytest.mark.parametrize("n,where,table", [(1, "anywhere", (16, 19)), (511, "anywhere", (16, 19)), (5003, "anywhere", (16, 19)), (16384, "anywhere", (16, 19)), (16385, "anywhere", (16, 19)),
+                                           (384, "two cells", (16, 19)), (385, "two cells", (16, 19)), (5003, "two cells", (16, 19)), (16384, "two cells", (16, 19)),
+                                           (9001, "outside", (16, 19)), (100, "anywhere", (6, 12)), (128, "two cells", (6, 12)), (7000, "anywhere", (1, 19)), (300, "anywhere", (3, 6))])
+def test_sorted_scatter_of_few_records(n, where, table):
+    """The sums are exact, so how a bucket is summed leaves no trace: a batch equals the one that has points without a gradient behind it, which is
+    large enough for the other kernel.  Overwriting, accumulating, with levels switched off, and for both layouts of the positions."""
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(**{**CFG, "n_levels": table[0], "log2_hashmap_size": table[1]})
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = (torch.rand(gg.n_params(), device="cuda", generator=gen) * 2 - 1).half()
+    dg = torch.zeros_like(dp)
+    gg.set_params(dp, dg)
+    large = 70000
+    x = torch.rand((3, large), device="cuda", generator=gen)
+    if where == "two cells":
+        x = 0.3 + 0.4 * (torch.arange(large, device="cuda") % 2) + 1e-5 * x
+    elif where == "outside":
+        x = x * 1.5 - 0.25
+    dy, g2, v = (torch.randn((w, large), device="cuda", generator=gen) for w in (2 * table[0], 2 * table[0], 3))
+    dy[:, n:] = 0
+    g2[:, n:] = 0
+    for mode, level, rows in ((GRAD_OVERWRITE, 1000.0, True), (GRAD_ACCUMULATE, 1000.0, True), (GRAD_OVERWRITE, 0.4, True), (GRAD_OVERWRITE, 1000.0, False)):
+        gg.set_max_level(level)
+        got = []
+        for points in (n, large):
+            gg.set_params(dp, dg)
+            assert gg.reserve_scatter_workspace(points)
+            dg.fill_(3.0)
+            at = x[:, :points].contiguous() if rows else x[:, :points].t().contiguous()
+            a, b, c = dy[:, :points].half().contiguous(), v[:, :points].contiguous(), g2[:, :points].half().contiguous()
+            if rows:
+                gg.backward_fused(at, a, b, c, want_dL_ddLdy=False, mode=mode)
+            else:
+                gg.backward(None, at, a, mode=mode)
+            got.append(dg.clone())
+        assert torch.equal(got[0], got[1]) and bool((got[0] != (3.0 if mode == GRAD_ACCUMULATE else 0.0)).any()), (mode, level, rows)
+
+
 # the last batch of one point per thread and the next one, workspaces that are just large enough and larger; buckets of up to 65536 records are whole
 @pytest.mark.parametrize("levels,log2_size,line,whole", [(16, 19, 24576, True), (7, 16, 55808, True), (7, 14, 55808, False), (2, 6, 196608, False)])
 def test_sorted_scatter_at_the_line_between_the_tiles(levels, log2_size, line, whole):
