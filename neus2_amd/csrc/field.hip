@@ -499,18 +499,25 @@ int n2_field_forward_listed(n2_field_t* f, n2_stream_t stream, const float* d_co
 	                              reinterpret_cast<n2_half*>(f->rgb_in), d_output, nullptr, d_list, d_counts, round, est_samples);
 }
 
+static int field_backward(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n, const n2_half* d_dL_doutput, uint32_t ek_batch_size,
+                          n2_grad_mode mode, N2SlabReduce* sums);
+
 N2_API int n2_field_backward(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n,
                              const n2_half* d_dL_doutput, uint32_t ek_batch_size, n2_grad_mode mode) {
-	N2SlabReduce sums = {};
-	if (int rc = n2_field_backward_deferred(f, stream, d_coords, n, d_dL_doutput, ek_batch_size, mode, &sums)) return rc;
-	return n2_slab_reduce_launch(stream, sums);
+	return field_backward(f, stream, d_coords, n, d_dL_doutput, ek_batch_size, mode, nullptr);
+}
+int n2_field_backward_deferred(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n, const n2_half* d_dL_doutput, uint32_t ek_batch_size,
+                               n2_grad_mode mode, N2SlabReduce* sums) {
+	*sums = N2SlabReduce{};
+	return field_backward(f, stream, d_coords, n, d_dL_doutput, ek_batch_size, mode, sums);
 }
 
 static int field_backward_passes(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n, const n2_half* d_dL_doutput, uint32_t ek_batch_size,
                                  n2_grad_mode mode, N2SlabReduce* sums);
 
-int n2_field_backward_deferred(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n, const n2_half* d_dL_doutput, uint32_t ek_batch_size,
-                               n2_grad_mode mode, N2SlabReduce* sums) {
+// sums: the plan of the slab summation for the caller to run, or null: it is run beside the scatter
+static int field_backward(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n, const n2_half* d_dL_doutput, uint32_t ek_batch_size,
+                          n2_grad_mode mode, N2SlabReduce* sums) {
 	if (f != nullptr && f->frags_ready) {
 		// the weight-gradient kernels' fragments as the forward's gather launch built them, once for all workgroups
 		const n2_half* image = reinterpret_cast<const n2_half*>(f->frag_image);
@@ -526,14 +533,13 @@ int n2_field_backward_deferred(n2_field_t* f, n2_stream_t stream, const float* d
 		// a pass that ran before the failure left partial sums pending in its network: nobody will reduce them
 		n2_mlp_drop_pending(f->rgb);
 		n2_mlp_drop_pending(f->sdf);
-		*sums = N2SlabReduce{};
+		if (sums) *sums = N2SlabReduce{};
 	}
 	return rc;
 }
 
 static int field_backward_passes(n2_field_t* f, n2_stream_t stream, const float* d_coords, uint32_t n, const n2_half* d_dL_doutput, uint32_t ek_batch_size,
                                  n2_grad_mode mode, N2SlabReduce* sums) {
-	*sums = N2SlabReduce{};
 	if (int rc = check_field(f, "n2_field_backward", n)) return rc;
 	N2_REQUIRE(n <= f->max_batch_bwd, "n2_field_backward: batch %u exceeds the workspace's backward capacity %u", n, f->max_batch_bwd);
 	N2_REQUIRE(mode == N2_GRAD_OVERWRITE || mode == N2_GRAD_ACCUMULATE, "n2_field_backward: mode must be OVERWRITE or ACCUMULATE");
@@ -585,15 +591,17 @@ static int field_backward_passes(n2_field_t* f, n2_stream_t stream, const float*
 	                                                      reinterpret_cast<const n2_half*>(f->d_rgb_in), f->slopes_saved ? N2_LAYOUT_AOS : N2_LAYOUT_SOA,
 	                                                      reinterpret_cast<n2_half*>(f->d_sdf_in),
 	                                                      reinterpret_cast<const n2_half*>(f->d_density_in), nullptr, mode, true)) return rc;
+	// the three weight-gradient passes (colour net, SDF net first and second order) left their per-workgroup partial sums
+	// pending: one plan sums them, and with them the partial sums of the variance gradient
+	N2SlabReduce plan;
+	if (int rc = n2_mlp_reduce_deferred_plan(f->rgb, f->sdf, f->var_part, var_parts, reinterpret_cast<n2_half*>(f->grads + f->off_var),
+	                                         mode == N2_GRAD_ACCUMULATE ? 1 : 0, &plan)) return rc;
 	// grid: first-order and second-order gradients in one scatter pass (the reference's backward with
 	// Overwrite followed by backward_backward_input with Accumulate)
 	if (int rc = n2_grid_backward_fused_indexed(f->grid, stream, f->xyz, n_src, index, n, reinterpret_cast<const n2_half*>(f->d_sdf_in + (size_t)3 * n), f->v,
-	                                            reinterpret_cast<const n2_half*>(f->dsdf_din + (size_t)3 * n_src), mode)) return rc;
-	// the three weight-gradient passes (colour net, SDF net first and second order) left their per-workgroup partial sums
-	// pending: one plan sums them, and with them the partial sums of the variance gradient (the caller runs it: as a launch,
-	// or inside the optimiser's kernel)
-	return n2_mlp_reduce_deferred_plan(f->rgb, f->sdf, f->var_part, var_parts, reinterpret_cast<n2_half*>(f->grads + f->off_var),
-	                                   mode == N2_GRAD_ACCUMULATE ? 1 : 0, sums);
+	                                            reinterpret_cast<const n2_half*>(f->dsdf_din + (size_t)3 * n_src), mode, sums ? nullptr : &plan)) return rc;
+	if (sums) *sums = plan;
+	return N2_OK;
 }
 
 N2_API int n2_field_select(n2_field_t* f, n2_stream_t stream, const uint32_t* d_source_index, uint32_t n_source, uint32_t n) {

@@ -309,11 +309,8 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_scatter_kernel(N2LevelTable t
 // ones: eight rows' loads are under way together (one row at a time: 10.5 us for 5003 points, 23.5 for 2^18; now 4.4 and 20.3).
 constexpr uint32_t BWD_IN_ROWS = 8;
 template <bool STREAM>
-__global__ void __launch_bounds__(GRID_BLOCK) grid_backward_input_kernel(uint32_t N, uint32_t n_out,
-                                                                         const __half* __restrict__ dL_dy,
-                                                                         const float* __restrict__ dy_dx,
-                                                                         float* __restrict__ dL_dx) {
-	const uint32_t i = blockIdx.x * GRID_BLOCK + threadIdx.x;
+__device__ __forceinline__ void grid_backward_input_point(uint32_t i, uint32_t N, uint32_t n_out, const __half* __restrict__ dL_dy, const float* __restrict__ dy_dx,
+                                                          float* __restrict__ dL_dx) {
 	if (i >= N) return;
 	float r0 = 0.f, r1 = 0.f, r2 = 0.f;
 	for (uint32_t k0 = 0; k0 < n_out; k0 += BWD_IN_ROWS) {
@@ -339,6 +336,13 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_backward_input_kernel(uint32_
 	dL_dx[i] = r0;
 	dL_dx[(size_t)N + i] = r1;
 	dL_dx[(size_t)2 * N + i] = r2;
+}
+template <bool STREAM>
+__global__ void __launch_bounds__(GRID_BLOCK) grid_backward_input_kernel(uint32_t N, uint32_t n_out,
+                                                                         const __half* __restrict__ dL_dy,
+                                                                         const float* __restrict__ dy_dx,
+                                                                         float* __restrict__ dL_dx) {
+	grid_backward_input_point<STREAM>(blockIdx.x * GRID_BLOCK + threadIdx.x, N, n_out, dL_dy, dy_dx, dL_dx);
 }
 
 // ----------------------------------------------------------------------------
@@ -735,7 +739,26 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	if (threadIdx.x <= BKT_MAX) offsets[((size_t)level * tiles + tile) * (BKT_MAX + 1) + threadIdx.x] = (uint16_t)prefix[threadIdx.x];
 }
 
-template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT>
+// What else a sorting launch does, in workgroups of its own: work that needs nothing of the scatter's and would be a launch behind it.
+// The input gradient streams the Jacobian while the others sort, its workgroups spread evenly among theirs (one behind each `every`): forward and
+// backward of 2^18 uniform points 206.7 -> 196.1 us, along rays 168.1 -> 159.3; 65 536 uniform 77.4 -> 72.7; 20 000 along rays 37.9 -> 34.0.
+struct N2RideNone {};
+template <bool STREAM>
+struct N2RideInput {
+	const float* dy_dx;
+	float* dL_dx;
+	uint32_t n_out, blocks, every;
+};
+// The networks' weight-gradient slabs, two units to a workgroup, in the first workgroups: the field's forward and backward on 2^18 samples
+// 251.0 -> 247.9 us, on 52 344 94.8 -> 91.6, on 2048 47.6 -> 41.3.
+struct N2RideSums {
+	N2SlabReduce sums;
+	uint32_t blocks;
+};
+template <class Ride> constexpr bool RIDES_INPUT = false;
+template <bool STREAM> constexpr bool RIDES_INPUT<N2RideInput<STREAM>> = true;
+
+template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT, class Ride>
 __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab, uint32_t first_level, uint32_t N, uint32_t tiles,
                                                               const float* __restrict__ xyz, uint32_t point_stride,
                                                               uint32_t dim_stride, const __half* __restrict__ dL_dy,
@@ -743,12 +766,34 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
                                                               const __half2* __restrict__ params, __half* __restrict__ dL_ddLdy,
                                                               uint32_t* __restrict__ rec_vals, uint16_t* __restrict__ rec_keys,
                                                               uint16_t* __restrict__ offsets,
-                                                              const uint32_t* __restrict__ index, uint32_t n_cols) {
+                                                              const uint32_t* __restrict__ index, uint32_t n_cols, Ride ride) {
 	__shared__ uint32_t hist[BKT_MAX];
 	__shared__ uint32_t prefix[BKT_MAX + 1];
 	__shared__ __align__(16) uint32_t stage_val[bin_records(PER)];  // sorted records: packed half2 value (a pair of them on pair levels) ...
 	__shared__ __align__(16) uint16_t stage_key[bin_records(PER)];  // ... and entry within its bucket
-	const uint32_t level = first_level + blockIdx.x / tiles, tile = blockIdx.x % tiles;
+	uint32_t block = blockIdx.x;
+	if constexpr (RIDES_INPUT<Ride>) {
+		const uint32_t q = block / (ride.every + 1u), m = block - q * (ride.every + 1u);
+		if (m == ride.every) {
+			const auto point = [&](auto stream) {
+				grid_backward_input_point<decltype(stream)::value>(q * BIN_BLOCK + threadIdx.x, N, ride.n_out, dL_dy, ride.dy_dx, ride.dL_dx);
+			};
+			point(std::bool_constant<std::is_same<Ride, N2RideInput<true>>::value>());
+			return;
+		}
+		block = q * ride.every + m;
+		if (block >= tiles * tab.n_levels) return;
+	} else if constexpr (std::is_same<Ride, N2RideSums>::value) {
+		if (block < ride.blocks) {
+			constexpr uint32_t UNITS = BIN_BLOCK / 256;
+			static_assert(sizeof(float) * 32 * 33 * UNITS <= sizeof(stage_val), "the units' folds");
+			float(*fold)[33] = reinterpret_cast<float(*)[33]>(stage_val) + (threadIdx.x >> 8) * 32;
+			n2_slab_reduce_unit(ride.sums, block * UNITS + (threadIdx.x >> 8), fold, [](const _Float16*, _Float16) {}, threadIdx.x & 255u);
+			return;
+		}
+		block -= ride.blocks;
+	}
+	const uint32_t level = first_level + block / tiles, tile = block % tiles;
 	if (threadIdx.x < BKT_MAX) hist[threadIdx.x] = 0;
 	__syncthreads();
 	if ((tab.pair_levels >> level) & 1u)
@@ -1518,10 +1563,18 @@ N2_API int n2_grid_set_workspace(n2_grid_t* grid, void* d_workspace, uint64_t n_
 	return N2_OK;
 }
 
+// What a scatter is asked to do beside it: the input gradient (first order alone: dL_dx set), or a slab summation (first and second order together
+// and no dL_ddLdy).
+struct N2ScatterRider {
+	const float* dy_dx = nullptr;
+	float* dL_dx = nullptr;
+	N2SlabReduce sums = {};
+};
+
 // Parameter gradients through the bin + reduce kernels.  The gradient buffer has been zeroed for OVERWRITE.
 static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
                            const __half* dL_dy, const float* v, const __half* g2, __half* dL_ddLdy, bool accumulate,
-                           const uint32_t* index, uint32_t n_cols) {
+                           const uint32_t* index, uint32_t n_cols, const N2ScatterRider& rider) {
 	const uint32_t tiles = n_bin_tiles(grid, n_points), per = bin_per_thread(grid, n_points), L = grid->tab.n_levels;
 	const bool first = dL_dy != nullptr, second = v != nullptr, out = dL_ddLdy != nullptr;
 	const dim3 bd(BIN_BLOCK);
@@ -1532,7 +1585,6 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	uint16_t* rec_keys = reinterpret_cast<uint16_t*>(grid->ws + now.keys);
 	uint16_t* offsets = reinterpret_cast<uint16_t*>(grid->ws + now.offsets);
 	float2* partials = reinterpret_cast<float2*>(grid->ws + full.partials);
-	const dim3 gd(tiles * L);
 	N2BucketPlan plan;
 	uint32_t wg = 0, images = 0, split = 0;
 	N2LevelTable tab = grid->tab;  // with this launch's bucket sizes
@@ -1561,13 +1613,22 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.split_begin[l] = split;
 	auto bin = [&](auto per_thread) {
 		constexpr uint32_t PER = decltype(per_thread)::value;
-#define LAUNCH(F, S, O) grid_bin_kernel<PER, F, S, O><<<gd, bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
-                                                                        grid->params, dL_ddLdy, rec_vals, rec_keys, offsets, index, n_cols)
-		if (first && second && out) LAUNCH(true, true, true);
-		else if (first && second) LAUNCH(true, true, false);
-		else if (second && out) LAUNCH(false, true, true);
-		else if (second) LAUNCH(false, true, false);
-		else LAUNCH(true, false, false);
+#define LAUNCH(F, S, O, RIDE, BLOCKS) grid_bin_kernel<PER, F, S, O><<<dim3(BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
+                                                                                                grid->params, dL_ddLdy, rec_vals, rec_keys, offsets, index, n_cols, RIDE)
+		const uint32_t blocks = tiles * L;
+		const N2RideNone none;
+		if (rider.dL_dx != nullptr) {  // (first order alone)
+			const uint32_t riders = (n_points + BIN_BLOCK - 1) / BIN_BLOCK, every = (blocks + riders - 1) / riders, rows = L * grid->n_features;
+			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
+			else LAUNCH(true, false, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
+		} else if (rider.sums.units > 0) {  // (both orders)
+			const uint32_t riders = (rider.sums.units + BIN_BLOCK / 256 - 1) / (BIN_BLOCK / 256);
+			LAUNCH(true, true, false, (N2RideSums{rider.sums, riders}), riders + blocks);
+		} else if (first && second && out) LAUNCH(true, true, true, none, blocks);
+		else if (first && second) LAUNCH(true, true, false, none, blocks);
+		else if (second && out) LAUNCH(false, true, true, none, blocks);
+		else if (second) LAUNCH(false, true, false, none, blocks);
+		else LAUNCH(true, false, false, none, blocks);
 #undef LAUNCH
 	};
 	if (per == 1u) bin(std::integral_constant<uint32_t, 1>());
@@ -1603,12 +1664,20 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	return N2_OK;
 }
 
+static int launch_input_gradient(const n2_grid_t* grid, hipStream_t s, uint32_t n_points, const __half* dL_dy, const float* dy_dx, float* dL_dx) {
+	const uint32_t rows = grid->tab.n_levels * grid->n_features;
+	auto* const kernel = n2_jacobian_streams(n_points, rows) ? grid_backward_input_kernel<true> : grid_backward_input_kernel<false>;
+	kernel<<<dim3(n_tiles(n_points)), dim3(GRID_BLOCK), 0, s>>>(n_points, rows, dL_dy, dy_dx, dL_dx);
+	N2_LAUNCH_CHECK();
+	return N2_OK;
+}
+
 // One scatter pass with any combination of first-order (dL_dy) and second-order (v, g2) terms.
 static int launch_scatter(n2_grid_t* grid, hipStream_t s, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
                           const __half* dL_dy, const float* v, const __half* g2, __half2* grads, __half* dL_ddLdy, bool accumulate,
-                          const uint32_t* index = nullptr, uint32_t n_cols = 0) {
+                          const uint32_t* index = nullptr, uint32_t n_cols = 0, const N2ScatterRider& rider = N2ScatterRider()) {
 	if (grads != nullptr && uses_bucketed(grid, n_points))
-		return launch_bucketed(grid, s, d_xyz, point_stride, dim_stride, n_points, dL_dy, v, g2, dL_ddLdy, accumulate, index, n_cols);
+		return launch_bucketed(grid, s, d_xyz, point_stride, dim_stride, n_points, dL_dy, v, g2, dL_ddLdy, accumulate, index, n_cols, rider);
 	const uint32_t tiles = n_pair_tiles(n_points);
 	const dim3 gd(tiles * grid->tab.n_levels), bd(GRID_BLOCK);
 	const bool first = dL_dy != nullptr, second = v != nullptr, out = dL_ddLdy != nullptr;
@@ -1621,7 +1690,10 @@ static int launch_scatter(n2_grid_t* grid, hipStream_t s, const float* d_xyz, ui
 	else LAUNCH(true, false, false);
 #undef LAUNCH
 	N2_LAUNCH_CHECK();
-	return N2_OK;
+	if (rider.dL_dx != nullptr) {
+		if (int rc = launch_input_gradient(grid, s, n_points, dL_dy, rider.dy_dx, rider.dL_dx)) return rc;
+	}
+	return n2_slab_reduce_launch(reinterpret_cast<n2_stream_t>(s), rider.sums);
 }
 
 N2_API int n2_grid_backward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
@@ -1633,18 +1705,13 @@ N2_API int n2_grid_backward(n2_grid_t* grid, n2_stream_t stream, const float* d_
 	hipStream_t s = n2_stream(stream);
 	if (int rc = prepare_grads(grid, "n2_grid_backward", s, mode, n_points)) return rc;
 	if (n_points == 0) return N2_OK;
-	if (mode != N2_GRAD_IGNORE) {
-		N2ProfScope prof(N2_PROF_GRID_BACKWARD_PARAMS, s);
-		if (int rc = launch_scatter(grid, s, d_xyz, point_stride, dim_stride, n_points, reinterpret_cast<const __half*>(d_dL_dy), nullptr,
-		                            nullptr, grid->grads, nullptr, mode == N2_GRAD_ACCUMULATE)) return rc;
-	}
-	if (d_dL_dx) {
-		const uint32_t rows = grid->tab.n_levels * grid->n_features;
-		auto* const kernel = n2_jacobian_streams(n_points, rows) ? grid_backward_input_kernel<true> : grid_backward_input_kernel<false>;
-		kernel<<<dim3(n_tiles(n_points)), dim3(GRID_BLOCK), 0, s>>>(n_points, rows, reinterpret_cast<const __half*>(d_dL_dy), d_dy_dx, d_dL_dx);
-		N2_LAUNCH_CHECK();
-	}
-	return N2_OK;
+	if (mode == N2_GRAD_IGNORE) return d_dL_dx ? launch_input_gradient(grid, s, n_points, reinterpret_cast<const __half*>(d_dL_dy), d_dy_dx, d_dL_dx) : N2_OK;
+	N2ScatterRider rider;
+	rider.dy_dx = d_dy_dx;
+	rider.dL_dx = d_dL_dx;
+	N2ProfScope prof(N2_PROF_GRID_BACKWARD_PARAMS, s);
+	return launch_scatter(grid, s, d_xyz, point_stride, dim_stride, n_points, reinterpret_cast<const __half*>(d_dL_dy), nullptr, nullptr, grid->grads, nullptr,
+	                      mode == N2_GRAD_ACCUMULATE, nullptr, 0, rider);
 }
 
 N2_API int n2_grid_backward_fused(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
@@ -1665,7 +1732,7 @@ N2_API int n2_grid_backward_fused(n2_grid_t* grid, n2_stream_t stream, const flo
 
 int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz_rows, uint32_t n_cols, const uint32_t* d_index,
                                    uint32_t n_points, const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second,
-                                   n2_grad_mode mode) {
+                                   n2_grad_mode mode, const N2SlabReduce* sums) {
 	if (d_index == nullptr) n_cols = n_points;  // the rows hold the batch itself
 	if (int rc = check_batch(grid, "n2_grid_backward_fused", d_xyz_rows, 1, n_cols, n_points)) return rc;
 	N2_REQUIRE((d_dL_dy && d_dL_ddLdx && d_dL_dy_second) || n_points == 0, "n2_grid_backward_fused: d_dL_dy, d_dL_ddLdx and d_dL_dy_second are required");
@@ -1673,10 +1740,12 @@ int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const fl
 	N2_REQUIRE(n_cols >= 1, "n2_grid_backward_fused: an indexed input needs at least one column");
 	hipStream_t s = n2_stream(stream);
 	if (int rc = prepare_grads(grid, "n2_grid_backward_fused", s, mode, n_points)) return rc;
-	if (n_points == 0) return N2_OK;
+	if (n_points == 0) return sums ? n2_slab_reduce_launch(stream, *sums) : N2_OK;
+	N2ScatterRider rider;
+	if (sums) rider.sums = *sums;
 	N2ProfScope prof(N2_PROF_GRID_BACKWARD_PARAMS, s);
 	return launch_scatter(grid, s, d_xyz_rows, 1, n_cols, n_points, reinterpret_cast<const __half*>(d_dL_dy), d_dL_ddLdx,
-	                      reinterpret_cast<const __half*>(d_dL_dy_second), grid->grads, nullptr, mode == N2_GRAD_ACCUMULATE, d_index, n_cols);
+	                      reinterpret_cast<const __half*>(d_dL_dy_second), grid->grads, nullptr, mode == N2_GRAD_ACCUMULATE, d_index, n_cols, rider);
 }
 
 N2_API int n2_grid_backward_backward_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz,

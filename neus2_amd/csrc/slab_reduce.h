@@ -88,21 +88,52 @@ __device__ __forceinline__ void n2_image_combine_unit(const N2ImageCombine& r, u
 	done(g + 1, h[1]);
 }
 
-// Unit `unit` of the plan, run by the 256 threads of a workgroup.  A unit owns 32 consecutive parameters (one 128-byte line
+// Unit `unit` of the plan, run by 256 threads (numbered tid) of a workgroup, which may run several units at once, each with a fold of its
+// own (units past the last one do nothing).  A unit owns 32 consecutive parameters (one 128-byte line
 // of every slab): 8 lanes cover the line with 16-byte loads, 32 lane groups share the slabs, eight loads in flight per
 // lane, LDS folds the groups.  n_params is a multiple of 16, so lines are never ragged.  The fp16 gradient is stored, and
 // done(address of the stored gradient, its value) is called by the thread that stored it.  Contains one __syncthreads().
 template <class Done>
-__device__ __forceinline__ void n2_slab_reduce_unit(const N2SlabReduce& r, uint32_t unit, float (*fold)[33], Done done) {
-	const uint32_t tid = threadIdx.x;
-	if (unit >= r.units_a + r.units_b) {  // the extra sum
+__device__ __forceinline__ void n2_slab_reduce_unit(const N2SlabReduce& r, uint32_t unit, float (*fold)[33], Done done, const uint32_t tid = threadIdx.x) {
+	const bool extra = unit >= r.units_a + r.units_b, first = unit < r.units_a;
+	const float* partials = first ? r.pa : r.pb;
+	const uint32_t n_slabs = first ? r.slabs_a : r.slabs_b, n_params = first ? r.params_a : r.params_b, line = first ? unit : unit - r.units_a;
+	_Float16* grads = first ? r.ga : r.gb;
+	const int accumulate = first ? r.acc_a : r.acc_b;
+	if (extra) {  // the extra sum
 		float s = 0.f;
-		for (uint32_t i = tid; i < r.extra_n; i += 256) s += r.extra[i];
+		if (unit < r.units)
+			for (uint32_t i = tid; i < r.extra_n; i += 256) s += r.extra[i];
 #pragma unroll
 		for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
 		if ((tid & 63u) == 0) fold[0][tid >> 6] = s;
-		__syncthreads();
-		if (tid == 0) {
+	} else {
+		const uint32_t q = tid & 7u, grp = tid >> 3;
+		const uint32_t i = line * 32 + q * 4;
+		float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+		if (i < n_params) {
+			const float* p = partials + i;
+			uint32_t k = grp;
+			for (; k + 7 * 32 < n_slabs; k += 8 * 32) {
+				float4 v[8];
+#pragma unroll
+				for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(p + (size_t)(k + u * 32) * n_params);
+#pragma unroll
+				for (int u = 0; u < 8; ++u) { acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w; }
+			}
+			for (; k < n_slabs; k += 32) {
+				const float4 v = *reinterpret_cast<const float4*>(p + (size_t)k * n_params);
+				acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+			}
+		}
+		fold[grp][q * 4 + 0] = acc.x;
+		fold[grp][q * 4 + 1] = acc.y;
+		fold[grp][q * 4 + 2] = acc.z;
+		fold[grp][q * 4 + 3] = acc.w;
+	}
+	__syncthreads();
+	if (extra) {
+		if (tid == 0 && unit < r.units) {
 			const float t = (fold[0][0] + fold[0][1]) + (fold[0][2] + fold[0][3]);
 			const _Float16 h = r.extra_acc ? (_Float16)((float)r.extra_out[0] + t) : (_Float16)t;
 			r.extra_out[0] = h;
@@ -110,34 +141,6 @@ __device__ __forceinline__ void n2_slab_reduce_unit(const N2SlabReduce& r, uint3
 		}
 		return;
 	}
-	const bool first = unit < r.units_a;
-	const float* partials = first ? r.pa : r.pb;
-	const uint32_t n_slabs = first ? r.slabs_a : r.slabs_b, n_params = first ? r.params_a : r.params_b, line = first ? unit : unit - r.units_a;
-	_Float16* grads = first ? r.ga : r.gb;
-	const int accumulate = first ? r.acc_a : r.acc_b;
-	const uint32_t q = tid & 7u, grp = tid >> 3;
-	const uint32_t i = line * 32 + q * 4;
-	float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-	if (i < n_params) {
-		const float* p = partials + i;
-		uint32_t k = grp;
-		for (; k + 7 * 32 < n_slabs; k += 8 * 32) {
-			float4 v[8];
-#pragma unroll
-			for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(p + (size_t)(k + u * 32) * n_params);
-#pragma unroll
-			for (int u = 0; u < 8; ++u) { acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w; }
-		}
-		for (; k < n_slabs; k += 32) {
-			const float4 v = *reinterpret_cast<const float4*>(p + (size_t)k * n_params);
-			acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
-		}
-	}
-	fold[grp][q * 4 + 0] = acc.x;
-	fold[grp][q * 4 + 1] = acc.y;
-	fold[grp][q * 4 + 2] = acc.z;
-	fold[grp][q * 4 + 3] = acc.w;
-	__syncthreads();
 	// 8 lanes per parameter fold 4 groups each, then a shuffle tree
 	const uint32_t pl = tid >> 3, part = tid & 7u;
 	float t = fold[part * 4][pl] + fold[part * 4 + 1][pl] + fold[part * 4 + 2][pl] + fold[part * 4 + 3][pl];

@@ -341,6 +341,33 @@ def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and bool((got[0][0] != 0).any())
 
 
+# edges of the workgroups that take the input gradient along, tiles of one and of two points per thread, streamed Jacobians, tables of other widths, and
+# a scatter that has no workspace and so takes nothing along
+@pytest.mark.parametrize("n,levels,room", [(1, 16, True), (511, 16, True), (513, 16, True), (24576, 16, True), (24577, 16, True), (180001, 16, True), (5003, 1, True), (5003, 3, True), (5003, 16, False)])
+def test_input_gradient_beside_the_scatter(n, levels, room):
+    """Both gradients from one call are those of two."""
+    from neus2_amd.tcnn_api import GRAD_IGNORE, GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(**{**CFG, "n_levels": levels})
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = (torch.rand(gg.n_params(), device="cuda", generator=gen) * 2 - 1).half()
+    dg = torch.zeros_like(dp)
+    gg.set_params(dp, dg)
+    if room:
+        assert gg.reserve_scatter_workspace(n)
+    x = torch.rand((3, n), device="cuda", generator=gen)
+    dy = torch.randn((2 * levels, n), device="cuda", generator=gen).half()
+    _, ctx = gg.forward(x, prepare_input_gradients=True)
+    dx = gg.backward(ctx, x, dy, want_input_grad=True, mode=GRAD_OVERWRITE)
+    both = dg.clone()
+    assert torch.equal(dx, gg.backward(ctx, x, dy, want_input_grad=True, mode=GRAD_IGNORE)) and bool((dx != 0).any())
+    dg.fill_(9.0)
+    gg.backward(None, x, dy, mode=GRAD_OVERWRITE)
+    if room:
+        assert torch.equal(both, dg)
+    else:  # atomics add in the order of their arrival, a rounding to fp16 each
+        assert rel_l2(host(both), host(dg)) < RTOL
+
+
 # batches whose buckets hold few records, up to the last one and the next; points that all fall into a few cells, in turn (no runs to merge), so that
 # single buckets hold more records than sums can be claimed for; tables of few and of small buckets
 @pytest.mark.parametrize("n,where,table", [(1, "anywhere", (16, 19)), (511, "anywhere", (16, 19)), (5003, "anywhere", (16, 19)), (16384, "anywhere", (16, 19)), (16385, "anywhere", (16, 19)),
