@@ -34,6 +34,7 @@ struct n2_grid {
 	unsigned char* ws;
 	uint64_t ws_bytes;
 	uint32_t ws_max_points;
+	uint64_t ws_partials;  // where the images of split buckets stand in it
 	bool lattice_order;  // points of the next forwards come in lattice order (n2_grid_set_point_order)
 };
 
@@ -1239,6 +1240,7 @@ N2_API int n2_grid_create(uint32_t n_levels, uint32_t n_features_per_level, uint
 	g->ws = nullptr;
 	g->ws_bytes = 0;
 	g->ws_max_points = 0;
+	g->ws_partials = 0;
 	g->lattice_order = false;
 	g->costs_set = false;
 	*out = g;
@@ -1430,7 +1432,6 @@ N2_API int n2_grid_corner_indices(n2_grid_t* grid, n2_stream_t stream, const flo
 }
 
 static bool uses_bucketed(const n2_grid_t* grid, uint32_t n_points);
-static uint32_t bucket_groups(const n2_grid_t* grid, uint32_t level, uint32_t n_points, uint32_t tiles);
 
 // OVERWRITE: the gradient buffer starts from zero.  The bucketed scatter writes every entry itself (with plain stores),
 // so only the scatter with atomics needs the buffer cleared beforehand.
@@ -1460,8 +1461,7 @@ static bool bucket_supported(const n2_grid_t* grid) {
 struct BucketCarve {
 	uint64_t vals, keys, offsets, partials, total;
 };
-static uint32_t split_images(const n2_grid_t* grid, uint32_t n_points);
-static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points) {
+static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points, uint32_t images) {
 	const uint64_t tiles = n_bin_tiles(grid, max_points), L = grid->tab.n_levels;
 	const uint64_t n_rec = L * tiles * bin_records(bin_per_thread(grid, max_points));
 	auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
@@ -1472,11 +1472,10 @@ static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points) {
 	c.partials = up(c.offsets + L * tiles * (BKT_MAX + 1) * sizeof(uint16_t));
 	// (a batch of half as many points per tile has twice the tiles and bucket offsets: the images of a larger one stand behind those, too)
 	const uint32_t largest = n2_bin_single_points(grid->tab.n_levels, BIN_BLOCK);
-	if (max_points > largest) c.partials = std::max(c.partials, bucket_carve(grid, largest).partials);
-	c.total = up(c.partials + (uint64_t)split_images(grid, max_points) * BKT_ENTRIES * sizeof(float2));
+	if (max_points > largest) c.partials = std::max(c.partials, bucket_carve(grid, largest, 0u).partials);
+	c.total = up(c.partials + (uint64_t)images * BKT_ENTRIES * sizeof(float2));
 	return c;
 }
-static uint64_t bucket_ws_bytes(const n2_grid_t* grid, uint32_t max_points) { return bucket_carve(grid, max_points).total; }
 
 // With a workspace every batch size takes the bucketed scatter, whose result does not depend on the order in which
 // workgroups run; the scatter with atomics (no workspace, or more points than it was sized for) sums in arrival order.
@@ -1487,65 +1486,55 @@ static bool uses_bucketed(const n2_grid_t* grid, uint32_t n_points) {
 // encoded against that size); the others take the largest size (a power of two, at most 4096 entries and at most BKT_MAX
 // buckets) under which a bucket holds at most `target` of the level's 8 records per point, or the smallest there is: small
 // dense levels get many small buckets instead of few that outlast the others.  When even the smallest buckets hold more than
-// 65536, they stay large and are split (bucket_groups).
+// 65536, they stay large and are split.
 // The target is 16384 for grid_reduce_kernel (8192 and 32768: the same within 2 %, 65536: 49 us against 36 at 1.2e5 points, where a dense
 // level's few workgroups outlast the others) and 512, a record per thread, for grid_reduce_few_kernel.
-static uint32_t bucket_shift(const n2_grid_t* grid, uint32_t level, uint32_t n_points, uint64_t target) {
+static uint32_t bucket_shift(const n2_grid_t* grid, uint32_t level, uint32_t n_points, uint32_t target) {
 	if ((grid->tab.pair_levels >> level) & 1u) return BKT_SHIFT;
 	const uint32_t entries = grid->tab.entries[level];
+	const uint64_t records = (uint64_t)n_points * 8;
 	for (uint32_t shift = BKT_SHIFT; shift >= BKT_MIN_SHIFT; --shift) {
 		const uint32_t nb = (entries + (1u << shift) - 1u) >> shift, finer = (entries + (1u << (shift - 1u)) - 1u) >> (shift - 1u);
 		if (nb > BKT_MAX) break;
-		const uint64_t records = (uint64_t)n_points * 8 / nb;
-		if (records <= target || (records <= 65536u && (shift == BKT_MIN_SHIFT || finer > BKT_MAX))) return shift;
+		if (records < (target + 1ull) * nb || (records < 65537ull * nb && (shift == BKT_MIN_SHIFT || finer > BKT_MAX))) return shift;
 	}
 	return BKT_SHIFT;
 }
-// Whether a batch takes grid_reduce_few_kernel: on average its buckets hold no more records than threads on levels of pair records, which is two thirds of
-// the claims there are, and 2048 on the others, whose buckets are the smallest there can be.  With the default table that is up to 16 384 points.
-// Encoding forward and backward in us, grid_reduce_kernel | this one: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5, 8192 33.5 | 29.1, 12 288 35.5 | 32.7,
-// 16 384 37.7 | 37.0; along rays 3000 28.7 | 25.2, 16 384 34.9 | 31.1, 32 768 41.8 | 43.2.
-static bool few_records(const n2_grid_t* grid, uint32_t n_points) {
-	if (n_bin_tiles(grid, n_points) > FEW_TILES) return false;
-	for (uint32_t l = 0; l < grid->tab.n_levels; ++l) {
+static inline uint32_t bucket_count(uint32_t entries, uint32_t shift) { return (entries + (1u << shift) - 1u) >> shift; }
+
+// A batch's buckets.  few: it takes grid_reduce_few_kernel.  That is where on average its buckets hold no more records than threads on levels of pair
+// records, which is two thirds of the claims there are, and 2048 on the others, whose buckets are the smallest there can be: with the default table
+// up to 16 384 points.  Encoding forward and backward in us, grid_reduce_kernel | grid_reduce_few_kernel: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5,
+// 8192 33.5 | 29.1, 12 288 35.5 | 32.7, 16 384 37.7 | 37.0; along rays 3000 28.7 | 25.2, 16 384 34.9 | 31.1, 32 768 41.8 | 43.2.
+// groups: workgroups a bucket is split over; images: fp32 images of all split buckets (never more for a smaller batch: the groups per bucket grow with it).
+struct BatchBuckets {
+	bool few;
+	uint8_t shift[N2_MAX_LEVELS];
+	uint32_t count[N2_MAX_LEVELS], groups[N2_MAX_LEVELS], images;
+};
+static BatchBuckets batch_buckets(const n2_grid_t* grid, uint32_t n_points) {
+	BatchBuckets b;
+	const uint32_t tiles = n_bin_tiles(grid, n_points), L = grid->tab.n_levels;
+	b.few = tiles <= FEW_TILES;
+	for (uint32_t l = 0; l < L && b.few; ++l) {
 		const bool pair = (grid->tab.pair_levels >> l) & 1u;
-		const uint32_t shift = bucket_shift(grid, l, n_points, FEW_BLOCK), nb = (grid->tab.entries[l] + (1u << shift) - 1u) >> shift;
-		if ((uint64_t)n_points * (pair ? 4u : 8u) > (uint64_t)nb * (pair ? FEW_BLOCK : 4u * FEW_BLOCK)) return false;
+		b.shift[l] = (uint8_t)bucket_shift(grid, l, n_points, FEW_BLOCK);
+		b.few = (uint64_t)n_points * (pair ? 4u : 8u) <= (uint64_t)bucket_count(grid->tab.entries[l], b.shift[l]) * (pair ? FEW_BLOCK : 4u * FEW_BLOCK);
 	}
-	return true;
-}
-static uint32_t bucket_shift_for(const n2_grid_t* grid, uint32_t level, uint32_t n_points) {
-	return bucket_shift(grid, level, n_points, few_records(grid, n_points) ? FEW_BLOCK : 16384u);
-}
-static inline uint32_t level_buckets(const n2_grid_t* grid, uint32_t level, uint32_t n_points) {
-	const uint32_t shift = bucket_shift_for(grid, level, n_points);
-	return (grid->tab.entries[level] + (1u << shift) - 1u) >> shift;
-}
-
-static uint32_t bucket_groups(const n2_grid_t* grid, uint32_t level, uint32_t n_points, uint32_t tiles) {
-	const uint32_t nb = level_buckets(grid, level, n_points);
-	const uint64_t per_bucket = (uint64_t)n_points * 8 / nb;
-	uint32_t groups = (uint32_t)((per_bucket + 65535) / 65536);
-	if (groups > N2_CMB_MAX_GROUPS) groups = N2_CMB_MAX_GROUPS;
-	if (groups > tiles) groups = tiles;
-	if (groups < 1) groups = 1;
-	return groups;
-}
-
-// fp32 images of all split buckets of a batch (never more for a smaller batch: the groups per bucket grow with the batch)
-static uint32_t split_images(const n2_grid_t* grid, uint32_t n_points) {
-	const uint32_t tiles = n_bin_tiles(grid, n_points);
-	uint32_t n = 0;
-	for (uint32_t l = 0; l < grid->tab.n_levels; ++l) {
-		const uint32_t nb = level_buckets(grid, l, n_points), groups = bucket_groups(grid, l, n_points, tiles);
-		if (groups > 1) n += nb * groups;
+	b.images = 0;
+	for (uint32_t l = 0; l < L; ++l) {
+		if (!b.few) b.shift[l] = (uint8_t)bucket_shift(grid, l, n_points, 16384u);
+		b.count[l] = bucket_count(grid->tab.entries[l], b.shift[l]);
+		const uint64_t per_bucket = (uint64_t)n_points * 8 / b.count[l];
+		b.groups[l] = std::max<uint32_t>(1u, std::min<uint64_t>((per_bucket + 65535) / 65536, std::min(N2_CMB_MAX_GROUPS, tiles)));
+		if (b.groups[l] > 1) b.images += b.count[l] * b.groups[l];
 	}
-	return n;
+	return b;
 }
 
 N2_API uint64_t n2_grid_workspace_bytes(const n2_grid_t* grid, uint32_t max_points) {
 	if (!grid || !bucket_supported(grid)) return 0;
-	return bucket_ws_bytes(grid, max_points);
+	return bucket_carve(grid, max_points, batch_buckets(grid, max_points).images).total;
 }
 
 N2_API int n2_grid_set_workspace(n2_grid_t* grid, void* d_workspace, uint64_t n_bytes, uint32_t max_points) {
@@ -1560,6 +1549,7 @@ N2_API int n2_grid_set_workspace(n2_grid_t* grid, void* d_workspace, uint64_t n_
 	grid->ws = reinterpret_cast<unsigned char*>(d_workspace);
 	grid->ws_bytes = n_bytes;
 	grid->ws_max_points = bucket_supported(grid) ? max_points : 0;
+	grid->ws_partials = bucket_carve(grid, max_points, 0u).partials;
 	return N2_OK;
 }
 
@@ -1580,19 +1570,19 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	const dim3 bd(BIN_BLOCK);
 	// The records of this batch are packed as for a workspace of exactly this size (values, keys, offsets one behind the
 	// other); the images of split buckets stand where the workspace's own size put them.
-	const BucketCarve now = bucket_carve(grid, n_points), full = bucket_carve(grid, grid->ws_max_points);
+	const BucketCarve now = bucket_carve(grid, n_points, 0u);
 	uint32_t* rec_vals = reinterpret_cast<uint32_t*>(grid->ws + now.vals);
 	uint16_t* rec_keys = reinterpret_cast<uint16_t*>(grid->ws + now.keys);
 	uint16_t* offsets = reinterpret_cast<uint16_t*>(grid->ws + now.offsets);
-	float2* partials = reinterpret_cast<float2*>(grid->ws + full.partials);
+	float2* partials = reinterpret_cast<float2*>(grid->ws + grid->ws_partials);
 	N2BucketPlan plan;
 	uint32_t wg = 0, images = 0, split = 0;
 	N2LevelTable tab = grid->tab;  // with this launch's bucket sizes
 	const bool few = tiles <= FLIGHT_TILES;
+	const BatchBuckets buckets = batch_buckets(grid, n_points);
 	for (uint32_t l = 0; l < L; ++l) {
-		tab.bucket_shift[l] = (uint8_t)bucket_shift_for(grid, l, n_points);
-		const uint32_t nb = level_buckets(grid, l, n_points);
-		const uint32_t groups = bucket_groups(grid, l, n_points, tiles);
+		const uint32_t nb = buckets.count[l], groups = buckets.groups[l];
+		tab.bucket_shift[l] = buckets.shift[l];
 		plan.wg_begin[l] = wg;
 		plan.n_buckets[l] = nb;
 		plan.groups[l] = groups;
@@ -1635,7 +1625,7 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	else bin(std::integral_constant<uint32_t, 2>());
 	N2_LAUNCH_CHECK();
 #define LAUNCH(F) grid_reduce_kernel<F><<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials)
-	if (few_records(grid, n_points))
+	if (buckets.few)
 		grid_reduce_few_kernel<<<dim3(wg), dim3(FEW_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
 	else if (few) LAUNCH(2);
 	else LAUNCH(4);
