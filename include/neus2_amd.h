@@ -424,6 +424,33 @@ int n2_sdf_normals_and_eikonal_loss(n2_stream_t stream, uint32_t n, uint32_t enc
                                     n2_half* d_dL_doutput, float* d_dL_dnormal, n2_half* d_second_order_input, float* d_loss, void* d_workspace,
                                     uint64_t workspace_bytes);
 
+/* The whole step of such a caller in two calls.  The buffers are the caller's, n columns each (fp16 SoA but where stated), 16-byte aligned and kept from
+ * the forward to the backward.  Behind the encoding's rows, input and second_order_input hold zeros, as do rows 1.. of dL_doutput, which the caller
+ * clears once: the calls may write zeros there, but need not.
+ *   n2_sdf_forward_and_loss  = n2_sdf_pack_input, n2_grid_forward with the Jacobian, n2_mlp_forward_and_input_gradient of output 0 and
+ *                              n2_sdf_normals_and_eikonal_loss (for a network of 48 inputs over 32 features in two launches and the loss's sum)
+ *   n2_sdf_loss_backward     = n2_mlp_backward_and_second_order and n2_grid_backward_fused, into the gradient buffers of both objects; of
+ *                              dL_dinput only the encoding's rows are defined */
+typedef struct n2_sdf_buffers {
+	n2_half* input;              /* [input_width] */
+	float* dy_dx;                /* fp32 [encoding_width][n][3] */
+	n2_half* output;             /* [16] */
+	n2_half* dsdf_dinput;        /* [input_width] */
+	float* normal;               /* fp32 [3] */
+	n2_half* dL_doutput;         /* [16] */
+	float* dL_dnormal;           /* fp32 [3] */
+	n2_half* second_order_input; /* [input_width] */
+	n2_half* dL_dinput;          /* [input_width] */
+	float* loss;                 /* one float */
+	void* workspace;             /* n2_sdf_step_workspace_bytes(n) */
+	uint64_t workspace_bytes;
+} n2_sdf_buffers;
+uint64_t n2_sdf_step_workspace_bytes(uint32_t n);
+int n2_sdf_forward_and_loss(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n,
+                            float ek_weight, float loss_scale, const n2_sdf_buffers* buffers);
+int n2_sdf_loss_backward(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n,
+                         const n2_sdf_buffers* buffers, n2_grad_mode mode);
+
 /* ------------------------------------------------------------------------
  * Adam on fp32 master weights with an fp16 working copy: tcnn's Adam as the
  * trainer runs it, Trainer::optimizer_step(stream, LOSS_SCALE) at

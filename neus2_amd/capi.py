@@ -70,6 +70,12 @@ class OccupancyBuffers(C.Structure):
                 ("ema_step", C.c_uint32), ("n_uniform", C.c_uint32), ("rng_state", C.c_uint64), ("rng_inc", C.c_uint64)]
 
 
+class SdfBuffers(C.Structure):
+    """struct n2_sdf_buffers"""
+    _fields_ = [(name, C.c_void_p) for name in ("input", "dy_dx", "output", "dsdf_dinput", "normal", "dL_doutput", "dL_dnormal", "second_order_input", "dL_dinput",
+                                                "loss", "workspace")] + [("workspace_bytes", C.c_uint64)]
+
+
 class N2Error(RuntimeError):
     """A C-ABI call returned a non-zero status (mirrors the reference's std::runtime_error)."""
 
@@ -117,6 +123,8 @@ def lib():
         _lib.n2_sampler_workspace_bytes.argtypes = [C.c_uint32]
         _lib.n2_sdf_eikonal_workspace_bytes.restype = C.c_uint64
         _lib.n2_sdf_eikonal_workspace_bytes.argtypes = [C.c_uint32]
+        _lib.n2_sdf_step_workspace_bytes.restype = C.c_uint64
+        _lib.n2_sdf_step_workspace_bytes.argtypes = [C.c_uint32]
         _lib.n2_trainer_workspace_bytes.restype = C.c_uint64
         _lib.n2_trainer_workspace_bytes.argtypes = [C.c_void_p]
         _lib.n2_trainer_destroy.restype = None

@@ -12,6 +12,7 @@
 #include "slab_reduce.h"
 #include "grid_device.h"
 
+#include <algorithm>
 #include <new>
 
 typedef _Float16 hf;
@@ -832,6 +833,73 @@ N2_API int n2_sdf_normals_and_eikonal_loss(n2_stream_t stream, uint32_t n, uint3
 	sdf_loss_sum_kernel<<<dim3(1), dim3(256), 0, s>>>(parts, fgrid(n).x, 1.f / (float)n, d_loss);
 	N2_LAUNCH_CHECK();
 	return N2_OK;
+}
+
+N2_API uint64_t n2_sdf_step_workspace_bytes(uint32_t n) {
+	return std::max<uint64_t>(n2_sdf_eikonal_workspace_bytes(n), 4ull * n2_fused_sdf_eikonal_parts(n));
+}
+
+static int check_sdf_step(const char* fn, const n2_grid_t* grid, const n2_mlp_t* mlp, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n,
+                          const n2_sdf_buffers* b, uint32_t& enc_w, uint32_t& in_w) {
+	N2_REQUIRE(grid != nullptr && mlp != nullptr && b != nullptr && d_xyz != nullptr, "%s: null argument", fn);
+	N2_REQUIRE(n > 0 && n % 8 == 0 && n <= (1u << 28), "%s: batch size %u is not a multiple of 8 up to 2^28", fn, n);
+	N2_REQUIRE(point_stride >= 1 && dim_stride >= 1, "%s: strides must be >= 1", fn);
+	N2_REQUIRE(b->input && b->dy_dx && b->output && b->dsdf_dinput && b->normal && b->dL_doutput && b->dL_dnormal && b->second_order_input && b->dL_dinput && b->loss &&
+	           b->workspace, "%s: null buffer", fn);
+	const uintptr_t all = reinterpret_cast<uintptr_t>(b->input) | reinterpret_cast<uintptr_t>(b->output) | reinterpret_cast<uintptr_t>(b->dsdf_dinput) |
+	                      reinterpret_cast<uintptr_t>(b->dL_doutput) | reinterpret_cast<uintptr_t>(b->second_order_input) | reinterpret_cast<uintptr_t>(b->dL_dinput);
+	N2_REQUIRE(all % 16 == 0, "%s: buffers must be 16-byte aligned", fn);
+	enc_w = n2_grid_output_width(grid);
+	in_w = n2_mlp_input_width(mlp);
+	N2_REQUIRE(in_w >= 3 + enc_w, "%s: a network of %u inputs does not hold 3 + %u rows", fn, in_w, enc_w);
+	N2_REQUIRE(b->workspace_bytes >= n2_sdf_step_workspace_bytes(n), "%s: workspace of %llu bytes, %llu needed", fn, (unsigned long long)b->workspace_bytes,
+	           (unsigned long long)n2_sdf_step_workspace_bytes(n));
+	return N2_OK;
+}
+
+N2_API int n2_sdf_forward_and_loss(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n,
+                                   float ek_weight, float loss_scale, const n2_sdf_buffers* b) {
+	const char* fn = "n2_sdf_forward_and_loss";
+	uint32_t enc_w, in_w;
+	if (int rc = check_sdf_step(fn, grid, mlp, d_xyz, point_stride, dim_stride, n, b, enc_w, in_w)) return rc;
+	N2_REQUIRE(n2_mlp_weights(mlp) != nullptr, "%s: n2_mlp_set_params has not been called", fn);
+	if (int rc = n2_grid_forward_sdf_input(grid, stream, d_xyz, point_stride, dim_stride, n, b->input, b->dy_dx)) return rc;
+	// (the kernel's lanes hold sixteen levels and the coordinates of a network with one hidden layer)
+	if (in_w == 48 && enc_w == 32 && n2_mlp_n_params(mlp) == 64 * 48 + 16 * 64) {
+		hipStream_t s = n2_stream(stream);
+		float* parts = reinterpret_cast<float*>(b->workspace);
+		if (int rc = n2_fused_sdf_eikonal(s, n2_mlp_weights(mlp), n, b->input, b->dy_dx, b->output, b->dsdf_dinput, b->normal, ek_weight, loss_scale / (float)n,
+		                                  b->dL_doutput, b->dL_dnormal, b->second_order_input, parts)) return rc;
+		sdf_loss_sum_kernel<<<dim3(1), dim3(256), 0, s>>>(parts, n2_fused_sdf_eikonal_parts(n), 1.f / (float)n, b->loss);
+		N2_LAUNCH_CHECK();
+		return N2_OK;
+	}
+	if (int rc = n2_mlp_forward_and_input_gradient(mlp, stream, 0, b->input, n, b->output, N2_LAYOUT_SOA, b->dsdf_dinput)) return rc;
+	return n2_sdf_normals_and_eikonal_loss(stream, n, enc_w, in_w, b->output, b->dsdf_dinput, b->dy_dx, b->normal, ek_weight, loss_scale, b->dL_doutput, b->dL_dnormal,
+	                                       b->second_order_input, b->loss, b->workspace, b->workspace_bytes);
+}
+
+N2_API int n2_sdf_loss_backward(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n,
+                                const n2_sdf_buffers* b, n2_grad_mode mode) {
+	const char* fn = "n2_sdf_loss_backward";
+	uint32_t enc_w, in_w;
+	if (int rc = check_sdf_step(fn, grid, mlp, d_xyz, point_stride, dim_stride, n, b, enc_w, in_w)) return rc;
+	// The weights' slabs are summed beside the encoding's scatter, unless the network's owner keeps them pending.
+	const bool beside = !n2_mlp_defers(mlp);
+	if (beside) {
+		if (int rc = n2_mlp_set_deferred_reduction(mlp, 1)) return rc;
+	}
+	N2SlabReduce sums = {};
+	int rc = n2_mlp_backward_and_second_order_indexed(mlp, stream, b->input, 0, nullptr, n, b->dL_doutput, N2_LAYOUT_SOA, b->dL_dinput, b->second_order_input,
+	                                                  nullptr, mode, enc_w <= 32);  // (of 48 inputs that pass stores rows 3..34 alone)
+	if (beside) {
+		if (rc == N2_OK) rc = n2_mlp_reduce_deferred_plan(mlp, nullptr, nullptr, 0, nullptr, 0, &sums);
+		n2_mlp_drop_pending(mlp);
+		n2_mlp_set_deferred_reduction(mlp, 0);
+	}
+	if (rc != N2_OK) return rc;
+	return n2_grid_backward_fused_and_sums(grid, stream, d_xyz, point_stride, dim_stride, n, b->dL_dinput + (size_t)3 * n, b->dL_dnormal,
+	                                       b->dsdf_dinput + (size_t)3 * n, nullptr, mode, &sums);
 }
 
 // The inference paths for points in no particular order gather the features into the rows of the SDF net's input, at the

@@ -840,6 +840,157 @@ static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream
 // 5000 points: 1000 9.4 | 7.2, 8192 11.7 | 9.7.)
 constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 256 * FQ_POINTS;
 
+// ----------------------------------------------------------------------------
+// The SDF network on its own (48 inputs: coordinates, 32 features, padding) with the eikonal loss: network, d sdf / d input, normals from the
+// encoding's fp32 Jacobian, the loss's terms and everything the backward takes, in one pass over the input rows and the Jacobian.
+// ----------------------------------------------------------------------------
+struct SdfEikonalArgs {
+	const hf* weights;
+	uint32_t N;
+	const hf* input;       // [48][N]
+	const float* dy_dx;    // [32][N][3]
+	hf* output;            // [16][N]
+	hf* dsdf;              // [48][N]
+	float* normal;         // [3][N]
+	float ek_weight, scale;
+	hf* dL_dy;             // [16][N], row 0
+	float* v;              // [3][N]
+	hf* v_in;              // [48][N], rows 0 .. 34
+	float* parts;          // a workgroup's part of the loss's sum
+};
+constexpr int SE_FRAGS = C_W0;  // the SDF net's fragments come first
+
+// d sdf / d input's rows behind the features: tile row t < 3 is a coordinate, the others are the padding inputs (whose weights count like any)
+__device__ __forceinline__ int sdf_tail_col(int t) { return t < 3 ? t : 32 + t; }
+// Bound by memory: 678 bytes a point, of which the Jacobian's rows are 384; at 2^18 points 38.7 us, 4.6 TB/s (network and normals in two launches 17.7 + 30.0),
+// at 2^14 7.0 (6.1 + 6.0).  No store stands in a branch (lanes behind the last point repeat it), so that a tile waits for its own loads alone, and matrices are
+// addressed by a scalar row and a 32-bit offset: with 64-bit addresses per lane and the next tile's Jacobian under way too the registers spill (56 us).
+template <bool STREAM>
+__global__ void __launch_bounds__(FF_BLOCK, 2) sdf_eikonal_forward_kernel(const SdfEikonalArgs a) {
+	constexpr int RAW = mlp_n_params<3, 1>();
+	__shared__ __align__(16) hf F[SE_FRAGS * 512], raw[RAW];
+	__shared__ float part[FF_BLOCK / 64];
+	const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
+	const uint32_t N = a.N, n_tiles = (N + 31u) / 32u;
+	const uint32_t wave_gid = blockIdx.x * (FF_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (FF_BLOCK / 64);
+	// Of a matrix [rows][N], row u + 4 g of the lane's point: the row u stands in a scalar address, the rest in a 32-bit lane offset.
+	auto at = [&](auto* matrix, uint32_t u, uint32_t lane_at, uint32_t width) __attribute__((always_inline)) {
+		typedef typename std::conditional<std::is_const<std::remove_pointer_t<decltype(matrix)>>::value, const char, char>::type bytes;
+		typedef std::remove_pointer_t<decltype(matrix)> value;
+		return reinterpret_cast<value*>(reinterpret_cast<bytes*>(matrix + (size_t)u * N * width) + lane_at * (uint32_t)(sizeof(value) * width));
+	};
+	auto row_of = [](int r) { return 8u * (uint32_t)(r >> 2) + (uint32_t)(r & 3); };  // of D register r, without 4 g
+	struct Start {
+		hf feat[16], p[3];
+	};
+	auto start = [&](uint32_t tile) __attribute__((always_inline)) {
+		Start t;
+		const uint32_t col = min(tile * 32u + n, N - 1u), mine = 4u * g * N + col;
+#pragma unroll
+		for (int d = 0; d < 3; ++d) t.p[d] = *at(a.input, d, col, 1u);
+#pragma unroll
+		for (int r = 0; r < 16; ++r) t.feat[r] = *at(a.input, 3u + row_of(r), mine, 1u);
+		return t;
+	};
+	Start next = start(min(wave_gid, n_tiles - 1u));
+	copy_to_lds<FF_BLOCK, RAW / 8>(raw, a.weights);
+	__syncthreads();
+	for (int idx = threadIdx.x; idx < SE_FRAGS * 64; idx += FF_BLOCK) {
+		const int f = idx >> 6, l = idx & 63, m = l & 31, lg = l >> 5;
+		half8 w = zero8();
+		if (f < S_W0T) {
+			w = sdf_forward_frag(raw, 48, 32u, f, l);
+		} else if (f < S_DH) {
+			const int q = f - S_W0T, t = 32 * (q >> 2) + m, col = t < 32 ? 3 + t : sdf_tail_col(t - 32);
+#pragma unroll
+			for (int e = 0; e < 8; ++e) w[e] = col < 48 ? raw[chained_k(q & 3, lg, e) * 48 + col] : (hf)0;
+		} else {
+#pragma unroll
+			for (int e = 0; e < 8; ++e) w[e] = raw[MLP_WIDTH * 48 + chained_k(f - S_DH, lg, e)];
+		}
+		*reinterpret_cast<half8*>(F + (size_t)idx * 8) = w;
+	}
+	__syncthreads();
+	float term = 0.f;
+	for (uint32_t tile = wave_gid; tile < n_tiles; tile += n_waves) {
+		const uint32_t col_raw = tile * 32u + n, col = min(col_raw, N - 1u), next_tile = tile + n_waves;
+		const uint32_t mine = 4u * g * N + col;
+		const Start cur = next;
+		n2_float3 j[16];
+#pragma unroll
+		for (int r = 0; r < 16; ++r) j[r] = n2_load3<STREAM>(at(a.dy_dx, row_of(r), mine, 3u));
+		next = start(next_tile < n_tiles ? next_tile : tile);
+		half8 xs[3], h[4], dh[4];
+#pragma unroll
+		for (int r = 0; r < 16; ++r) xs[r >> 3][r & 7] = cur.feat[r];
+		xs[2] = zero8();
+#pragma unroll
+		for (int d = 0; d < 3; ++d) xs[2][d] = g == 0 ? cur.p[d] : (hf)0;
+		const half8 y = sdf_net(F, lane, xs, h);
+		// d sdf / d input: dh = mask * W_out[0, :], dX = W_0^T dh
+#pragma unroll
+		for (int c = 0; c < 4; ++c) dh[c] = mask8(frag(F, S_DH + c, lane), h[c]);
+		float16v dx0 = zero16(), dx1 = zero16();
+#pragma unroll
+		for (int c = 0; c < 4; ++c) dx0 = N2_MFMA(frag(F, S_W0T + c, lane), dh[c], dx0);
+#pragma unroll
+		for (int c = 0; c < 4; ++c) dx1 = N2_MFMA(frag(F, S_W0T + 4 + c, lane), dh[c], dx1);
+		const half8 lo = round8(dx0, 0), hi = round8(dx0, 8), tail = round8(dx1, 0);
+		float nrm[3];
+#pragma unroll
+		for (int d = 0; d < 3; ++d) nrm[d] = 0.f;
+#pragma unroll
+		for (int r = 0; r < 16; ++r) {
+			const float f = (float)(r < 8 ? lo[r & 7] : hi[r & 7]);
+			nrm[0] = fmaf(f, j[r].x, nrm[0]);
+			nrm[1] = fmaf(f, j[r].y, nrm[1]);
+			nrm[2] = fmaf(f, j[r].z, nrm[2]);
+		}
+		float len2 = 0.f, x[3];
+#pragma unroll
+		for (int d = 0; d < 3; ++d) {
+			const float gx = g == 0 ? (float)tail[d] : 0.f;  // the direct rows: the first half of the wave holds them
+			nrm[d] += __shfl_xor(nrm[d], 32);
+			nrm[d] += gx + __shfl_xor(gx, 32);
+			len2 = fmaf(nrm[d], nrm[d], len2);
+		}
+		const float len = fmaxf(sqrtf(len2), 1e-12f), k = 2.f * a.ek_weight * (len - 1.f) / len * a.scale, sdf = (float)y[0];
+		if (col_raw < N && g == 0) term += fabsf(sdf) + a.ek_weight * (len - 1.f) * (len - 1.f);
+#pragma unroll
+		for (int d = 0; d < 3; ++d) x[d] = nrm[d] * k;
+		// (the next tile's start has arrived before this one's stores are issued: where it is used the compiler would wait for those, too)
+#pragma unroll
+		for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(next.feat[r]));
+#pragma unroll
+		for (int d = 0; d < 3; ++d) asm volatile("" : "+v"(next.p[d]));
+#pragma unroll
+		for (int r = 0; r < 8; ++r) {
+			*at(a.output, row_of(r), mine, 1u) = y[r];
+			// (the second half's tail rows 4.. are columns 36..; of the first half's rows the coordinates are columns 0..2)
+			if (r < 3) *(at(a.dsdf, r, col, 1u) + (g ? (size_t)36 * N : 0)) = tail[r];
+			else *at(a.dsdf, 32u + row_of(r), mine, 1u) = tail[r];
+		}
+#pragma unroll
+		for (int r = 0; r < 16; ++r) {
+			*at(a.dsdf, 3u + row_of(r), mine, 1u) = r < 8 ? lo[r & 7] : hi[r & 7];
+			*at(a.v_in, 3u + row_of(r), mine, 1u) = (hf)fmaf(j[r].x, x[0], fmaf(j[r].y, x[1], j[r].z * x[2]));
+		}
+		float* const out3 = g ? a.v : a.normal;
+#pragma unroll
+		for (int d = 0; d < 3; ++d) out3[(size_t)d * N + col] = g ? x[d] : nrm[d];
+		// row 0 of dL_dy and row 0 of v_in by the first half, rows 1 and 2 by the second
+		const hf sign = (hf)((sdf > 0.f ? 1.f : sdf < 0.f ? -1.f : 0.f) * a.scale);
+		*(g ? a.v_in + (size_t)N + col : a.dL_dy + col) = g ? (hf)x[1] : sign;
+		a.v_in[(g ? (size_t)2 * N : 0) + col] = g ? (hf)x[2] : (hf)x[0];
+		tile_fence();
+	}
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) term += __shfl_xor(term, o);
+	if (lane == 0) part[threadIdx.x >> 6] = term;
+	__syncthreads();
+	if (threadIdx.x == 0) a.parts[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 static uint32_t fused_grid(uint32_t n, uint32_t most = 512u) {
 	const uint32_t tiles = (n + 31u) / 32u, blocks = (tiles + 3u) / 4u;
 	return blocks < most ? blocks : most;
@@ -944,6 +1095,29 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 	// take 28.8 | 26.8 | 31 us for 2^20 points and 45.8 | 38.2 | 41.6 for 2^21; every workgroup builds the fragments, which
 	// costs smaller batches more than it gains: 2^17 to 2^19 points 0.5 to 1.4 us)
 	field_fused_forward_kernel<false, false><<<dim3(fused_grid(n, n >= (1u << 20) ? 1024u : 512u)), dim3(FF_BLOCK), fused_lds(FF_SDF_COUNT), s>>>(a);
+	N2_LAUNCH_CHECK();
+	return N2_OK;
+}
+
+uint32_t n2_fused_sdf_eikonal_parts(uint32_t n) { return fused_grid(n); }
+int n2_fused_sdf_eikonal(hipStream_t s, const n2_half* weights, uint32_t n, const n2_half* input, const float* dy_dx, n2_half* output, n2_half* dsdf, float* normal,
+                         float ek_weight, float scale, n2_half* dL_dy, float* v, n2_half* v_in, float* parts) {
+	SdfEikonalArgs a{};
+	a.weights = reinterpret_cast<const hf*>(weights);
+	a.N = n;
+	a.input = reinterpret_cast<const hf*>(input);
+	a.dy_dx = dy_dx;
+	a.output = reinterpret_cast<hf*>(output);
+	a.dsdf = reinterpret_cast<hf*>(dsdf);
+	a.normal = normal;
+	a.ek_weight = ek_weight;
+	a.scale = scale;
+	a.dL_dy = reinterpret_cast<hf*>(dL_dy);
+	a.v = v;
+	a.v_in = reinterpret_cast<hf*>(v_in);
+	a.parts = parts;
+	if (n2_jacobian_streams(n, 32u)) sdf_eikonal_forward_kernel<true><<<dim3(fused_grid(n)), dim3(FF_BLOCK), 0, s>>>(a);
+	else sdf_eikonal_forward_kernel<false><<<dim3(fused_grid(n)), dim3(FF_BLOCK), 0, s>>>(a);
 	N2_LAUNCH_CHECK();
 	return N2_OK;
 }

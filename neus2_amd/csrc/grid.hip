@@ -104,7 +104,12 @@ template <uint32_t MODE, bool WANT_DYDX, bool STREAM>
 __device__ __forceinline__ void grid_forward_item(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t N,
                                                   const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                                   const __half2* __restrict__ params, __half* __restrict__ out,
-                                                  float* __restrict__ dy_dx) {
+                                                  float* __restrict__ dy_dx, __half* __restrict__ centred) {
+	if (centred != nullptr && level == 0 && i < N) {
+		const float* q = xyz + (size_t)i * point_stride;
+#pragma unroll
+		for (uint32_t d = 0; d < 3; ++d) centred[(size_t)d * N + i] = __float2half_rn(q[(size_t)d * dim_stride]) - __float2half_rn(0.5f);
+	}
 	const bool off = n2_level_masked(tab, level, min(i, N - 1u));
 	float feat[2] = {0.f, 0.f}, J[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
 	if (!__all(off)) {
@@ -129,16 +134,17 @@ __device__ __forceinline__ void grid_forward_item(const N2LevelTable& tab, uint3
 	}
 }
 
-// STREAM: dy_dx is written past the last-level cache (n2_jacobian_streams)
+// STREAM: dy_dx is written past the last-level cache (n2_jacobian_streams).  centred (or null): three rows for the positions minus 0.5, the SDF network's first inputs
 template <bool WANT_DYDX, bool STREAM>
 __global__ void __launch_bounds__(GRID_BLOCK) grid_forward_kernel(N2LevelTable tab, N2XcdPlan plan, uint32_t N, uint32_t tiles,
                                                                   const float* __restrict__ xyz, uint32_t point_stride,
                                                                   uint32_t dim_stride, const __half2* __restrict__ params,
-                                                                  __half* __restrict__ out, float* __restrict__ dy_dx) {
+                                                                  __half* __restrict__ out, float* __restrict__ dy_dx,
+                                                                  __half* __restrict__ centred) {
 	uint32_t level, tile;
 	if (!(plan.begin[N_XCD] ? n2_xcd_item(plan, tiles, level, tile) : n2_gather_item(blockIdx.x, blockIdx.y, plan.height, tab.n_levels, tiles, level, tile))) return;
 	const uint32_t i = tile * FWD_POINTS + threadIdx.x;
-#define CALL(M) grid_forward_item<M, WANT_DYDX, STREAM>(tab, level, i, N, xyz, point_stride, dim_stride, params, out, dy_dx)
+#define CALL(M) grid_forward_item<M, WANT_DYDX, STREAM>(tab, level, i, N, xyz, point_stride, dim_stride, params, out, dy_dx, centred)
 	N2_DISPATCH_MODE(tab.mode[level], CALL)
 #undef CALL
 }
@@ -1391,14 +1397,14 @@ static uint32_t make_xcd_plan(const n2_grid_t* grid, uint32_t tiles, N2XcdPlan& 
 	return longest;
 }
 
-N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
-                           uint32_t dim_stride, uint32_t n_points, n2_half* d_out, float* d_dy_dx) {
+static int grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
+                        uint32_t dim_stride, uint32_t n_points, n2_half* d_out, float* d_dy_dx, n2_half* d_centred) {
 	if (int rc = check_batch(grid, "n2_grid_forward", d_xyz, point_stride, dim_stride, n_points)) return rc;
 	if (n_points == 0) return N2_OK;
 	N2_REQUIRE(d_out != nullptr, "n2_grid_forward: d_out is null");
 	N2XcdPlan plan;
 	N2ProfScope prof(N2_PROF_GRID_FORWARD, n2_stream(stream));
-	if (grid->lattice_order && !d_dy_dx) {
+	if (grid->lattice_order && !d_dy_dx && !d_centred) {
 		const uint32_t tiles = n_tiles(n_points);
 		const dim3 grid_dim(tiles * grid->tab.n_levels);
 		grid_forward_point_kernel<<<grid_dim, dim3(GRID_BLOCK), 0, n2_stream(stream)>>>(grid->tab, n_points, tiles, d_xyz, point_stride, dim_stride,
@@ -1414,9 +1420,17 @@ N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_x
 	const bool streams = n2_jacobian_streams(n_points, grid->tab.n_levels * grid->n_features);
 	auto* const kernel = !d_dy_dx ? grid_forward_kernel<false, false> : streams ? grid_forward_kernel<true, true> : grid_forward_kernel<true, false>;
 	kernel<<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride, dim_stride, grid->params,
-	                                                  reinterpret_cast<__half*>(d_out), d_dy_dx);
+	                                                  reinterpret_cast<__half*>(d_out), d_dy_dx, reinterpret_cast<__half*>(d_centred));
 	N2_LAUNCH_CHECK();
 	return N2_OK;
+}
+N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
+                           uint32_t dim_stride, uint32_t n_points, n2_half* d_out, float* d_dy_dx) {
+	return grid_forward(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_out, d_dy_dx, nullptr);
+}
+int n2_grid_forward_sdf_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points, n2_half* d_input,
+                              float* d_dy_dx) {
+	return grid_forward(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_input ? d_input + (size_t)3 * n_points : nullptr, d_dy_dx, d_input);
 }
 
 N2_API int n2_grid_corner_indices(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
@@ -1704,20 +1718,27 @@ N2_API int n2_grid_backward(n2_grid_t* grid, n2_stream_t stream, const float* d_
 	                      mode == N2_GRAD_ACCUMULATE, nullptr, 0, rider);
 }
 
-N2_API int n2_grid_backward_fused(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
-                                  uint32_t dim_stride, uint32_t n_points, const n2_half* d_dL_dy,
-                                  const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy,
-                                  n2_grad_mode mode) {
+int n2_grid_backward_fused_and_sums(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
+                                    const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy, n2_grad_mode mode,
+                                    const N2SlabReduce* sums) {
 	if (int rc = check_batch(grid, "n2_grid_backward_fused", d_xyz, point_stride, dim_stride, n_points)) return rc;
 	N2_REQUIRE((d_dL_dy && d_dL_ddLdx && d_dL_dy_second) || n_points == 0, "n2_grid_backward_fused: d_dL_dy, d_dL_ddLdx and d_dL_dy_second are required");
 	N2_REQUIRE(mode == N2_GRAD_OVERWRITE || mode == N2_GRAD_ACCUMULATE, "n2_grid_backward_fused: mode must be OVERWRITE or ACCUMULATE");
 	hipStream_t s = n2_stream(stream);
 	if (int rc = prepare_grads(grid, "n2_grid_backward_fused", s, mode, n_points)) return rc;
-	if (n_points == 0) return N2_OK;
+	if (n_points == 0) return sums ? n2_slab_reduce_launch(stream, *sums) : N2_OK;
+	N2ScatterRider rider;
+	if (sums) rider.sums = *sums;
 	N2ProfScope prof(N2_PROF_GRID_BACKWARD_PARAMS, s);
 	return launch_scatter(grid, s, d_xyz, point_stride, dim_stride, n_points, reinterpret_cast<const __half*>(d_dL_dy), d_dL_ddLdx,
 	                      reinterpret_cast<const __half*>(d_dL_dy_second), grid->grads, reinterpret_cast<__half*>(d_dL_ddLdy),
-	                      mode == N2_GRAD_ACCUMULATE);
+	                      mode == N2_GRAD_ACCUMULATE, nullptr, 0, rider);
+}
+N2_API int n2_grid_backward_fused(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
+                                  uint32_t dim_stride, uint32_t n_points, const n2_half* d_dL_dy,
+                                  const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy,
+                                  n2_grad_mode mode) {
+	return n2_grid_backward_fused_and_sums(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_dL_dy, d_dL_ddLdx, d_dL_dy_second, d_dL_ddLdy, mode, nullptr);
 }
 
 int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz_rows, uint32_t n_cols, const uint32_t* d_index,

@@ -529,6 +529,8 @@ static int check_pending(n2_mlp_t* mlp, const char* fn, uint32_t n_slabs, n2_gra
 	return N2_OK;
 }
 
+const n2_half* n2_mlp_weights(const n2_mlp_t* mlp) { return reinterpret_cast<const n2_half*>(mlp->params); }
+bool n2_mlp_defers(const n2_mlp_t* mlp) { return mlp->deferred; }
 void n2_mlp_drop_pending(n2_mlp_t* mlp) {
 	if (mlp) mlp->pending_slabs = 0;
 }

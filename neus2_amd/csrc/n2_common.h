@@ -128,6 +128,17 @@ int n2_generate_training_samples_rows(n2_stream_t stream, uint32_t n_rays, uint3
 // else a level-major gather into the feature rows 3.. of sdf_in (SoA, n columns) followed by the network kernel.
 int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
                        float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n = 0xFFFFFFFFu);
+// The SDF network with 48 inputs on its own: output, d sdf / d input, normals, the eikonal loss's terms (n2_fused_sdf_eikonal_parts(n) partial sums) and what
+// its backward takes, but for the zero rows of dL_dy and v_in (fused.hip).  input's padding rows are not read.
+uint32_t n2_fused_sdf_eikonal_parts(uint32_t n);
+int n2_fused_sdf_eikonal(hipStream_t s, const n2_half* weights, uint32_t n, const n2_half* input, const float* dy_dx, n2_half* output, n2_half* dsdf, float* normal,
+                         float ek_weight, float scale, n2_half* dL_dy, float* v, n2_half* v_in, float* parts);
+// n2_grid_forward into rows 3.. of the SDF network's input (n_points columns), and the centred positions into rows 0..2
+int n2_grid_forward_sdf_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points, n2_half* d_input,
+                              float* d_dy_dx);
+// the network's weights (null: not set) and whether its slab sums are deferred by its owner
+const n2_half* n2_mlp_weights(const n2_mlp_t* mlp);
+bool n2_mlp_defers(const n2_mlp_t* mlp);
 // Row 0 of NerfNetwork::sdf as fp32 on a whole lattice, x fastest: point c at (c / res) * extent + corner (lattice.hip).  The
 // lattice is worked off in slabs, whose size follows from d_scratch: 44 bytes for each of `chunk` points.  d_frags holds
 // n2_lattice_frag_bytes().  The values do not depend on where the slabs are cut.
@@ -220,8 +231,12 @@ int n2_field_backward_deferred(n2_field_t* field, n2_stream_t stream, const floa
                                n2_grad_mode mode, N2SlabReduce* sums);
 // n2_field_select without the copy of the index: d_source_index must stay valid and unchanged until the backward has run
 int n2_field_select_borrow(n2_field_t* field, const uint32_t* d_source_index, uint32_t n_source, uint32_t n);
+// n2_grid_backward_fused with a slab summation (or null) that is run beside the scatter (d_dL_ddLdy null), by workgroups of its first launch
+int n2_grid_backward_fused_and_sums(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
+                                    const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy, n2_grad_mode mode,
+                                    const N2SlabReduce* sums);
 // n2_grid_backward_fused whose positions (SoA 3 x n_cols) and d_dL_dy_second rows (n_cols columns) are read through d_index.
-// sums (or null): a slab summation that is run beside the scatter, by workgroups of its first launch.
+// sums: as there
 int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz_rows, uint32_t n_cols, const uint32_t* d_index,
                                    uint32_t n_points, const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second,
                                    n2_grad_mode mode, const N2SlabReduce* sums = nullptr);

@@ -16,7 +16,7 @@ import torch
 
 from . import capi
 from .capi import check, ptr
-from .tcnn_api import GRAD_OVERWRITE, LAYOUT_SOA, FullyFusedMLP, GridEncoding, _stream
+from .tcnn_api import GRAD_OVERWRITE, FullyFusedMLP, GridEncoding, _stream
 
 
 class SdfNet:
@@ -36,56 +36,45 @@ class SdfNet:
         if n != self._n:
             h = lambda rows: torch.empty((rows, n), dtype=torch.float16, device=device)
             f = lambda rows: torch.empty((rows, n), dtype=torch.float32, device=device)
-            self._inp, self._g, self._y, self._dL_dy, self._v_in, self._d_inp = h(self.in_w), h(self.in_w), h(16), h(16), h(self.in_w), h(self.in_w)
-            self._dy_dx = torch.empty((self.enc_w, n, 3), dtype=torch.float32, device=device)
-            self._normal, self._v = f(3), f(3)
-            self._loss = torch.empty(1, dtype=torch.float32, device=device)
-            nb = int(capi.lib().n2_sdf_eikonal_workspace_bytes(C.c_uint32(n)))
-            self._ws = torch.empty(nb, dtype=torch.uint8, device=device)
-            self._ws_bytes = nb
+            z = lambda rows: torch.zeros((rows, n), dtype=torch.float16, device=device)  # rows that stay zero: the inputs' padding, the outputs without a loss
+            nb = int(capi.lib().n2_sdf_step_workspace_bytes(C.c_uint32(n)))
+            b = dict(input=z(self.in_w), dy_dx=torch.empty((self.enc_w, n, 3), dtype=torch.float32, device=device), output=h(16), dsdf_dinput=h(self.in_w), normal=f(3),
+                     dL_doutput=z(16), dL_dnormal=f(3), second_order_input=z(self.in_w), dL_dinput=h(self.in_w),
+                     loss=torch.empty(1, dtype=torch.float32, device=device), workspace=torch.empty(nb, dtype=torch.uint8, device=device))
+            self._b = (capi.SdfBuffers(workspace_bytes=nb, **{k: t.data_ptr() for k, t in b.items()}), b)
             self._n = n
+        return self._b
 
     def forward(self, x, ek_weight=0.1, loss_scale=128.0):
         """x fp32 [3, N].  Returns a context dict with sdf (fp16 [N]), normal (fp32 [3, N]), the loss (one-element device
         tensor) and what backward needs.  The tensors are the net's own buffers: they are overwritten by the next
         forward of the same batch size."""
-        L, s = capi.lib(), _stream()
         n = x.shape[1]
-        self._buffers(n, x.device)
-        inp, g, y = self._inp, self._g, self._y
-        check(L.n2_sdf_pack_input(s, ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), ptr(inp)),
-              "n2_sdf_pack_input")
-        enc = inp[3:3 + self.enc_w]
-        check(L.n2_grid_forward(self.grid._h, s, ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), ptr(enc), ptr(self._dy_dx)), "n2_grid_forward")
-        check(L.n2_mlp_forward_and_input_gradient(self.mlp._h, s, C.c_uint32(0), ptr(inp), C.c_uint32(n), ptr(y), C.c_int(LAYOUT_SOA), ptr(g)),
-              "n2_mlp_forward_and_input_gradient")
-        ctx = dict(x=x, inp=inp, dy_dx=self._dy_dx, y=y, g=g, sdf=y[0], normal=self._normal, loss=self._loss)
-        self._eikonal(ctx, ek_weight, loss_scale)
-        return ctx
+        own, b = buffers = self._buffers(n, x.device)
+        check(capi.lib().n2_sdf_forward_and_loss(self.grid._h, self.mlp._h, _stream(), ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), C.c_float(ek_weight),
+                                                 C.c_float(loss_scale), C.byref(own)), "n2_sdf_forward_and_loss")
+        return dict(x=x, inp=b["input"], dy_dx=b["dy_dx"], y=b["output"], g=b["dsdf_dinput"], sdf=b["output"][0], normal=b["normal"], loss=b["loss"],
+                    weights=(ek_weight, loss_scale), buffers=buffers)
 
     def _eikonal(self, ctx, ek_weight, loss_scale):
-        n = ctx["x"].shape[1]
+        """The loss and what backward takes with other weights."""
+        n, b = ctx["x"].shape[1], ctx["buffers"][1]
         # normals: encoding backward of d sdf / d encoding without parameter gradients, J^T g (nerf_network.h:230-234)
-        check(capi.lib().n2_sdf_normals_and_eikonal_loss(_stream(), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), ptr(ctx["y"]),
-                                                         ptr(ctx["g"]), ptr(ctx["dy_dx"]), ptr(self._normal), C.c_float(ek_weight),
-                                                         C.c_float(loss_scale), ptr(self._dL_dy), ptr(self._v), ptr(self._v_in), ptr(self._loss),
-                                                         ptr(self._ws), C.c_uint64(self._ws_bytes)),
+        check(capi.lib().n2_sdf_normals_and_eikonal_loss(_stream(), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), ptr(b["output"]),
+                                                         ptr(b["dsdf_dinput"]), ptr(b["dy_dx"]), ptr(b["normal"]), C.c_float(ek_weight),
+                                                         C.c_float(loss_scale), ptr(b["dL_doutput"]), ptr(b["dL_dnormal"]), ptr(b["second_order_input"]),
+                                                         ptr(b["loss"]), ptr(b["workspace"]), C.c_uint64(b["workspace"].numel())),
               "n2_sdf_normals_and_eikonal_loss")
         ctx["weights"] = (ek_weight, loss_scale)
 
     def loss_backward(self, ctx, ek_weight=0.1, loss_scale=128.0):
         """Returns the loss as a one-element device tensor (no host synchronisation)."""
-        L, s = capi.lib(), _stream()
-        x, inp, g, n = ctx["x"], ctx["inp"], ctx["g"], ctx["x"].shape[1]
+        x, n = ctx["x"], ctx["x"].shape[1]
         if ctx["weights"] != (ek_weight, loss_scale):
             self._eikonal(ctx, ek_weight, loss_scale)
         # both orders through the MLP in one pass (the second's first-order output gradient was e_0), then both through the grid;
         # the grid's dL_ddLdoutput (rows 3.. of the MLP's second-order input) was already formed from the saved Jacobian with
         # the loss
-        check(L.n2_mlp_backward_and_second_order(self.mlp._h, s, ptr(inp), C.c_uint32(n), ptr(self._dL_dy), C.c_int(LAYOUT_SOA), ptr(self._d_inp),
-                                                 ptr(self._v_in), None, C.c_int(GRAD_OVERWRITE)),
-              "n2_mlp_backward_and_second_order")
-        check(L.n2_grid_backward_fused(self.grid._h, s, ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), ptr(self._d_inp[3:3 + self.enc_w]),
-                                       ptr(self._v), ptr(g[3:3 + self.enc_w]), None, C.c_int(GRAD_OVERWRITE)),
-              "n2_grid_backward_fused")
-        return self._loss
+        check(capi.lib().n2_sdf_loss_backward(self.grid._h, self.mlp._h, _stream(), ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), C.byref(ctx["buffers"][0]),
+                                              C.c_int(GRAD_OVERWRITE)), "n2_sdf_loss_backward")
+        return ctx["loss"]

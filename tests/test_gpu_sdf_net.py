@@ -81,3 +81,57 @@ def test_normals_and_loss_in_one_pass_equal_the_two_calls(n_levels, n):
         outs.append((normal, v, dL_dy, v_in, loss))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+# less than a wave's tile, its edges, several tiles per wave, a streamed Jacobian; networks whose lanes do not hold their levels
+@pytest.mark.parametrize("n_levels,n", [(16, 8), (16, 24), (16, 32), (16, 40), (16, 5000), (16, 65536 + 8), (16, 180000), (3, 256), (15, 1000), (20, 776)])
+def test_step_equals_the_single_calls(n_levels, n):
+    """n2_sdf_forward_and_loss and n2_sdf_loss_backward against the entry points they stand for.  The one-pass kernel adds the network's products and the
+    normals' terms in another order (one fp16 rounding of the first output moves by a digit now and then)."""
+    import ctypes as C
+    from neus2_amd import capi
+    from neus2_amd.capi import check, ptr
+    from neus2_amd.sdf_net import SdfNet
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, LAYOUT_SOA, _stream
+    L, u = capi.lib(), C.c_uint32
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    net = SdfNet(n_levels, 14, 16, 1.3, max_batch=n)
+    P = (torch.randn(net.grid.n_params(), device="cuda", generator=gen) * 0.01).half()
+    W = (torch.randn(net.mlp.n_params(), device="cuda", generator=gen) * 0.15).half()
+    gP, gW = torch.zeros_like(P), torch.zeros_like(W)
+    net.set_params(P, gP, W, gW)
+    x = torch.rand((3, n), device="cuda", generator=gen)
+    for _ in range(2):  # (and on buffers that a step has used)
+        ctx = net.forward(x, 0.2, 64.0)
+        loss = net.loss_backward(ctx, 0.2, 64.0)
+    got = dict(y=ctx["y"], g=ctx["g"], normal=ctx["normal"], loss=loss, grid=gP, mlp=gW, inp=ctx["inp"])
+    got = {k: t.clone() for k, t in got.items()}
+    rows, in_w = net.enc_w, net.in_w
+    h = lambda r: torch.full((r, n), 7.0, dtype=torch.float16, device="cuda")
+    f = lambda r: torch.full((r, n), 7.0, device="cuda")
+    inp, y, g, dL_dy, v_in, d_inp, normal, v, loss = h(in_w), h(16), h(in_w), h(16), h(in_w), h(in_w), f(3), f(3), torch.zeros(1, device="cuda")
+    dy_dx = torch.empty((rows, n, 3), device="cuda")
+    ws = torch.empty(int(L.n2_sdf_eikonal_workspace_bytes(u(n))), dtype=torch.uint8, device="cuda")
+    check(L.n2_sdf_pack_input(_stream(), ptr(x), u(1), u(n), u(n), u(rows), u(in_w), ptr(inp)))
+    check(L.n2_grid_forward(net.grid._h, _stream(), ptr(x), u(1), u(n), u(n), ptr(inp[3:]), ptr(dy_dx)))
+    check(L.n2_mlp_forward_and_input_gradient(net.mlp._h, _stream(), u(0), ptr(inp), u(n), ptr(y), C.c_int(LAYOUT_SOA), ptr(g)))
+    check(L.n2_sdf_normals_and_eikonal_loss(_stream(), u(n), u(rows), u(in_w), ptr(y), ptr(g), ptr(dy_dx), ptr(normal), C.c_float(0.2), C.c_float(64.0), ptr(dL_dy), ptr(v),
+                                            ptr(v_in), ptr(loss), ptr(ws), C.c_uint64(ws.numel())))
+    check(L.n2_mlp_backward_and_second_order(net.mlp._h, _stream(), ptr(inp), u(n), ptr(dL_dy), C.c_int(LAYOUT_SOA), ptr(d_inp), ptr(v_in), None, C.c_int(GRAD_OVERWRITE)))
+    check(L.n2_grid_backward_fused(net.grid._h, _stream(), ptr(x), u(1), u(n), u(n), ptr(d_inp[3:]), ptr(v), ptr(g[3:]), None, C.c_int(GRAD_OVERWRITE)))
+    want = dict(y=y, g=g, normal=normal, loss=loss, grid=gP, mlp=gW, inp=inp)
+    for k, t in want.items():
+        if n_levels != 16 or k == "inp":
+            assert torch.equal(got[k], t), k
+        else:
+            assert bool((t != 0).any()) and rel_l2(host(got[k]), host(t)) < 1e-3, (k, rel_l2(host(got[k]), host(t)))
+
+
+def test_step_errors():
+    from neus2_amd.sdf_net import SdfNet
+    from neus2_amd.tcnn_api import N2Error
+    net = SdfNet(3, 10, 4, 1.5, max_batch=64)
+    with pytest.raises(N2Error, match="multiple of 8"):
+        net.forward(torch.rand((3, 12), device="cuda"))
+    with pytest.raises(N2Error, match="set_params"):
+        net.forward(torch.rand((3, 16), device="cuda"))
