@@ -98,7 +98,7 @@ __device__ __forceinline__ uint32_t occ_morton3d_invert(uint32_t x) {
 // evaluated in is free: when n is a power of two, slot t holds sample i(t) = t P^-1 mod n (P^-1 mod 2^32, masked), whose
 // candidate cell is t + const mod n: consecutive slots splat into consecutive cells of (at most 128^3 / n) runs, and a
 // wave's 64 atomics fall into a few lines.  Other n: slot t holds sample t.
-constexpr uint32_t OCC_WALK = 56924617u;
+constexpr uint32_t OCC_WALK = 56924617u, OCC_FIRST = 96925573u;
 constexpr uint32_t occ_inverse_mod_2_32(uint32_t a) {  // a odd; Newton's iteration doubles the number of correct low bits
 	uint32_t x = a;                                     // a * a = 1 mod 8
 	for (int k = 0; k < 5; ++k) x *= 2u - a * x;
@@ -107,6 +107,40 @@ constexpr uint32_t occ_inverse_mod_2_32(uint32_t a) {  // a odd; Newton's iterat
 constexpr uint32_t OCC_WALK_INV = occ_inverse_mod_2_32(OCC_WALK);
 static_assert(OCC_WALK * OCC_WALK_INV == 1u, "inverse of the walk's multiplier");
 static inline uint32_t occ_order_mul(uint32_t n) { return (n >= 2 && (n & (n - 1)) == 0) ? OCC_WALK_INV : 0u; }
+
+// The rows of positions that the encoding's gather reads, and with them the densities, stand in another order yet where n is a power of two: a wave's 64
+// cells are a brick of 16 x 2 x 2 along x instead of 4 x 4 x 4, because a line of the encoding's tables is 32 vertices along x, and a load is served
+// in fewer clocks when neighbouring lanes ask for the same line.  The bricks lie on the cells' grid: a row's place gives its cell (of n, modulo n), the cell
+// its slot.  Gather and whole update of 128^3 cells in us: slots' order 381 | 468, the same laid on the cells' grid - | 458, bricks 353 | 430.
+// Where there are fewer samples than cells, 2 x 2 x 2 cells stay together in a brick: 2^20 samples 270 | 258, 2^19 161 | 157 (whole bricks along
+// x 262 and 163), 2^19 and 2^19 others 286 | 282.  Samples that look for an occupied cell end up anywhere: their rows are in the slots' order (2^19 of either
+// kind 289 with the others' in bricks, too).
+struct OccOrder {
+	uint32_t mul;    // slot -> sample (0: the same)
+	uint32_t shift;  // a slot's first candidate cell is slot + shift mod n
+	uint32_t mask;   // n - 1 where the rows have an order of their own, else 0
+};
+// Bit of the cell's number (x, y, z interleaved) that each bit of the row's place is, for samples of all cells and of fewer
+constexpr uint32_t OCC_BRICK_BITS = 15;
+constexpr uint8_t OCC_BRICK_ALL[OCC_BRICK_BITS] = {0, 3, 6, 9, 1, 2, 12, 4, 5, 7, 8, 10, 11, 13, 14};
+constexpr uint8_t OCC_BRICK_SOME[OCC_BRICK_BITS] = {0, 3, 1, 2, 6, 9, 4, 5, 7, 8, 10, 11, 12, 13, 14};
+__device__ __forceinline__ uint32_t occ_row_place(const OccOrder& o, uint32_t slot) {
+	if (o.mask == 0u) return slot;
+	const uint32_t cell = (slot + o.shift) & o.mask;
+	const bool all = o.mask >= OCC_CELLS - 1u;
+	uint32_t at = cell & ~((1u << OCC_BRICK_BITS) - 1u);
+#pragma unroll
+	for (uint32_t b = 0; b < OCC_BRICK_BITS; ++b) at |= ((cell >> (all ? OCC_BRICK_ALL[b] : OCC_BRICK_SOME[b])) & 1u) << b;
+	return at;
+}
+__device__ __forceinline__ uint32_t occ_row_slot(const OccOrder& o, uint32_t at) {
+	if (o.mask == 0u) return at;
+	const bool all = o.mask >= OCC_CELLS - 1u;
+	uint32_t cell = at & ~((1u << OCC_BRICK_BITS) - 1u);
+#pragma unroll
+	for (uint32_t b = 0; b < OCC_BRICK_BITS; ++b) cell |= ((at >> b) & 1u) << (all ? OCC_BRICK_ALL[b] : OCC_BRICK_SOME[b]);
+	return (cell - o.shift) & o.mask;
+}
 
 // The generator skips 4 i draws ahead for sample i: state -> mult^(4 i) state + inc (1 + mult + .. + mult^(4 i - 1)).  The skip is
 // composed from the hexadecimal digits of i, whose two factors are a table of constants: a multiply-add per digit instead of
@@ -141,7 +175,7 @@ constexpr OccSkips occ_build_skips() {
 static __device__ const OccSkips OCC_SKIPS = occ_build_skips();
 
 __global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uint32_t n_pad, Pcg32 rng, uint32_t n_digits, uint32_t step, const float* __restrict__ grid,
-                                                                 uint32_t n_cascades, float thresh, uint32_t order_mul,
+                                                                 uint32_t n_cascades, float thresh, OccOrder order,
                                                                  float* __restrict__ positions, uint32_t* __restrict__ indices, float* __restrict__ rows, uint32_t n_rows,
                                                                  float* __restrict__ tmp, uint32_t n_tmp) {
 	__shared__ ulonglong2 skip[OCC_DIGITS][16];
@@ -154,7 +188,7 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uin
 	if (slot >= n_pad) return;
 	float pos[3] = {0.5f, 0.5f, 0.5f};
 	if (slot < n) {
-		const uint32_t i = order_mul ? (slot * order_mul) & (n - 1u) : slot;
+		const uint32_t i = order.mul ? (slot * order.mul) & (n - 1u) : slot;
 		for (uint32_t p = 0; p < n_digits; ++p) {
 			const ulonglong2 f = skip[p][(i >> (4u * p)) & 15u];
 			rng.state = f.x * rng.state + f.y;
@@ -162,7 +196,7 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uin
 		const uint32_t level = (uint32_t)(rng.next_float() * n_cascades) % n_cascades;
 		uint32_t idx = 0;
 		for (uint32_t j = 0; j < 10; ++j) {
-			idx = ((i + step * n) * OCC_WALK + j * 19349663u + 96925573u) % OCC_CELLS;
+			idx = ((i + step * n) * OCC_WALK + j * 19349663u + OCC_FIRST) % OCC_CELLS;
 			idx += level * OCC_CELLS;
 			if (grid[idx] > thresh) break;
 		}
@@ -176,19 +210,21 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uin
 		}
 		indices[slot] = idx;
 	}
+	const uint32_t at = rows && slot < n ? occ_row_place(order, slot) : slot;
 #pragma unroll
 	for (int d = 0; d < 3; ++d) {
 		positions[(size_t)slot * 3 + d] = pos[d];
-		if (rows) rows[(size_t)d * n_rows + slot] = pos[d];
+		if (rows) rows[(size_t)d * n_rows + at] = pos[d];
 	}
 }
 
-// splat_grid_samples_nerf_max_nearest_neighbor (:662-680): positive floats order like their bit patterns
+// splat_grid_samples_nerf_max_nearest_neighbor (:662-680): positive floats order like their bit patterns.  Density i is that of row i.
 __global__ void __launch_bounds__(OCC_BLOCK) occ_splat_kernel(uint32_t n, const uint32_t* __restrict__ indices, const float* __restrict__ density,
-                                                              float* __restrict__ tmp) {
+                                                              float* __restrict__ tmp, uint32_t n_uniform, OccOrder uniform, OccOrder others) {
 	const uint32_t i = blockIdx.x * OCC_BLOCK + threadIdx.x;
 	if (i >= n) return;
-	atomicMax(reinterpret_cast<uint32_t*>(tmp) + indices[i], __float_as_uint(density[i]));
+	const uint32_t slot = i < n_uniform ? occ_row_slot(uniform, i) : n_uniform + occ_row_slot(others, i - n_uniform);
+	atomicMax(reinterpret_cast<uint32_t*>(tmp) + indices[slot], __float_as_uint(density[i]));
 }
 
 // ema_grid_samples_nerf (:698-727), fused with the partial sums of max(v, 0) over the first cascade (:3383).
@@ -445,10 +481,15 @@ N2_API int n2_occupancy_update(n2_occupancy_t* occ, n2_field_t* field, n2_stream
 	// path writes only after it has read them)
 	const uint32_t n8 = (n + 7) / 8 * 8;
 	float* rows = n8 <= occ->chunk ? reinterpret_cast<float*>(occ->mlp_out) : nullptr;
-	auto generate = [&](uint32_t count, uint32_t pad, uint32_t first, float thresh, bool clear) -> int {
+	auto order_of = [&](uint32_t count) {
+		return OccOrder{occ_order_mul(count), occ->ema_step * count * OCC_WALK + OCC_FIRST, 0u};
+	};
+	OccOrder uniform = order_of(n_uniform), others = order_of(n_nonuniform);
+	if (rows != nullptr && uniform.mul != 0u && n_uniform >= (1u << OCC_BRICK_BITS)) uniform.mask = n_uniform - 1u;
+	auto generate = [&](uint32_t count, uint32_t pad, uint32_t first, float thresh, bool clear, const OccOrder& order) -> int {
 		uint32_t digits = 1;
 		while (digits < OCC_DIGITS && (count >> (4u * digits)) != 0) ++digits;
-		occ_generate_kernel<<<ogrid(pad), dim3(OCC_BLOCK), 0, s>>>(count, pad, rng, digits, occ->ema_step, occ->grid, occ->n_cascades, thresh, occ_order_mul(count),
+		occ_generate_kernel<<<ogrid(pad), dim3(OCC_BLOCK), 0, s>>>(count, pad, rng, digits, occ->ema_step, occ->grid, occ->n_cascades, thresh, order,
 		                                                          occ->positions + (size_t)first * 3, occ->indices + first, rows ? rows + first : nullptr, n8,
 		                                                          occ->tmp, clear ? n_elements : 0u);
 		N2_LAUNCH_CHECK();
@@ -459,11 +500,11 @@ N2_API int n2_occupancy_update(n2_occupancy_t* occ, n2_field_t* field, n2_stream
 	}
 	if (n_uniform) {
 		// slots of the second group are written by the second launch; only the last launch pads
-		if (int rc = generate(n_uniform, n_nonuniform ? n_uniform : n8, 0, -0.01f, true)) return rc;
+		if (int rc = generate(n_uniform, n_nonuniform ? n_uniform : n8, 0, -0.01f, true, uniform)) return rc;
 	}
 	rng.advance(1ull << 32);
 	if (n_nonuniform) {
-		if (int rc = generate(n_nonuniform, n8 - n_uniform, n_uniform, OCC_MIN_OPTICAL_THICKNESS, n_uniform == 0)) return rc;
+		if (int rc = generate(n_nonuniform, n8 - n_uniform, n_uniform, OCC_MIN_OPTICAL_THICKNESS, n_uniform == 0, others)) return rc;
 	}
 	rng.advance(1ull << 32);
 	occ->rng_state = rng.state;
@@ -474,7 +515,7 @@ N2_API int n2_occupancy_update(n2_occupancy_t* occ, n2_field_t* field, n2_stream
 		float* row0 = reinterpret_cast<float*>(occ->mlp_out + (size_t)16 * occ->chunk);
 		if (int rc = n2_field_sdf_row0(field, stream, rows ? rows : occ->positions + (size_t)a * 3, rows ? 1u : 3u, rows ? n8 : 1u, m8, m8, row0,
 		                               reinterpret_cast<n2_half*>(occ->mlp_out), true)) return rc;
-		occ_splat_kernel<<<ogrid(m), dim3(OCC_BLOCK), 0, s>>>(m, occ->indices + a, row0, occ->tmp);
+		occ_splat_kernel<<<ogrid(m), dim3(OCC_BLOCK), 0, s>>>(m, occ->indices + a, row0, occ->tmp, n_uniform, uniform, others);
 		N2_LAUNCH_CHECK();
 	}
 	occ_ema_kernel<true><<<dim3((n_elements + OCC_BLOCK * 32 - 1) / (OCC_BLOCK * 32)), dim3(OCC_BLOCK), 0, s>>>(n_elements, decay, occ->grid, occ->tmp,

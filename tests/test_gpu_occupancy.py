@@ -196,3 +196,21 @@ def test_a_step_after_an_update_with_larger_chunks_matches_the_oracle(oracle):
     res = verify_step(Field(fp16=True), params16, oc_cams(oracle, cams), rgba, bits, n_rays, n_rays, 2, n_inf, T, c, gpu, host(tr.grads),
                       background=(1.0, 1.0, 1.0))
     assert res["compacted"] > T // 2, res
+
+
+# the smallest group whose rows have an order of their own, one below it, all cells, more samples than cells, and other samples behind
+@pytest.mark.parametrize("n_uniform,n_nonuniform,cascades", [(1 << 14, 0, 1), (1 << 15, 0, 1), (1 << 15, 1 << 15, 1), (1 << 17, 1003, 1), (1 << 21, 0, 1), (1 << 22, 0, 2)])
+def test_order_of_the_rows_leaves_no_trace(n_uniform, n_nonuniform, cascades):
+    """Samples evaluated in bricks of cells (one chunk) and in the order of their slots (several chunks) give the same grid: every sample's density is its own."""
+    from neus2_amd.training import OccupancyGrid, Trainer, default_config
+    trainer = Trainer(default_config(target_batch_size=1 << 12, max_rays_per_batch=1 << 8, max_samples=1 << 22))
+    trainer.initialize_params(seed=3)
+    out = []
+    for chunk in (n_uniform + n_nonuniform, 1 << 13):
+        occ = OccupancyGrid(cascades, seed=5, max_chunk=(chunk + 7) // 8 * 8)
+        for _ in range(2):  # the step moves the cells' numbers
+            occ.update(trainer._field, n_uniform, n_nonuniform)
+        pos, idx = occ.last_samples()
+        out.append([t.clone() for t in (occ.density_grid, occ.bitfield, occ.mean, pos, idx)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b) and bool((a != 0).any())
