@@ -76,6 +76,17 @@ class SdfBuffers(C.Structure):
                                                 "loss", "workspace")] + [("workspace_bytes", C.c_uint64)]
 
 
+# Arguments of the calls that a program makes for every batch: p pointer or handle, u uint32, f float, i int or enum, q uint64.  Python's numbers and
+# addresses then go in as they are; without a signature ctypes wants an object around each (a third of what such a call takes on the host).
+_SIGNATURES = {
+    "n2_grid_forward": "pppuuupp", "n2_grid_backward": "pppuuupppi", "n2_grid_backward_backward_input": "pppuuuppppi", "n2_grid_backward_fused": "pppuuuppppi",
+    "n2_field_forward": "pppup", "n2_field_backward": "pppupui", "n2_field_sdf": "pppuuup", "n2_field_density": "pppuuup",
+    "n2_sdf_forward_and_loss": "ppppuuuffp", "n2_sdf_loss_backward": "ppppuuupi",
+    "n2_trainer_set_training_step": "pu", "n2_trainer_step": "ppuuu", "n2_occupancy_update": "pppfuu",
+    "n2_marching_cubes_count": "ppppfppqpp", "n2_marching_cubes_emit": "ppppfpppppuu",
+}
+
+
 class N2Error(RuntimeError):
     """A C-ABI call returned a non-zero status (mirrors the reference's std::runtime_error)."""
 
@@ -95,6 +106,9 @@ def lib():
         except ImportError:
             pass
         _lib = C.CDLL(LIB_PATH)
+        kinds = dict(p=C.c_void_p, u=C.c_uint32, f=C.c_float, i=C.c_int, q=C.c_uint64)
+        for name, signature in _SIGNATURES.items():
+            getattr(_lib, name).argtypes = [kinds[k] for k in signature]
         _lib.n2_last_error.restype = C.c_char_p
         _lib.n2_version.restype = C.c_char_p
         _lib.n2_field_encoding.restype = C.c_void_p

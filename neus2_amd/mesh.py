@@ -8,7 +8,7 @@ import torch
 
 from . import capi
 from .capi import N2Error, check, ptr
-from .tcnn_api import _stream
+from .tcnn_api import _stream, _stream_address
 
 
 def _u3(v):
@@ -59,17 +59,21 @@ def marching_cubes(density, thresh, aabb_min=(0, 0, 0), aabb_max=(1, 1, 1), want
     nbytes = int(L.n2_marching_cubes_workspace_bytes(_u3(res)))
     if nbytes == 0:
         raise N2Error("n2_marching_cubes_workspace_bytes: " + L.n2_last_error().decode())
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=density.device)
+    device = density.device
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
     totals = torch.empty(2, dtype=torch.int32, pin_memory=True)  # pinned: a kernel leaves the totals there by itself, without a copy
-    nv, nt = (C.c_uint32.from_address(totals.data_ptr() + 4 * k) for k in range(2))
-    check(L.n2_marching_cubes_count(_stream(), _u3(res), _f3(aabb_min), _f3(aabb_max), C.c_float(thresh), ptr(density), ptr(ws),
-                                    C.c_uint64(nbytes), C.byref(nv), C.byref(nt)), "n2_marching_cubes_count")
-    verts = torch.empty((nv.value, 3), dtype=torch.float32, device=density.device)
-    idx = torch.empty((nt.value, 3), dtype=torch.int32, device=density.device)
-    normals = torch.empty((nv.value, 3), dtype=torch.float32, device=density.device) if want_normals else None
-    check(L.n2_marching_cubes_emit(_stream(), _u3(res), _f3(aabb_min), _f3(aabb_max), C.c_float(thresh), ptr(density), ptr(ws),
-                                   ptr(verts) if nv.value else None, ptr(idx) if nt.value else None,
-                                   ptr(normals) if (want_normals and nv.value) else None, nv, nt), "n2_marching_cubes_emit")
+    at = totals.data_ptr()
+    nv, nt = (C.c_uint32.from_address(at + 4 * k) for k in range(2))
+    # (what the second call takes is ready before the first one waits for the totals)
+    head = (_stream_address(), _u3(res), _f3(aabb_min), _f3(aabb_max), thresh, density.data_ptr(), ws.data_ptr())
+    emit = L.n2_marching_cubes_emit
+    check(L.n2_marching_cubes_count(*head, nbytes, at, at + 4), "n2_marching_cubes_count")
+    n_verts, n_tris = nv.value, nt.value
+    verts = torch.empty(n_verts, 3, dtype=torch.float32, device=device)
+    idx = torch.empty(n_tris, 3, dtype=torch.int32, device=device)
+    normals = torch.empty(n_verts, 3, dtype=torch.float32, device=device) if want_normals else None
+    check(emit(*head, verts.data_ptr() if n_verts else None, idx.data_ptr() if n_tris else None, normals.data_ptr() if (want_normals and n_verts) else None,
+               n_verts, n_tris), "n2_marching_cubes_emit")
     return verts, idx, normals
 
 

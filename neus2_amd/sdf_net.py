@@ -16,7 +16,7 @@ import torch
 
 from . import capi
 from .capi import check, ptr
-from .tcnn_api import GRAD_OVERWRITE, FullyFusedMLP, GridEncoding, _stream
+from .tcnn_api import GRAD_OVERWRITE, FullyFusedMLP, GridEncoding, _stream, _stream_address
 
 
 class SdfNet:
@@ -51,8 +51,7 @@ class SdfNet:
         forward of the same batch size."""
         n = x.shape[1]
         own, b = buffers = self._buffers(n, x.device)
-        check(capi.lib().n2_sdf_forward_and_loss(self.grid._h, self.mlp._h, _stream(), ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), C.c_float(ek_weight),
-                                                 C.c_float(loss_scale), C.byref(own)), "n2_sdf_forward_and_loss")
+        check(capi.lib().n2_sdf_forward_and_loss(self.grid._h, self.mlp._h, _stream_address(), x.data_ptr(), 1, n, n, ek_weight, loss_scale, C.byref(own)), "n2_sdf_forward_and_loss")
         return dict(x=x, inp=b["input"], dy_dx=b["dy_dx"], y=b["output"], g=b["dsdf_dinput"], sdf=b["output"][0], normal=b["normal"], loss=b["loss"],
                     weights=(ek_weight, loss_scale), buffers=buffers)
 
@@ -75,6 +74,6 @@ class SdfNet:
         # both orders through the MLP in one pass (the second's first-order output gradient was e_0), then both through the grid;
         # the grid's dL_ddLdoutput (rows 3.. of the MLP's second-order input) was already formed from the saved Jacobian with
         # the loss
-        check(capi.lib().n2_sdf_loss_backward(self.grid._h, self.mlp._h, _stream(), ptr(x), C.c_uint32(1), C.c_uint32(n), C.c_uint32(n), C.byref(ctx["buffers"][0]),
-                                              C.c_int(GRAD_OVERWRITE)), "n2_sdf_loss_backward")
+        check(capi.lib().n2_sdf_loss_backward(self.grid._h, self.mlp._h, _stream_address(), x.data_ptr(), 1, n, n, C.byref(ctx["buffers"][0]),
+                                              GRAD_OVERWRITE), "n2_sdf_loss_backward")
         return ctx["loss"]

@@ -19,11 +19,20 @@ from .capi import (GRAD_ACCUMULATE, GRAD_IGNORE, GRAD_OVERWRITE, LAYOUT_AOS, LAY
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream():
-    """torch's current stream as a hipStream_t.  (torch.cuda.current_stream() builds a Stream object: 3 us of a small query's 12.)"""
+def _stream_address():
+    """Address of torch's current stream.  (torch.cuda.current_stream() builds a Stream object: 3 us of a small query's 12.)"""
     if _raw_stream is None:
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return C.c_void_p(_raw_stream(torch.cuda.current_device()))
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
+
+
+def _stream():
+    """torch's current stream as a hipStream_t."""
+    return C.c_void_p(_stream_address())
+
+
+def _address(t):
+    return None if t is None else t.data_ptr()
 
 
 def _positions(xyz):
@@ -33,11 +42,19 @@ def _positions(xyz):
         raise N2Error("positions must be a float32 CUDA tensor")
     if not xyz.is_contiguous():
         raise N2Error("positions must be contiguous")
-    if xyz.dim() == 2 and xyz.shape[0] == 3:
-        return xyz, 1, max(xyz.shape[1], 1), xyz.shape[1]
-    if xyz.dim() == 2 and xyz.shape[1] >= 3:
-        return xyz, xyz.shape[1], 1, xyz.shape[0]
-    raise N2Error(f"positions must be 3 x N or N x C, got {tuple(xyz.shape)}")
+    shape = xyz.shape
+    if len(shape) == 2:
+        rows, columns = shape
+        if rows == 3:
+            return xyz, 1, max(columns, 1), columns
+        if columns >= 3:
+            return xyz, columns, 1, rows
+    raise N2Error(f"positions must be 3 x N or N x C, got {tuple(shape)}")
+
+
+def _check_rows(t, dtype, rows, n, message):
+    if t.dtype != dtype or t.shape != (rows, n) or not t.is_contiguous():
+        raise N2Error(message)
 
 
 class GridEncoding:
@@ -50,6 +67,7 @@ class GridEncoding:
                                         C.c_uint32(log2_hashmap_size), C.c_uint32(base_resolution),
                                         C.c_float(per_level_scale), C.byref(self._h)), "n2_grid_create")
         self.n_levels = n_levels
+        self._width = self.output_width()
         self._params = self._grads = None
         self._owner = None
 
@@ -61,6 +79,7 @@ class GridEncoding:
         g._owner = owner
         g._params = g._grads = None
         g.n_levels = int(capi.lib().n2_grid_n_levels(g._h))
+        g._width = g.output_width()
         return g
 
     def __del__(self):
@@ -140,52 +159,45 @@ class GridEncoding:
         """Returns (out fp16 [width, N], ctx) where ctx holds dy_dx when requested; ``out`` may be a [width, N]
         row block of a wider matrix (the encoding rows of the network input, nerf_network.h:184-190)."""
         x, ps, ds, n = _positions(xyz)
+        w = self._width
         if out is None:
-            out = torch.empty((self.output_width(), n), dtype=torch.float16, device=x.device)
+            out = torch.empty(w, n, dtype=torch.float16, device=x.device)
         else:
-            _check_half(out, (self.output_width(), n), "grid output")
-        dy_dx = torch.empty((self.output_width(), n, 3), dtype=torch.float32, device=x.device) \
-            if prepare_input_gradients else None
-        check(capi.lib().n2_grid_forward(self._h, _stream(), ptr(x), C.c_uint32(ps), C.c_uint32(ds), C.c_uint32(n),
-                                         ptr(out), ptr(dy_dx)), "n2_grid_forward")
+            _check_half(out, (w, n), "grid output")
+        dy_dx = torch.empty(w, n, 3, dtype=torch.float32, device=x.device) if prepare_input_gradients else None
+        check(capi.lib().n2_grid_forward(self._h, _stream_address(), x.data_ptr(), ps, ds, n, out.data_ptr(), _address(dy_dx)), "n2_grid_forward")
         return out, dy_dx
 
     def backward(self, ctx, xyz, dL_dy, want_input_grad=False, mode=GRAD_OVERWRITE):
         x, ps, ds, n = _positions(xyz)
-        if dL_dy.dtype != torch.float16 or tuple(dL_dy.shape) != (self.output_width(), n) or not dL_dy.is_contiguous():
-            raise N2Error("dL_dy must be a contiguous fp16 [output_width, N] tensor")
-        dx = torch.empty((3, n), dtype=torch.float32, device=x.device) if want_input_grad else None
-        check(capi.lib().n2_grid_backward(self._h, _stream(), ptr(x), C.c_uint32(ps), C.c_uint32(ds), C.c_uint32(n),
-                                          ptr(dL_dy), ptr(ctx), ptr(dx), C.c_int(mode)), "n2_grid_backward")
+        _check_rows(dL_dy, torch.float16, self._width, n, "dL_dy must be a contiguous fp16 [output_width, N] tensor")
+        dx = torch.empty(3, n, dtype=torch.float32, device=x.device) if want_input_grad else None
+        check(capi.lib().n2_grid_backward(self._h, _stream_address(), x.data_ptr(), ps, ds, n, dL_dy.data_ptr(), _address(ctx), _address(dx), mode),
+              "n2_grid_backward")
         return dx
 
     def backward_backward_input(self, xyz, dL_ddLdx, dL_dy, want_dL_ddLdy=True, want_dL_dx=False,
                                 mode=GRAD_ACCUMULATE):
         x, ps, ds, n = _positions(xyz)
-        if dL_ddLdx.dtype != torch.float32 or tuple(dL_ddLdx.shape) != (3, n) or not dL_ddLdx.is_contiguous():
-            raise N2Error("dL_ddLdx must be a contiguous fp32 [3, N] tensor")
-        if dL_dy.dtype != torch.float16 or tuple(dL_dy.shape) != (self.output_width(), n) or not dL_dy.is_contiguous():
-            raise N2Error("dL_dy must be a contiguous fp16 [output_width, N] tensor")
-        o = torch.empty((self.output_width(), n), dtype=torch.float16, device=x.device) if want_dL_ddLdy else None
-        dx = torch.empty((3, n), dtype=torch.float32, device=x.device) if want_dL_dx else None
-        check(capi.lib().n2_grid_backward_backward_input(self._h, _stream(), ptr(x), C.c_uint32(ps), C.c_uint32(ds),
-                                                         C.c_uint32(n), ptr(dL_ddLdx), ptr(dL_dy), ptr(o), ptr(dx),
-                                                         C.c_int(mode)), "n2_grid_backward_backward_input")
+        w = self._width
+        _check_rows(dL_ddLdx, torch.float32, 3, n, "dL_ddLdx must be a contiguous fp32 [3, N] tensor")
+        _check_rows(dL_dy, torch.float16, w, n, "dL_dy must be a contiguous fp16 [output_width, N] tensor")
+        o = torch.empty(w, n, dtype=torch.float16, device=x.device) if want_dL_ddLdy else None
+        dx = torch.empty(3, n, dtype=torch.float32, device=x.device) if want_dL_dx else None
+        check(capi.lib().n2_grid_backward_backward_input(self._h, _stream_address(), x.data_ptr(), ps, ds, n, dL_ddLdx.data_ptr(), dL_dy.data_ptr(), _address(o),
+                                                         _address(dx), mode), "n2_grid_backward_backward_input")
         return o, dx
 
     def backward_fused(self, xyz, dL_dy, dL_ddLdx, dL_dy_second, want_dL_ddLdy=True, mode=GRAD_OVERWRITE):
         """backward (parameter gradients only) + backward_backward_input in one scatter pass."""
         x, ps, ds, n = _positions(xyz)
-        w = self.output_width()
-        for t, what in ((dL_dy, "dL_dy"), (dL_dy_second, "dL_dy_second")):
-            if t.dtype != torch.float16 or tuple(t.shape) != (w, n) or not t.is_contiguous():
-                raise N2Error(f"{what} must be a contiguous fp16 [output_width, N] tensor")
-        if dL_ddLdx.dtype != torch.float32 or tuple(dL_ddLdx.shape) != (3, n) or not dL_ddLdx.is_contiguous():
-            raise N2Error("dL_ddLdx must be a contiguous fp32 [3, N] tensor")
-        o = torch.empty((w, n), dtype=torch.float16, device=x.device) if want_dL_ddLdy else None
-        check(capi.lib().n2_grid_backward_fused(self._h, _stream(), ptr(x), C.c_uint32(ps), C.c_uint32(ds), C.c_uint32(n),
-                                                ptr(dL_dy), ptr(dL_ddLdx), ptr(dL_dy_second), ptr(o), C.c_int(mode)),
-              "n2_grid_backward_fused")
+        w = self._width
+        _check_rows(dL_dy, torch.float16, w, n, "dL_dy must be a contiguous fp16 [output_width, N] tensor")
+        _check_rows(dL_dy_second, torch.float16, w, n, "dL_dy_second must be a contiguous fp16 [output_width, N] tensor")
+        _check_rows(dL_ddLdx, torch.float32, 3, n, "dL_ddLdx must be a contiguous fp32 [3, N] tensor")
+        o = torch.empty(w, n, dtype=torch.float16, device=x.device) if want_dL_ddLdy else None
+        check(capi.lib().n2_grid_backward_fused(self._h, _stream_address(), x.data_ptr(), ps, ds, n, dL_dy.data_ptr(), dL_ddLdx.data_ptr(), dL_dy_second.data_ptr(),
+                                                _address(o), mode), "n2_grid_backward_fused")
         return o
 
     def corner_indices(self, xyz):
@@ -405,9 +417,10 @@ class NerfNetwork:
 
     def forward(self, coords, out=None):
         n = self._coords(coords)
-        self.reserve(n)
-        y = torch.empty((n, 16), dtype=torch.float16, device=coords.device) if out is None else out
-        check(capi.lib().n2_field_forward(self._h, _stream(), ptr(coords), C.c_uint32(n), ptr(y)), "n2_field_forward")
+        if n > self.max_batch:
+            self.reserve(n)
+        y = torch.empty(n, 16, dtype=torch.float16, device=coords.device) if out is None else out
+        check(capi.lib().n2_field_forward(self._h, _stream_address(), coords.data_ptr(), n, y.data_ptr()), "n2_field_forward")
         return y
 
     inference_mixed_precision = forward
@@ -415,9 +428,8 @@ class NerfNetwork:
     def backward(self, coords, dL_doutput, ek_batch_size=None, mode=GRAD_OVERWRITE):
         n = self._coords(coords)
         _check_half(dL_doutput, (n, 16), "dL_doutput")
-        check(capi.lib().n2_field_backward(self._h, _stream(), ptr(coords), C.c_uint32(n), ptr(dL_doutput),
-                                           C.c_uint32(n if ek_batch_size is None else ek_batch_size), C.c_int(mode)),
-              "n2_field_backward")
+        check(capi.lib().n2_field_backward(self._h, _stream_address(), coords.data_ptr(), n, dL_doutput.data_ptr(), n if ek_batch_size is None else ek_batch_size,
+                                           mode), "n2_field_backward")
 
     def select(self, source_index, n_source):
         """Makes the samples source_index (uint32/int32 CUDA tensor) of the last forward, which ran over n_source
@@ -427,19 +439,21 @@ class NerfNetwork:
         check(capi.lib().n2_field_select(self._h, _stream(), ptr(source_index), C.c_uint32(n_source), C.c_uint32(source_index.numel())),
               "n2_field_select")
 
-    def _sdf(self, fn, xyz):
+    def _sdf(self, call, what, xyz):
         x, ps, ds, n = _positions(xyz)
-        self.reserve(n)
-        out = torch.empty((16, n), dtype=torch.float16, device=x.device)
-        check(getattr(capi.lib(), fn)(self._h, _stream(), ptr(x), C.c_uint32(ps), C.c_uint32(ds), C.c_uint32(n),
-                                      ptr(out)), fn)
+        if n > self.max_batch:
+            self.reserve(n)
+        out = torch.empty(16, n, dtype=torch.float16, device=x.device)
+        rc = call(self._h, _stream_address(), x.data_ptr(), ps, ds, n, out.data_ptr())
+        if rc:
+            check(rc, what)
         return out
 
     def sdf(self, xyz):
-        return self._sdf("n2_field_sdf", xyz)
+        return self._sdf(capi.lib().n2_field_sdf, "n2_field_sdf", xyz)
 
     def density(self, xyz):
-        return self._sdf("n2_field_density", xyz)
+        return self._sdf(capi.lib().n2_field_density, "n2_field_density", xyz)
 
 
 class Adam:

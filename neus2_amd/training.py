@@ -301,9 +301,9 @@ class Trainer:
         n_rays = self.budget.rays_per_batch if n_rays is None else n_rays
         n_inference = self.budget.n_inference() if n_inference is None else n_inference
         seed = self.step_index if seed is None else seed
-        check(capi.lib().n2_trainer_set_training_step(self._h, C.c_uint32(self.step_index)), "n2_trainer_set_training_step")
-        check(capi.lib().n2_trainer_step(self._h, self._stream(), C.c_uint32(n_rays), C.c_uint32(n_inference),
-                                         C.c_uint32(seed)), "n2_trainer_step")
+        L = capi.lib()
+        check(L.n2_trainer_set_training_step(self._h, self.step_index), "n2_trainer_set_training_step")
+        check(L.n2_trainer_step(self._h, self._stream(), n_rays, n_inference, seed), "n2_trainer_step")
         self.step_index += 1
         if self.lr_schedule is not None:
             before = self.lr_schedule.learning_rate
