@@ -996,15 +996,17 @@ __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable 
 // holds 160 records when the batch has 5000 points.  Here a record claims a sum: every record writes its own number to the 16-bit place of its entry, and
 // whichever number stands there afterwards is the entry's sum (64-bit fixed point as above, so the result is the same whoever wins).  Nothing is cleared but
 // the sums that exist; the other entries' zeros go out while the first loads are under way (an accumulating launch leaves them alone), and a workgroup's
-// 32 KiB let four of 512 threads share a CU.  Every thread finds its records by their number among the bucket's, so no lane has to
+// 40 KiB let four of 512 threads share a CU.  Every thread finds its records by their number among the bucket's, so no lane has to
 // match a tile's run.  Levels of few entries keep an image, as does (range by range) a bucket with more records than
 // there are sums to claim.  What bounds it is the chain level -> bounds -> records -> sums and the 25 MB the gradient's zeros take.
 // Launch in us, image -> claims: 600 uniform points 15 -> 10.1, 5003 along rays 15.1 -> 10.6 (accumulating 15.6 -> 9.5), training step of 2^14 samples 17.5 -> 14.8.
-// (256 threads: the same up to 5000 points, 16 384 uniform points +4; 1024: +4; 128: +0.5)
-constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 4096;
+// (256 threads: the same up to 5000 points, 16 384 uniform points +4; 1024: +4; 128: +0.5.  32 KiB hold the claims of two thirds of the
+// points: 20 000 along rays 34.0, by grid_reduce_kernel, against 29.5.)
+constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 5120;
 constexpr uint32_t FEW_TILES = 64;                                  // a lane of every wave looks up one tile's run
 constexpr uint32_t FEW_CLAIMS = (FEW_WORDS - BKT_ENTRIES / 4) / 2;  // sums of both features, beside the table of 16-bit claims
 constexpr uint32_t FEW_RANGE = FEW_WORDS / 2;                       // entries of an image
+constexpr uint32_t FEW_PAIRS = 768;                                 // pair records of a bucket, on average, in a batch that takes the kernel (batch_buckets)
 
 // A bucket's records, numbered through its tiles' runs.
 struct N2FewRuns {
@@ -1516,10 +1518,11 @@ static uint32_t bucket_shift(const n2_grid_t* grid, uint32_t level, uint32_t n_p
 }
 static inline uint32_t bucket_count(uint32_t entries, uint32_t shift) { return (entries + (1u << shift) - 1u) >> shift; }
 
-// A batch's buckets.  few: it takes grid_reduce_few_kernel.  That is where on average its buckets hold no more records than threads on levels of pair
-// records, which is two thirds of the claims there are, and 2048 on the others, whose buckets are the smallest there can be: with the default table
-// up to 16 384 points.  Encoding forward and backward in us, grid_reduce_kernel | grid_reduce_few_kernel: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5,
-// 8192 33.5 | 29.1, 12 288 35.5 | 32.7, 16 384 37.7 | 37.0; along rays 3000 28.7 | 25.2, 16 384 34.9 | 31.1, 32 768 41.8 | 43.2.
+// A batch's buckets.  few: it takes grid_reduce_few_kernel.  That is where on average its buckets hold no more records than three quarters of the claims there
+// are on levels of pair records, and four times as many on the others, whose buckets are the smallest there can be: with the default table up to 24 576
+// points.  Encoding forward and backward in us, grid_reduce_kernel | grid_reduce_few_kernel: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5,
+// 8192 33.5 | 29.1, 12 288 35.5 | 32.7, 16 384 37.7 | 37.0, 20 000 37.5 | 36.4, 24 576 40.4 | 40.5; along rays 3000 28.7 | 25.2, 16 384 34.9 | 31.1, 20 000 34.0 | 29.5,
+// 24 576 36.0 | 32.0, 32 768 41.8 | 43.2.
 // groups: workgroups a bucket is split over; images: fp32 images of all split buckets (never more for a smaller batch: the groups per bucket grow with it).
 struct BatchBuckets {
 	bool few;
@@ -1533,7 +1536,7 @@ static BatchBuckets batch_buckets(const n2_grid_t* grid, uint32_t n_points) {
 	for (uint32_t l = 0; l < L && b.few; ++l) {
 		const bool pair = (grid->tab.pair_levels >> l) & 1u;
 		b.shift[l] = (uint8_t)bucket_shift(grid, l, n_points, FEW_BLOCK);
-		b.few = (uint64_t)n_points * (pair ? 4u : 8u) <= (uint64_t)bucket_count(grid->tab.entries[l], b.shift[l]) * (pair ? FEW_BLOCK : 4u * FEW_BLOCK);
+		b.few = (uint64_t)n_points * (pair ? 4u : 8u) <= (uint64_t)bucket_count(grid->tab.entries[l], b.shift[l]) * (pair ? FEW_PAIRS : 4u * FEW_PAIRS);
 	}
 	b.images = 0;
 	for (uint32_t l = 0; l < L; ++l) {
