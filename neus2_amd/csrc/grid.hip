@@ -498,9 +498,8 @@ __device__ __forceinline__ N2BinInput grid_bin_load(uint32_t level, uint32_t i, 
 	return in;
 }
 
-template <uint32_t MODE, bool FIRST, bool SECOND, bool WANT_OUT, bool CLAMP_X>
-__device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t N, const N2BinInput& in,
-                                               const __half2* __restrict__ params, __half* __restrict__ dL_ddLdy, uint32_t* e_out, float* r0_out, float* r1_out,
+template <uint32_t MODE, bool FIRST, bool SECOND, bool CLAMP_X>
+__device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t level, const N2BinInput& in, uint32_t* e_out, float* r0_out, float* r1_out,
                                                uint32_t* cell) {
 	const float scale = tab.scale[level];
 	N2Point p;
@@ -510,7 +509,6 @@ __device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t
 	cell[0] = p.c[0]; cell[1] = p.c[1]; cell[2] = p.c[2];
 	uint32_t e[8];
 	n2_corner_entries<MODE>(p, tab.entries[level], tab.resolution[level], e);
-	const size_t row = (size_t)level * 2;
 	float a0 = 0.f, a1 = 0.f, c0 = 0.f, c1 = 0.f, v0 = 0.f, v1 = 0.f, v2 = 0.f;
 	if (FIRST) {
 		a0 = __half2float(in.dy[0]);
@@ -521,8 +519,6 @@ __device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t
 		c1 = __half2float(in.g2[1]);
 		v0 = in.v[0] * scale; v1 = in.v[1] * scale; v2 = in.v[2] * scale;
 	}
-	const __half2* P = params + tab.offset[level];
-	float o0 = 0.f, o1 = 0.f;
 	// Corner k = i + 2 j + 4 l has weight X_i Y_j Z_l and signs (sx_i, sy_j, sz_l).  Its record is
 	//   a X Y Z + c (v0 sx Y Z + v1 sy X Z + v2 sz X Y)  =  (Y Z) (a X + c v0 sx) + (c X) (v1 sy Z + v2 sz Y),
 	// so the eight corners share two x terms per feature and four (y, z) terms.
@@ -548,20 +544,10 @@ __device__ __forceinline__ void grid_bin_point(const N2LevelTable& tab, uint32_t
 		if (SECOND) {
 			r0 = fmaf(B0[ix], Qyz[jl], r0);
 			r1 = fmaf(B1[ix], Qyz[jl], r1);
-			if (WANT_OUT) {
-				const float coef = fmaf(ix ? v0 : -v0, Pyz[jl], X[ix] * Qyz[jl]);
-				const float2 val = __half22float2(P[e[k]]);
-				o0 = fmaf(coef, val.x, o0);
-				o1 = fmaf(coef, val.y, o1);
-			}
 		}
 		e_out[k] = e[k];
 		r0_out[k] = r0;
 		r1_out[k] = r1;
-	}
-	if (SECOND && WANT_OUT) {
-		dL_ddLdy[row * N + i] = __float2half_rn(o0);
-		dL_ddLdy[(row + 1) * N + i] = __float2half_rn(o1);
 	}
 }
 
@@ -611,11 +597,10 @@ constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 // updates and prefix look-ups are therefore issued together, and nothing waits in a branch.  With each of them awaited where it was used,
 // and the second point's loads behind the first one's counters: training step at 2^18 samples 69 us, now 59 (57 and 47 on another card); trained 58, now 51; 2^18 uniform points
 // 51.5, now 47.8; 52344 samples 15.1, now 12.7.
-template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT, bool PAIR>
+template <uint32_t PER, bool FIRST, bool SECOND, bool PAIR>
 __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uint32_t level, const uint32_t tile, uint32_t N, uint32_t tiles,
                                               const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                               const __half* __restrict__ dL_dy, const float* __restrict__ v, const __half* __restrict__ g2,
-                                              const __half2* __restrict__ params, __half* __restrict__ dL_ddLdy,
                                               uint32_t* __restrict__ rec_vals, uint16_t* __restrict__ rec_keys, uint16_t* __restrict__ offsets,
                                               uint32_t* hist, uint32_t* prefix, uint32_t* stage_val, uint16_t* stage_key,
                                               const uint32_t* __restrict__ index, uint32_t n_cols) {
@@ -647,22 +632,16 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 		const uint32_t i = tile * bin_points(PER) + j * BIN_BLOCK + threadIdx.x;
 		const N2BinInput in = next;
 		bool valid = i < N;
-		if (valid && n2_level_masked(tab, level, i)) {  // a switched-off level: no records, zero second-order output
-			valid = false;
-			if (SECOND && WANT_OUT) {
-				dL_ddLdy[(size_t)level * 2 * N + i] = __float2half_rn(0.f);
-				dL_ddLdy[((size_t)level * 2 + 1) * N + i] = __float2half_rn(0.f);
-			}
-		}
+		if (valid && n2_level_masked(tab, level, i)) valid = false;  // a switched-off level: no records
 		uint32_t e[8], cell[3] = {0, 0, 0};
 		float r0[8], r1[8];
 #pragma unroll
 		for (uint32_t k = 0; k < 8; ++k) { e[k] = 0; r0[k] = 0.f; r1[k] = 0.f; }
 		if (valid) {
 			if (PAIR) {
-				grid_bin_point<N2_LEVEL_HASH, FIRST, SECOND, WANT_OUT, true>(tab, level, i, N, in, params, dL_ddLdy, e, r0, r1, cell);
+				grid_bin_point<N2_LEVEL_HASH, FIRST, SECOND, true>(tab, level, in, e, r0, r1, cell);
 			} else {
-#define CALL(M) grid_bin_point<M, FIRST, SECOND, WANT_OUT, false>(tab, level, i, N, in, params, dL_ddLdy, e, r0, r1, cell)
+#define CALL(M) grid_bin_point<M, FIRST, SECOND, false>(tab, level, in, e, r0, r1, cell)
 				N2_DISPATCH_MODE(tab.mode[level], CALL)
 #undef CALL
 			}
@@ -762,15 +741,47 @@ struct N2RideSums {
 	N2SlabReduce sums;
 	uint32_t blocks;
 };
+// The second order's dL_ddLdy = J v, gathered like the forward's Jacobian and contracted where it is formed: a group of eight workgroups that sort (an XCD each)
+// follows `every` groups that gather, in the order of n2_gather_item.  Inside the sorting itself, where a lane took the eight corners of its point and any
+// XCD's L2 came to hold every level, the gather took longer than all else: 2^18 second-order points (uniform) 154 -> 121 us for the launch (of which the
+// sorting is 59), 131 072 along rays 61 -> 51, 5003 9.4 -> 7.0; the calls 400 -> 363 (forward and first order included), 189 -> 173 and 39.2 -> 36.9.
+struct N2RideSecond {
+	__half* dL_ddLdy;
+	uint32_t blocks, every;  // workgroups that gather, and groups of them per group that sorts
+	uint32_t tiles, height;  // as n2_gather_item takes them
+};
 template <class Ride> constexpr bool RIDES_INPUT = false;
 template <bool STREAM> constexpr bool RIDES_INPUT<N2RideInput<STREAM>> = true;
 
-template <uint32_t PER, bool FIRST, bool SECOND, bool WANT_OUT, class Ride>
+template <uint32_t MODE>
+__device__ __forceinline__ void grid_second_item(const N2LevelTable& tab, uint32_t level, uint32_t i, uint32_t N, const float* __restrict__ xyz, uint32_t point_stride,
+                                                 uint32_t dim_stride, const __half2* __restrict__ params, const float* __restrict__ v, __half* __restrict__ dL_ddLdy) {
+	const uint32_t at = min(i, N - 1u);  // (lanes behind the last point take part in its pair's exchange)
+	const bool off = n2_level_masked(tab, level, at);
+	uint32_t both = 0u;
+	if (!__all(off)) {
+		const float* q = xyz + (size_t)at * point_stride;
+		const float p[3] = {n2_to_pairs(q[0]), n2_to_pairs(q[dim_stride]), n2_to_pairs(q[2 * (size_t)dim_stride])}, scale = tab.scale[level];
+		const float along[3] = {n2_to_pairs(v[at]), n2_to_pairs(v[(size_t)N + at]), n2_to_pairs(v[2 * (size_t)N + at])};
+		float feat[2], J[2][3];
+		n2_encode_level<MODE, true>(reinterpret_cast<const char*>(params + tab.offset[level]), tab.entries[level], tab.resolution[level], scale, p, scale, feat, J);
+		const __half2 h = __floats2half2_rn(fmaf(J[0][0], along[0], fmaf(J[0][1], along[1], J[0][2] * along[2])),
+		                                    fmaf(J[1][0], along[0], fmaf(J[1][1], along[1], J[1][2] * along[2])));
+		both = n2_from_pairs(*reinterpret_cast<const uint32_t*>(&h));
+	}
+	if (i >= N) return;
+	if (off) both = 0u;
+	const __half2 h = *reinterpret_cast<const __half2*>(&both);
+	dL_ddLdy[(size_t)level * 2 * N + i] = __low2half(h);
+	dL_ddLdy[((size_t)level * 2 + 1) * N + i] = __high2half(h);
+}
+
+template <uint32_t PER, bool FIRST, bool SECOND, class Ride>
 __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab, uint32_t first_level, uint32_t N, uint32_t tiles,
                                                               const float* __restrict__ xyz, uint32_t point_stride,
                                                               uint32_t dim_stride, const __half* __restrict__ dL_dy,
                                                               const float* __restrict__ v, const __half* __restrict__ g2,
-                                                              const __half2* __restrict__ params, __half* __restrict__ dL_ddLdy,
+                                                              const __half2* __restrict__ params,
                                                               uint32_t* __restrict__ rec_vals, uint16_t* __restrict__ rec_keys,
                                                               uint16_t* __restrict__ offsets,
                                                               const uint32_t* __restrict__ index, uint32_t n_cols, Ride ride) {
@@ -790,6 +801,20 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 		}
 		block = q * ride.every + m;
 		if (block >= tiles * tab.n_levels) return;
+	} else if constexpr (std::is_same<Ride, N2RideSecond>::value) {
+		const uint32_t group = block / N_XCD, lane = block - group * N_XCD, q = group / (ride.every + 1u), m = group - q * (ride.every + 1u);
+		if (m < ride.every) {
+			const uint32_t item = (q * ride.every + m) * N_XCD + lane, y = ride.height == 1u ? 0u : item / ride.tiles;
+			uint32_t level, tile;
+			if (item >= ride.blocks || !n2_gather_item(item - y * ride.tiles, y, ride.height, tab.n_levels, ride.tiles, level, tile)) return;
+			const uint32_t i = tile * BIN_BLOCK + threadIdx.x;
+#define CALL(M) grid_second_item<M>(tab, level, i, N, xyz, point_stride, dim_stride, params, v, ride.dL_ddLdy)
+			N2_DISPATCH_MODE(tab.mode[level], CALL)
+#undef CALL
+			return;
+		}
+		block = q * N_XCD + lane;
+		if (block >= tiles * tab.n_levels) return;
 	} else if constexpr (std::is_same<Ride, N2RideSums>::value) {
 		if (block < ride.blocks) {
 			constexpr uint32_t UNITS = BIN_BLOCK / 256;
@@ -804,11 +829,11 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 	if (threadIdx.x < BKT_MAX) hist[threadIdx.x] = 0;
 	__syncthreads();
 	if ((tab.pair_levels >> level) & 1u)
-		grid_bin_tile<PER, FIRST, SECOND, WANT_OUT, true>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, rec_vals,
-		                                             rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
+		grid_bin_tile<PER, FIRST, SECOND, true>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, rec_vals,
+		                                        rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
 	else
-		grid_bin_tile<PER, FIRST, SECOND, WANT_OUT, false>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, params, dL_ddLdy, rec_vals,
-		                                              rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
+		grid_bin_tile<PER, FIRST, SECOND, false>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, rec_vals,
+		                                         rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
 }
 
 // LDS float atomics retire about one lane every three clocks on this part, integer ones at ~9 (32-bit) and
@@ -1620,22 +1645,27 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.split_begin[l] = split;
 	auto bin = [&](auto per_thread) {
 		constexpr uint32_t PER = decltype(per_thread)::value;
-#define LAUNCH(F, S, O, RIDE, BLOCKS) grid_bin_kernel<PER, F, S, O><<<dim3(BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
-                                                                                                grid->params, dL_ddLdy, rec_vals, rec_keys, offsets, index, n_cols, RIDE)
+#define LAUNCH(F, S, RIDE, BLOCKS) grid_bin_kernel<PER, F, S><<<dim3(BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
+                                                                                          grid->params, rec_vals, rec_keys, offsets, index, n_cols, RIDE)
 		const uint32_t blocks = tiles * L;
 		const N2RideNone none;
 		if (rider.dL_dx != nullptr) {  // (first order alone)
 			const uint32_t riders = (n_points + BIN_BLOCK - 1) / BIN_BLOCK, every = (blocks + riders - 1) / riders, rows = L * grid->n_features;
-			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
-			else LAUNCH(true, false, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
+			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
+			else LAUNCH(true, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
 		} else if (rider.sums.units > 0) {  // (both orders)
 			const uint32_t riders = (rider.sums.units + BIN_BLOCK / 256 - 1) / (BIN_BLOCK / 256);
-			LAUNCH(true, true, false, (N2RideSums{rider.sums, riders}), riders + blocks);
-		} else if (first && second && out) LAUNCH(true, true, true, none, blocks);
-		else if (first && second) LAUNCH(true, true, false, none, blocks);
-		else if (second && out) LAUNCH(false, true, true, none, blocks);
-		else if (second) LAUNCH(false, true, false, none, blocks);
-		else LAUNCH(true, false, false, none, blocks);
+			LAUNCH(true, true, (N2RideSums{rider.sums, riders}), riders + blocks);
+		} else if (out) {
+			const N2GatherGrid g = n2_gather_grid(N2_ENCODING_XCD_MAX, n_points, L, BIN_BLOCK);
+			const uint32_t gather = g.x * g.y, every = (gather + blocks - 1) / blocks, sort_groups = (blocks + N_XCD - 1) / N_XCD;
+			const uint32_t gather_groups = (gather + N_XCD * every - 1) / (N_XCD * every), groups = std::max(sort_groups, gather_groups) * (every + 1);
+			const N2RideSecond ride{dL_ddLdy, gather, every, (n_points + BIN_BLOCK - 1) / BIN_BLOCK, g.y};
+			if (first) LAUNCH(true, true, ride, groups * N_XCD);
+			else LAUNCH(false, true, ride, groups * N_XCD);
+		} else if (first && second) LAUNCH(true, true, none, blocks);
+		else if (second) LAUNCH(false, true, none, blocks);
+		else LAUNCH(true, false, none, blocks);
 #undef LAUNCH
 	};
 	if (per == 1u) bin(std::integral_constant<uint32_t, 1>());

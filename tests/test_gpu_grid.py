@@ -368,6 +368,41 @@ def test_input_gradient_beside_the_scatter(n, levels, room):
         assert rel_l2(host(both), host(dg)) < RTOL
 
 
+# one point, the edges of a wave, of a workgroup and of the tiles (claims up to 24 576 points), batches above the size whose gathers are dealt by XCD; levels dealt in short turns;
+# both orders in the launch and the second alone
+@pytest.mark.parametrize("n,levels", [(1, 16), (63, 16), (65, 16), (511, 16), (513, 16), (5003, 16), (24576, 16), (24577, 16), (140001, 16), (600001, 16), (5003, 1), (5003, 3), (513, 7)])
+@pytest.mark.parametrize("first", [False, True])
+def test_second_order_output_beside_the_scatter(n, levels, first):
+    """dL_ddLdy is the same with and without scratch space for the sorted scatter, whose launch gathers it, up to the rounding of its fp32 sums; the parameters' gradients
+    are those of a call without it."""
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
+    sorting, adding = (GridEncoding(**{**CFG, "n_levels": levels}) for _ in range(2))
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = (torch.rand(sorting.n_params(), device="cuda", generator=gen) * 2 - 1).half()
+    dg = torch.zeros_like(dp)
+    assert sorting.reserve_scatter_workspace(n)
+    x, v = torch.rand((3, n), device="cuda", generator=gen), torch.randn((3, n), device="cuda", generator=gen) * 1e-3
+    dy, g2 = (torch.randn((2 * levels, n), device="cuda", generator=gen).half() for _ in range(2))
+    for off in ("none", "level", "per point"):
+        per_point = torch.randint(0, 2, (n,), device="cuda", generator=gen).float() if off == "per point" else None
+
+        def call(grid, want):
+            grid.set_params(dp, dg)
+            grid.set_max_level(0.5 if off == "level" else 1000.0)
+            grid.set_max_level_gpu(per_point)
+            dg.fill_(9.0)
+            if first:
+                out = grid.backward_fused(x, dy, v, g2, want_dL_ddLdy=want, mode=GRAD_OVERWRITE)
+            else:
+                out, _ = grid.backward_backward_input(x, v, g2, want_dL_ddLdy=want, mode=GRAD_OVERWRITE)
+            return out, dg.clone()
+
+        got, grads = call(sorting, True)
+        # eight products and their sum in fp32 on both sides (2^-24 each of values up to 4096 * 5e-3 * 2), one rounding to fp16 each
+        torch.testing.assert_close(got.float(), call(adding, True)[0].float(), rtol=2.0 ** -10, atol=2e-5)
+        assert (off != "none" or bool((got != 0).any())) and torch.equal(grads, call(sorting, False)[1])
+
+
 # batches whose buckets hold few records, up to the last one and the next; points that all fall into a few cells, in turn (no runs to merge), so that
 # single buckets hold more records than sums can be claimed for; tables of few and of small buckets
 @pytest.mark.parametrize("n,where,table", [(1, "anywhere", (16, 19)), (511, "anywhere", (16, 19)), (5003, "anywhere", (16, 19)), (16384, "anywhere", (16, 19)), (24576, "anywhere", (16, 19)), (24577, "anywhere", (16, 19)),
