@@ -88,6 +88,7 @@ struct FusedArgs {
 	float* row0;            // [row0_n] fp32 copy of row 0 of the first row0_n samples, or null
 	uint32_t row0_n;
 	int density;            // row 0 becomes the logistic density
+	uint32_t staged;        // levels that a query's gather leaves to its network kernel
 };
 
 // lane l's 16 bytes of fragment f
@@ -432,6 +433,7 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 	// (the full field's workgroups are counted along x alone)
 	const uint32_t y = FULL && !by_xcd ? blockIdx.x / tiles : blockIdx.y, x = FULL ? blockIdx.x - y * tiles : blockIdx.x;
 	if (!n2_gather_item(x, y, by_xcd ? 1u : a.n_levels, a.n_levels, tiles, level, tile)) return;
+	if (!FULL) level += a.staged;
 	const uint32_t n_live = a.live ? min(*a.live, a.N) : a.N;
 	const uint32_t i = tile * FG_BLOCK + threadIdx.x;
 	if (FULL) {
@@ -578,6 +580,111 @@ __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a
 	const bool valid = first + n < q.N;
 	store_sdf(q, y, valid ? first + n : q.N - 1u, valid, first + n, (int)g);
 }
+
+// The network of a large query, which takes the two coarsest levels' features from tables of its own in LDS (of the default grid 16^3 and 24^3 entries, with
+// the weights' fragments 80 KiB): one workgroup per CU stages them, half a wave works on each level's feature of the tile's 32 samples.  Gathered from memory
+// these levels cost a query nearly what fine ones do; here they are issue beside a chain of loads, and their rows are neither written nor read.  The next tile's
+// loads are under way meanwhile.  Level 2 of the default grid takes 157 KB and a launch of its own, beside which levels 0 to 2 were no cheaper than gathered
+// (staged by 256 workgroups 17.6 us for 2^20 points; points along rays 187 -> 192.5).  Tables copied four bytes a lane: 3.5 us more.
+constexpr int FS_BLOCK = 1024;
+constexpr uint32_t FS_GRID = 256, FS_LEVELS = 2, FS_LDS_MAX = 160 * 1024;
+__global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const FusedArgs a) {
+	extern __shared__ __align__(16) unsigned char smem[];
+	hf* F = reinterpret_cast<hf*>(smem);
+	unsigned char* const tables = smem + FF_SDF_COUNT * 1024;
+	const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
+	const uint32_t N = a.N, n_tiles = (N + 31u) / 32u, wave = blockIdx.x * (FS_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (FS_BLOCK / 64);
+	struct Start {
+		hf feat[16];
+		float p[3];
+	};
+	auto start = [&](uint32_t tile) __attribute__((always_inline)) {
+		Start t;
+		const uint32_t col = min(tile * 32u + n, N - 1u);
+		const float* q = a.pos + (size_t)col * a.ps;
+#pragma unroll
+		for (int d = 0; d < 3; ++d) t.p[d] = q[(size_t)d * a.ds];
+#pragma unroll
+		for (int j = 0; j < 8; ++j) {
+			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
+			// (levels that have no rows read those of the first level that does and are replaced, or meet weights of zero)
+			const uint32_t lr = level < FS_LEVELS || 2u * level >= a.enc_w ? FS_LEVELS : level;
+			t.feat[2 * j] = a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
+			t.feat[2 * j + 1] = a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
+		}
+		return t;
+	};
+	Start next = start(min(wave, n_tiles - 1u));
+	const uint32_t second = 4u * a.lv.entries[0], bytes = second + 4u * a.lv.entries[1];
+	{
+		// (the parameters are 16-byte aligned, and weights and levels come in multiples of that)
+		const uint4 *const from0 = reinterpret_cast<const uint4*>(a.table + a.lv.offset[0]), *const from1 = reinterpret_cast<const uint4*>(a.table + a.lv.offset[1]);
+		const uint32_t all = bytes / 16u, firsts = second / 16u;
+		constexpr uint32_t AHEAD = 5;
+		for (uint32_t k0 = threadIdx.x; k0 < all; k0 += AHEAD * FS_BLOCK) {
+			uint4 v[AHEAD];
+#pragma unroll
+			for (uint32_t q = 0; q < AHEAD; ++q) {
+				const uint32_t k = min(k0 + q * FS_BLOCK, all - 1u);
+				v[q] = k < firsts ? from0[k] : from1[k - firsts];
+			}
+#pragma unroll
+			for (uint32_t q = 0; q < AHEAD; ++q)
+				if (k0 + q * FS_BLOCK < all) reinterpret_cast<uint4*>(tables)[k0 + q * FS_BLOCK] = v[q];
+		}
+	}
+	for (int idx = threadIdx.x; idx < FF_SDF_COUNT * 64; idx += FS_BLOCK) *reinterpret_cast<half8*>(F + (size_t)idx * 8) = fused_frag_value(a, idx >> 6, idx & 63);
+	const float scale = a.lv.scale[g];
+	const uint32_t entries = a.lv.entries[g], res = a.lv.res[g];
+	const unsigned char* const table = tables + (g ? second : 0u);
+	const bool on = (uint32_t)g < a.lv.active_levels;  // a switched-off level: zero features
+	__syncthreads();
+	for (uint32_t tile = wave; tile < n_tiles; tile += n_waves) {
+		const uint32_t col_raw = tile * 32u + n;
+		const bool valid = col_raw < N;
+		half8 xs[3];
+#pragma unroll
+		for (int j = 0; j < 8; ++j) {
+			xs[j >> 2][2 * (j & 3)] = next.feat[2 * j];
+			xs[j >> 2][2 * (j & 3) + 1] = next.feat[2 * j + 1];
+		}
+		const float p[3] = {next.p[0], next.p[1], next.p[2]};
+		xs[2] = zero8();
+		if (g == 0) {
+#pragma unroll
+			for (int d = 0; d < 3; ++d) xs[2][d] = (hf)p[d] - (hf)0.5f;
+		}
+		next = start(tile + n_waves < n_tiles ? tile + n_waves : tile);
+		// sample n's feature of level g, summed up as in n2_encode_level
+		float w[3], s[2][2];  // [x corner][feature]
+		uint32_t c[3];
+#pragma unroll
+		for (int d = 0; d < 3; ++d) n2_locate(p[d], scale, w[d], c[d]);
+		const float uy = 1.f - w[1], uz = 1.f - w[2], w00 = uy * uz, w10 = w[1] * uz, w01 = uy * w[2], w11 = w[1] * w[2], ux = 1.f - w[0];
+#pragma unroll
+		for (uint32_t b = 0; b < 2; ++b) {
+			uint32_t at[4];
+			n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, c[0] + b, c[1], c[2], at);
+			float2 v[4];
+#pragma unroll
+			for (int k = 0; k < 4; ++k) v[k] = __half22float2(*reinterpret_cast<const __half2*>(table + at[k]));
+			s[b][0] = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, fmaf(w11, v[3].x, 0.f))));
+			s[b][1] = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, fmaf(w11, v[3].y, 0.f))));
+		}
+		const half2v feat = {(hf)fmaf(ux, s[0][0], w[0] * s[1][0]), (hf)fmaf(ux, s[0][1], w[0] * s[1][1])};
+		const uint32_t own = on ? __builtin_bit_cast(uint32_t, feat) : 0u, other = (uint32_t)__shfl_xor((int)own, 32);
+		if (g == 0) {
+			const half2v f0 = __builtin_bit_cast(half2v, own), f1 = __builtin_bit_cast(half2v, other);
+			xs[0][0] = f0[0]; xs[0][1] = f0[1];
+			xs[0][2] = f1[0]; xs[0][3] = f1[1];
+		}
+		half8 h[4];
+		const half8 y = sdf_net(F, lane, xs, h);
+		store_sdf(a, y, valid ? col_raw : N - 1u, valid, col_raw, g);
+		tile_fence();
+	}
+}
+
 
 // ----------------------------------------------------------------------------
 // the network kernel: a wave takes 32 samples per pass, lane (n, g) works for sample b0 + n on the levels l(j, g).
@@ -827,9 +934,9 @@ bool n2_fused_supported(const N2LevelTable& tab, uint32_t sdf_hidden_layers, uin
 }
 
 template <bool FULL>
-static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream_t s) {
+static void launch_gather(const FusedArgs& a, hipStream_t s) {
 	const uint32_t tiles = (a.N + FG_BLOCK - 1) / FG_BLOCK;
-	const N2GatherGrid g = n2_gather_grid(FULL ? N2_FIELD_XCD_MAX : N2_QUERY_XCD_MAX, a.N, tab.n_levels, FG_BLOCK);
+	const N2GatherGrid g = n2_gather_grid(FULL ? N2_FIELD_XCD_MAX : N2_QUERY_XCD_MAX, a.N, a.n_levels, FG_BLOCK);
 	const dim3 grid = FULL ? dim3(g.x * g.y + (a.frags ? FRAG_BLOCKS : 0u)) : dim3(g.x, g.y);
 	field_gather_kernel<FULL><<<grid, dim3(FG_BLOCK), 0, s>>>(a, tiles, g.y == 1u ? 1 : 0);
 }
@@ -839,6 +946,11 @@ static void launch_gather(const FusedArgs& a, const N2LevelTable& tab, hipStream
 // 4096 10.3 | 6.9, 6144 11.5 | 8.4, 8192 11.7 | 9.7, 10 240 12.85 | 12.7, 12 288 12.8 | 13.4, 16 384 14.1 | 16.3; a call from Python, bound by the host below
 // 5000 points: 1000 9.4 | 7.2, 8192 11.7 | 9.7.)
 constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 256 * FQ_POINTS;
+// From here on the two coarsest levels are the network kernel's (field_staged_forward_kernel): its start, two tables to every CU, costs smaller queries more than their
+// two levels.  (Call in us, gathered | staged, uniform points: 32 768 18.2 | 20.9, 65 536 28.6 | 29.3, 98 304 38.7 | 37.0, 2^17 50.4 | 46.9, 2^18 86.6 | 79.4, 2^20 294 | 279,
+// 2^21 567 | 532; along rays 65 536 20.2 | 21.7, 98 304 26.6 | 27.6, 2^17 34.0 | 34.4, 2^18 58.2 | 57.0, 2^20 187 | 185; on a lattice 2^17 32.8 | 33.0, 2^20 144.3 | 142.4.  Updates of
+// the occupancy grid: 2^17 samples 67.5 | 65.0, 2^20 254 | 248, 2^21 427 | 419, 700 000 266 | 252.)
+constexpr uint32_t QUERY_STAGED_MIN = 1u << 17;
 
 // ----------------------------------------------------------------------------
 // The SDF network on its own (48 inputs: coordinates, 32 features, padding) with the eikonal loss: network, d sdf / d input, normals from the
@@ -1060,7 +1172,7 @@ int n2_fused_field_forward(const N2FusedNets& nets, hipStream_t s, const float* 
 	}
 	{
 		N2ProfScope prof(N2_PROF_FIELD_GATHER, s);
-		launch_gather<true>(a, *nets.tab, s);
+		launch_gather<true>(a, s);
 	}
 	N2_LAUNCH_CHECK();
 	field_fused_forward_kernel<true, false><<<dim3(fused_grid(n)), dim3(FF_BLOCK), fused_lds(FF_COUNT, true), s>>>(a);
@@ -1089,7 +1201,22 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 		return N2_OK;
 	}
 	a.sdf_in = reinterpret_cast<hf*>(sdf_in);
-	launch_gather<false>(a, *nets.tab, s);
+	const N2LevelTable& tab = *nets.tab;
+	const bool dense = tab.n_levels > FS_LEVELS &&  // (one level at least is gathered)
+	                    tab.mode[0] == N2_LEVEL_DENSE && tab.mode[1] == N2_LEVEL_DENSE;
+	const uint64_t lds = FF_SDF_COUNT * 1024ull + 4ull * ((uint64_t)tab.entries[0] + tab.entries[1]);
+	if (n >= QUERY_STAGED_MIN && dense && lds <= FS_LDS_MAX) {
+		a.staged = FS_LEVELS;
+		FusedArgs others = a;
+		others.n_levels -= FS_LEVELS;
+		launch_gather<false>(others, s);
+		N2_LAUNCH_CHECK();
+		N2_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(field_staged_forward_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FS_LDS_MAX));
+		field_staged_forward_kernel<<<dim3(FS_GRID), dim3(FS_BLOCK), lds, s>>>(a);
+		N2_LAUNCH_CHECK();
+		return N2_OK;
+	}
+	launch_gather<false>(a, s);
 	N2_LAUNCH_CHECK();
 	// (bound by the latency of its loads at few registers: four workgroups per CU for large batches, where 512 | 1024 | 2048 of them
 	// take 28.8 | 26.8 | 31 us for 2^20 points and 45.8 | 38.2 | 41.6 for 2^21; every workgroup builds the fragments, which

@@ -168,6 +168,29 @@ def test_small_batches_equal_the_same_samples_in_a_large_one(n, active):
     assert torch.equal(net.forward(coords[:n].contiguous()), large[:n]) and bool(torch.isfinite(large.float()).all())
 
 
+# the last batch whose levels are all gathered and the first whose two coarsest are the network kernel's, tiles of 32 samples that are not whole; as few levels as that takes, and
+# fewer; levels switched off, of the two as well; tables that fill an LDS with the fragments and such that do not (32^3 entries and 39^3, 46^3)
+@pytest.mark.parametrize("n,cfg,active", [((1 << 17) - 8, {}, 1.0), (1 << 17, {}, 1.0), ((1 << 17) + 8, {}, 1.0), (300008, {}, 1.0), ((1 << 17) + 24, dict(n_levels=3), 1.0),
+                                                ((1 << 17) + 24, dict(n_levels=2), 1.0), ((1 << 17) + 24, {}, 0.25), ((1 << 17) + 24, {}, 0.0625), ((1 << 17) + 24, {}, 0.0),
+                                                ((1 << 17) + 24, dict(base_resolution=24, per_level_scale=1.1), 1.0), ((1 << 17) + 24, dict(base_resolution=32), 1.0),
+                                                ((1 << 17) + 24, dict(log2_hashmap_size=13), 1.0)])
+def test_large_queries_equal_their_parts(n, cfg, active):
+    """Bit for bit what smaller queries give, whose levels are all gathered."""
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork(**cfg)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    params = ((torch.rand(net.n_params(), device="cuda", generator=gen) - 0.5) * 0.3).half()
+    net.set_params(params)
+    net.encoding().set_max_level(active)
+    x = torch.rand((3, n), device="cuda", generator=gen) * 1.2 - 0.1
+    part = 1 << 15
+    for query, points in ((net.sdf, x), (net.density, x.t().contiguous())):
+        got = query(points)
+        for a in range(0, n, part):
+            want = query(x[:, a:a + part].contiguous())
+            assert torch.equal(got[:, a:a + part].view(torch.int16), want.view(torch.int16)), a
+
+
 # one tile past the line at which a query's and a forward's levels are no longer dealt to the XCDs
 @pytest.mark.parametrize("levels", [16, 14, 1])
 def test_batches_past_the_deal_by_xcd_equal_their_parts(levels):
