@@ -906,6 +906,8 @@ N2_API int n2_sdf_loss_backward(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stre
 // pitch of THEIR batch: whatever the training forward left there is gone, and with another batch size the rows land on what
 // the training layout keeps as zero padding (rows 3 + enc_w .. sdf_in_w, which the weight-gradient kernels read against
 // non-zero weight columns).  So the padding counts as not cleared, and a backward pass has to follow a new forward.
+// (The Jacobian's rows, which only that backward reads, serve as scratch: fused_scratch_bytes.)
+static uint64_t fused_scratch_bytes(const n2_field_t* f) { return 12ull * f->enc_w * f->max_batch; }
 static void inference_takes_sdf_in(n2_field_t* f) {
 	f->pad_n.sdf_in = 0;
 	f->last_n = 0;
@@ -925,7 +927,7 @@ static int field_sdf_impl(n2_field_t* f, const char* fn, n2_stream_t stream, con
 		const bool scratch = !n2_grid_lattice_order(f->grid);
 		if (scratch) inference_takes_sdf_in(f);
 		return n2_fused_field_sdf(fused_nets(f), s, d_xyz, ps, ds, n, d_output, nullptr, density,
-		                          scratch ? reinterpret_cast<n2_half*>(f->sdf_in) : nullptr);
+		                          scratch ? reinterpret_cast<n2_half*>(f->sdf_in) : nullptr, n, f->dy_dx, fused_scratch_bytes(f));
 	}
 	if (int rc = zero_padding(s, f->sdf_in, 3 + f->enc_w, f->sdf_in_w, n, f->pad_n.sdf_in)) return rc;
 	f->last_n = 0;  // the rows below are overwritten: a backward pass needs a new n2_field_forward
@@ -963,7 +965,7 @@ int n2_field_sdf_row0(n2_field_t* f, n2_stream_t stream, const float* d_xyz, uin
 		const bool scratch = !n2_grid_lattice_order(f->grid);
 		if (scratch) inference_takes_sdf_in(f);
 		return n2_fused_field_sdf(fused_nets(f), s, d_xyz, ps, ds, n, nullptr, d_row0, density,
-		                          scratch ? reinterpret_cast<n2_half*>(f->sdf_in) : nullptr, n_keep);
+		                          scratch ? reinterpret_cast<n2_half*>(f->sdf_in) : nullptr, n_keep, f->dy_dx, fused_scratch_bytes(f));
 	}
 	if (int rc = field_sdf_impl(f, "n2_field_sdf", stream, d_xyz, ps, ds, n, d_scratch16, density)) return rc;
 	const uint32_t keep = n_keep < n ? n_keep : n;

@@ -54,6 +54,7 @@ struct FusedLevels {
 	uint32_t active_levels;  // levels >= this are switched off (or do not exist)
 };
 
+constexpr uint32_t FS_LEVELS = 2, FB_LEVELS = 3;  // the coarsest levels of a large query (field_staged_forward_kernel): from LDS, and from blocks
 struct FusedArgs {
 	FusedLevels lv;
 	const __half2* table;   // grid parameters
@@ -88,7 +89,9 @@ struct FusedArgs {
 	float* row0;            // [row0_n] fp32 copy of row 0 of the first row0_n samples, or null
 	uint32_t row0_n;
 	int density;            // row 0 becomes the logistic density
-	uint32_t staged;        // levels that a query's gather leaves to its network kernel
+	uint32_t first_level;   // levels that a query's gather leaves to its network kernel
+	N2Block* blocks;        // [n_blocks] of the levels FS_LEVELS .. first_level - 1, each from a multiple of 256 on; written by the gather's launch
+	uint32_t n_blocks, block_first[FB_LEVELS];
 };
 
 // lane l's 16 bytes of fragment f
@@ -430,10 +433,20 @@ __global__ void __launch_bounds__(FG_BLOCK) field_gather_kernel(const FusedArgs 
 		return;
 	}
 	uint32_t level, tile;
+	if (!FULL && a.n_blocks > 0 && (by_xcd ? blockIdx.x >= gather_blocks : blockIdx.y >= a.n_levels)) {  // the workgroups behind those that gather: the coarse levels' blocks
+		const uint32_t k = (by_xcd ? blockIdx.x - gather_blocks : (blockIdx.y - a.n_levels) * gridDim.x + blockIdx.x) * FG_BLOCK + threadIdx.x;
+		if (k >= a.n_blocks) return;
+		uint32_t q = 0;
+#pragma unroll
+		for (uint32_t l = 1; l < FB_LEVELS; ++l) q += k >= a.block_first[l] ? 1u : 0u;
+		const uint32_t in = k - a.block_first[q], res = a.lv.res[FS_LEVELS + q];
+		if (in < n2_block_count(res)) a.blocks[k] = n2_make_block(reinterpret_cast<const char*>(a.table + a.lv.offset[FS_LEVELS + q]), a.lv.entries[FS_LEVELS + q], res, in);
+		return;
+	}
 	// (the full field's workgroups are counted along x alone)
 	const uint32_t y = FULL && !by_xcd ? blockIdx.x / tiles : blockIdx.y, x = FULL ? blockIdx.x - y * tiles : blockIdx.x;
 	if (!n2_gather_item(x, y, by_xcd ? 1u : a.n_levels, a.n_levels, tiles, level, tile)) return;
-	if (!FULL) level += a.staged;
+	if (!FULL) level += a.first_level;
 	const uint32_t n_live = a.live ? min(*a.live, a.N) : a.N;
 	const uint32_t i = tile * FG_BLOCK + threadIdx.x;
 	if (FULL) {
@@ -581,40 +594,47 @@ __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a
 	store_sdf(q, y, valid ? first + n : q.N - 1u, valid, first + n, (int)g);
 }
 
-// The network of a large query, which takes the two coarsest levels' features from tables of its own in LDS (of the default grid 16^3 and 24^3 entries, with
-// the weights' fragments 80 KiB): one workgroup per CU stages them, half a wave works on each level's feature of the tile's 32 samples.  Gathered from memory
-// these levels cost a query nearly what fine ones do; here they are issue beside a chain of loads, and their rows are neither written nor read.  The next tile's
-// loads are under way meanwhile.  Level 2 of the default grid takes 157 KB and a launch of its own, beside which levels 0 to 2 were no cheaper than gathered
-// (staged by 256 workgroups 17.6 us for 2^20 points; points along rays 187 -> 192.5).  Tables copied four bytes a lane: 3.5 us more.
+// The network of a large query, which takes the coarsest levels itself: gathered from memory they cost a query nearly what fine ones do, four lookups and lines a
+// point and level, here they are issue beside a chain of loads, and their rows are neither written nor read.
+//  * The two coarsest from tables of its own in LDS (of the default grid 16^3 and 24^3 entries, with the weights' fragments 80 KiB): one workgroup per CU stages
+//    them, half a wave works on each level's feature of the tile's 32 samples.  Level 2 of the default grid takes 157 KB and a launch of its own, beside which
+//    levels 0 to 2 were no cheaper than gathered (staged by 256 workgroups 17.6 us for 2^20 points; points along rays 187 -> 192.5).
+//  * BLOCKS: the three dense levels behind them from blocks (N2Block), a line a point instead of four.  The gather's launch writes them, in workgroups behind those that
+//    gather (in front 2 us more, in a launch of their own 4); nothing is kept for another call.  Lower lanes work on level 4, upper ones on 2 and 3, where
+//    the network's operands want them.  Held by the blocks' lines and latency: 2^20 uniform points 57 us against 32 without, of the gather's 260 it takes 43.  With 64
+//    samples to a wave and tile, so that no lane idles, uniform points took 2 % less and points in order and small batches up to 4 % more; with the next tile's blocks
+//    under way meanwhile (122 registers) uniform points 0.6 % less, ordered ones 1.5 % more.
 constexpr int FS_BLOCK = 1024;
-constexpr uint32_t FS_GRID = 256, FS_LEVELS = 2, FS_LDS_MAX = 160 * 1024;
+constexpr uint32_t FS_GRID = 256, FS_LDS_MAX = 160 * 1024;
+// features of one level of a sample from its entries at either x corner, summed up as in n2_encode_level
+__device__ __forceinline__ uint32_t staged_feature(const float (&w)[3], const uint32_t (&raw)[2][4]) {
+	const float uy = 1.f - w[1], uz = 1.f - w[2], w00 = uy * uz, w10 = w[1] * uz, w01 = uy * w[2], w11 = w[1] * w[2], ux = 1.f - w[0];
+	float s[2][2];  // [x corner][feature]
+#pragma unroll
+	for (uint32_t b = 0; b < 2; ++b) {
+		float2 v[4];
+#pragma unroll
+		for (int k = 0; k < 4; ++k) v[k] = __half22float2(*reinterpret_cast<const __half2*>(&raw[b][k]));
+		s[b][0] = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, fmaf(w11, v[3].x, 0.f))));
+		s[b][1] = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, fmaf(w11, v[3].y, 0.f))));
+	}
+	const half2v feat = {(hf)fmaf(ux, s[0][0], w[0] * s[1][0]), (hf)fmaf(ux, s[0][1], w[0] * s[1][1])};
+	return __builtin_bit_cast(uint32_t, feat);
+}
+template <bool BLOCKS>
 __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const FusedArgs a) {
 	extern __shared__ __align__(16) unsigned char smem[];
 	hf* F = reinterpret_cast<hf*>(smem);
 	unsigned char* const tables = smem + FF_SDF_COUNT * 1024;
 	const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
 	const uint32_t N = a.N, n_tiles = (N + 31u) / 32u, wave = blockIdx.x * (FS_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (FS_BLOCK / 64);
-	struct Start {
-		hf feat[16];
-		float p[3];
-	};
-	auto start = [&](uint32_t tile) __attribute__((always_inline)) {
-		Start t;
-		const uint32_t col = min(tile * 32u + n, N - 1u);
-		const float* q = a.pos + (size_t)col * a.ps;
+	auto position = [&](uint32_t tile, float (&p)[3]) __attribute__((always_inline)) {
+		const float* q = a.pos + (size_t)min(tile * 32u + n, N - 1u) * a.ps;
 #pragma unroll
-		for (int d = 0; d < 3; ++d) t.p[d] = q[(size_t)d * a.ds];
-#pragma unroll
-		for (int j = 0; j < 8; ++j) {
-			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
-			// (levels that have no rows read those of the first level that does and are replaced, or meet weights of zero)
-			const uint32_t lr = level < FS_LEVELS || 2u * level >= a.enc_w ? FS_LEVELS : level;
-			t.feat[2 * j] = a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
-			t.feat[2 * j + 1] = a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
-		}
-		return t;
+		for (int d = 0; d < 3; ++d) p[d] = q[(size_t)d * a.ds];
 	};
-	Start next = start(min(wave, n_tiles - 1u));
+	float next[3];
+	position(min(wave, n_tiles - 1u), next);
 	const uint32_t second = 4u * a.lv.entries[0], bytes = second + 4u * a.lv.entries[1];
 	{
 		// (the parameters are 16-byte aligned, and weights and levels come in multiples of that)
@@ -638,49 +658,84 @@ __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const Fu
 	const uint32_t entries = a.lv.entries[g], res = a.lv.res[g];
 	const unsigned char* const table = tables + (g ? second : 0u);
 	const bool on = (uint32_t)g < a.lv.active_levels;  // a switched-off level: zero features
+	float bscale[2];
+	uint32_t bres[2];
+	const N2Block* bfrom[2];
+	bool bon[2];
+#pragma unroll
+	for (uint32_t e = 0; e < 2; ++e) {
+		const uint32_t level = g ? 2u + e : 4u;
+		bscale[e] = a.lv.scale[level];
+		bres[e] = a.lv.res[level];
+		bfrom[e] = a.blocks + a.block_first[level - FS_LEVELS];
+		bon[e] = level < a.lv.active_levels;
+	}
 	__syncthreads();
 	for (uint32_t tile = wave; tile < n_tiles; tile += n_waves) {
 		const uint32_t col_raw = tile * 32u + n;
 		const bool valid = col_raw < N;
+		const uint32_t col = valid ? col_raw : N - 1u;
+		const float p[3] = {next[0], next[1], next[2]};
 		half8 xs[3];
 #pragma unroll
 		for (int j = 0; j < 8; ++j) {
-			xs[j >> 2][2 * (j & 3)] = next.feat[2 * j];
-			xs[j >> 2][2 * (j & 3) + 1] = next.feat[2 * j + 1];
+			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
+			// (levels that have no rows read those of the first level that does and are replaced, or meet weights of zero)
+			const uint32_t lr = level < a.first_level || 2u * level >= a.enc_w ? a.first_level : level;
+			xs[j >> 2][2 * (j & 3)] = a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
+			xs[j >> 2][2 * (j & 3) + 1] = a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
 		}
-		const float p[3] = {next.p[0], next.p[1], next.p[2]};
+		// the levels from blocks: lower lanes 4, upper ones 2 and 3, where the network's operands have them
+		constexpr uint32_t ITEMS = BLOCKS ? 2 : 0;
+		float bw[ITEMS + 1][3];
+		uint32_t braw[ITEMS + 1][2][4];
+#pragma unroll
+		for (uint32_t e = 0; e < ITEMS; ++e) {
+			uint32_t c[3];
+#pragma unroll
+			for (int d = 0; d < 3; ++d) n2_locate(p[d], bscale[e], bw[e][d], c[d]);
+			const N2Block* const row = bfrom[e] + n2_block_row(bres[e], c[1], c[2]);
+#pragma unroll
+			for (uint32_t b = 0; b < 2; ++b) {
+				const N2Block v = row[min(c[0] + b, bres[e])];
+#pragma unroll
+				for (int q = 0; q < 4; ++q) braw[e][b][q] = v.entry[q];
+			}
+		}
+		position(tile + n_waves < n_tiles ? tile + n_waves : tile, next);
 		xs[2] = zero8();
 		if (g == 0) {
 #pragma unroll
 			for (int d = 0; d < 3; ++d) xs[2][d] = (hf)p[d] - (hf)0.5f;
 		}
-		next = start(tile + n_waves < n_tiles ? tile + n_waves : tile);
-		// sample n's feature of level g, summed up as in n2_encode_level
-		float w[3], s[2][2];  // [x corner][feature]
-		uint32_t c[3];
+		// sample n's feature of level g
+		float w[3];
+		uint32_t c[3], raw[2][4];
 #pragma unroll
 		for (int d = 0; d < 3; ++d) n2_locate(p[d], scale, w[d], c[d]);
-		const float uy = 1.f - w[1], uz = 1.f - w[2], w00 = uy * uz, w10 = w[1] * uz, w01 = uy * w[2], w11 = w[1] * w[2], ux = 1.f - w[0];
 #pragma unroll
 		for (uint32_t b = 0; b < 2; ++b) {
 			uint32_t at[4];
 			n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, c[0] + b, c[1], c[2], at);
-			float2 v[4];
 #pragma unroll
-			for (int k = 0; k < 4; ++k) v[k] = __half22float2(*reinterpret_cast<const __half2*>(table + at[k]));
-			s[b][0] = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, fmaf(w11, v[3].x, 0.f))));
-			s[b][1] = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, fmaf(w11, v[3].y, 0.f))));
+			for (int k = 0; k < 4; ++k) raw[b][k] = *reinterpret_cast<const uint32_t*>(table + at[k]);
 		}
-		const half2v feat = {(hf)fmaf(ux, s[0][0], w[0] * s[1][0]), (hf)fmaf(ux, s[0][1], w[0] * s[1][1])};
-		const uint32_t own = on ? __builtin_bit_cast(uint32_t, feat) : 0u, other = (uint32_t)__shfl_xor((int)own, 32);
-		if (g == 0) {
-			const half2v f0 = __builtin_bit_cast(half2v, own), f1 = __builtin_bit_cast(half2v, other);
-			xs[0][0] = f0[0]; xs[0][1] = f0[1];
-			xs[0][2] = f1[0]; xs[0][3] = f1[1];
+		const uint32_t own = on ? staged_feature(w, raw) : 0u, other = (uint32_t)__shfl_xor((int)own, 32);
+		uint32_t x4[4] = {0u, 0u, 0u, 0u};
+		*reinterpret_cast<half8*>(x4) = xs[0];
+		if constexpr (BLOCKS) {
+			const uint32_t b0 = bon[0] ? staged_feature(bw[0], braw[0]) : 0u, b1 = bon[1] ? staged_feature(bw[1], braw[1]) : 0u;
+			x4[0] = g ? b0 : own;
+			x4[1] = g ? b1 : other;
+			x4[2] = g ? x4[2] : b0;
+		} else if (g == 0) {
+			x4[0] = own;
+			x4[1] = other;
 		}
+		xs[0] = *reinterpret_cast<half8*>(x4);
 		half8 h[4];
 		const half8 y = sdf_net(F, lane, xs, h);
-		store_sdf(a, y, valid ? col_raw : N - 1u, valid, col_raw, g);
+		store_sdf(a, y, col, valid, col_raw, g);
 		tile_fence();
 	}
 }
@@ -937,7 +992,8 @@ template <bool FULL>
 static void launch_gather(const FusedArgs& a, hipStream_t s) {
 	const uint32_t tiles = (a.N + FG_BLOCK - 1) / FG_BLOCK;
 	const N2GatherGrid g = n2_gather_grid(FULL ? N2_FIELD_XCD_MAX : N2_QUERY_XCD_MAX, a.N, a.n_levels, FG_BLOCK);
-	const dim3 grid = FULL ? dim3(g.x * g.y + (a.frags ? FRAG_BLOCKS : 0u)) : dim3(g.x, g.y);
+	const uint32_t more = (a.n_blocks + FG_BLOCK - 1) / FG_BLOCK;
+	const dim3 grid = FULL ? dim3(g.x * g.y + (a.frags ? FRAG_BLOCKS : 0u)) : g.y == 1u ? dim3(g.x + more) : dim3(g.x, g.y + (more + g.x - 1) / g.x);
 	field_gather_kernel<FULL><<<grid, dim3(FG_BLOCK), 0, s>>>(a, tiles, g.y == 1u ? 1 : 0);
 }
 
@@ -951,6 +1007,10 @@ constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 256 * FQ_POINTS;
 // 2^21 567 | 532; along rays 65 536 20.2 | 21.7, 98 304 26.6 | 27.6, 2^17 34.0 | 34.4, 2^18 58.2 | 57.0, 2^20 187 | 185; on a lattice 2^17 32.8 | 33.0, 2^20 144.3 | 142.4.  Updates of
 // the occupancy grid: 2^17 samples 67.5 | 65.0, 2^20 254 | 248, 2^21 427 | 419, 700 000 266 | 252.)
 constexpr uint32_t QUERY_STAGED_MIN = 1u << 17;
+// ... and from here on three more come from blocks: making these costs smaller queries what they save.  (Call in us, staged | with blocks: uniform points 2^17 46.8 | 46.5, 2^18
+// 79.3 | 74.9, 2^19 149 | 140, 2^20 279 | 260, 2^21 533 | 495; along rays 33.6 | 36.0, 57.3 | 58.0, 101 | 99, 184 | 178, 344 | 331; on a lattice 32.6 | 34.7, 56.4 | 56.9, 79.1 | 78.1,
+// 142.5 | 136.1, 261 | 251.  Updates of the occupancy grid: 2^19 samples 161.6 | 155.7, 700 000 252 | 239, 2^21 418 | 403.)
+constexpr uint32_t QUERY_BLOCKS_MIN = 1u << 18;
 
 // ----------------------------------------------------------------------------
 // The SDF network on its own (48 inputs: coordinates, 32 features, padding) with the eikonal loss: network, d sdf / d input, normals from the
@@ -1181,7 +1241,7 @@ int n2_fused_field_forward(const N2FusedNets& nets, hipStream_t s, const float* 
 }
 
 int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
-                       float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n) {
+                       float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n, void* scratch, uint64_t scratch_bytes) {
 	FusedArgs a = fused_base(nets, n);
 	a.pos = d_xyz; a.ps = ps; a.ds = ds;
 	a.sdf_out = reinterpret_cast<hf*>(d_out_soa);
@@ -1206,13 +1266,27 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 	                    tab.mode[0] == N2_LEVEL_DENSE && tab.mode[1] == N2_LEVEL_DENSE;
 	const uint64_t lds = FF_SDF_COUNT * 1024ull + 4ull * ((uint64_t)tab.entries[0] + tab.entries[1]);
 	if (n >= QUERY_STAGED_MIN && dense && lds <= FS_LDS_MAX) {
-		a.staged = FS_LEVELS;
+		a.first_level = FS_LEVELS;
+		uint32_t blocks = 0;
+		bool blocked = a.n_levels > FS_LEVELS + FB_LEVELS && n >= QUERY_BLOCKS_MIN;
+		for (uint32_t l = 0; l < FB_LEVELS && blocked; ++l) {
+			blocked = tab.mode[FS_LEVELS + l] == N2_LEVEL_DENSE;
+			a.block_first[l] = blocks;
+			blocks += (n2_block_count(tab.resolution[FS_LEVELS + l]) + FG_BLOCK - 1) / FG_BLOCK * FG_BLOCK;
+		}
+		blocked = blocked && sizeof(N2Block) * (uint64_t)blocks <= scratch_bytes;
+		if (blocked) {
+			a.first_level += FB_LEVELS;
+			a.blocks = reinterpret_cast<N2Block*>(scratch);
+			a.n_blocks = blocks;
+		}
 		FusedArgs others = a;
-		others.n_levels -= FS_LEVELS;
+		others.n_levels -= a.first_level;
 		launch_gather<false>(others, s);
 		N2_LAUNCH_CHECK();
-		N2_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(field_staged_forward_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FS_LDS_MAX));
-		field_staged_forward_kernel<<<dim3(FS_GRID), dim3(FS_BLOCK), lds, s>>>(a);
+		auto* const kernel = blocked ? field_staged_forward_kernel<true> : field_staged_forward_kernel<false>;
+		N2_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FS_LDS_MAX));
+		kernel<<<dim3(FS_GRID), dim3(FS_BLOCK), lds, s>>>(a);
 		N2_LAUNCH_CHECK();
 		return N2_OK;
 	}

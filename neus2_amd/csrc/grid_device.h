@@ -71,6 +71,23 @@ __device__ __forceinline__ void n2_corner_bytes(uint32_t entries, uint32_t res, 
 	}
 }
 
+// A dense level's entries in blocks: block (x, y, z) holds the four (y, z) corners, at x corner x and in the order of n2_corner_bytes, of the cell that
+// starts at y - 1 and z - 1.  x runs up to the level's resolution, y and z one further: cells are bounded as there, and cell -1 is the first.
+struct alignas(16) N2Block {
+	uint32_t entry[4];
+};
+N2_HD inline uint32_t n2_block_count(uint32_t res) { return (res + 1u) * (res + 2u) * (res + 2u); }
+__device__ __forceinline__ uint32_t n2_block_row(uint32_t res, uint32_t cy, uint32_t cz) { return (res + 1u) * (min(cy + 1u, res + 1u) + (res + 2u) * min(cz + 1u, res + 1u)); }
+__device__ __forceinline__ N2Block n2_make_block(const char* __restrict__ table, uint32_t entries, uint32_t res, uint32_t k) {
+	const uint32_t row = k / (res + 1u), x = k - row * (res + 1u), z = row / (res + 2u), y = row - z * (res + 2u);
+	uint32_t at[4];
+	n2_corner_bytes<N2_LEVEL_DENSE>(entries, res, x, y - 1u, z - 1u, at);
+	N2Block b;
+#pragma unroll
+	for (int q = 0; q < 4; ++q) b.entry[q] = *reinterpret_cast<const uint32_t*>(table + at[q]);
+	return b;
+}
+
 // value held by the other lane of the pair (lane ^ 1), and by the pair's lane M: quad permutes inside the VALU, no LDS crossbar
 __device__ __forceinline__ uint32_t n2_pair_swap(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, true); }
 __device__ __forceinline__ float n2_pair_swap(float x) { return __uint_as_float(n2_pair_swap(__float_as_uint(x))); }

@@ -168,12 +168,14 @@ def test_small_batches_equal_the_same_samples_in_a_large_one(n, active):
     assert torch.equal(net.forward(coords[:n].contiguous()), large[:n]) and bool(torch.isfinite(large.float()).all())
 
 
-# the last batch whose levels are all gathered and the first whose two coarsest are the network kernel's, tiles of 32 samples that are not whole; as few levels as that takes, and
-# fewer; levels switched off, of the two as well; tables that fill an LDS with the fragments and such that do not (32^3 entries and 39^3, 46^3)
-@pytest.mark.parametrize("n,cfg,active", [((1 << 17) - 8, {}, 1.0), (1 << 17, {}, 1.0), ((1 << 17) + 8, {}, 1.0), (300008, {}, 1.0), ((1 << 17) + 24, dict(n_levels=3), 1.0),
-                                                ((1 << 17) + 24, dict(n_levels=2), 1.0), ((1 << 17) + 24, {}, 0.25), ((1 << 17) + 24, {}, 0.0625), ((1 << 17) + 24, {}, 0.0),
-                                                ((1 << 17) + 24, dict(base_resolution=24, per_level_scale=1.1), 1.0), ((1 << 17) + 24, dict(base_resolution=32), 1.0),
-                                                ((1 << 17) + 24, dict(log2_hashmap_size=13), 1.0)])
+# the last batch whose levels are all gathered and the first whose two coarsest are the network kernel's, the last and first with three more from blocks; tiles of 32 samples that are
+# not whole; as few levels as that takes, and fewer; levels switched off, of these as well; tables that fill an LDS with the fragments and such that do not (base resolutions 24 and 32);
+# a fifth level that is hashed, all of them but one
+@pytest.mark.parametrize("n,cfg,active", [((1 << 17) - 8, {}, 1.0), (1 << 17, {}, 1.0), ((1 << 17) + 8, {}, 1.0), ((1 << 18) - 8, {}, 1.0), (1 << 18, {}, 1.0), ((1 << 18) + 8, {}, 1.0), (700008, {}, 1.0),
+                                          ((1 << 17) + 24, dict(n_levels=3), 1.0), ((1 << 17) + 24, dict(n_levels=2), 1.0), ((1 << 18) + 24, dict(n_levels=6), 1.0), ((1 << 18) + 24, dict(n_levels=5), 1.0),
+                                          ((1 << 18) + 24, {}, 0.25), ((1 << 18) + 24, {}, 0.1875), ((1 << 18) + 24, {}, 0.125), ((1 << 18) + 24, {}, 0.0625), ((1 << 17) + 24, {}, 0.0625), ((1 << 18) + 24, {}, 0.0),
+                                          ((1 << 18) + 24, dict(base_resolution=24, per_level_scale=1.1), 1.0), ((1 << 18) + 24, dict(base_resolution=32), 1.0),
+                                          ((1 << 18) + 24, dict(log2_hashmap_size=17), 1.0), ((1 << 18) + 24, dict(log2_hashmap_size=13), 1.0)])
 def test_large_queries_equal_their_parts(n, cfg, active):
     """Bit for bit what smaller queries give, whose levels are all gathered."""
     from neus2_amd.tcnn_api import NerfNetwork
