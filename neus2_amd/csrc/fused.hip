@@ -353,7 +353,10 @@ __device__ __forceinline__ float pair_finish(const PairItem& it, uint32_t b) {
 	asm volatile("" : "+v"(feat));  // rounded to fp32 before fp16, as in the gather kernels: one instruction could do both and round once
 	return feat;
 }
-// Inference on points in no particular order: the features of one (point, level) item per lane
+// Inference on points in no particular order: between gather and network a level's features stand side by side, a row of N words to each level.  (In the training forward's
+// rows of halves, which they were, the network's loads and the gather's stores took the address units twice: queries of 2^20 uniform points 259 -> 254 us, 2^21 494 -> 484.)
+__device__ __forceinline__ uint32_t* query_rows(const FusedArgs& a) { return reinterpret_cast<uint32_t*>(a.sdf_in); }
+// The features of one (point, level) item per lane
 __device__ __forceinline__ void gather_features(const FusedArgs& a, uint32_t level, uint32_t i, uint32_t n_live) {
 	uint32_t both = 0u;
 	if (level < a.lv.active_levels) {  // a switched-off level: zero features
@@ -368,10 +371,7 @@ __device__ __forceinline__ void gather_features(const FusedArgs& a, uint32_t lev
 		const half2v packed = {(hf)feat[0], (hf)feat[1]};
 		both = n2_from_pairs(__builtin_bit_cast(uint32_t, packed));
 	}
-	if (i >= n_live) return;
-	const half2v feat = __builtin_bit_cast(half2v, both);
-	a.sdf_in[(size_t)(3 + 2 * level) * a.N + i] = feat[0];
-	a.sdf_in[(size_t)(4 + 2 * level) * a.N + i] = feat[1];
+	if (i < n_live) query_rows(a)[(size_t)level * a.N + i] = both;
 }
 
 // first column and number of samples of a listed pass
@@ -600,26 +600,30 @@ __global__ void __launch_bounds__(FQ_BLOCK) field_query_kernel(const FusedArgs a
 //    them, half a wave works on each level's feature of the tile's 32 samples.  Level 2 of the default grid takes 157 KB and a launch of its own, beside which
 //    levels 0 to 2 were no cheaper than gathered (staged by 256 workgroups 17.6 us for 2^20 points; points along rays 187 -> 192.5).
 //  * BLOCKS: the three dense levels behind them from blocks (N2Block), a line a point instead of four.  The gather's launch writes them, in workgroups behind those that
-//    gather (in front 2 us more, in a launch of their own 4); nothing is kept for another call.  Lower lanes work on level 4, upper ones on 2 and 3, where
-//    the network's operands want them.  Held by the blocks' lines and latency: 2^20 uniform points 57 us against 32 without, of the gather's 260 it takes 43.  With 64
-//    samples to a wave and tile, so that no lane idles, uniform points took 2 % less and points in order and small batches up to 4 % more; with the next tile's blocks
-//    under way meanwhile (122 registers) uniform points 0.6 % less, ordered ones 1.5 % more.
+//    gather (in front 2 us more, in a launch of their own 4); nothing is kept for another call.  Lower lanes take level 4, upper ones level 2, where the network's
+//    operands want them, and of level 3 either half an x corner.  Held by the blocks' lines and latency: 2^20 uniform points 47 us against 32 without, of the gather's
+//    260 it takes 45.  With 64 samples to a wave and tile points in order and small batches took up to 4 % more; with the next tile's blocks under way meanwhile
+//    ordered points 1.5 % more; tables that an index can run past, which spares the modulo: no change.
 constexpr int FS_BLOCK = 1024;
 constexpr uint32_t FS_GRID = 256, FS_LDS_MAX = 160 * 1024;
-// features of one level of a sample from its entries at either x corner, summed up as in n2_encode_level
-__device__ __forceinline__ uint32_t staged_feature(const float (&w)[3], const uint32_t (&raw)[2][4]) {
-	const float uy = 1.f - w[1], uz = 1.f - w[2], w00 = uy * uz, w10 = w[1] * uz, w01 = uy * w[2], w11 = w[1] * w[2], ux = 1.f - w[0];
-	float s[2][2];  // [x corner][feature]
+// a level's features at one x corner of a sample's cell from the four entries there, and in between: summed up as in n2_encode_level
+__device__ __forceinline__ float2 staged_corner(const float (&w)[3], const uint32_t (&raw)[4]) {
+	const float uy = 1.f - w[1], uz = 1.f - w[2], w00 = uy * uz, w10 = w[1] * uz, w01 = uy * w[2], w11 = w[1] * w[2];
+	float2 v[4];
 #pragma unroll
-	for (uint32_t b = 0; b < 2; ++b) {
-		float2 v[4];
-#pragma unroll
-		for (int k = 0; k < 4; ++k) v[k] = __half22float2(*reinterpret_cast<const __half2*>(&raw[b][k]));
-		s[b][0] = fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, fmaf(w11, v[3].x, 0.f))));
-		s[b][1] = fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, fmaf(w11, v[3].y, 0.f))));
-	}
-	const half2v feat = {(hf)fmaf(ux, s[0][0], w[0] * s[1][0]), (hf)fmaf(ux, s[0][1], w[0] * s[1][1])};
+	for (int k = 0; k < 4; ++k) v[k] = __half22float2(*reinterpret_cast<const __half2*>(&raw[k]));
+	return make_float2(fmaf(w00, v[0].x, fmaf(w10, v[1].x, fmaf(w01, v[2].x, fmaf(w11, v[3].x, 0.f)))), fmaf(w00, v[0].y, fmaf(w10, v[1].y, fmaf(w01, v[2].y, fmaf(w11, v[3].y, 0.f)))));
+}
+__device__ __forceinline__ uint32_t staged_feature(float wx, const float2 lo, const float2 hi) {
+	const float ux = 1.f - wx;
+	const half2v feat = {(hf)fmaf(ux, lo.x, wx * hi.x), (hf)fmaf(ux, lo.y, wx * hi.y)};
 	return __builtin_bit_cast(uint32_t, feat);
+}
+// what lanes n and n + 32 hold, for both of them
+__device__ __forceinline__ void staged_halves(float own, float& lower, float& upper) {
+	const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(own), __float_as_uint(own), false, false);
+	lower = __uint_as_float(r[0]);
+	upper = __uint_as_float(r[1]);
 }
 template <bool BLOCKS>
 __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const FusedArgs a) {
@@ -658,18 +662,24 @@ __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const Fu
 	const uint32_t entries = a.lv.entries[g], res = a.lv.res[g];
 	const unsigned char* const table = tables + (g ? second : 0u);
 	const bool on = (uint32_t)g < a.lv.active_levels;  // a switched-off level: zero features
-	float bscale[2];
-	uint32_t bres[2];
-	const N2Block* bfrom[2];
-	bool bon[2];
+	// the levels from blocks: lower lanes have 4, upper ones 2, where the network's operands want them; of level 3 either half of the wave takes an x corner
+	const uint32_t blevel = g ? 2u : 4u, bres = a.lv.res[blevel], cres = a.lv.res[3];
+	const float bscale = a.lv.scale[blevel], cscale = a.lv.scale[3];
+	const N2Block *const bfrom = a.blocks + a.block_first[blevel - FS_LEVELS], *const cfrom = a.blocks + a.block_first[3 - FS_LEVELS];
+	const bool bon = blevel < a.lv.active_levels, con = 3u < a.lv.active_levels;
+	// (the next tile's rows are fetched ahead where waves take several tiles)
+	uint32_t ahead[8];
+	auto fetch_rows = [&](uint32_t tile) __attribute__((always_inline)) {
+		const uint32_t col = min(tile * 32u + n, N - 1u);
 #pragma unroll
-	for (uint32_t e = 0; e < 2; ++e) {
-		const uint32_t level = g ? 2u + e : 4u;
-		bscale[e] = a.lv.scale[level];
-		bres[e] = a.lv.res[level];
-		bfrom[e] = a.blocks + a.block_first[level - FS_LEVELS];
-		bon[e] = level < a.lv.active_levels;
-	}
+		for (int j = 0; j < 8; ++j) {
+			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
+			// (levels that have no row read that of the first level that does and are replaced, or meet weights of zero)
+			const uint32_t lr = level < a.first_level || 2u * level >= a.enc_w ? a.first_level : level;
+			ahead[j] = query_rows(a)[(size_t)lr * N + col];
+		}
+	};
+	if constexpr (BLOCKS) fetch_rows(min(wave, n_tiles - 1u));
 	__syncthreads();
 	for (uint32_t tile = wave; tile < n_tiles; tile += n_waves) {
 		const uint32_t col_raw = tile * 32u + n;
@@ -677,32 +687,29 @@ __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const Fu
 		const uint32_t col = valid ? col_raw : N - 1u;
 		const float p[3] = {next[0], next[1], next[2]};
 		half8 xs[3];
+		if constexpr (!BLOCKS) fetch_rows(tile);
 #pragma unroll
 		for (int j = 0; j < 8; ++j) {
-			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
-			// (levels that have no rows read those of the first level that does and are replaced, or meet weights of zero)
-			const uint32_t lr = level < a.first_level || 2u * level >= a.enc_w ? a.first_level : level;
-			xs[j >> 2][2 * (j & 3)] = a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
-			xs[j >> 2][2 * (j & 3) + 1] = a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
+			const half2v f = __builtin_bit_cast(half2v, ahead[j]);
+			xs[j >> 2][2 * (j & 3)] = f[0];
+			xs[j >> 2][2 * (j & 3) + 1] = f[1];
 		}
-		// the levels from blocks: lower lanes 4, upper ones 2 and 3, where the network's operands have them
-		constexpr uint32_t ITEMS = BLOCKS ? 2 : 0;
-		float bw[ITEMS + 1][3];
-		uint32_t braw[ITEMS + 1][2][4];
-#pragma unroll
-		for (uint32_t e = 0; e < ITEMS; ++e) {
+		float bw[3], cw[3];
+		uint32_t braw[2][4], craw[4];
+		if constexpr (BLOCKS) {
 			uint32_t c[3];
 #pragma unroll
-			for (int d = 0; d < 3; ++d) n2_locate(p[d], bscale[e], bw[e][d], c[d]);
-			const N2Block* const row = bfrom[e] + n2_block_row(bres[e], c[1], c[2]);
+			for (int d = 0; d < 3; ++d) n2_locate(p[d], bscale, bw[d], c[d]);
+			const N2Block* const row = bfrom + n2_block_row(bres, c[1], c[2]);
+			const N2Block v0 = row[min(c[0], bres)], v1 = row[min(c[0] + 1u, bres)];
 #pragma unroll
-			for (uint32_t b = 0; b < 2; ++b) {
-				const N2Block v = row[min(c[0] + b, bres[e])];
+			for (int d = 0; d < 3; ++d) n2_locate(p[d], cscale, cw[d], c[d]);
+			const N2Block v2 = (cfrom + n2_block_row(cres, c[1], c[2]))[min(c[0] + (uint32_t)g, cres)];
 #pragma unroll
-				for (int q = 0; q < 4; ++q) braw[e][b][q] = v.entry[q];
-			}
+			for (int q = 0; q < 4; ++q) { braw[0][q] = v0.entry[q]; braw[1][q] = v1.entry[q]; craw[q] = v2.entry[q]; }
 		}
 		position(tile + n_waves < n_tiles ? tile + n_waves : tile, next);
+		if constexpr (BLOCKS) fetch_rows(tile + n_waves < n_tiles ? tile + n_waves : tile);
 		xs[2] = zero8();
 		if (g == 0) {
 #pragma unroll
@@ -720,11 +727,16 @@ __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const Fu
 #pragma unroll
 			for (int k = 0; k < 4; ++k) raw[b][k] = *reinterpret_cast<const uint32_t*>(table + at[k]);
 		}
-		const uint32_t own = on ? staged_feature(w, raw) : 0u, other = (uint32_t)__shfl_xor((int)own, 32);
+		const uint32_t own = on ? staged_feature(w[0], staged_corner(w, raw[0]), staged_corner(w, raw[1])) : 0u, other = (uint32_t)__shfl_xor((int)own, 32);
 		uint32_t x4[4] = {0u, 0u, 0u, 0u};
 		*reinterpret_cast<half8*>(x4) = xs[0];
 		if constexpr (BLOCKS) {
-			const uint32_t b0 = bon[0] ? staged_feature(bw[0], braw[0]) : 0u, b1 = bon[1] ? staged_feature(bw[1], braw[1]) : 0u;
+			const uint32_t b0 = bon ? staged_feature(bw[0], staged_corner(bw, braw[0]), staged_corner(bw, braw[1])) : 0u;
+			const float2 mine = staged_corner(cw, craw);
+			float2 lo, hi;
+			staged_halves(mine.x, lo.x, hi.x);
+			staged_halves(mine.y, lo.y, hi.y);
+			const uint32_t b1 = con ? staged_feature(cw[0], lo, hi) : 0u;
 			x4[0] = g ? b0 : own;
 			x4[1] = g ? b1 : other;
 			x4[2] = g ? x4[2] : b0;
@@ -838,8 +850,11 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) field_fused_forward_kernel(const 
 				const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
 				// levels the grid does not have read level 0's rows and are ignored (their weights are zero)
 				const uint32_t lr = 2u * level < a.enc_w ? level : 0u;
-				xs[j >> 2][2 * (j & 3)] = FULL ? next.feat[2 * j] : a.sdf_in[(size_t)(3 + 2 * lr) * N + col];
-				xs[j >> 2][2 * (j & 3) + 1] = FULL ? next.feat[2 * j + 1] : a.sdf_in[(size_t)(4 + 2 * lr) * N + col];
+				half2v f;
+				if (FULL) f = half2v{next.feat[2 * j], next.feat[2 * j + 1]};
+				else f = __builtin_bit_cast(half2v, query_rows(a)[(size_t)lr * N + col]);
+				xs[j >> 2][2 * (j & 3)] = f[0];
+				xs[j >> 2][2 * (j & 3) + 1] = f[1];
 				if (FULL) slope[j] = a.slopes[(size_t)lr * N + col];
 			}
 		}
@@ -1003,13 +1018,13 @@ static void launch_gather(const FusedArgs& a, hipStream_t s) {
 // 5000 points: 1000 9.4 | 7.2, 8192 11.7 | 9.7.)
 constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 256 * FQ_POINTS;
 // From here on the two coarsest levels are the network kernel's (field_staged_forward_kernel): its start, two tables to every CU, costs smaller queries more than their
-// two levels.  (Call in us, gathered | staged, uniform points: 32 768 18.2 | 20.9, 65 536 28.6 | 29.3, 98 304 38.7 | 37.0, 2^17 50.4 | 46.9, 2^18 86.6 | 79.4, 2^20 294 | 279,
-// 2^21 567 | 532; along rays 65 536 20.2 | 21.7, 98 304 26.6 | 27.6, 2^17 34.0 | 34.4, 2^18 58.2 | 57.0, 2^20 187 | 185; on a lattice 2^17 32.8 | 33.0, 2^20 144.3 | 142.4.  Updates of
-// the occupancy grid: 2^17 samples 67.5 | 65.0, 2^20 254 | 248, 2^21 427 | 419, 700 000 266 | 252.)
-constexpr uint32_t QUERY_STAGED_MIN = 1u << 17;
-// ... and from here on three more come from blocks: making these costs smaller queries what they save.  (Call in us, staged | with blocks: uniform points 2^17 46.8 | 46.5, 2^18
-// 79.3 | 74.9, 2^19 149 | 140, 2^20 279 | 260, 2^21 533 | 495; along rays 33.6 | 36.0, 57.3 | 58.0, 101 | 99, 184 | 178, 344 | 331; on a lattice 32.6 | 34.7, 56.4 | 56.9, 79.1 | 78.1,
-// 142.5 | 136.1, 261 | 251.  Updates of the occupancy grid: 2^19 samples 161.6 | 155.7, 700 000 252 | 239, 2^21 418 | 403.)
+// two levels.  (Call in us, gathered | staged, uniform points: 32 768 18.3 | 20.5, 65 536 28.7 | 28.7, 98 304 39.1 | 36.4, 2^17 49.1 | 44.2, 2^18 87.2 | 77.7, 2^20 292 | 278,
+// 2^21 566 | 531; along rays 65 536 20.3 | 21.2, 98 304 26.5 | 26.8, 2^17 33.7 | 32.1, 2^20 184 | 182; on a lattice 65 536 19.6 | 20.0, 98 304 26.1 | 25.7, 2^20 142 | 141.  Updates of
+// the occupancy grid: 2^17 samples 67.5 | 64.0, 700 000 264 | 250, 2^20 252 | 245, 2^21 421 | 415.)
+constexpr uint32_t QUERY_STAGED_MIN = 3u << 15;
+// ... and from here on three more come from blocks: making these costs smaller queries what they save.  (Call in us, staged | with blocks, uniform points: 98 304 36.4 | 37.3, 2^17
+// 44.2 | 43.9, 2^18 77.7 | 73.3, 2^19 148 | 136, 2^20 278 | 250, 2^21 531 | 480; along rays 2^17 32.1 | 35.2, 2^18 56.1 | 57.8, 2^19 99.0 | 98.2, 2^20 182 | 177; on a lattice 2^17
+// 31.4 | 34.4, 2^18 55.1 | 56.5, 2^19 77.2 | 77.6, 2^20 141 | 136.  Updates of the occupancy grid: 2^19 samples 160.4 | 157.2, 700 000 250 | 231, 2^20 245 | 236, 2^21 415 | 400.)
 constexpr uint32_t QUERY_BLOCKS_MIN = 1u << 18;
 
 // ----------------------------------------------------------------------------

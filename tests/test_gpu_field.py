@@ -171,7 +171,7 @@ def test_small_batches_equal_the_same_samples_in_a_large_one(n, active):
 # the last batch whose levels are all gathered and the first whose two coarsest are the network kernel's, the last and first with three more from blocks; tiles of 32 samples that are
 # not whole; as few levels as that takes, and fewer; levels switched off, of these as well; tables that fill an LDS with the fragments and such that do not (base resolutions 24 and 32);
 # a fifth level that is hashed, all of them but one
-@pytest.mark.parametrize("n,cfg,active", [((1 << 17) - 8, {}, 1.0), (1 << 17, {}, 1.0), ((1 << 17) + 8, {}, 1.0), ((1 << 18) - 8, {}, 1.0), (1 << 18, {}, 1.0), ((1 << 18) + 8, {}, 1.0), (700008, {}, 1.0),
+@pytest.mark.parametrize("n,cfg,active", [((3 << 15) - 8, {}, 1.0), (3 << 15, {}, 1.0), ((3 << 15) + 8, {}, 1.0), ((1 << 18) - 8, {}, 1.0), (1 << 18, {}, 1.0), ((1 << 18) + 8, {}, 1.0), (700008, {}, 1.0),
                                           ((1 << 17) + 24, dict(n_levels=3), 1.0), ((1 << 17) + 24, dict(n_levels=2), 1.0), ((1 << 18) + 24, dict(n_levels=6), 1.0), ((1 << 18) + 24, dict(n_levels=5), 1.0),
                                           ((1 << 18) + 24, {}, 0.25), ((1 << 18) + 24, {}, 0.1875), ((1 << 18) + 24, {}, 0.125), ((1 << 18) + 24, {}, 0.0625), ((1 << 17) + 24, {}, 0.0625), ((1 << 18) + 24, {}, 0.0),
                                           ((1 << 18) + 24, dict(base_resolution=24, per_level_scale=1.1), 1.0), ((1 << 18) + 24, dict(base_resolution=32), 1.0),
