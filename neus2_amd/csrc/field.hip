@@ -839,6 +839,32 @@ N2_API uint64_t n2_sdf_step_workspace_bytes(uint32_t n) {
 	return std::max<uint64_t>(n2_sdf_eikonal_workspace_bytes(n), 4ull * n2_fused_sdf_eikonal_parts(n));
 }
 
+// the rows of three matrices that stay zero, in one launch: a caller's first step waits for it
+struct SdfPadding {
+	uint4* at[3];
+	uint32_t n[3];  // in 16 bytes
+};
+__global__ void __launch_bounds__(256) sdf_clear_padding_kernel(const SdfPadding pad) {
+#pragma unroll
+	for (int k = 0; k < 3; ++k)
+		for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < pad.n[k]; i += gridDim.x * 256u) pad.at[k][i] = make_uint4(0u, 0u, 0u, 0u);
+}
+N2_API int n2_sdf_clear_padding(n2_stream_t stream, uint32_t n, uint32_t encoding_width, uint32_t input_width, const n2_sdf_buffers* b) {
+	const char* fn = "n2_sdf_clear_padding";
+	N2_REQUIRE(b != nullptr && b->input && b->second_order_input && b->dL_doutput, "%s: null buffer", fn);
+	N2_REQUIRE(n > 0 && n % 8 == 0 && n <= (1u << 28), "%s: batch size %u is not a multiple of 8 up to 2^28", fn, n);
+	N2_REQUIRE(input_width >= 3 + encoding_width && input_width <= 64, "%s: input width %u does not hold 3 + %u rows", fn, input_width, encoding_width);
+	const uintptr_t all = reinterpret_cast<uintptr_t>(b->input) | reinterpret_cast<uintptr_t>(b->second_order_input) | reinterpret_cast<uintptr_t>(b->dL_doutput);
+	N2_REQUIRE(all % 16 == 0, "%s: buffers must be 16-byte aligned", fn);
+	const uint32_t used = 3 + encoding_width, rows = input_width - used;
+	const SdfPadding pad = {{reinterpret_cast<uint4*>(b->input + (size_t)used * n), reinterpret_cast<uint4*>(b->second_order_input + (size_t)used * n),
+	                         reinterpret_cast<uint4*>(b->dL_doutput + n)}, {rows * (n / 8), rows * (n / 8), 15u * (n / 8)}};
+	const uint32_t blocks = (15u * (n / 8) + 255) / 256;
+	sdf_clear_padding_kernel<<<dim3(blocks < 2048u ? blocks : 2048u), dim3(256), 0, n2_stream(stream)>>>(pad);
+	N2_LAUNCH_CHECK();
+	return N2_OK;
+}
+
 static int check_sdf_step(const char* fn, const n2_grid_t* grid, const n2_mlp_t* mlp, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n,
                           const n2_sdf_buffers* b, uint32_t& enc_w, uint32_t& in_w) {
 	N2_REQUIRE(grid != nullptr && mlp != nullptr && b != nullptr && d_xyz != nullptr, "%s: null argument", fn);

@@ -36,12 +36,12 @@ class SdfNet:
         if n != self._n:
             h = lambda rows: torch.empty((rows, n), dtype=torch.float16, device=device)
             f = lambda rows: torch.empty((rows, n), dtype=torch.float32, device=device)
-            z = lambda rows: torch.zeros((rows, n), dtype=torch.float16, device=device)  # rows that stay zero: the inputs' padding, the outputs without a loss
             nb = int(capi.lib().n2_sdf_step_workspace_bytes(C.c_uint32(n)))
-            b = dict(input=z(self.in_w), dy_dx=torch.empty((self.enc_w, n, 3), dtype=torch.float32, device=device), output=h(16), dsdf_dinput=h(self.in_w), normal=f(3),
-                     dL_doutput=z(16), dL_dnormal=f(3), second_order_input=z(self.in_w), dL_dinput=h(self.in_w),
+            b = dict(input=h(self.in_w), dy_dx=torch.empty((self.enc_w, n, 3), dtype=torch.float32, device=device), output=h(16), dsdf_dinput=h(self.in_w), normal=f(3),
+                     dL_doutput=h(16), dL_dnormal=f(3), second_order_input=h(self.in_w), dL_dinput=h(self.in_w),
                      loss=torch.empty(1, dtype=torch.float32, device=device), workspace=torch.empty(nb, dtype=torch.uint8, device=device))
             self._b = (capi.SdfBuffers(workspace_bytes=nb, **{k: t.data_ptr() for k, t in b.items()}), b)
+            check(capi.lib().n2_sdf_clear_padding(_stream(), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), C.byref(self._b[0])), "n2_sdf_clear_padding")
             self._n = n
         return self._b
 

@@ -135,3 +135,14 @@ def test_step_errors():
         net.forward(torch.rand((3, 12), device="cuda"))
     with pytest.raises(N2Error, match="set_params"):
         net.forward(torch.rand((3, 16), device="cuda"))
+
+
+@pytest.mark.parametrize("n,enc_w,in_w", [(8, 32, 48), (1000, 32, 48), (264, 13, 16), (72, 40, 48)])  # thirteen rows of padding, none, five; the smallest batch
+def test_padding_is_cleared_and_nothing_else(n, enc_w, in_w):
+    import ctypes as C
+    from neus2_amd import capi
+    b = {k: torch.full((rows, n), float("nan"), dtype=torch.float16, device="cuda") for k, rows in (("input", in_w), ("second_order_input", in_w), ("dL_doutput", 16))}
+    own = capi.SdfBuffers(**{k: t.data_ptr() for k, t in b.items()})
+    capi.check(capi.lib().n2_sdf_clear_padding(None, C.c_uint32(n), C.c_uint32(enc_w), C.c_uint32(in_w), C.byref(own)), "n2_sdf_clear_padding")
+    for k, used in (("input", 3 + enc_w), ("second_order_input", 3 + enc_w), ("dL_doutput", 1)):
+        assert bool(torch.isnan(b[k][:used]).all()) and bool((b[k][used:] == 0).all()), k
