@@ -700,22 +700,14 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 				// planes per wave: 16 where that leaves every SIMD several waves (a wave's start costs as much as two steps), fewer on
 				// small lattices; the slab's planes in equal shares
 				const uint64_t runs = (uint64_t)a.x_runs * a.ny * a.nz;
-				const uint32_t most = runs >= 16u * 4096u ? 16u : runs <= 4u * 4096u ? 4u : (uint32_t)(runs / 4096u);
-				auto share = [&](uint32_t planes) {
-					const uint32_t parts = (a.nz + planes - 1u) / planes;
-					a.walk = (a.nz + parts - 1u) / parts;
-					const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk);
-					return (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
-				};
+				const uint32_t most = runs >= 16u * 4096u ? 16u : runs <= 4u * 4096u ? 4u : (uint32_t)(runs / 4096u), parts = (a.nz + most - 1u) / most;
+				a.walk = (a.nz + parts - 1u) / parts;
+				const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk), blocks = (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
 				if (n_fine) {
-					// (a wave of the fine kernel keeps nothing from step to step, starts cheaply, and shorter ones leave less of the chip idle at a slab's end:
-					// 5 | 6 | 8 | 10 | 16 planes at most 512^3 4839 | 4802 | 4758 | 4797 | 4807 us, 400^3 2969 | 2921 | 2904 | 2893 | 2925, 256^3 891 | 887 | 884 | 886 | 889, 208^3 587 | 586 | 582 | 586 | 592)
-					const uint32_t blocks = share(most < 8u ? most : 8u);
 					const bool first = x0 == 0 && y0 == 0 && z0 == 0;
 					lattice_fine_kernel<<<dim3(blocks * n_fine + (first ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks);
 					N2_LAUNCH_CHECK();
 				}
-				const uint32_t blocks = share(most);
 				walk_kernel<<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
 				N2_LAUNCH_CHECK();
 			}
