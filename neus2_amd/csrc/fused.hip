@@ -1060,7 +1060,7 @@ __global__ void __launch_bounds__(FF_BLOCK, 2) sdf_eikonal_forward_kernel(const 
 	const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
 	const uint32_t N = a.N, n_tiles = (N + 31u) / 32u;
 	const uint32_t wave_gid = blockIdx.x * (FF_BLOCK / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (FF_BLOCK / 64);
-	// Of a matrix [rows][N], row u + 4 g of the lane's point: the row u stands in a scalar address, the rest in a 32-bit lane offset.
+	// Of a matrix [rows][N], row u + 4 g of the lane's point: the row u stands in a scalar address, the rest in a 32-bit lane offset (n2_sdf_one_pass: 60 N - 12 bytes at most).
 	auto at = [&](auto* matrix, uint32_t u, uint32_t lane_at, uint32_t width) __attribute__((always_inline)) {
 		typedef typename std::conditional<std::is_const<std::remove_pointer_t<decltype(matrix)>>::value, const char, char>::type bytes;
 		typedef std::remove_pointer_t<decltype(matrix)> value;
@@ -1318,6 +1318,7 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 uint32_t n2_fused_sdf_eikonal_parts(uint32_t n) { return fused_grid(n); }
 int n2_fused_sdf_eikonal(hipStream_t s, const n2_half* weights, uint32_t n, const n2_half* input, const float* dy_dx, n2_half* output, n2_half* dsdf, float* normal,
                          float ek_weight, float scale, n2_half* dL_dy, float* v, n2_half* v_in, float* parts) {
+	N2_REQUIRE(n2_sdf_one_pass(n), "n2_fused_sdf_eikonal: %u points are beyond the lanes' 32-bit offsets", n);
 	SdfEikonalArgs a{};
 	a.weights = reinterpret_cast<const hf*>(weights);
 	a.N = n;

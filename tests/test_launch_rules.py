@@ -33,6 +33,7 @@ extern "C" uint32_t row_levels(const float* scale, uint32_t nx, float step_x, fl
 extern "C" int by_rows(uint32_t rows, uint32_t walked, uint64_t points) { return n2_lattice_by_rows(rows, walked, points); }
 extern "C" uint32_t bin_points_per_thread(uint32_t levels, uint32_t n) { return n2_bin_points_per_thread(levels, n, 512); }
 extern "C" uint32_t bin_single_points(uint32_t levels) { return n2_bin_single_points(levels, 512); }
+extern "C" int sdf_one_pass(uint32_t n) { return n2_sdf_one_pass(n); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
 
@@ -153,3 +154,9 @@ def test_one_point_per_thread_while_all_sorting_workgroups_run_at_once(rules, le
     line = rules.bin_single_points(C.c_uint32(levels))
     assert levels * (line // 512) <= 768 < levels * (line // 512 + 1) and line % 512 == 0
     assert [rules.bin_points_per_thread(C.c_uint32(levels), C.c_uint32(n)) for n in (1, line, line + 1, 1 << 31)] == [1, 1, 2, 2]
+
+
+@pytest.mark.parametrize("n,fits", [(8, 1), (1 << 18, 1), (1 << 26, 1), (71582784, 1), (71582792, 0), (1 << 27, 0), (1 << 28, 0)])
+def test_one_pass_of_the_sdf_network_while_its_offsets_fit_32_bits(rules, n, fits):
+    """The last lane's place in the Jacobian: row 4 of its scalar base, the last point, three floats each."""
+    assert rules.sdf_one_pass(C.c_uint32(n)) == fits == ((4 * n + n - 1) * 12 + 11 < 1 << 32)
