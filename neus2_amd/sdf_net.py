@@ -41,8 +41,11 @@ class SdfNet:
                      dL_doutput=h(16), dL_dnormal=f(3), second_order_input=h(self.in_w), dL_dinput=h(self.in_w),
                      loss=torch.empty(1, dtype=torch.float32, device=device), workspace=torch.empty(nb, dtype=torch.uint8, device=device))
             self._b = (capi.SdfBuffers(workspace_bytes=nb, **{k: t.data_ptr() for k, t in b.items()}), b)
+            self._n, self._cleared = n, False
+        if not self._cleared:
             check(capi.lib().n2_sdf_clear_padding(_stream(), C.c_uint32(n), C.c_uint32(self.enc_w), C.c_uint32(self.in_w), C.byref(self._b[0])), "n2_sdf_clear_padding")
-            self._n = n
+            # (under capture the clearing has only become part of the graph: a call outside it may come before the first replay)
+            self._cleared = not torch.cuda.is_current_stream_capturing()
         return self._b
 
     def forward(self, x, ek_weight=0.1, loss_scale=128.0):

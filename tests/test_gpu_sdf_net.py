@@ -153,6 +153,46 @@ def test_points_beyond_the_one_pass_kernels_offsets():
     torch.cuda.empty_cache()
 
 
+def test_a_batch_size_first_met_under_capture():
+    """The captured step clears the padding of its buffers when it is replayed; a step outside the graph comes first and has to clear it for itself."""
+    from neus2_amd.sdf_net import SdfNet
+    n = 1000
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    net = SdfNet(16, 14, 16, 1.3, max_batch=n)
+    P = (torch.randn(net.grid.n_params(), device="cuda", generator=gen) * 0.01).half()
+    W = (torch.randn(net.mlp.n_params(), device="cuda", generator=gen) * 0.15).half()
+    gP, gW = torch.zeros_like(P), torch.zeros_like(W)
+    net.set_params(P, gP, W, gW)
+    x = torch.rand((3, n), device="cuda", generator=gen)
+    def outputs(ctx):
+        return [t.clone() for t in (ctx["y"], ctx["g"], ctx["normal"], ctx["loss"], gP, gW)]
+    ctx = net.forward(x)
+    net.loss_backward(ctx)
+    want = outputs(ctx)
+    net.forward(x[:, :8].contiguous())  # the next forward of n points has buffers of its own
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        for _ in range(2):
+            ctx = net.forward(x)
+            net.loss_backward(ctx)
+    torch.cuda.synchronize()
+    own = ctx["buffers"][1]
+    for k in ("input", "dL_doutput", "second_order_input"):
+        own[k].fill_(float("nan"))  # what memory that nothing has written may hold
+    ctx = net.forward(x)
+    net.loss_backward(ctx)
+    assert ctx["buffers"][1] is own
+    assert all(torch.equal(a, b) for a, b in zip(outputs(ctx), want))
+    for _ in range(3):
+        own["normal"].zero_()
+        gP.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outputs(ctx), want))
+
+
 def test_step_errors():
     from neus2_amd.sdf_net import SdfNet
     from neus2_amd.tcnn_api import N2Error
