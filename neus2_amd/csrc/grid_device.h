@@ -201,7 +201,15 @@ __device__ __forceinline__ void n2_encode_level(const char* __restrict__ base, u
 //   word 0: q0 | q1 << 20     word 1: q1 >> 12 | q2 << 8 | q3 << 28     word 2: q3 >> 4 | q4 << 16
 //   word 3: q4 >> 16 | q5 << 4 | e << 24
 // ----------------------------------------------------------------------------
-__device__ __forceinline__ uint4 n2_slopes_pack(const float (&v)[6]) {
+__device__ __forceinline__ uint4 n2_slopes_pack(const float (&slopes)[6]) {
+	float v[6];
+#pragma unroll
+	for (int i = 0; i < 6; ++i) v[i] = slopes[i];
+	// A slope that is no number counts as zero (the bounds below would make the lowest mantissa of it), an infinite one as the largest there is.
+	if (__builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3]) || __builtin_isunordered(v[4], v[5])) {
+#pragma unroll
+		for (int i = 0; i < 6; ++i) v[i] = __builtin_isnan(v[i]) ? 0.f : v[i];
+	}
 	float m = 0.f;
 #pragma unroll
 	for (int i = 0; i < 6; ++i) m = fmaxf(m, fabsf(v[i]));

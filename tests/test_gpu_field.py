@@ -332,3 +332,29 @@ def test_direction_encoding_rows(oracle):
     # rows 0..2 and 11..15 of the output are the colour net's own rows (3..10 are overwritten by sdf, normal, ...)
     for r in (0, 1, 2, 11, 12, 13, 14, 15):
         assert_close(out[r], q16(sh[r]), rtol=RTOL, what=f"SH row {r}", scale=1.0)
+
+
+@pytest.mark.parametrize("infinite", ["all", "even_x"])
+def test_slopes_that_are_no_numbers_count_as_zero(oracle, infinite):
+    """Infinite entries of one level and feature: differences of two of them are no numbers and add nothing to the normal; a difference to a finite
+    entry is the largest slope a block holds, (2^19 - 1) 2^-19 of the level's scale where it is the block's own exponent."""
+    of, gf, p, dp, dg, rng = make(oracle, seed=12, log2_hashmap_size=14)
+    n, w = 512, of.sdf_in_w
+    coords = rand_coords(rng, n)
+    coords[:, :3] = 0.1 + 0.8 * coords[:, :3]
+    W0, Wo = p[:64 * w].reshape(64, w), p[64 * w:of.off_rgb].reshape(16, 64)
+    W0[:, 3] = q16(np.where(rng.random(64) < 0.5, -1, 1) * (0.1 + rng.random(64)))  # the sign alone decides about a neuron
+    res, off = int(of.grid.resolution[0]), of.off_grid + 2 * int(of.grid.offset[0])
+    level = p[off:off + 2 * int(of.grid.entries[0])].reshape(-1, 2)
+    level[:, 0] = 0
+    J = of.grid.forward(p[of.off_grid:of.off_var], np.ascontiguousarray(coords[:, :3].T), want_dy_dx=True)[1].astype(np.float64)
+    assert not J[0].any()
+    level[:, 0] = np.where((np.arange(len(level)) % res % 2 == 0) | (infinite == "all"), np.inf, 0.25)
+    if infinite == "even_x":
+        cell = np.floor(coords[:, 0] * of.grid.scale[0] + np.float32(0.5)).astype(int)
+        J[0, :, 0] = np.where(cell % 2 == 0, -1, 1) * (2 ** 19 - 1) / 2 ** 19 * float(of.grid.scale[0])
+    g = q16(W0.T.astype(np.float64) @ (Wo[0].astype(np.float64) * (W0[:, 3] > 0)))
+    want = np.einsum("k,knd->dn", g[3:3 + of.enc_w].astype(np.float64), J) + g[:3, None]
+    dp.copy_(dev(p, torch.float16))
+    got = host(gf.forward(dev(coords))).T[4:7]
+    assert_close(got, want.astype(np.float32), what="normal")
