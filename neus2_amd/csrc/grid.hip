@@ -733,7 +733,7 @@ template <bool STREAM>
 struct N2RideInput {
 	const float* dy_dx;
 	float* dL_dx;
-	uint32_t n_out, blocks, every;
+	uint32_t n_out, every;
 };
 // The networks' weight-gradient slabs, two units to a workgroup, in the first workgroups: the field's forward and backward on 2^18 samples
 // 251.0 -> 247.9 us, on 52 344 94.8 -> 91.6, on 2048 47.6 -> 41.3.
@@ -791,29 +791,29 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 	__shared__ __align__(16) uint16_t stage_key[bin_records(PER)];  // ... and entry within its bucket
 	uint32_t block = blockIdx.x;
 	if constexpr (RIDES_INPUT<Ride>) {
-		const uint32_t q = block / (ride.every + 1u), m = block - q * (ride.every + 1u);
-		if (m == ride.every) {
+		bool rides;
+		block = n2_turn(block, ride.every, 1u, rides);
+		if (rides) {
 			const auto point = [&](auto stream) {
-				grid_backward_input_point<decltype(stream)::value>(q * BIN_BLOCK + threadIdx.x, N, ride.n_out, dL_dy, ride.dy_dx, ride.dL_dx);
+				grid_backward_input_point<decltype(stream)::value>(block * BIN_BLOCK + threadIdx.x, N, ride.n_out, dL_dy, ride.dy_dx, ride.dL_dx);
 			};
 			point(std::bool_constant<std::is_same<Ride, N2RideInput<true>>::value>());
 			return;
 		}
-		block = q * ride.every + m;
 		if (block >= tiles * tab.n_levels) return;
 	} else if constexpr (std::is_same<Ride, N2RideSecond>::value) {
-		const uint32_t group = block / N_XCD, lane = block - group * N_XCD, q = group / (ride.every + 1u), m = group - q * (ride.every + 1u);
-		if (m < ride.every) {
-			const uint32_t item = (q * ride.every + m) * N_XCD + lane, y = ride.height == 1u ? 0u : item / ride.tiles;
+		bool sorts;
+		block = n2_turn(block + blockIdx.y * gridDim.x, ride.every, N_XCD, sorts);
+		if (!sorts) {
+			const uint32_t y = ride.height == 1u ? 0u : block / ride.tiles;
 			uint32_t level, tile;
-			if (item >= ride.blocks || !n2_gather_item(item - y * ride.tiles, y, ride.height, tab.n_levels, ride.tiles, level, tile)) return;
+			if (block >= ride.blocks || !n2_gather_item(block - y * ride.tiles, y, ride.height, tab.n_levels, ride.tiles, level, tile)) return;
 			const uint32_t i = tile * BIN_BLOCK + threadIdx.x;
 #define CALL(M) grid_second_item<M>(tab, level, i, N, xyz, point_stride, dim_stride, params, v, ride.dL_ddLdy)
 			N2_DISPATCH_MODE(tab.mode[level], CALL)
 #undef CALL
 			return;
 		}
-		block = q * N_XCD + lane;
 		if (block >= tiles * tab.n_levels) return;
 	} else if constexpr (std::is_same<Ride, N2RideSums>::value) {
 		if (block < ride.blocks) {
@@ -1645,24 +1645,30 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.split_begin[l] = split;
 	auto bin = [&](auto per_thread) {
 		constexpr uint32_t PER = decltype(per_thread)::value;
-#define LAUNCH(F, S, RIDE, BLOCKS) grid_bin_kernel<PER, F, S><<<dim3(BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
-                                                                                          grid->params, rec_vals, rec_keys, offsets, index, n_cols, RIDE)
+		// (the other launches' records exceed the card's memory before their threads exceed 32 bits: 8 and 9 threads a point of sixteen levels)
+		const auto launch_dim = [](auto ride, uint32_t blocks) {
+			if (!std::is_same<decltype(ride), N2RideSecond>::value) return dim3(blocks);
+			const N2GatherGrid g = n2_rows_of_blocks(blocks, BIN_BLOCK);
+			return dim3(g.x, g.y);
+		};
+#define LAUNCH(F, S, RIDE, BLOCKS) grid_bin_kernel<PER, F, S><<<launch_dim(RIDE, BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
+                                                                                                    grid->params, rec_vals, rec_keys, offsets, index, n_cols, RIDE)
 		const uint32_t blocks = tiles * L;
 		const N2RideNone none;
 		if (rider.dL_dx != nullptr) {  // (first order alone)
-			const uint32_t riders = (n_points + BIN_BLOCK - 1) / BIN_BLOCK, every = (blocks + riders - 1) / riders, rows = L * grid->n_features;
-			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
-			else LAUNCH(true, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, riders, every}), riders * (every + 1));
+			const N2Turns turns = n2_turns(blocks, (n_points + BIN_BLOCK - 1) / BIN_BLOCK, 1u);
+			const uint32_t rows = L * grid->n_features;
+			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, turns.every}), turns.blocks);
+			else LAUNCH(true, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, turns.every}), turns.blocks);
 		} else if (rider.sums.units > 0) {  // (both orders)
 			const uint32_t riders = (rider.sums.units + BIN_BLOCK / 256 - 1) / (BIN_BLOCK / 256);
 			LAUNCH(true, true, (N2RideSums{rider.sums, riders}), riders + blocks);
 		} else if (out) {
 			const N2GatherGrid g = n2_gather_grid(N2_ENCODING_XCD_MAX, n_points, L, BIN_BLOCK);
-			const uint32_t gather = g.x * g.y, every = (gather + blocks - 1) / blocks, sort_groups = (blocks + N_XCD - 1) / N_XCD;
-			const uint32_t gather_groups = (gather + N_XCD * every - 1) / (N_XCD * every), groups = std::max(sort_groups, gather_groups) * (every + 1);
-			const N2RideSecond ride{dL_ddLdy, gather, every, (n_points + BIN_BLOCK - 1) / BIN_BLOCK, g.y};
-			if (first) LAUNCH(true, true, ride, groups * N_XCD);
-			else LAUNCH(false, true, ride, groups * N_XCD);
+			const N2Turns turns = n2_turns(g.x * g.y, blocks, N_XCD);
+			const N2RideSecond ride{dL_ddLdy, g.x * g.y, turns.every, (n_points + BIN_BLOCK - 1) / BIN_BLOCK, g.y};
+			if (first) LAUNCH(true, true, ride, turns.blocks);
+			else LAUNCH(false, true, ride, turns.blocks);
 		} else if (first && second) LAUNCH(true, true, none, blocks);
 		else if (second) LAUNCH(false, true, none, blocks);
 		else LAUNCH(true, false, none, blocks);

@@ -146,3 +146,28 @@ N2_HD inline bool n2_gather_item(uint32_t x, uint32_t y, uint32_t height, uint32
 	tile = x;
 	return true;
 }
+
+// A launch of two kinds of work in turn: `every` groups of workgroups of the first kind, then one group of the second, each `group` workgroups long.
+struct N2Turns {
+	uint32_t every, blocks;
+};
+static inline N2Turns n2_turns(uint32_t first, uint32_t second, uint32_t group) {
+	const uint32_t every = (first + second - 1u) / second, a = (first + every * group - 1u) / (every * group), b = (second + group - 1u) / group;
+	return {every, (a > b ? a : b) * (every + 1u) * group};
+}
+// The number of a workgroup among those of its kind, which may be past the last one.
+N2_HD inline uint32_t n2_turn(uint32_t block, uint32_t every, uint32_t group, bool& second) {
+	const uint32_t g = block / group, lane = block - g * group, q = g / (every + 1u), m = g - q * (every + 1u);
+	second = m == every;
+	return (second ? q : q * every + m) * group + lane;
+}
+
+// Workgroups beyond what a launch can count along x (2^32 - 1 threads) go into further rows in y, numbered through: row by row, each a multiple of the
+// XCDs long, so that a number keeps its XCD.  The last ones may be past `blocks`.  (With the second order's output gathered beside it the sorting launch
+// has 24 threads a point of sixteen levels: 2^28 points and less than 2^32 / 24 do not go together.)
+static inline N2GatherGrid n2_rows_of_blocks(uint32_t blocks, uint32_t threads) {
+	const uint32_t most = 0xFFFFFFFFu / threads / N2_XCDS * N2_XCDS;
+	if (blocks <= most) return {blocks, 1u};
+	const uint32_t y = blocks / most + (blocks % most != 0u), x = blocks / y + (blocks % y != 0u);
+	return {(x + N2_XCDS - 1u) / N2_XCDS * N2_XCDS, y};
+}

@@ -33,6 +33,21 @@ extern "C" uint32_t row_levels(const float* scale, uint32_t nx, float step_x, fl
 extern "C" int by_rows(uint32_t rows, uint32_t walked, uint64_t points) { return n2_lattice_by_rows(rows, walked, points); }
 extern "C" uint32_t bin_points_per_thread(uint32_t levels, uint32_t n) { return n2_bin_points_per_thread(levels, n, 512); }
 extern "C" uint32_t bin_single_points(uint32_t levels) { return n2_bin_single_points(levels, 512); }
+extern "C" uint32_t turns(uint32_t first, uint32_t second, uint32_t group, uint32_t* blocks) {
+	const N2Turns t = n2_turns(first, second, group);
+	*blocks = t.blocks;
+	return t.every;
+}
+extern "C" uint32_t turn(uint32_t block, uint32_t every, uint32_t group, uint32_t* second) {
+	bool s;
+	const uint32_t at = n2_turn(block, every, group, s);
+	*second = s;
+	return at;
+}
+extern "C" void rows_of_blocks(uint32_t blocks, uint32_t threads, uint32_t* out) {
+	const N2GatherGrid g = n2_rows_of_blocks(blocks, threads);
+	out[0] = g.x; out[1] = g.y;
+}
 extern "C" int sdf_one_pass(uint32_t n) { return n2_sdf_one_pass(n); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
@@ -160,3 +175,28 @@ def test_one_point_per_thread_while_all_sorting_workgroups_run_at_once(rules, le
 def test_one_pass_of_the_sdf_network_while_its_offsets_fit_32_bits(rules, n, fits):
     """The last lane's place in the Jacobian: row 4 of its scalar base, the last point, three floats each."""
     assert rules.sdf_one_pass(C.c_uint32(n)) == fits == ((4 * n + n - 1) * 12 + 11 < 1 << 32)
+
+
+# sorting workgroups and those of the input gradient (600 points, 2^14, one level), gathering workgroups and those that sort (groups of the XCDs)
+@pytest.mark.parametrize("first,second,group", [(32, 2, 1), (512, 32, 1), (1, 2, 1), (5, 3, 1), (32, 32, 8), (160, 80, 8), (24, 13, 8), (1, 1, 8), (7, 100, 8)])
+def test_workgroups_of_two_kinds_are_all_met_once(rules, first, second, group):
+    blocks, kind = C.c_uint32(), C.c_uint32()
+    every = rules.turns(C.c_uint32(first), C.c_uint32(second), C.c_uint32(group), C.byref(blocks))
+    seen = [[], []]
+    for b in range(blocks.value):
+        at = rules.turn(C.c_uint32(b), C.c_uint32(every), C.c_uint32(group), C.byref(kind))
+        assert at % group == b % group  # the XCD is the workgroup's own
+        seen[kind.value].append(at)
+    for got, n in zip(seen, (first, second)):
+        assert [k for k in sorted(got) if k < n] == list(range(n))
+
+
+# launches that fit one row, by one workgroup less, exactly and by one more; the second order's launch for 2^28 points of sixteen levels; the largest batch of 32 levels
+@pytest.mark.parametrize("blocks,threads", [(1, 512), (8388599, 512), (8388600, 512), (8388601, 512), (3 * (1 << 28) // 1024 * 16, 512), (3 * (1 << 30) // 1024 * 32, 512), (1 << 31, 1024)])
+def test_rows_of_workgroups_stay_below_the_thread_limit(rules, blocks, threads):
+    out = (C.c_uint32 * 2)()
+    rules.rows_of_blocks(C.c_uint32(blocks), C.c_uint32(threads), out)
+    x, y = out
+    assert x * threads < 1 << 32 and y < 1 << 16 and blocks <= x * y < blocks + 16 * y
+    assert y == 1 or x % 8 == 0
+    assert (y == 1) == (blocks <= 8388600 * 512 // threads // 8 * 8)
