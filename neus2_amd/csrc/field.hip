@@ -925,7 +925,7 @@ N2_API int n2_sdf_loss_backward(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stre
 	}
 	if (rc != N2_OK) return rc;
 	return n2_grid_backward_fused_and_sums(grid, stream, d_xyz, point_stride, dim_stride, n, b->dL_dinput + (size_t)3 * n, b->dL_dnormal,
-	                                       b->dsdf_dinput + (size_t)3 * n, nullptr, mode, &sums);
+	                                       b->dsdf_dinput + (size_t)3 * n, mode, &sums);
 }
 
 // The inference paths for points in no particular order gather the features into the rows of the SDF net's input, at the

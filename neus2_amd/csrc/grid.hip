@@ -1609,6 +1609,8 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
                            const uint32_t* index, uint32_t n_cols, const N2ScatterRider& rider) {
 	const uint32_t tiles = n_bin_tiles(grid, n_points), per = bin_per_thread(grid, n_points), L = grid->tab.n_levels;
 	const bool first = dL_dy != nullptr, second = v != nullptr, out = dL_ddLdy != nullptr;
+	N2_REQUIRE(rider.dL_dx == nullptr || (first && !second), "n2_grid: the input gradient goes with a first-order scatter");
+	N2_REQUIRE(rider.sums.units == 0 || (first && second && !out), "n2_grid: a slab summation goes with a scatter of both orders and no dL_ddLdy");
 	const dim3 bd(BIN_BLOCK);
 	// The records of this batch are packed as for a workspace of exactly this size (values, keys, offsets one behind the
 	// other); the images of split buckets stand where the workspace's own size put them.
@@ -1757,12 +1759,13 @@ N2_API int n2_grid_backward(n2_grid_t* grid, n2_stream_t stream, const float* d_
 	                      mode == N2_GRAD_ACCUMULATE, nullptr, 0, rider);
 }
 
-int n2_grid_backward_fused_and_sums(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
-                                    const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy, n2_grad_mode mode,
-                                    const N2SlabReduce* sums) {
+static int backward_fused(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
+                          const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy, n2_grad_mode mode,
+                          const N2SlabReduce* sums, const uint32_t* d_index, uint32_t n_cols) {
 	if (int rc = check_batch(grid, "n2_grid_backward_fused", d_xyz, point_stride, dim_stride, n_points)) return rc;
 	N2_REQUIRE((d_dL_dy && d_dL_ddLdx && d_dL_dy_second) || n_points == 0, "n2_grid_backward_fused: d_dL_dy, d_dL_ddLdx and d_dL_dy_second are required");
 	N2_REQUIRE(mode == N2_GRAD_OVERWRITE || mode == N2_GRAD_ACCUMULATE, "n2_grid_backward_fused: mode must be OVERWRITE or ACCUMULATE");
+	N2_REQUIRE(d_index == nullptr || n_cols >= 1, "n2_grid_backward_fused: an indexed input needs at least one column");
 	hipStream_t s = n2_stream(stream);
 	if (int rc = prepare_grads(grid, "n2_grid_backward_fused", s, mode, n_points)) return rc;
 	if (n_points == 0) return sums ? n2_slab_reduce_launch(stream, *sums) : N2_OK;
@@ -1771,31 +1774,24 @@ int n2_grid_backward_fused_and_sums(n2_grid_t* grid, n2_stream_t stream, const f
 	N2ProfScope prof(N2_PROF_GRID_BACKWARD_PARAMS, s);
 	return launch_scatter(grid, s, d_xyz, point_stride, dim_stride, n_points, reinterpret_cast<const __half*>(d_dL_dy), d_dL_ddLdx,
 	                      reinterpret_cast<const __half*>(d_dL_dy_second), grid->grads, reinterpret_cast<__half*>(d_dL_ddLdy),
-	                      mode == N2_GRAD_ACCUMULATE, nullptr, 0, rider);
+	                      mode == N2_GRAD_ACCUMULATE, d_index, n_cols, rider);
+}
+// (a launch has workgroups for one of the two beside its own: a slab summation, or dL_ddLdy)
+int n2_grid_backward_fused_and_sums(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
+                                    const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_grad_mode mode, const N2SlabReduce* sums) {
+	return backward_fused(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_dL_dy, d_dL_ddLdx, d_dL_dy_second, nullptr, mode, sums, nullptr, 0);
 }
 N2_API int n2_grid_backward_fused(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
                                   uint32_t dim_stride, uint32_t n_points, const n2_half* d_dL_dy,
                                   const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy,
                                   n2_grad_mode mode) {
-	return n2_grid_backward_fused_and_sums(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_dL_dy, d_dL_ddLdx, d_dL_dy_second, d_dL_ddLdy, mode, nullptr);
+	return backward_fused(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_dL_dy, d_dL_ddLdx, d_dL_dy_second, d_dL_ddLdy, mode, nullptr, nullptr, 0);
 }
-
 int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz_rows, uint32_t n_cols, const uint32_t* d_index,
                                    uint32_t n_points, const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second,
                                    n2_grad_mode mode, const N2SlabReduce* sums) {
 	if (d_index == nullptr) n_cols = n_points;  // the rows hold the batch itself
-	if (int rc = check_batch(grid, "n2_grid_backward_fused", d_xyz_rows, 1, n_cols, n_points)) return rc;
-	N2_REQUIRE((d_dL_dy && d_dL_ddLdx && d_dL_dy_second) || n_points == 0, "n2_grid_backward_fused: d_dL_dy, d_dL_ddLdx and d_dL_dy_second are required");
-	N2_REQUIRE(mode == N2_GRAD_OVERWRITE || mode == N2_GRAD_ACCUMULATE, "n2_grid_backward_fused: mode must be OVERWRITE or ACCUMULATE");
-	N2_REQUIRE(n_cols >= 1, "n2_grid_backward_fused: an indexed input needs at least one column");
-	hipStream_t s = n2_stream(stream);
-	if (int rc = prepare_grads(grid, "n2_grid_backward_fused", s, mode, n_points)) return rc;
-	if (n_points == 0) return sums ? n2_slab_reduce_launch(stream, *sums) : N2_OK;
-	N2ScatterRider rider;
-	if (sums) rider.sums = *sums;
-	N2ProfScope prof(N2_PROF_GRID_BACKWARD_PARAMS, s);
-	return launch_scatter(grid, s, d_xyz_rows, 1, n_cols, n_points, reinterpret_cast<const __half*>(d_dL_dy), d_dL_ddLdx,
-	                      reinterpret_cast<const __half*>(d_dL_dy_second), grid->grads, nullptr, mode == N2_GRAD_ACCUMULATE, d_index, n_cols, rider);
+	return backward_fused(grid, stream, d_xyz_rows, 1, n_cols, n_points, d_dL_dy, d_dL_ddLdx, d_dL_dy_second, nullptr, mode, sums, d_index, n_cols);
 }
 
 N2_API int n2_grid_backward_backward_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz,

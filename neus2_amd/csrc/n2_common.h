@@ -232,10 +232,9 @@ int n2_field_backward_deferred(n2_field_t* field, n2_stream_t stream, const floa
                                n2_grad_mode mode, N2SlabReduce* sums);
 // n2_field_select without the copy of the index: d_source_index must stay valid and unchanged until the backward has run
 int n2_field_select_borrow(n2_field_t* field, const uint32_t* d_source_index, uint32_t n_source, uint32_t n);
-// n2_grid_backward_fused with a slab summation (or null) that is run beside the scatter (d_dL_ddLdy null), by workgroups of its first launch
+// n2_grid_backward_fused without d_dL_ddLdy, with a slab summation (or null) that is run beside the scatter, by workgroups of its first launch
 int n2_grid_backward_fused_and_sums(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points,
-                                    const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_half* d_dL_ddLdy, n2_grad_mode mode,
-                                    const N2SlabReduce* sums);
+                                    const n2_half* d_dL_dy, const float* d_dL_ddLdx, const n2_half* d_dL_dy_second, n2_grad_mode mode, const N2SlabReduce* sums);
 // n2_grid_backward_fused whose positions (SoA 3 x n_cols) and d_dL_dy_second rows (n_cols columns) are read through d_index.
 // sums: as there
 int n2_grid_backward_fused_indexed(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz_rows, uint32_t n_cols, const uint32_t* d_index,
