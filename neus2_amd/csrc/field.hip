@@ -910,6 +910,9 @@ N2_API int n2_sdf_loss_backward(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t stre
 	const char* fn = "n2_sdf_loss_backward";
 	uint32_t enc_w, in_w;
 	if (int rc = check_sdf_step(fn, grid, mlp, d_xyz, point_stride, dim_stride, n, b, enc_w, in_w)) return rc;
+	// (nothing runs where the scatter would be refused: the network's sums ride in it)
+	N2_REQUIRE(mode == N2_GRAD_OVERWRITE || mode == N2_GRAD_ACCUMULATE, "%s: mode must be OVERWRITE or ACCUMULATE", fn);
+	N2_REQUIRE(n2_grid_has_gradients(grid), "%s: the encoding has no gradient buffer (n2_grid_set_params)", fn);
 	// The weights' slabs are summed beside the encoding's scatter, unless the network's owner keeps them pending.
 	const bool beside = !n2_mlp_defers(mlp);
 	if (beside) {

@@ -1485,6 +1485,8 @@ static int prepare_grads(n2_grid_t* grid, const char* fn, hipStream_t stream, n2
 	return N2_OK;
 }
 
+bool n2_grid_has_gradients(const n2_grid_t* grid) { return grid->params != nullptr && grid->grads != nullptr; }
+
 static inline uint32_t n_pair_tiles(uint32_t n_points) { return (n_points + PAIR_POINTS - 1) / PAIR_POINTS; }
 static inline uint32_t bin_per_thread(const n2_grid_t* grid, uint32_t n_points) { return n2_bin_points_per_thread(grid->tab.n_levels, n_points, BIN_BLOCK); }
 static inline uint32_t n_bin_tiles(const n2_grid_t* grid, uint32_t n_points) {

@@ -137,6 +137,7 @@ int n2_fused_sdf_eikonal(hipStream_t s, const n2_half* weights, uint32_t n, cons
 // n2_grid_forward into rows 3.. of the SDF network's input (n_points columns), and the centred positions into rows 0..2
 int n2_grid_forward_sdf_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points, n2_half* d_input,
                               float* d_dy_dx);
+bool n2_grid_has_gradients(const n2_grid_t* grid);  // parameters and gradients are set
 // the network's weights (null: not set) and whether its slab sums are deferred by its owner
 const n2_half* n2_mlp_weights(const n2_mlp_t* mlp);
 bool n2_mlp_defers(const n2_mlp_t* mlp);

@@ -203,6 +203,26 @@ def test_step_errors():
         net.forward(torch.rand((3, 16), device="cuda"))
 
 
+def test_a_refused_backward_leaves_everything_as_it_was():
+    from neus2_amd.sdf_net import SdfNet
+    from neus2_amd.tcnn_api import N2Error
+    n = 64
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    net = SdfNet(16, 14, 16, 1.3, max_batch=n)
+    P = (torch.randn(net.grid.n_params(), device="cuda", generator=gen) * 0.01).half()
+    W = (torch.randn(net.mlp.n_params(), device="cuda", generator=gen) * 0.15).half()
+    gP, gW = torch.zeros_like(P), torch.full_like(W, 7.0)
+    net.set_params(P, None, W, gW)
+    ctx = net.forward(torch.rand((3, n), device="cuda", generator=gen))
+    d_inp = ctx["buffers"][1]["dL_dinput"].fill_(7.0)
+    with pytest.raises(N2Error, match="n2_sdf_loss_backward.*no gradient buffer"):
+        net.loss_backward(ctx)
+    assert bool((gW == 7).all()) and bool((d_inp == 7).all())
+    net.set_params(P, gP, W, gW)
+    net.loss_backward(ctx)
+    assert bool((gP != 0).any()) and not bool((gW == 7).any())
+
+
 @pytest.mark.parametrize("n,enc_w,in_w", [(8, 32, 48), (1000, 32, 48), (264, 13, 16), (72, 40, 48)])  # thirteen rows of padding, none, five; the smallest batch
 def test_padding_is_cleared_and_nothing_else(n, enc_w, in_w):
     import ctypes as C
