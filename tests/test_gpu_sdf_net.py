@@ -83,28 +83,39 @@ def test_normals_and_loss_in_one_pass_equal_the_two_calls(n_levels, n):
         assert torch.equal(a, b)
 
 
-# less than a wave's tile, its edges, several tiles per wave, a streamed Jacobian; networks whose lanes do not hold their levels
-@pytest.mark.parametrize("n_levels,n", [(16, 8), (16, 24), (16, 32), (16, 40), (16, 5000), (16, 65536 + 8), (16, 180000), (3, 256), (15, 1000), (20, 776)])
-def test_step_equals_the_single_calls(n_levels, n):
-    """n2_sdf_forward_and_loss and n2_sdf_loss_backward against the entry points they stand for.  The one-pass kernel adds the network's products and the
-    normals' terms in another order (one fp16 rounding of the first output moves by a digit now and then)."""
+# less than a wave's tile, its edges, several tiles per wave, a streamed Jacobian; networks whose lanes do not hold their levels; gradients added to what is there, a
+# network whose owner sums its slabs, and a scatter without a workspace
+@pytest.mark.parametrize("n_levels,n,kind", [(16, 8, ""), (16, 24, ""), (16, 32, ""), (16, 40, ""), (16, 5000, ""), (16, 65536 + 8, ""), (16, 180000, ""), (3, 256, ""), (15, 1000, ""),
+                                             (20, 776, ""), (16, 1000, "accumulate"), (16, 1000, "deferred"), (16, 1000, "atomics"), (3, 1000, "accumulate"), (3, 1000, "deferred")])
+def test_step_equals_the_single_calls(n_levels, n, kind):
+    """n2_sdf_forward_and_loss and n2_sdf_loss_backward against the entry points they stand for.  The one-pass kernel adds the network's products and the normals' terms in
+    another order: an fp16 output moves by a digit, 2^-10 at most, in one value of 500 (bound: of 100, or two), the rest in its fp32 sums.  The other bounds are four times the
+    largest of six seeds at eight sizes (normals 1.1e-7, loss 1.9e-7, gradients of a level 7.1e-5, of the network 4.2e-5, of one of its input columns 5.8e-4)."""
     import ctypes as C
     from neus2_amd import capi
     from neus2_amd.capi import check, ptr
     from neus2_amd.sdf_net import SdfNet
-    from neus2_amd.tcnn_api import GRAD_OVERWRITE, LAYOUT_SOA, _stream
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, LAYOUT_SOA, _stream
     L, u = capi.lib(), C.c_uint32
     gen = torch.Generator(device="cuda").manual_seed(n)
-    net = SdfNet(n_levels, 14, 16, 1.3, max_batch=n)
+    net = SdfNet(n_levels, 14, 16, 1.3, max_batch=n // 2 if kind == "atomics" else n)
     P = (torch.randn(net.grid.n_params(), device="cuda", generator=gen) * 0.01).half()
     W = (torch.randn(net.mlp.n_params(), device="cuda", generator=gen) * 0.15).half()
-    gP, gW = torch.zeros_like(P), torch.zeros_like(W)
+    before = [(torch.randn(t.shape, device="cuda", generator=gen) * 0.01).half() for t in (P, W)]  # where gradients go
+    gP, gW = (t.clone() for t in before)
     net.set_params(P, gP, W, gW)
+    net.mlp.set_deferred_reduction(kind == "deferred")
     x = torch.rand((3, n), device="cuda", generator=gen)
+    mode = GRAD_ACCUMULATE if kind == "accumulate" else GRAD_OVERWRITE
     for _ in range(2):  # (and on buffers that a step has used)
+        gP.copy_(before[0])
+        gW.copy_(before[1])
         ctx = net.forward(x, 0.2, 64.0)
-        loss = net.loss_backward(ctx, 0.2, 64.0)
-    got = dict(y=ctx["y"], g=ctx["g"], normal=ctx["normal"], loss=loss, grid=gP, mlp=gW, inp=ctx["inp"])
+        check(L.n2_sdf_loss_backward(net.grid._h, net.mlp._h, _stream(), x.data_ptr(), 1, n, n, C.byref(ctx["buffers"][0]), mode))
+        if kind == "deferred":
+            assert torch.equal(gW, before[1])
+            check(L.n2_mlp_reduce_deferred(net.mlp._h, None, _stream()))
+    got = dict(y=ctx["y"], g=ctx["g"], normal=ctx["normal"], loss=ctx["loss"], grid=gP, mlp=gW, inp=ctx["inp"])
     got = {k: t.clone() for k, t in got.items()}
     rows, in_w = net.enc_w, net.in_w
     h = lambda r: torch.full((r, n), 7.0, dtype=torch.float16, device="cuda")
@@ -112,19 +123,39 @@ def test_step_equals_the_single_calls(n_levels, n):
     inp, y, g, dL_dy, v_in, d_inp, normal, v, loss = h(in_w), h(16), h(in_w), h(16), h(in_w), h(in_w), f(3), f(3), torch.zeros(1, device="cuda")
     dy_dx = torch.empty((rows, n, 3), device="cuda")
     ws = torch.empty(int(L.n2_sdf_eikonal_workspace_bytes(u(n))), dtype=torch.uint8, device="cuda")
+    gP.copy_(before[0])
+    gW.copy_(before[1])
     check(L.n2_sdf_pack_input(_stream(), ptr(x), u(1), u(n), u(n), u(rows), u(in_w), ptr(inp)))
     check(L.n2_grid_forward(net.grid._h, _stream(), ptr(x), u(1), u(n), u(n), ptr(inp[3:]), ptr(dy_dx)))
     check(L.n2_mlp_forward_and_input_gradient(net.mlp._h, _stream(), u(0), ptr(inp), u(n), ptr(y), C.c_int(LAYOUT_SOA), ptr(g)))
     check(L.n2_sdf_normals_and_eikonal_loss(_stream(), u(n), u(rows), u(in_w), ptr(y), ptr(g), ptr(dy_dx), ptr(normal), C.c_float(0.2), C.c_float(64.0), ptr(dL_dy), ptr(v),
                                             ptr(v_in), ptr(loss), ptr(ws), C.c_uint64(ws.numel())))
-    check(L.n2_mlp_backward_and_second_order(net.mlp._h, _stream(), ptr(inp), u(n), ptr(dL_dy), C.c_int(LAYOUT_SOA), ptr(d_inp), ptr(v_in), None, C.c_int(GRAD_OVERWRITE)))
-    check(L.n2_grid_backward_fused(net.grid._h, _stream(), ptr(x), u(1), u(n), u(n), ptr(d_inp[3:]), ptr(v), ptr(g[3:]), None, C.c_int(GRAD_OVERWRITE)))
-    want = dict(y=y, g=g, normal=normal, loss=loss, grid=gP, mlp=gW, inp=inp)
-    for k, t in want.items():
-        if n_levels != 16 or k == "inp":
+    check(L.n2_mlp_backward_and_second_order(net.mlp._h, _stream(), ptr(inp), u(n), ptr(dL_dy), C.c_int(LAYOUT_SOA), ptr(d_inp), ptr(v_in), None, C.c_int(mode)))
+    if kind == "deferred":
+        check(L.n2_mlp_reduce_deferred(net.mlp._h, None, _stream()))
+    check(L.n2_grid_backward_fused(net.grid._h, _stream(), ptr(x), u(1), u(n), u(n), ptr(d_inp[3:]), ptr(v), ptr(g[3:]), None, C.c_int(mode)))
+    assert torch.equal(got["inp"], inp) and torch.equal(got["g"], g)
+    want = dict(y=y, normal=normal, loss=loss, grid=gP, mlp=gW)
+    if n_levels != 16:
+        for k, t in want.items():
             assert torch.equal(got[k], t), k
-        else:
-            assert bool((t != 0).any()) and rel_l2(host(got[k]), host(t)) < 1e-3, (k, rel_l2(host(got[k]), host(t)))
+        return
+    def close(a, b, bound, what):  # (rows of zeros are equal)
+        err = float((a.double() - b.double()).norm() / b.double().norm()) if bool((b != 0).any()) else float((a != b).any())
+        assert err <= bound, (what, err, bound)
+    for r in range(16):
+        close(got["y"][r], y[r], 2.0 ** -10 * max(0.01, 2 / n) ** 0.5, ("output", r))
+    for d in range(3):
+        close(got["normal"][d], normal[d], 5e-7, ("normal", d))
+    close(got["loss"], loss, 1e-6, "loss")
+    first = net.grid.level_table()[3]
+    for l in range(16):
+        part = slice(2 * int(first[l]), 2 * int(first[l + 1]))
+        # (fp16 atomics add in the order of arrival, a rounding of 2^-11 each, up to 8 n / entries of them)
+        close(got["grid"][part], gP[part], 5e-3 if kind == "atomics" else 3e-4, ("level", l))
+    close(got["mlp"], gW, 2e-4, "network")
+    for c in range(in_w):
+        close(got["mlp"][:64 * in_w].view(64, in_w)[:, c], gW[:64 * in_w].view(64, in_w)[:, c], 2.4e-3, ("column", c))
 
 
 def test_points_beyond_the_one_pass_kernels_offsets():
@@ -139,16 +170,16 @@ def test_points_beyond_the_one_pass_kernels_offsets():
     x = torch.rand((3, n), device="cuda", generator=gen)
     ctx = net.forward(x, 0.2, 64.0)
     pick = lambda ctx, k: ctx["buffers"][1][k][:, -m:].float().clone()
-    scale = dict(output=1, dsdf_dinput=1, normal=1, dL_dnormal=n / m)  # (the loss is a mean over the batch)
-    got = {k: pick(ctx, k) * f for k, f in scale.items()}
+    # (the kernels for few and for many points add in another order: an fp16 output moves by a digit now and then, normals in their fp32 sums)
+    bound = dict(output=1e-4, dsdf_dinput=0, normal=5e-7, dL_dnormal=2e-6)
+    got = {k: pick(ctx, k) * (n / m if k == "dL_dnormal" else 1) for k in bound}  # (the loss is a mean over the batch)
     del ctx
     net._n, net._b = 0, None
     torch.cuda.empty_cache()
     ctx = net.forward(x[:, -m:].contiguous(), 0.2, 64.0)
-    for k in scale:
+    for k in bound:
         want = pick(ctx, k)
-        # (the kernels for few and for many points add in another order: an fp16 output moves by a digit now and then)
-        assert bool((want != 0).any()) and rel_l2(host(got[k]), host(want)) < 1e-3, k
+        assert bool((want != 0).any()) and rel_l2(host(got[k]), host(want)) <= bound[k], (k, rel_l2(host(got[k]), host(want)))
     del x, got
     torch.cuda.empty_cache()
 
