@@ -105,54 +105,55 @@ def lib():
             import torch  # noqa: F401
         except ImportError:
             pass
-        _lib = C.CDLL(LIB_PATH)
+        L = C.CDLL(LIB_PATH)
         kinds = dict(p=C.c_void_p, u=C.c_uint32, f=C.c_float, i=C.c_int, q=C.c_uint64)
         for name, signature in _SIGNATURES.items():
-            getattr(_lib, name).argtypes = [kinds[k] for k in signature]
-        _lib.n2_last_error.restype = C.c_char_p
-        _lib.n2_version.restype = C.c_char_p
-        _lib.n2_field_encoding.restype = C.c_void_p
-        _lib.n2_field_encoding.argtypes = [C.c_void_p]
+            getattr(L, name).argtypes = [kinds[k] for k in signature]
+        L.n2_last_error.restype = C.c_char_p
+        L.n2_version.restype = C.c_char_p
+        L.n2_field_encoding.restype = C.c_void_p
+        L.n2_field_encoding.argtypes = [C.c_void_p]
         for name in ("n2_grid_n_params", "n2_grid_output_width", "n2_grid_n_levels", "n2_grid_active_levels"):
-            getattr(_lib, name).restype = C.c_uint32
-            getattr(_lib, name).argtypes = [C.c_void_p]
-        _lib.n2_grid_workspace_bytes.restype = C.c_uint64
-        _lib.n2_grid_workspace_bytes.argtypes = [C.c_void_p, C.c_uint32]
-        _lib.n2_grid_destroy.restype = None
-        _lib.n2_grid_destroy.argtypes = [C.c_void_p]
+            getattr(L, name).restype = C.c_uint32
+            getattr(L, name).argtypes = [C.c_void_p]
+        L.n2_grid_workspace_bytes.restype = C.c_uint64
+        L.n2_grid_workspace_bytes.argtypes = [C.c_void_p, C.c_uint32]
+        L.n2_grid_destroy.restype = None
+        L.n2_grid_destroy.argtypes = [C.c_void_p]
         for name in ("n2_mlp_n_params", "n2_mlp_input_width", "n2_mlp_output_width"):
-            getattr(_lib, name).restype = C.c_uint32
-            getattr(_lib, name).argtypes = [C.c_void_p]
-        _lib.n2_mlp_workspace_bytes.restype = C.c_uint64
-        _lib.n2_mlp_workspace_bytes.argtypes = [C.c_void_p]
-        _lib.n2_mlp_destroy.restype = None
-        _lib.n2_mlp_destroy.argtypes = [C.c_void_p]
-        _lib.n2_field_n_params.restype = C.c_uint32
-        _lib.n2_field_n_params.argtypes = [C.c_void_p]
-        _lib.n2_field_workspace_bytes.restype = C.c_uint64
-        _lib.n2_field_workspace_bytes.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32]
-        _lib.n2_composite_workspace_bytes.restype = C.c_uint64
-        _lib.n2_composite_workspace_bytes.argtypes = [C.c_uint32]
-        _lib.n2_sampler_workspace_bytes.restype = C.c_uint64
-        _lib.n2_sampler_workspace_bytes.argtypes = [C.c_uint32]
-        _lib.n2_sdf_eikonal_workspace_bytes.restype = C.c_uint64
-        _lib.n2_sdf_eikonal_workspace_bytes.argtypes = [C.c_uint32]
-        _lib.n2_sdf_step_workspace_bytes.restype = C.c_uint64
-        _lib.n2_sdf_step_workspace_bytes.argtypes = [C.c_uint32]
-        _lib.n2_trainer_workspace_bytes.restype = C.c_uint64
-        _lib.n2_trainer_workspace_bytes.argtypes = [C.c_void_p]
-        _lib.n2_trainer_destroy.restype = None
-        _lib.n2_trainer_destroy.argtypes = [C.c_void_p]
-        _lib.n2_trainer_field.restype = C.c_void_p
-        _lib.n2_trainer_field.argtypes = [C.c_void_p]
-        _lib.n2_field_destroy.restype = None
-        _lib.n2_field_destroy.argtypes = [C.c_void_p]
-        _lib.n2_occupancy_workspace_bytes.restype = C.c_uint64
-        _lib.n2_occupancy_workspace_bytes.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32]
-        _lib.n2_snapshot_close.restype = None
-        _lib.n2_snapshot_close.argtypes = [C.c_void_p]
-        _lib.n2_occupancy_destroy.restype = None
-        _lib.n2_occupancy_destroy.argtypes = [C.c_void_p]
+            getattr(L, name).restype = C.c_uint32
+            getattr(L, name).argtypes = [C.c_void_p]
+        L.n2_mlp_workspace_bytes.restype = C.c_uint64
+        L.n2_mlp_workspace_bytes.argtypes = [C.c_void_p]
+        L.n2_mlp_destroy.restype = None
+        L.n2_mlp_destroy.argtypes = [C.c_void_p]
+        L.n2_field_n_params.restype = C.c_uint32
+        L.n2_field_n_params.argtypes = [C.c_void_p]
+        L.n2_field_workspace_bytes.restype = C.c_uint64
+        L.n2_field_workspace_bytes.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32]
+        L.n2_composite_workspace_bytes.restype = C.c_uint64
+        L.n2_composite_workspace_bytes.argtypes = [C.c_uint32]
+        L.n2_sampler_workspace_bytes.restype = C.c_uint64
+        L.n2_sampler_workspace_bytes.argtypes = [C.c_uint32]
+        L.n2_sdf_eikonal_workspace_bytes.restype = C.c_uint64
+        L.n2_sdf_eikonal_workspace_bytes.argtypes = [C.c_uint32]
+        L.n2_sdf_step_workspace_bytes.restype = C.c_uint64
+        L.n2_sdf_step_workspace_bytes.argtypes = [C.c_uint32]
+        L.n2_trainer_workspace_bytes.restype = C.c_uint64
+        L.n2_trainer_workspace_bytes.argtypes = [C.c_void_p]
+        L.n2_trainer_destroy.restype = None
+        L.n2_trainer_destroy.argtypes = [C.c_void_p]
+        L.n2_trainer_field.restype = C.c_void_p
+        L.n2_trainer_field.argtypes = [C.c_void_p]
+        L.n2_field_destroy.restype = None
+        L.n2_field_destroy.argtypes = [C.c_void_p]
+        L.n2_occupancy_workspace_bytes.restype = C.c_uint64
+        L.n2_occupancy_workspace_bytes.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32]
+        L.n2_snapshot_close.restype = None
+        L.n2_snapshot_close.argtypes = [C.c_void_p]
+        L.n2_occupancy_destroy.restype = None
+        L.n2_occupancy_destroy.argtypes = [C.c_void_p]
+        _lib = L  # (not before: without its signature a call takes an address for a 32-bit number, and other threads call what stands here)
     return _lib
 
 

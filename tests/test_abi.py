@@ -29,6 +29,32 @@ def test_library_exports_every_declared_symbol():
     assert not missing, missing
 
 
+def test_nobody_sees_the_library_before_its_signatures_are_set(monkeypatch):
+    """A thread that calls lib() meanwhile must not get it: Python's numbers go in as 32 bits where a function has no argtypes."""
+    from neus2_amd import capi
+    seen, real = [], capi.C.CDLL
+
+    class Watched(real):
+        def __getattr__(self, name):
+            seen.append(capi._lib)
+            return super().__getattr__(name)
+
+    monkeypatch.setattr(capi, "_lib", None)
+    monkeypatch.setattr(capi.C, "CDLL", Watched)
+    L = capi.lib()
+    assert len(seen) > len(capi._SIGNATURES) and not any(seen)
+    assert capi.lib() is L and L.n2_grid_forward.argtypes[2] is ctypes.c_void_p
+
+
+def test_signatures_are_the_headers():
+    from neus2_amd import capi
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "neus2_amd.h")).read(), flags=re.S)
+    kind = lambda a: "p" if "*" in a or "n2_stream_t" in a or "[" in a else {"uint32_t": "u", "float": "f", "uint64_t": "q"}.get(a.split()[0], "i")
+    for name, signature in capi._SIGNATURES.items():
+        arguments = re.search(r"\b%s\s*\((.*?)\)" % name, text, re.S).group(1).split(",")
+        assert "".join(kind(a.replace("const ", "").strip()) for a in arguments) == signature, name
+
+
 def test_host_only_entry_points_work_without_gpu():
     """Object creation and the level table are pure host code."""
     import numpy as np
