@@ -1022,7 +1022,8 @@ constexpr uint32_t QUERY_ONE_LAUNCH_MAX = 256 * FQ_POINTS;
 // 2^21 566 | 531; along rays 65 536 20.3 | 21.2, 98 304 26.5 | 26.8, 2^17 33.7 | 32.1, 2^20 184 | 182; on a lattice 65 536 19.6 | 20.0, 98 304 26.1 | 25.7, 2^20 142 | 141.  Updates of
 // the occupancy grid: 2^17 samples 67.5 | 64.0, 700 000 264 | 250, 2^20 252 | 245, 2^21 421 | 415.)
 constexpr uint32_t QUERY_STAGED_MIN = 3u << 15;
-// ... and from here on three more come from blocks: making these costs smaller queries what they save.  (Call in us, staged | with blocks, uniform points: 98 304 36.4 | 37.3, 2^17
+// ... and from here on three more come from blocks: making these costs smaller queries what they save.  The line is that of points in no order; points that come in one share lines
+// without blocks, and those between here and 2^19 lose two to three per cent to them.  (Call in us, staged | with blocks, uniform points: 98 304 36.4 | 37.3, 2^17
 // 44.2 | 43.9, 2^18 77.7 | 73.3, 2^19 148 | 136, 2^20 278 | 250, 2^21 531 | 480; along rays 2^17 32.1 | 35.2, 2^18 56.1 | 57.8, 2^19 99.0 | 98.2, 2^20 182 | 177; on a lattice 2^17
 // 31.4 | 34.4, 2^18 55.1 | 56.5, 2^19 77.2 | 77.6, 2^20 141 | 136.  Updates of the occupancy grid: 2^19 samples 160.4 | 157.2, 700 000 250 | 231, 2^20 245 | 236, 2^21 415 | 400.)
 constexpr uint32_t QUERY_BLOCKS_MIN = 1u << 18;

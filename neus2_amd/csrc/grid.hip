@@ -970,7 +970,10 @@ __device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const uin
 	}
 }
 
-// FLIGHT: 2 for batches of few tiles, whose runs rarely hold more (30 000 points: forward and backward 41.6 -> 41.3 us)
+// FLIGHT: 2 for batches of few tiles, whose runs rarely hold more.  Backward in us (device time in a graph), 4 | 2: the default table uniform 24 584 28.6 | 28.3, 28 672 29.5 | 29.0,
+// 32 768 30.4 | 29.9, along rays 24 584 26.4 | 25.9, 30 000 28.0 | 27.4, 32 768 29.2 | 28.4; tables of 2^16 entries a level, uniform 10 000 17.1 | 16.0, 16 384 19.5 | 20.3, 30 000 23.8 | 24.7, along
+// rays 10 000 14.4 | 13.2, 16 384 16.0 | 15.0, 30 000 21.4 | 20.8; of 2^14, uniform 5000 13.0 | 13.7, 30 000 30.4 | 32.3, along rays 3000 10.2 | 9.6, 30 000 29.0 | 30.6: no line on the tables' size
+// is right for either order.
 template <uint32_t FLIGHT>
 __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
@@ -1025,8 +1028,8 @@ __global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable 
 // match a tile's run.  Levels of few entries keep an image, as does (range by range) a bucket with more records than
 // there are sums to claim.  What bounds it is the chain level -> bounds -> records -> sums and the 25 MB the gradient's zeros take.
 // Launch in us, image -> claims: 600 uniform points 15 -> 10.1, 5003 along rays 15.1 -> 10.6 (accumulating 15.6 -> 9.5), training step of 2^14 samples 17.5 -> 14.8.
-// (256 threads: the same up to 5000 points, 16 384 uniform points +4; 1024: +4; 128: +0.5.  32 KiB hold the claims of two thirds of the
-// points: 20 000 along rays 34.0, by grid_reduce_kernel, against 29.5.)
+// (256 threads: the same up to 5000 points, 16 384 uniform points +4; 1024: +4; 128: +0.5.  In 32 KiB there are 1536 sums instead of 2048,
+// and batches beyond 16 384 points took grid_reduce_kernel: 20 000 along rays 34.0 against 29.5.)
 constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 5120;
 constexpr uint32_t FEW_TILES = 64;                                  // a lane of every wave looks up one tile's run
 constexpr uint32_t FEW_CLAIMS = (FEW_WORDS - BKT_ENTRIES / 4) / 2;  // sums of both features, beside the table of 16-bit claims

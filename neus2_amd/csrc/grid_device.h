@@ -144,7 +144,7 @@ __device__ __forceinline__ void n2_encode_level(const char* __restrict__ base, u
 	// of point m's x corner b: the bilinear value s, and its y and z differences ty, tz
 	float s[2][2], ty[2][2], tz[2][2];  // [point][feature]
 	// (differences as multiply-adds as well, by a one that the compiler does not see through: it would convert the halves first, an instruction
-	// each.  With the shorter n2_slopes_pack 28 fewer of 265: gather of 2^18 samples along rays 64.1 -> 61.2 us, second order of 131 072
+	// each.  With the shorter n2_slopes_pack 25 fewer of 265: gather of 2^18 samples along rays 64.1 -> 61.2 us, second order of 131 072
 	// points 174.3 -> 169.7 for the call)
 	float one = 1.f;
 	asm("" : "+s"(one));

@@ -125,8 +125,9 @@ int n2_generate_training_samples_rows(n2_stream_t stream, uint32_t n_rays, uint3
                                       float* d_coords, void* d_workspace, uint64_t workspace_bytes, float* d_xyz_rows);
 // NerfNetwork::sdf / density: d_out_soa (16 x n, may be null) and / or d_row0 (fp32 copy of row 0, may be null).
 // sdf_in null: one kernel that gathers sample by sample (points in lattice order, whose table lines stay cached);
-// else a level-major gather into the feature rows 3.. of sdf_in (SoA, n columns) followed by the network kernel.  scratch (16-byte aligned, or null): for the coarse
-// levels of large queries, whose rows of sdf_in are then not written.
+// else a level-major gather into sdf_in followed by the network kernel: from its start on a row of n words to each level, both features side by side, whatever stood in the
+// training forward's rows of halves there (16 levels take 64 bytes a point of 96).  scratch (16-byte aligned, or null): for the coarse levels of large queries, whose
+// rows of sdf_in are then not written.
 int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xyz, uint32_t ps, uint32_t ds, uint32_t n, n2_half* d_out_soa,
                        float* d_row0, bool density, n2_half* sdf_in, uint32_t row0_n = 0xFFFFFFFFu, void* scratch = nullptr, uint64_t scratch_bytes = 0);
 // The SDF network with 48 inputs on its own: output, d sdf / d input, normals, the eikonal loss's terms (n2_fused_sdf_eikonal_parts(n) partial sums) and what
