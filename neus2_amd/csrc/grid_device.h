@@ -144,7 +144,7 @@ __device__ __forceinline__ void n2_encode_level(const char* __restrict__ base, u
 	// of point m's x corner b: the bilinear value s, and its y and z differences ty, tz
 	float s[2][2], ty[2][2], tz[2][2];  // [point][feature]
 	// (differences as multiply-adds as well, by a one that the compiler does not see through: it would convert the halves first, an instruction
-	// each.  With the shorter n2_slopes_pack 25 fewer of 265: gather of 2^18 samples along rays 64.1 -> 61.2 us, second order of 131 072
+	// each.  With the shorter n2_slopes_pack 27 fewer of 265: gather of 2^18 samples along rays 64.1 -> 61.2 us, second order of 131 072
 	// points 174.3 -> 169.7 for the call)
 	float one = 1.f;
 	asm("" : "+s"(one));
@@ -205,14 +205,18 @@ __device__ __forceinline__ uint4 n2_slopes_pack(const float (&slopes)[6]) {
 	float v[6];
 #pragma unroll
 	for (int i = 0; i < 6; ++i) v[i] = slopes[i];
+	float m = 0.f;  // no number where one of the slopes is none
+#pragma unroll
+	for (int i = 0; i < 6; ++i) m = __builtin_elementwise_maximum(m, fabsf(v[i]));
 	// A slope that is no number counts as zero (the bounds below would make the lowest mantissa of it), an infinite one as the largest there is.
-	if (__builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3]) || __builtin_isunordered(v[4], v[5])) {
+	if (__builtin_isnan(m)) {
+		m = 0.f;
 #pragma unroll
-		for (int i = 0; i < 6; ++i) v[i] = __builtin_isnan(v[i]) ? 0.f : v[i];
+		for (int i = 0; i < 6; ++i) {
+			v[i] = __builtin_isnan(v[i]) ? 0.f : v[i];
+			m = fmaxf(m, fabsf(v[i]));
+		}
 	}
-	float m = 0.f;
-#pragma unroll
-	for (int i = 0; i < 6; ++i) m = fmaxf(m, fabsf(v[i]));
 	int e = 0;
 	(void)frexpf(m, &e);  // m = f * 2^e with f in [0.5, 1); 0 for m = 0
 	e = min(max(e, -100), 100);
