@@ -426,7 +426,7 @@ int n2_sdf_normals_and_eikonal_loss(n2_stream_t stream, uint32_t n, uint32_t enc
 
 /* The whole step of such a caller in two calls.  The buffers are the caller's, n columns each (fp16 SoA but where stated), 16-byte aligned and kept from
  * the forward to the backward.  Behind the encoding's rows, input and second_order_input hold zeros, as do rows 1.. of dL_doutput, which the caller
- * has cleared once (n2_sdf_clear_padding): the calls may write zeros there, but need not.
+ * has cleared once (n2_sdf_clear_padding; a clearing that is captured happens when the graph is replayed): the calls may write zeros there, but need not.
  *   n2_sdf_forward_and_loss  = n2_sdf_pack_input, n2_grid_forward with the Jacobian, n2_mlp_forward_and_input_gradient of output 0 and
  *                              n2_sdf_normals_and_eikonal_loss (for a network of 48 inputs over 32 features in two launches and the loss's sum)
  *   n2_sdf_loss_backward     = n2_mlp_backward_and_second_order and n2_grid_backward_fused, into the gradient buffers of both objects; of
