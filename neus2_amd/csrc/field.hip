@@ -436,9 +436,14 @@ static bool fused_ok(const n2_field_t* f) {
 // Rows [first_row, n_rows) of the rows x n matrix m are padding: the networks read them and they must be zero.  No kernel
 // writes them, so they are cleared when the batch size (the row pitch) differs from the one they were last cleared for.
 static int zero_padding(hipStream_t s, hf* m, uint32_t first_row, uint32_t n_rows, uint32_t n, uint32_t& cleared_for) {
-	if (cleared_for == n || first_row >= n_rows) return N2_OK;
+	if (first_row >= n_rows) return N2_OK;
+	// A captured call clears whenever its graph is replayed, whatever has run in between, and has cleared nothing yet for a call outside the graph.
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+	const bool captured = capture != hipStreamCaptureStatusNone;
+	if (cleared_for == n && !captured) return N2_OK;
 	if (int rc = n2_fill_zero_u32(s, m + (size_t)first_row * n, (size_t)(n_rows - first_row) * n * sizeof(hf))) return rc;
-	cleared_for = n;
+	cleared_for = captured ? 0u : n;
 	return N2_OK;
 }
 

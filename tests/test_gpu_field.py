@@ -358,3 +358,43 @@ def test_slopes_that_are_no_numbers_count_as_zero(oracle, infinite):
     dp.copy_(dev(p, torch.float16))
     got = host(gf.forward(dev(coords))).T[4:7]
     assert_close(got, want.astype(np.float32), what="normal")
+
+
+@pytest.mark.parametrize("n_levels", [16, 12, 20])  # the fused kernels, others of them, and the separate ones
+def test_captured_steps_and_the_padding_rows(n_levels):
+    """A batch size that is first met under capture: a step outside the graph comes before the first replay.  Queries between replays, which use the padding's place."""
+    from neus2_amd.tcnn_api import NerfNetwork
+    n = 1000
+    gen = torch.Generator(device="cuda").manual_seed(n_levels)
+    net = NerfNetwork(n_levels, 14)
+    P = (torch.randn(net.n_params(), device="cuda", generator=gen) * 0.2).half()
+    G = torch.zeros_like(P)
+    net.set_params(P, G)
+    coords = torch.rand((n, 7), device="cuda", generator=gen)
+    dL = (torch.randn((n, 16), device="cuda", generator=gen) * 0.01).half()
+    x = torch.rand((3, 16384), device="cuda", generator=gen)
+    def step():
+        y = net.forward(coords)
+        net.backward(coords, dL)
+        return y
+    net.reserve(16384)
+    want = [step().clone(), G.clone()]
+    assert all(bool(torch.isfinite(t).all()) for t in want)
+    net.sdf(x)  # (another batch size: nothing counts as cleared any more)
+    net.reserve(16392)  # a workspace of its own for this batch size ...
+    net._ws.fill_(255)  # ... and what memory that nothing has written may hold: no numbers
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        y = step()
+    torch.cuda.synchronize()
+    got = [step(), G]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    for k in range(3):
+        net.sdf(x)
+        y.zero_()
+        G.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want[0]) and torch.equal(G, want[1]), k
