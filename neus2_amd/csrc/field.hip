@@ -596,7 +596,8 @@ static int field_backward_passes(n2_field_t* f, n2_stream_t stream, const float*
 	if (int rc = n2_mlp_backward_and_second_order_indexed(f->sdf, stream, reinterpret_cast<const n2_half*>(f->sdf_in), n_src, index, n,
 	                                                      reinterpret_cast<const n2_half*>(f->d_rgb_in), f->slopes_saved ? N2_LAYOUT_AOS : N2_LAYOUT_SOA,
 	                                                      reinterpret_cast<n2_half*>(f->d_sdf_in),
-	                                                      reinterpret_cast<const n2_half*>(f->d_density_in), nullptr, mode, true)) return rc;
+	                                                      reinterpret_cast<const n2_half*>(f->d_density_in), nullptr, mode,
+	                                                      f->enc_w <= 32)) return rc;  // (of 48 inputs that pass stores rows 3..34 alone)
 	// the three weight-gradient passes (colour net, SDF net first and second order) left their per-workgroup partial sums
 	// pending: one plan sums them, and with them the partial sums of the variance gradient
 	N2SlabReduce plan;

@@ -334,6 +334,29 @@ def test_direction_encoding_rows(oracle):
         assert_close(out[r], q16(sh[r]), rtol=RTOL, what=f"SH row {r}", scale=1.0)
 
 
+@pytest.mark.parametrize("n_levels", [15, 17, 20, 22])  # networks of 48 inputs, whose encodings have 30 to 44 rows
+def test_backward_of_more_levels_than_the_fused_kernels_take(oracle, n_levels):
+    of, gf, p, dp, dg, rng = make(oracle, seed=13, n_levels=n_levels, log2_hashmap_size=14, per_level_scale=1.2)
+    assert of.sdf_in_w == 48
+    n = 2048
+    coords = rand_coords(rng, n)
+    dL = q16(rng.standard_normal((16, n)) * np.array([.1, .1, .1, .1, 3, 3, 3, .1, .003, .003, .003, 0, 0, 0, 0, 0])[:, None])
+    _, ctx = of.forward(p, coords)
+    ref = of.backward(p, ctx, dL, ek_batch_size=n)
+    gf.reserve(n)
+    gf._ws.fill_(0x3C)  # (nothing may be left from another call: halves of 1.06)
+    d_coords = dev(coords)
+    gf.forward(d_coords)
+    gf.backward(d_coords, dev(np.ascontiguousarray(dL.T), torch.float16), ek_batch_size=n)
+    got = host(dg)
+    assert_grad_close(got[:of.off_rgb], ref[:of.off_rgb], what="SDF MLP gradients", rtol=2 * RTOL)
+    for l in range(n_levels):
+        a, b = (of.off_grid + 2 * int(of.grid.offset[l + k]) for k in range(2))
+        k = 8.0 * n / max(1, int(of.grid.entries[l]))
+        tol = 2 * RTOL * max(1.0, np.sqrt(k))
+        assert rel_l2(got[a:b], ref[a:b]) < tol, (l, rel_l2(got[a:b], ref[a:b]), tol)
+
+
 @pytest.mark.parametrize("infinite", ["all", "even_x"])
 def test_slopes_that_are_no_numbers_count_as_zero(oracle, infinite):
     """Infinite entries of one level and feature: differences of two of them are no numbers and add nothing to the normal; a difference to a finite
