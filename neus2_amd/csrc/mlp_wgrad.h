@@ -92,7 +92,7 @@ enum : int {
 	WG_DX_NONE = 0,
 	WG_DX_ALL = 1,
 	WG_DX_OUT_AND_NORMAL = 2,  // rows 0..15 and 35..37: the field's colour net (gradient of the SDF net's output and of the normal)
-	WG_DX_ENCODING = 3         // rows 3..34: the field's SDF net (gradient of the encoding; positions are not optimised)
+	WG_DX_ENCODING = 3         // rows 3..34: the field's SDF net over up to 16 levels (gradient of the encoding; positions are not optimised)
 };
 __device__ __forceinline__ constexpr bool wg_dx_row(int mode, int row, int in_w) {
 	return row < in_w && (mode == WG_DX_ALL || (mode == WG_DX_OUT_AND_NORMAL && (row < 16 || (row >= 35 && row < 38))) ||

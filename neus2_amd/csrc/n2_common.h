@@ -197,7 +197,7 @@ uint32_t n2_mlp_wgrad_blocks(uint32_t n);
 // indexed by i.  The field's backward uses them to read the activations its forward saved for ALL marched samples.
 // dx_out_and_normal_only (48-input network with two hidden layers, the field's colour net): of d_dL_dinput only rows 0..15
 // and 35..37 are written (the gradients of the SDF net's output and of the normal; nothing reads the others).
-// dx_encoding_only (48-input network, the field's SDF net): only rows 3..34, the encoding's, are written.
+// dx_encoding_only (48-input network over an encoding of at most 32 rows, the field's SDF net): only rows 3..34, the encoding's, are written.
 int n2_mlp_backward_rows_indexed(n2_mlp_t* mlp, n2_stream_t stream, const n2_half* d_input, uint32_t n_cols, const uint32_t* d_index, uint32_t n,
                                  const n2_half* d_dL_doutput, n2_layout dL_layout, uint32_t n_rows, n2_half* d_dL_dinput, n2_grad_mode mode,
                                  bool dx_out_and_normal_only, const N2FieldPrepTail* tail = nullptr);
