@@ -435,18 +435,11 @@ __global__ void __launch_bounds__(GRID_BLOCK) grid_bbi_kernel(N2LevelTable tab, 
 // LDS atomics are two orders of magnitude faster, so the scatter is turned
 // into a two-kernel counting sort on entry ranges:
 //
-//  bin     one workgroup per (level, tile of 1024 points): computes the 8192
-//          (entry, value) records of the tile, sorts them in LDS by bucket
-//          (bucket = entry / 8192, at most 64 per level) and writes the sorted
-//          tile (64 KiB, fully coalesced) plus its 65 bucket offsets.
-//  reduce  one workgroup per (level, bucket[, tile group]): walks the bucket's
-//          run in every tile (contiguous, ~1 KiB each), accumulates in an LDS
-//          table of 8192 fp32 pairs with LDS atomics, and writes the bucket's
-//          entries with plain stores.  Coarse levels have few buckets, so their
-//          work is split over tile groups and folded with (few, contention-free)
-//          global atomics.
-// Accumulation is fp32 until the single rounding to fp16 at the store, which
-// also removes the rounding drift of chained fp16 atomics.
+//  bin     one workgroup per (level, tile of up to 1024 points): computes the tile's records (an entry, or a pair of neighbouring ones, and what is added
+//          there), sorts them in LDS by bucket (up to 4096 entries, at most 128 to a level) and writes the sorted tile, fully coalesced, plus its bucket offsets.
+//  reduce  a workgroup per (level, bucket[, group of tiles]) at a time: walks the bucket's run in every tile, accumulates in an LDS
+//          image of 64-bit integers with LDS atomics, and writes the bucket's entries with plain stores.
+// The sums are exact until their one rounding at the store, which also removes the rounding drift of chained fp16 atomics.
 // ----------------------------------------------------------------------------
 #ifndef N2_BKT_SHIFT
 #define N2_BKT_SHIFT 12
@@ -462,16 +455,21 @@ constexpr uint32_t BIN_BLOCK = 512;       // 8 waves: three workgroups (3 x 49 K
 __host__ __device__ constexpr uint32_t bin_points(uint32_t per) { return BIN_BLOCK * per; }
 __host__ __device__ constexpr uint32_t bin_records(uint32_t per) { return bin_points(per) * 8u; }
 
+// (see n2_queue_draw)
+constexpr uint32_t QUEUE_STRIDE = 32, QUEUE_WORDS = N_XCD * QUEUE_STRIDE;
+
+// The items of a reduce launch, a (bucket, group of tiles) each, by level: first the levels of single records, then those of pair records.
 struct N2BucketPlan {
-	uint32_t wg_begin[N2_MAX_LEVELS + 1];  // first reduce workgroup of each level
-	uint32_t n_buckets[N2_MAX_LEVELS];
-	uint32_t groups[N2_MAX_LEVELS];        // tile groups per bucket
-	// levels whose buckets are split over several workgroups (groups > 1): where the level's partial images start (images:
-	// bucket-major, then group) and the number of split buckets in the levels below
-	uint32_t part_begin[N2_MAX_LEVELS];
-	uint32_t split_begin[N2_MAX_LEVELS + 1];
-	// log2 of the lanes that take one tile's run
-	uint8_t run_lanes[N2_MAX_LEVELS];
+	uint32_t begin[N2_MAX_LEVELS + 1];  // first item of each place in that order
+	struct Level {
+		uint32_t level, n_buckets;
+		uint32_t groups;          // tile groups per bucket
+		uint32_t part_begin;      // of split buckets (groups > 1): where the level's partial images start (bucket-major, then group)
+		uint32_t bucket_entries;  // split buckets always have BKT_ENTRIES
+		uint32_t entries, offset; // the level's table
+		uint32_t pair;
+	} at[N2_MAX_LEVELS];
+	uint32_t pairs_from;  // first item of a level of pair records
 };
 
 // what a point brings along: its position, dL/dy of the level's two features, g2 of them and v
@@ -717,7 +715,7 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	// 16 bytes per lane; the last store of each array may run past `total` inside the tile's own slot, which nobody reads
 	const size_t slot = ((size_t)level * tiles + tile) * bin_records(PER);
 	uint4* out_val = reinterpret_cast<uint4*>(rec_vals + slot);
-	uint4* out_key = reinterpret_cast<uint4*>(rec_keys + slot);
+	uint4* out_key = reinterpret_cast<uint4*>(rec_keys + (size_t)level * tiles * bin_records(PER) + (size_t)tile * (bin_records(PER) / (PAIR ? 2u : 1u)));
 	const uint4* sv = reinterpret_cast<const uint4*>(stage_val);
 	const uint4* sk = reinterpret_cast<const uint4*>(stage_key);
 	for (uint32_t t = threadIdx.x; (PAIR ? 2 : 4) * t < total; t += BIN_BLOCK) out_val[t] = sv[t];
@@ -783,13 +781,14 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
                                                               const float* __restrict__ v, const __half* __restrict__ g2,
                                                               const __half2* __restrict__ params,
                                                               uint32_t* __restrict__ rec_vals, uint16_t* __restrict__ rec_keys,
-                                                              uint16_t* __restrict__ offsets,
+                                                              uint16_t* __restrict__ offsets, uint32_t* __restrict__ queue,
                                                               const uint32_t* __restrict__ index, uint32_t n_cols, Ride ride) {
 	__shared__ uint32_t hist[BKT_MAX];
 	__shared__ uint32_t prefix[BKT_MAX + 1];
 	__shared__ __align__(16) uint32_t stage_val[bin_records(PER)];  // sorted records: packed half2 value (a pair of them on pair levels) ...
 	__shared__ __align__(16) uint16_t stage_key[bin_records(PER)];  // ... and entry within its bucket
 	uint32_t block = blockIdx.x;
+	if (blockIdx.x == 0u && blockIdx.y == 0u && threadIdx.x < N_XCD) queue[threadIdx.x * QUEUE_STRIDE] = 0u;
 	if constexpr (RIDES_INPUT<Ride>) {
 		bool rides;
 		block = n2_turn(block, ride.every, 1u, rides);
@@ -838,185 +837,292 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 
 // LDS float atomics retire about one lane every three clocks on this part, integer ones at ~9 (32-bit) and
 // ~5.5 (64-bit) lanes per clock.  The reduce therefore accumulates in 64-bit fixed point: a record holds
-// fp16 values, i.e. multiples of 2^-24 below 2^16, so value * 2^32 is an exact integer below 2^48 and the
+// fp16 values, i.e. multiples of 2^-24 below 2^16, so value * 2^24 is an exact integer below 2^40 and the
 // sum of a whole bucket stays far inside 64 bits.  The accumulation is exact and independent of order.
-constexpr uint32_t RED_BLOCK = 1024;              // 16 waves; two workgroups share a CU
-constexpr uint32_t FLIGHT_TILES = 32;             // batches of at most this many tiles: see grid_reduce_kernel
-constexpr float FIX_SCALE = 4294967296.0f;        // 2^32
+constexpr uint32_t RED_BLOCK = 512;               // 8 waves; two workgroups share a CU
+constexpr uint32_t RED_AT_A_TIME = 512;           // workgroups of a launch: what runs at one time (a multiple of the XCDs)
+constexpr float FIX_SCALE = 16777216.0f;          // 2^24
 
-// x * 2^32 as a two's complement 64-bit integer, for |x| < 2^31 with at most 24 significant bits (any fp16 value):
-// the high word is floor(x), the low word fract(x) * 2^32, both exact.  Five ALU operations instead of the generic
-// float -> int64 sequence.
+// x * 2^24 as a two's complement 64-bit integer, for |x| < 128, given that product, which has 32 bits then: two instructions.  Beyond, it is cut to 32 bits;
+// no number gives zero.
+__device__ __forceinline__ unsigned long long small_fixed(float scaled) { return (unsigned long long)(long long)(int32_t)scaled; }
+__device__ __forceinline__ bool is_small_fixed(float scaled) { return !(fabsf(scaled) >= 2147483648.f); }
+// For any fp16 value.  An infinite one counts as 2^22: 65536 of them stay inside 64 bits, and one of them is infinite again as fp16.
 __device__ __forceinline__ unsigned long long to_fixed(float x) {
-	const float fl = floorf(x);
-	const uint32_t hi = (uint32_t)(int32_t)fl, lo = (uint32_t)((x - fl) * FIX_SCALE);
-	return ((unsigned long long)hi << 32) | lo;
+	const float scaled = x * FIX_SCALE;
+	unsigned long long q = small_fixed(scaled);
+	if (__any(!is_small_fixed(scaled))) {  // (six times as long)
+		const long long large = (long long)((double)fminf(fmaxf(x, -4194304.f), 4194304.f) * (double)FIX_SCALE);
+		q = is_small_fixed(scaled) ? q : (unsigned long long)large;
+	}
+	return q;
 }
-__device__ __forceinline__ float from_fixed(unsigned long long q) { return (float)((double)(long long)q * (1.0 / 4294967296.0)); }
+__device__ __forceinline__ float from_fixed(unsigned long long q) {
+	return (float)fma((double)(int32_t)(q >> 32), 4294967296.0, (double)(uint32_t)q) * (1.f / FIX_SCALE);
+}
 
-// which (level, bucket, group of tiles) is this workgroup?  (Lane l asks about level l: sixteen scalar loads one after the other
-// were a microsecond of every workgroup.)
+// Which (level, bucket, group of tiles) is an item?  (Lane l asks about place l: sixteen scalar loads one after the other were a microsecond.)
 struct N2ReduceItem {
-	uint32_t level, bucket, group, groups, entries;  // entries per bucket: the level's own size (split buckets always have BKT_ENTRIES)
-	bool pair;
+	uint32_t bucket, group;
+	N2BucketPlan::Level l;
 };
-__device__ __forceinline__ N2ReduceItem n2_reduce_item(const N2LevelTable& tab, const N2BucketPlan& plan) {
+__device__ __forceinline__ uint32_t n2_lane_end(const N2BucketPlan& plan) {  // end of place `lane`
 	const uint32_t lane = threadIdx.x & 63u;
+	return lane < N2_MAX_LEVELS ? plan.begin[lane + 1u] : 0xFFFFFFFFu;
+}
+__device__ __forceinline__ N2ReduceItem n2_reduce_item(const N2BucketPlan& plan, uint32_t lane_end, uint32_t item) {
 	N2ReduceItem it;
-	it.level = __builtin_amdgcn_readfirstlane(__popcll(__ballot(lane < N2_MAX_LEVELS && blockIdx.x >= plan.wg_begin[min(lane, N2_MAX_LEVELS - 1u) + 1u])));
-	const uint32_t local = blockIdx.x - plan.wg_begin[it.level];
-	it.groups = plan.groups[it.level];
-	it.bucket = local / it.groups;
-	it.group = local - it.bucket * it.groups;
-	it.pair = (tab.pair_levels >> it.level) & 1u;
-	it.entries = it.pair ? BKT_ENTRIES : 1u << tab.bucket_shift[it.level];
-	// A tile's runs for neighbouring buckets meet inside a 128-byte line, which both buckets' workgroups fetch.  Workgroup
-	// ids are dealt round-robin over the XCDs: XCD x takes the x-th eighth of the level's buckets, in order, so that both
-	// fetches of such a line go through the same L2 at about the same time.
-	const uint32_t nb = plan.n_buckets[it.level];
-	if (it.groups == 1 && nb % N_XCD == 0) it.bucket = (blockIdx.x % N_XCD) * (nb / N_XCD) + local / N_XCD;
+	const uint32_t place = __popcll(__ballot(item >= lane_end)), local = item - plan.begin[place];
+	it.l = plan.at[place];
+	it.bucket = local;
+	it.group = 0u;
+	if (it.l.groups > 1u) {
+		it.bucket = __builtin_amdgcn_readfirstlane(local / it.l.groups);
+		it.group = local - it.bucket * it.l.groups;
+	} else if (it.l.n_buckets % N_XCD == 0u) {
+		// A tile's runs for neighbouring buckets meet inside a 128-byte line, which both buckets' workgroups fetch.  Workgroup
+		// ids are dealt round-robin over the XCDs (and an item's number is its workgroup's but for whole rounds of them): XCD x takes the x-th eighth
+		// of the level's buckets, in order, so that both fetches of such a line go through the same L2 at about the same time.
+		it.bucket = (item % N_XCD) * (it.l.n_buckets / N_XCD) + local / N_XCD;
+	}
 	return it;
 }
 
-// A bucket's runs: 2^run_lanes lanes take a tile's run (as many as hold its records in one step, on average), the workgroup's
-// groups of lanes take the tiles in turn.  A lane has FLIGHT records being added while the next FLIGHT are on their way.
-// (Cutting all runs into items listed in LDS, for an even load, costs a scan, a list and three more barriers in front of the
-// first record: 27 us against 17 for 5e3 points, where a workgroup's time is the chain of round trips, 33 against 25 for
-// 6.5e4, 39 against 33 for 1.2e5, 63 against 62 for 2^18.)
-template <bool PAIR, uint32_t FLIGHT>
-__device__ __forceinline__ void grid_reduce_runs(const uint32_t tiles, const uint32_t slot_records, const N2ReduceItem& it, const uint32_t run_lanes,
-                                                   const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
-                                                   const uint16_t* __restrict__ offsets, unsigned long long* acc) {
-	const uint32_t lanes = 1u << run_lanes, r = threadIdx.x & (lanes - 1u), group = threadIdx.x >> run_lanes, groups = RED_BLOCK >> run_lanes;
-	const size_t level_tile0 = (size_t)it.level * tiles;
-	const uint16_t* off = offsets + level_tile0 * (BKT_MAX + 1) + it.bucket;
-	const uint32_t step = groups * it.groups;  // (a split bucket's workgroup takes the tiles it.group, it.group + it.groups, ...)
-	// Where the next step's records are; the bounds of the run behind it are on their way, two 16-bit offsets as they lie in memory: taken apart
-	// where they are loaded, they were waited for there, and with them all records under way (2^18 uniform points 52.2 -> 50.5 us,
-	// a trained step 47 -> 44.6, 5003 points 17.1 -> 15.5; a training step in its initial state 55 before and after, the SDF network's 64.6).
-	uint32_t tile = group * it.groups + it.group, i, end;
-	auto bounds = [&](uint32_t t) {
-		uint32_t two;
-		__builtin_memcpy(&two, off + (size_t)min(t, tiles - 1u) * (BKT_MAX + 1), sizeof(two));
-		return two;
-	};
-	const uint32_t first = bounds(tile);
-	i = (first & 0xFFFFu) + r;
-	end = tile < tiles ? first >> 16 : 0u;
-	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
-	struct Step {
-		value v[FLIGHT];
-		uint32_t key[FLIGHT], n;  // n: records of this lane that count
-		uint32_t next;            // bounds of the run behind the one the next step begins with
-	};
-	auto load = [&](Step& q, uint32_t& next) {
-		// (lanes without a record read the level's first one: every load is issued, so the compiler can wait for one step only)
-		const uint32_t left = i < end ? (end - i + lanes - 1u) >> run_lanes : 0u;
-		q.n = left < FLIGHT ? left : FLIGHT;
-		const size_t slot = (level_tile0 + (tile < tiles ? tile : 0u)) * slot_records;
-#pragma unroll
-		for (uint32_t u = 0; u < FLIGHT; ++u) {
-			const uint32_t at = u < q.n ? i + u * lanes : 0u;
-			q.key[u] = rec_keys[slot + at];
-			if constexpr (PAIR) q.v[u] = reinterpret_cast<const uint2*>(rec_vals + slot)[at];
-			else q.v[u] = rec_vals[slot + at];
-		}
-		asm volatile("" : "+v"(next) : : "memory");  // (awaited behind the records' loads, not in front of them)
-		i += FLIGHT * lanes;
-		if (i - r >= end) {  // (the same for all lanes of the run) on to the next run
-			tile += step;
-			i = (next & 0xFFFFu) + r;
-			end = tile < tiles ? next >> 16 : 0u;
-		}
-		q.next = bounds(tile + step);
-	};
-	auto add = [&](const Step& q) {
-#pragma unroll
-		for (uint32_t u = 0; u < FLIGHT; ++u) {
-			if (u >= q.n) break;
-			if constexpr (PAIR) {
-				const uint32_t a1 = q.key[u] & (BKT_ENTRIES - 1u), a2 = a1 ^ ((2u << (q.key[u] >> BKT_SHIFT)) - 1u);  // x ^ (x + 1) = 2^(t+1) - 1
-				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&q.v[u].x)), g = __half22float2(*reinterpret_cast<const __half2*>(&q.v[u].y));
-				atomicAdd(&acc[a1], to_fixed(f.x));
-				atomicAdd(&acc[BKT_ENTRIES + a1], to_fixed(f.y));
-				atomicAdd(&acc[a2], to_fixed(g.x));
-				atomicAdd(&acc[BKT_ENTRIES + a2], to_fixed(g.y));
-			} else {
-				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&q.v[u]));
-				atomicAdd(&acc[q.key[u]], to_fixed(f.x));
-				atomicAdd(&acc[BKT_ENTRIES + q.key[u]], to_fixed(f.y));
-			}
-		}
-	};
-	Step qa, qb;
-	qb.next = bounds(tile + step);
-	ulonglong2* a2 = reinterpret_cast<ulonglong2*>(acc);
-	for (uint32_t e = threadIdx.x; e < it.entries / 2; e += RED_BLOCK) {
-		a2[e] = make_ulonglong2(0ull, 0ull);
-		a2[BKT_ENTRIES / 2 + e] = make_ulonglong2(0ull, 0ull);
-	}
-	const bool any = __any(tile < tiles);  // (of a small batch's waves some have no tile)
-	if (any) load(qa, qb.next);
-	__syncthreads();
-	while (any) {
-		const bool last_b = tile >= tiles;
-		load(qb, qa.next);
-		add(qa);
-		if (last_b) break;
-		const bool last_a = tile >= tiles;
-		load(qa, qb.next);
-		add(qb);
-		if (last_a) break;
-	}
-}
-
-// FLIGHT: 2 for batches of few tiles, whose runs rarely hold more.  Backward in us (device time in a graph), 4 | 2: the default table uniform 24 584 28.6 | 28.3, 28 672 29.5 | 29.0,
-// 32 768 30.4 | 29.9, along rays 24 584 26.4 | 25.9, 30 000 28.0 | 27.4, 32 768 29.2 | 28.4; tables of 2^16 entries a level, uniform 10 000 17.1 | 16.0, 16 384 19.5 | 20.3, 30 000 23.8 | 24.7, along
-// rays 10 000 14.4 | 13.2, 16 384 16.0 | 15.0, 30 000 21.4 | 20.8; of 2^14, uniform 5000 13.0 | 13.7, 30 000 30.4 | 32.3, along rays 3000 10.2 | 9.6, 30 000 29.0 | 30.6: no line on the tables' size
-// is right for either order.
-template <uint32_t FLIGHT>
-__global__ void __launch_bounds__(RED_BLOCK, 8) grid_reduce_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
-                                                                   const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
-                                                                   const uint16_t* __restrict__ offsets,
-                                                                   __half2* __restrict__ grads, int accumulate,
-                                                                   float2* __restrict__ partials) {
-	// one plane per feature: lanes of a wave's atomic then spread over all bank pairs (entry-major pairs of features would
-	// leave every other pair unused)
-	__shared__ __align__(16) unsigned long long acc[2 * BKT_ENTRIES];
-	const N2ReduceItem it = n2_reduce_item(tab, plan);
-	const uint32_t run_lanes = plan.run_lanes[it.level];
-	if (it.pair) grid_reduce_runs<true, FLIGHT>(tiles, slot_records, it, run_lanes, rec_vals, rec_keys, offsets, acc);
-	else grid_reduce_runs<false, FLIGHT>(tiles, slot_records, it, run_lanes, rec_vals, rec_keys, offsets, acc);
-	__syncthreads();
-	if (it.groups > 1) {
+// The sums of a bucket's records: out to the gradients, or as they are where the bucket is split, and back to zero.
+__device__ __forceinline__ void grid_reduce_out(const N2ReduceItem& it, unsigned long long* acc, __half2* __restrict__ grads, bool accumulate, float2* __restrict__ partials) {
+	ulonglong2* const wide_acc = reinterpret_cast<ulonglong2*>(acc);
+	const ulonglong2 none = make_ulonglong2(0ull, 0ull);
+	if (it.l.groups > 1u) {
 		// Several workgroups hold parts of this bucket's sums (coarse levels of large batches).  Each leaves its image as
 		// fp32 and grid_combine_kernel adds the G images up in the order of the groups: every entry is the same sum of the
 		// same terms in the same order however the workgroups were scheduled (the images themselves are exact integer sums).
-		float2* mine = partials + ((size_t)plan.part_begin[it.level] + (size_t)it.bucket * it.groups + it.group) * BKT_ENTRIES;
-		for (uint32_t e = threadIdx.x; e < BKT_ENTRIES; e += RED_BLOCK) mine[e] = make_float2(from_fixed(acc[e]), from_fixed(acc[BKT_ENTRIES + e]));
+		float2* mine = partials + ((size_t)it.l.part_begin + (size_t)it.bucket * it.l.groups + it.group) * BKT_ENTRIES;
+		for (uint32_t e = threadIdx.x; e < BKT_ENTRIES; e += RED_BLOCK) {
+			mine[e] = make_float2(from_fixed(acc[e]), from_fixed(acc[BKT_ENTRIES + e]));
+			acc[e] = acc[BKT_ENTRIES + e] = 0ull;
+		}
 		return;
 	}
 	// four entries (16 bytes) per lane: a level's table is whole multiples of eight entries and a bucket of 32
-	const uint32_t entries = tab.entries[it.level];
-	__half2* Gd = grads + tab.offset[it.level];
-	for (uint32_t e = threadIdx.x * 4u; e < it.entries; e += RED_BLOCK * 4u) {
-		const uint32_t idx = it.bucket * it.entries + e;
-		if (idx >= entries) break;
+	__half2* Gd = grads + it.l.offset;
+	for (uint32_t e = threadIdx.x * 4u; e < it.l.bucket_entries; e += RED_BLOCK * 4u) {
+		const uint32_t idx = it.bucket * it.l.bucket_entries + e;
+		if (idx >= it.l.entries) break;
 		typedef uint32_t wide __attribute__((ext_vector_type(4)));
 		wide* at = reinterpret_cast<wide*>(Gd + idx);
-		const wide old = accumulate ? *at : wide(0u);
+		float2 f[4];
+#pragma unroll
+		for (uint32_t q = 0; q < 4; q += 2) {
+			const ulonglong2 x = wide_acc[(e + q) / 2u], y = wide_acc[(BKT_ENTRIES + e + q) / 2u];
+			wide_acc[(e + q) / 2u] = wide_acc[(BKT_ENTRIES + e + q) / 2u] = none;
+			f[q] = make_float2(from_fixed(x.x), from_fixed(y.x));
+			f[q + 1u] = make_float2(from_fixed(x.y), from_fixed(y.y));
+		}
+		if (accumulate) {
+			const wide old = *at;
+#pragma unroll
+			for (uint32_t q = 0; q < 4; ++q) {
+				const uint32_t o = old[q];
+				const float2 g = __half22float2(*reinterpret_cast<const __half2*>(&o));
+				f[q] = make_float2(f[q].x + g.x, f[q].y + g.y);
+			}
+		}
 		wide out;
 #pragma unroll
 		for (uint32_t q = 0; q < 4; ++q) {
-			const uint32_t o = old[q];
-			float2 f = __half22float2(*reinterpret_cast<const __half2*>(&o));
-			f.x += from_fixed(acc[e + q]);
-			f.y += from_fixed(acc[BKT_ENTRIES + e + q]);
-			const __half2 h = __floats2half2_rn(f.x, f.y);
+			const __half2 h = __floats2half2_rn(f[q].x, f[q].y);
 			out[q] = *reinterpret_cast<const uint32_t*>(&h);
 		}
 		*at = out;
 	}
+}
+
+// A reduce launch's queue: a workgroup begins with the item of its own number and goes on with what it draws, for items differ by a factor of three in what
+// they take (dealt out by numbers alone, a training step's launch had its median workgroup end at 32 us and its last one at 46.9; drawn two ahead 34.2 and 43.6, so 34.5 and 40.9).
+// One counter for each XCD, in a line of its own; the sorting launch in front clears them.
+__device__ __forceinline__ uint32_t n2_queue_draw(uint32_t* queue) { return atomicAdd(queue + blockIdx.x % N_XCD * QUEUE_STRIDE, 1u); }
+__device__ __forceinline__ uint32_t n2_queue_item(uint32_t drawn) { return blockIdx.x % N_XCD + N_XCD * ((gridDim.x + N_XCD - 1u) / N_XCD + drawn); }  // (behind all first ones)
+
+// What a workgroup works on, as long as it is below `end` (all of one kind of records): `item`, then what it draws.  `acc` is all zeros before and after.
+//
+// Lane j of wave w takes run w + 16 j of the bucket's (a tile's run, or one of the 2^part_shift parts of it, so that a batch of few
+// tiles keeps all waves busy), and the wave walks through the records of its up to 64 runs as if they stood one behind the other, 64 at a time: which
+// runs the next 64 meet is the same question for the whole wave, so a run costs it two lane reads and three vector instructions, and every lane has a
+// record until the last.  FLIGHT times 64 records are being added while the next are on their way, the next item's first ones while this item's sums are written
+// (its bounds before that).
+template <bool PAIR, uint32_t FLIGHT>
+__device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, const uint32_t lane_end, uint32_t& item, const uint32_t end, const uint32_t tiles, const uint32_t slot_records,
+                                                  const uint32_t part_shift, const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
+                                                  const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, const bool accumulate, float2* __restrict__ partials,
+                                                  unsigned long long* acc, uint32_t* queue, uint32_t* drawn) {
+	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
+	constexpr uint32_t WAVES = RED_BLOCK / 64, STEP = 64u * FLIGHT;
+	if (item >= end) return;
+	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	N2ReduceItem it = n2_reduce_item(plan, lane_end, item);
+	// Of the wave's 64 runs at hand, lane j: the records up to the end of run j, and what takes a record's number among them to its place in the arrays.
+	uint32_t upto, place, total;
+	uint32_t at, k, k_upto, k_place;  // the next records begin at number `at`, in run k
+	const value* vals;
+	const uint16_t* keys;
+	auto rewind = [&]() __attribute__((always_inline)) {
+		at = k = 0u;
+		k_upto = (uint32_t)__builtin_amdgcn_readlane((int)upto, 0);
+		k_place = (uint32_t)__builtin_amdgcn_readlane((int)place, 0);
+	};
+	auto tile_of = [&](const N2ReduceItem& i, uint32_t run) { return min(i.group + i.l.groups * (run >> part_shift), tiles - 1u); };
+	auto bounds = [&](const N2ReduceItem& i, uint32_t first) __attribute__((always_inline)) {  // of the lane's run
+		uint32_t two;
+		__builtin_memcpy(&two, offsets + ((size_t)i.l.level * tiles + tile_of(i, first + WAVES * lane)) * (BKT_MAX + 1) + i.bucket, sizeof(two));
+		return two;
+	};
+	auto runs_of = [&](const N2ReduceItem& i) { return (i.l.groups == 1u ? tiles : (tiles - i.group + i.l.groups - 1u) / i.l.groups) << part_shift; };
+	auto take = [&](const N2ReduceItem& i, uint32_t first, uint32_t two) __attribute__((always_inline)) {
+		const uint32_t run = first + WAVES * lane, part = run & ((1u << part_shift) - 1u);
+		const uint32_t all = (two >> 16) - (two & 0xFFFFu), begin = all * part >> part_shift, stop = all * (part + 1u) >> part_shift;
+		const uint32_t n = run < runs_of(i) ? stop - begin : 0u;
+		upto = n2_wave_prefix(n);
+		place = tile_of(i, run) * (PAIR ? slot_records / 2u : slot_records) + (two & 0xFFFFu) + begin - (upto - n);
+		total = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+		const size_t level0 = (size_t)i.l.level * tiles * slot_records;
+		vals = reinterpret_cast<const value*>(rec_vals + level0);
+		keys = rec_keys + level0;
+		rewind();
+	};
+	struct Record {
+		value v;
+		uint32_t key;
+	};
+	auto load = [&](Record& q) __attribute__((always_inline)) {  // (behind the last record the last one is read again: all loads are issued, so a wait can be for one step's)
+		const uint32_t last = min(at + 63u, total - 1u), r = min(at + lane, total - 1u);
+		uint32_t p = k_place;
+		while (k_upto <= last) {  // (the last run ends at `total`)
+			const uint32_t below = k_upto;
+			++k;
+			k_upto = (uint32_t)__builtin_amdgcn_readlane((int)upto, (int)k);
+			k_place = (uint32_t)__builtin_amdgcn_readlane((int)place, (int)k);
+			p = r >= below ? k_place : p;
+		}
+		q.key = keys[r + p];
+		q.v = vals[r + p];
+		at += 64u;
+	};
+	auto load_step = [&](Record (&q)[FLIGHT]) __attribute__((always_inline)) {
+#pragma unroll
+		for (uint32_t u = 0; u < FLIGHT; ++u) load(q[u]);
+	};
+	// a record's places among the sums, and the two features of either
+	constexpr uint32_t EACH = PAIR ? 2u : 1u;
+	auto places = [&](const Record& q, unsigned long long* (&to)[EACH], __half2 (&h)[EACH]) __attribute__((always_inline)) {
+		const uint32_t a = q.key << 3;  // (bytes)
+		auto sum_at = [&](uint32_t bytes) { return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(acc) + bytes); };
+		if constexpr (PAIR) {
+			to[0] = sum_at(a & (BKT_ENTRIES - 1u) << 3);
+			to[1] = sum_at((a ^ ((16u << (q.key >> BKT_SHIFT)) - 8u)) & (BKT_ENTRIES - 1u) << 3);  // x ^ (x + 1) = 2^(t+1) - 1
+			h[0] = *reinterpret_cast<const __half2*>(&q.v.x);
+			h[1] = *reinterpret_cast<const __half2*>(&q.v.y);
+		} else {
+			to[0] = sum_at(a);
+			h[0] = *reinterpret_cast<const __half2*>(&q.v);
+		}
+	};
+	float most = 0.f;
+	auto add_step = [&](const Record (&q)[FLIGHT], uint32_t from) __attribute__((always_inline)) {
+#pragma unroll
+		for (uint32_t u = 0; u < FLIGHT; ++u) {
+			if (from + 64u * u + lane >= total) break;
+			unsigned long long* to[EACH];
+			__half2 h[EACH];
+			places(q[u], to, h);
+#pragma unroll
+			for (uint32_t e = 0; e < EACH; ++e) {
+				const float x = fmaf(__low2float(h[e]), FIX_SCALE, 0.f), y = fmaf(__high2float(h[e]), FIX_SCALE, 0.f);
+				most = fmaxf(fmaxf(fabsf(x), fabsf(y)), most);
+				atomicAdd(to[e], small_fixed(x));
+				atomicAdd(to[e] + BKT_ENTRIES, small_fixed(y));
+			}
+		}
+	};
+	Record qa[FLIGHT], qb[FLIGHT];
+	take(it, wave, bounds(it, wave));
+	if (total > 0u) load_step(qa);
+	__syncthreads();  // the sums are zero
+	while (true) {
+		uint32_t draw = 0u;
+		if (threadIdx.x == 0u) draw = n2_queue_draw(queue);
+		for (uint32_t first = wave;;) {
+			while (total > 0u) {
+				if (at >= total) {
+					add_step(qa, at - STEP);
+					break;
+				}
+				load_step(qb);
+				add_step(qa, at - 2u * STEP);
+				if (at >= total) {
+					add_step(qb, at - STEP);
+					break;
+				}
+				load_step(qa);
+				add_step(qb, at - 2u * STEP);
+			}
+			if (__any(!is_small_fixed(most))) {  // some values were cut: once more through the records, for what those lack
+				rewind();
+				while (at < total) {
+					Record q;
+					load(q);
+					if (at - 64u + lane >= total) break;
+					unsigned long long* to[EACH];
+					__half2 h[EACH];
+					places(q, to, h);
+#pragma unroll
+					for (uint32_t e = 0; e < EACH; ++e) {
+						const float2 f = __half22float2(h[e]);
+						atomicAdd(to[e], to_fixed(f.x) - small_fixed(f.x * FIX_SCALE));
+						atomicAdd(to[e] + BKT_ENTRIES, to_fixed(f.y) - small_fixed(f.y * FIX_SCALE));
+					}
+				}
+				most = 0.f;
+			}
+			first += WAVES * 64u;
+			if (first >= runs_of(it)) break;
+			take(it, first, bounds(it, first));
+			if (total > 0u) load_step(qa);
+		}
+		if (threadIdx.x == 0u) *drawn = draw;
+		__syncthreads();
+		item = n2_queue_item(__builtin_amdgcn_readfirstlane(*drawn));
+		const N2ReduceItem next = n2_reduce_item(plan, lane_end, min(item, end - 1u));
+		const uint32_t two = bounds(next, wave);
+		grid_reduce_out(it, acc, grads, accumulate, partials);
+		if (item < end) {
+			take(next, wave, two);
+			if (total > 0u) load_step(qa);
+		}
+		__syncthreads();
+		if (item >= end) return;
+		it = next;
+	}
+}
+
+// What bounds it is instructions and the records' way through memory, about half and half: without the LDS additions 2^18 uniform points take 45.6 of 50.4 us, with
+// records out of the L1 46.8, with neither 39.6, without writing the sums 44.9.  Before, one workgroup of 1024 threads to a bucket, groups of 8 or 16
+// lanes to a tile's run, values in 2^32 fixed point by five instructions each, | now, launch in us: a training step's 56.6 | 44.5, trained 44.8 | 41.1, the SDF network's
+// 63.9 | 56.5, 52 344 samples 20.0 | 18.0, 2^18 uniform points 50.6 | 50.7 (vector instructions 24.9 | 15.5 M).  Other shapes: 256 threads 59.8, 768 (two waves' records fewer
+// in flight) 50.6, 1024 (64 registers spill) 66.0; two, three or four times 64 records in flight 51.3, 50.7, 50.4; items dealt out by number 53.2, training step 51.0.
+__global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records, uint32_t part_shift,
+                                                                   const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
+                                                                   const uint16_t* __restrict__ offsets,
+                                                                   __half2* __restrict__ grads, int accumulate,
+                                                                   float2* __restrict__ partials, uint32_t* __restrict__ queue) {
+	// one plane per feature: lanes of a wave's atomic then spread over all bank pairs (entry-major pairs of features would
+	// leave every other pair unused)
+	__shared__ __align__(16) unsigned long long acc[2 * BKT_ENTRIES];
+	__shared__ uint32_t drawn;
+	const uint32_t lane_end = n2_lane_end(plan), items = plan.begin[N2_MAX_LEVELS];
+	for (uint32_t e = threadIdx.x; e < BKT_ENTRIES; e += RED_BLOCK) reinterpret_cast<ulonglong2*>(acc)[e] = make_ulonglong2(0ull, 0ull);
+	uint32_t item = blockIdx.x;
+	grid_reduce_items<false, 6>(plan, lane_end, item, plan.pairs_from, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, accumulate != 0, partials, acc, queue, &drawn);
+	grid_reduce_items<true, 3>(plan, lane_end, item, items, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, accumulate != 0, partials, acc, queue, &drawn);
 }
 
 // Small batches: the gradient of a bucket with few records.
@@ -1052,19 +1158,19 @@ struct N2FewRuns {
 };
 
 template <bool PAIR>
-__device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_records, const uint32_t tiles, const N2ReduceItem& it, const uint32_t entries,
+__device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_records, const uint32_t tiles, const N2ReduceItem& it,
                                                        const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
-                                                       const uint16_t* __restrict__ offsets, __half2* __restrict__ Gd, const bool accumulate, unsigned long long* mem) {
+                                                       const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, const bool accumulate, unsigned long long* mem) {
 	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
 	constexpr uint32_t EACH = PAIR ? 2u : 1u;                                               // entries of a record
 	constexpr uint32_t K = (FEW_CLAIMS / EACH + FEW_BLOCK - 1u) / FEW_BLOCK;  // records of a thread that may claim
-	const size_t level_tile0 = (size_t)it.level * tiles;
+	const size_t level_tile0 = (size_t)it.l.level * tiles;
 	const uint32_t lane = threadIdx.x & 63u;
 	uint32_t two;
 	__builtin_memcpy(&two, offsets + (level_tile0 + min(lane, tiles - 1u)) * (BKT_MAX + 1) + it.bucket, sizeof(two));
-	const uint32_t left = min(it.entries, entries - it.bucket * it.entries);  // entries of the bucket (a level's are a multiple of eight)
-	__half2* G = Gd + it.bucket * it.entries;
-	const bool claims = it.entries > FEW_RANGE;
+	const uint32_t left = min(it.l.bucket_entries, it.l.entries - it.bucket * it.l.bucket_entries);  // entries of the bucket (a level's are a multiple of eight)
+	__half2* G = grads + it.l.offset + it.bucket * it.l.bucket_entries;
+	const bool claims = it.l.bucket_entries > FEW_RANGE;
 	typedef uint32_t wide __attribute__((ext_vector_type(4)));
 	if (claims && !accumulate)
 		for (uint32_t e = threadIdx.x * 4u; e < left; e += FEW_BLOCK * 4u) *reinterpret_cast<wide*>(G + e) = wide(0u);
@@ -1076,9 +1182,10 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 	auto load = [&](uint32_t r, uint32_t& key, value& v) {
 		uint32_t tile, at;
 		runs.find(r, tile, at);
-		const size_t slot = (level_tile0 + tile) * slot_records + at;
-		key = rec_keys[slot];
-		v = reinterpret_cast<const value*>(rec_vals + (level_tile0 + tile) * slot_records)[at];
+		const size_t slot = level_tile0 * slot_records;
+		const uint32_t record = tile * (slot_records / EACH) + at;
+		key = rec_keys[slot + record];
+		v = reinterpret_cast<const value*>(rec_vals + slot)[record];
 	};
 	auto places = [&](uint32_t key, uint32_t (&e)[EACH]) {
 		if constexpr (PAIR) {
@@ -1178,15 +1285,13 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 	}
 }
 
-__global__ void __launch_bounds__(FEW_BLOCK, 8) grid_reduce_few_kernel(N2LevelTable tab, N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
+__global__ void __launch_bounds__(FEW_BLOCK, 8) grid_reduce_few_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
                                                                     const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                     const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, int accumulate) {
 	__shared__ __align__(16) unsigned long long mem[FEW_WORDS];
-	const N2ReduceItem it = n2_reduce_item(tab, plan);
-	__half2* Gd = grads + tab.offset[it.level];
-	const uint32_t entries = tab.entries[it.level];
-	if (it.pair) grid_reduce_few_bucket<true>(slot_records, tiles, it, entries, rec_vals, rec_keys, offsets, Gd, accumulate != 0, mem);
-	else grid_reduce_few_bucket<false>(slot_records, tiles, it, entries, rec_vals, rec_keys, offsets, Gd, accumulate != 0, mem);
+	const N2ReduceItem it = n2_reduce_item(plan, n2_lane_end(plan), blockIdx.x);
+	if (it.l.pair) grid_reduce_few_bucket<true>(slot_records, tiles, it, rec_vals, rec_keys, offsets, grads, accumulate != 0, mem);
+	else grid_reduce_few_bucket<false>(slot_records, tiles, it, rec_vals, rec_keys, offsets, grads, accumulate != 0, mem);
 }
 
 // Split buckets: the sum of a bucket's G partial images in a fixed order (n2_image_combine_unit, slab_reduce.h: with the
@@ -1502,17 +1607,18 @@ static bool bucket_supported(const n2_grid_t* grid) {
 		if (grid->tab.entries[l] > BKT_ENTRIES * BKT_MAX) return false;
 	return true;
 }
-// workspace: the records' values, their keys, the tiles' bucket offsets, then one fp32 image per (bucket, group) of the
+// workspace: the reduce launch's queue, the records' values, their keys, the tiles' bucket offsets, then one fp32 image per (bucket, group) of the
 // split buckets
 struct BucketCarve {
-	uint64_t vals, keys, offsets, partials, total;
+	uint64_t queue, vals, keys, offsets, partials, total;
 };
 static BucketCarve bucket_carve(const n2_grid_t* grid, uint32_t max_points, uint32_t images) {
 	const uint64_t tiles = n_bin_tiles(grid, max_points), L = grid->tab.n_levels;
 	const uint64_t n_rec = L * tiles * bin_records(bin_per_thread(grid, max_points));
 	auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
 	BucketCarve c{};
-	c.vals = 0;
+	c.queue = 0;
+	c.vals = QUEUE_WORDS * sizeof(uint32_t);
 	c.keys = c.vals + n_rec * sizeof(uint32_t);
 	c.offsets = c.keys + n_rec * sizeof(uint16_t);
 	c.partials = up(c.offsets + L * tiles * (BKT_MAX + 1) * sizeof(uint16_t));
@@ -1620,36 +1726,35 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	// The records of this batch are packed as for a workspace of exactly this size (values, keys, offsets one behind the
 	// other); the images of split buckets stand where the workspace's own size put them.
 	const BucketCarve now = bucket_carve(grid, n_points, 0u);
+	uint32_t* queue = reinterpret_cast<uint32_t*>(grid->ws + now.queue);
 	uint32_t* rec_vals = reinterpret_cast<uint32_t*>(grid->ws + now.vals);
 	uint16_t* rec_keys = reinterpret_cast<uint16_t*>(grid->ws + now.keys);
 	uint16_t* offsets = reinterpret_cast<uint16_t*>(grid->ws + now.offsets);
 	float2* partials = reinterpret_cast<float2*>(grid->ws + grid->ws_partials);
-	N2BucketPlan plan;
+	N2BucketPlan plan{};
 	uint32_t wg = 0, images = 0, split = 0;
 	N2LevelTable tab = grid->tab;  // with this launch's bucket sizes
-	const bool few = tiles <= FLIGHT_TILES;
+	uint32_t part_shift = 0;  // about four parts of runs per wave of a reduce workgroup
+	while (part_shift < 6u && tiles << part_shift < RED_BLOCK / 64u * 4u) ++part_shift;
 	const BatchBuckets buckets = batch_buckets(grid, n_points);
+	uint32_t split_begin[N2_MAX_LEVELS], part_begin[N2_MAX_LEVELS];
 	for (uint32_t l = 0; l < L; ++l) {
-		const uint32_t nb = buckets.count[l], groups = buckets.groups[l];
 		tab.bucket_shift[l] = buckets.shift[l];
-		plan.wg_begin[l] = wg;
-		plan.n_buckets[l] = nb;
-		plan.groups[l] = groups;
-		{
-			// lanes per run: with their records in flight, about the records a tile's run holds on average
-			const uint32_t per_run = (((tab.pair_levels >> l) & 1u) ? bin_records(per) / 2 : bin_records(per)) / nb;
-			uint32_t lanes = 4;  // (3 for tiles of one point per thread: 16.0 -> 16.8 us at 5003 points)
-			while (lanes < 10 && ((few ? 2u : 4u) << lanes) < per_run) ++lanes;
-			plan.run_lanes[l] = (uint8_t)lanes;
-		}
-		plan.part_begin[l] = images;
-		plan.split_begin[l] = split;
-		wg += nb * groups;
-		if (groups > 1) { images += nb * groups; split += nb; }
+		part_begin[l] = images;
+		split_begin[l] = split;
+		if (buckets.groups[l] > 1) { images += buckets.count[l] * buckets.groups[l]; split += buckets.count[l]; }
 	}
-	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.wg_begin[l] = wg;
-	for (uint32_t l = L; l < N2_MAX_LEVELS; ++l) { plan.n_buckets[l] = 0; plan.groups[l] = 1; plan.part_begin[l] = images; plan.run_lanes[l] = 0; }
-	for (uint32_t l = L; l <= N2_MAX_LEVELS; ++l) plan.split_begin[l] = split;
+	uint32_t place = 0;
+	for (uint32_t pair = 0; pair < 2; ++pair) {
+		if (pair) plan.pairs_from = wg;
+		for (uint32_t l = 0; l < L; ++l) {
+			if (((tab.pair_levels >> l) & 1u) != pair) continue;
+			plan.begin[place] = wg;
+			plan.at[place++] = {l, buckets.count[l], buckets.groups[l], part_begin[l], 1u << buckets.shift[l], tab.entries[l], tab.offset[l], pair};
+			wg += buckets.count[l] * buckets.groups[l];
+		}
+	}
+	for (; place <= N2_MAX_LEVELS; ++place) plan.begin[place] = wg;
 	auto bin = [&](auto per_thread) {
 		constexpr uint32_t PER = decltype(per_thread)::value;
 		// (the other launches' records exceed the card's memory before their threads exceed 32 bits: 8 and 9 threads a point of sixteen levels)
@@ -1659,7 +1764,7 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 			return dim3(g.x, g.y);
 		};
 #define LAUNCH(F, S, RIDE, BLOCKS) grid_bin_kernel<PER, F, S><<<launch_dim(RIDE, BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
-                                                                                                    grid->params, rec_vals, rec_keys, offsets, index, n_cols, RIDE)
+                                                                                                    grid->params, rec_vals, rec_keys, offsets, queue, index, n_cols, RIDE)
 		const uint32_t blocks = tiles * L;
 		const N2RideNone none;
 		if (rider.dL_dx != nullptr) {  // (first order alone)
@@ -1684,12 +1789,11 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	if (per == 1u) bin(std::integral_constant<uint32_t, 1>());
 	else bin(std::integral_constant<uint32_t, 2>());
 	N2_LAUNCH_CHECK();
-#define LAUNCH(F) grid_reduce_kernel<F><<<dim3(wg), dim3(RED_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0, partials)
 	if (buckets.few)
-		grid_reduce_few_kernel<<<dim3(wg), dim3(FEW_BLOCK), 0, s>>>(tab, plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
-	else if (few) LAUNCH(2);
-	else LAUNCH(4);
-#undef LAUNCH
+		grid_reduce_few_kernel<<<dim3(wg), dim3(FEW_BLOCK), 0, s>>>(plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
+	else
+		grid_reduce_kernel<<<dim3(wg < RED_AT_A_TIME ? wg : RED_AT_A_TIME), dim3(RED_BLOCK), 0, s>>>(plan, tiles, bin_records(per), part_shift, rec_vals, rec_keys, offsets, grid->grads,
+		                                                                                              accumulate ? 1 : 0, partials, queue);
 	N2_LAUNCH_CHECK();
 	if (split > 0) {
 		N2ImageCombine cmb{};
@@ -1699,9 +1803,9 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 		cmb.accumulate = accumulate ? 1 : 0;
 		uint32_t k = 0;  // the split levels, in order
 		for (uint32_t l = 0; l < L; ++l) {
-			if (plan.groups[l] <= 1) continue;
+			if (buckets.groups[l] <= 1) continue;
 			N2_REQUIRE(tab.bucket_shift[l] == BKT_SHIFT, "grid scatter: level %u splits buckets of %u entries", l, 1u << tab.bucket_shift[l]);
-			cmb.split_begin[k] = plan.split_begin[l]; cmb.groups[k] = plan.groups[l]; cmb.part_begin[k] = plan.part_begin[l];
+			cmb.split_begin[k] = split_begin[l]; cmb.groups[k] = buckets.groups[l]; cmb.part_begin[k] = part_begin[l];
 			cmb.entries[k] = grid->tab.entries[l]; cmb.offset[k] = grid->tab.offset[l];
 			++k;
 		}

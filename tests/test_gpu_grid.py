@@ -316,6 +316,46 @@ def test_sorted_scatter_batch_sizes(oracle, n):
             assert rel_l2(got[a:b], times * ref[a:b]) < RTOL, (mode, l)
 
 
+@pytest.mark.parametrize("n", [3, 200, 40000])  # the kernel for few records and the other one
+@pytest.mark.parametrize("levels,log2_size,base", [(1, 19, 16), (1, 16, 64), (1, 16, 37), (2, 19, 16)])  # dense, hashed, a number of buckets that is no multiple of eight
+def test_sorted_scatter_is_exact_for_values_of_all_sizes(n, levels, log2_size, base):
+    """Points in the middle of their cells: every record is dL_dy / 8, exactly, and the sums are exact until they are rounded, from the smallest fp16
+    values to those above 128 that do not fit the short form; infinite values stay infinite, values that are no number count as zero."""
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(n_levels=levels, log2_hashmap_size=log2_size, base_resolution=base, per_level_scale=1.0)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = torch.zeros(gg.n_params(), device="cuda").half()
+    dg = torch.full_like(dp, 5.0)
+    gg.set_params(dp, dg)
+    assert gg.reserve_scatter_workspace(n)
+    x = torch.randint(0, base - 1, (3, n), device="cuda", generator=gen).float() / (base - 1)
+    size = torch.randint(-18, 9, (2 * levels, n), device="cuda", generator=gen)
+    size = torch.where(torch.rand(size.shape, device="cuda", generator=gen) < 0.02, size + 5, size)
+    dy = torch.ldexp(torch.randint(-7, 8, size.shape, device="cuda", generator=gen).float(), size)  # (multiples of 2^-18, up to 7 * 2^13)
+    dy[0, 0] = float("inf")
+    dy[1, n // 2] = float("nan")
+    dy = dy.half()
+    at = gg.corner_indices(x).long()
+    offsets = gg.level_table()[3]
+    want = torch.zeros((dg.numel() // 2, 2), device="cuda", dtype=torch.float64)
+    special = torch.zeros_like(want)
+    for l in range(levels):
+        for f in range(2):
+            rec = (dy[2 * l + f].double() / 8)
+            special[:, f].index_add_(0, at[l].reshape(-1) + int(offsets[l]), rec.isinf().double().repeat(8))
+            rec = torch.where(rec.isfinite(), rec, 0.0)
+            want[:, f].index_add_(0, at[l].reshape(-1) + int(offsets[l]), rec.repeat(8))
+    for mode, times in ((GRAD_OVERWRITE, 1), (GRAD_ACCUMULATE, 2)):
+        gg.backward(None, x, dy, mode=mode)
+        got = dg.reshape(-1, 2)
+        once = want.float().half()
+        ref = once if times == 1 else (want.float() + once.float()).half()
+        ref = torch.where(special > 0, float("inf"), ref.float()).half()
+        skip = torch.isinf(once) & (special == 0) if times == 2 else torch.zeros_like(special, dtype=torch.bool)
+        bad = (got != ref) & ~skip
+        assert not bad.any(), (mode, int(bad.sum()), got[bad][:4], ref[bad][:4], want[bad][:4])
+
+
 @pytest.mark.parametrize("n,room", [(512, 512), (513, 513), (513, 70000), (16384, 16384), (16384, 16385)])
 def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     """The sums are exact, so the size of a tile leaves no trace: a batch equals the one that has points without a gradient behind it, up to where
