@@ -843,20 +843,15 @@ constexpr uint32_t RED_BLOCK = 512;               // 8 waves; two workgroups sha
 constexpr uint32_t RED_AT_A_TIME = 512;           // workgroups of a launch: what runs at one time (a multiple of the XCDs)
 constexpr float FIX_SCALE = 16777216.0f;          // 2^24
 
-// x * 2^24 as a two's complement 64-bit integer, for |x| < 128, given that product, which has 32 bits then: two instructions.  Beyond, it is cut to 32 bits;
-// no number gives zero.
-__device__ __forceinline__ unsigned long long small_fixed(float scaled) { return (unsigned long long)(long long)(int32_t)scaled; }
-__device__ __forceinline__ bool is_small_fixed(float scaled) { return !(fabsf(scaled) >= 2147483648.f); }
-// For any fp16 value.  An infinite one counts as 2^22: 65536 of them stay inside 64 bits, and one of them is infinite again as fp16.
-__device__ __forceinline__ unsigned long long to_fixed(float x) {
-	const float scaled = x * FIX_SCALE;
-	unsigned long long q = small_fixed(scaled);
-	if (__any(!is_small_fixed(scaled))) {  // (six times as long)
-		const long long large = (long long)((double)fminf(fmaxf(x, -4194304.f), 4194304.f) * (double)FIX_SCALE);
-		q = is_small_fixed(scaled) ? q : (unsigned long long)large;
-	}
-	return q;
+// x * 2^24 as a two's complement 64-bit integer, given that product (of an fp16 value, so it is a whole number).  For |x| < 128 it has 32 bits: two instructions.
+__device__ __forceinline__ unsigned long long fixed_small(float scaled) { return (unsigned long long)(long long)(int32_t)scaled; }
+__device__ __forceinline__ bool is_fixed_small(float scaled) { return fabsf(scaled) < 2147483648.f; }
+// Up to 2^51: added to 3 * 2^51 it stands in the sum's low bits.
+__device__ __forceinline__ unsigned long long fixed_large(float scaled) {
+	return __builtin_bit_cast(unsigned long long, (double)scaled + 6755399441055744.0) - 0x4338000000000000ull;
 }
+// What is not finite, for fixed_large: an infinite value counts as 2^22, which 65536 of stay inside 64 bits and one of is infinite again as fp16; no number as zero.
+__device__ __forceinline__ float fixed_bounded(float scaled) { return scaled != scaled ? 0.f : fminf(fmaxf(scaled, -70368744177664.f), 70368744177664.f); }
 __device__ __forceinline__ float from_fixed(unsigned long long q) {
 	return (float)fma((double)(int32_t)(q >> 32), 4294967296.0, (double)(uint32_t)q) * (1.f / FIX_SCALE);
 }
@@ -888,8 +883,21 @@ __device__ __forceinline__ N2ReduceItem n2_reduce_item(const N2BucketPlan& plan,
 	return it;
 }
 
+// The gradients of a bucket that a lane writes, four entries (16 bytes) at a time: a level's table is whole multiples of eight entries and a bucket of 32.  An
+// accumulating launch has their old values under way before the last records are added.  (Loaded where they are added they were a trip to memory each, of four in
+// a workgroup's life: forward, backward and second order of 180 000 points 214 -> 245 us.)
+constexpr uint32_t RED_WRITES = BKT_ENTRIES / (RED_BLOCK * 4u);
+static_assert(RED_WRITES * RED_BLOCK * 4u == BKT_ENTRIES, "a bucket is whole rounds of a workgroup");
+typedef uint32_t n2_four_entries __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void grid_reduce_old(const N2ReduceItem& it, const __half2* __restrict__ grads, n2_four_entries (&old)[RED_WRITES]) {
+#pragma unroll
+	for (uint32_t k = 0; k < RED_WRITES; ++k)
+		old[k] = *reinterpret_cast<const n2_four_entries*>(grads + it.l.offset + min(it.bucket * it.l.bucket_entries + (k * RED_BLOCK + threadIdx.x) * 4u, it.l.entries - 4u));
+}
 // The sums of a bucket's records: out to the gradients, or as they are where the bucket is split, and back to zero.
-__device__ __forceinline__ void grid_reduce_out(const N2ReduceItem& it, unsigned long long* acc, __half2* __restrict__ grads, bool accumulate, float2* __restrict__ partials) {
+template <bool ACCUMULATE>
+__device__ __forceinline__ void grid_reduce_out(const N2ReduceItem& it, unsigned long long* acc, __half2* __restrict__ grads, const n2_four_entries (&old)[RED_WRITES],
+                                                float2* __restrict__ partials) {
 	ulonglong2* const wide_acc = reinterpret_cast<ulonglong2*>(acc);
 	const ulonglong2 none = make_ulonglong2(0ull, 0ull);
 	if (it.l.groups > 1u) {
@@ -903,37 +911,29 @@ __device__ __forceinline__ void grid_reduce_out(const N2ReduceItem& it, unsigned
 		}
 		return;
 	}
-	// four entries (16 bytes) per lane: a level's table is whole multiples of eight entries and a bucket of 32
 	__half2* Gd = grads + it.l.offset;
-	for (uint32_t e = threadIdx.x * 4u; e < it.l.bucket_entries; e += RED_BLOCK * 4u) {
-		const uint32_t idx = it.bucket * it.l.bucket_entries + e;
-		if (idx >= it.l.entries) break;
-		typedef uint32_t wide __attribute__((ext_vector_type(4)));
-		wide* at = reinterpret_cast<wide*>(Gd + idx);
-		float2 f[4];
+#pragma unroll
+	for (uint32_t k = 0; k < RED_WRITES; ++k) {
+		const uint32_t e = (k * RED_BLOCK + threadIdx.x) * 4u, idx = it.bucket * it.l.bucket_entries + e;
+		if (e >= it.l.bucket_entries || idx >= it.l.entries) break;
+		n2_four_entries out;
 #pragma unroll
 		for (uint32_t q = 0; q < 4; q += 2) {
 			const ulonglong2 x = wide_acc[(e + q) / 2u], y = wide_acc[(BKT_ENTRIES + e + q) / 2u];
 			wide_acc[(e + q) / 2u] = wide_acc[(BKT_ENTRIES + e + q) / 2u] = none;
-			f[q] = make_float2(from_fixed(x.x), from_fixed(y.x));
-			f[q + 1u] = make_float2(from_fixed(x.y), from_fixed(y.y));
-		}
-		if (accumulate) {
-			const wide old = *at;
 #pragma unroll
-			for (uint32_t q = 0; q < 4; ++q) {
-				const uint32_t o = old[q];
-				const float2 g = __half22float2(*reinterpret_cast<const __half2*>(&o));
-				f[q] = make_float2(f[q].x + g.x, f[q].y + g.y);
+			for (uint32_t p = 0; p < 2; ++p) {
+				float2 f = make_float2(from_fixed(p ? x.y : x.x), from_fixed(p ? y.y : y.x));
+				if (ACCUMULATE) {
+					const uint32_t o = old[k][q + p];
+					const float2 g = __half22float2(*reinterpret_cast<const __half2*>(&o));
+					f = make_float2(f.x + g.x, f.y + g.y);
+				}
+				const __half2 h = __floats2half2_rn(f.x, f.y);
+				out[q + p] = *reinterpret_cast<const uint32_t*>(&h);
 			}
 		}
-		wide out;
-#pragma unroll
-		for (uint32_t q = 0; q < 4; ++q) {
-			const __half2 h = __floats2half2_rn(f[q].x, f[q].y);
-			out[q] = *reinterpret_cast<const uint32_t*>(&h);
-		}
-		*at = out;
+		*reinterpret_cast<n2_four_entries*>(Gd + idx) = out;
 	}
 }
 
@@ -950,10 +950,10 @@ __device__ __forceinline__ uint32_t n2_queue_item(uint32_t drawn) { return block
 // runs the next 64 meet is the same question for the whole wave, so a run costs it two lane reads and three vector instructions, and every lane has a
 // record until the last.  FLIGHT times 64 records are being added while the next are on their way, the next item's first ones while this item's sums are written
 // (its bounds before that).
-template <bool PAIR, uint32_t FLIGHT>
+template <bool PAIR, uint32_t FLIGHT, bool ACCUMULATE>
 __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, const uint32_t lane_end, uint32_t& item, const uint32_t end, const uint32_t tiles, const uint32_t slot_records,
                                                   const uint32_t part_shift, const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
-                                                  const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, const bool accumulate, float2* __restrict__ partials,
+                                                  const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, float2* __restrict__ partials,
                                                   unsigned long long* acc, uint32_t* queue, uint32_t* drawn) {
 	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
 	constexpr uint32_t WAVES = RED_BLOCK / 64, STEP = 64u * FLIGHT;
@@ -965,11 +965,6 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 	uint32_t at, k, k_upto, k_place;  // the next records begin at number `at`, in run k
 	const value* vals;
 	const uint16_t* keys;
-	auto rewind = [&]() __attribute__((always_inline)) {
-		at = k = 0u;
-		k_upto = (uint32_t)__builtin_amdgcn_readlane((int)upto, 0);
-		k_place = (uint32_t)__builtin_amdgcn_readlane((int)place, 0);
-	};
 	auto tile_of = [&](const N2ReduceItem& i, uint32_t run) { return min(i.group + i.l.groups * (run >> part_shift), tiles - 1u); };
 	auto bounds = [&](const N2ReduceItem& i, uint32_t first) __attribute__((always_inline)) {  // of the lane's run
 		uint32_t two;
@@ -987,7 +982,9 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 		const size_t level0 = (size_t)i.l.level * tiles * slot_records;
 		vals = reinterpret_cast<const value*>(rec_vals + level0);
 		keys = rec_keys + level0;
-		rewind();
+		at = k = 0u;
+		k_upto = (uint32_t)__builtin_amdgcn_readlane((int)upto, 0);
+		k_place = (uint32_t)__builtin_amdgcn_readlane((int)place, 0);
 	};
 	struct Record {
 		value v;
@@ -1011,37 +1008,46 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 #pragma unroll
 		for (uint32_t u = 0; u < FLIGHT; ++u) load(q[u]);
 	};
-	// a record's places among the sums, and the two features of either
-	constexpr uint32_t EACH = PAIR ? 2u : 1u;
-	auto places = [&](const Record& q, unsigned long long* (&to)[EACH], __half2 (&h)[EACH]) __attribute__((always_inline)) {
-		const uint32_t a = q.key << 3;  // (bytes)
-		auto sum_at = [&](uint32_t bytes) { return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(acc) + bytes); };
-		if constexpr (PAIR) {
-			to[0] = sum_at(a & (BKT_ENTRIES - 1u) << 3);
-			to[1] = sum_at((a ^ ((16u << (q.key >> BKT_SHIFT)) - 8u)) & (BKT_ENTRIES - 1u) << 3);  // x ^ (x + 1) = 2^(t+1) - 1
-			h[0] = *reinterpret_cast<const __half2*>(&q.v.x);
-			h[1] = *reinterpret_cast<const __half2*>(&q.v.y);
-		} else {
-			to[0] = sum_at(a);
-			h[0] = *reinterpret_cast<const __half2*>(&q.v);
-		}
-	};
-	float most = 0.f;
+	constexpr uint32_t EACH = PAIR ? 2u : 1u;  // entries of a record
 	auto add_step = [&](const Record (&q)[FLIGHT], uint32_t from) __attribute__((always_inline)) {
+		float f[FLIGHT][2 * EACH], most = 0.f;  // (of lanes behind the last record those of the last one)
 #pragma unroll
-		for (uint32_t u = 0; u < FLIGHT; ++u) {
-			if (from + 64u * u + lane >= total) break;
-			unsigned long long* to[EACH];
-			__half2 h[EACH];
-			places(q[u], to, h);
+		for (uint32_t u = 0; u < FLIGHT; ++u)
 #pragma unroll
 			for (uint32_t e = 0; e < EACH; ++e) {
-				const float x = fmaf(__low2float(h[e]), FIX_SCALE, 0.f), y = fmaf(__high2float(h[e]), FIX_SCALE, 0.f);
-				most = fmaxf(fmaxf(fabsf(x), fabsf(y)), most);
-				atomicAdd(to[e], small_fixed(x));
-				atomicAdd(to[e] + BKT_ENTRIES, small_fixed(y));
+				uint32_t raw;
+				if constexpr (PAIR) raw = e ? q[u].v.y : q[u].v.x;
+				else raw = q[u].v;
+				const __half2 h = *reinterpret_cast<const __half2*>(&raw);
+				f[u][2 * e] = fmaf(__low2float(h), FIX_SCALE, 0.f);
+				f[u][2 * e + 1] = fmaf(__high2float(h), FIX_SCALE, 0.f);
+				most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(f[u][2 * e]), fabsf(f[u][2 * e + 1])), most);  // (no number where one is none)
 			}
-		}
+		auto add = [&](auto fixed) __attribute__((always_inline)) {
+#pragma unroll
+			for (uint32_t u = 0; u < FLIGHT; ++u) {
+				if (from + 64u * u + lane >= total) break;
+				const uint32_t a = q[u].key << 3;  // (bytes into a plane of sums)
+				auto sum_at = [&](uint32_t bytes) { return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(acc) + bytes); };
+				unsigned long long* to[EACH];
+				to[0] = sum_at(PAIR ? a & (BKT_ENTRIES - 1u) << 3 : a);
+				if constexpr (PAIR) to[1] = sum_at((a ^ ((16u << (q[u].key >> BKT_SHIFT)) - 8u)) & (BKT_ENTRIES - 1u) << 3);  // x ^ (x + 1) = 2^(t+1) - 1
+#pragma unroll
+				for (uint32_t e = 0; e < EACH; ++e) {
+					atomicAdd(to[e], fixed(f[u][2 * e]));
+					atomicAdd(to[e] + BKT_ENTRIES, fixed(f[u][2 * e + 1]));
+				}
+			}
+		};
+		if (__any(!is_fixed_small(most))) {
+			if (__any(!(most < FIX_SCALE * 65536.f))) {
+#pragma unroll
+				for (uint32_t u = 0; u < FLIGHT; ++u)
+#pragma unroll
+					for (uint32_t e = 0; e < 2 * EACH; ++e) f[u][e] = fixed_bounded(f[u][e]);
+			}
+			add([](float x) { return fixed_large(x); });
+		} else add([](float x) { return fixed_small(x); });
 	};
 	Record qa[FLIGHT], qb[FLIGHT];
 	take(it, wave, bounds(it, wave));
@@ -1065,35 +1071,19 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 				load_step(qa);
 				add_step(qb, at - 2u * STEP);
 			}
-			if (__any(!is_small_fixed(most))) {  // some values were cut: once more through the records, for what those lack
-				rewind();
-				while (at < total) {
-					Record q;
-					load(q);
-					if (at - 64u + lane >= total) break;
-					unsigned long long* to[EACH];
-					__half2 h[EACH];
-					places(q, to, h);
-#pragma unroll
-					for (uint32_t e = 0; e < EACH; ++e) {
-						const float2 f = __half22float2(h[e]);
-						atomicAdd(to[e], to_fixed(f.x) - small_fixed(f.x * FIX_SCALE));
-						atomicAdd(to[e] + BKT_ENTRIES, to_fixed(f.y) - small_fixed(f.y * FIX_SCALE));
-					}
-				}
-				most = 0.f;
-			}
 			first += WAVES * 64u;
 			if (first >= runs_of(it)) break;
 			take(it, first, bounds(it, first));
 			if (total > 0u) load_step(qa);
 		}
+		n2_four_entries old[RED_WRITES];
+		if (ACCUMULATE) grid_reduce_old(it, grads, old);
 		if (threadIdx.x == 0u) *drawn = draw;
 		__syncthreads();
 		item = n2_queue_item(__builtin_amdgcn_readfirstlane(*drawn));
 		const N2ReduceItem next = n2_reduce_item(plan, lane_end, min(item, end - 1u));
 		const uint32_t two = bounds(next, wave);
-		grid_reduce_out(it, acc, grads, accumulate, partials);
+		grid_reduce_out<ACCUMULATE>(it, acc, grads, old, partials);
 		if (item < end) {
 			take(next, wave, two);
 			if (total > 0u) load_step(qa);
@@ -1109,11 +1099,13 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 // lanes to a tile's run, values in 2^32 fixed point by five instructions each, | now, launch in us: a training step's 56.6 | 44.5, trained 44.8 | 41.1, the SDF network's
 // 63.9 | 56.5, 52 344 samples 20.0 | 18.0, 2^18 uniform points 50.6 | 50.7 (vector instructions 24.9 | 15.5 M).  Other shapes: 256 threads 59.8, 768 (two waves' records fewer
 // in flight) 50.6, 1024 (64 registers spill) 66.0; two, three or four times 64 records in flight 51.3, 50.7, 50.4; items dealt out by number 53.2, training step 51.0.
+// Values from 128 on (a second order's, whose J holds the level's scale) take an instruction more, chosen for a wave's step as a whole: second order and both others on 60 000
+// points along rays 100.0 -> 95.7, 2^18 287 -> 285.  Points packed into a fifth of the cube's side lose 3 to 5 per cent: a few full buckets, with half the threads to each.
+template <bool ACCUMULATE>
 __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records, uint32_t part_shift,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                    const uint16_t* __restrict__ offsets,
-                                                                   __half2* __restrict__ grads, int accumulate,
-                                                                   float2* __restrict__ partials, uint32_t* __restrict__ queue) {
+                                                                   __half2* __restrict__ grads, float2* __restrict__ partials, uint32_t* __restrict__ queue) {
 	// one plane per feature: lanes of a wave's atomic then spread over all bank pairs (entry-major pairs of features would
 	// leave every other pair unused)
 	__shared__ __align__(16) unsigned long long acc[2 * BKT_ENTRIES];
@@ -1121,8 +1113,8 @@ __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan 
 	const uint32_t lane_end = n2_lane_end(plan), items = plan.begin[N2_MAX_LEVELS];
 	for (uint32_t e = threadIdx.x; e < BKT_ENTRIES; e += RED_BLOCK) reinterpret_cast<ulonglong2*>(acc)[e] = make_ulonglong2(0ull, 0ull);
 	uint32_t item = blockIdx.x;
-	grid_reduce_items<false, 6>(plan, lane_end, item, plan.pairs_from, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, accumulate != 0, partials, acc, queue, &drawn);
-	grid_reduce_items<true, 3>(plan, lane_end, item, items, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, accumulate != 0, partials, acc, queue, &drawn);
+	grid_reduce_items<false, 6, ACCUMULATE>(plan, lane_end, item, plan.pairs_from, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, queue, &drawn);
+	grid_reduce_items<true, 3, ACCUMULATE>(plan, lane_end, item, items, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, queue, &drawn);
 }
 
 // Small batches: the gradient of a bucket with few records.
@@ -1134,13 +1126,26 @@ __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan 
 // match a tile's run.  Levels of few entries keep an image, as does (range by range) a bucket with more records than
 // there are sums to claim.  What bounds it is the chain level -> bounds -> records -> sums and the 25 MB the gradient's zeros take.
 // Launch in us, image -> claims: 600 uniform points 15 -> 10.1, 5003 along rays 15.1 -> 10.6 (accumulating 15.6 -> 9.5), training step of 2^14 samples 17.5 -> 14.8.
-// (256 threads: the same up to 5000 points, 16 384 uniform points +4; 1024: +4; 128: +0.5.  In 32 KiB there are 1536 sums instead of 2048,
+// (256 threads: the same up to 5000 points, 16 384 uniform +4; 1024: +4; 128: +0.5.  In 32 KiB there are 1536 sums instead of 2048,
 // and batches beyond 16 384 points took grid_reduce_kernel: 20 000 along rays 34.0 against 29.5.)
+// With the next item's bounds on their way meanwhile (its level and tiles looked up behind the last item's stores before): forward, backward and second order, 1000
+// points along rays 32.4 -> 30.3, 2000 33.7 -> 31.3, 5003 36.2 -> 35.2, uniform 42.7 -> 41.4; points packed into a twentieth of the cube 51.8 -> 53.4.  Half the sums and threads, seven
+// workgroups to a CU: 5003 along rays 32.6, but 6000 points of a cube's fifth 17.7 -> 31.9, whose buckets hold more records than there are sums then.
 constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 5120;
+constexpr uint32_t FEW_AT_A_TIME = 1024;                            // workgroups of a launch: what runs at one time (a multiple of the XCDs)
 constexpr uint32_t FEW_TILES = 64;                                  // a lane of every wave looks up one tile's run
 constexpr uint32_t FEW_CLAIMS = (FEW_WORDS - BKT_ENTRIES / 4) / 2;  // sums of both features, beside the table of 16-bit claims
 constexpr uint32_t FEW_RANGE = FEW_WORDS / 2;                       // entries of an image
 constexpr uint32_t FEW_PAIRS = 768;                                 // pair records of a bucket, on average, in a batch that takes the kernel (batch_buckets)
+
+// Here x * 2^32 as a two's complement 64-bit integer, for any fp16 value x: the high word is floor(x), the low word the rest, both exact.  (Five instructions and no
+// branch, whatever the value: a few records a thread, whose latency counts.)
+__device__ __forceinline__ unsigned long long few_to_fixed(float x) {
+	const float fl = floorf(x);
+	const uint32_t hi = (uint32_t)(int32_t)fl, lo = (uint32_t)((x - fl) * 4294967296.f);
+	return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ float few_from_fixed(unsigned long long q) { return from_fixed(q) * (FIX_SCALE / 4294967296.f); }
 
 // A bucket's records, numbered through its tiles' runs.
 struct N2FewRuns {
@@ -1160,14 +1165,12 @@ struct N2FewRuns {
 template <bool PAIR>
 __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_records, const uint32_t tiles, const N2ReduceItem& it,
                                                        const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
-                                                       const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, const bool accumulate, unsigned long long* mem) {
+                                                       const uint32_t two, __half2* __restrict__ grads, const bool accumulate, unsigned long long* mem) {
 	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
 	constexpr uint32_t EACH = PAIR ? 2u : 1u;                                               // entries of a record
 	constexpr uint32_t K = (FEW_CLAIMS / EACH + FEW_BLOCK - 1u) / FEW_BLOCK;  // records of a thread that may claim
 	const size_t level_tile0 = (size_t)it.l.level * tiles;
 	const uint32_t lane = threadIdx.x & 63u;
-	uint32_t two;
-	__builtin_memcpy(&two, offsets + (level_tile0 + min(lane, tiles - 1u)) * (BKT_MAX + 1) + it.bucket, sizeof(two));
 	const uint32_t left = min(it.l.bucket_entries, it.l.entries - it.bucket * it.l.bucket_entries);  // entries of the bucket (a level's are a multiple of eight)
 	__half2* G = grads + it.l.offset + it.bucket * it.l.bucket_entries;
 	const bool claims = it.l.bucket_entries > FEW_RANGE;
@@ -1199,7 +1202,7 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 	};
 	auto sum_of = [&](uint32_t old, unsigned long long a, unsigned long long b) {
 		float2 f = accumulate ? __half22float2(*reinterpret_cast<const __half2*>(&old)) : make_float2(0.f, 0.f);
-		return __floats2half2_rn(f.x + from_fixed(a), f.y + from_fixed(b));
+		return __floats2half2_rn(f.x + few_from_fixed(a), f.y + few_from_fixed(b));
 	};
 	if (claims && runs.total * EACH <= FEW_CLAIMS) {
 		uint16_t* claim = reinterpret_cast<uint16_t*>(mem);
@@ -1232,8 +1235,8 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 				by[k][q] = claim[e[k][q]];
 				const uint32_t raw = word(v[k], q);
 				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
-				atomicAdd(&acc[by[k][q]], to_fixed(f.x));
-				atomicAdd(&acc[FEW_CLAIMS + by[k][q]], to_fixed(f.y));
+				atomicAdd(&acc[by[k][q]], few_to_fixed(f.x));
+				atomicAdd(&acc[FEW_CLAIMS + by[k][q]], few_to_fixed(f.y));
 				old[k][q] = accumulate && by[k][q] == (threadIdx.x + k * FEW_BLOCK) * EACH + q && e[k][q] < left ? *reinterpret_cast<const uint32_t*>(G + e[k][q]) : 0u;
 			}
 		}
@@ -1265,8 +1268,8 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 				const uint32_t at = e[q] - from, raw = word(v, q);
 				if (r >= runs.total || at >= n) continue;
 				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
-				atomicAdd(&mem[at], to_fixed(f.x));
-				atomicAdd(&mem[FEW_RANGE + at], to_fixed(f.y));
+				atomicAdd(&mem[at], few_to_fixed(f.x));
+				atomicAdd(&mem[FEW_RANGE + at], few_to_fixed(f.y));
 			}
 		}
 		__syncthreads();
@@ -1285,13 +1288,31 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 	}
 }
 
+// A workgroup takes the items of its number, that and a round of workgroups further, ...; where the next one's runs lie is on its way meanwhile.
 __global__ void __launch_bounds__(FEW_BLOCK, 8) grid_reduce_few_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
                                                                     const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                     const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, int accumulate) {
 	__shared__ __align__(16) unsigned long long mem[FEW_WORDS];
-	const N2ReduceItem it = n2_reduce_item(plan, n2_lane_end(plan), blockIdx.x);
-	if (it.l.pair) grid_reduce_few_bucket<true>(slot_records, tiles, it, rec_vals, rec_keys, offsets, grads, accumulate != 0, mem);
-	else grid_reduce_few_bucket<false>(slot_records, tiles, it, rec_vals, rec_keys, offsets, grads, accumulate != 0, mem);
+	const uint32_t lane_end = n2_lane_end(plan), items = plan.begin[N2_MAX_LEVELS], lane = threadIdx.x & 63u;
+	auto bounds = [&](const N2ReduceItem& it) __attribute__((always_inline)) {  // of the bucket's run in tile `lane`
+		uint32_t two;
+		__builtin_memcpy(&two, offsets + ((size_t)it.l.level * tiles + min(lane, tiles - 1u)) * (BKT_MAX + 1) + it.bucket, sizeof(two));
+		return two;
+	};
+	N2ReduceItem it = n2_reduce_item(plan, lane_end, blockIdx.x);
+	uint32_t two = bounds(it);
+	for (uint32_t item = blockIdx.x;;) {
+		const uint32_t next = item + gridDim.x;
+		const N2ReduceItem next_it = n2_reduce_item(plan, lane_end, min(next, items - 1u));
+		const uint32_t next_two = bounds(next_it);
+		if (it.l.pair) grid_reduce_few_bucket<true>(slot_records, tiles, it, rec_vals, rec_keys, two, grads, accumulate != 0, mem);
+		else grid_reduce_few_bucket<false>(slot_records, tiles, it, rec_vals, rec_keys, two, grads, accumulate != 0, mem);
+		if (next >= items) return;
+		__syncthreads();  // the sums have been read
+		item = next;
+		it = next_it;
+		two = next_two;
+	}
 }
 
 // Split buckets: the sum of a bucket's G partial images in a fixed order (n2_image_combine_unit, slab_reduce.h: with the
@@ -1656,7 +1677,7 @@ static inline uint32_t bucket_count(uint32_t entries, uint32_t shift) { return (
 
 // A batch's buckets.  few: it takes grid_reduce_few_kernel.  That is where on average its buckets hold no more records than three quarters of the claims there
 // are on levels of pair records, and four times as many on the others, whose buckets are the smallest there can be: with the default table up to 24 576
-// points.  Encoding forward and backward in us, grid_reduce_kernel | grid_reduce_few_kernel: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5,
+// points.  Encoding forward and backward in us, grid_reduce_kernel (before it drew its buckets) | grid_reduce_few_kernel: uniform 600 30.1 | 25.5, 5003 32.6 | 27.5,
 // 8192 33.5 | 29.1, 12 288 35.5 | 32.7, 16 384 37.7 | 37.0, 20 000 37.5 | 36.4, 24 576 40.4 | 40.5; along rays 3000 28.7 | 25.2, 16 384 34.9 | 31.1, 20 000 34.0 | 29.5,
 // 24 576 36.0 | 32.0, 32 768 41.8 | 43.2.
 // groups: workgroups a bucket is split over; images: fp32 images of all split buckets (never more for a smaller batch: the groups per bucket grow with it).
@@ -1790,10 +1811,11 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	else bin(std::integral_constant<uint32_t, 2>());
 	N2_LAUNCH_CHECK();
 	if (buckets.few)
-		grid_reduce_few_kernel<<<dim3(wg), dim3(FEW_BLOCK), 0, s>>>(plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
-	else
-		grid_reduce_kernel<<<dim3(wg < RED_AT_A_TIME ? wg : RED_AT_A_TIME), dim3(RED_BLOCK), 0, s>>>(plan, tiles, bin_records(per), part_shift, rec_vals, rec_keys, offsets, grid->grads,
-		                                                                                              accumulate ? 1 : 0, partials, queue);
+		grid_reduce_few_kernel<<<dim3(wg < FEW_AT_A_TIME ? wg : FEW_AT_A_TIME), dim3(FEW_BLOCK), 0, s>>>(plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
+	else {
+		auto* const kernel = accumulate ? grid_reduce_kernel<true> : grid_reduce_kernel<false>;
+		kernel<<<dim3(wg < RED_AT_A_TIME ? wg : RED_AT_A_TIME), dim3(RED_BLOCK), 0, s>>>(plan, tiles, bin_records(per), part_shift, rec_vals, rec_keys, offsets, grid->grads, partials, queue);
+	}
 	N2_LAUNCH_CHECK();
 	if (split > 0) {
 		N2ImageCombine cmb{};
