@@ -571,16 +571,6 @@ __device__ __forceinline__ void n2_row_add(float (&a)[8], float (&b)[8], const f
 	      "+&v"(b[0]), "+&v"(b[1]), "+&v"(b[2]), "+&v"(b[3]), "+&v"(b[4]), "+&v"(b[5]), "+&v"(b[6]), "+&v"(b[7]) : "v"(take), "n"(D));
 #undef N2_ROW_ADD
 }
-// sum over the lanes up to this one (all 64 lanes active): lane shifts inside the rows of 16, then the rows' totals
-__device__ __forceinline__ uint32_t n2_wave_prefix(uint32_t x) {
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // a row's last lane to the next row, rows 1 and 3
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2 and 3
-	return x;
-}
 constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 
 // Pair records.  On a hashed level the entry of corner (x, y, z) is (x ^ y P1 ^ z P2) & (T - 1); while x + 1 stays below

@@ -157,8 +157,8 @@ __device__ const McRing MC_RING = mc_build_ring();
 // a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 81 (6.6 TB/s), count 16, scan 8, emit 34, normals 26, with
-// the host's wait for the totals 182 in all.  Deciding every point from the four rows of the density itself took 242 for the
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 82 (6.6 TB/s), count 14.5, scan 4.6, emit 32, normals 26, with
+// the host's wait for the totals 173 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
 struct McGrid {
@@ -303,16 +303,6 @@ __device__ __forceinline__ uint32_t mc_case(const McBits& B, uint32_t lane) {
 	return m;
 }
 
-// inclusive sum over the lanes of a wave
-__device__ __forceinline__ uint32_t mc_wave_scan(uint32_t v, uint32_t lane) {
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t u = __shfl_up(v, o);
-		if ((int)lane >= o) v += u;
-	}
-	return v;
-}
-
 // The number of triangles of 64 cubes at a time.  A cube that the surface crosses in one piece has two triangles fewer than cut edges; bits
 // 0, 1, 2 of that number follow from a carry-save addition of the twelve edges' words.  `several`: the cubes that it may cross in several
 // pieces, namely those with a face whose four edges are cut, and those with two opposite corners (inside or outside) alone; their numbers
@@ -392,7 +382,8 @@ __device__ __forceinline__ void mc_own(const McBits& B, McRecord& r, uint32_t& n
 
 // One wave per block of 256 words, four consecutive words per lane: with their neighbours in y and z four loads of 32 bytes, and nothing to
 // wait for but these.  (A lane per word in workgroups of four waves, with a table of triangle numbers in LDS: four rounds of workgroups that
-// each waited for the table, the bits and each other, 28 us for 512^3, of which walking through the cut cubes took 3; now 16.)
+// each waited for the table, the bits and each other, 28 us for 512^3, of which walking through the cut cubes took 3; then 16, and 14.5 where blocks
+// away from the surface, two of three, stop at their bits.)
 constexpr uint32_t MC_EACH = 4;
 static_assert(MC_BLOCK == 64u * MC_EACH, "a wave takes a block");
 __global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* __restrict__ bits, McRecord* __restrict__ records,
@@ -414,6 +405,20 @@ __global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* _
 				b[j][q + 1u] = v.y;
 			}
 			b[j][MC_EACH] = lane == 63u ? at[MC_EACH] : 0ull;
+		}
+		// Most blocks lie away from the surface: all their bits and their neighbours' are the same.
+		mc_word any = 0ull, all = ~0ull;
+#pragma unroll
+		for (uint32_t j = 0; j < 4; ++j) {
+#pragma unroll
+			for (uint32_t q = 0; q < MC_EACH; ++q) { any |= b[j][q]; all &= b[j][q]; }
+			any |= b[j][MC_EACH];
+			all &= lane == 63u ? b[j][MC_EACH] : ~0ull;
+		}
+		if (!__any(any != 0ull) || !__any(all != ~0ull)) {
+			if (lane < MC_EACH) active[blockIdx.x * MC_EACH + lane] = 0ull;
+			if (lane == 0) blocks[blockIdx.x] = make_uint2(0u, 0u);
+			return;
 		}
 #pragma unroll
 		for (uint32_t j = 0; j < 4; ++j) {
@@ -454,7 +459,7 @@ __global__ void __launch_bounds__(64) mc_count_kernel(McGrid g, const mc_word* _
 		const mc_word mask = __ballot(nv[q] + nt[q] > 0u);
 		if (lane == 0) active[blockIdx.x * MC_EACH + q] = mask;
 	}
-	const uint32_t iv = mc_wave_scan(sum_v, lane), it = mc_wave_scan(sum_t, lane);
+	const uint32_t iv = n2_wave_prefix(sum_v), it = n2_wave_prefix(sum_t);
 	uint32_t first_v = iv - sum_v, first_t = it - sum_t;
 #pragma unroll
 	for (uint32_t q = 0; q < MC_EACH; ++q) {
@@ -507,7 +512,7 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_short_kernel(McGrid g, cons
 		if (threadIdx.x == 0) blocks[blockIdx.x] = make_uint2(0, 0);
 		return;
 	}
-	const uint32_t iv = mc_wave_scan(nv, lane), it = mc_wave_scan(nt, lane);
+	const uint32_t iv = n2_wave_prefix(nv), it = n2_wave_prefix(nt);
 	if (lane == 63) { sum_v[wave] = iv; sum_t[wave] = it; }
 	__syncthreads();
 	uint32_t before_v = 0, before_t = 0, all_v = 0, all_t = 0;
@@ -527,49 +532,54 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_count_short_kernel(McGrid g, cons
 
 // Exclusive prefix sums of the blocks' counts in place; element n_blocks receives the totals.  The blocks that own something are listed, their
 // number goes behind the totals.
-constexpr uint32_t MC_SCAN_EACH = 8;
+// 8192 blocks a round, consecutive lanes on consecutive ones: a group of 64 blocks is summed by a wave, the 128 groups by one wave.  (With eight consecutive blocks to
+// a lane every load and store was 64 lines apart, for one CU's L1: 8 us for 512^3, now 4.6.)
+constexpr uint32_t MC_SCAN_EACH = 8, MC_SCAN_GROUPS = 16 * MC_SCAN_EACH;
 __global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2* __restrict__ blocks, uint32_t* __restrict__ listed,
                                                        uint32_t* to_v, uint32_t* to_t) {
-	__shared__ uint2 wave_sum[16];
-	__shared__ uint32_t wave_n[16];
+	__shared__ uint32_t group[3][MC_SCAN_GROUPS + 1];
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	uint2 carry = make_uint2(0, 0);
-	uint32_t carry_n = 0;
+	uint32_t carry[3] = {0u, 0u, 0u};
 	for (uint32_t c0 = 0; c0 < n_blocks; c0 += 1024u * MC_SCAN_EACH) {
-		const uint32_t i0 = c0 + threadIdx.x * MC_SCAN_EACH;
-		uint2 v[MC_SCAN_EACH], own = make_uint2(0, 0);
-		uint32_t n = 0;
+		uint2 v[MC_SCAN_EACH];
+		uint32_t upto[MC_SCAN_EACH][3];
 #pragma unroll
-		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) v[k] = i0 + k < n_blocks ? blocks[i0 + k] : make_uint2(0, 0);
-#pragma unroll
-		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) { own.x += v[k].x; own.y += v[k].y; n += (v[k].x | v[k].y) ? 1u : 0u; }
-		const uint32_t ix = mc_wave_scan(own.x, lane), iy = mc_wave_scan(own.y, lane), in = mc_wave_scan(n, lane);
-		if (lane == 63) { wave_sum[wave] = make_uint2(ix, iy); wave_n[wave] = in; }
-		__syncthreads();
-		uint2 run = make_uint2(carry.x + ix - own.x, carry.y + iy - own.y);
-		uint32_t run_n = carry_n + in - n;
-#pragma unroll
-		for (uint32_t k = 0; k < 16; ++k) {
-			const uint2 s = wave_sum[k];
-			const uint32_t m = wave_n[k];
-			if (k < wave) { run.x += s.x; run.y += s.y; run_n += m; }
-			carry.x += s.x;
-			carry.y += s.y;
-			carry_n += m;
+		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) {
+			const uint32_t i = c0 + k * 1024u + threadIdx.x;
+			v[k] = i < n_blocks ? blocks[i] : make_uint2(0u, 0u);
 		}
 #pragma unroll
 		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) {
-			if (i0 + k < n_blocks) blocks[i0 + k] = run;
-			if (v[k].x | v[k].y) listed[run_n++] = i0 + k;
-			run.x += v[k].x;
-			run.y += v[k].y;
+			upto[k][0] = n2_wave_prefix(v[k].x);
+			upto[k][1] = n2_wave_prefix(v[k].y);
+			upto[k][2] = n2_wave_prefix((v[k].x | v[k].y) ? 1u : 0u);
+			if (lane == 63u) {
+#pragma unroll
+				for (uint32_t q = 0; q < 3; ++q) group[q][k * 16u + wave] = upto[k][q];
+			}
 		}
+		__syncthreads();
+		if (wave < 3u) {  // sum q by wave q, two groups to a lane
+			const uint32_t a = group[wave][2u * lane], b = group[wave][2u * lane + 1u], both = n2_wave_prefix(a + b);
+			group[wave][2u * lane] = both - a - b;
+			group[wave][2u * lane + 1u] = both - b;
+			if (lane == 63u) group[wave][MC_SCAN_GROUPS] = both;
+		}
+		__syncthreads();
+#pragma unroll
+		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) {
+			const uint32_t i = c0 + k * 1024u + threadIdx.x, g = k * 16u + wave;
+			if (i < n_blocks) blocks[i] = make_uint2(carry[0] + group[0][g] + upto[k][0] - v[k].x, carry[1] + group[1][g] + upto[k][1] - v[k].y);
+			if (v[k].x | v[k].y) listed[carry[2] + group[2][g] + upto[k][2] - 1u] = i;
+		}
+#pragma unroll
+		for (uint32_t q = 0; q < 3; ++q) carry[q] += group[q][MC_SCAN_GROUPS];
 		__syncthreads();  // the sums have been read
 	}
 	if (threadIdx.x == 0) {
-		blocks[n_blocks] = carry;
-		blocks[n_blocks + 1u] = make_uint2(carry_n, 0u);
-		if (to_v) { *to_v = carry.x; *to_t = carry.y; }
+		blocks[n_blocks] = make_uint2(carry[0], carry[1]);
+		blocks[n_blocks + 1u] = make_uint2(carry[2], 0u);
+		if (to_v) { *to_v = carry[0]; *to_t = carry[1]; }
 	}
 }
 
@@ -599,7 +609,7 @@ constexpr uint32_t MC_LIST = 2048;
 template <class Visit>
 __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, uint32_t* wave_sum, Visit visit) {
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	const uint32_t n = (uint32_t)__popcll(points), incl = mc_wave_scan(n, lane);
+	const uint32_t n = (uint32_t)__popcll(points), incl = n2_wave_prefix(n);
 	if (lane == 63) wave_sum[wave] = incl;
 	__syncthreads();
 	uint32_t first = incl - n, total = 0;
@@ -626,7 +636,7 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // the density is by now, a triangle's corners are vertices that this pass writes.
 // (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 34; with the case from the density 33.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
-constexpr uint32_t MC_EMIT_GRID = 1536;  // as many as run at a time: six per CU, by their LDS
+constexpr uint32_t MC_EMIT_GRID = 2304;  // 1536 run at a time, six per CU, by their LDS (512^3, 2646 blocks: 768 41.8 us, 1536 33.0, 2304 31.6, 6144 32.2)
 typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t mc_words3 __attribute__((ext_vector_type(3), aligned(4)));
 typedef float mc_float2 __attribute__((ext_vector_type(2), aligned(4)));

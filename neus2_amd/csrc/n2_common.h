@@ -34,6 +34,19 @@ void n2_set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 
 constexpr uint32_t N2_MAX_LEVELS = 32;
 
+#ifdef __HIPCC__
+// sum over the lanes up to this one (all 64 lanes active): lane shifts inside the rows of 16, then the rows' totals
+__device__ __forceinline__ uint32_t n2_wave_prefix(uint32_t x) {
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // a row's last lane to the next row, rows 1 and 3
+	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2 and 3
+	return x;
+}
+#endif
+
 struct N2SlabReduce;
 struct N2StepEpilogue;  // slab_reduce.h
 

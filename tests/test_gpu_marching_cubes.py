@@ -76,6 +76,24 @@ def test_a_plane_through_every_block_of_words(res):
     assert bool((n[..., 1:] == 0).all()) and bool((n[1:-1, 1:-1, 0].abs() == 6).all())  # six triangles of twice the area one
 
 
+@pytest.mark.parametrize("inside_first", [False, True])
+@pytest.mark.parametrize("res,axis,at", [((64, 512, 6), 1, 256), ((64, 512, 6), 1, 255), ((128, 64, 10), 2, 4), ((128, 64, 10), 2, 3), ((128, 64, 10), 2, 8), ((256, 128, 5), 0, 64), ((256, 128, 5), 0, 63),
+                                         ((130, 100, 9), 2, 8), ((512, 512, 700), 2, 699), ((512, 512, 700), 2, 513), ((512, 512, 1100), 2, 1030)])
+def test_a_plane_between_blocks_without_a_surface(res, axis, at, inside_first):
+    """A plane across `axis` between the points at - 1 and at, where blocks of 256 words begin and end, all bits of the others the same; with more than 8192 and 16 384 blocks."""
+    from neus2_amd.mesh import marching_cubes
+    x = torch.arange(res[axis], device="cuda", dtype=torch.float32) - (at - 0.25)
+    shape = [1, 1, 1]
+    shape[2 - axis] = res[axis]
+    f = (-x if inside_first else x).view(shape).expand(res[2], res[1], res[0]).contiguous()
+    v, t, n = marching_cubes(f, 0.0, (0, 0, 0), res)
+    others = [res[d] for d in range(3) if d != axis]
+    assert v.shape == (others[0] * others[1], 3) and t.shape == (2 * (others[0] - 1) * (others[1] - 1), 3)
+    want = torch.stack(torch.meshgrid(*[torch.arange(r, device="cuda").float() if d != 2 - axis else torch.tensor([at - 0.25], device="cuda") for d, r in enumerate(reversed(res))], indexing="ij")[::-1], -1)
+    assert torch.equal(v, want.reshape(-1, 3))
+    assert torch.equal(t.long().reshape(-1).unique(), torch.arange(len(v), device="cuda"))
+
+
 def test_meshes_counted_by_several_threads_at_once():
     """Each call waits for totals of its own."""
     from concurrent.futures import ThreadPoolExecutor
