@@ -484,6 +484,34 @@ def test_sorted_scatter_of_few_records(n, where, table):
 
 
 # the last batch of one point per thread and the next one, workspaces that are just large enough and larger; buckets of up to 65536 records are whole
+@pytest.mark.parametrize("n", [1, 70, 5003, 40001])
+@pytest.mark.parametrize("second", [False, True])
+def test_points_that_a_mask_leaves_out_of_the_scatter_may_hold_anything(n, second):
+    """Points along lines, whose runs of equal cells are summed across lanes, every third one switched off: what those hold reaches no other point's gradient."""
+    from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(**CFG)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = (torch.rand(gg.n_params(), device="cuda", generator=gen) * 2 - 1).half()
+    dg = torch.zeros_like(dp)
+    gg.set_params(dp, dg)
+    assert gg.reserve_scatter_workspace(n)
+    off = torch.arange(n, device="cuda") % 3 == 2
+    x = (0.2 + 0.6 * torch.arange(n, device="cuda") / n).repeat(3, 1) + torch.tensor([[0.0], [0.01], [0.02]], device="cuda")
+    dy, g2, v = (torch.randn((w, n), device="cuda", generator=gen) for w in (32, 32, 3))
+    gg.set_max_level_gpu(torch.where(off, -1.0, 1.0))
+    got = []
+    for bad in (False, True):
+        fill = lambda t, value: torch.where(off, torch.full_like(t, value), t).contiguous()
+        a = (fill(x, float("nan") if bad else 0.5), fill(dy, float("inf") if bad else 0.0).half(), fill(v, float("nan") if bad else 0.0), fill(g2, float("-inf") if bad else 0.0).half())
+        dg.fill_(9.0)
+        if second:
+            gg.backward_fused(a[0], a[1], a[2], a[3], want_dL_ddLdy=False, mode=GRAD_OVERWRITE)
+        else:
+            gg.backward(None, a[0], a[1], mode=GRAD_OVERWRITE)
+        got.append(dg.clone())
+    assert torch.equal(got[0], got[1]) and bool(torch.isfinite(got[0].float()).all()) and bool((got[0] != 0).any())
+
+
 @pytest.mark.parametrize("levels,log2_size,line,whole", [(16, 19, 24576, True), (7, 16, 55808, True), (7, 14, 55808, False), (2, 6, 196608, False)])
 def test_sorted_scatter_at_the_line_between_the_tiles(levels, log2_size, line, whole):
     from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
