@@ -13,12 +13,13 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.8 ms, per slab of 7.6e6 points 140 us for six fine levels and 130 us for the walk.  Before: 5.76, 148 and 176, with
-// vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  The fine levels are held by the L1's
+// 512^3 lattice 4.70 ms, per slab of 7.6e6 points 140 us for six fine levels and 120 us for the walk.  (4.80 and 130 when a walk's start waited for its planes
+// one after the other and then for the fine features.  Before: 5.76, 148 and 176, with vertices picked out of LDS row by row, and four gathers per
+// point and plane by two waves per SIMD.)  The fine levels are held by the L1's
 // data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and by
 // the features, which come from beyond the L2 (28 % hits).
-// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before | now: 80^3 86 | 81 us, 128^3 187 | 176, 208^3 654 | 595,
-// 256^3 1008 | 890, 320^3 1750 | 1605, 400^3 3410 | 2925, 464^3 5130 | 4550, 512 x 64 x 512 752 | 625, 64 x 512 x 512 1672 | 1624.
+// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, waves of up to 16 planes and such starts | now: 80^3 81 | 74 us, 96^3 105 | 97,
+// 128^3 178 | 170, 208^3 594 | 570, 256^3 890 | 870, 320^3 1605 | 1529, 400^3 2925 | 2815, 464^3 4543 | 4327, 512 x 64 x 512 624 | 599, 64 x 512 x 512 1619 | 1588.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -43,7 +44,7 @@ struct LatticeArgs {
 	float sdf_bias;
 	N2Lattice lat;
 	uint32_t y0, ny, z0, nz;  // the slab: rows y0 .. y0 + ny of planes z0 .. z0 + nz,
-	uint32_t x_runs, walk;    // runs of 64 points per row of the slab; planes per wave
+	uint32_t x_runs, walk;    // runs of 64 points per row of the slab; planes per wave of this launch
 	uint32_t first_fine;      // levels first_fine .. n_levels - 1 come from `features`
 	uint32_t* features;       // [n_levels - first_fine][nz ny nx] half2
 	float* out;               // row 0 of point (x0, y0, z0)
@@ -354,9 +355,9 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	n2_locate(lane_f32(px, 63), my_scale, unused, my_last);
 	my_first = (uint32_t)min((int32_t)my_first, (int32_t)my_last);
 	// the plane of vertices whose rows y, y + 1 are at byte offsets row0, row1
-	auto fetch = [&](int l, uint32_t row0, uint32_t row1, uint32_t (&raw)[2]) __attribute__((always_inline)) {
+	auto fetch = [&](int l, uint32_t vertex_of_run, uint32_t row0, uint32_t row1, uint32_t (&raw)[2]) __attribute__((always_inline)) {
 		const char* base = reinterpret_cast<const char*>(a.table + a.offset[l]);
-		const uint32_t entries = lane_u32(my_entries, l), v = lane_u32(my_first, l) + lane;
+		const uint32_t entries = lane_u32(my_entries, l), v = lane_u32(my_first, l) + vertex_of_run;
 		if ((a.hash_mask >> l) & 1u) {
 			const uint32_t xo = x_part(true, entries, 0u, v);
 			raw[0] = *reinterpret_cast<const uint32_t*>(base + (xo ^ row0));
@@ -389,20 +390,20 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		r1 = row_part(my_hashed, my_entries, my_res, my_cy + 1u, cz);
 	};
 	float2 hi[NM], rise[NM];  // the plane above, and by how much it is above the one below
-	auto one_plane = [&](uint32_t which, uint32_t cz, float2 (&to)[NM]) __attribute__((always_inline)) {
-		uint32_t r0, r1, raw[NM][2];
+	// (all levels, also those that are switched off: behind branches the loads would be waited for one by one)
+	auto fetch_plane = [&](uint32_t cz, uint32_t (&raw)[NM][2]) __attribute__((always_inline)) {
+		uint32_t r0, r1, v = lane;
+		asm volatile("" : "+v"(v));  // (addresses formed here: kept for the next start, they take registers that a step needs)
 		rows_of(cz, r0, r1);
-		// (all levels' loads in flight together)
 #pragma unroll
-		for (int l = 0; l < NM; ++l)
-			if ((which >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+		for (int l = 0; l < NM; ++l) fetch(l, v, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+	};
+	auto blend_plane = [&](const uint32_t (&raw)[NM][2], float2 (&to)[NM]) __attribute__((always_inline)) {
 #pragma unroll
-		for (int l = 0; l < NM; ++l)
-			if ((which >> l) & 1u) blend_y(l, raw[l]);
+		for (int l = 0; l < NM; ++l) blend_y(l, raw[l]);
 		__builtin_amdgcn_wave_barrier();
 #pragma unroll
-		for (int l = 0; l < NM; ++l)
-			if ((which >> l) & 1u) blend_x(l, to[l]);
+		for (int l = 0; l < NM; ++l) blend_x(l, to[l]);
 		__builtin_amdgcn_wave_barrier();
 	};
 	const uint64_t feat_level = (uint64_t)plane * a.nz;
@@ -425,14 +426,21 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	while (true) {
 	n2_locate(lattice_coord(a.lat, 2, z + k), my_scale, my_back, my_cz);
 	my_back -= 1.f;
+	{
+		// (all of a start's loads under way together)
+		uint32_t below[NM][2], above[NM][2];
+		fetch_plane(my_cz, below);
+		fetch_plane(my_cz + 1u, above);
+		load_fine(k, fine);
+		blend_plane(below, rise);
+		load_fine(min(k + 1u, nz - 1u), ahead);
+		blend_plane(above, hi);
+	}
 #pragma unroll
-	for (int l = 0; l < NM; ++l) hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched-off levels
-	one_plane(on, my_cz, rise);
-	one_plane(on, my_cz + 1u, hi);
-#pragma unroll
-	for (int l = 0; l < NM; ++l) rise[l] = make_float2(hi[l].x - rise[l].x, hi[l].y - rise[l].y);
-	load_fine(k, fine);
-	load_fine(min(k + 1u, nz - 1u), ahead);
+	for (int l = 0; l < NM; ++l) {
+		rise[l] = make_float2(hi[l].x - rise[l].x, hi[l].y - rise[l].y);
+		if (!((on >> l) & 1u)) hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched off
+	}
 	while (true) {
 		const float pz = lattice_coord(a.lat, 2, z + k);
 		// features of this step
@@ -459,7 +467,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		uint32_t raw[NM][2];
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+			if ((one >> l) & 1u) fetch(l, lane, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
 		// Behind them the fine features of the step after the next (they come from far away): the planes can then be waited for
 		// without waiting for these.
 #pragma unroll
@@ -697,18 +705,16 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 				a.z0 = z0; a.nz = slab.nz < rz - z0 ? slab.nz : rz - z0;
 				a.out = d_out + ((size_t)z0 * ry + y0) * rx + x0;
 				a.x_runs = (a.nx + 63u) / 64u;
-				// planes per wave: 16 where that leaves every SIMD several waves (a wave's start costs as much as two steps), fewer on
-				// small lattices; the slab's planes in equal shares
-				const uint64_t runs = (uint64_t)a.x_runs * a.ny * a.nz;
-				const uint32_t most = runs >= 16u * 4096u ? 16u : runs <= 4u * 4096u ? 4u : (uint32_t)(runs / 4096u), parts = (a.nz + most - 1u) / most;
-				a.walk = (a.nz + parts - 1u) / parts;
-				const uint32_t waves = a.x_runs * a.ny * ((a.nz + a.walk - 1u) / a.walk), blocks = (waves + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64);
+				const uint32_t runs = a.x_runs * a.ny;  // per plane
+				auto blocks = [&]() { return (runs * ((a.nz + a.walk - 1u) / a.walk) + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64); };
 				if (n_fine) {
 					const bool first = x0 == 0 && y0 == 0 && z0 == 0;
-					lattice_fine_kernel<<<dim3(blocks * n_fine + (first ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks);
+					a.walk = n2_lattice_fine_walk(runs, a.nz);
+					lattice_fine_kernel<<<dim3(blocks() * n_fine + (first ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks());
 					N2_LAUNCH_CHECK();
 				}
-				walk_kernel<<<dim3(blocks), dim3(LT_BLOCK), 0, s>>>(a);
+				a.walk = n2_lattice_walk(runs, a.nz, by_rows ? 3u : 2u);
+				walk_kernel<<<dim3(blocks()), dim3(LT_BLOCK), 0, s>>>(a);
 				N2_LAUNCH_CHECK();
 			}
 	return N2_OK;

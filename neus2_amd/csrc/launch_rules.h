@@ -57,6 +57,32 @@ static inline N2LatticeSlab n2_lattice_slab(const uint32_t res[3], uint64_t poin
 	return {nx, res[1], rows / res[1] < res[2] ? rows / res[1] : res[2]};
 }
 
+// Planes that a wave of a lattice's kernels walks, of nz with `runs` runs of 64 points each; parts of equal length.
+static inline uint32_t n2_lattice_part(uint32_t nz, uint32_t most) {
+	const uint32_t parts = (nz - 1u) / most + 1u;
+	return (nz - 1u) / parts + 1u;
+}
+// Fine levels: few enough that the last waves are done soon, fewer still where a SIMD would not get several waves
+// (256^3, 208^3, 320^3 in us with 16 | 12 planes: 892 | 873, 572 | 565, 1547 | 1536; 96^3 with 8 | 4: 122 | 106).
+static inline uint32_t n2_lattice_fine_walk(uint32_t runs, uint32_t nz) {
+	const uint64_t waves = (uint64_t)runs * nz / 4096u;
+	return n2_lattice_part(nz, waves >= 16u ? 12u : waves <= 4u ? 4u : (uint32_t)waves);
+}
+// The walk, `per_simd` of whose waves a SIMD holds: the 1024 SIMDs take the waves in rounds, of which each costs a wave's planes and a start as long
+// as two of them.  (By eye, up to 16 planes where there are many | by this count: 96^3 101 | 97, 128^3 174 | 171, 320^3 1547 | 1524, 512 x 64 x 512 623 | 600; with up to
+// 30 planes 96^3 to 320^3 lose up to 1.5 %.)
+static inline uint32_t n2_lattice_walk(uint32_t runs, uint32_t nz, uint32_t per_simd) {
+	const uint64_t at_a_time = 1024u * per_simd;
+	uint64_t least = ~0ull;
+	uint32_t walk = 1;
+	for (uint32_t most = 4; most <= 24u; ++most) {
+		const uint32_t part = n2_lattice_part(nz, most);
+		const uint64_t waves = (uint64_t)runs * ((nz - 1u) / part + 1u), cost = ((waves - 1u) / at_a_time + 1u) * (part + 2u);
+		if (cost < least) { least = cost; walk = part; }
+	}
+	return walk;
+}
+
 // The chunks of four entries along x that the cells c_first .. c_last of a run and their neighbours at +1 lie in (either end may be
 // the larger one): `chunks` of them from cell c_lo on.  Cells are signed: a box far outside the unit cube has them saturated at
 // the ends of the 32-bit range, 2^32 apart.

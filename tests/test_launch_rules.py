@@ -13,6 +13,8 @@ extern "C" void lattice_slab(const uint32_t* res, uint64_t points, uint32_t* out
 	const N2LatticeSlab s = n2_lattice_slab(res, points);
 	out[0] = s.nx; out[1] = s.ny; out[2] = s.nz;
 }
+extern "C" uint32_t lattice_fine_walk(uint32_t runs, uint32_t nz) { return n2_lattice_fine_walk(runs, nz); }
+extern "C" uint32_t lattice_walk(uint32_t runs, uint32_t nz, uint32_t per_simd) { return n2_lattice_walk(runs, nz, per_simd); }
 extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels, uint32_t points_per_block, uint32_t* visits, uint32_t* grid) {
 	const N2GatherGrid g = n2_gather_grid(by_xcd_max, n, n_levels, points_per_block);
 	grid[0] = g.x; grid[1] = g.y;
@@ -86,6 +88,16 @@ def test_lattice_slabs_fit_the_scratch_and_the_launch(rules, res, chunk, n_fine)
         assert nx * (ny + 1) > points or runs * (ny + 1) > 1 << 22
     elif nz < res[2]:
         assert nx * ny * (nz + 1) > points or runs * ny * (nz + 1) > 1 << 22
+
+
+# one run and plane, small lattices, 512^3, the most runs of a launch, lattices that are all planes
+@pytest.mark.parametrize("runs,nz", [(1, 1), (1, 3), (64, 64), (192, 96), (4096, 29), (4096, 88), (1 << 22, 1), (1, 1 << 22), (2, 1 << 21)])
+@pytest.mark.parametrize("per_simd", [2, 3])
+def test_planes_of_a_wave_are_equal_shares_of_the_slab(rules, runs, nz, per_simd):
+    for walk, most in ((rules.lattice_fine_walk(runs, nz), 12), (rules.lattice_walk(runs, nz, per_simd), 24)):
+        assert 1 <= walk <= min(most, nz)
+        parts = -(-nz // walk)
+        assert walk == -(-nz // parts)  # no shorter waves for as many of them
 
 
 # parameters of the field with tables of 2^14 to 2^22 entries a level (18 bytes of optimiser state each), batch, streamed
