@@ -826,7 +826,8 @@ int n2_marching_cubes_emit(n2_stream_t stream, const uint32_t res[3], const floa
                            uint32_t* d_indices, float* d_normals, uint32_t n_vertices, uint32_t n_triangles);
 /* get_density_on_grid: the field's SDF (row 0 of NerfNetwork::sdf, fp16 widened to fp32) at the lattice points
  * (x, y, z)/res * (aabb_max - aabb_min) + aabb_min, evaluated `chunk` points at a time (a multiple of 8, at most the
- * field's max_batch; the reference uses 2^20).  d_density fp32 [rx*ry*rz]. */
+ * field's max_batch; the reference uses 2^20).  d_density fp32 [rx*ry*rz]; until the call's work is done its unwritten part may hold
+ * intermediate values. */
 uint64_t n2_density_on_grid_scratch_bytes(uint32_t chunk);
 int n2_density_on_grid(n2_field_t* field, n2_stream_t stream, const uint32_t res[3], const float aabb_min[3],
                        const float aabb_max[3], float* d_density, void* d_scratch, uint64_t scratch_bytes, uint32_t chunk);

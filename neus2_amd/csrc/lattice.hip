@@ -13,13 +13,13 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.70 ms, per slab of 7.6e6 points 140 us for six fine levels and 120 us for the walk.  (4.80 and 130 when a walk's start waited for its planes
-// one after the other and then for the fine features.  Before: 5.76, 148 and 176, with vertices picked out of LDS row by row, and four gathers per
-// point and plane by two waves per SIMD.)  The fine levels are held by the L1's
-// data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and by
-// the features, which come from beyond the L2 (28 % hits).
-// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, waves of up to 16 planes and such starts | now: 80^3 81 | 74 us, 96^3 105 | 97,
-// 128^3 178 | 170, 208^3 594 | 570, 256^3 890 | 870, 320^3 1605 | 1529, 400^3 2925 | 2815, 464^3 4543 | 4327, 512 x 64 x 512 624 | 599, 64 x 512 x 512 1619 | 1588.
+// 512^3 lattice 4.49 ms in ten slabs: a plane takes 4.7 us for six fine levels and 4.2 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
+// the L1's data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and
+// by the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
+// fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's walk and
+// the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
+// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before these slabs, starts and lengths of waves | now: 80^3 81 | 74 us, 96^3
+// 105 | 97, 128^3 178 | 171, 208^3 594 | 570, 256^3 891 | 863, 320^3 1607 | 1516, 400^3 2929 | 2760, 464^3 4553 | 4218, 512 x 64 x 512 624 | 613, 64 x 512 x 512 1619 | 1583.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -46,11 +46,18 @@ struct LatticeArgs {
 	uint32_t y0, ny, z0, nz;  // the slab: rows y0 .. y0 + ny of planes z0 .. z0 + nz,
 	uint32_t x_runs, walk;    // runs of 64 points per row of the slab; planes per wave of this launch
 	uint32_t first_fine;      // levels first_fine .. n_levels - 1 come from `features`
-	uint32_t* features;       // [n_levels - first_fine][nz ny nx] half2
+	// [nz ny nx] half2 for each of the levels from first_fine on: rows of one buffer for the first `near_levels` of them, of another for the rest
+	uint32_t *near, *beyond;  // (`beyond` counts its rows from first_fine on, too)
+	uint32_t near_levels;
+	uint64_t points;          // of the slab
 	float* out;               // row 0 of point (x0, y0, z0)
 	uint32_t x0, nx;          // columns x0 .. x0 + nx of the slab
 };
 
+// the features of the slab's points on level first_fine + f
+__device__ __forceinline__ uint32_t* lattice_features(const LatticeArgs& a, uint32_t f) {
+	return (f < a.near_levels ? a.near : a.beyond) + f * a.points;
+}
 // coordinate of lattice index c on axis d: each step rounded on its own (positions are part of a bit-exact contract)
 __device__ __forceinline__ float lattice_coord(const N2Lattice& lat, int d, uint32_t c) {
 	return __fadd_rn(__fmul_rn(__fmul_rn((float)c, lat.inv_res[d]), lat.extent[d]), lat.corner[d]);
@@ -166,7 +173,7 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	if (!lattice_run(a, wave, x, y, z, nz)) return;
 	const bool inside = x < a.nx;
 	const uint32_t lane = threadIdx.x & 63u, plane = a.nx * a.ny;
-	uint32_t* out = a.features + (size_t)(level - a.first_fine) * plane * a.nz + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + x;
+	uint32_t* out = lattice_features(a, level - a.first_fine) + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + x;
 	if (level >= a.active_levels) {
 		for (uint32_t k = 0; k < nz; ++k)
 			if (inside) out[(size_t)k * plane] = 0u;
@@ -406,18 +413,20 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		for (int l = 0; l < NM; ++l) blend_x(l, to[l]);
 		__builtin_amdgcn_wave_barrier();
 	};
-	const uint64_t feat_level = (uint64_t)plane * a.nz;
-	const uint32_t* feat = a.features + (uint64_t)(z - a.z0) * plane + (uint64_t)(y - a.y0) * a.nx;  // (the same for the wave, like out)
+	const uint64_t feat_at = (uint64_t)(z - a.z0) * plane + (uint64_t)(y - a.y0) * a.nx;  // (the same for the wave, like out)
 	const uint32_t feat_x = min(x, a.nx - 1u);
 	float* out = a.out + (uint64_t)(z - a.z0) * ((uint64_t)a.lat.res[0] * a.lat.res[1]) + (uint64_t)(y - a.y0) * a.lat.res[0];
 	uint32_t xc0, xc1;
 	lattice_xy(px, py, lane >> 5, xc0, xc1);
 	// (levels that the table does not have read the last one's row: their weights are zero)
 	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
+	const uint32_t* row[LT_LEVELS - NM];
+#pragma unroll
+	for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) row[f] = lattice_features(a, have_fine ? min(f, a.n_levels - 1u - NM) : 0u) + feat_at;
 	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
 	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) __attribute__((always_inline)) {
 #pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = (feat + (have_fine ? min(f, a.n_levels - 1u - NM) : 0u) * feat_level + (uint64_t)k * plane)[feat_x];
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = (row[f] + (uint64_t)k * plane)[feat_x];
 	};
 	// Steps one after the other from plane k on, until the end or to where some level's next plane is not the one above (a box upside down;
 	// steps of more than a cell): there the walk starts anew.  (With that case inside the loop, where it is hardly ever met, its
@@ -594,17 +603,19 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 #pragma unroll
 	for (int l = 0; l < NM; ++l) lo[l] = hi[l] = rise[l] = make_float2(0.f, 0.f);  // switched-off levels
 	both_planes(on, my_cz);
-	const uint32_t* feat = a.features + (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + min(x, a.nx - 1u);
-	const size_t feat_level = (size_t)plane * a.nz;
+	const size_t feat_at = (size_t)(z - a.z0) * plane + (size_t)(y - a.y0) * a.nx + min(x, a.nx - 1u);
 	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + x;
 	uint32_t xc0, xc1;
 	lattice_xy(px, py, lane >> 5, xc0, xc1);
 	// (levels that the table does not have read the last one's row: their weights are zero)
 	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
+	const uint32_t* row[LT_LEVELS - NM];
+#pragma unroll
+	for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) row[f] = lattice_features(a, have_fine ? min(f, a.n_levels - 1u - NM) : 0u);
 	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
 	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) {
 #pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = feat[(size_t)(have_fine ? min(f, a.n_levels - 1u - NM) : 0u) * feat_level + (size_t)k * plane];
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = row[f][feat_at + (size_t)k * plane];
 	};
 	load_fine(0, fine);
 	load_fine(min(1u, nz - 1u), ahead);
@@ -659,7 +670,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 
 uint64_t n2_lattice_frag_bytes() { return SDF_FRAG_COUNT * 1024ull; }
 
-// d_scratch holds LT_MAX_FINE 4-byte rows of `chunk` points, d_frags the fragment image.
+// d_scratch holds LT_MAX_FINE 4-byte rows of `chunk` points, d_frags the fragment image.  The part of d_out behind a slab holds features too.
 int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice& lat, uint32_t chunk, void* d_scratch, void* d_frags, float* d_out) {
 	const N2LevelTable& tab = *nets.tab;
 	LatticeArgs a{};
@@ -679,7 +690,7 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 	a.sdf_in_w = nets.sdf_in_w;
 	a.sdf_bias = nets.sdf_bias;
 	a.lat = lat;
-	a.features = reinterpret_cast<uint32_t*>(d_scratch);
+	a.near = reinterpret_cast<uint32_t*>(d_scratch);
 	const float step_z = lat.inv_res[2] * lat.extent[2], end_x = lat.corner[0] + lat.extent[0];
 	const uint32_t rows = n2_lattice_row_levels(a.scale, lat.res[0], fabsf(lat.inv_res[0] * lat.extent[0]), fmaxf(fabsf(lat.corner[0]), fabsf(end_x)), step_z);
 	const uint32_t walked = n2_lattice_walked_levels(a.scale, fabsf(step_z));
@@ -694,28 +705,46 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 		lattice_frags_kernel<<<dim3(FRAG_BLOCKS), dim3(LT_BLOCK), 0, s>>>(a);
 		N2_LAUNCH_CHECK();
 	}
-	// a slab holds as many points as the scratch has room for the fine levels' features of
 	const uint32_t rx = lat.res[0], ry = lat.res[1], rz = lat.res[2];
-	const N2LatticeSlab slab = n2_lattice_slab(lat.res, (uint64_t)LT_MAX_FINE * chunk / (n_fine ? n_fine : 1u));
-	for (uint32_t z0 = 0; z0 < rz; z0 += slab.nz)
+	const uint64_t words = (uint64_t)LT_MAX_FINE * chunk, all = (uint64_t)rx * ry * rz;
+	const bool large = n2_lattice_large_slabs(all, words, n_fine);
+	uint64_t done = 0;
+	auto launch = [&](uint32_t x0, uint32_t nx, uint32_t y0, uint32_t ny, uint32_t z0, uint32_t nz, uint32_t near_levels) -> int {
+		a.x0 = x0; a.nx = nx; a.y0 = y0; a.ny = ny; a.z0 = z0; a.nz = nz;
+		a.points = (uint64_t)nx * ny * nz;
+		a.out = d_out + done;
+		a.near_levels = near_levels;
+		a.beyond = reinterpret_cast<uint32_t*>(a.out + a.points) - near_levels * a.points;
+		a.x_runs = (nx + 63u) / 64u;
+		const uint32_t runs = a.x_runs * ny;  // per plane
+		auto blocks = [&]() { return (runs * ((nz + a.walk - 1u) / a.walk) + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64); };
+		if (n_fine) {
+			a.walk = n2_lattice_fine_walk(runs, nz);
+			lattice_fine_kernel<<<dim3(blocks() * n_fine + (done == 0 ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks());
+			N2_LAUNCH_CHECK();
+		}
+		a.walk = n2_lattice_walk(runs, nz, by_rows ? 3u : 2u);
+		walk_kernel<<<dim3(blocks()), dim3(LT_BLOCK), 0, s>>>(a);
+		N2_LAUNCH_CHECK();
+		done += a.points;
+		return N2_OK;
+	};
+	for (uint32_t z0 = 0; z0 < rz;) {
+		uint32_t near_levels;
+		const uint32_t left[3] = {rx, ry, rz - z0};
+		N2LatticeSlab slab = n2_lattice_slab(left, n2_lattice_slab_points(all - done, words, n_fine, large, near_levels));
+		if (slab.ny == ry) {
+			if (!large || left[2] < 2u * slab.nz) slab.nz = n2_lattice_part(left[2], slab.nz);  // slabs alike (large ones: the last two)
+			if (const int rc = launch(0, rx, 0, ry, z0, slab.nz, near_levels)) return rc;
+			z0 += slab.nz;
+			continue;
+		}
+		// a plane in parts: rows, or pieces of one, by what the scratch alone holds
+		slab = n2_lattice_slab(left, words / (n_fine ? n_fine : 1u));
 		for (uint32_t y0 = 0; y0 < ry; y0 += slab.ny)
-			for (uint32_t x0 = 0; x0 < rx; x0 += slab.nx) {
-				a.x0 = x0; a.nx = slab.nx < rx - x0 ? slab.nx : rx - x0;
-				a.y0 = y0; a.ny = slab.ny < ry - y0 ? slab.ny : ry - y0;
-				a.z0 = z0; a.nz = slab.nz < rz - z0 ? slab.nz : rz - z0;
-				a.out = d_out + ((size_t)z0 * ry + y0) * rx + x0;
-				a.x_runs = (a.nx + 63u) / 64u;
-				const uint32_t runs = a.x_runs * a.ny;  // per plane
-				auto blocks = [&]() { return (runs * ((a.nz + a.walk - 1u) / a.walk) + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64); };
-				if (n_fine) {
-					const bool first = x0 == 0 && y0 == 0 && z0 == 0;
-					a.walk = n2_lattice_fine_walk(runs, a.nz);
-					lattice_fine_kernel<<<dim3(blocks() * n_fine + (first ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks());
-					N2_LAUNCH_CHECK();
-				}
-				a.walk = n2_lattice_walk(runs, a.nz, by_rows ? 3u : 2u);
-				walk_kernel<<<dim3(blocks()), dim3(LT_BLOCK), 0, s>>>(a);
-				N2_LAUNCH_CHECK();
-			}
+			for (uint32_t x0 = 0; x0 < rx; x0 += slab.nx)
+				if (const int rc = launch(x0, slab.nx < rx - x0 ? slab.nx : rx - x0, y0, slab.ny < ry - y0 ? slab.ny : ry - y0, z0, 1, n_fine ? n_fine : 1u)) return rc;
+		++z0;
+	}
 	return N2_OK;
 }

@@ -57,6 +57,23 @@ static inline N2LatticeSlab n2_lattice_slab(const uint32_t res[3], uint64_t poin
 	return {nx, res[1], rows / res[1] < res[2] ? rows / res[1] : res[2]};
 }
 
+// A slab's features, a 4-byte word per point and fine level, lie in the scratch (of `words` words) and, where a lattice has large slabs, in the output
+// behind the slab's own points too, where nothing has been written yet.  A slab ends with workgroups that have most of a CU to themselves, which takes
+// its two launches 33 us together; on the other hand features of more than the scratch of a 2^22 points' chunk no longer stay in the 256 MiB behind
+// the L2s.  In us, scratch alone | both, (slabs): 512^3 4702 (18) | 4492 (10), 464^3 4327 (14) | 4218 (8), 400^3 2815 (9) | 2760 (7), 320^3 1516 (5) | 1519 (4),
+// 256^3 863 (3) | 874 (2), 64 x 512 x 512 1583 (3) | 1605 (3), 300 x 500 x 200 with ten fine levels 1542 (7) | 1574 (6).
+static inline bool n2_lattice_large_slabs(uint64_t all, uint64_t words, uint32_t n_fine) { return n_fine != 0 && all > words / n_fine * 8u; }
+// Points that the next slab may have, `rest` of the lattice's being left, and how many levels' features go to the scratch.
+static inline uint64_t n2_lattice_slab_points(uint64_t rest, uint64_t words, uint32_t n_fine, bool large, uint32_t& in_scratch) {
+	in_scratch = n_fine ? n_fine : 1u;  // (without fine levels the walk reads, and does not use, a row of the scratch)
+	uint64_t most = words / in_scratch < rest ? words / in_scratch : rest;
+	for (uint32_t k = n_fine; large && k-- > 0;) {
+		const uint64_t here = k ? words / k : rest, there = rest / (n_fine - k + 1u), points = here < there ? here : there;
+		if (points > most) { most = points; in_scratch = k; }
+	}
+	return most;
+}
+
 // Planes that a wave of a lattice's kernels walks, of nz with `runs` runs of 64 points each; parts of equal length.
 static inline uint32_t n2_lattice_part(uint32_t nz, uint32_t most) {
 	const uint32_t parts = (nz - 1u) / most + 1u;

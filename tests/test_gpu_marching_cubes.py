@@ -237,6 +237,55 @@ def test_lattices_walked_by_rows_equal_the_same_points_queried(side, res, part, 
     assert_close(got, want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
 
 
+# The features of a slab lie in the scratch and, behind the slab, in the output: slabs that take both, the output alone (a scratch of less than a plane),
+# planes in parts at the end, gathered and by rows, an output that starts anywhere; no fine level at all
+@pytest.mark.parametrize("res,chunk,levels", [((70, 9, 60), 512, 16), ((70, 9, 60), 64, 16), ((130, 7, 33), 8, 16), ((300, 11, 90), 4096, 16), ((96, 33, 300), 1 << 14, 16),
+                                              ((64, 8, 40), 256, 4)])
+def test_a_lattice_in_slabs_equals_the_lattice_at_once(res, chunk, levels):
+    import ctypes as C
+    from neus2_amd import capi
+    from neus2_amd.mesh import density_on_grid
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork(n_levels=levels)
+    p = torch.randn(net.param_offsets()[4], device="cuda", generator=torch.Generator(device="cuda").manual_seed(res[0])) * 0.1
+    net.set_params(p.half(), None)
+    n = res[0] * res[1] * res[2]
+    net.reserve((n + 7) // 8 * 8)
+    whole = density_on_grid(net._h, res, (0, 0, 0), (1, 0.3, 0.4), chunk=(n + 7) // 8 * 8).flatten()
+    L = capi.lib()
+    L.n2_density_on_grid_scratch_bytes.restype = C.c_uint64
+    nbytes = int(L.n2_density_on_grid_scratch_bytes(C.c_uint32(chunk)))
+    scratch = torch.full((nbytes + 256,), 0x7B, dtype=torch.uint8, device="cuda")
+    out = torch.full((n + 130,), 7.0, device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for _ in range(2):  # the second time over the results of the first
+        capi.check(L.n2_density_on_grid(net._h, stream, (C.c_uint32 * 3)(*res), (C.c_float * 3)(0, 0, 0), (C.c_float * 3)(1, 0.3, 0.4), C.c_void_p(out.data_ptr() + 4),
+                                        C.c_void_p(scratch.data_ptr()), C.c_uint64(nbytes), C.c_uint32(chunk)), "n2_density_on_grid")
+        assert torch.equal(out[1:1 + n], whole)
+        assert (out[0] == 7) and (out[1 + n:] == 7).all() and (scratch[nbytes:] == 0x7B).all()
+
+
+# levels switched off, among those that are walked too, whose entries may hold anything; walked by rows, and gathered
+@pytest.mark.parametrize("res,active", [((130, 6, 64), 4), ((130, 6, 64), 9), ((130, 6, 64), 12), ((40, 9, 11), 3)])
+def test_a_lattice_with_levels_switched_off(res, active):
+    from neus2_amd.mesh import density_on_grid
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork()
+    o = net.param_offsets()
+    p = (torch.randn(o[4], device="cuda", generator=torch.Generator(device="cuda").manual_seed(active)) * 0.1).half()
+    net.reserve(1 << 16)
+    net.encoding().set_max_level((active - 0.5) / 16)
+    active = net.encoding().active_levels()
+    assert active < 16
+    first = net.encoding().level_table()[3]  # entry that a level starts at
+    got = []
+    for anything in (0.0, float("nan")):
+        p[o[2] + (o[3] - o[2]) // int(first[-1]) * int(first[active]):o[3]] = anything
+        net.set_params(p, None)
+        got.append(density_on_grid(net._h, res, (0, 0, 0), (130 / 512, 0.02, 0.125)))
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)
+
+
 # rows longer than the chunk, down to the smallest one: slabs of a few runs, and of less than one
 @pytest.mark.parametrize("res,chunk", [((513, 3, 5), 64), ((200, 4, 3), 8)])
 def test_lattice_of_rows_longer_than_the_chunk(res, chunk):

@@ -13,6 +13,10 @@ extern "C" void lattice_slab(const uint32_t* res, uint64_t points, uint32_t* out
 	const N2LatticeSlab s = n2_lattice_slab(res, points);
 	out[0] = s.nx; out[1] = s.ny; out[2] = s.nz;
 }
+extern "C" uint64_t lattice_slab_points(uint64_t rest, uint64_t words, uint32_t n_fine, int large, uint32_t* in_scratch) {
+	return n2_lattice_slab_points(rest, words, n_fine, large, *in_scratch);
+}
+extern "C" int lattice_large_slabs(uint64_t all, uint64_t words, uint32_t n_fine) { return n2_lattice_large_slabs(all, words, n_fine); }
 extern "C" uint32_t lattice_fine_walk(uint32_t runs, uint32_t nz) { return n2_lattice_fine_walk(runs, nz); }
 extern "C" uint32_t lattice_walk(uint32_t runs, uint32_t nz, uint32_t per_simd) { return n2_lattice_walk(runs, nz, per_simd); }
 extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels, uint32_t points_per_block, uint32_t* visits, uint32_t* grid) {
@@ -88,6 +92,27 @@ def test_lattice_slabs_fit_the_scratch_and_the_launch(rules, res, chunk, n_fine)
         assert nx * (ny + 1) > points or runs * (ny + 1) > 1 << 22
     elif nz < res[2]:
         assert nx * ny * (nz + 1) > points or runs * ny * (nz + 1) > 1 << 22
+
+
+# one point, fewer than the scratch has words, about as many as it takes, 512^3, the largest lattice; down to the smallest scratch
+@pytest.mark.parametrize("rest", [1, 7, 88, 1 << 16, 1 << 22, 1 << 27, 1 << 31])
+@pytest.mark.parametrize("chunk", [8, 1 << 14, 1 << 20, 1 << 22, 1 << 31])
+@pytest.mark.parametrize("n_fine", [0, 1, 6, 12])
+def test_features_of_a_slab_fit_the_scratch_and_the_output_behind_it(rules, rest, chunk, n_fine):
+    rules.lattice_slab_points.restype = C.c_uint64
+    words, k = 11 * chunk, C.c_uint32(99)
+    alone = words // max(n_fine, 1)
+    for large in (0, 1):
+        left, slabs = rest, 0
+        while left > 0 and slabs < 1000:
+            m = rules.lattice_slab_points(C.c_uint64(left), C.c_uint64(words), n_fine, large, C.byref(k))
+            assert min(left, alone) <= m <= left  # never fewer than the scratch alone takes
+            assert k.value * m <= words and (k.value == max(n_fine, 1) or k.value < n_fine)
+            if k.value < n_fine:
+                assert large and m > alone and (n_fine - k.value) * m <= left - m
+            left -= m
+            slabs += 1
+    assert rules.lattice_large_slabs(C.c_uint64(rest), C.c_uint64(words), n_fine) == (n_fine > 0 and rest > 8 * alone)
 
 
 # one run and plane, small lattices, 512^3, the most runs of a launch, lattices that are all planes
