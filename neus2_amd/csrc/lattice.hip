@@ -13,13 +13,13 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.49 ms in ten slabs: a plane takes 4.7 us for six fine levels and 4.2 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
+// 512^3 lattice 4.36 ms in ten slabs: a plane takes 4.7 us for six fine levels and 3.9 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
 // the L1's data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and
 // by the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
 // fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's walk and
 // the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
 // Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before these slabs, starts and lengths of waves | now: 80^3 81 | 74 us, 96^3
-// 105 | 97, 128^3 178 | 171, 208^3 594 | 570, 256^3 891 | 863, 320^3 1607 | 1516, 400^3 2929 | 2760, 464^3 4553 | 4218, 512 x 64 x 512 624 | 613, 64 x 512 x 512 1619 | 1583.
+// 105 | 97, 128^3 178 | 170, 208^3 594 | 566, 256^3 891 | 854, 320^3 1607 | 1500, 400^3 2929 | 2680, 464^3 4553 | 4097, 512 x 64 x 512 624 | 593, 64 x 512 x 512 1619 | 1583.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -307,15 +307,19 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 	xs[1][2] = __builtin_bit_cast(half8, uint4v{xc1, zcm, 0u, 0u});
 	// The second layer, of which only row 0 is wanted: a lane holds half of its sample's hidden values (the other group the
 	// other half).  Dot products on the vector unit take a third of the time of four more MFMAs per tile.
-	// (one tile after the other: side by side they take 32 registers more, and a third wave has no room)
+	// (one tile after the other: side by side they take 32 registers more, and a third wave has no room; the weights of 32 rows serve both: read for each
+	// tile anew, and with registers spilled whose return waits for the loads of two steps, the walk took 4.2 us a plane of 512^2, then 3.9)
 	float dot[2] = {0.f, 0.f};
 #pragma unroll
-	for (int t = 0; t < 2; ++t)
+	for (int mt = 0; mt < 2; ++mt) {
+		half8 w[3];
 #pragma unroll
-		for (int mt = 0; mt < 2; ++mt) {
+		for (int c = 0; c < 3; ++c) w[c] = frag(F, SDF_FRAG_W0 + mt * 3 + c, lane);
+#pragma unroll
+		for (int t = 0; t < 2; ++t) {
 			float16v acc = zero16();
 #pragma unroll
-			for (int c = 0; c < 3; ++c) acc = N2_MFMA(frag(F, SDF_FRAG_W0 + mt * 3 + c, lane), xs[t][c], acc);
+			for (int c = 0; c < 3; ++c) acc = N2_MFMA(w[c], xs[t][c], acc);
 			half8 h[2];
 			relu_pack(acc, h[0], h[1]);
 #pragma unroll
@@ -327,6 +331,7 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 			}
 			__builtin_amdgcn_sched_barrier(0);
 		}
+	}
 	// tile 0 belongs to lanes 0..31, tile 1 to the upper ones
 	uint32_t s0 = __float_as_uint(dot[0]), s1 = __float_as_uint(dot[1]);
 	swap_halves(s0, s1);
@@ -414,7 +419,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		__builtin_amdgcn_wave_barrier();
 	};
 	const uint64_t feat_at = (uint64_t)(z - a.z0) * plane + (uint64_t)(y - a.y0) * a.nx;  // (the same for the wave, like out)
-	const uint32_t feat_x = min(x, a.nx - 1u);
+	const uint32_t feat_x = min(x, a.nx - 1u) * 4u;  // in bytes
 	float* out = a.out + (uint64_t)(z - a.z0) * ((uint64_t)a.lat.res[0] * a.lat.res[1]) + (uint64_t)(y - a.y0) * a.lat.res[0];
 	uint32_t xc0, xc1;
 	lattice_xy(px, py, lane >> 5, xc0, xc1);
@@ -425,8 +430,10 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) row[f] = lattice_features(a, have_fine ? min(f, a.n_levels - 1u - NM) : 0u) + feat_at;
 	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
 	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) __attribute__((always_inline)) {
+		uint32_t at = feat_x;
+		asm volatile("" : "+v"(at));  // (the lane's 32 bits beside a uniform address; their sum, formed in front of the loop, takes registers that a step needs)
 #pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = (row[f] + (uint64_t)k * plane)[feat_x];
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(row[f] + (uint64_t)k * plane) + at);
 	};
 	// Steps one after the other from plane k on, until the end or to where some level's next plane is not the one above (a box upside down;
 	// steps of more than a cell): there the walk starts anew.  (With that case inside the loop, where it is hardly ever met, its
@@ -471,19 +478,24 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		n2_locate(lattice_coord(a.lat, 2, z + next), my_scale, wz, cz);
 		const uint32_t moved = cz - my_cz;
 		const uint32_t one = (uint32_t)__ballot(moved == 1u) & on, far = (uint32_t)__ballot(moved > 1u) & on;  // lanes 0..15 speak for the levels
-		uint32_t r0, r1;
+		uint32_t r0, r1, v = lane;
+		asm volatile("" : "+v"(v));
 		rows_of(cz + 1u, r0, r1);
 		uint32_t raw[NM][2];
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) fetch(l, lane, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+			if ((one >> l) & 1u) fetch(l, v, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
 		// Behind them the fine features of the step after the next (they come from far away): the planes can then be waited for
 		// without waiting for these.
 #pragma unroll
 		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
 		load_fine(min(k + 2u, nz - 1u), ahead);
-		const hf sdf = lattice_network(F, lane, enc, xc0, xc1, pz, a.sdf_bias);
-		if (inside) out[x] = (float)sdf;
+		float bias = a.sdf_bias;
+		asm volatile("" : "+s"(bias));
+		const hf sdf = lattice_network(F, lane, enc, xc0, xc1, pz, bias);
+		uint32_t out_x = x * 4u;
+		asm volatile("" : "+v"(out_x));
+		if (inside) *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + out_x) = (float)sdf;
 		out += (uint64_t)a.lat.res[0] * a.lat.res[1];
 		if (++k == nz) return;
 		if (far) break;
