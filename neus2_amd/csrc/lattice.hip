@@ -13,13 +13,13 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.36 ms in ten slabs: a plane takes 4.7 us for six fine levels and 3.9 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
+// 512^3 lattice 4.49 ms in ten slabs: a plane takes 4.7 us for six fine levels and 4.2 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
 // the L1's data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and
 // by the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
 // fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's walk and
 // the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
 // Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before these slabs, starts and lengths of waves | now: 80^3 81 | 74 us, 96^3
-// 105 | 97, 128^3 178 | 170, 208^3 594 | 566, 256^3 891 | 854, 320^3 1607 | 1500, 400^3 2929 | 2680, 464^3 4553 | 4097, 512 x 64 x 512 624 | 593, 64 x 512 x 512 1619 | 1583.
+// 105 | 97, 128^3 178 | 171, 208^3 594 | 570, 256^3 891 | 863, 320^3 1607 | 1516, 400^3 2929 | 2760, 464^3 4553 | 4218, 512 x 64 x 512 624 | 613, 64 x 512 x 512 1619 | 1583.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -345,6 +345,7 @@ template <int NM>
 __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const LatticeArgs a) {
 	__shared__ __align__(16) hf F[SDF_FRAG_COUNT * 512];
 	__shared__ float2 line[LT_BLOCK / 64][NM][64];
+	__shared__ uint2 place[LT_BLOCK / 64][NM][64];  // of the lane's point in a level's row: its weight, and the byte in `line` where its two vertices begin
 	for (uint32_t i = threadIdx.x; i < SDF_FRAG_COUNT * 64u; i += LT_BLOCK) *reinterpret_cast<half8*>(F + i * 8u) = *reinterpret_cast<const half8*>(a.frags + i * 8u);
 	__syncthreads();
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (LT_BLOCK / 64) + (threadIdx.x >> 6));
@@ -366,6 +367,8 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	n2_locate(lane_f32(px, 0), my_scale, unused, my_first);
 	n2_locate(lane_f32(px, 63), my_scale, unused, my_last);
 	my_first = (uint32_t)min((int32_t)my_first, (int32_t)my_last);
+	float one = 1.f;  // (a product with a literal 1 would be taken out, and the operands converted one by one)
+	asm("" : "+s"(one));
 	// the plane of vertices whose rows y, y + 1 are at byte offsets row0, row1
 	auto fetch = [&](int l, uint32_t vertex_of_run, uint32_t row0, uint32_t row1, uint32_t (&raw)[2]) __attribute__((always_inline)) {
 		const char* base = reinterpret_cast<const char*>(a.table + a.offset[l]);
@@ -384,17 +387,23 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		const float2 v0 = lt_h2f(raw[0]), v1 = lt_h2f(raw[1]);
 		const float wy = lane_f32(my_wy, l);
 		// (the differences as multiply-adds: those take half-precision operands as they are)
-		mine[l][lane] = make_float2(fmaf(wy, fmaf(1.f, v1.x, -v0.x), v0.x), fmaf(wy, fmaf(1.f, v1.y, -v0.y), v0.y));
+		mine[l][lane] = make_float2(fmaf(wy, fmaf(one, v1.x, -v0.x), v0.x), fmaf(wy, fmaf(one, v1.y, -v0.y), v0.y));
 	};
-	// What depends on x is worked out at each plane, from an opaque copy of the position: kept across the loop, cell and weight of
-	// every level take 20 registers.
-	auto blend_x = [&](int l, float2& to) __attribute__((always_inline)) {
-		float p = px, w;
+	// What depends on x waits in LDS: kept in registers, cell and weight of every level take 20, and working them out at each plane takes 40 clocks of a
+	// level's 110.
+	uint2 (&places)[NM][64] = place[threadIdx.x >> 6];
+#pragma unroll
+	for (int l = 0; l < NM; ++l) {
+		float w;
 		uint32_t cx;
-		asm volatile("" : "+v"(p));
-		n2_locate(p, lane_f32(my_scale, l), w, cx);
-		const float2* at = &mine[l][min(cx - lane_u32(my_first, l), 62u)];
+		n2_locate(px, lane_f32(my_scale, l), w, cx);
+		places[l][lane] = make_uint2(__float_as_uint(w), ((threadIdx.x >> 6) * NM + l) * 512u + min(cx - lane_u32(my_first, l), 62u) * 8u);
+	}
+	auto blend_x = [&](int l, float2& to) __attribute__((always_inline)) {
+		const uint2 p = places[l][lane];
+		const float2* at = reinterpret_cast<const float2*>(reinterpret_cast<const char*>(line) + p.y);
 		const float2 lo = at[0], hi = at[1];
+		const float w = __uint_as_float(p.x);
 		to = make_float2(fmaf(w, hi.x - lo.x, lo.x), fmaf(w, hi.y - lo.y, lo.y));
 	};
 	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) __attribute__((always_inline)) {
