@@ -24,6 +24,7 @@
 // Vertex positions are part of the bit-exact contract with the CPU oracle:
 // floating-point contraction is off for this file.
 #include "n2_common.h"
+#include "launch_rules.h"
 
 #include <cstring>
 
@@ -764,11 +765,15 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 // The triangles' other corners are worked out again from the density, by the arithmetic that placed them: the eighteen values of the four
 // cubes tell which triangles there are (MC_RING) and where their corners lie.  That is 18 loads a vertex and vector instructions; going
 // through the words' records to the triangles and from those to the vertices was some 45 loads, most of them lines of their own, one a
-// clock and CU: 32.5 us for 512^3, now 25.6.
+// clock and CU: 32.5 us for 512^3, then 25.8, and 23.9 where an XCD takes consecutive vertices and finds the rows and planes next to one's own in its
+// L2.  What bounds it is the vector unit, some 140 instructions for a triangle; rows loaded as three values at a time, and all triangles of a vertex in
+// one loop instead of one per cube, changed nothing (24.1).
 template <bool SHORT>
 __global__ void __launch_bounds__(MC_BLOCK) mc_normals_kernel(McGrid g, uint32_t n_verts, const float* __restrict__ density, float* __restrict__ normals) {
 	__shared__ float values[18][MC_BLOCK];  // [slow -1 .. 1][fast -1 .. 1][along 0, 1]
-	const uint32_t i = blockIdx.x * MC_BLOCK + threadIdx.x;
+	// (workgroups go to the XCDs in turn: each XCD takes consecutive vertices)
+	const uint32_t xcd = blockIdx.x % N2_XCDS, item = xcd * (gridDim.x / N2_XCDS) + min(xcd, gridDim.x % N2_XCDS) + blockIdx.x / N2_XCDS;
+	const uint32_t i = item * MC_BLOCK + threadIdx.x;
 	if (i >= n_verts) return;
 	float* mine = normals + (size_t)i * 3;
 	const uint32_t w = __float_as_uint(mine[0]), place = __float_as_uint(mine[1]);
