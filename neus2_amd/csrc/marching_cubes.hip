@@ -158,8 +158,8 @@ __device__ const McRing MC_RING = mc_build_ring();
 // a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 82 (6.6 TB/s), count 14.5, scan 4.6, emit 32, normals 26, with
-// the host's wait for the totals 173 in all.  Deciding every point from the four rows of the density itself took 242 for the
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 82 (6.6 TB/s), count 14.5, scan 4.6, emit 27.5, normals 24, with
+// the host's wait for the totals 168 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
 struct McGrid {
@@ -635,9 +635,10 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // corners pick theirs.  What bounds the launch is the chain of round trips: which words own something, their records (they stay in LDS, for
 // their neighbours in y too), then all that a point needs at once.  A cube's case comes from the bits, as its number of triangles did: whatever
 // the density is by now, a triangle's corners are vertices that this pass writes.
-// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, now 34; with the case from the density 33.)
+// (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, then 34; with the case from the density 33; with the neighbours'
+// records one behind the other, each in a branch of its own, 31.8, now 27.8.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
-constexpr uint32_t MC_EMIT_GRID = 2304;  // 1536 run at a time, six per CU, by their LDS (512^3, 2646 blocks: 768 41.8 us, 1536 33.0, 2304 31.6, 6144 32.2)
+constexpr uint32_t MC_EMIT_GRID = 2304;  // 1280 run at a time, five per CU, by their registers (512^3, 2646 blocks: 1280 31.0 us, 2304 27.5, 6144 31.1; six per CU with four registers spilled 29.4)
 typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t mc_words3 __attribute__((ext_vector_type(3), aligned(4)));
 typedef float mc_float2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -668,15 +669,9 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 			first[threadIdx.x] = make_uint2(before.x + r.first_v, before.y + r.first_t);
 		}
 		// (mc_for_points' first barrier stands between these stores and their readers)
-		auto owned = [&](uint32_t w) {
-			McOwned o;
-			if (w - block0 < MC_BLOCK) {
-				o = McOwned{{edges[0][w - block0], edges[1][w - block0], edges[2][w - block0]}, first[w - block0].x};
-			} else {
-				const McRecord& r = records[w];
-				o = McOwned{{r.edge[0], r.edge[1], r.edge[2]}, blocks[w / MC_BLOCK].x + r.first_v};
-			}
-			return o;
+		auto from_memory = [&](uint32_t w) {
+			const McRecord& r = records[w];
+			return McOwned{{r.edge[0], r.edge[1], r.edge[2]}, blocks[w / MC_BLOCK].x + r.first_v};
 		};
 		mc_for_points(points, list, wave_sum, [&](uint32_t entry) {
 			const uint32_t at0 = entry >> 6, w = block0 + at0, p = entry & 63u;
@@ -704,12 +699,34 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 				const mc_words2 two = *reinterpret_cast<const mc_words2*>(reinterpret_cast<const uint32_t*>(bits) + 2u * min(at[j], g.n_words - 1u) + (bit[j] >> 5));
 				pair[j] = (uint32_t)(((uint64_t)two.y << 32 | two.x) >> (bit[j] & 31u)) & 3u;
 			}
+			// (corners run round a face)
+			auto turned = [](uint32_t two) { return two >> 1 | (two & 1u) << 1; };
+			const uint32_t mask = pair[0] | turned(pair[1]) << 2 | pair[2] << 4 | turned(pair[3]) << 6;
+			uint4 row4 = make_uint4(0u, 0u, 0u, 0u);
 			if (tris) {  // (the points one further along x, y and z exist)
+				// The words of the plane at z + 1, most often of another block, are under way together; the one at y + 1 most often stands in LDS.
+				McOwned o[4];
+				o[0] = own;
+				o[2] = from_memory(at[2]);
+				o[3] = from_memory(at[3]);
+				row4 = *reinterpret_cast<const uint4*>(MC_TABLE.tri[mask]);
+				const uint32_t at1 = at[1] - block0;
+				if (at1 < MC_BLOCK) o[1] = McOwned{{edges[0][at1], edges[1][at1], edges[2][at1]}, first[at1].x};
+				else o[1] = from_memory(at[1]);
 #pragma unroll
 				for (uint32_t j = 0; j < 4; ++j) {
-					const McOwned o = j == 0 ? own : owned(at[j]);
-					slot_of[2 * j][threadIdx.x] = mc_vertex_slot(o, bit[j]);
-					slot_of[2 * j + 1][threadIdx.x] = bit[j] < 63u ? mc_vertex_slot(o, bit[j] + 1u) : mc_vertex_slot(owned(at[j] + 1u), 0u);
+					const uint32_t slot = mc_vertex_slot(o[j], bit[j]), up = bit[j] + 1u;
+					slot_of[2 * j][threadIdx.x] = slot;
+					uint32_t next = (slot & 0x1FFFFFFFu) + (uint32_t)__popc(slot >> 29);
+#pragma unroll
+					for (uint32_t a = 0; a < 3; ++a) next |= (uint32_t)((o[j].e[a] >> (up & 63u)) & 1ull) << (29u + a);
+					slot_of[2 * j + 1][threadIdx.x] = next;
+				}
+				if (!SHORT && p == 63u) {
+#pragma unroll
+					for (uint32_t j = 0; j < 4; ++j) o[j] = from_memory(at[j] + 1u);
+#pragma unroll
+					for (uint32_t j = 0; j < 4; ++j) slot_of[2 * j + 1][threadIdx.x] = mc_vertex_slot(o[j], 0u);
 				}
 			}
 			const uint32_t slot0 = mc_vertex_slot(own, p), flags = slot0 >> 29;
@@ -730,13 +747,10 @@ __global__ void __launch_bounds__(MC_BLOCK) mc_emit_kernel(McGrid g, const float
 			}
 			if (tris == 0) return;
 			const uint32_t first_t = first[at0].y + mc_below(t0, p) + 2u * mc_below(t1, p) + 4u * mc_below(t2, p);
-			auto turned = [](uint32_t two) { return two >> 1 | (two & 1u) << 1; };  // (corners run round a face)
-			const uint32_t mask = pair[0] | turned(pair[1]) << 2 | pair[2] << 4 | turned(pair[3]) << 6;
 			// Lattice point and direction that own each cube edge (src/marching_cubes.cu:690-706), five bits per edge:
 			// the owner's offset from this point in x, y, z and the edge's axis.
 			constexpr uint64_t OWNER = 0ull | 9ull << 5 | 2ull << 10 | 8ull << 15 | 4ull << 20 | 13ull << 25 | 6ull << 30 | 12ull << 35 |
 			                           16ull << 40 | 17ull << 45 | 19ull << 50 | 18ull << 55;
-			const uint4 row4 = *reinterpret_cast<const uint4*>(MC_TABLE.tri[mask]);
 			const uint32_t trow[4] = {row4.x, row4.y, row4.z, row4.w};
 			uint32_t* out = indices + (size_t)first_t * 3;
 #pragma unroll
