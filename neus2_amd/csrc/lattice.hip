@@ -13,13 +13,13 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.49 ms in ten slabs: a plane takes 4.7 us for six fine levels and 4.2 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
+// 512^3 lattice 4.26 ms in ten slabs: a plane takes 4.7 us for six fine levels and 3.5 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
 // the L1's data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and
 // by the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
 // fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's walk and
 // the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
 // Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before these slabs, starts and lengths of waves | now: 80^3 81 | 74 us, 96^3
-// 105 | 97, 128^3 178 | 171, 208^3 594 | 570, 256^3 891 | 863, 320^3 1607 | 1516, 400^3 2929 | 2760, 464^3 4553 | 4218, 512 x 64 x 512 624 | 613, 64 x 512 x 512 1619 | 1583.
+// 105 | 96, 128^3 178 | 169, 208^3 594 | 570, 256^3 891 | 843, 320^3 1607 | 1482, 400^3 2929 | 2632, 464^3 4553 | 4055, 512 x 64 x 512 624 | 580, 64 x 512 x 512 1619 | 1583.
 #include "n2_common.h"
 
 #include "grid_device.h"
