@@ -946,7 +946,7 @@ __device__ __forceinline__ uint32_t n2_queue_item(uint32_t drawn) { return block
 
 // What a workgroup works on, as long as it is below `end` (all of one kind of records): `item`, then what it draws.  `acc` is all zeros before and after.
 //
-// Lane j of wave w takes run w + 16 j of the bucket's (a tile's run, or one of the 2^part_shift parts of it, so that a batch of few
+// Lane j of wave w takes run w + WAVES j of the bucket's (a tile's run, or one of the 2^part_shift parts of it, so that a batch of few
 // tiles keeps all waves busy), and the wave walks through the records of its up to 64 runs as if they stood one behind the other, 64 at a time: which
 // runs the next 64 meet is the same question for the whole wave, so a run costs it two lane reads and three vector instructions, and every lane has a
 // record until the last.  FLIGHT times 64 records are being added while the next are on their way, the next item's first ones while this item's sums are written
@@ -961,12 +961,12 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 	if (item >= end) return;
 	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	N2ReduceItem it = n2_reduce_item(plan, lane_end, item);
-	// Of the wave's 64 runs at hand, lane j: the records up to the end of run j, and what takes a record's number among them to its place in the arrays.
+	// Of the wave's 64 runs at hand, lane j: the records up to the end of run j, and what takes a record's number among them to its place behind `vals` and `keys`.
 	uint32_t upto, place, total;
 	uint32_t at, k, k_upto, k_place;  // the next records begin at number `at`, in run k
 	const value* vals;
 	const uint16_t* keys;
-	auto tile_of = [&](const N2ReduceItem& i, uint32_t run) { return min(i.group + i.l.groups * (run >> part_shift), tiles - 1u); };
+	auto tile_of = [&](const N2ReduceItem& i, uint32_t run) { return n2_run_tile(i.group, i.l.groups, run, part_shift, tiles); };
 	auto bounds = [&](const N2ReduceItem& i, uint32_t first) __attribute__((always_inline)) {  // of the lane's run
 		uint32_t two;
 		__builtin_memcpy(&two, offsets + ((size_t)i.l.level * tiles + tile_of(i, first + WAVES * lane)) * (BKT_MAX + 1) + i.bucket, sizeof(two));
@@ -978,11 +978,12 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 		const uint32_t all = (two >> 16) - (two & 0xFFFFu), begin = all * part >> part_shift, stop = all * (part + 1u) >> part_shift;
 		const uint32_t n = run < runs_of(i) ? stop - begin : 0u;
 		upto = n2_wave_prefix(n);
-		place = tile_of(i, run) * (PAIR ? slot_records / 2u : slot_records) + (two & 0xFFFFu) + begin - (upto - n);
+		const uint32_t tile_records = PAIR ? slot_records / 2u : slot_records, first_tile = tile_of(i, first);
+		place = n2_run_place(first_tile, tile_of(i, run), tile_records) + (two & 0xFFFFu) + begin - (upto - n);
 		total = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
-		const size_t level0 = (size_t)i.l.level * tiles * slot_records;
-		vals = reinterpret_cast<const value*>(rec_vals + level0);
-		keys = rec_keys + level0;
+		const size_t level0 = (size_t)i.l.level * tiles * slot_records, base = n2_run_base(first_tile, tile_records);
+		vals = reinterpret_cast<const value*>(rec_vals + level0) + base;
+		keys = rec_keys + level0 + base;
 		at = k = 0u;
 		k_upto = (uint32_t)__builtin_amdgcn_readlane((int)upto, 0);
 		k_place = (uint32_t)__builtin_amdgcn_readlane((int)place, 0);

@@ -34,6 +34,17 @@ constexpr uint32_t N2_BIN_AT_A_TIME = 768;
 static inline uint32_t n2_bin_single_points(uint32_t n_levels, uint32_t block) { return N2_BIN_AT_A_TIME / n_levels * block; }
 static inline uint32_t n2_bin_points_per_thread(uint32_t n_levels, uint32_t n_points, uint32_t block) { return n_points <= n2_bin_single_points(n_levels, block) ? 1u : 2u; }
 
+// Where the summing kernel finds a bucket's runs (grid_reduce_items).  Run r of a bucket, of which a workgroup has the tiles group, group + groups, ..., is a part of
+// this tile (runs behind the last one: of the last tile).
+static inline N2_HD uint32_t n2_run_tile(uint32_t group, uint32_t groups, uint32_t run, uint32_t part_shift, uint32_t tiles) {
+	const uint32_t tile = group + groups * (run >> part_shift);
+	return tile < tiles ? tile : tiles - 1u;
+}
+// A level's records are up to 2^33 (2^30 points, eight each), more than 32 bits count.  The 64 runs that a wave has at hand, every `stride`-th one, lie in at most
+// 63 * 16 * 32 tiles behind the first one's: the wave's two addresses stand at that tile, and a lane counts from there.
+static inline N2_HD uint64_t n2_run_base(uint32_t first_tile, uint32_t tile_records) { return (uint64_t)first_tile * tile_records; }
+static inline N2_HD uint32_t n2_run_place(uint32_t first_tile, uint32_t tile, uint32_t tile_records) { return (tile - first_tile) * tile_records; }
+
 // Whether the SDF network's step takes its one-pass kernel (sdf_eikonal_forward_kernel): a lane keeps its place in a matrix as a 32-bit number of bytes, 12 for each row and
 // point of the Jacobian, of which the last lane starts at 60 n - 12 (row 4 of a scalar base).  Larger batches take the single kernels, whose places are 64-bit.  (In 64 bits per
 // lane the kernel's registers spill: 56 us instead of 38.7 for 2^18 points.)

@@ -54,6 +54,9 @@ extern "C" void rows_of_blocks(uint32_t blocks, uint32_t threads, uint32_t* out)
 	const N2GatherGrid g = n2_rows_of_blocks(blocks, threads);
 	out[0] = g.x; out[1] = g.y;
 }
+extern "C" uint32_t run_tile(uint32_t group, uint32_t groups, uint32_t run, uint32_t part_shift, uint32_t tiles) { return n2_run_tile(group, groups, run, part_shift, tiles); }
+extern "C" uint64_t run_base(uint32_t first_tile, uint32_t tile_records) { return n2_run_base(first_tile, tile_records); }
+extern "C" uint32_t run_place(uint32_t first_tile, uint32_t tile, uint32_t tile_records) { return n2_run_place(first_tile, tile, tile_records); }
 extern "C" int sdf_one_pass(uint32_t n) { return n2_sdf_one_pass(n); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
@@ -206,6 +209,28 @@ def test_one_point_per_thread_while_all_sorting_workgroups_run_at_once(rules, le
     line = rules.bin_single_points(C.c_uint32(levels))
     assert levels * (line // 512) <= 768 < levels * (line // 512 + 1) and line % 512 == 0
     assert [rules.bin_points_per_thread(C.c_uint32(levels), C.c_uint32(n)) for n in (1, line, line + 1, 1 << 31)] == [1, 1, 2, 2]
+
+
+# one tile, few of them in parts, an ordinary batch, the last one whose level of single records 32 bits count, the first one that they do not, the largest; whole and split buckets
+@pytest.mark.parametrize("n,part_shift", [(8, 6), (5000, 2), (1 << 18, 0), (1 << 29, 0), ((1 << 29) + 1024, 0), (1 << 30, 0)])
+@pytest.mark.parametrize("tile_records", [8192, 4096])
+@pytest.mark.parametrize("group,groups", [(0, 1), (0, 32), (31, 32)])
+def test_places_of_a_levels_records_beyond_32_bits(rules, n, part_shift, tile_records, group, groups):
+    """What a wave's lanes count from its addresses leads to their tiles' records, of which 64 runs lie within 32 bits."""
+    rules.run_base.restype, rules.run_place.restype = C.c_uint64, C.c_uint32
+    tiles = -(-n // 1024)
+    groups, group = min(groups, tiles), min(group, tiles - 1)
+    runs = -(-(tiles - group) // groups) << part_shift
+    for stride in (8, 12, 16):
+        for first in {w + k * 64 * stride for w in (0, 1, stride - 1) for k in (0, 1, (runs - 1) // (64 * stride))}:
+            first_tile = rules.run_tile(group, groups, first, part_shift, tiles)
+            base = rules.run_base(first_tile, tile_records)
+            for lane in range(64):
+                run = first + stride * lane
+                tile = rules.run_tile(group, groups, run, part_shift, tiles)
+                assert tile == min(group + groups * (run >> part_shift), tiles - 1)
+                if run < runs:
+                    assert base + rules.run_place(first_tile, tile, tile_records) == tile * tile_records <= (tiles - 1) * tile_records
 
 
 @pytest.mark.parametrize("n,fits", [(8, 1), (1 << 18, 1), (1 << 26, 1), (71582784, 1), (71582792, 0), (1 << 27, 0), (1 << 28, 0)])
