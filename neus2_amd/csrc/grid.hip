@@ -562,6 +562,7 @@ constexpr unsigned long long ROW_HEADS = 0x0001000100010001ull;  // first lane o
 // r += take * (r of the lane D places below in the same 16-lane row; 0 if that leaves the row), for the sixteen values of a point.
 // (Written out: the compiler makes a move with the lane shift, a wait state and a multiply-add of each.  s_nop: a lane shift must not
 // read what one of the two instructions before it wrote.  &: `take` is read after the first values are written, so no value may share its register.)
+// A value that is not finite makes no numbers of the sums above it in its row that do not take it, either: those count as zero.
 template <int D>
 __device__ __forceinline__ void n2_row_add(float (&a)[8], float (&b)[8], const float take) {
 #define N2_ROW_ADD(K) "v_fmac_f32_dpp %" #K ", %" #K ", %16 row_shr:%17 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
@@ -851,8 +852,16 @@ __device__ __forceinline__ bool is_fixed_small(float scaled) { return fabsf(scal
 __device__ __forceinline__ unsigned long long fixed_large(float scaled) {
 	return __builtin_bit_cast(unsigned long long, (double)scaled + 6755399441055744.0) - 0x4338000000000000ull;
 }
-// What is not finite, for fixed_large: an infinite value counts as 2^22, which 65536 of stay inside 64 bits and one of is infinite again as fp16; no number as zero.
-__device__ __forceinline__ float fixed_bounded(float scaled) { return scaled != scaled ? 0.f : fminf(fmaxf(scaled, -70368744177664.f), 70368744177664.f); }
+// What is not finite adds nothing to a sum: no number counts as zero, and an infinite value leaves a mark beside it, two bits for each feature (one for either sign), four for an
+// entry.  (A large whole number in its place is brought back by enough finite values of the other sign, or wraps round with others like it: both gave finite gradients.)
+__device__ __forceinline__ float finite_or_zero(float x) { return fabsf(x) < __builtin_inff() ? x : 0.f; }
+__device__ __forceinline__ uint32_t infinite_mark(float x) { return fabsf(x) == __builtin_inff() ? 1u + (__builtin_bit_cast(uint32_t, x) >> 31) : 0u; }
+__device__ __forceinline__ uint32_t infinite_mark(float x, float y) { return infinite_mark(x) | infinite_mark(y) << 2; }
+__device__ __forceinline__ float marked_sum(float sum, uint32_t bits) {  // infinite, or no number where there were both signs
+	return bits == 0u ? sum : __builtin_bit_cast(float, 0x7F800000u | (bits & 2u) << 30 | (bits & bits >> 1) << 22);
+}
+__device__ __forceinline__ float2 marked_sums(float2 sums, uint32_t bits) { return make_float2(marked_sum(sums.x, bits & 3u), marked_sum(sums.y, bits >> 2 & 3u)); }
+constexpr uint32_t MARKS_PER_WORD = 8;  // entries' marks in 32 bits
 __device__ __forceinline__ float from_fixed(unsigned long long q) {
 	return (float)fma((double)(int32_t)(q >> 32), 4294967296.0, (double)(uint32_t)q) * (1.f / FIX_SCALE);
 }
@@ -938,6 +947,25 @@ __device__ __forceinline__ void grid_reduce_out(const N2ReduceItem& it, unsigned
 	}
 }
 
+// What is infinite of them, over those sums: the marks of four entries at a time, and back to zero.
+template <bool ACCUMULATE>
+__device__ __forceinline__ void grid_reduce_marked(const N2ReduceItem& it, uint16_t* marks, __half2* __restrict__ grads, float2* __restrict__ partials) {
+	__syncthreads();  // (the sums may be other threads')
+	float* const image = reinterpret_cast<float*>(partials + ((size_t)it.l.part_begin + (size_t)it.bucket * it.l.groups + it.group) * BKT_ENTRIES);
+	__half* const grad = reinterpret_cast<__half*>(grads + it.l.offset + it.bucket * it.l.bucket_entries);
+	for (uint32_t at = threadIdx.x; at < BKT_ENTRIES / 4u; at += RED_BLOCK) {
+		const uint32_t m = marks[at];
+		if (m == 0u) continue;
+		marks[at] = 0u;
+		for (uint32_t v = 0; v < 8; ++v) {  // two values of four entries
+			const uint32_t bits = m >> (2u * v) & 3u, place = at * 8u + v;
+			if (bits == 0u) continue;
+			if (it.l.groups > 1u) image[place] = marked_sum(0.f, bits);
+			else grad[place] = __float2half(marked_sum(0.f, bits) + (ACCUMULATE ? __half2float(grad[place]) : 0.f));
+		}
+	}
+}
+
 // A reduce launch's queue: a workgroup begins with the item of its own number and goes on with what it draws, for items differ by a factor of three in what
 // they take (dealt out by numbers alone, a training step's launch had its median workgroup end at 32 us and its last one at 46.9; drawn two ahead 34.2 and 43.6, so 34.5 and 40.9).
 // One counter for each XCD, in a line of its own; the sorting launch in front clears them.
@@ -955,7 +983,7 @@ template <bool PAIR, uint32_t FLIGHT, bool ACCUMULATE>
 __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, const uint32_t lane_end, uint32_t& item, const uint32_t end, const uint32_t tiles, const uint32_t slot_records,
                                                   const uint32_t part_shift, const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                   const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, float2* __restrict__ partials,
-                                                  unsigned long long* acc, uint32_t* queue, uint32_t* drawn) {
+                                                  unsigned long long* acc, uint32_t* marks, uint32_t* queue, uint2* drawn) {
 	typedef typename std::conditional<PAIR, uint2, uint32_t>::type value;
 	constexpr uint32_t WAVES = RED_BLOCK / 64, STEP = 64u * FLIGHT;
 	if (item >= end) return;
@@ -1011,6 +1039,7 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 		for (uint32_t u = 0; u < FLIGHT; ++u) load(q[u]);
 	};
 	constexpr uint32_t EACH = PAIR ? 2u : 1u;  // entries of a record
+	bool not_finite = false;  // a value of the wave's records of this item is not
 	auto add_step = [&](const Record (&q)[FLIGHT], uint32_t from) __attribute__((always_inline)) {
 		float f[FLIGHT][2 * EACH], most = 0.f;  // (of lanes behind the last record those of the last one)
 #pragma unroll
@@ -1046,7 +1075,8 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 #pragma unroll
 				for (uint32_t u = 0; u < FLIGHT; ++u)
 #pragma unroll
-					for (uint32_t e = 0; e < 2 * EACH; ++e) f[u][e] = fixed_bounded(f[u][e]);
+					for (uint32_t e = 0; e < 2 * EACH; ++e) f[u][e] = finite_or_zero(f[u][e]);
+				not_finite = true;
 			}
 			add([](float x) { return fixed_large(x); });
 		} else add([](float x) { return fixed_small(x); });
@@ -1078,14 +1108,40 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 			take(it, first, bounds(it, first));
 			if (total > 0u) load_step(qa);
 		}
+		if (not_finite) {  // (once more through them, for the marks: with those left on the way, 2^18 uniform points lose 4 % of the launch)
+			not_finite = false;
+			for (uint32_t first = wave; first < runs_of(it); first += WAVES * 64u) {
+				take(it, first, bounds(it, first));
+				while (at < total) {
+					Record q;
+					load(q);
+					if (at - 64u + lane >= total) continue;
+					for (uint32_t e = 0; e < EACH; ++e) {
+						uint32_t raw, entry = q.key & (BKT_ENTRIES - 1u);
+						if constexpr (PAIR) {
+							raw = e ? q.v.y : q.v.x;
+							if (e) entry ^= (2u << (q.key >> BKT_SHIFT)) - 1u;
+						} else raw = q.v;
+						const float2 v = __half22float2(*reinterpret_cast<const __half2*>(&raw));
+						const uint32_t mark = infinite_mark(v.x, v.y);
+						if (mark == 0u) continue;
+						atomicOr(&marks[entry / MARKS_PER_WORD], mark << (entry % MARKS_PER_WORD * 4u));
+						drawn->y = 1u;
+					}
+				}
+			}
+		}
 		n2_four_entries old[RED_WRITES];
 		if (ACCUMULATE) grid_reduce_old(it, grads, old);
-		if (threadIdx.x == 0u) *drawn = draw;
+		if (threadIdx.x == 0u) drawn->x = draw;
 		__syncthreads();
-		item = n2_queue_item(__builtin_amdgcn_readfirstlane(*drawn));
+		const uint2 now = *drawn;
+		const bool any_marks = __builtin_amdgcn_readfirstlane(now.y) != 0u;
+		item = n2_queue_item(__builtin_amdgcn_readfirstlane(now.x));
 		const N2ReduceItem next = n2_reduce_item(plan, lane_end, min(item, end - 1u));
 		const uint32_t two = bounds(next, wave);
 		grid_reduce_out<ACCUMULATE>(it, acc, grads, old, partials);
+		if (any_marks) grid_reduce_marked<ACCUMULATE>(it, reinterpret_cast<uint16_t*>(marks), grads, partials);
 		if (item < end) {
 			take(next, wave, two);
 			if (total > 0u) load_step(qa);
@@ -1111,12 +1167,15 @@ __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan 
 	// one plane per feature: lanes of a wave's atomic then spread over all bank pairs (entry-major pairs of features would
 	// leave every other pair unused)
 	__shared__ __align__(16) unsigned long long acc[2 * BKT_ENTRIES];
-	__shared__ uint32_t drawn;
+	__shared__ uint32_t marks[BKT_ENTRIES / MARKS_PER_WORD];
+	__shared__ uint2 drawn;  // x: the item drawn, y: whether there were marks since the workgroup began
 	const uint32_t lane_end = n2_lane_end(plan), items = plan.begin[N2_MAX_LEVELS];
 	for (uint32_t e = threadIdx.x; e < BKT_ENTRIES; e += RED_BLOCK) reinterpret_cast<ulonglong2*>(acc)[e] = make_ulonglong2(0ull, 0ull);
+	for (uint32_t e = threadIdx.x; e < BKT_ENTRIES / MARKS_PER_WORD; e += RED_BLOCK) marks[e] = 0u;
+	if (threadIdx.x == 0u) drawn.y = 0u;
 	uint32_t item = blockIdx.x;
-	grid_reduce_items<false, 6, ACCUMULATE>(plan, lane_end, item, plan.pairs_from, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, queue, &drawn);
-	grid_reduce_items<true, 3, ACCUMULATE>(plan, lane_end, item, items, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, queue, &drawn);
+	grid_reduce_items<false, 6, ACCUMULATE>(plan, lane_end, item, plan.pairs_from, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, marks, queue, &drawn);
+	grid_reduce_items<true, 3, ACCUMULATE>(plan, lane_end, item, items, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, marks, queue, &drawn);
 }
 
 // Small batches: the gradient of a bucket with few records.
@@ -1137,10 +1196,10 @@ constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 5120;
 constexpr uint32_t FEW_AT_A_TIME = 1024;                            // workgroups of a launch: what runs at one time (a multiple of the XCDs)
 constexpr uint32_t FEW_TILES = 64;                                  // a lane of every wave looks up one tile's run
 constexpr uint32_t FEW_CLAIMS = (FEW_WORDS - BKT_ENTRIES / 4) / 2;  // sums of both features, beside the table of 16-bit claims
-constexpr uint32_t FEW_RANGE = FEW_WORDS / 2;                       // entries of an image
+constexpr uint32_t FEW_RANGE = FEW_WORDS * 16 / 33 / 8 * 8;          // entries of an image: two sums and four bits of marks each
 constexpr uint32_t FEW_PAIRS = 768;                                 // pair records of a bucket, on average, in a batch that takes the kernel (batch_buckets)
 
-// Here x * 2^32 as a two's complement 64-bit integer, for any fp16 value x: the high word is floor(x), the low word the rest, both exact.  (Five instructions and no
+// Here x * 2^32 as a two's complement 64-bit integer, for any finite fp16 value x: the high word is floor(x), the low word the rest, both exact; zero for what is no number.  (Five instructions and no
 // branch, whatever the value: a few records a thread, whose latency counts.)
 __device__ __forceinline__ unsigned long long few_to_fixed(float x) {
 	const float fl = floorf(x);
@@ -1202,14 +1261,25 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 		if constexpr (sizeof(value) == 8) return q ? v.y : v.x;
 		else return v;
 	};
-	auto sum_of = [&](uint32_t old, unsigned long long a, unsigned long long b) {
-		float2 f = accumulate ? __half22float2(*reinterpret_cast<const __half2*>(&old)) : make_float2(0.f, 0.f);
-		return __floats2half2_rn(f.x + few_from_fixed(a), f.y + few_from_fixed(b));
+	auto sum_of = [&](uint32_t old, unsigned long long a, unsigned long long b, uint32_t marks) {
+		const float2 f = accumulate ? __half22float2(*reinterpret_cast<const __half2*>(&old)) : make_float2(0.f, 0.f);
+		float2 sum = make_float2(few_from_fixed(a), few_from_fixed(b));
+		if (marks != 0u) sum = marked_sums(sum, marks);
+		return __floats2half2_rn(f.x + sum.x, f.y + sum.y);
+	};
+	// adds a record's two values; `mark` leaves the marks of infinite ones
+	auto add = [&](unsigned long long* x, unsigned long long* y, uint32_t raw, auto mark) __attribute__((always_inline)) {
+		const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
+		if (fabsf(f.x) == __builtin_inff() || fabsf(f.y) == __builtin_inff()) mark(infinite_mark(f.x, f.y));  // (whatever it adds to its sum, the mark stands for it)
+		atomicAdd(x, few_to_fixed(f.x));
+		atomicAdd(y, few_to_fixed(f.y));
 	};
 	if (claims && runs.total * EACH <= FEW_CLAIMS) {
-		uint16_t* claim = reinterpret_cast<uint16_t*>(mem);
+		uint16_t* claim = reinterpret_cast<uint16_t*>(mem);  // a record's number, and from 2^12 on the entry's marks
+		constexpr uint32_t NUMBERS = (1u << 12) - 1u;
+		static_assert(FEW_CLAIMS <= NUMBERS, "the numbers of records leave room for the marks");
 		unsigned long long* acc = mem + BKT_ENTRIES / 4;
-		uint32_t key[K], e[K][EACH], by[K][EACH], old[K][EACH];
+		uint32_t key[K], e[K][EACH], old[K][EACH];
 		value v[K];
 #pragma unroll
 		for (uint32_t k = 0; k < K; ++k) {
@@ -1234,12 +1304,9 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 			if (threadIdx.x + k * FEW_BLOCK >= runs.total) break;
 #pragma unroll
 			for (uint32_t q = 0; q < EACH; ++q) {
-				by[k][q] = claim[e[k][q]];
-				const uint32_t raw = word(v[k], q);
-				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
-				atomicAdd(&acc[by[k][q]], few_to_fixed(f.x));
-				atomicAdd(&acc[FEW_CLAIMS + by[k][q]], few_to_fixed(f.y));
-				old[k][q] = accumulate && by[k][q] == (threadIdx.x + k * FEW_BLOCK) * EACH + q && e[k][q] < left ? *reinterpret_cast<const uint32_t*>(G + e[k][q]) : 0u;
+				const uint32_t by = claim[e[k][q]] & NUMBERS;
+				add(&acc[by], &acc[FEW_CLAIMS + by], word(v[k], q), [&](uint32_t m) { atomicOr(reinterpret_cast<uint32_t*>(mem) + e[k][q] / 2u, m << (e[k][q] % 2u * 16u + 12u)); });
+				old[k][q] = accumulate && by == (threadIdx.x + k * FEW_BLOCK) * EACH + q && e[k][q] < left ? *reinterpret_cast<const uint32_t*>(G + e[k][q]) : 0u;
 			}
 		}
 		__syncthreads();
@@ -1249,16 +1316,21 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 			if (r >= runs.total) break;
 #pragma unroll
 			for (uint32_t q = 0; q < EACH; ++q) {
-				const uint32_t id = r * EACH + q;
-				if (by[k][q] != id || e[k][q] >= left) continue;
-				G[e[k][q]] = sum_of(old[k][q], acc[id], acc[FEW_CLAIMS + id]);
+				const uint32_t id = r * EACH + q, by = claim[e[k][q]];
+				const unsigned long long x = acc[id], y = acc[FEW_CLAIMS + id];
+				if ((by & NUMBERS) != id || e[k][q] >= left) continue;
+				G[e[k][q]] = sum_of(old[k][q], x, y, by >> 12);
 			}
 		}
 		return;
 	}
+	uint32_t* const marks = reinterpret_cast<uint32_t*>(mem + 2u * FEW_RANGE);
+	static_assert(2u * FEW_RANGE * sizeof(*mem) + FEW_RANGE / MARKS_PER_WORD * sizeof(*marks) <= FEW_WORDS * sizeof(*mem), "an image and its marks");
 	for (uint32_t from = 0; from < left; from += FEW_RANGE) {
 		const uint32_t n = min(FEW_RANGE, left - from);
 		for (uint32_t e = threadIdx.x; e < n; e += FEW_BLOCK) { mem[e] = 0ull; mem[FEW_RANGE + e] = 0ull; }
+		if (threadIdx.x < FEW_RANGE / MARKS_PER_WORD) marks[threadIdx.x] = 0u;
+		static_assert(FEW_RANGE / MARKS_PER_WORD <= FEW_BLOCK, "a word of marks to a thread");
 		__syncthreads();
 		for (uint32_t r = threadIdx.x; __any(r < runs.total); r += FEW_BLOCK) {
 			uint32_t key, e[EACH];
@@ -1267,11 +1339,9 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 			places(key, e);
 #pragma unroll
 			for (uint32_t q = 0; q < EACH; ++q) {
-				const uint32_t at = e[q] - from, raw = word(v, q);
+				const uint32_t at = e[q] - from;
 				if (r >= runs.total || at >= n) continue;
-				const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&raw));
-				atomicAdd(&mem[at], few_to_fixed(f.x));
-				atomicAdd(&mem[FEW_RANGE + at], few_to_fixed(f.y));
+				add(&mem[at], &mem[FEW_RANGE + at], word(v, q), [&](uint32_t m) { atomicOr(&marks[at / MARKS_PER_WORD], m << (at % MARKS_PER_WORD * 4u)); });
 			}
 		}
 		__syncthreads();
@@ -1279,9 +1349,10 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 			wide* at = reinterpret_cast<wide*>(G + from + e);
 			const wide old = accumulate ? *at : wide(0u);
 			wide out;
+			const uint32_t four_marks = marks[e / MARKS_PER_WORD] >> (e % MARKS_PER_WORD * 4u);
 #pragma unroll
 			for (uint32_t q = 0; q < 4; ++q) {
-				const __half2 h = sum_of(old[q], mem[e + q], mem[FEW_RANGE + e + q]);
+				const __half2 h = sum_of(old[q], mem[e + q], mem[FEW_RANGE + e + q], four_marks >> (q * 4u) & 15u);
 				out[q] = *reinterpret_cast<const uint32_t*>(&h);
 			}
 			*at = out;

@@ -356,6 +356,59 @@ def test_sorted_scatter_is_exact_for_values_of_all_sizes(n, levels, log2_size, b
         assert not bad.any(), (mode, int(bad.sum()), got[bad][:4], ref[bad][:4], want[bad][:4])
 
 
+@pytest.mark.parametrize("n", [200, 40000])  # the kernel for few records and the other one
+@pytest.mark.parametrize("levels,log2_size,base", [(1, 19, 16), (1, 16, 64), (1, 16, 37), (2, 6, 16)])  # dense, hashed, levels that keep an image, buckets split over several workgroups
+def test_infinite_records_are_neither_cancelled_nor_wrapped(n, levels, log2_size, base):
+    """An entry with infinite records of one sign has an infinite gradient, however many there are (two, every 64th point) and however large finite ones of the
+    other sign (up to 65504 / 8, over a thousand of them); one with both signs has no number, as the sum has none.  No two points of a run of equal cells that would be merged."""
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
+    gg = GridEncoding(n_levels=levels, log2_hashmap_size=log2_size, base_resolution=base, per_level_scale=1.0)
+    gen = torch.Generator(device="cuda").manual_seed(n + base)
+    dp = torch.zeros(gg.n_params(), device="cuda").half()
+    dg = torch.full_like(dp, 5.0)
+    gg.set_params(dp, dg)
+    assert gg.reserve_scatter_workspace(n)
+    cells = torch.randint(0, base - 1, (3, n), device="cuda", generator=gen)
+    i = torch.arange(n, device="cuda")
+    dy = torch.randn((2 * levels, n), device="cuda", generator=gen)
+    for k, cell, values in ((3, 2, (65504.0, -65504.0)), (5, 6, (-65504.0, 65504.0)), (7, 10, (65504.0, 1.0))):  # every eighth point: three cells with large values
+        cells[:, i % 8 == k] = cell
+        dy[:, i % 8 == k] = torch.tensor(values * levels, device="cuda").view(-1, 1)
+    inf = float("inf")
+    for start, pair in ((3, (-inf, inf)), (5, (inf, -inf)), (7, (-inf, -inf))):  # of those points every 64th, and so more than one of 200
+        dy[:, start::64] = torch.tensor(pair * levels, device="cuda").view(-1, 1)
+    dy[0, 15] = inf  # both signs at the third one
+    dy = dy.half()
+    x = (cells.float() / (base - 1)).contiguous()
+    at = gg.corner_indices(x).long()
+    offsets = gg.level_table()[3]
+    ref = torch.zeros((dg.numel() // 2, 2), device="cuda", dtype=torch.float64)
+    marks = torch.zeros((2,) + ref.shape, device="cuda", dtype=torch.float64)
+    for l in range(levels):
+        to = at[l].reshape(-1) + int(offsets[l])
+        for f in range(2):
+            rec = dy[2 * l + f].double() / 8
+            ref[:, f].index_add_(0, to, torch.where(rec.isfinite(), rec, 0.0).repeat(8))
+            for sign in range(2):
+                marks[sign, :, f].index_add_(0, to, (rec == (-inf if sign else inf)).double().repeat(8))
+    assert (marks.amax((1, 2)) >= 2).all() and bool(((marks[0] > 0) & (marks[1] > 0)).any())
+    want = torch.where(marks[0] > 0, inf, torch.where(marks[1] > 0, -inf, ref))
+    want = torch.where((marks[0] > 0) & (marks[1] > 0), float("nan"), want).half()
+    for mode in (GRAD_OVERWRITE, GRAD_ACCUMULATE, GRAD_OVERWRITE):  # (the second order of calls: nothing stays marked)
+        gg.backward(None, x, dy, mode=mode)
+        got = dg.reshape(-1, 2)
+        special = ~want.isfinite()
+        same = (got == want) | (got.isnan() & want.isnan())
+        assert bool(same[special].all()), (mode, got[special & ~same][:4], want[special & ~same][:4])
+        if mode == GRAD_OVERWRITE:
+            assert bool(got[~special].isfinite().all())
+            assert rel_l2(host(got[~special]), host(want[~special])) < RTOL
+    dy = torch.where(dy.isfinite(), dy, torch.zeros_like(dy))
+    gg.backward(None, x, dy, mode=GRAD_OVERWRITE)
+    fits = ref.half().isfinite()
+    assert rel_l2(host(dg.reshape(-1, 2)[fits]), host(ref[fits])) < RTOL
+
+
 @pytest.mark.parametrize("n,room", [(512, 512), (513, 513), (513, 70000), (16384, 16384), (16384, 16385)])
 def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     """The sums are exact, so the size of a tile leaves no trace: a batch equals the one that has points without a gradient behind it, up to where
