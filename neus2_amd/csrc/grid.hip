@@ -866,6 +866,13 @@ __device__ __forceinline__ float from_fixed(unsigned long long q) {
 	return (float)fma((double)(int32_t)(q >> 32), 4294967296.0, (double)(uint32_t)q) * (1.f / FIX_SCALE);
 }
 
+// A sum in fp32 and the gradient that it is added to, in fp32, so that all ways to the sum round alike, to fp32 and then to fp16.  (Left to the compiler, the sum's factor,
+// the addition and the conversion are one instruction in some kernels, which rounds once.)
+__device__ __forceinline__ float2 added_to(float2 sum, float2 old) {
+#pragma clang fp contract(off)
+	return make_float2(sum.x + old.x, sum.y + old.y);
+}
+
 // Which (level, bucket, group of tiles) is an item?  (Lane l asks about place l: sixteen scalar loads one after the other were a microsecond.)
 struct N2ReduceItem {
 	uint32_t bucket, group;
@@ -937,7 +944,7 @@ __device__ __forceinline__ void grid_reduce_out(const N2ReduceItem& it, unsigned
 				if (ACCUMULATE) {
 					const uint32_t o = old[k][q + p];
 					const float2 g = __half22float2(*reinterpret_cast<const __half2*>(&o));
-					f = make_float2(f.x + g.x, f.y + g.y);
+					f = added_to(f, g);
 				}
 				const __half2 h = __floats2half2_rn(f.x, f.y);
 				out[q + p] = *reinterpret_cast<const uint32_t*>(&h);
@@ -1265,7 +1272,8 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 		const float2 f = accumulate ? __half22float2(*reinterpret_cast<const __half2*>(&old)) : make_float2(0.f, 0.f);
 		float2 sum = make_float2(few_from_fixed(a), few_from_fixed(b));
 		if (marks != 0u) sum = marked_sums(sum, marks);
-		return __floats2half2_rn(f.x + sum.x, f.y + sum.y);
+		const float2 all = added_to(sum, f);
+		return __floats2half2_rn(all.x, all.y);
 	};
 	// adds a record's two values; `mark` leaves the marks of infinite ones
 	auto add = [&](unsigned long long* x, unsigned long long* y, uint32_t raw, auto mark) __attribute__((always_inline)) {

@@ -409,6 +409,30 @@ def test_infinite_records_are_neither_cancelled_nor_wrapped(n, levels, log2_size
     assert rel_l2(host(dg.reshape(-1, 2)[fits]), host(ref[fits])) < RTOL
 
 
+@pytest.mark.parametrize("n", [200, 40000])  # the kernel for few records and the other one
+@pytest.mark.parametrize("levels,log2_size,base", [(1, 19, 16), (1, 16, 64), (1, 16, 37)])  # dense, hashed, buckets of several sizes
+def test_an_accumulating_scatter_rounds_to_fp32_and_then_to_fp16(n, levels, log2_size, base):
+    """1024 + (0.5 + 2^-24) is 1024.5 in fp32 and, of two neighbours at the same distance, the even 1024 in fp16; in one rounding it would be 1025."""
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GridEncoding
+    gg = GridEncoding(n_levels=levels, log2_hashmap_size=log2_size, base_resolution=base, per_level_scale=1.0)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    dp = torch.zeros(gg.n_params(), device="cuda").half()
+    dg = torch.full_like(dp, 1024.0)
+    gg.set_params(dp, dg)
+    assert gg.reserve_scatter_workspace(n)
+    cells = torch.randint(0, base - 1, (3, n), device="cuda", generator=gen)
+    cells[:, n // 3::n // 3] = 2
+    i = torch.arange(n, device="cuda")
+    dy = torch.where(i == n // 3, 4.0, torch.where(i == n // 3 * 2, 2.0 ** -21, 0.0)).expand(2 * levels, n).half().contiguous()  # (a record is an eighth of it)
+    x = (cells.float() / (base - 1)).contiguous()
+    at = gg.corner_indices(x)[0].long()
+    ref = torch.zeros(dg.numel() // 2, device="cuda", dtype=torch.float64).index_add_(0, at.reshape(-1), dy[0].double().repeat(8) / 8)
+    assert int((ref == 0.5 + 2.0 ** -24).sum()) == 8
+    gg.backward(None, x, dy, mode=GRAD_ACCUMULATE)
+    want = (ref.float() + 1024.0).half()
+    assert bool((want == 1024.0).all()) and torch.equal(dg.reshape(-1, 2), want[:, None].expand(-1, 2))
+
+
 @pytest.mark.parametrize("n,room", [(512, 512), (513, 513), (513, 70000), (16384, 16384), (16384, 16385)])
 def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     """The sums are exact, so the size of a tile leaves no trace: a batch equals the one that has points without a gradient behind it, up to where
