@@ -458,7 +458,7 @@ __host__ __device__ constexpr uint32_t bin_records(uint32_t per) { return bin_po
 // (see n2_queue_draw)
 constexpr uint32_t QUEUE_STRIDE = 32, QUEUE_WORDS = N_XCD * QUEUE_STRIDE;
 
-// The items of a reduce launch, a (bucket, group of tiles) each, by level: first the levels of single records, then those of pair records.
+// The items of a reduce launch, a (bucket, group of tiles) each, by level: levels of one kind of records, single ones or pairs, then those of the other.
 struct N2BucketPlan {
 	uint32_t begin[N2_MAX_LEVELS + 1];  // first item of each place in that order
 	struct Level {
@@ -469,7 +469,7 @@ struct N2BucketPlan {
 		uint32_t entries, offset; // the level's table
 		uint32_t pair;
 	} at[N2_MAX_LEVELS];
-	uint32_t pairs_from;  // first item of a level of pair records
+	uint32_t second_from;  // first item of the second kind
 };
 
 // what a point brings along: its position, dL/dy of the level's two features, g2 of them and v
@@ -842,6 +842,7 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 // fp16 values, i.e. multiples of 2^-24 below 2^16, so value * 2^24 is an exact integer below 2^40 and the
 // sum of a whole bucket stays far inside 64 bits.  The accumulation is exact and independent of order.
 constexpr uint32_t RED_BLOCK = 512;               // 8 waves; two workgroups share a CU
+constexpr uint32_t RED_FLIGHT = 6, RED_FLIGHT_PAIRS = 3;  // single records, and pairs, that a lane has under way at a time
 constexpr uint32_t RED_AT_A_TIME = 512;           // workgroups of a launch: what runs at one time (a multiple of the XCDs)
 constexpr float FIX_SCALE = 16777216.0f;          // 2^24
 
@@ -1166,7 +1167,7 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 // in flight) 50.6, 1024 (64 registers spill) 66.0; two, three or four times 64 records in flight 51.3, 50.7, 50.4; items dealt out by number 53.2, training step 51.0.
 // Values from 128 on (a second order's, whose J holds the level's scale) take an instruction more, chosen for a wave's step as a whole: second order and both others on 60 000
 // points along rays 100.0 -> 95.7, 2^18 287 -> 285.  Points packed into a fifth of the cube's side lose 3 to 5 per cent: a few full buckets, with half the threads to each.
-template <bool ACCUMULATE>
+template <bool ACCUMULATE, bool PAIRS_FIRST>
 __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records, uint32_t part_shift,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                    const uint16_t* __restrict__ offsets,
@@ -1181,8 +1182,15 @@ __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan 
 	for (uint32_t e = threadIdx.x; e < BKT_ENTRIES / MARKS_PER_WORD; e += RED_BLOCK) marks[e] = 0u;
 	if (threadIdx.x == 0u) drawn.y = 0u;
 	uint32_t item = blockIdx.x;
-	grid_reduce_items<false, 6, ACCUMULATE>(plan, lane_end, item, plan.pairs_from, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, marks, queue, &drawn);
-	grid_reduce_items<true, 3, ACCUMULATE>(plan, lane_end, item, items, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, marks, queue, &drawn);
+#define ITEMS(P, FLIGHT, END) grid_reduce_items<P, FLIGHT, ACCUMULATE>(plan, lane_end, item, END, tiles, slot_records, part_shift, rec_vals, rec_keys, offsets, grads, partials, acc, marks, queue, &drawn)
+	if (PAIRS_FIRST) {
+		ITEMS(true, RED_FLIGHT_PAIRS, plan.second_from);
+		ITEMS(false, RED_FLIGHT, items);
+	} else {
+		ITEMS(false, RED_FLIGHT, plan.second_from);
+		ITEMS(true, RED_FLIGHT_PAIRS, items);
+	}
+#undef ITEMS
 }
 
 // Small batches: the gradient of a bucket with few records.
@@ -1846,9 +1854,20 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 		split_begin[l] = split;
 		if (buckets.groups[l] > 1) { images += buckets.count[l] * buckets.groups[l]; split += buckets.count[l]; }
 	}
+	// The kind whose largest items, on average, have more additions comes first, or a launch ends with one of them that has just begun.  Levels of pairs have those where
+	// their buckets are full (tables of 2^14 and 2^16 entries a level, whose pairs' items have 65 536 additions of 2^18 points, the others' 16 384 to 27 000): single ones
+	// first | pairs first, the launch in us, 2^18 points along rays 48.3 | 30.8 and 52.8 | 36.1, uniform 52.3 | 48.6 (2^16).  With the default table they have as many or fewer:
+	// 2^18 uniform points 52.6 | 56.1, along rays 45.4 | 46.5, 52 344 18.9 | 19.9.
+	uint64_t largest[2] = {0, 0};
+	for (uint32_t l = 0; l < L; ++l) {
+		uint64_t& most = largest[(tab.pair_levels >> l) & 1u];
+		most = std::max(most, (uint64_t)n_points * 8u / (buckets.count[l] * buckets.groups[l]));
+	}
+	const bool pairs_first = !buckets.few && largest[1] > largest[0];  // (the kernel for few records has them behind the others always: its items are small)
 	uint32_t place = 0;
-	for (uint32_t pair = 0; pair < 2; ++pair) {
-		if (pair) plan.pairs_from = wg;
+	for (uint32_t kind = 0; kind < 2; ++kind) {
+		const uint32_t pair = pairs_first == (kind == 0u);
+		if (kind) plan.second_from = wg;
 		for (uint32_t l = 0; l < L; ++l) {
 			if (((tab.pair_levels >> l) & 1u) != pair) continue;
 			plan.begin[place] = wg;
@@ -1894,7 +1913,7 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	if (buckets.few)
 		grid_reduce_few_kernel<<<dim3(wg < FEW_AT_A_TIME ? wg : FEW_AT_A_TIME), dim3(FEW_BLOCK), 0, s>>>(plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
 	else {
-		auto* const kernel = accumulate ? grid_reduce_kernel<true> : grid_reduce_kernel<false>;
+		auto* const kernel = pairs_first ? (accumulate ? grid_reduce_kernel<true, true> : grid_reduce_kernel<false, true>) : accumulate ? grid_reduce_kernel<true, false> : grid_reduce_kernel<false, false>;
 		kernel<<<dim3(wg < RED_AT_A_TIME ? wg : RED_AT_A_TIME), dim3(RED_BLOCK), 0, s>>>(plan, tiles, bin_records(per), part_shift, rec_vals, rec_keys, offsets, grid->grads, partials, queue);
 	}
 	N2_LAUNCH_CHECK();

@@ -433,6 +433,29 @@ def test_an_accumulating_scatter_rounds_to_fp32_and_then_to_fp16(n, levels, log2
     assert bool((want == 1024.0).all()) and torch.equal(dg.reshape(-1, 2), want[:, None].expand(-1, 2))
 
 
+# full buckets of pair records in front of the others: split, whole, in accumulating launches of more items than run at one time; behind them; single records alone
+@pytest.mark.parametrize("levels,log2_size,n", [(4, 14, 40000), (5, 16, 70000), (16, 16, 140000), (5, 19, 70000), (2, 19, 40000)])
+def test_sorted_scatter_with_either_kind_of_records_first(oracle, levels, log2_size, n):
+    from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
+    cfg = {**CFG, "n_levels": levels, "log2_hashmap_size": log2_size}
+    og = oracle.Grid(cfg["n_levels"], cfg["log2_hashmap_size"], cfg["base_resolution"], cfg["per_level_scale"])
+    gg = GridEncoding(**cfg)
+    rng = np.random.default_rng(n)
+    dp = dev(q16(rng.uniform(-1, 1, og.n_params)), torch.float16)
+    dg = torch.full_like(dp, 9.0)
+    gg.set_params(dp, dg)
+    assert gg.reserve_scatter_workspace(n)
+    xyz = rng.random((3, n), dtype=np.float32)
+    dy = q16(rng.standard_normal((2 * levels, n)))
+    ref, _ = og.backward(host(dp), xyz, dy, want_dx=False)
+    for mode, times in ((GRAD_OVERWRITE, 1), (GRAD_ACCUMULATE, 2)):
+        gg.backward(None, dev(xyz), dev(dy, torch.float16), mode=mode)
+        got = host(dg)
+        for l in range(levels):
+            a, b = int(og.offset[l]) * 2, int(og.offset[l + 1]) * 2
+            assert rel_l2(got[a:b], times * ref[a:b]) < RTOL, (mode, l)
+
+
 @pytest.mark.parametrize("n,room", [(512, 512), (513, 513), (513, 70000), (16384, 16384), (16384, 16385)])
 def test_sorted_scatter_tiles_of_one_and_two_points_per_thread(oracle, n, room):
     """The sums are exact, so the size of a tile leaves no trace: a batch equals the one that has points without a gradient behind it, up to where
