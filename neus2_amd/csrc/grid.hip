@@ -975,7 +975,9 @@ __device__ __forceinline__ void grid_reduce_marked(const N2ReduceItem& it, uint1
 }
 
 // A reduce launch's queue: a workgroup begins with the item of its own number and goes on with what it draws, for items differ by a factor of three in what
-// they take (dealt out by numbers alone, a training step's launch had its median workgroup end at 32 us and its last one at 46.9; drawn two ahead 34.2 and 43.6, so 34.5 and 40.9).
+// they take (dealt out by numbers alone, a training step's launch had its median workgroup end at 32 us and its last one at 46.9; drawn two ahead 34.2 and 43.6).  It draws when
+// it has asked for the last records of what it is at: drawn when it began, an item waited for a workgroup that a full bucket kept, and the launch for that item (52 344 points
+// in a box of a fifth of the cube's side: backward 94.4 us, now 90.7; 2^18 points 331 and 324, uniform 89.3 and 88.6).
 // One counter for each XCD, in a line of its own; the sorting launch in front clears them.
 __device__ __forceinline__ uint32_t n2_queue_draw(uint32_t* queue) { return atomicAdd(queue + blockIdx.x % N_XCD * QUEUE_STRIDE, 1u); }
 __device__ __forceinline__ uint32_t n2_queue_item(uint32_t drawn) { return blockIdx.x % N_XCD + N_XCD * ((gridDim.x + N_XCD - 1u) / N_XCD + drawn); }  // (behind all first ones)
@@ -1095,16 +1097,21 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 	__syncthreads();  // the sums are zero
 	while (true) {
 		uint32_t draw = 0u;
-		if (threadIdx.x == 0u) draw = n2_queue_draw(queue);
 		for (uint32_t first = wave;;) {
+			auto draw_behind_the_last = [&]() __attribute__((always_inline)) {
+				if (wave == 0u && first + WAVES * 64u >= runs_of(it) && lane == 0u) draw = n2_queue_draw(queue);
+			};
+			if (total == 0u) draw_behind_the_last();
 			while (total > 0u) {
 				if (at >= total) {
+					draw_behind_the_last();
 					add_step(qa, at - STEP);
 					break;
 				}
 				load_step(qb);
 				add_step(qa, at - 2u * STEP);
 				if (at >= total) {
+					draw_behind_the_last();
 					add_step(qb, at - STEP);
 					break;
 				}
