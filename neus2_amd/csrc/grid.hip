@@ -1212,7 +1212,9 @@ __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan 
 // (256 threads: the same up to 5000 points, 16 384 uniform +4; 1024: +4; 128: +0.5.  In 32 KiB there are 1536 sums instead of 2048,
 // and batches beyond 16 384 points took grid_reduce_kernel: 20 000 along rays 34.0 against 29.5.)
 // With the next item's bounds on their way meanwhile (its level and tiles looked up behind the last item's stores before): forward, backward and second order, 1000
-// points along rays 32.4 -> 30.3, 2000 33.7 -> 31.3, 5003 36.2 -> 35.2, uniform 42.7 -> 41.4; points packed into a twentieth of the cube 51.8 -> 53.4.  Half the sums and threads, seven
+// points along rays 32.4 -> 30.3, 2000 33.7 -> 31.3, 5003 36.2 -> 35.2, uniform 42.7 -> 41.4; points packed into a fifth or a twentieth of the cube's side lose the time of an
+// item, 5003 backward 33.5 -> 35.2 and 55.2 -> 56.1: a workgroup with a full bucket has another one to do.  (Drawn from the queue, late where an item is long, those take 33.0 and
+// 57.4, but 5003 along rays 19.2 -> 21.4, the way to the counter and to the bounds behind it; full buckets' kinds a workgroup each, the others in turn: 21.1.)  Half the sums and threads, seven
 // workgroups to a CU: 5003 along rays 32.6, but 6000 points of a cube's fifth 17.7 -> 31.9, whose buckets hold more records than there are sums then.
 constexpr uint32_t FEW_BLOCK = 512, FEW_WORDS = 5120;
 constexpr uint32_t FEW_AT_A_TIME = 1024;                            // workgroups of a launch: what runs at one time (a multiple of the XCDs)
@@ -1384,7 +1386,8 @@ __device__ __forceinline__ void grid_reduce_few_bucket(const uint32_t slot_recor
 	}
 }
 
-// A workgroup takes the items of its number, that and a round of workgroups further, ...; where the next one's runs lie is on its way meanwhile.
+// A workgroup takes the items of its number, that and a round of workgroups further, ... (if the launch has fewer workgroups than items); where the next one's runs lie is on
+// its way meanwhile.
 __global__ void __launch_bounds__(FEW_BLOCK, 8) grid_reduce_few_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records,
                                                                     const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
                                                                     const uint16_t* __restrict__ offsets, __half2* __restrict__ grads, int accumulate) {
@@ -1882,7 +1885,7 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 			wg += buckets.count[l] * buckets.groups[l];
 		}
 	}
-	for (; place <= N2_MAX_LEVELS; ++place) plan.begin[place] = wg;
+	for (uint32_t end = place; end <= N2_MAX_LEVELS; ++end) plan.begin[end] = wg;
 	auto bin = [&](auto per_thread) {
 		constexpr uint32_t PER = decltype(per_thread)::value;
 		// (the other launches' records exceed the card's memory before their threads exceed 32 bits: 8 and 9 threads a point of sixteen levels)
@@ -1917,9 +1920,18 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	if (per == 1u) bin(std::integral_constant<uint32_t, 1>());
 	else bin(std::integral_constant<uint32_t, 2>());
 	N2_LAUNCH_CHECK();
-	if (buckets.few)
-		grid_reduce_few_kernel<<<dim3(wg < FEW_AT_A_TIME ? wg : FEW_AT_A_TIME), dim3(FEW_BLOCK), 0, s>>>(plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
-	else {
+	if (buckets.few) {
+		// In turn, unless a workgroup with more than three records a thread of a claimed bucket would have another item to do.  Default table (its fifth level, from 16 897 points on),
+		// backward in us, a workgroup an item | in turn: uniform 12 000 points 26.2 | 25.2, 16 384 29.9 | 29.6, 18 000 31.9 | 34.2, 20 000 32.4 | 35.0, 24 000 35.5 | 38.1, along rays
+		// 12 000 22.2 | 21.8, 16 384 24.6 | 23.7, 18 000 25.3 | 24.9, 24 000 28.4 | 28.0, accumulating 16 384 24.6 | 23.6, 18 000 25.8 | 24.8, 24 000 28.4 | 27.3; with twelve of its
+		// levels, few enough that those workgroups have one item, uniform 18 000 28.8 | 28.5, 24 000 32.4 | 32.5, along rays 21.0 | 20.4, 23.4 | 22.4.
+		bool in_turn = true;
+		for (uint32_t l = 0; l < place; ++l) {
+			const N2BucketPlan::Level& at = plan.at[l];
+			if (!at.pair && at.bucket_entries > FEW_RANGE && (uint64_t)n_points * 8u > 3ull * FEW_BLOCK * at.n_buckets && plan.begin[l] + FEW_AT_A_TIME < wg) in_turn = false;
+		}
+		grid_reduce_few_kernel<<<dim3(in_turn && wg > FEW_AT_A_TIME ? FEW_AT_A_TIME : wg), dim3(FEW_BLOCK), 0, s>>>(plan, tiles, bin_records(per), rec_vals, rec_keys, offsets, grid->grads, accumulate ? 1 : 0);
+	} else {
 		auto* const kernel = pairs_first ? (accumulate ? grid_reduce_kernel<true, true> : grid_reduce_kernel<false, true>) : accumulate ? grid_reduce_kernel<true, false> : grid_reduce_kernel<false, false>;
 		kernel<<<dim3(wg < RED_AT_A_TIME ? wg : RED_AT_A_TIME), dim3(RED_BLOCK), 0, s>>>(plan, tiles, bin_records(per), part_shift, rec_vals, rec_keys, offsets, grid->grads, partials, queue);
 	}

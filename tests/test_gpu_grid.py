@@ -433,8 +433,9 @@ def test_an_accumulating_scatter_rounds_to_fp32_and_then_to_fp16(n, levels, log2
     assert bool((want == 1024.0).all()) and torch.equal(dg.reshape(-1, 2), want[:, None].expand(-1, 2))
 
 
-# full buckets of pair records in front of the others: split, whole, in accumulating launches of more items than run at one time; behind them; single records alone
-@pytest.mark.parametrize("levels,log2_size,n", [(4, 14, 40000), (5, 16, 70000), (16, 16, 140000), (5, 19, 70000), (2, 19, 40000)])
+# full buckets of pair records in front of the others: split, whole, in accumulating launches of more items than run at one time; behind them; single records alone;
+# the last batch whose few records' items are taken in turn, and the first one with a workgroup for each
+@pytest.mark.parametrize("levels,log2_size,n", [(4, 14, 40000), (5, 16, 70000), (16, 16, 140000), (5, 19, 70000), (2, 19, 40000), (16, 19, 16896), (16, 19, 16897)])
 def test_sorted_scatter_with_either_kind_of_records_first(oracle, levels, log2_size, n):
     from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
     cfg = {**CFG, "n_levels": levels, "log2_hashmap_size": log2_size}
