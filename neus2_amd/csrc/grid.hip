@@ -1167,13 +1167,14 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 	}
 }
 
-// What bounds it is instructions and the records' way through memory, about half and half: without the LDS additions 2^18 uniform points take 45.6 of 50.4 us, with
-// records out of the L1 46.8, with neither 39.6, without writing the sums 44.9.  Before, one workgroup of 1024 threads to a bucket, groups of 8 or 16
-// lanes to a tile's run, values in 2^32 fixed point by five instructions each, | now, launch in us: a training step's 56.6 | 44.5, trained 44.8 | 41.1, the SDF network's
-// 63.9 | 56.5, 52 344 samples 20.0 | 18.0, 2^18 uniform points 50.6 | 50.7 (vector instructions 24.9 | 15.5 M).  Other shapes: 256 threads 59.8, 768 (two waves' records fewer
-// in flight) 50.6, 1024 (64 registers spill) 66.0; two, three or four times 64 records in flight 51.3, 50.7, 50.4; items dealt out by number 53.2, training step 51.0.
+// What bounds it is the LDS (busy in 67 % of a CU's clocks on 2^18 uniform points, two thirds of that bank conflicts), vector instructions (69 %) and the records' way through memory;
+// of 50.4 us it took without the LDS additions 45.6, with records out of the L1 46.8, with neither 39.6, without writing the sums 44.9 (buckets drawn early then).  Before, one
+// workgroup of 1024 threads to a bucket, groups of 8 or 16 lanes to a tile's run, values in 2^32 fixed point by five instructions each, | now, launch in us: a training
+// step's 54.6 | 43.1, trained 44.5 | 40.2, the SDF network's 65.2 | 54.8, 52 344 samples 20.0 | 18.3, 2^18 uniform points 51.8 | 48.0 (vector instructions 24.9 | 15.3 M).  Other shapes, of 50.7
+// uniform: 256 threads 59.8, 768 50.6 (registers spill: an accumulating launch for 52 344 points 22 -> 29), 1024 66.0; items dealt out by number 53.2, training step 51.0.  Records under
+// way, single ones and pairs, 6 and 3: 4 and 2, and 4 and 3, take the same within 1 %, 6 and 4 1 to 2 % longer, 8 and 3 spill and take 3 to 6.
 // Values from 128 on (a second order's, whose J holds the level's scale) take an instruction more, chosen for a wave's step as a whole: second order and both others on 60 000
-// points along rays 100.0 -> 95.7, 2^18 287 -> 285.  Points packed into a fifth of the cube's side lose 3 to 5 per cent: a few full buckets, with half the threads to each.
+// points along rays 100.0 -> 95.7.  Points packed into a fifth of the cube's side, which meet a few full buckets, lose 2 per cent of a backward: 52 344 88.4 | 90.7, 2^18 319 | 325.
 template <bool ACCUMULATE, bool PAIRS_FIRST>
 __global__ void __launch_bounds__(RED_BLOCK, 4) grid_reduce_kernel(N2BucketPlan plan, uint32_t tiles, uint32_t slot_records, uint32_t part_shift,
                                                                    const uint32_t* __restrict__ rec_vals, const uint16_t* __restrict__ rec_keys,
@@ -1854,7 +1855,9 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 	N2BucketPlan plan{};
 	uint32_t wg = 0, images = 0, split = 0;
 	N2LevelTable tab = grid->tab;  // with this launch's bucket sizes
-	uint32_t part_shift = 0;  // about four parts of runs per wave of a reduce workgroup
+	// At least four runs, or parts of them, for a wave of a reduce workgroup.  One | two | four | eight, backward in us: 30 000 points uniform 35.6 | 35.3 | 35.9 | 36.9, in a box of a fifth
+	// of the cube's side 71.9 | 72.0 | 70.4 | 70.0, 52 344 uniform 40.9 | 40.9 | 40.9 | 41.6, with tables of 2^14 entries a level 42.3 | 42.2 | 42.3 | 41.3.
+	uint32_t part_shift = 0;
 	while (part_shift < 6u && tiles << part_shift < RED_BLOCK / 64u * 4u) ++part_shift;
 	const BatchBuckets buckets = batch_buckets(grid, n_points);
 	uint32_t split_begin[N2_MAX_LEVELS], part_begin[N2_MAX_LEVELS];

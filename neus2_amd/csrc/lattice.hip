@@ -14,8 +14,8 @@
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
 // 512^3 lattice 4.26 ms in ten slabs: a plane takes 4.7 us for six fine levels and 3.5 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
-// the L1's data return (busy in 88 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by vector instructions (64 %) and
-// by the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
+// the L1's data return (busy in 95 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by the same (87 %), vector instructions (70 %) and
+// the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
 // fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's walk and
 // the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
 // Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before these slabs, starts and lengths of waves | now: 80^3 81 | 74 us, 96^3
@@ -308,7 +308,7 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 	// The second layer, of which only row 0 is wanted: a lane holds half of its sample's hidden values (the other group the
 	// other half).  Dot products on the vector unit take a third of the time of four more MFMAs per tile.
 	// (one tile after the other: side by side they take 32 registers more, and a third wave has no room; the weights of 32 rows serve both: read for each
-	// tile anew, and with registers spilled whose return waits for the loads of two steps, the walk took 4.2 us a plane of 512^2, then 3.9)
+	// tile anew, and with registers spilled whose return waits for the loads of two steps, the walk took 4.2 us a plane of 512^2, then 3.9; 3.5 with what depends on x in LDS)
 	float dot[2] = {0.f, 0.f};
 #pragma unroll
 	for (int mt = 0; mt < 2; ++mt) {
@@ -367,8 +367,8 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	n2_locate(lane_f32(px, 0), my_scale, unused, my_first);
 	n2_locate(lane_f32(px, 63), my_scale, unused, my_last);
 	my_first = (uint32_t)min((int32_t)my_first, (int32_t)my_last);
-	float one = 1.f;  // (a product with a literal 1 would be taken out, and the operands converted one by one)
-	asm("" : "+s"(one));
+	float unit = 1.f;  // (a product with a literal 1 would be taken out, and the operands converted one by one)
+	asm("" : "+s"(unit));
 	// the plane of vertices whose rows y, y + 1 are at byte offsets row0, row1
 	auto fetch = [&](int l, uint32_t vertex_of_run, uint32_t row0, uint32_t row1, uint32_t (&raw)[2]) __attribute__((always_inline)) {
 		const char* base = reinterpret_cast<const char*>(a.table + a.offset[l]);
@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		const float2 v0 = lt_h2f(raw[0]), v1 = lt_h2f(raw[1]);
 		const float wy = lane_f32(my_wy, l);
 		// (the differences as multiply-adds: those take half-precision operands as they are)
-		mine[l][lane] = make_float2(fmaf(wy, fmaf(one, v1.x, -v0.x), v0.x), fmaf(wy, fmaf(one, v1.y, -v0.y), v0.y));
+		mine[l][lane] = make_float2(fmaf(wy, fmaf(unit, v1.x, -v0.x), v0.x), fmaf(wy, fmaf(unit, v1.y, -v0.y), v0.y));
 	};
 	// What depends on x waits in LDS: kept in registers, cell and weight of every level take 20, and working them out at each plane takes 40 clocks of a
 	// level's 110.

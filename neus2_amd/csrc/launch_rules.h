@@ -70,9 +70,12 @@ static inline N2LatticeSlab n2_lattice_slab(const uint32_t res[3], uint64_t poin
 
 // A slab's features, a 4-byte word per point and fine level, lie in the scratch (of `words` words) and, where a lattice has large slabs, in the output
 // behind the slab's own points too, where nothing has been written yet.  A slab ends with workgroups that have most of a CU to themselves, which takes
-// its two launches 33 us together; on the other hand features of more than the scratch of a 2^22 points' chunk no longer stay in the 256 MiB behind
-// the L2s.  In us, scratch alone | both, (slabs): 512^3 4702 (18) | 4492 (10), 464^3 4327 (14) | 4218 (8), 400^3 2815 (9) | 2760 (7), 320^3 1516 (5) | 1519 (4),
-// 256^3 863 (3) | 874 (2), 64 x 512 x 512 1583 (3) | 1605 (3), 300 x 500 x 200 with ten fine levels 1542 (7) | 1574 (6).
+// its two launches 33 us together.  On the other hand the scratch of a chunk of 2^22 points is 176 MiB, and features of more than that no longer stay in the 256 MiB
+// behind the L2s: the line is for such chunks, where it makes a difference of 4 % at most.  Smaller chunks' scratches are far below that; there a line at four slabs would serve
+// lattices of four to eight better.  In us, scratch alone | both (slabs that the scratch alone takes):
+//   chunk 2^22: 64 x 512 x 512 1555 | 1576 (2.2), 320^3 1480 | 1473 (5.7), 384^3 2205 | 2172 (8.6), 400^3 2699 | 2630 (9.7), 464^3 4127 | 4025 (15), 512^3 4472 | 4290 (17)
+//   chunk 2^20: 160^3 345 | 347 (3.2), 192^3 506 | 482 (5.5), 224^3 736 | 730 (7.8), 512 x 64 x 512 682 | 642 (8.7), 256^3 1039 | 977 (12), 320^3 1856 | 1661 (23), 400^3 3273 | 2831 (39)
+//   chunk 2^18: 96^3 187 | 183 (3.4), 112^3 271 | 238 (4.9), 128^3 344 | 321 (7.3), 160^3 572 | 451 (13), 192^3 971 | 662 (22), 256^3 1752 | 1142 (47)
 static inline bool n2_lattice_large_slabs(uint64_t all, uint64_t words, uint32_t n_fine) { return n_fine != 0 && all > words / n_fine * 8u; }
 // Points that the next slab may have, `rest` of the lattice's being left, and how many levels' features go to the scratch.
 static inline uint64_t n2_lattice_slab_points(uint64_t rest, uint64_t words, uint32_t n_fine, bool large, uint32_t& in_scratch) {

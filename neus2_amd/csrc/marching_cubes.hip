@@ -158,7 +158,7 @@ __device__ const McRing MC_RING = mc_build_ring();
 // a power of two, the pitch: a word's neighbours in y are then its own bits and the next word's, shifted by the pitch.  (With a
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
-// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 82 (6.6 TB/s), count 14.5, scan 4.6, emit 27.5, normals 24, with
+// 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 82 (6.6 TB/s), count 14.6, scan 4.7, emit 27.7, normals 24, with
 // the host's wait for the totals 168 in all.  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
@@ -636,9 +636,12 @@ __device__ __forceinline__ void mc_for_points(mc_word points, uint16_t* list, ui
 // their neighbours in y too), then all that a point needs at once.  A cube's case comes from the bits, as its number of triangles did: whatever
 // the density is by now, a triangle's corners are vertices that this pass writes.
 // (With the records read again for each point, then the bits and then the case's row: 47 us for 512^3, then 34; with the case from the density 33; with the neighbours'
-// records one behind the other, each in a branch of its own, 31.8, now 27.8.)
+// records one behind the other, each in a branch of its own, 31.8, now 27.7.)
 // Vertices that normals are asked for leave their word and place in the normal's slot, for mc_normals_kernel.
-constexpr uint32_t MC_EMIT_GRID = 2304;  // 1280 run at a time, five per CU, by their registers (512^3, 2646 blocks: 1280 31.0 us, 2304 27.5, 6144 31.1; six per CU with four registers spilled 29.4)
+// 1280 run at a time, five per CU, by their registers, and the rest begin as those end.  What the number is hardly matters: the call with 1280 | 1536 | 1792 | 2304 | 4096 in us, 512^3
+// with 0.9 M triangles 170.1 | 167.8 | 166.7 | 168.9 | 169.6, with 1.6 M 191.4 | 197.0 | 190.2 | 189.8 | 191.4, 448^3 1.2 M 152.0 | 149.1 | 149.3 | 150.0 | 150.4, 384^3 0.9 M 113.7 | 112.0 |
+// 112.0 | 112.2 | 112.1; the same within 1 % for 320^3, 256^3, 192^3, 128^3, 64^3 and lattices of 512 x 512 x 64 points on any side.  (Six per CU, with four registers spilled: 29.4 us for 27.5.)
+constexpr uint32_t MC_EMIT_GRID = 2304;
 typedef uint32_t mc_words2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t mc_words3 __attribute__((ext_vector_type(3), aligned(4)));
 typedef float mc_float2 __attribute__((ext_vector_type(2), aligned(4)));

@@ -145,7 +145,7 @@ class GridEncoding:
         return int(capi.lib().n2_grid_active_levels(self._h))
 
     def reserve_scatter_workspace(self, max_points):
-        """Scratch that lets backward passes of >= 4096 points sort their updates in LDS instead of issuing
+        """Scratch that lets backward passes of up to max_points points sort their updates in LDS instead of issuing
         global atomics.  Returns False when the table shape does not support it."""
         nbytes = int(capi.lib().n2_grid_workspace_bytes(self._h, C.c_uint32(max_points)))
         if nbytes == 0:

@@ -584,7 +584,7 @@ def test_sorted_scatter_of_few_records(n, where, table):
         assert torch.equal(got[0], got[1]) and bool((got[0] != (3.0 if mode == GRAD_ACCUMULATE else 0.0)).any()), (mode, level, rows)
 
 
-# the last batch of one point per thread and the next one, workspaces that are just large enough and larger; buckets of up to 65536 records are whole
+# one point, a wave and a few, the kernel for few records and the other one
 @pytest.mark.parametrize("n", [1, 70, 5003, 40001])
 @pytest.mark.parametrize("second", [False, True])
 def test_points_that_a_mask_leaves_out_of_the_scatter_may_hold_anything(n, second):
@@ -613,6 +613,7 @@ def test_points_that_a_mask_leaves_out_of_the_scatter_may_hold_anything(n, secon
     assert torch.equal(got[0], got[1]) and bool(torch.isfinite(got[0].float()).all()) and bool((got[0] != 0).any())
 
 
+# the last batch of one point per thread and the next one, workspaces that are just large enough and larger; buckets of up to 65536 records are whole
 @pytest.mark.parametrize("levels,log2_size,line,whole", [(16, 19, 24576, True), (7, 16, 55808, True), (7, 14, 55808, False), (2, 6, 196608, False)])
 def test_sorted_scatter_at_the_line_between_the_tiles(levels, log2_size, line, whole):
     from neus2_amd.tcnn_api import GRAD_OVERWRITE, GridEncoding
