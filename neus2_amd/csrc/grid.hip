@@ -1171,7 +1171,7 @@ __device__ __forceinline__ void grid_reduce_items(const N2BucketPlan& plan, cons
 // of 50.4 us it took without the LDS additions 45.6, with records out of the L1 46.8, with neither 39.6, without writing the sums 44.9 (buckets drawn early then).  Before, one
 // workgroup of 1024 threads to a bucket, groups of 8 or 16 lanes to a tile's run, values in 2^32 fixed point by five instructions each, | now, launch in us: a training
 // step's 54.6 | 43.1, trained 44.5 | 40.2, the SDF network's 65.2 | 54.8, 52 344 samples 20.0 | 18.3, 2^18 uniform points 51.8 | 48.0 (vector instructions 24.9 | 15.3 M).  Other shapes, of 50.7
-// uniform: 256 threads 59.8, 768 50.6 (registers spill: an accumulating launch for 52 344 points 22 -> 29), 1024 66.0; items dealt out by number 53.2, training step 51.0.  Records under
+// uniform: 256 threads 59.8, 768 50.6 (registers spill: an accumulating backward of 52 344 points 40 -> 47), 1024 66.0; items dealt out by number 53.2, training step 51.0.  Records under
 // way, single ones and pairs, 6 and 3: 4 and 2, and 4 and 3, take the same within 1 %, 6 and 4 1 to 2 % longer, 8 and 3 spill and take 3 to 6.
 // Values from 128 on (a second order's, whose J holds the level's scale) take an instruction more, chosen for a wave's step as a whole: second order and both others on 60 000
 // points along rays 100.0 -> 95.7.  Points packed into a fifth of the cube's side, which meet a few full buckets, lose 2 per cent of a backward: 52 344 88.4 | 90.7, 2^18 319 | 325.
