@@ -356,9 +356,10 @@ def test_sorted_scatter_is_exact_for_values_of_all_sizes(n, levels, log2_size, b
         assert not bad.any(), (mode, int(bad.sum()), got[bad][:4], ref[bad][:4], want[bad][:4])
 
 
-@pytest.mark.parametrize("n", [200, 40000])  # the kernel for few records and the other one
+# the kernel for few records, the same with more records in a bucket than claims (an image by ranges), the other one
+@pytest.mark.parametrize("n,within", [(200, None), (3000, 6), (40000, None)])
 @pytest.mark.parametrize("levels,log2_size,base", [(1, 19, 16), (1, 16, 64), (1, 16, 37), (2, 6, 16)])  # dense, hashed, levels that keep an image, buckets split over several workgroups
-def test_infinite_records_are_neither_cancelled_nor_wrapped(n, levels, log2_size, base):
+def test_infinite_records_are_neither_cancelled_nor_wrapped(n, within, levels, log2_size, base):
     """An entry with infinite records of one sign has an infinite gradient, however many there are (two, every 64th point) and however large finite ones of the
     other sign (up to 65504 / 8, over a thousand of them); one with both signs has no number, as the sum has none.  No two points of a run of equal cells that would be merged."""
     from neus2_amd.tcnn_api import GRAD_ACCUMULATE, GRAD_OVERWRITE, GridEncoding
@@ -368,7 +369,7 @@ def test_infinite_records_are_neither_cancelled_nor_wrapped(n, levels, log2_size
     dg = torch.full_like(dp, 5.0)
     gg.set_params(dp, dg)
     assert gg.reserve_scatter_workspace(n)
-    cells = torch.randint(0, base - 1, (3, n), device="cuda", generator=gen)
+    cells = torch.randint(0, within or base - 1, (3, n), device="cuda", generator=gen)
     i = torch.arange(n, device="cuda")
     dy = torch.randn((2 * levels, n), device="cuda", generator=gen)
     for k, cell, values in ((3, 2, (65504.0, -65504.0)), (5, 6, (-65504.0, 65504.0)), (7, 10, (65504.0, 1.0))):  # every eighth point: three cells with large values
