@@ -108,13 +108,20 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_frags_kernel(const LatticeAr
 
 // Fine levels, level-major workgroup ids; the workgroups behind those write the fragments (a launch for them alone was 5 us of the 60
 // that a lattice of 64^3 takes).  A run needs eight vertices per point, on four rows (y, z), (y + 1, z), (y, z + 1),
-// (y + 1, z + 1).  On a hashed level a row's neighbours in x stand in one aligned 128-byte line per 32, permuted; a load
-// instruction costs the L1 one clock per group of four lanes at least, and up to four where the lanes' spacing makes their
-// banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks per 4-byte load).  So the wave loads the rows as a
-// whole, 2, 4 or 8 entries per lane as the run's length asks for, and weighs the four rows against each other where they are, in
+// (y + 1, z + 1).  On a hashed level a row's neighbours in x stand in one aligned 128-byte line per 32, permuted; a load of four bytes per lane costs the L1 one clock per
+// group of four lanes at least, and up to four where the lanes' spacing makes their banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks).  So the wave
+// loads the rows as a whole and weighs the four rows against each other where they are, in
 // registers; what remains is one row, which goes through LDS (in fp32, a slot left out after every 32 entries so that lanes any
-// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 39 % of the
+// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 32 % of the
 // clocks; 73 % when the eight vertices were picked there).  Runs longer than that (coarse lattices) and dense levels gather from memory.
+//  * Rows of up to 384 entries come a word per lane (walk_words).  64 words of which sixteen lanes each meet aligned 64 bytes, in any order, take an L1 4.4 clocks; a load of 8
+//    or 16 bytes per lane takes it 16.5 however few lanes take part, and a row seldom fills the last of those.
+//  * Longer ones, 16 bytes per lane (walk_wide): eight words a lane and row would be as many clocks and four times the instructions.
+//  * The waves of a small lattice, of four planes at most, take 8 or 16 bytes per lane always: there the number of a plane's loads counts and not what an L1 makes of them (64^3
+//    60 us with wide loads, 65 with words).
+// The kernel's launches for 512^3, wide loads alone | this: 2.57 | 2.44 ms; lattices 256^3 935 | 910 us, 320^3 1605 | 1534, 400^3 2706 | 2624, 464^3 4047 | 3850, 512 x 64 x 512 680 | 655.
+// It takes a line of 128 bytes in every 3.0 clocks (3.2 before; 2.3 at best, 216 lines for 64 points on six levels), beside vector issue (79 % of the clocks).  Each point taking the
+// aligned 8 bytes round its corners by itself, without LDS, is slower where rows are of 64 entries and more (finest levels of 512^3 527 -> 575 and 690 -> 750 us).
 constexpr uint32_t FINE_CHUNKS = 128;  // chunks of four entries a row may have
 constexpr uint32_t FINE_SLOTS = FINE_CHUNKS * 4u + FINE_CHUNKS / 8u;
 __device__ __forceinline__ uint32_t fine_slot(uint32_t entry) { return entry + (entry >> 5); }
@@ -218,7 +225,60 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	if (hashed && chunks <= FINE_CHUNKS) {
 		float2* st = staged[threadIdx.x >> 6];
 		const uint32_t at0 = fine_slot(cx - c_lo), at1 = fine_slot(cx - c_lo + 1u);
-		auto walk = [&](auto each) __attribute__((always_inline)) {
+		// a plane's sums go through LDS, from the lanes' places in the row to the points
+		auto finish_row = [&](auto put) __attribute__((always_inline)) {
+			__builtin_amdgcn_wave_barrier();
+			put();
+			__builtin_amdgcn_wave_barrier();
+			const float2 lo = st[at0], hi = st[at1];
+			if (inside) *out = lt_pack(fmaf(ux, lo.x, wx * hi.x), fmaf(ux, lo.y, wx * hi.y));
+			out += plane;
+		};
+		auto plane_rows = [&](uint32_t k, uint32_t (&row)[4], float (&weight)[4]) __attribute__((always_inline)) {
+#pragma unroll
+			for (uint32_t q = 0; q < 4; ++q) {
+				row[q] = lane_u32(rows[q], k);
+				weight[q] = lane_f32(weights[q], k);
+			}
+		};
+		auto walk_words = [&](auto loads) __attribute__((always_inline)) {
+			constexpr uint32_t LOADS = decltype(loads)::value;
+			// The run's entries start anywhere in 64 bytes: the lanes are turned so that sixteen of them meet one aligned 64 bytes.  (Lanes behind the last entry
+			// load that again: behind a branch the loads would be waited for one by one.)
+			uint32_t off[LOADS], slot[LOADS];
+#pragma unroll
+			for (uint32_t h = 0; h < LOADS; ++h) {
+				uint32_t at = lane + 64u * h - c_lo % 16u;
+				if (h == 0u && (int32_t)at < 0) at += 64u * LOADS;
+				off[h] = ((c_lo + min(at, chunks * 4u - 1u)) & (entries - 1u)) << 2;
+				slot[h] = fine_slot(at);
+			}
+			for (uint32_t k = 0; k < nz; ++k) {
+				uint32_t row[4], v[4][LOADS];
+				float weight[4];
+				plane_rows(k, row, weight);
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q)
+#pragma unroll
+					for (uint32_t h = 0; h < LOADS; ++h) v[q][h] = *reinterpret_cast<const uint32_t*>(base + (off[h] ^ row[q]));
+				float2 sum[LOADS];
+#pragma unroll
+				for (uint32_t h = 0; h < LOADS; ++h) sum[h] = make_float2(0.f, 0.f);
+#pragma unroll
+				for (uint32_t q = 0; q < 4; ++q)
+#pragma unroll
+					for (uint32_t h = 0; h < LOADS; ++h) {
+						const float2 f = lt_h2f(v[q][h]);
+						sum[h].x = fmaf(weight[q], f.x, sum[h].x);
+						sum[h].y = fmaf(weight[q], f.y, sum[h].y);
+					}
+				finish_row([&]() __attribute__((always_inline)) {
+#pragma unroll
+					for (uint32_t h = 0; h < LOADS; ++h) st[slot[h]] = sum[h];
+				});
+			}
+		};
+		auto walk_wide = [&](auto each) __attribute__((always_inline)) {
 			constexpr uint32_t EACH = decltype(each)::value, W = EACH < 4u ? EACH : 4u, H = EACH / W;
 			// The run's places, of W entries each, start anywhere in 64 bytes.  The lanes are turned so that those of a group meet one
 			// aligned 64 bytes (permuted), which the address unit takes at once; a group across two of them costs twice the time.
@@ -234,25 +294,24 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 			for (uint32_t k = 0; k < nz; ++k) {
 				uint32_t row[4];
 				float weight[4];
-#pragma unroll
-				for (uint32_t q = 0; q < 4; ++q) {
-					row[q] = lane_u32(rows[q], k);
-					weight[q] = lane_f32(weights[q], k);
-				}
+				plane_rows(k, row, weight);
 				float2 sum[EACH];
 				fine_sum_rows<EACH>(base, off, have, row, weight, sum);
-				__builtin_amdgcn_wave_barrier();
+				finish_row([&]() __attribute__((always_inline)) {
 #pragma unroll
-				for (uint32_t e = 0; e < EACH; ++e) st[slot[e / W] + e % W] = sum[e];
-				__builtin_amdgcn_wave_barrier();
-				const float2 lo = st[at0], hi = st[at1];
-				if (inside) *out = lt_pack(fmaf(ux, lo.x, wx * hi.x), fmaf(ux, lo.y, wx * hi.y));
-				out += plane;
+					for (uint32_t e = 0; e < EACH; ++e) st[slot[e / W] + e % W] = sum[e];
+				});
 			}
 		};
-		if (chunks > 64u) walk(std::integral_constant<uint32_t, 8>());
-		else if (chunks > 32u) walk(std::integral_constant<uint32_t, 4>());
-		else walk(std::integral_constant<uint32_t, 2>());
+		if (chunks > 96u) walk_wide(std::integral_constant<uint32_t, 8>());
+		else if (a.walk > 4u) {
+			if (chunks > 64u) walk_words(std::integral_constant<uint32_t, 6>());
+			else if (chunks > 48u) walk_words(std::integral_constant<uint32_t, 4>());
+			else if (chunks > 32u) walk_words(std::integral_constant<uint32_t, 3>());
+			else walk_words(std::integral_constant<uint32_t, 2>());
+		} else if (chunks > 64u) walk_wide(std::integral_constant<uint32_t, 8>());
+		else if (chunks > 32u) walk_wide(std::integral_constant<uint32_t, 4>());
+		else walk_wide(std::integral_constant<uint32_t, 2>());
 		return;
 	}
 	const uint32_t x0 = x_part(hashed, entries, res, cx), x1 = x_part(hashed, entries, res, cx + 1u);

@@ -239,6 +239,39 @@ def test_lattices_walked_by_rows_equal_the_same_points_queried(side, res, part, 
 
 # The features of a slab lie in the scratch and, behind the slab, in the output: slabs that take both, the output alone (a scratch of less than a plane),
 # planes in parts at the end, gathered and by rows, an output that starts anywhere; no fine level at all
+# The finest level's row that a run of 64 points meets, in chunks of four entries: each number of words a lane takes, and both sides of where it becomes one
+# more, wide loads begin and the points gather for themselves; by waves of two planes, whose loads are wide always, and of five.
+@pytest.mark.parametrize("rows", [(6, 9), (160, 130)])
+@pytest.mark.parametrize("chunks", [2, 16, 32, 33, 48, 49, 64, 65, 96, 97, 128, 129])
+def test_fine_rows_of_every_length(chunks, rows):
+    from neus2_amd.mesh import density_on_grid
+    from neus2_amd.tcnn_api import NerfNetwork
+    net = NerfNetwork()
+    f = np.float32
+    scale = net.encoding().level_table()[0][15]
+    res = (64, *rows)
+    lo = np.array([0.3, 0.2, 0.1], f)
+
+    def met(extent):
+        x = (np.arange(64, dtype=f) * f(f(1.0) / f(64))) * f(extent) + lo[0]
+        cell = np.floor(x.astype(np.float64) * float(scale) + 0.5).astype(int)
+        return (cell[-1] + 1 - (cell[0] & ~3)) // 4 + 1
+
+    extent = next(f(e) for e in np.arange(1, 1500) * 1e-4 if met(e) == chunks)
+    hi = lo + np.array([extent, 0.7, 0.8], f)
+    p = torch.randn(net.param_offsets()[4], device="cuda", generator=torch.Generator(device="cuda").manual_seed(chunks)) * 0.1
+    net.set_params(p.half(), None)
+    n = res[0] * res[1] * res[2]
+    net.reserve((n + 7) // 8 * 8)
+    d = density_on_grid(net._h, res, tuple(lo), tuple(hi), chunk=1 << 22)
+    z, y, x = np.meshgrid(*(np.arange(r, dtype=f) for r in reversed(res)), indexing="ij")
+    ext = hi - lo
+    padded = np.full((3, (n + 7) // 8 * 8), 0.5, f)
+    padded[:, :n] = np.stack([(c * f(f(1.0) / f(r))) * e + b for c, r, e, b in zip((x, y, z), res, ext, lo)]).reshape(3, -1)
+    want = host(net.sdf(dev(padded)))[0, :n].reshape(z.shape)
+    assert_close(host(d), want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
+
+
 @pytest.mark.parametrize("res,chunk,levels", [((70, 9, 60), 512, 16), ((70, 9, 60), 64, 16), ((130, 7, 33), 8, 16), ((300, 11, 90), 4096, 16), ((96, 33, 300), 1 << 14, 16),
                                               ((64, 8, 40), 256, 4)])
 def test_a_lattice_in_slabs_equals_the_lattice_at_once(res, chunk, levels):
