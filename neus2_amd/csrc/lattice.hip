@@ -13,13 +13,13 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.26 ms in ten slabs: a plane takes 4.7 us for six fine levels and 3.5 us for the walk, a slab 14 and 19 us more.  The fine levels are held by
-// the L1's data return (busy in 95 % of the clocks: a wave's load of 16 bytes per lane takes 17 to 20 of them), the walk by the same (87 %), vector instructions (70 %) and
-// the features, which come from beyond the L2 (28 % hits).  (4.80 ms in 18 slabs, when a walk's start waited for its planes one after the other and then for the
-// fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's walk and
-// the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
-// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before these slabs, starts and lengths of waves | now: 80^3 81 | 74 us, 96^3
-// 105 | 96, 128^3 178 | 169, 208^3 594 | 570, 256^3 891 | 843, 320^3 1607 | 1482, 400^3 2929 | 2632, 464^3 4553 | 4055, 512 x 64 x 512 624 | 580, 64 x 512 x 512 1619 | 1583.
+// 512^3 lattice 4.00 ms in ten slabs: 2.43 ms for six fine levels and 1.81 ms for the walk under the profiler.  The fine levels are held by lines (one of 128 bytes into an L1 in every
+// 3.0 clocks; 2.3 at best) beside vector issue (79 %), the walk by vector instructions, waits of three waves per SIMD and
+// the features, which come from beyond the L2 (28 % hits).  (4.30 ms with 2.57 and 2.06, before what stands at the two kernels; 4.80 in 18 slabs, when a walk's start waited for its planes one after
+// the other and then for the fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's
+// walk and the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
+// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before | now, us: 64^3 59.7 | 57.7, 80^3 73 | 72, 96^3 96 | 96, 128^3 171 | 166, 208^3 611 | 571, 256^3 935 | 890,
+// 320^3 1600 | 1480, 400^3 2720 | 2500, 464^3 4047 | 3656, 512 x 64 x 512 690 | 630, 64 x 512 x 512 1575 | 1550; with a chunk of 2^20 points 256^3 1045 | 981, 512^3 4550 | 4263.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -335,14 +335,14 @@ __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
 }
 
 // The SDF of the wave's 64 points from their features (enc: one word per level), two tiles of the network.  Tile 0 works for lanes
-// 0..31, tile 1 for lanes 32..63; xc0, xc1: the x and y coordinate for either, in the lanes that need them (the lower half).
+// 0..31, tile 1 for lanes 32..63; at: the coordinates for either, x and y in word 0, in the lanes that need them (the lower half), z written here.
 __device__ __forceinline__ void lattice_xy(float px, float py, uint32_t g, uint32_t& xc0, uint32_t& xc1) {
 	xc0 = xc1 = lt_pack((float)((hf)px - (hf)0.5f), (float)((hf)py - (hf)0.5f));
 	swap_halves(xc0, xc1);
 	xc0 = g == 0u ? xc0 : 0u;
 	xc1 = g == 0u ? xc1 : 0u;
 }
-__device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32_t (&enc)[LT_LEVELS], uint32_t xc0, uint32_t xc1, float pz, float bias) {
+__device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32_t (&enc)[LT_LEVELS], uint4v (&at)[2], float pz, float bias) {
 	// (the fence keeps the network's fragments in LDS: hoisted out of the walk's loop they would take 40 registers)
 	tile_fence();
 	half8 xs[2][3];
@@ -362,13 +362,19 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 	}
 	const half2v zc = {(hf)pz - (hf)0.5f, (hf)0};
 	const uint32_t zcm = lane < 32u ? __builtin_bit_cast(uint32_t, zc) : 0u;
-	xs[0][2] = __builtin_bit_cast(half8, uint4v{xc0, zcm, 0u, 0u});
-	xs[1][2] = __builtin_bit_cast(half8, uint4v{xc1, zcm, 0u, 0u});
+#pragma unroll
+	for (int t = 0; t < 2; ++t) {
+		at[t][1] = zcm;
+		asm("" : "+v"(at[t]));  // (one set of registers for the whole walk: otherwise a second one, and eight moves a step)
+		xs[t][2] = __builtin_bit_cast(half8, at[t]);
+	}
 	// The second layer, of which only row 0 is wanted: a lane holds half of its sample's hidden values (the other group the
-	// other half).  Dot products on the vector unit take a third of the time of four more MFMAs per tile.
+	// other half), and a product of sixteen 4 x 4 blocks takes four of them with the weights that the lanes of a block share; all four rows come out alike.  (Dot
+	// products on the vector unit, which the walk has least to spare of: 1.88 ms for 512^3, now 1.81; four more of the large products per tile took longer than those.)
 	// (one tile after the other: side by side they take 32 registers more, and a third wave has no room; the weights of 32 rows serve both: read for each
 	// tile anew, and with registers spilled whose return waits for the loads of two steps, the walk took 4.2 us a plane of 512^2, then 3.9; 3.5 with what depends on x in LDS)
-	float dot[2] = {0.f, 0.f};
+	typedef float float4v __attribute__((ext_vector_type(4)));
+	float4v dot[2] = {float4v(0.f), float4v(0.f)};
 #pragma unroll
 	for (int mt = 0; mt < 2; ++mt) {
 		half8 w[3];
@@ -383,16 +389,15 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 			relu_pack(acc, h[0], h[1]);
 #pragma unroll
 			for (int c = 0; c < 2; ++c) {
-				const uint4v wv = __builtin_bit_cast(uint4v, frag(F, SDF_FRAG_WO + 2 * mt + c, lane & 32)), hv = __builtin_bit_cast(uint4v, h[c]);  // row 0 of W_out in the order of h
-#pragma unroll
-				for (int q = 0; q < 4; ++q)
-					dot[t] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, (uint32_t)hv[q]), __builtin_bit_cast(half2v, (uint32_t)wv[q]), dot[t], false);
+				const half8 wv = frag(F, SDF_FRAG_WO + 2 * mt + c, lane & 32);  // row 0 of W_out in the order of h
+				dot[t] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_shufflevector(wv, wv, 0, 1, 2, 3), __builtin_shufflevector(h[c], h[c], 0, 1, 2, 3), dot[t], 0, 0, 0);
+				dot[t] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_shufflevector(wv, wv, 4, 5, 6, 7), __builtin_shufflevector(h[c], h[c], 4, 5, 6, 7), dot[t], 0, 0, 0);
 			}
 			__builtin_amdgcn_sched_barrier(0);
 		}
 	}
 	// tile 0 belongs to lanes 0..31, tile 1 to the upper ones
-	uint32_t s0 = __float_as_uint(dot[0]), s1 = __float_as_uint(dot[1]);
+	uint32_t s0 = __float_as_uint(dot[0][0]), s1 = __float_as_uint(dot[1][0]);
 	swap_halves(s0, s1);
 	return (hf)(__uint_as_float(s0) + __uint_as_float(s1)) + (hf)bias;
 }
@@ -400,6 +405,9 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 // The walk.  NM levels are interpolated here, the others come from a.features.  A row of a walked level's vertices that a run of 64
 // points meets fits the wave's lanes (n2_lattice_row_levels): lane v holds vertex v of the run, the two rows of a plane are loaded
 // as consecutive words and interpolated in y there, and the points pick their two neighbours through LDS.
+// Three waves per SIMD (157 registers), whose vector instructions and waits fill the time.  What took instructions away, the walk of 512^3 in ms: masks kept as they are (below) and rows'
+// offsets by one product instead of five 2.06 -> 1.92, the coordinates in registers of their own 1.91, features loaded one step ahead instead of two, without twelve moves a
+// step, 1.87, the second layer by small matrix products 1.81.
 template <int NM>
 __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const LatticeArgs a) {
 	__shared__ __align__(16) hf F[SDF_FRAG_COUNT * 512];
@@ -428,18 +436,28 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	my_first = (uint32_t)min((int32_t)my_first, (int32_t)my_last);
 	float unit = 1.f;  // (a product with a literal 1 would be taken out, and the operands converted one by one)
 	asm("" : "+s"(unit));
-	// the plane of vertices whose rows y, y + 1 are at byte offsets row0, row1
-	auto fetch = [&](int l, uint32_t vertex_of_run, uint32_t row0, uint32_t row1, uint32_t (&raw)[2]) __attribute__((always_inline)) {
+	// A row of vertices (y, z) is at byte offset  y part ^ z part  on a hashed level (within its table) and  y part + z part  on a dense one: row_part, with one product a step.
+	const uint32_t my_z_factor = (my_hashed ? 805459861u : my_res * my_res) << 2, my_z_most = my_hashed ? ~0u : my_res;
+	const uint32_t my_bytes = my_entries << 2, my_in_table = (my_entries - 1u) << 2;
+	const uint32_t my_y0 = (my_hashed ? my_cy * 2654435761u : min(my_cy, my_res) * my_res) << 2, my_y1 = (my_hashed ? (my_cy + 1u) * 2654435761u : min(my_cy + 1u, my_res) * my_res) << 2;
+	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) __attribute__((always_inline)) {
+		const uint32_t z = min(cz, my_z_most) * my_z_factor;
+		r0 = my_hashed ? (my_y0 ^ z) & my_in_table : my_y0 + z;
+		r1 = my_hashed ? (my_y1 ^ z) & my_in_table : my_y1 + z;
+	};
+	// the plane of vertices whose rows y, y + 1 are at byte offsets row0, row1; of_run: four times the vertex's number in the run
+	my_first <<= 2;
+	auto fetch = [&](int l, uint32_t of_run, uint32_t row0, uint32_t row1, uint32_t hash_mask, uint32_t (&raw)[2]) __attribute__((always_inline)) {
 		const char* base = reinterpret_cast<const char*>(a.table + a.offset[l]);
-		const uint32_t entries = lane_u32(my_entries, l), v = lane_u32(my_first, l) + vertex_of_run;
-		if ((a.hash_mask >> l) & 1u) {
-			const uint32_t xo = x_part(true, entries, 0u, v);
+		const uint32_t bytes = lane_u32(my_bytes, l), v = lane_u32(my_first, l) + of_run;
+		if ((hash_mask >> l) & 1u) {
+			const uint32_t xo = v & (bytes - 4u);
 			raw[0] = *reinterpret_cast<const uint32_t*>(base + (xo ^ row0));
 			raw[1] = *reinterpret_cast<const uint32_t*>(base + (xo ^ row1));
 		} else {
-			const uint32_t xo = x_part(false, entries, lane_u32(my_res, l), v);
-			raw[0] = *reinterpret_cast<const uint32_t*>(base + vertex(false, entries << 2, xo, row0));
-			raw[1] = *reinterpret_cast<const uint32_t*>(base + vertex(false, entries << 2, xo, row1));
+			const uint32_t xo = min(v, lane_u32(my_res, l) << 2);
+			raw[0] = *reinterpret_cast<const uint32_t*>(base + vertex(false, bytes, xo, row0));
+			raw[1] = *reinterpret_cast<const uint32_t*>(base + vertex(false, bytes, xo, row1));
 		}
 	};
 	auto blend_y = [&](int l, const uint32_t (&raw)[2]) __attribute__((always_inline)) {
@@ -456,34 +474,29 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		float w;
 		uint32_t cx;
 		n2_locate(px, lane_f32(my_scale, l), w, cx);
-		places[l][lane] = make_uint2(__float_as_uint(w), ((threadIdx.x >> 6) * NM + l) * 512u + min(cx - lane_u32(my_first, l), 62u) * 8u);
+		places[l][lane] = make_uint2(__float_as_uint(w), ((threadIdx.x >> 6) * NM + l) * 512u + min(cx * 4u - lane_u32(my_first, l), 62u * 4u) * 2u);
 	}
-	auto blend_x = [&](int l, float2& to) __attribute__((always_inline)) {
-		const uint2 p = places[l][lane];
+	auto blend_at = [&](const uint2 p, float2& to) __attribute__((always_inline)) {
 		const float2* at = reinterpret_cast<const float2*>(reinterpret_cast<const char*>(line) + p.y);
 		const float2 lo = at[0], hi = at[1];
 		const float w = __uint_as_float(p.x);
 		to = make_float2(fmaf(w, hi.x - lo.x, lo.x), fmaf(w, hi.y - lo.y, lo.y));
 	};
-	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) __attribute__((always_inline)) {
-		r0 = row_part(my_hashed, my_entries, my_res, my_cy, cz);
-		r1 = row_part(my_hashed, my_entries, my_res, my_cy + 1u, cz);
-	};
 	float2 hi[NM], rise[NM];  // the plane above, and by how much it is above the one below
 	// (all levels, also those that are switched off: behind branches the loads would be waited for one by one)
 	auto fetch_plane = [&](uint32_t cz, uint32_t (&raw)[NM][2]) __attribute__((always_inline)) {
-		uint32_t r0, r1, v = lane;
+		uint32_t r0, r1, v = lane * 4u;
 		asm volatile("" : "+v"(v));  // (addresses formed here: kept for the next start, they take registers that a step needs)
 		rows_of(cz, r0, r1);
 #pragma unroll
-		for (int l = 0; l < NM; ++l) fetch(l, v, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+		for (int l = 0; l < NM; ++l) fetch(l, v, lane_u32(r0, l), lane_u32(r1, l), a.hash_mask, raw[l]);
 	};
 	auto blend_plane = [&](const uint32_t (&raw)[NM][2], float2 (&to)[NM]) __attribute__((always_inline)) {
 #pragma unroll
 		for (int l = 0; l < NM; ++l) blend_y(l, raw[l]);
 		__builtin_amdgcn_wave_barrier();
 #pragma unroll
-		for (int l = 0; l < NM; ++l) blend_x(l, to[l]);
+		for (int l = 0; l < NM; ++l) blend_at(places[l][lane], to[l]);
 		__builtin_amdgcn_wave_barrier();
 	};
 	const uint64_t feat_at = (uint64_t)(z - a.z0) * plane + (uint64_t)(y - a.y0) * a.nx;  // (the same for the wave, like out)
@@ -491,12 +504,13 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 	float* out = a.out + (uint64_t)(z - a.z0) * ((uint64_t)a.lat.res[0] * a.lat.res[1]) + (uint64_t)(y - a.y0) * a.lat.res[0];
 	uint32_t xc0, xc1;
 	lattice_xy(px, py, lane >> 5, xc0, xc1);
+	uint4v at[2] = {uint4v{xc0, 0u, 0u, 0u}, uint4v{xc1, 0u, 0u, 0u}};
 	// (levels that the table does not have read the last one's row: their weights are zero)
 	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
 	const uint32_t* row[LT_LEVELS - NM];
 #pragma unroll
 	for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) row[f] = lattice_features(a, have_fine ? min(f, a.n_levels - 1u - NM) : 0u) + feat_at;
-	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
+	uint32_t fine[LT_LEVELS - NM];
 	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) __attribute__((always_inline)) {
 		uint32_t at = feat_x;
 		asm volatile("" : "+v"(at));  // (the lane's 32 bits beside a uniform address; their sum, formed in front of the loop, takes registers that a step needs)
@@ -517,7 +531,6 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		fetch_plane(my_cz + 1u, above);
 		load_fine(k, fine);
 		blend_plane(below, rise);
-		load_fine(min(k + 1u, nz - 1u), ahead);
 		blend_plane(above, hi);
 	}
 #pragma unroll
@@ -536,8 +549,15 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		}
 #pragma unroll
 		for (int f = 0; f < (int)LT_LEVELS - NM; ++f) {
-			enc[NM + f] = fine[f] & have_fine;
+			enc[NM + f] = fine[f];
 			asm volatile("" : "+v"(enc[NM + f]));  // waited for here, in front of the next step's loads: behind them the wait would include those
+		}
+		if (!have_fine) {  // (a branch that is hardly ever taken, not a select a level)
+#pragma unroll
+			for (int f = 0; f < (int)LT_LEVELS - NM; ++f) {
+				enc[NM + f] = 0u;
+				asm volatile("" : "+v"(enc[NM + f]));
+			}
 		}
 		// the next step: where it stands, and the loads it needs (the last step looks at its own position again: no loads)
 		const uint32_t next = k + 1u < nz ? k + 1u : k;
@@ -546,37 +566,45 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		n2_locate(lattice_coord(a.lat, 2, z + next), my_scale, wz, cz);
 		const uint32_t moved = cz - my_cz;
 		const uint32_t one = (uint32_t)__ballot(moved == 1u) & on, far = (uint32_t)__ballot(moved > 1u) & on;  // lanes 0..15 speak for the levels
-		uint32_t r0, r1, v = lane;
+		uint32_t r0, r1, v = lane * 4u;
 		asm volatile("" : "+v"(v));
 		rows_of(cz + 1u, r0, r1);
-		uint32_t raw[NM][2];
+		// (bits of a mask are looked up where they are needed: what the compiler takes for the same condition at two places it keeps as a mask of lanes, through a vector
+		// register, two instructions a level and step)
+		uint32_t raw[NM][2], hash_mask = a.hash_mask;
+		asm("" : "+s"(hash_mask));
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) fetch(l, v, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
-		// Behind them the fine features of the step after the next (they come from far away): the planes can then be waited for
-		// without waiting for these.
-#pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
-		load_fine(min(k + 2u, nz - 1u), ahead);
+			if ((one >> l) & 1u) fetch(l, v, lane_u32(r0, l), lane_u32(r1, l), hash_mask, raw[l]);
+		// Behind them the next step's fine features (they come from far away): the planes can then be waited for without waiting for these.
+		load_fine(next, fine);
 		float bias = a.sdf_bias;
 		asm volatile("" : "+s"(bias));
-		const hf sdf = lattice_network(F, lane, enc, xc0, xc1, pz, bias);
+		const hf sdf = lattice_network(F, lane, enc, at, pz, bias);
 		uint32_t out_x = x * 4u;
 		asm volatile("" : "+v"(out_x));
 		if (inside) *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + out_x) = (float)sdf;
 		out += (uint64_t)a.lat.res[0] * a.lat.res[1];
 		if (++k == nz) return;
 		if (far) break;
-		// the planes the next step has crossed into
+		// the planes the next step has crossed into (the points' places come into the registers that held the vertices)
+		uint32_t into = one;
+		asm("" : "+s"(into));
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) blend_y(l, raw[l]);
+			if ((into >> l) & 1u) {
+				blend_y(l, raw[l]);
+				const uint2 p = places[l][lane];
+				raw[l][0] = p.x;
+				raw[l][1] = p.y;
+			}
 		__builtin_amdgcn_wave_barrier();
+		asm("" : "+s"(into));
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) {
+			if ((into >> l) & 1u) {
 				const float2 below = hi[l];
-				blend_x(l, hi[l]);
+				blend_at(make_uint2(raw[l][0], raw[l][1]), hi[l]);
 				rise[l] = make_float2(hi[l].x - below.x, hi[l].y - below.y);
 			}
 		my_cz = cz;
@@ -687,6 +715,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 	float* out = a.out + (size_t)(z - a.z0) * ((size_t)rx * a.lat.res[1]) + (size_t)(y - a.y0) * rx + x;
 	uint32_t xc0, xc1;
 	lattice_xy(px, py, lane >> 5, xc0, xc1);
+	uint4v at[2] = {uint4v{xc0, 0u, 0u, 0u}, uint4v{xc1, 0u, 0u, 0u}};
 	// (levels that the table does not have read the last one's row: their weights are zero)
 	const uint32_t have_fine = a.n_levels > (uint32_t)NM ? ~0u : 0u;
 	const uint32_t* row[LT_LEVELS - NM];
@@ -731,7 +760,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 #pragma unroll
 		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
 		load_fine(min(k + 2u, nz - 1u), ahead);
-		const hf sdf = lattice_network(F, lane, enc, xc0, xc1, pz, a.sdf_bias);
+		const hf sdf = lattice_network(F, lane, enc, at, pz, a.sdf_bias);
 		if (inside) out[0] = (float)sdf;
 		out += (size_t)rx * a.lat.res[1];
 		// the planes the next step has crossed into
