@@ -614,9 +614,11 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 }
 
 // The walk for lattices of a few dozen points along x, or with steps along z of more than a walked level's cell: every point gathers
-// its own vertices, and a step meets any planes.
+// its own vertices, and a step meets any planes.  Masks, rows and features as in lattice_walk_kernel: 96 x 304 x 304 833 -> 802 us, 64^3 57.9 -> 56.8; with six levels it
+// fits three waves per SIMD then, 256 x 256 x 64 277 -> 250 us, 512 x 64 x 64 113 -> 105.
+constexpr uint32_t lattice_gather_waves(uint32_t levels) { return levels <= 6u ? 3u : 2u; }  // per SIMD
 template <int NM>
-__global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const LatticeArgs a) {
+__global__ void __launch_bounds__(LT_BLOCK, lattice_gather_waves(NM)) lattice_gather_walk_kernel(const LatticeArgs a) {
 	__shared__ __align__(16) hf F[SDF_FRAG_COUNT * 512];
 	for (uint32_t i = threadIdx.x; i < SDF_FRAG_COUNT * 64u; i += LT_BLOCK) *reinterpret_cast<half8*>(F + i * 8u) = *reinterpret_cast<const half8*>(a.frags + i * 8u);
 	__syncthreads();
@@ -650,8 +652,8 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 		asm volatile("" : "+v"(p));
 		n2_locate(p, a.scale[l], w, c);
 	};
-	auto fetch = [&](int l, uint32_t row0, uint32_t row1, uint32_t (&raw)[4]) {
-		const bool hashed = (a.hash_mask >> l) & 1u;
+	auto fetch = [&](int l, uint32_t row0, uint32_t row1, uint32_t hash_mask, uint32_t (&raw)[4]) __attribute__((always_inline)) {
+		const bool hashed = (hash_mask >> l) & 1u;
 		const uint32_t bytes = a.entries[l] << 2;
 		float w;
 		uint32_t cx;
@@ -681,26 +683,30 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 		p.x = fmaf(w0, v0.x, fmaf(w1, v1.x, fmaf(w2, v2.x, fmaf(w3, v3.x, 0.f))));
 		p.y = fmaf(w0, v0.y, fmaf(w1, v1.y, fmaf(w2, v2.y, fmaf(w3, v3.y, 0.f))));
 	};
-	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) {
-		r0 = row_part(my_hashed, my_entries, my_res, my_cy, cz);
-		r1 = row_part(my_hashed, my_entries, my_res, my_cy + 1u, cz);
+	const uint32_t my_z_factor = (my_hashed ? 805459861u : my_res * my_res) << 2, my_z_most = my_hashed ? ~0u : my_res, my_in_table = (my_entries - 1u) << 2;
+	const uint32_t my_y0 = (my_hashed ? my_cy * 2654435761u : min(my_cy, my_res) * my_res) << 2, my_y1 = (my_hashed ? (my_cy + 1u) * 2654435761u : min(my_cy + 1u, my_res) * my_res) << 2;
+	auto rows_of = [&](uint32_t cz, uint32_t& r0, uint32_t& r1) __attribute__((always_inline)) {
+		const uint32_t z = min(cz, my_z_most) * my_z_factor;
+		r0 = my_hashed ? (my_y0 ^ z) & my_in_table : my_y0 + z;
+		r1 = my_hashed ? (my_y1 ^ z) & my_in_table : my_y1 + z;
 	};
 	float2 lo[NM], hi[NM], rise[NM];  // planes below and above, and their difference
 	auto both_planes = [&](uint32_t which, uint32_t cz) {
 		uint32_t r0, r1, q0, q1;
 		rows_of(cz, r0, r1);
 		rows_of(cz + 1u, q0, q1);
-		uint32_t raw[NM][4];
+		uint32_t raw[NM][4], hash_mask = a.hash_mask;
+		asm("" : "+s"(hash_mask));
 		// (all levels' loads of a plane in flight together)
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((which >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
+			if ((which >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), hash_mask, raw[l]);
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
 			if ((which >> l) & 1u) blend(l, raw[l], lo[l]);
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((which >> l) & 1u) fetch(l, lane_u32(q0, l), lane_u32(q1, l), raw[l]);
+			if ((which >> l) & 1u) fetch(l, lane_u32(q0, l), lane_u32(q1, l), hash_mask, raw[l]);
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
 			if ((which >> l) & 1u) {
@@ -721,13 +727,12 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 	const uint32_t* row[LT_LEVELS - NM];
 #pragma unroll
 	for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) row[f] = lattice_features(a, have_fine ? min(f, a.n_levels - 1u - NM) : 0u);
-	uint32_t fine[LT_LEVELS - NM], ahead[LT_LEVELS - NM];
+	uint32_t fine[LT_LEVELS - NM];
 	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) {
 #pragma unroll
 		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = row[f][feat_at + (size_t)k * plane];
 	};
 	load_fine(0, fine);
-	load_fine(min(1u, nz - 1u), ahead);
 	for (uint32_t k = 0; k < nz; ++k) {
 		const float pz = lattice_coord(a.lat, 2, z + k);
 		// features of this step
@@ -739,8 +744,15 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 		}
 #pragma unroll
 		for (int f = 0; f < (int)LT_LEVELS - NM; ++f) {
-			enc[NM + f] = fine[f] & have_fine;
+			enc[NM + f] = fine[f];
 			asm volatile("" : "+v"(enc[NM + f]));  // waited for here, in front of the next step's loads: behind them the wait would include those
+		}
+		if (!have_fine) {  // (as there)
+#pragma unroll
+			for (int f = 0; f < (int)LT_LEVELS - NM; ++f) {
+				enc[NM + f] = 0u;
+				asm volatile("" : "+v"(enc[NM + f]));
+			}
 		}
 		// the next step: where it stands, and the loads it needs (the last step looks at its own position again: no loads)
 		const uint32_t next = k + 1u < nz ? k + 1u : k;
@@ -751,22 +763,22 @@ __global__ void __launch_bounds__(LT_BLOCK, 2) lattice_gather_walk_kernel(const 
 		const uint32_t one = (uint32_t)__ballot(moved == 1u) & on, far = (uint32_t)__ballot(moved > 1u) & on;  // lanes 0..15 speak for the levels
 		uint32_t r0, r1;
 		rows_of(cz + 1u, r0, r1);
-		uint32_t raw[NM][4];
+		uint32_t raw[NM][4], hash_mask = a.hash_mask;
+		asm("" : "+s"(hash_mask));
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), raw[l]);
-		// Behind them the fine features of the step after the next (they come from far away): the planes can then be waited for
-		// without waiting for these.
-#pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) fine[f] = ahead[f];
-		load_fine(min(k + 2u, nz - 1u), ahead);
+			if ((one >> l) & 1u) fetch(l, lane_u32(r0, l), lane_u32(r1, l), hash_mask, raw[l]);
+		// Behind them the next step's fine features (they come from far away): the planes can then be waited for without waiting for these.
+		load_fine(next, fine);
 		const hf sdf = lattice_network(F, lane, enc, at, pz, a.sdf_bias);
 		if (inside) out[0] = (float)sdf;
 		out += (size_t)rx * a.lat.res[1];
 		// the planes the next step has crossed into
+		uint32_t into = one;
+		asm("" : "+s"(into));
 #pragma unroll
 		for (int l = 0; l < NM; ++l)
-			if ((one >> l) & 1u) {
+			if ((into >> l) & 1u) {
 				lo[l] = hi[l];
 				blend(l, raw[l], hi[l]);
 				rise[l] = make_float2(hi[l].x - lo[l].x, hi[l].y - lo[l].y);
@@ -832,7 +844,7 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 			lattice_fine_kernel<<<dim3(blocks() * n_fine + (done == 0 ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks());
 			N2_LAUNCH_CHECK();
 		}
-		a.walk = n2_lattice_walk(runs, nz, by_rows ? 3u : 2u);
+		a.walk = n2_lattice_walk(runs, nz, by_rows ? 3u : lattice_gather_waves(nm));
 		walk_kernel<<<dim3(blocks()), dim3(LT_BLOCK), 0, s>>>(a);
 		N2_LAUNCH_CHECK();
 		done += a.points;
