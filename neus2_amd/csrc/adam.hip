@@ -1,7 +1,7 @@
 // Adam step over the whole parameter vector: a pure streaming kernel.
 // Four parameters per lane so that every buffer is moved with 8- or 16-byte
-// accesses; parameters whose gradient is zero (most of the hash table in any
-// one step) cost only the 2-byte gradient read.
+// accesses; parameters whose gradient is zero (most of the hash table in a small
+// step) cost only the 2-byte gradient read, or a share of the 64 bytes they stand in.
 #include "n2_common.h"
 #include <hip/hip_ext.h>
 #include "slab_reduce.h"
@@ -73,6 +73,7 @@ __device__ __forceinline__ bool adam_summed(const N2SlabReduce& r, const hf* gra
 	return (g >= r.ga && g < r.ga + r.params_a) || (g >= r.gb && g < r.gb + r.params_b) || (r.extra_n > 0 && g == r.extra_out);
 }
 
+constexpr uint32_t ADAM_WHOLE = 4;  // consecutive quads, 64 bytes of each fp32 buffer
 // STREAM: the moments are read and written past the last-level cache, for a caller whose state and samples do not fit it (the
 // trainer: n2_moments_stream, launch_rules.h).  Master weights streamed too: the training step at 2^18 382 -> 384 us, at 2^14 132 -> 134.
 template <typename StepT, bool STREAM>
@@ -139,18 +140,21 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 	}
 	if (i0 + 4 <= n) {
 		const half4 g = *reinterpret_cast<const half4*>(grads + i0);
-		const bool all_zero = g[0] == (hf)0 && g[1] == (hf)0 && g[2] == (hf)0 && g[3] == (hf)0;
-		if (all_zero && i0 >= n_matrix) return;  // nothing but the gradient is touched
+		const bool touched = i0 < n_matrix || !(g[0] == (hf)0 && g[1] == (hf)0 && g[2] == (hf)0 && g[3] == (hf)0);
+		// ADAM_WHOLE quads are read and written together, those without a gradient as they were: memory takes pieces of a line below 64 bytes at the cost of
+		// whole ones and more.  (Training steps in us, quads on their own | two together | four | eight: 2^14 131.5 | 131.2 | 130.6 | 135.3, 2^15 150.9 | 148.6 | 146.4 | 148.4,
+		// 2^16 200.6 | 195.0 | 187.5 | 188.4, 2^17 252.8 | 245.9 | 241.7 | 241.9, 2^18 343.2 | 340.0 | 338.6 | 339.2, trained 495.8 | 493.3 | 492.3 | 493.3.)
+		const uint32_t any = (uint32_t)(__ballot(touched) >> (threadIdx.x & 63u & ~(ADAM_WHOLE - 1u))) & ((1u << ADAM_WHOLE) - 1u);
+		if (any == 0u) return;  // nothing but the gradient is touched
 		float4 w = *reinterpret_cast<float4*>(master + i0);
 		float4 a = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m1 + i0)) : *reinterpret_cast<const float4*>(m1 + i0);
 		float4 b = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m2 + i0)) : *reinterpret_cast<const float4*>(m2 + i0);
 		uint4 t = step_load4(steps + i0);
-		bool any = false;
-		any |= adam_one(i0 + 0, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[0], w.x, a.x, b.x, t.x);
-		any |= adam_one(i0 + 1, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[1], w.y, a.y, b.y, t.y);
-		any |= adam_one(i0 + 2, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[2], w.z, a.z, b.z, t.z);
-		any |= adam_one(i0 + 3, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[3], w.w, a.w, b.w, t.w);
-		if (!any) return;
+		bool moved = false;
+		moved |= adam_one(i0 + 0, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[0], w.x, a.x, b.x, t.x);
+		moved |= adam_one(i0 + 1, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[1], w.y, a.y, b.y, t.y);
+		moved |= adam_one(i0 + 2, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[2], w.z, a.z, b.z, t.z);
+		moved |= adam_one(i0 + 3, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[3], w.w, a.w, b.w, t.w);
 		*reinterpret_cast<float4*>(master + i0) = w;
 		if (STREAM) {
 			n2_stream_store(reinterpret_cast<float4*>(m1 + i0), a);
@@ -160,7 +164,8 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 			*reinterpret_cast<float4*>(m2 + i0) = b;
 		}
 		step_store4(steps + i0, t);
-		*reinterpret_cast<half4*>(params + i0) = half4{(hf)w.x, (hf)w.y, (hf)w.z, (hf)w.w};
+		// (the working copy of a quad that has not moved is the caller's, whatever it holds)
+		if (moved) *reinterpret_cast<half4*>(params + i0) = half4{(hf)w.x, (hf)w.y, (hf)w.z, (hf)w.w};
 	} else {
 		for (uint32_t i = i0; i < n; ++i) {
 			float w = master[i], a = m1[i], b = m2[i];

@@ -32,6 +32,29 @@ def test_adam_steps_match_oracle(oracle, n, n_matrix):
     np.testing.assert_array_equal(host(opt.master)[never], w0[never])
 
 
+@pytest.mark.parametrize("n,every", [(4 * 64 * 3 + 1, 16), (4 * 256 + 20, 20), (16, 16), (20, 12), (7, 5)])
+def test_parameters_beside_a_moved_one_stay_as_they_are(n, every):
+    """Quads without a gradient are written back with the ones beside them: no bit of their state may change, and their working copy is left alone."""
+    from neus2_amd.tcnn_api import Adam
+    rng = np.random.default_rng(n)
+    state = [rng.integers(0, 2 ** 32, n, dtype=np.uint32).view(np.float32) for _ in range(3)]  # any bits: infinities, no numbers, denormal ones
+    opt = Adam(dev(state[0]), 0)
+    opt.m1, opt.m2 = dev(state[1]), dev(state[2])
+    opt.steps.copy_(torch.arange(n))
+    params = dev(rng.integers(0, 2 ** 16, n, dtype=np.uint16).view(np.int16)).view(torch.float16)
+    before = params.view(torch.int16).clone()
+    g = np.zeros(n, np.float32)
+    g[every // 2::every] = 1.0
+    opt.step(params, dev(g, torch.float16))
+    still = g == 0
+    for got, was in zip((opt.master, opt.m1, opt.m2), state):
+        assert np.array_equal(host(got).view(np.uint32)[still], was.view(np.uint32)[still])
+    assert np.array_equal(host(opt.steps).view(np.int32), np.arange(n) + ~still)
+    quads = np.repeat(np.add.reduceat(~still, np.arange(0, n, 4)) > 0, 4)[:n]
+    alone = ~quads
+    assert np.array_equal(host(params.view(torch.int16))[alone], host(before)[alone])
+
+
 def test_adam_errors():
     from neus2_amd.tcnn_api import Adam, N2Error
     m = torch.zeros(16, device="cuda")
