@@ -74,9 +74,10 @@ __device__ __forceinline__ bool adam_summed(const N2SlabReduce& r, const hf* gra
 }
 
 constexpr uint32_t ADAM_WHOLE = 4;  // consecutive quads, 64 bytes of each fp32 buffer
+constexpr uint32_t ADAM_LIST = 3;   // quads per lane that a wave makes its list from
 // STREAM: the moments are read and written past the last-level cache, for a caller whose state and samples do not fit it (the
 // trainer: n2_moments_stream, launch_rules.h).  Master weights streamed too: the training step at 2^18 382 -> 384 us, at 2^14 132 -> 134.
-template <typename StepT, bool STREAM>
+template <typename StepT, bool STREAM, bool LISTED>
 __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32_t n, uint32_t n_matrix, float loss_scale, float inv_loss_scale, int saturated,
                                                         uint32_t slot, const uint32_t* __restrict__ gate, float* __restrict__ master, hf* __restrict__ params, const hf* __restrict__ grads,
                                                         float* __restrict__ m1, float* __restrict__ m2, StepT* __restrict__ steps, N2SlabReduce sums,
@@ -122,12 +123,10 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 		});
 		return;
 	}
-	const uint32_t q = (block - sums.units) * 256 + threadIdx.x;
-	const uint32_t i0 = q * 4;
-	if (i0 >= n) return;
-	if (adam_summed(sums, grads, i0) || adam_summed(sums, grads, min(i0 + 3u, n - 1u))) {
-		// a quad that touches summed parameters (the networks' weights are whole quads; the single extra value may share its
-		// quad with others): one parameter at a time, leaving out the summed ones
+	// parameters one at a time, leaving out the summed ones: the last ones of a vector that is no whole number of quads, and quads that touch summed parameters (the
+	// networks' weights are whole quads; the single extra value may share its quad with others)
+	auto on_its_own = [&](uint32_t i0) { return i0 + 4u > n || adam_summed(sums, grads, i0) || adam_summed(sums, grads, i0 + 3u); };
+	auto one_by_one = [&](uint32_t i0) {
 		for (uint32_t i = i0; i < min(i0 + 4u, n); ++i) {
 			if (adam_summed(sums, grads, i)) continue;
 			float w = master[i], a = m1[i], b = m2[i];
@@ -136,16 +135,9 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 				master[i] = w; m1[i] = a; m2[i] = b; step_store(steps + i, t); params[i] = (hf)w;
 			}
 		}
-		return;
-	}
-	if (i0 + 4 <= n) {
-		const half4 g = *reinterpret_cast<const half4*>(grads + i0);
-		const bool touched = i0 < n_matrix || !(g[0] == (hf)0 && g[1] == (hf)0 && g[2] == (hf)0 && g[3] == (hf)0);
-		// ADAM_WHOLE quads are read and written together, those without a gradient as they were: memory takes pieces of a line below 64 bytes at the cost of
-		// whole ones and more.  (Training steps in us, quads on their own | two together | four | eight: 2^14 131.5 | 131.2 | 130.6 | 135.3, 2^15 150.9 | 148.6 | 146.4 | 148.4,
-		// 2^16 200.6 | 195.0 | 187.5 | 188.4, 2^17 252.8 | 245.9 | 241.7 | 241.9, 2^18 343.2 | 340.0 | 338.6 | 339.2, trained 495.8 | 493.3 | 492.3 | 493.3.)
-		const uint32_t any = (uint32_t)(__ballot(touched) >> (threadIdx.x & 63u & ~(ADAM_WHOLE - 1u))) & ((1u << ADAM_WHOLE) - 1u);
-		if (any == 0u) return;  // nothing but the gradient is touched
+	};
+	auto is_touched = [&](uint32_t i0, half4 g) { return i0 < n_matrix || !(g[0] == (hf)0 && g[1] == (hf)0 && g[2] == (hf)0 && g[3] == (hf)0); };
+	auto step_quad = [&](uint32_t i0, half4 g) __attribute__((always_inline)) {
 		float4 w = *reinterpret_cast<float4*>(master + i0);
 		float4 a = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m1 + i0)) : *reinterpret_cast<const float4*>(m1 + i0);
 		float4 b = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m2 + i0)) : *reinterpret_cast<const float4*>(m2 + i0);
@@ -166,14 +158,49 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 		step_store4(steps + i0, t);
 		// (the working copy of a quad that has not moved is the caller's, whatever it holds)
 		if (moved) *reinterpret_cast<half4*>(params + i0) = half4{(hf)w.x, (hf)w.y, (hf)w.z, (hf)w.w};
-	} else {
-		for (uint32_t i = i0; i < n; ++i) {
-			float w = master[i], a = m1[i], b = m2[i];
-			uint32_t t = step_load(steps + i);
-			if (adam_one(i, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)grads[i], w, a, b, t)) {
-				master[i] = w; m1[i] = a; m2[i] = b; step_store(steps + i, t); params[i] = (hf)w;
-			}
+	};
+	const uint32_t lane = threadIdx.x & 63u;
+	if constexpr (LISTED) {
+		// A wave lists the quads that have a gradient among its ADAM_LIST for each lane, and steps those.  What bounds a small batch's step is instructions where a
+		// lane in ten of nearly every wave has something to do (n2_adam_lists, launch_rules.h).
+		__shared__ half4 gradient[256 / 64][64 * ADAM_LIST];
+		__shared__ uint32_t place[256 / 64][64 * ADAM_LIST];
+		half4(&listed)[64 * ADAM_LIST] = gradient[threadIdx.x >> 6];
+		uint32_t(&at)[64 * ADAM_LIST] = place[threadIdx.x >> 6];
+		const uint32_t first = ((block - sums.units) * 256u + (threadIdx.x & ~63u)) * ADAM_LIST + lane;
+		half4 g[ADAM_LIST];
+#pragma unroll
+		for (uint32_t u = 0; u < ADAM_LIST; ++u) {
+			const uint32_t i0 = (first + 64u * u) * 4u;
+			g[u] = i0 + 4u <= n ? *reinterpret_cast<const half4*>(grads + i0) : half4(0);
 		}
+		uint32_t count = 0;
+#pragma unroll
+		for (uint32_t u = 0; u < ADAM_LIST; ++u) {
+			const uint32_t i0 = (first + 64u * u) * 4u;
+			const bool alone = i0 < n && on_its_own(i0);
+			if (alone) one_by_one(i0);
+			const bool mine = i0 < n && !alone && is_touched(i0, g[u]);
+			const uint64_t all = __ballot(mine);
+			if (mine) {
+				const uint32_t k = count + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0u));
+				listed[k] = g[u];
+				at[k] = i0;
+			}
+			count += (uint32_t)__popcll(all);
+		}
+		__builtin_amdgcn_wave_barrier();
+		for (uint32_t k = lane; k < count; k += 64u) step_quad(at[k], listed[k]);
+	} else {
+		const uint32_t i0 = ((block - sums.units) * 256u + threadIdx.x) * 4u;
+		if (i0 >= n) return;
+		if (on_its_own(i0)) return one_by_one(i0);
+		const half4 g = *reinterpret_cast<const half4*>(grads + i0);
+		// ADAM_WHOLE quads are read and written together, those without a gradient as they were: memory takes pieces of a line below 64 bytes at the cost of
+		// whole ones and more.  (Training steps in us, quads on their own | two together | four | eight: 2^14 131.5 | 131.2 | 130.6 | 135.3, 2^15 150.9 | 148.6 | 146.4 | 148.4,
+		// 2^16 200.6 | 195.0 | 187.5 | 188.4, 2^17 252.8 | 245.9 | 241.7 | 241.9, 2^18 343.2 | 340.0 | 338.6 | 339.2, trained 495.8 | 493.3 | 492.3 | 493.3.)
+		const uint32_t any = (uint32_t)(__ballot(is_touched(i0, g)) >> (lane & ~(ADAM_WHOLE - 1u))) & ((1u << ADAM_WHOLE) - 1u);
+		if (any != 0u) step_quad(i0, g);  // (else nothing but the gradient is touched)
 	}
 }
 
@@ -191,7 +218,7 @@ N2_API int n2_adam_step(n2_stream_t stream, const n2_adam_config* config, uint32
 int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_t n_params, uint32_t n_matrix_params,
                        float loss_scale, float* d_master, n2_half* d_params, const n2_half* d_gradients, float* d_m1,
                        float* d_m2, void* d_steps, uint32_t steps_bits, const uint32_t* d_gate, const N2SlabReduce* sums, const N2StepEpilogue* epilogue,
-                       hipEvent_t done_event, bool stream_moments) {
+                       hipEvent_t done_event, bool stream_moments, bool listed) {
 	N2_REQUIRE(config != nullptr, "n2_adam_step: config is null");
 	if (n_params == 0) return N2_OK;
 	N2_REQUIRE(d_master && d_params && d_gradients && d_m1 && d_m2 && d_steps, "n2_adam_step: null buffer");
@@ -255,29 +282,34 @@ int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_
 		N2_REQUIRE(epi.n_ptr != nullptr && epi.sum_out != nullptr && epi.copy_n <= 256 && (epi.copy_n == 0 || (epi.copy_src && epi.copy_dst)),
 		           "n2_adam_step: incomplete step epilogue");
 	}
-	const dim3 grid((quads + 255) / 256 + plan.units + (epi.values ? 1u : 0u));
+	const uint32_t per_block = listed ? 256u * ADAM_LIST : 256u;
+	const dim3 grid((quads + per_block - 1u) / per_block + plan.units + (epi.values ? 1u : 0u));
 	N2_REQUIRE(steps_bits == 32 || steps_bits == 16, "n2_adam_step: step counters of %u bits", steps_bits);
 	N2_REQUIRE(steps_bits == 32 || saturated, "n2_adam_step: 16-bit step counters need betas whose powers underflow within %u steps", ADAM_TABLE);
-	auto launch = [&](auto* steps, auto stream_tag) {
+	auto launch = [&](auto* steps, auto stream_tag, auto listed_tag) {
 		using StepT = std::remove_pointer_t<decltype(steps)>;
-		constexpr bool STREAM = decltype(stream_tag)::value;
+		constexpr bool STREAM = decltype(stream_tag)::value, LISTED = decltype(listed_tag)::value;
 		if (done_event != nullptr) {
 			// the event is tied to this launch's own completion: no packet of its own behind the kernel, where an event record
 			// costs the stream about 5 us before its next kernel starts
-			hipExtLaunchKernelGGL((adam_step_kernel<StepT, STREAM>), grid, dim3(256), 0, s, nullptr, done_event, 0, *config, n_params, n_matrix_params, loss_scale,
+			hipExtLaunchKernelGGL((adam_step_kernel<StepT, STREAM, LISTED>), grid, dim3(256), 0, s, nullptr, done_event, 0, *config, n_params, n_matrix_params, loss_scale,
 			                      inv_loss_scale, saturated, slot, d_gate, d_master, reinterpret_cast<hf*>(d_params), reinterpret_cast<const hf*>(d_gradients),
 			                      d_m1, d_m2, steps, plan, epi);
 		} else {
-			adam_step_kernel<StepT, STREAM><<<grid, dim3(256), 0, s>>>(*config, n_params, n_matrix_params, loss_scale, inv_loss_scale, saturated, slot, d_gate, d_master,
+			adam_step_kernel<StepT, STREAM, LISTED><<<grid, dim3(256), 0, s>>>(*config, n_params, n_matrix_params, loss_scale, inv_loss_scale, saturated, slot, d_gate, d_master,
 				reinterpret_cast<hf*>(d_params), reinterpret_cast<const hf*>(d_gradients), d_m1, d_m2, steps, plan, epi);
 		}
 	};
-	auto with_steps = [&](auto stream_tag) {
-		if (steps_bits == 16) launch(static_cast<uint16_t*>(d_steps), stream_tag);
-		else launch(static_cast<uint32_t*>(d_steps), stream_tag);
+	auto with_steps = [&](auto stream_tag, auto listed_tag) {
+		if (steps_bits == 16) launch(static_cast<uint16_t*>(d_steps), stream_tag, listed_tag);
+		else launch(static_cast<uint32_t*>(d_steps), stream_tag, listed_tag);
 	};
-	if (stream_moments) with_steps(std::true_type{});
-	else with_steps(std::false_type{});
+	auto with_list = [&](auto stream_tag) {
+		if (listed) with_steps(stream_tag, std::true_type{});
+		else with_steps(stream_tag, std::false_type{});
+	};
+	if (stream_moments) with_list(std::true_type{});
+	else with_list(std::false_type{});
 	N2_LAUNCH_CHECK();
 	return N2_OK;
 }

@@ -21,6 +21,17 @@ static inline bool n2_moments_stream(uint64_t state_bytes, uint64_t batch) {
 	return state_bytes + N2_STEP_BYTES_PER_SAMPLE * batch > N2_LAST_LEVEL_CACHE_BYTES;
 }
 
+// Whether a training step's optimiser makes lists of the parameters that have a gradient before it steps them (adam_step_kernel): in small batches on large tables, whose
+// samples, with eight entries of two parameters on every level each, meet at most a sixth of the parameters.  Beyond, what a step takes is its lines, which lists meet in
+// smaller pieces; small tables have most of their parameters met at any batch.  Steps in us, without | with lists:
+//   table of 2^19 entries a level (12.6 M parameters): batch 2048 97.4 | 79.3, 4096 106.2 | 94, 6144 110.8 | 99.6, 8192 116.8 | 108.1, 12 288 121.6 | 119.5, 16 384 131.1 | 134.2
+//   2^20 (24 M): 4096 145.7 | 124.2, 8192 180.5 | 160.1, 16 384 232.3 | 230.8, 20 480 259.5 | 266.4      2^22 (85 M): 8192 291 | 234, 16 384 373 | 307, 32 768 496 | 473, 65 536 724 | 765
+//   2^17 (3.5 M): 2048 65.5 to 73 | 65.3, 4096 68 to 77 | 69, 8192 74.5 | 75 to 84                         2^14 (0.5 M): 256 52 to 58 | 59 to 62, 4096 59 to 62 | 65
+constexpr uint64_t N2_LIST_PARAMS_MIN = 1u << 21, N2_LIST_BATCH_MAX = 40960;
+static inline bool n2_adam_lists(uint64_t n_params, uint32_t n_levels, uint64_t batch) {
+	return n_params >= N2_LIST_PARAMS_MIN && batch <= N2_LIST_BATCH_MAX && batch * n_levels * 16u * 6u <= n_params;
+}
+
 // Points per thread of the scatter's sorting kernel.  Three of its workgroups share a CU, 768 run at a time.  One point per thread where all workgroups
 // (levels x tiles) then start together: the launch takes one workgroup's chain of round trips, which is shorter for one point.  Beyond, a
 // workgroup of two points per thread takes less than two of one, and the summing kernel finds half as many runs.  Both kernels in us, one | two:

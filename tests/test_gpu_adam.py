@@ -55,6 +55,35 @@ def test_parameters_beside_a_moved_one_stay_as_they_are(n, every):
     assert np.array_equal(host(params.view(torch.int16))[alone], host(before)[alone])
 
 
+@pytest.mark.parametrize("batch,beta2,ema", [(512, 0.99, 0.0), (8192, 0.99, 0.0), (4096, 0.9999, 0.0), (2048, 0.99, 0.95), (8320, 0.99, 0.0)])
+def test_small_batches_of_the_trainer_match_oracle(oracle, batch, beta2, ema):
+    """The optimiser of small batches lists the parameters that have a gradient (all batches here but the last, which is the first one that does not;
+    16- and 32-bit step counters, moments streamed and not): parameters, moments and counters after two steps."""
+    from neus2_amd import scene
+    from neus2_amd.tcnn_api import pack_cameras
+    from neus2_amd.training import Trainer, default_config
+    cams = scene.cameras_on_sphere(8, 96)
+    cfg = default_config(target_batch_size=batch, max_rays_per_batch=512, max_samples=1 << 17, ema_decay=ema)
+    cfg.adam.beta2 = beta2
+    tr = Trainer(cfg)
+    tr.set_scene(pack_cameras(cams), len(cams), dev(scene.render_sphere_images(cams)), dev(scene.sphere_bitfield()))
+    tr.initialize_params(seed=5, sdf_mlp_weights=None)
+    w, m1, m2, steps = host(tr.master).copy(), np.zeros(tr.n_params, np.float32), np.zeros(tr.n_params, np.float32), np.zeros(tr.n_params, np.uint32)
+    for seed in (3, 4):
+        tr.step(n_rays=max(16, batch // 40), n_inference=1 << 17, seed=seed)
+        g = host(tr.grads)
+        oracle.adam_step(w, g, m1, m2, steps, n_matrix_params=tr.offsets[2], beta2=beta2)
+    s = tr.optimizer_state()
+    assert s.param_steps_bits == (16 if beta2 == 0.99 else 32)
+    got = host(tr._view(s.param_steps, tr.n_params, torch.int16 if s.param_steps_bits == 16 else torch.int32))
+    met = 2 * batch * 16 * 8 * 2 + tr.offsets[2] + tr.n_params - tr.offsets[3]  # two steps, eight entries of two parameters on 16 levels; the networks and the variance
+    assert tr.offsets[2] < (steps > 0).sum() <= met and np.array_equal(got, steps.astype(got.dtype))
+    np.testing.assert_allclose(host(tr.master), w, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(host(tr._view(s.first_moments, tr.n_params, torch.float32)), m1, rtol=1e-5, atol=1e-7)
+    np.testing.assert_allclose(host(tr._view(s.second_moments, tr.n_params, torch.float32)), m2, rtol=1e-5, atol=1e-9)
+    np.testing.assert_array_equal(host(tr.params), q16(host(tr.master)))
+
+
 def test_adam_errors():
     from neus2_amd.tcnn_api import Adam, N2Error
     m = torch.zeros(16, device="cuda")
