@@ -55,15 +55,32 @@ __device__ __forceinline__ uint32_t step_load(const uint32_t* p) { return *p; }
 __device__ __forceinline__ uint32_t step_load(const uint16_t* p) { return *p; }
 __device__ __forceinline__ void step_store(uint32_t* p, uint32_t t) { *p = t; }
 __device__ __forceinline__ void step_store(uint16_t* p, uint32_t t) { *p = (uint16_t)min(t, 65535u); }
-__device__ __forceinline__ uint4 step_load4(const uint32_t* p) { return *reinterpret_cast<const uint4*>(p); }
-__device__ __forceinline__ uint4 step_load4(const uint16_t* p) {
-	const ushort4 v = *reinterpret_cast<const ushort4*>(p);
+// (STREAM: past the last-level cache)
+template <bool STREAM>
+__device__ __forceinline__ uint4 step_load4(const uint32_t* p) {
+	typedef uint32_t four __attribute__((ext_vector_type(4)));
+	const four v = STREAM ? __builtin_nontemporal_load(reinterpret_cast<const four*>(p)) : *reinterpret_cast<const four*>(p);
 	return make_uint4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ void step_store4(uint32_t* p, uint4 t) { *reinterpret_cast<uint4*>(p) = t; }
+template <bool STREAM>
+__device__ __forceinline__ uint4 step_load4(const uint16_t* p) {
+	typedef uint16_t four __attribute__((ext_vector_type(4)));
+	const four v = STREAM ? __builtin_nontemporal_load(reinterpret_cast<const four*>(p)) : *reinterpret_cast<const four*>(p);
+	return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <bool STREAM>
+__device__ __forceinline__ void step_store4(uint32_t* p, uint4 t) {
+	typedef uint32_t four __attribute__((ext_vector_type(4)));
+	const four v = {t.x, t.y, t.z, t.w};
+	if (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<four*>(p));
+	else *reinterpret_cast<four*>(p) = v;
+}
+template <bool STREAM>
 __device__ __forceinline__ void step_store4(uint16_t* p, uint4 t) {
-	*reinterpret_cast<ushort4*>(p) = make_ushort4((unsigned short)min(t.x, 65535u), (unsigned short)min(t.y, 65535u), (unsigned short)min(t.z, 65535u),
-	                                              (unsigned short)min(t.w, 65535u));
+	typedef uint16_t four __attribute__((ext_vector_type(4)));
+	const four v = {(uint16_t)min(t.x, 65535u), (uint16_t)min(t.y, 65535u), (uint16_t)min(t.z, 65535u), (uint16_t)min(t.w, 65535u)};
+	if (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<four*>(p));
+	else *reinterpret_cast<four*>(p) = v;
 }
 
 // parameters whose gradients a slab summation produces (r.units > 0): the workgroups that run its units step them
@@ -75,8 +92,10 @@ __device__ __forceinline__ bool adam_summed(const N2SlabReduce& r, const hf* gra
 
 constexpr uint32_t ADAM_WHOLE = 4;  // consecutive quads, 64 bytes of each fp32 buffer
 constexpr uint32_t ADAM_LIST = 3;   // quads per lane that a wave makes its list from
-// STREAM: the moments are read and written past the last-level cache, for a caller whose state and samples do not fit it (the
-// trainer: n2_moments_stream, launch_rules.h).  Master weights streamed too: the training step at 2^18 382 -> 384 us, at 2^14 132 -> 134.
+// STREAM: the state is read and written past the last-level cache, for a caller whose state and samples do not fit it (the trainer: n2_optimiser_streams, launch_rules.h);
+// of lists, which are written in pieces, the moments alone.  Training steps in us, moments alone | master weights too | counters too | gradients too (whose pieces are read once):
+// 2^14 124.3 | 122.0 | 122.2 | 123.2, 2^16 187.8 | 180.3 | 178.8 | 178.3, 2^18 340.5 | 338.8 | 337.7 | 337.3, trained 493.2 | 491.8 | 491.2 | 491.6; with lists 4096 83.4 | 85 to 94 |
+// 93 | 100, 8192 102.4 | 107.8 | 113.8 | 115.9.  (Written in pieces, all of it streamed was slower at every batch.)
 template <typename StepT, bool STREAM, bool LISTED>
 __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32_t n, uint32_t n_matrix, float loss_scale, float inv_loss_scale, int saturated,
                                                         uint32_t slot, const uint32_t* __restrict__ gate, float* __restrict__ master, hf* __restrict__ params, const hf* __restrict__ grads,
@@ -138,24 +157,28 @@ __global__ void __launch_bounds__(256) adam_step_kernel(n2_adam_config c, uint32
 	};
 	auto is_touched = [&](uint32_t i0, half4 g) { return i0 < n_matrix || !(g[0] == (hf)0 && g[1] == (hf)0 && g[2] == (hf)0 && g[3] == (hf)0); };
 	auto step_quad = [&](uint32_t i0, half4 g) __attribute__((always_inline)) {
-		float4 w = *reinterpret_cast<float4*>(master + i0);
-		float4 a = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m1 + i0)) : *reinterpret_cast<const float4*>(m1 + i0);
-		float4 b = STREAM ? n2_stream_load(reinterpret_cast<const float4*>(m2 + i0)) : *reinterpret_cast<const float4*>(m2 + i0);
-		uint4 t = step_load4(steps + i0);
+		constexpr bool ALL = STREAM && !LISTED;
+		auto load = [&](const float* p, auto past) {
+			if constexpr (decltype(past)::value) return n2_stream_load(reinterpret_cast<const float4*>(p + i0));
+			else return *reinterpret_cast<const float4*>(p + i0);
+		};
+		auto store = [&](float* p, float4 v, auto past) {
+			if constexpr (decltype(past)::value) n2_stream_store(reinterpret_cast<float4*>(p + i0), v);
+			else *reinterpret_cast<float4*>(p + i0) = v;
+		};
+		constexpr std::bool_constant<STREAM> moments{};
+		constexpr std::bool_constant<ALL> others{};
+		float4 w = load(master, others), a = load(m1, moments), b = load(m2, moments);
+		uint4 t = step_load4<ALL>(steps + i0);
 		bool moved = false;
 		moved |= adam_one(i0 + 0, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[0], w.x, a.x, b.x, t.x);
 		moved |= adam_one(i0 + 1, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[1], w.y, a.y, b.y, t.y);
 		moved |= adam_one(i0 + 2, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[2], w.z, a.z, b.z, t.z);
 		moved |= adam_one(i0 + 3, n_matrix, loss_scale, inv_loss_scale, saturated, c, table, (float)g[3], w.w, a.w, b.w, t.w);
-		*reinterpret_cast<float4*>(master + i0) = w;
-		if (STREAM) {
-			n2_stream_store(reinterpret_cast<float4*>(m1 + i0), a);
-			n2_stream_store(reinterpret_cast<float4*>(m2 + i0), b);
-		} else {
-			*reinterpret_cast<float4*>(m1 + i0) = a;
-			*reinterpret_cast<float4*>(m2 + i0) = b;
-		}
-		step_store4(steps + i0, t);
+		store(master, w, others);
+		store(m1, a, moments);
+		store(m2, b, moments);
+		step_store4<ALL>(steps + i0, t);
 		// (the working copy of a quad that has not moved is the caller's, whatever it holds)
 		if (moved) *reinterpret_cast<half4*>(params + i0) = half4{(hf)w.x, (hf)w.y, (hf)w.z, (hf)w.w};
 	};
@@ -218,7 +241,7 @@ N2_API int n2_adam_step(n2_stream_t stream, const n2_adam_config* config, uint32
 int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_t n_params, uint32_t n_matrix_params,
                        float loss_scale, float* d_master, n2_half* d_params, const n2_half* d_gradients, float* d_m1,
                        float* d_m2, void* d_steps, uint32_t steps_bits, const uint32_t* d_gate, const N2SlabReduce* sums, const N2StepEpilogue* epilogue,
-                       hipEvent_t done_event, bool stream_moments, bool listed) {
+                       hipEvent_t done_event, bool streamed, bool listed) {
 	N2_REQUIRE(config != nullptr, "n2_adam_step: config is null");
 	if (n_params == 0) return N2_OK;
 	N2_REQUIRE(d_master && d_params && d_gradients && d_m1 && d_m2 && d_steps, "n2_adam_step: null buffer");
@@ -308,7 +331,7 @@ int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_
 		if (listed) with_steps(stream_tag, std::true_type{});
 		else with_steps(stream_tag, std::false_type{});
 	};
-	if (stream_moments) with_list(std::true_type{});
+	if (streamed) with_list(std::true_type{});
 	else with_list(std::false_type{});
 	N2_LAUNCH_CHECK();
 	return N2_OK;

@@ -9,13 +9,8 @@
 #define N2_HD
 #endif
 
-// Whether a training step streams its optimiser's moments past the last-level cache (n2_adam_step_gated): when what the step
-// passes over between two uses of a moment is more than the cache holds, the moments do not stay there and only push out
-// what the next kernels read.  That is the optimiser's state and, for each sample of the batch, about 1600 bytes of coordinates,
-// network rows, slopes and scatter records.  Steps in us, plain | streamed:
-//   state 227 MB (table of 2^19 entries a level): batch 4096 113 | 120, 20 480 140 | 142, 24 576 147 | 146, 28 672 154 | 152, 2^16 198 | 187, 2^18 381 | 373
-//   434 MB (2^20): 4096 149 | 148, 8192 187 | 180, 2^15 349 | 335        1.5 GB (2^22): 4096 236 | 234, 2^14 385 | 379
-//   63 MB (2^17): 2^14 100 | 102, 2^16 141 | 143, 2^17 201 | 199, 2^18 325 | 323        9 MB (2^14): 2^17 184 | 184, 2^18 305 | 304
+// Whether what a training step passes over between two uses of an optimiser's moment is more than the last-level cache holds, so that moments do not stay there and only push
+// out what the next kernels read.  That is the optimiser's state and, for each sample of the batch, about 1600 bytes of coordinates, network rows, slopes and scatter records.
 constexpr uint64_t N2_LAST_LEVEL_CACHE_BYTES = 256ull << 20, N2_STEP_BYTES_PER_SAMPLE = 1600;
 static inline bool n2_moments_stream(uint64_t state_bytes, uint64_t batch) {
 	return state_bytes + N2_STEP_BYTES_PER_SAMPLE * batch > N2_LAST_LEVEL_CACHE_BYTES;
@@ -30,6 +25,18 @@ static inline bool n2_moments_stream(uint64_t state_bytes, uint64_t batch) {
 constexpr uint64_t N2_LIST_PARAMS_MIN = 1u << 21, N2_LIST_BATCH_MAX = 40960;
 static inline bool n2_adam_lists(uint64_t n_params, uint32_t n_levels, uint64_t batch) {
 	return n_params >= N2_LIST_PARAMS_MIN && batch <= N2_LIST_BATCH_MAX && batch * n_levels * 16u * 6u <= n_params;
+}
+
+// Whether the optimiser's state is streamed past that cache (adam_step_kernel).  Where whole pieces of 64 bytes are written that pays long before all is full: a sample counts
+// twice, and the line is 96 MiB lower.  Lists are written in pieces, and of them only the moments are streamed; their batches are small.  Steps in us, plain | streamed:
+//   state 227 MB (table of 2^19 entries a level): batch 9088 117.6 | 113.4, 16 384 130.4 | 122.2, 24 576 148.7 | 132.3, 2^15 163.8 | 143.6, 2^16 202.5 | 178.8, 2^18 351 | 337.7; with lists 1024
+//   75.7 | 76.0, 2048 79.1 | 79.1, 4096 85 to 95 | 83.4, 8192 107.9 | 102.4
+//   434 MB (2^20): 16 384 240.6 | 228, 2^16 554 | 527; with lists 4096 125.7 | 124.2      1.5 GB (2^22): 2^16 745 | 719, 2^18 2000 | 1921; with lists 16 384 308.5 | 306.7
+//   120 MB (2^18): 8192 83.1 | 87 to 95, 16 384 105.7 | 104.4, 2^15 124.3 | 119.8, 2^16 160.6 | 150; with lists 4096 73.3 | 75.9
+//   63 MB (2^17): 16 384 81.3 | 83 to 91, 2^15 103.5 | 103.2, 2^16 138.5 | 134.7, 2^18 293.7 | 289.2
+//   33 MB (2^16): 16 384 73.2 | 75.8, 2^16 127.0 | 127.0, 2^18 293.2 | 291.7        9 MB (2^14): 2^15 95.9 | 97.3, 2^18 270.2 | 270.0
+static inline bool n2_optimiser_streams(uint64_t state_bytes, uint64_t batch, bool listed) {
+	return listed ? n2_moments_stream(state_bytes, 8u * batch) : n2_moments_stream(state_bytes + (96ull << 20), 2u * batch);
 }
 
 // Points per thread of the scatter's sorting kernel.  Three of its workgroups share a CU, 768 run at a time.  One point per thread where all workgroups

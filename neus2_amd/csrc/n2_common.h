@@ -224,12 +224,12 @@ int n2_mlp_backward_and_second_order_indexed(n2_mlp_t* mlp, n2_stream_t stream, 
 // d_steps: uint32_t (steps_bits 32) or uint16_t counters (16)
 // epilogue (or null): one more workgroup of the launch does the caller's bookkeeping (slab_reduce.h), gated or not
 // done_event (or null): recorded by the completion of the launch itself (hipExtLaunchKernel's stop event)
-// stream_moments: the moments pass by the last-level cache (for a caller that moves more than the cache holds between two steps)
+// streamed: the optimiser's state passes by the last-level cache (for a caller that moves more than the cache holds between two steps)
 // listed: few of the gradients are other than zero (n2_adam_lists); the results are the same
 int n2_adam_step_gated(n2_stream_t stream, const n2_adam_config* config, uint32_t n_params, uint32_t n_matrix_params,
                        float loss_scale, float* d_master, n2_half* d_params, const n2_half* d_gradients, float* d_m1,
                        float* d_m2, void* d_steps, uint32_t steps_bits, const uint32_t* d_gate, const N2SlabReduce* sums = nullptr,
-                       const N2StepEpilogue* epilogue = nullptr, hipEvent_t done_event = nullptr, bool stream_moments = false, bool listed = false);
+                       const N2StepEpilogue* epilogue = nullptr, hipEvent_t done_event = nullptr, bool streamed = false, bool listed = false);
 // true when 1 - beta^t is exactly 1 in fp32 for both betas from the end of the kernel's bias-correction table on: the step
 // counters may then be 16 bits wide (steps_bits 16, saturating at 65535) instead of 32
 bool n2_adam_counters_may_saturate(float beta1, float beta2);

@@ -419,11 +419,12 @@ N2_API int n2_trainer_step(n2_trainer_t* t, n2_stream_t stream, uint32_t n_rays,
 	N2StepEpilogue epi{};
 	epi.values = t->ray_loss; epi.n_ptr = ray_counter; epi.n_max = n_rays; epi.sum_out = reinterpret_cast<float*>(t->counters) + 4;
 	epi.copy_src = set.counters; epi.copy_dst = t->counters; epi.copy_n = 2;
+	const bool listed = n2_adam_lists(t->n_params, t->cfg.field.n_levels, T);
 	// master, moments, counters, fp16 parameters and gradients, and the average's two copies
 	const uint64_t state_bytes = (uint64_t)t->n_params * (16u + t->steps_bits / 8u + (t->ema ? 6u : 0u));
 	if (int rc = n2_adam_step_gated(stream, &t->cfg.adam, t->n_params, t->n_matrix_params, t->cfg.loss_scale, t->master, reinterpret_cast<n2_half*>(t->params),
 	                                reinterpret_cast<const n2_half*>(t->grads), t->m1, t->m2, t->steps, t->steps_bits, compacted_counter, &sums, &epi,
-	                                t->side ? t->ev_main : nullptr, n2_moments_stream(state_bytes, T), n2_adam_lists(t->n_params, t->cfg.field.n_levels, T))) return rc;
+	                                t->side ? t->ev_main : nullptr, n2_optimiser_streams(state_bytes, T, listed), listed)) return rc;
 	t->ev_main_from_adam = t->side != nullptr;
 	t->optimizer_steps += 1;
 	t->training_step += 1;
