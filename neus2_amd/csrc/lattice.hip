@@ -18,7 +18,9 @@
 // the features, which come from beyond the L2 (28 % hits).  (4.30 ms with 2.57 and 2.06, before what stands at the two kernels; 4.80 in 18 slabs, when a walk's start waited for its planes one after
 // the other and then for the fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's
 // walk and the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
-// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before | now, us: 64^3 59.7 | 57.7, 80^3 73 | 72, 96^3 96 | 96, 128^3 171 | 166, 208^3 611 | 571, 256^3 935 | 890,
+// Features and SDF are written, and features read, as streams that pass by the caches: each is met once, and the tables stay where they are (us: 512^3 3905 -> 3840, the walk's alone 3815;
+// 464^3 3628 -> 3546, 400^3 2367 -> 2315, 192^3 399 -> 392, 128^3 160.9 -> 159.6; 448 x 512 x 96 1026 -> 1024, with the walk's alone 1035).
+// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before the features were streams, before | now, us: 64^3 59.7 | 57.7, 80^3 73 | 72, 96^3 96 | 96, 128^3 171 | 166, 208^3 611 | 571, 256^3 935 | 890,
 // 320^3 1600 | 1480, 400^3 2720 | 2500, 464^3 4047 | 3656, 512 x 64 x 512 690 | 630, 64 x 512 x 512 1575 | 1550; with a chunk of 2^20 points 256^3 1045 | 981, 512^3 4550 | 4263.
 #include "n2_common.h"
 
@@ -216,7 +218,7 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 				s[b][1] = fmaf(w, v.y, s[b][1]);
 			}
 		}
-		if (inside) *out = lt_pack(fmaf(ux, s[0][0], wx * s[1][0]), fmaf(ux, s[0][1], wx * s[1][1]));
+		if (inside) __builtin_nontemporal_store(lt_pack(fmaf(ux, s[0][0], wx * s[1][0]), fmaf(ux, s[0][1], wx * s[1][1])), out);
 		out += plane;
 	};
 	// chunks of four entries that the run meets: from c_lo's to the one behind c_hi's
@@ -231,7 +233,7 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 			put();
 			__builtin_amdgcn_wave_barrier();
 			const float2 lo = st[at0], hi = st[at1];
-			if (inside) *out = lt_pack(fmaf(ux, lo.x, wx * hi.x), fmaf(ux, lo.y, wx * hi.y));
+			if (inside) __builtin_nontemporal_store(lt_pack(fmaf(ux, lo.x, wx * hi.x), fmaf(ux, lo.y, wx * hi.y)), out);
 			out += plane;
 		};
 		auto plane_rows = [&](uint32_t k, uint32_t (&row)[4], float (&weight)[4]) __attribute__((always_inline)) {
@@ -515,7 +517,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		uint32_t at = feat_x;
 		asm volatile("" : "+v"(at));  // (the lane's 32 bits beside a uniform address; their sum, formed in front of the loop, takes registers that a step needs)
 #pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(row[f] + (uint64_t)k * plane) + at);
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(row[f] + (uint64_t)k * plane) + at));
 	};
 	// Steps one after the other from plane k on, until the end or to where some level's next plane is not the one above (a box upside down;
 	// steps of more than a cell): there the walk starts anew.  (With that case inside the loop, where it is hardly ever met, its
@@ -583,7 +585,7 @@ __global__ void __launch_bounds__(LT_BLOCK, 3) lattice_walk_kernel(const Lattice
 		const hf sdf = lattice_network(F, lane, enc, at, pz, bias);
 		uint32_t out_x = x * 4u;
 		asm volatile("" : "+v"(out_x));
-		if (inside) *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + out_x) = (float)sdf;
+		if (inside) __builtin_nontemporal_store((float)sdf, reinterpret_cast<float*>(reinterpret_cast<char*>(out) + out_x));
 		out += (uint64_t)a.lat.res[0] * a.lat.res[1];
 		if (++k == nz) return;
 		if (far) break;
@@ -730,7 +732,7 @@ __global__ void __launch_bounds__(LT_BLOCK, lattice_gather_waves(NM)) lattice_ga
 	uint32_t fine[LT_LEVELS - NM];
 	auto load_fine = [&](uint32_t k, uint32_t (&to)[LT_LEVELS - NM]) {
 #pragma unroll
-		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = row[f][feat_at + (size_t)k * plane];
+		for (uint32_t f = 0; f < LT_LEVELS - NM; ++f) to[f] = __builtin_nontemporal_load(row[f] + feat_at + (size_t)k * plane);
 	};
 	load_fine(0, fine);
 	for (uint32_t k = 0; k < nz; ++k) {
@@ -771,7 +773,7 @@ __global__ void __launch_bounds__(LT_BLOCK, lattice_gather_waves(NM)) lattice_ga
 		// Behind them the next step's fine features (they come from far away): the planes can then be waited for without waiting for these.
 		load_fine(next, fine);
 		const hf sdf = lattice_network(F, lane, enc, at, pz, a.sdf_bias);
-		if (inside) out[0] = (float)sdf;
+		if (inside) __builtin_nontemporal_store((float)sdf, out);
 		out += (size_t)rx * a.lat.res[1];
 		// the planes the next step has crossed into
 		uint32_t into = one;
