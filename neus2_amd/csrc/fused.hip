@@ -476,7 +476,7 @@ __device__ __forceinline__ half8 sdf_net(const hf* F, int lane, const half8 (&xs
 }
 
 // inference: bias, density and what the caller wants stored of sample `col` (col_raw: its number before clamping)
-template <class Args>
+template <bool STREAM = false, class Args>
 __device__ __forceinline__ void store_sdf(const Args& a, half8 y, uint32_t col, bool valid, uint32_t col_raw, int g) {
 	if (g == 0) {
 		hf s = y[0] + (hf)a.sdf_bias;
@@ -493,8 +493,14 @@ __device__ __forceinline__ void store_sdf(const Args& a, half8 y, uint32_t col, 
 		const size_t off4 = (size_t)4u * g * a.N + col;
 #pragma unroll
 		for (int e = 0; e < 4; ++e) {
-			a.sdf_out[(size_t)e * a.N + off4] = y[e];
-			a.sdf_out[(size_t)(8 + e) * a.N + off4] = y[4 + e];
+			hf *const lo = a.sdf_out + (size_t)e * a.N + off4, *const hi = a.sdf_out + (size_t)(8 + e) * a.N + off4;
+			if (STREAM) {
+				__builtin_nontemporal_store(y[e], lo);
+				__builtin_nontemporal_store(y[4 + e], hi);
+			} else {
+				*lo = y[e];
+				*hi = y[4 + e];
+			}
 		}
 	}
 }
@@ -625,7 +631,8 @@ __device__ __forceinline__ void staged_halves(float own, float& lower, float& up
 	lower = __uint_as_float(r[0]);
 	upper = __uint_as_float(r[1]);
 }
-template <bool BLOCKS>
+// STREAM (with BLOCKS): rows are read and outputs written past the caches, each of which is met once, so that the blocks stay there (QUERY_STREAM_MIN).
+template <bool BLOCKS, bool STREAM>
 __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const FusedArgs a) {
 	extern __shared__ __align__(16) unsigned char smem[];
 	hf* F = reinterpret_cast<hf*>(smem);
@@ -676,7 +683,8 @@ __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const Fu
 			const uint32_t level = 4u * (j >> 1) + 2u * g + (j & 1);
 			// (levels that have no row read that of the first level that does and are replaced, or meet weights of zero)
 			const uint32_t lr = level < a.first_level || 2u * level >= a.enc_w ? a.first_level : level;
-			ahead[j] = query_rows(a)[(size_t)lr * N + col];
+			const uint32_t* const at = query_rows(a) + (size_t)lr * N + col;
+			ahead[j] = STREAM ? __builtin_nontemporal_load(at) : *at;
 		}
 	};
 	if constexpr (BLOCKS) fetch_rows(min(wave, n_tiles - 1u));
@@ -747,7 +755,7 @@ __global__ void __launch_bounds__(FS_BLOCK) field_staged_forward_kernel(const Fu
 		xs[0] = *reinterpret_cast<half8*>(x4);
 		half8 h[4];
 		const half8 y = sdf_net(F, lane, xs, h);
-		store_sdf(a, y, col, valid, col_raw, g);
+		store_sdf<STREAM>(a, y, col, valid, col_raw, g);
 		tile_fence();
 	}
 }
@@ -1027,6 +1035,9 @@ constexpr uint32_t QUERY_STAGED_MIN = 3u << 15;
 // 44.2 | 43.9, 2^18 77.7 | 73.3, 2^19 148 | 136, 2^20 278 | 250, 2^21 531 | 480; along rays 2^17 32.1 | 35.2, 2^18 56.1 | 57.8, 2^19 99.0 | 98.2, 2^20 182 | 177; on a lattice 2^17
 // 31.4 | 34.4, 2^18 55.1 | 56.5, 2^19 77.2 | 77.6, 2^20 141 | 136.  Updates of the occupancy grid: 2^19 samples 160.4 | 157.2, 700 000 250 | 231, 2^20 245 | 236, 2^21 415 | 400.)
 constexpr uint32_t QUERY_BLOCKS_MIN = 1u << 18;
+// ... and from here on rows and outputs are streams, which smaller queries find in the caches.  (Call in us, cached | streamed, uniform points: 2^18 71.9 | 73.6, 2^19 135.6 | 137,
+// 655 360 163.3 | 164.3, 786 432 193.7 | 193.1, 2^20 254.6 | 249.7, 1 572 864 371.5 | 363.5, 2^21 490.7 | 476.5; update of the occupancy grid, which keeps one row, 2^21 398.3 | 398.1.)
+constexpr uint32_t QUERY_STREAM_MIN = 3u << 18;
 
 // ----------------------------------------------------------------------------
 // The SDF network on its own (48 inputs: coordinates, 32 features, padding) with the eikonal loss: network, d sdf / d input, normals from the
@@ -1300,7 +1311,7 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 		others.n_levels -= a.first_level;
 		launch_gather<false>(others, s);
 		N2_LAUNCH_CHECK();
-		auto* const kernel = blocked ? field_staged_forward_kernel<true> : field_staged_forward_kernel<false>;
+		auto* const kernel = !blocked ? field_staged_forward_kernel<false, false> : n >= QUERY_STREAM_MIN ? field_staged_forward_kernel<true, true> : field_staged_forward_kernel<true, false>;
 		N2_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FS_LDS_MAX));
 		kernel<<<dim3(FS_GRID), dim3(FS_BLOCK), lds, s>>>(a);
 		N2_LAUNCH_CHECK();
