@@ -816,6 +816,11 @@ uint64_t n2_marching_cubes_workspace_bytes(const uint32_t res[3]);
 int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3],
                             float thresh, const float* d_density, void* d_workspace, uint64_t workspace_bytes,
                             uint32_t* n_vertices, uint32_t* n_triangles);
+/* The same for a caller that goes on with n2_marching_cubes_emit on the same stream: with totals in pinned host memory it waits for these and not for
+ * the stream, whose last launch may still be writing the workspace when it returns. */
+int n2_marching_cubes_count_totals(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3],
+                                   float thresh, const float* d_density, void* d_workspace, uint64_t workspace_bytes,
+                                   uint32_t* n_vertices, uint32_t* n_triangles);
 /* Second pass with the workspace of the first (it holds one bit per lattice point and what each word of 64 of them owns) and the
  * same res, density and thresh.  (Which vertices there are and which of them a triangle has comes from the workspace; with another
  * density or threshold the vertices lie elsewhere on their edges, or beyond them, and the normals are those of the other surface.)

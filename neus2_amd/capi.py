@@ -83,7 +83,7 @@ _SIGNATURES = {
     "n2_field_forward": "pppup", "n2_field_backward": "pppupui", "n2_field_sdf": "pppuuup", "n2_field_density": "pppuuup",
     "n2_sdf_forward_and_loss": "ppppuuuffp", "n2_sdf_loss_backward": "ppppuuupi",
     "n2_trainer_set_training_step": "pu", "n2_trainer_step": "ppuuu", "n2_occupancy_update": "pppfuu",
-    "n2_marching_cubes_count": "ppppfppqpp", "n2_marching_cubes_emit": "ppppfpppppuu",
+    "n2_marching_cubes_count": "ppppfppqpp", "n2_marching_cubes_count_totals": "ppppfppqpp", "n2_marching_cubes_emit": "ppppfpppppuu",
 }
 
 

@@ -159,7 +159,7 @@ __device__ const McRing MC_RING = mc_build_ring();
 // word to each row, rows of two points need 36 bytes of workspace per point; so 2.3.  All 64 bits need 1.1, but leave
 // twice as much behind one another in a workgroup: 2 x 512 x 512 points 69, 73 and 102 us.)
 // 512^3 lattice of a bumpy sphere (1.2 M triangles), in us: bits 82 (6.6 TB/s), count 14.6, scan 4.7, emit 27.7, normals 24, with
-// the host's wait for the totals 168 in all.  Deciding every point from the four rows of the density itself took 242 for the
+// the host's wait for the totals 162 in all (168 while that was for the stream; 64^3 48 -> 43, 256^3 60 -> 55).  Deciding every point from the four rows of the density itself took 242 for the
 // count alone and read the rows again for each output: 868 in all.
 // ---------------------------------------------------------------------------
 struct McGrid {
@@ -567,6 +567,10 @@ __global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2*
 			if (lane == 63u) group[wave][MC_SCAN_GROUPS] = both;
 		}
 		__syncthreads();
+		if (threadIdx.x == 0 && to_v && c0 + 1024u * MC_SCAN_EACH >= n_blocks) {  // (in front of the stores: the host waits for these)
+			__hip_atomic_store(to_v, carry[0] + group[0][MC_SCAN_GROUPS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+			__hip_atomic_store(to_t, carry[1] + group[1][MC_SCAN_GROUPS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+		}
 #pragma unroll
 		for (uint32_t k = 0; k < MC_SCAN_EACH; ++k) {
 			const uint32_t i = c0 + k * 1024u + threadIdx.x, g = k * 16u + wave;
@@ -580,7 +584,6 @@ __global__ void __launch_bounds__(1024) mc_scan_kernel(uint32_t n_blocks, uint2*
 	if (threadIdx.x == 0) {
 		blocks[n_blocks] = make_uint2(carry[0], carry[1]);
 		blocks[n_blocks + 1u] = make_uint2(carry[2], 0u);
-		if (to_v) { *to_v = carry[0]; *to_t = carry[1]; }
 	}
 }
 
@@ -952,15 +955,28 @@ static void mc_totals_of(uint32_t* n_vertices, uint32_t* n_triangles, uint32_t*&
 	if (t) { to_v = v; to_t = t; }
 }
 
-N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,
-                                   const float* d_density, void* d_workspace, uint64_t workspace_bytes, uint32_t* n_vertices,
-                                   uint32_t* n_triangles) {
+// Waits for the totals that the scan leaves in pinned memory (MC_NO_TOTAL before): for them alone, not for the end of the launch and what the runtime does about it.
+// Where the work in front takes long, fails, or is being captured, for the stream.
+constexpr uint32_t MC_NO_TOTAL = 0xFFFFFFFFu;
+static hipError_t mc_await_totals(hipStream_t s, const uint32_t* n_vertices, const uint32_t* n_triangles) {
+	hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
+		for (int spins = 0; spins < 1 << 15; ++spins) {  // (some 1000 us)
+			if (__atomic_load_n(n_vertices, __ATOMIC_ACQUIRE) != MC_NO_TOTAL && __atomic_load_n(n_triangles, __ATOMIC_ACQUIRE) != MC_NO_TOTAL) return hipSuccess;
+			__builtin_ia32_pause();
+		}
+	}
+	return hipStreamSynchronize(s);
+}
+
+static int mc_count(const char* name, n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh, const float* d_density, void* d_workspace,
+                    uint64_t workspace_bytes, uint32_t* n_vertices, uint32_t* n_triangles, bool totals_only) {
 	uint64_t n;
-	if (int rc = mc_check("n2_marching_cubes_count", res, n)) return rc;
-	N2_REQUIRE(d_density && d_workspace && n_vertices && n_triangles && aabb_min && aabb_max, "n2_marching_cubes_count: null argument");
-	N2_REQUIRE(reinterpret_cast<uintptr_t>(d_workspace) % 256 == 0, "n2_marching_cubes_count: workspace must be 256-byte aligned");
+	if (int rc = mc_check(name, res, n)) return rc;
+	N2_REQUIRE(d_density && d_workspace && n_vertices && n_triangles && aabb_min && aabb_max, "%s: null argument", name);
+	N2_REQUIRE(reinterpret_cast<uintptr_t>(d_workspace) % 256 == 0, "%s: workspace must be 256-byte aligned", name);
 	const McCarve c = mc_carve(res);
-	N2_REQUIRE(workspace_bytes >= c.total, "n2_marching_cubes_count: %llu bytes of workspace given, %llu needed",
+	N2_REQUIRE(workspace_bytes >= c.total, "%s: %llu bytes of workspace given, %llu needed", name,
 	           (unsigned long long)workspace_bytes, (unsigned long long)c.total);
 	hipStream_t s = n2_stream(stream);
 	unsigned char* b = reinterpret_cast<unsigned char*>(d_workspace);
@@ -978,16 +994,37 @@ N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], co
 	// (left there by the scan: 512^3 182 us, 64^3 53; copied, with a copy kernel and its staging, 191 and 61)
 	uint32_t *to_v, *to_t;
 	mc_totals_of(n_vertices, n_triangles, to_v, to_t);
+	if (to_v && totals_only) {
+		__atomic_store_n(n_vertices, MC_NO_TOTAL, __ATOMIC_RELEASE);
+		__atomic_store_n(n_triangles, MC_NO_TOTAL, __ATOMIC_RELEASE);
+	}
 	mc_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(c.n_blocks, blocks, reinterpret_cast<uint32_t*>(b + c.listed), to_v, to_t);
 	N2_LAUNCH_CHECK();
 	uint32_t host[2] = {0, 0};
-	if (!to_v) N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
-	N2_HIP(hipStreamSynchronize(s));
-	if (to_v) { host[0] = *n_vertices; host[1] = *n_triangles; }
-	N2_REQUIRE(host[0] < (1u << 29), "n2_marching_cubes_count: %u vertices exceed the 2^29 limit", host[0]);
+	if (to_v) {
+		N2_HIP(totals_only ? mc_await_totals(s, n_vertices, n_triangles) : hipStreamSynchronize(s));
+		host[0] = *n_vertices;
+		host[1] = *n_triangles;
+	} else {
+		N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
+		N2_HIP(hipStreamSynchronize(s));
+	}
+	N2_REQUIRE(host[0] < (1u << 29), "%s: %u vertices exceed the 2^29 limit", name, host[0]);
 	*n_vertices = host[0];
 	*n_triangles = host[1];
 	return N2_OK;
+}
+
+N2_API int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,
+                                   const float* d_density, void* d_workspace, uint64_t workspace_bytes, uint32_t* n_vertices,
+                                   uint32_t* n_triangles) {
+	return mc_count("n2_marching_cubes_count", stream, res, aabb_min, aabb_max, thresh, d_density, d_workspace, workspace_bytes, n_vertices, n_triangles, false);
+}
+
+N2_API int n2_marching_cubes_count_totals(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,
+                                          const float* d_density, void* d_workspace, uint64_t workspace_bytes, uint32_t* n_vertices,
+                                          uint32_t* n_triangles) {
+	return mc_count("n2_marching_cubes_count_totals", stream, res, aabb_min, aabb_max, thresh, d_density, d_workspace, workspace_bytes, n_vertices, n_triangles, true);
 }
 
 N2_API int n2_marching_cubes_emit(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3], float thresh,

@@ -67,7 +67,7 @@ def marching_cubes(density, thresh, aabb_min=(0, 0, 0), aabb_max=(1, 1, 1), want
     # (what the second call takes is ready before the first one waits for the totals)
     head = (_stream_address(), _u3(res), _f3(aabb_min), _f3(aabb_max), thresh, density.data_ptr(), ws.data_ptr())
     emit = L.n2_marching_cubes_emit
-    check(L.n2_marching_cubes_count(*head, nbytes, at, at + 4), "n2_marching_cubes_count")
+    check(L.n2_marching_cubes_count_totals(*head, nbytes, at, at + 4), "n2_marching_cubes_count_totals")
     n_verts, n_tris = nv.value, nt.value
     verts = torch.empty(n_verts, 3, dtype=torch.float32, device=device)
     idx = torch.empty(n_tris, 3, dtype=torch.int32, device=device)

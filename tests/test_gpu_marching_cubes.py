@@ -165,6 +165,34 @@ def test_totals_in_pinned_and_in_other_host_memory():
             assert int((pinned == -1).sum() + (pageable == -1).sum()) == 46
 
 
+@pytest.mark.parametrize("res", [(2, 2, 2), (9, 8, 21), (65, 64, 3), (17, 1500, 1500)])  # one block of words, short rows, several blocks, more than the scan takes in a round
+@pytest.mark.parametrize("busy", [False, True])  # nothing in front, or more work than the wait for the totals alone lasts
+def test_totals_that_are_waited_for_alone(res, busy):
+    import ctypes as C
+
+    from neus2_amd import capi
+    from neus2_amd.mesh import _f3, _stream_address, _u3, marching_cubes
+    L = capi.lib()
+    L.n2_marching_cubes_workspace_bytes.restype = C.c_uint64
+    x, y, z = (torch.arange(r, device="cuda") for r in res)
+    f = (torch.sin(1.7 * x + 1)[None, None, :] + torch.sin(0.11 * y)[None, :, None] + torch.sin(0.13 * z + 2)[:, None, None]).contiguous()
+    v, t, n = marching_cubes(f, 0.0)
+    nbytes = int(L.n2_marching_cubes_workspace_bytes(_u3(res)))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    head = (_stream_address(), _u3(res), _f3((0, 0, 0)), _f3((1, 1, 1)), 0.0, f.data_ptr(), ws.data_ptr())
+    load = torch.zeros(1 << 28, device="cuda")
+    for totals in (torch.empty(2, dtype=torch.int32, pin_memory=True), torch.empty(2, dtype=torch.int32)):
+        totals.fill_(7)
+        torch.cuda.synchronize()
+        for _ in range(20 if busy else 0):
+            load.add_(1.0)
+        capi.check(L.n2_marching_cubes_count_totals(*head, nbytes, totals.data_ptr(), totals.data_ptr() + 4), "count_totals")
+        assert totals.tolist() == [len(v), len(t)]
+        verts, normals, idx = torch.zeros_like(v), torch.zeros_like(n), torch.zeros_like(t)
+        capi.check(L.n2_marching_cubes_emit(*head, verts.data_ptr() or None, idx.data_ptr() or None, normals.data_ptr() or None, len(v), len(t)), "emit")
+        assert torch.equal(verts, v) and torch.equal(idx, t) and torch.equal(normals, n)
+
+
 def test_empty_lattice_and_errors():
     from neus2_amd import capi
     from neus2_amd.mesh import marching_cubes
