@@ -895,9 +895,10 @@ N2_API int n2_sdf_forward_and_loss(n2_grid_t* grid, n2_mlp_t* mlp, n2_stream_t s
 	uint32_t enc_w, in_w;
 	if (int rc = check_sdf_step(fn, grid, mlp, d_xyz, point_stride, dim_stride, n, b, enc_w, in_w)) return rc;
 	N2_REQUIRE(n2_mlp_weights(mlp) != nullptr, "%s: n2_mlp_set_params has not been called", fn);
-	if (int rc = n2_grid_forward_sdf_input(grid, stream, d_xyz, point_stride, dim_stride, n, b->input, b->dy_dx)) return rc;
 	// (the kernel's lanes hold sixteen levels and the coordinates of a network with one hidden layer)
-	if (in_w == 48 && enc_w == 32 && n2_mlp_n_params(mlp) == 64 * 48 + 16 * 64 && n2_sdf_one_pass(n)) {
+	const bool one_pass = in_w == 48 && enc_w == 32 && n2_mlp_n_params(mlp) == 64 * 48 + 16 * 64 && n2_sdf_one_pass(n);
+	if (int rc = n2_grid_forward_sdf_input(grid, stream, d_xyz, point_stride, dim_stride, n, b->input, b->dy_dx, one_pass)) return rc;
+	if (one_pass) {
 		hipStream_t s = n2_stream(stream);
 		float* parts = reinterpret_cast<float*>(b->workspace);
 		if (int rc = n2_fused_sdf_eikonal(s, n2_mlp_weights(mlp), n, b->input, b->dy_dx, b->output, b->dsdf_dinput, b->normal, ek_weight, loss_scale / (float)n,

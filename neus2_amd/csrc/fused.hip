@@ -1345,7 +1345,7 @@ int n2_fused_sdf_eikonal(hipStream_t s, const n2_half* weights, uint32_t n, cons
 	a.v = v;
 	a.v_in = reinterpret_cast<hf*>(v_in);
 	a.parts = parts;
-	if (n2_jacobian_streams(n, 32u)) sdf_eikonal_forward_kernel<true><<<dim3(fused_grid(n)), dim3(FF_BLOCK), 0, s>>>(a);
+	if (n2_step_jacobian_loads_stream(n, 32u)) sdf_eikonal_forward_kernel<true><<<dim3(fused_grid(n)), dim3(FF_BLOCK), 0, s>>>(a);
 	else sdf_eikonal_forward_kernel<false><<<dim3(fused_grid(n)), dim3(FF_BLOCK), 0, s>>>(a);
 	N2_LAUNCH_CHECK();
 	return N2_OK;

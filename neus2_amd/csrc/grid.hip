@@ -1654,7 +1654,7 @@ static uint32_t make_xcd_plan(const n2_grid_t* grid, uint32_t tiles, N2XcdPlan& 
 }
 
 static int grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
-                        uint32_t dim_stride, uint32_t n_points, n2_half* d_out, float* d_dy_dx, n2_half* d_centred) {
+                        uint32_t dim_stride, uint32_t n_points, n2_half* d_out, float* d_dy_dx, n2_half* d_centred, bool one_reader) {
 	if (int rc = check_batch(grid, "n2_grid_forward", d_xyz, point_stride, dim_stride, n_points)) return rc;
 	if (n_points == 0) return N2_OK;
 	N2_REQUIRE(d_out != nullptr, "n2_grid_forward: d_out is null");
@@ -1673,7 +1673,8 @@ static int grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz,
 	plan.begin[N_XCD] = 0;
 	plan.height = dealt.y;
 	const dim3 grid_dim = grid->costs_set ? dim3(make_xcd_plan(grid, tiles, plan) * N_XCD) : dim3(dealt.x, dealt.y), block(GRID_BLOCK);
-	const bool streams = n2_jacobian_streams(n_points, grid->tab.n_levels * grid->n_features);
+	const uint32_t rows = grid->tab.n_levels * grid->n_features;
+	const bool streams = one_reader ? n2_step_jacobian_stores_stream(n_points, rows) : n2_jacobian_streams(n_points, rows);
 	auto* const kernel = !d_dy_dx ? grid_forward_kernel<false, false> : streams ? grid_forward_kernel<true, true> : grid_forward_kernel<true, false>;
 	kernel<<<grid_dim, block, 0, n2_stream(stream)>>>(grid->tab, plan, n_points, tiles, d_xyz, point_stride, dim_stride, grid->params,
 	                                                  reinterpret_cast<__half*>(d_out), d_dy_dx, reinterpret_cast<__half*>(d_centred));
@@ -1682,11 +1683,11 @@ static int grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz,
 }
 N2_API int n2_grid_forward(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,
                            uint32_t dim_stride, uint32_t n_points, n2_half* d_out, float* d_dy_dx) {
-	return grid_forward(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_out, d_dy_dx, nullptr);
+	return grid_forward(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_out, d_dy_dx, nullptr, false);
 }
 int n2_grid_forward_sdf_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points, n2_half* d_input,
-                              float* d_dy_dx) {
-	return grid_forward(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_input ? d_input + (size_t)3 * n_points : nullptr, d_dy_dx, d_input);
+                              float* d_dy_dx, bool one_reader) {
+	return grid_forward(grid, stream, d_xyz, point_stride, dim_stride, n_points, d_input ? d_input + (size_t)3 * n_points : nullptr, d_dy_dx, d_input, one_reader);
 }
 
 N2_API int n2_grid_corner_indices(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride,

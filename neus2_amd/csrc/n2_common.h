@@ -149,8 +149,9 @@ uint32_t n2_fused_sdf_eikonal_parts(uint32_t n);
 int n2_fused_sdf_eikonal(hipStream_t s, const n2_half* weights, uint32_t n, const n2_half* input, const float* dy_dx, n2_half* output, n2_half* dsdf, float* normal,
                          float ek_weight, float scale, n2_half* dL_dy, float* v, n2_half* v_in, float* parts);
 // n2_grid_forward into rows 3.. of the SDF network's input (n_points columns), and the centred positions into rows 0..2
+// one_reader: the Jacobian's next and only reader is n2_fused_sdf_eikonal
 int n2_grid_forward_sdf_input(n2_grid_t* grid, n2_stream_t stream, const float* d_xyz, uint32_t point_stride, uint32_t dim_stride, uint32_t n_points, n2_half* d_input,
-                              float* d_dy_dx);
+                              float* d_dy_dx, bool one_reader);
 bool n2_grid_has_gradients(const n2_grid_t* grid);  // parameters and gradients are set
 // the network's weights (null: not set) and whether its slab sums are deferred by its owner
 const n2_half* n2_mlp_weights(const n2_mlp_t* mlp);
@@ -305,3 +306,9 @@ __device__ __forceinline__ void n2_store3(float* p, n2_float3 v) {
 // 2^19 434 | 430 | 430 | 423; 2^17 (48 MiB) 108 in all four, along rays 92.  The SDF network with the eikonal term, 2^18: uniform 283 | 285 | 288 | 287,
 // along rays 244 | 236 | 241 | 235; 2^17 155 | 154 | 155 | 153.
 static inline bool n2_jacobian_streams(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (64ull << 20); }
+// In the SDF network's step it is read once, by the launch right behind the one that writes it (n2_fused_sdf_eikonal): the stores stay in the last-level cache up to where
+// that is full, and the loads, which nothing follows, are streamed much earlier.  Step in us, by the rule above | this one: 32 768 uniform 68.3 | 66.3, 65 536 along rays 83.2 | 81.8, 2^17
+// 124.7 | 124.1 (uniform 144.4 | 145.0), 180 000 159.0 | 154.4, 2^18 209.6 | 204.6 (uniform 257.2 | 253.2), 393 216 uniform 377.4 | 364.5; with the stores cached beyond 2^19 along rays
+// 380.6 | 385.0 (uniform 489.9 | 479.2), 2^20 752.9 | 771.8; with the loads streamed 8192 37.6 | 37.9.
+static inline bool n2_step_jacobian_stores_stream(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (160ull << 20); }
+static inline bool n2_step_jacobian_loads_stream(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (12ull << 20); }
