@@ -1037,6 +1037,8 @@ constexpr uint32_t QUERY_STAGED_MIN = 3u << 15;
 constexpr uint32_t QUERY_BLOCKS_MIN = 1u << 18;
 // ... and from here on rows and outputs are streams, which smaller queries find in the caches.  (Call in us, cached | streamed, uniform points: 2^18 71.9 | 73.6, 2^19 135.6 | 137,
 // 655 360 163.3 | 164.3, 786 432 193.7 | 193.1, 2^20 254.6 | 249.7, 1 572 864 371.5 | 363.5, 2^21 490.7 | 476.5; update of the occupancy grid, which keeps one row, 2^21 398.3 | 398.1.)
+// Only where every row of features starts a line: of a line that two tiles share, the first one's streamed load takes it from the second (800 008 points 206.4 | 208.4, 1 000 008
+// 251.7 | 253.6, 2 000 008 485.4 | 487.6).
 constexpr uint32_t QUERY_STREAM_MIN = 3u << 18;
 
 // ----------------------------------------------------------------------------
@@ -1311,7 +1313,7 @@ int n2_fused_field_sdf(const N2FusedNets& nets, hipStream_t s, const float* d_xy
 		others.n_levels -= a.first_level;
 		launch_gather<false>(others, s);
 		N2_LAUNCH_CHECK();
-		auto* const kernel = !blocked ? field_staged_forward_kernel<false, false> : n >= QUERY_STREAM_MIN ? field_staged_forward_kernel<true, true> : field_staged_forward_kernel<true, false>;
+		auto* const kernel = !blocked ? field_staged_forward_kernel<false, false> : n >= QUERY_STREAM_MIN && n2_rows_of_whole_lines(n, 4u) ? field_staged_forward_kernel<true, true> : field_staged_forward_kernel<true, false>;
 		N2_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FS_LDS_MAX));
 		kernel<<<dim3(FS_GRID), dim3(FS_BLOCK), lds, s>>>(a);
 		N2_LAUNCH_CHECK();

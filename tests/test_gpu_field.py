@@ -193,6 +193,12 @@ def test_large_queries_equal_their_parts(n, cfg, active):
             assert torch.equal(got[:, a:a + part].view(torch.int16), want.view(torch.int16)), a
 
 
+# both sides of where rows and outputs pass by the caches, and a size beyond whose rows do not start lines
+@pytest.mark.parametrize("n", [(3 << 18) - 32, 3 << 18, (3 << 18) + 8, (3 << 18) + 32])
+def test_streamed_queries_equal_their_parts(n):
+    test_large_queries_equal_their_parts(n, {}, 1.0)
+
+
 # one tile past the line at which a query's and a forward's levels are no longer dealt to the XCDs
 @pytest.mark.parametrize("levels", [16, 14, 1])
 def test_batches_past_the_deal_by_xcd_equal_their_parts(levels):

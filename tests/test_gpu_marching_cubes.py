@@ -265,8 +265,6 @@ def test_lattices_walked_by_rows_equal_the_same_points_queried(side, res, part, 
     assert_close(got, want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
 
 
-# The features of a slab lie in the scratch and, behind the slab, in the output: slabs that take both, the output alone (a scratch of less than a plane),
-# planes in parts at the end, gathered and by rows, an output that starts anywhere; no fine level at all
 # The finest level's row that a run of 64 points meets, in chunks of four entries: each number of words a lane takes, and both sides of where it becomes one
 # more, wide loads begin and the points gather for themselves; by waves of two planes, whose loads are wide always, and of five.
 @pytest.mark.parametrize("rows", [(6, 9), (160, 130)])
@@ -300,6 +298,8 @@ def test_fine_rows_of_every_length(chunks, rows):
     assert_close(host(d), want, rtol=RTOL, what="SDF lattice", outlier_frac=1e-3)
 
 
+# The features of a slab lie in the scratch and, behind the slab, in the output: slabs that take both, the output alone (a scratch of less than a plane),
+# planes in parts at the end, gathered and by rows, an output that starts anywhere; no fine level at all
 @pytest.mark.parametrize("res,chunk,levels", [((70, 9, 60), 512, 16), ((70, 9, 60), 64, 16), ((130, 7, 33), 8, 16), ((300, 11, 90), 4096, 16), ((96, 33, 300), 1 << 14, 16),
                                               ((64, 8, 40), 256, 4)])
 def test_a_lattice_in_slabs_equals_the_lattice_at_once(res, chunk, levels):

@@ -158,6 +158,12 @@ def test_step_equals_the_single_calls(n_levels, n, kind):
         close(got["mlp"][:64 * in_w].view(64, in_w)[:, c], gW[:64 * in_w].view(64, in_w)[:, c], 2.4e-3, ("column", c))
 
 
+# both sides of where the Jacobian's loads are streamed, and sizes beyond whose rows do not start lines, below and from 64 MiB on
+@pytest.mark.parametrize("n", [32768 - 32, 32768, 32768 + 8, 174763 + 5])
+def test_a_streamed_step_equals_the_single_calls(n):
+    test_step_equals_the_single_calls(16, n, "")
+
+
 def test_points_beyond_the_one_pass_kernels_offsets():
     """72 million points, whose last two million lie more than 2^32 bytes behind their row of the Jacobian: outputs, normals and J v of the last ones as in a batch of their own."""
     from neus2_amd.sdf_net import SdfNet
