@@ -477,7 +477,7 @@ struct N2BinInput {
 	float p[3], v[3];
 	__half dy[2], g2[2];
 };
-template <bool FIRST, bool SECOND>
+template <bool FIRST, bool SECOND, bool STREAM>
 __device__ __forceinline__ N2BinInput grid_bin_load(uint32_t level, uint32_t i, uint32_t N, const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                                     const __half* __restrict__ dL_dy, const float* __restrict__ v, const __half* __restrict__ g2, uint32_t xi, uint32_t Ng) {
 	N2BinInput in;
@@ -487,8 +487,8 @@ __device__ __forceinline__ N2BinInput grid_bin_load(uint32_t level, uint32_t i, 
 	for (int d = 0; d < 3; ++d) in.p[d] = q[(size_t)d * dim_stride];
 #pragma unroll
 	for (int f = 0; f < 2; ++f) {
-		if (FIRST) in.dy[f] = dL_dy[(row + f) * N + i];
-		if (SECOND) in.g2[f] = g2[(row + f) * Ng + xi];
+		if (FIRST) in.dy[f] = n2_load_half<STREAM>(dL_dy + (row + f) * N + i);
+		if (SECOND) in.g2[f] = n2_load_half<STREAM>(g2 + (row + f) * Ng + xi);
 	}
 #pragma unroll
 	for (int d = 0; d < 3; ++d)
@@ -586,7 +586,7 @@ constexpr uint32_t REC_SKIP = 0xFFFFFFFFu;
 // updates and prefix look-ups are therefore issued together, and nothing waits in a branch.  With each of them awaited where it was used,
 // and the second point's loads behind the first one's counters: training step at 2^18 samples 69 us, now 59 (57 and 47 on another card); trained 58, now 51; 2^18 uniform points
 // 51.5, now 47.8; 52344 samples 15.1, now 12.7.
-template <uint32_t PER, bool FIRST, bool SECOND, bool PAIR>
+template <uint32_t PER, bool FIRST, bool SECOND, bool PAIR, bool STREAM>
 __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uint32_t level, const uint32_t tile, uint32_t N, uint32_t tiles,
                                               const float* __restrict__ xyz, uint32_t point_stride, uint32_t dim_stride,
                                               const __half* __restrict__ dL_dy, const float* __restrict__ v, const __half* __restrict__ g2,
@@ -613,7 +613,7 @@ __device__ __forceinline__ void grid_bin_tile(const N2LevelTable& tab, const uin
 	}
 	auto load = [&](uint32_t j) __attribute__((always_inline)) {
 		const uint32_t i = min(tile * bin_points(PER) + j * BIN_BLOCK + threadIdx.x, N - 1u);
-		return grid_bin_load<FIRST, SECOND>(level, i, N, xyz, point_stride, dim_stride, dL_dy, v, g2, src[j], Ng);
+		return grid_bin_load<FIRST, SECOND, STREAM>(level, i, N, xyz, point_stride, dim_stride, dL_dy, v, g2, src[j], Ng);
 	};
 	N2BinInput next = load(0);
 #pragma unroll
@@ -776,7 +776,7 @@ __device__ __forceinline__ void grid_second_item(const N2LevelTable& tab, uint32
 	dL_ddLdy[((size_t)level * 2 + 1) * N + i] = __high2half(h);
 }
 
-template <uint32_t PER, bool FIRST, bool SECOND, class Ride>
+template <uint32_t PER, bool FIRST, bool SECOND, bool STREAM, class Ride>
 __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab, uint32_t first_level, uint32_t N, uint32_t tiles,
                                                               const float* __restrict__ xyz, uint32_t point_stride,
                                                               uint32_t dim_stride, const __half* __restrict__ dL_dy,
@@ -830,10 +830,10 @@ __global__ void __launch_bounds__(BIN_BLOCK, 6) grid_bin_kernel(N2LevelTable tab
 	if (threadIdx.x < BKT_MAX) hist[threadIdx.x] = 0;
 	__syncthreads();
 	if ((tab.pair_levels >> level) & 1u)
-		grid_bin_tile<PER, FIRST, SECOND, true>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, rec_vals,
+		grid_bin_tile<PER, FIRST, SECOND, true, STREAM>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, rec_vals,
 		                                        rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
 	else
-		grid_bin_tile<PER, FIRST, SECOND, false>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, rec_vals,
+		grid_bin_tile<PER, FIRST, SECOND, false, STREAM>(tab, level, tile, N, tiles, xyz, point_stride, dim_stride, dL_dy, v, g2, rec_vals,
 		                                         rec_keys, offsets, hist, prefix, stage_val, stage_key, index, n_cols);
 }
 
@@ -1898,27 +1898,33 @@ static int launch_bucketed(n2_grid_t* grid, hipStream_t s, const float* d_xyz, u
 			const N2GatherGrid g = n2_rows_of_blocks(blocks, BIN_BLOCK);
 			return dim3(g.x, g.y);
 		};
-#define LAUNCH(F, S, RIDE, BLOCKS) grid_bin_kernel<PER, F, S><<<launch_dim(RIDE, BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
+#define LAUNCH(F, S, STREAM, RIDE, BLOCKS) grid_bin_kernel<PER, F, S, STREAM><<<launch_dim(RIDE, BLOCKS), bd, 0, s>>>(tab, 0u, n_points, tiles, d_xyz, point_stride, dim_stride, dL_dy, v, g2, \
                                                                                                     grid->params, rec_vals, rec_keys, offsets, queue, index, n_cols, RIDE)
 		const uint32_t blocks = tiles * L;
 		const N2RideNone none;
+		// The rows of a fused backward are the step's own, and this is their last use: past the caches, where each wave of 64 points takes whole lines of them.  In us, cached | streamed: the
+		// field's forward and backward 2^18 240.9 | 237.4, SDF network's step 2^18 253.4 | 250.4, training step 2^18 338.4 | 336.5, trained 492.0 | 492.3, 2^16 184.1 | 183.6; of lines
+		// that two waves share, field 200 008 198.8 | 202.0, SDF network 100 008 131.3 | 133.3.  (The encoding's own backward reads a caller's rows, beside others that do.)
+		const bool rows_stream = n2_rows_of_whole_lines(n_points, 2u) && (!index || n2_rows_of_whole_lines(n_cols, 2u));
 		if (rider.dL_dx != nullptr) {  // (first order alone)
 			const N2Turns turns = n2_turns(blocks, (n_points + BIN_BLOCK - 1) / BIN_BLOCK, 1u);
 			const uint32_t rows = L * grid->n_features;
-			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, turns.every}), turns.blocks);
-			else LAUNCH(true, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, turns.every}), turns.blocks);
+			if (n2_jacobian_streams(n_points, rows)) LAUNCH(true, false, false, (N2RideInput<true>{rider.dy_dx, rider.dL_dx, rows, turns.every}), turns.blocks);
+			else LAUNCH(true, false, false, (N2RideInput<false>{rider.dy_dx, rider.dL_dx, rows, turns.every}), turns.blocks);
 		} else if (rider.sums.units > 0) {  // (both orders)
 			const uint32_t riders = (rider.sums.units + BIN_BLOCK / 256 - 1) / (BIN_BLOCK / 256);
-			LAUNCH(true, true, (N2RideSums{rider.sums, riders}), riders + blocks);
+			if (rows_stream) LAUNCH(true, true, true, (N2RideSums{rider.sums, riders}), riders + blocks);
+			else LAUNCH(true, true, false, (N2RideSums{rider.sums, riders}), riders + blocks);
 		} else if (out) {
 			const N2GatherGrid g = n2_gather_grid(N2_ENCODING_XCD_MAX, n_points, L, BIN_BLOCK);
 			const N2Turns turns = n2_turns(g.x * g.y, blocks, N_XCD);
 			const N2RideSecond ride{dL_ddLdy, g.x * g.y, turns.every, (n_points + BIN_BLOCK - 1) / BIN_BLOCK, g.y};
-			if (first) LAUNCH(true, true, ride, turns.blocks);
-			else LAUNCH(false, true, ride, turns.blocks);
-		} else if (first && second) LAUNCH(true, true, none, blocks);
-		else if (second) LAUNCH(false, true, none, blocks);
-		else LAUNCH(true, false, none, blocks);
+			if (first) LAUNCH(true, true, false, ride, turns.blocks);
+			else LAUNCH(false, true, false, ride, turns.blocks);
+		} else if (first && second && rows_stream) LAUNCH(true, true, true, none, blocks);
+		else if (first && second) LAUNCH(true, true, false, none, blocks);
+		else if (second) LAUNCH(false, true, false, none, blocks);
+		else LAUNCH(true, false, false, none, blocks);
 #undef LAUNCH
 	};
 	if (per == 1u) bin(std::integral_constant<uint32_t, 1>());

@@ -289,6 +289,11 @@ typedef uint32_t n2_u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float4 n2_stream_load(const float4* p) { return __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const n2_u32x4*>(p))); }
 __device__ __forceinline__ uint4 n2_stream_load(const uint4* p) { return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const n2_u32x4*>(p))); }
 __device__ __forceinline__ void n2_stream_store(float4* p, float4 v) { __builtin_nontemporal_store(__builtin_bit_cast(n2_u32x4, v), reinterpret_cast<n2_u32x4*>(p)); }
+template <bool STREAM>
+__device__ __forceinline__ __half n2_load_half(const __half* p) {
+	if constexpr (STREAM) return __builtin_bit_cast(__half, __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(p)));
+	else return *p;
+}
 // three floats at a 12-byte pitch: a point's row of the encoding's Jacobian
 typedef float n2_float3 __attribute__((ext_vector_type(3), aligned(4)));
 template <bool STREAM>
