@@ -21,7 +21,7 @@
 // Features and SDF are written, and features read, as streams that pass by the caches: each is met once, and the tables stay where they are (us: 512^3 3905 -> 3840, the walk's alone 3815;
 // 464^3 3628 -> 3546, 400^3 2367 -> 2315, 192^3 399 -> 392, 128^3 160.9 -> 159.6; 448 x 512 x 96 1026 -> 1024, with the walk's alone 1035).
 // Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before the features were streams, before | now, us: 64^3 59.7 | 57.7, 80^3 73 | 72, 96^3 96 | 96, 128^3 171 | 166, 208^3 611 | 571, 256^3 935 | 890,
-// 320^3 1600 | 1480, 400^3 2720 | 2500, 464^3 4047 | 3656, 512 x 64 x 512 690 | 630, 64 x 512 x 512 1575 | 1550; with a chunk of 2^20 points 256^3 1045 | 981, 512^3 4550 | 4263.
+// 320^3 1600 | 1480, 400^3 2720 | 2500, 464^3 4047 | 3656, 512 x 64 x 512 690 | 630, 64 x 512 x 512 1575 | 1423; with a chunk of 2^20 points 256^3 1045 | 981, 512^3 4550 | 4263.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -317,16 +317,26 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 		return;
 	}
 	const uint32_t x0 = x_part(hashed, entries, res, cx), x1 = x_part(hashed, entries, res, cx + 1u);
-	for (uint32_t k = 0; k < nz; ++k) {
-		uint32_t raw[8];
+	auto load = [&](uint32_t k, uint32_t (&raw)[8]) __attribute__((always_inline)) {
 #pragma unroll
 		for (uint32_t q = 0; q < 4; ++q) {
 			const uint32_t row = lane_u32(rows[q], k);
 			raw[2 * q] = *reinterpret_cast<const uint32_t*>(base + vertex(hashed, bytes, x0, row));
 			raw[2 * q + 1] = *reinterpret_cast<const uint32_t*>(base + vertex(hashed, bytes, x1, row));
 		}
-		finish(k, raw);
+	};
+	// The next plane's vertices are asked for in front of a plane's store: behind it, the wait for them is one for the store as well, which passes by the caches.  Lattices whose runs
+	// are longer than a row of LDS, in us, behind | in front: 64 x 512 x 512 1518 | 1423, 64 x 480 x 304 919 | 866, 80 x 512 x 512 1860 | 1808, 160 x 320 x 480 1538 | 1507, 64^3 56.1 | 54.0, 96^3 95.3 |
+	// 94.0, 128^3 161.3 | 158.8; others as before.
+	uint32_t raw[8], next[8];
+	load(0, raw);
+	for (uint32_t k = 1; k < nz; ++k) {
+		load(k, next);
+		finish(k - 1u, raw);
+#pragma unroll
+		for (uint32_t q = 0; q < 8; ++q) raw[q] = next[q];
 	}
+	finish(nz - 1u, raw);
 }
 
 // exchange of the upper 32 lanes of `a` with the lower 32 of `b`
