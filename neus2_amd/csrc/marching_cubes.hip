@@ -1009,6 +1009,7 @@ static int mc_count(const char* name, n2_stream_t stream, const uint32_t res[3],
 		N2_HIP(hipMemcpyAsync(host, blocks + c.n_blocks, sizeof(host), hipMemcpyDeviceToHost, s));
 		N2_HIP(hipStreamSynchronize(s));
 	}
+	if (host[0] >= (1u << 29) && totals_only) N2_HIP(hipStreamSynchronize(s));  // (no second pass will follow: nothing may be under way in a workspace that the caller frees or reuses)
 	N2_REQUIRE(host[0] < (1u << 29), "%s: %u vertices exceed the 2^29 limit", name, host[0]);
 	*n_vertices = host[0];
 	*n_triangles = host[1];

@@ -193,6 +193,29 @@ def test_totals_that_are_waited_for_alone(res, busy):
         assert torch.equal(verts, v) and torch.equal(idx, t) and torch.equal(normals, n)
 
 
+def test_too_many_vertices_leave_nothing_under_way():
+    """A caller that is told so goes on with no second pass, and may free the workspace: the call has waited for the stream, not for the totals alone."""
+    import ctypes as C
+
+    from neus2_amd import capi
+    from neus2_amd.mesh import _f3, _stream_address, _u3
+    L = capi.lib()
+    L.n2_marching_cubes_workspace_bytes.restype = C.c_uint64
+    side = 576  # every edge between neighbours is cut: 3 * 576 * 576 * 575 = 1.07 * 2^29 vertices
+    x = torch.arange(side, device="cuda", dtype=torch.int16)
+    f = (((x[None, None, :] + x[None, :, None] + x[:, None, None]) & 1).float() - 0.5).contiguous()
+    res = _u3((side, side, side))
+    nbytes = int(L.n2_marching_cubes_workspace_bytes(res))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    totals = torch.empty(2, dtype=torch.int32, pin_memory=True)
+    stream = torch.cuda.current_stream()
+    torch.cuda.synchronize()
+    for count in (L.n2_marching_cubes_count_totals, L.n2_marching_cubes_count):
+        rc = count(_stream_address(), res, _f3((0, 0, 0)), _f3((1, 1, 1)), 0.0, f.data_ptr(), ws.data_ptr(), nbytes, totals.data_ptr(), totals.data_ptr() + 4)
+        assert stream.query()
+        assert rc != 0 and b"vertices exceed" in L.n2_last_error()
+
+
 def test_empty_lattice_and_errors():
     from neus2_amd import capi
     from neus2_amd.mesh import marching_cubes
