@@ -816,9 +816,9 @@ uint64_t n2_marching_cubes_workspace_bytes(const uint32_t res[3]);
 int n2_marching_cubes_count(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3],
                             float thresh, const float* d_density, void* d_workspace, uint64_t workspace_bytes,
                             uint32_t* n_vertices, uint32_t* n_triangles);
-/* The same for a caller that goes on with n2_marching_cubes_emit on the same stream: with totals in pinned host memory it waits for these and not for
- * the stream, whose last launch may still be writing the workspace when it returns.  (Not where it returns that there are too many vertices, 2^29 or more: nothing is
- * under way then.) */
+/* The same for a caller that goes on with n2_marching_cubes_emit on the same stream.  With totals in pinned host memory it waits for these and not for the stream, whose last
+ * launch may still be writing the workspace when it returns; but it does wait for the stream where the totals are not there within a millisecond (long work in front of them),
+ * in a capture, which that ends with an error, and before it returns that there are too many vertices (2^29 or more). */
 int n2_marching_cubes_count_totals(n2_stream_t stream, const uint32_t res[3], const float aabb_min[3], const float aabb_max[3],
                                    float thresh, const float* d_density, void* d_workspace, uint64_t workspace_bytes,
                                    uint32_t* n_vertices, uint32_t* n_triangles);

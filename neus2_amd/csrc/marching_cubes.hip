@@ -24,6 +24,7 @@
 // Vertex positions are part of the bit-exact contract with the CPU oracle:
 // floating-point contraction is off for this file.
 #include "n2_common.h"
+#include "bounded_wait.h"
 #include "launch_rules.h"
 
 #include <cstring>
@@ -956,15 +957,14 @@ static void mc_totals_of(uint32_t* n_vertices, uint32_t* n_triangles, uint32_t*&
 }
 
 // Waits for the totals that the scan leaves in pinned memory (MC_NO_TOTAL before): for them alone, not for the end of the launch and what the runtime does about it.
-// Where the work in front takes long, fails, or is being captured, for the stream.
+// Where the work in front takes longer than MC_TOTALS_WAIT, fails, or is being captured, for the stream.
 constexpr uint32_t MC_NO_TOTAL = 0xFFFFFFFFu;
+constexpr std::chrono::milliseconds MC_TOTALS_WAIT(1);
 static hipError_t mc_await_totals(hipStream_t s, const uint32_t* n_vertices, const uint32_t* n_triangles) {
 	hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
 	if (hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
-		for (int spins = 0; spins < 1 << 15; ++spins) {  // (some 1000 us)
-			if (__atomic_load_n(n_vertices, __ATOMIC_ACQUIRE) != MC_NO_TOTAL && __atomic_load_n(n_triangles, __ATOMIC_ACQUIRE) != MC_NO_TOTAL) return hipSuccess;
-			__builtin_ia32_pause();
-		}
+		auto there = [&]() { return __atomic_load_n(n_vertices, __ATOMIC_ACQUIRE) != MC_NO_TOTAL && __atomic_load_n(n_triangles, __ATOMIC_ACQUIRE) != MC_NO_TOTAL; };
+		if (n2_poll(there, MC_TOTALS_WAIT)) return hipSuccess;
 	}
 	return hipStreamSynchronize(s);
 }
