@@ -148,7 +148,6 @@ __device__ __forceinline__ uint32_t occ_row_slot(const OccOrder& o, uint32_t at)
 // all of it; 42 us when every workgroup works the factors out itself).
 // The launch also clears tmp (n_tmp floats, a multiple of 4), which the samples' densities are splatted into, and leaves the
 // positions as three rows of n_rows floats beside the [n][3] array (rows: null or these): the encoding's gather reads them.
-// past: nobody here reads the [n][3] array, and it is written past the caches (OCC_PAST_MIN).
 constexpr uint32_t OCC_DIGITS = 8;
 struct OccSkips {
 	uint64_t mult[OCC_DIGITS * 16], plus[OCC_DIGITS * 16];  // [digit's place][digit]; plus for an increment of one
@@ -190,14 +189,11 @@ __device__ __forceinline__ uint32_t occ_spread_cell(uint32_t q) {
 		if (OCC_BRICK_ALL[k] < OCC_SPREAD_BITS) cell |= ((q >> b++) & 1u) << OCC_BRICK_ALL[k];
 	return cell;
 }
-// Samples of an update from which on the positions that are only kept for the caller pass by the caches, as what the splatting reads does at any number.  (Updates in us, neither | both:
-// 2^21 395.9 | 394.5, 2^20 233.3 | 229.9, 2^19 142.2 | 140.0, 2^18 89.8 | 89.7, 2^19 and 2^19 others 255.0 | 249.0, 2^18 and 2^18 156.9 | 154.2; with the positions streamed 2^17 65.5 | 66.1.)
-constexpr uint32_t OCC_PAST_MIN = 1u << 18;
 template <uint32_t EACH>
 __global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uint32_t n_pad, Pcg32 first, uint32_t n_digits, uint32_t step, const float* __restrict__ grid,
                                                                  uint32_t n_cascades, float thresh, OccOrder order,
                                                                  float* __restrict__ positions, uint32_t* __restrict__ indices, float* __restrict__ rows, uint32_t n_rows,
-                                                                 float* __restrict__ tmp, uint32_t n_tmp, bool past) {
+                                                                 float* __restrict__ tmp, uint32_t n_tmp) {
 	constexpr bool SPREAD = EACH > 1;
 	static_assert(!SPREAD || EACH * OCC_BLOCK == OCC_SPREAD, "a workgroup takes the cells that it spreads");
 	__shared__ ulonglong2 skip[OCC_DIGITS][16];
@@ -241,8 +237,7 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_generate_kernel(uint32_t n, uin
 		const uint32_t at = rows && slot < n ? occ_row_place(order, slot) : slot;
 #pragma unroll
 		for (int d = 0; d < 3; ++d) {
-			if (past) __builtin_nontemporal_store(pos[d], positions + (size_t)slot * 3 + d);
-			else positions[(size_t)slot * 3 + d] = pos[d];
+			positions[(size_t)slot * 3 + d] = pos[d];
 			if (SPREAD) spread[d][local] = pos[d];
 			else if (rows) rows[(size_t)d * n_rows + at] = pos[d];
 		}
@@ -264,7 +259,7 @@ __global__ void __launch_bounds__(OCC_BLOCK) occ_splat_kernel(uint32_t n, const 
 	const uint32_t i = blockIdx.x * OCC_BLOCK + threadIdx.x;
 	if (i >= n) return;
 	const uint32_t slot = i < n_uniform ? occ_row_slot(uniform, i) : n_uniform + occ_row_slot(others, i - n_uniform);
-	atomicMax(reinterpret_cast<uint32_t*>(tmp) + __builtin_nontemporal_load(indices + slot), __float_as_uint(__builtin_nontemporal_load(density + i)));  // (their last use)
+	atomicMax(reinterpret_cast<uint32_t*>(tmp) + indices[slot], __float_as_uint(density[i]));
 }
 
 // ema_grid_samples_nerf (:698-727), fused with the partial sums of max(v, 0) over the first cascade (:3383).
@@ -560,7 +555,7 @@ N2_API int n2_occupancy_update(n2_occupancy_t* occ, n2_field_t* field, n2_stream
 		auto* const kernel = spread ? occ_generate_kernel<EACH> : occ_generate_kernel<1>;
 		kernel<<<ogrid(spread ? pad / EACH : pad), dim3(OCC_BLOCK), 0, s>>>(count, pad, rng, digits, occ->ema_step, occ->grid, occ->n_cascades, thresh, order,
 		                                                                        occ->positions + (size_t)first * 3, occ->indices + first, rows ? rows + first : nullptr, n8,
-		                                                                        occ->tmp, clear ? n_elements : 0u, rows != nullptr && n >= OCC_PAST_MIN);
+		                                                                        occ->tmp, clear ? n_elements : 0u);
 		N2_LAUNCH_CHECK();
 		return N2_OK;
 	};
