@@ -129,11 +129,12 @@ constexpr uint32_t FINE_SLOTS = FINE_CHUNKS * 4u + FINE_CHUNKS / 8u;
 __device__ __forceinline__ uint32_t fine_slot(uint32_t entry) { return entry + (entry >> 5); }
 
 // EACH entries per lane: of the rows at byte offsets row[q] (on a hashed level: entry x is at x's bytes ^ row[q]), weighed by
-// weight[q], the sum.  off: the lane's places in a row, of up to four entries each; have: whether there is one.
-template <uint32_t EACH>
+// weight[q], the sums, W of them at a time to put(h, sums).  off: the lane's places in a row, of W entries each; have: whether there is one.
+// (A part's sums are put down before the next part's are formed, which takes eight registers less; the loads are under way together.)
+template <uint32_t EACH, uint32_t W, class Put>
 __device__ __forceinline__ void fine_sum_rows(const char* __restrict__ base, const uint32_t (&off)[2], const bool (&have)[2], const uint32_t (&row)[4],
-                                              const float (&weight)[4], float2 (&sum)[EACH]) {
-	constexpr uint32_t W = EACH < 4u ? EACH : 4u, H = EACH / W;  // entries per load, loads per row
+                                              const float (&weight)[4], Put put) {
+	constexpr uint32_t H = EACH / W;  // loads per row
 	typedef uint32_t words __attribute__((ext_vector_type(W)));
 	words v[4][H];  // (a lane without a place holds anything: its slots are not read)
 #pragma unroll
@@ -143,34 +144,40 @@ __device__ __forceinline__ void fine_sum_rows(const char* __restrict__ base, con
 			for (uint32_t q = 0; q < 4; ++q) v[q][h] = *reinterpret_cast<const words*>(base + (off[h] ^ (row[q] & ~(4u * W - 1u))));
 		}
 #pragma unroll
-	for (uint32_t e = 0; e < EACH; ++e) sum[e] = make_float2(0.f, 0.f);
+	for (uint32_t h = 0; h < H; ++h) {
+		float2 sum[W];
 #pragma unroll
-	for (uint32_t q = 0; q < 4; ++q) {
-		// the entries of a load are permuted by the row's low bits, the same for the whole wave
-		auto add = [&](auto flip) __attribute__((always_inline)) {
-			constexpr uint32_t F = decltype(flip)::value;
+		for (uint32_t e = 0; e < W; ++e) sum[e] = make_float2(0.f, 0.f);
 #pragma unroll
-			for (uint32_t e = 0; e < EACH; ++e) {
-				const float2 f = lt_h2f(v[q][e / W][(e % W) ^ F]);
-				sum[e].x = fmaf(weight[q], f.x, sum[e].x);
-				sum[e].y = fmaf(weight[q], f.y, sum[e].y);
-				asm volatile("; permutation %2" : "+v"(sum[e].x), "+v"(sum[e].y) : "n"(F));  // (the cases stay apart: merged, each entry is picked by selects)
+		for (uint32_t q = 0; q < 4; ++q) {
+			// the entries of a load are permuted by the row's low bits, the same for the whole wave
+			auto add = [&](auto flip) __attribute__((always_inline)) {
+				constexpr uint32_t F = decltype(flip)::value;
+#pragma unroll
+				for (uint32_t e = 0; e < W; ++e) {
+					const float2 f = lt_h2f(v[q][h][e ^ F]);
+					sum[e].x = fmaf(weight[q], f.x, sum[e].x);
+					sum[e].y = fmaf(weight[q], f.y, sum[e].y);
+					asm volatile("; permutation %2" : "+v"(sum[e].x), "+v"(sum[e].y) : "n"(F));  // (the cases stay apart: merged, each entry is picked by selects)
+				}
+			};
+			if (W > 2u && (row[q] & 8u)) {
+				if (row[q] & 4u) add(std::integral_constant<uint32_t, 3 % W>());
+				else add(std::integral_constant<uint32_t, 2 % W>());
+			} else {
+				if (row[q] & 4u) add(std::integral_constant<uint32_t, 1>());
+				else add(std::integral_constant<uint32_t, 0>());
 			}
-		};
-		if (W > 2u && (row[q] & 8u)) {
-			if (row[q] & 4u) add(std::integral_constant<uint32_t, 3 % W>());
-			else add(std::integral_constant<uint32_t, 2 % W>());
-		} else {
-			if (row[q] & 4u) add(std::integral_constant<uint32_t, 1>());
-			else add(std::integral_constant<uint32_t, 0>());
+			// (here the row's load has arrived, whichever case was taken; without saying so the next plane's loads wait for the store)
+			asm volatile("" ::"v"(v[q][h]));
 		}
-		// (here every load of the row has arrived, whichever case was taken; without saying so the next plane's loads wait for the store)
-#pragma unroll
-		for (uint32_t h = 0; h < H; ++h) asm volatile("" ::"v"(v[q][h]));
+		put(h, sum);
 	}
 }
 
-__global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArgs a, uint32_t blocks_per_level) {
+// WAVES per SIMD at most (n2_lattice_fine_waves, launch_rules.h).
+template <uint32_t WAVES>
+__global__ void __launch_bounds__(LT_BLOCK) __attribute__((amdgpu_waves_per_eu(1, WAVES))) lattice_fine_kernel(const LatticeArgs a, uint32_t blocks_per_level) {
 	if (blockIdx.x >= blocks_per_level * (a.n_levels - a.first_fine)) {
 		lattice_write_frags(a, blockIdx.x - blocks_per_level * (a.n_levels - a.first_fine));
 		return;
@@ -227,10 +234,8 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 	if (hashed && chunks <= FINE_CHUNKS) {
 		float2* st = staged[threadIdx.x >> 6];
 		const uint32_t at0 = fine_slot(cx - c_lo), at1 = fine_slot(cx - c_lo + 1u);
-		// a plane's sums go through LDS, from the lanes' places in the row to the points
-		auto finish_row = [&](auto put) __attribute__((always_inline)) {
-			__builtin_amdgcn_wave_barrier();
-			put();
+		// a plane's sums stand in LDS: from the lanes' places in the row to the points
+		auto finish_row = [&]() __attribute__((always_inline)) {
 			__builtin_amdgcn_wave_barrier();
 			const float2 lo = st[at0], hi = st[at1];
 			if (inside) __builtin_nontemporal_store(lt_pack(fmaf(ux, lo.x, wx * hi.x), fmaf(ux, lo.y, wx * hi.y)), out);
@@ -274,10 +279,10 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 						sum[h].x = fmaf(weight[q], f.x, sum[h].x);
 						sum[h].y = fmaf(weight[q], f.y, sum[h].y);
 					}
-				finish_row([&]() __attribute__((always_inline)) {
+				__builtin_amdgcn_wave_barrier();
 #pragma unroll
-					for (uint32_t h = 0; h < LOADS; ++h) st[slot[h]] = sum[h];
-				});
+				for (uint32_t h = 0; h < LOADS; ++h) st[slot[h]] = sum[h];
+				finish_row();
 			}
 		};
 		auto walk_wide = [&](auto each) __attribute__((always_inline)) {
@@ -297,22 +302,22 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_fine_kernel(const LatticeArg
 				uint32_t row[4];
 				float weight[4];
 				plane_rows(k, row, weight);
-				float2 sum[EACH];
-				fine_sum_rows<EACH>(base, off, have, row, weight, sum);
-				finish_row([&]() __attribute__((always_inline)) {
+				fine_sum_rows<EACH, W>(base, off, have, row, weight, [&](uint32_t h, const float2 (&sum)[W]) __attribute__((always_inline)) {
+					if (h == 0u) __builtin_amdgcn_wave_barrier();
 #pragma unroll
-					for (uint32_t e = 0; e < EACH; ++e) st[slot[e / W] + e % W] = sum[e];
+					for (uint32_t e = 0; e < W; ++e) st[slot[h] + e] = sum[e];
 				});
+				finish_row();
 			}
 		};
-		if (chunks > 96u) walk_wide(std::integral_constant<uint32_t, 8>());
+		// (walk_wide<8> once: what two copies of it keep for their loops takes a wave per SIMD)
+		if (chunks > 96u || (chunks > 64u && a.walk <= 4u)) walk_wide(std::integral_constant<uint32_t, 8>());
 		else if (a.walk > 4u) {
 			if (chunks > 64u) walk_words(std::integral_constant<uint32_t, 6>());
 			else if (chunks > 48u) walk_words(std::integral_constant<uint32_t, 4>());
 			else if (chunks > 32u) walk_words(std::integral_constant<uint32_t, 3>());
 			else walk_words(std::integral_constant<uint32_t, 2>());
-		} else if (chunks > 64u) walk_wide(std::integral_constant<uint32_t, 8>());
-		else if (chunks > 32u) walk_wide(std::integral_constant<uint32_t, 4>());
+		} else if (chunks > 32u) walk_wide(std::integral_constant<uint32_t, 4>());
 		else walk_wide(std::integral_constant<uint32_t, 2>());
 		return;
 	}
@@ -853,7 +858,8 @@ int n2_fused_lattice_sdf(const N2FusedNets& nets, hipStream_t s, const N2Lattice
 		auto blocks = [&]() { return (runs * ((nz + a.walk - 1u) / a.walk) + LT_BLOCK / 64 - 1) / (LT_BLOCK / 64); };
 		if (n_fine) {
 			a.walk = n2_lattice_fine_walk(runs, nz);
-			lattice_fine_kernel<<<dim3(blocks() * n_fine + (done == 0 ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks());
+			auto* const fine_kernel = n2_lattice_fine_waves(runs, nz) == 5u ? lattice_fine_kernel<5> : lattice_fine_kernel<6>;
+			fine_kernel<<<dim3(blocks() * n_fine + (done == 0 ? FRAG_BLOCKS : 0u)), dim3(LT_BLOCK), 0, s>>>(a, blocks());
 			N2_LAUNCH_CHECK();
 		}
 		a.walk = n2_lattice_walk(runs, nz, by_rows ? 3u : lattice_gather_waves(nm));

@@ -117,6 +117,11 @@ static inline uint32_t n2_lattice_fine_walk(uint32_t runs, uint32_t nz) {
 	const uint64_t waves = (uint64_t)runs * nz / 4096u;
 	return n2_lattice_part(nz, waves >= 16u ? 12u : waves <= 4u ? 4u : (uint32_t)waves);
 }
+// The waves that a SIMD holds of its kernel, which has the registers for six (66; 87 and five for every lattice when it had two copies of the loop over the longest rows): five
+// where a launch is small, by measurement.  Lattices in us, five | six: 48^3 47.3 | 46.9, 32 x 64 x 64 45.6 | 47.5, 64^3 53.9 | 55.5, 64 x 64 x 80 58.3 | 60.4,
+// 96 x 64 x 64 57.1 | 58.6, 64 x 64 x 128 69.2 | 69.4, 80 x 96 x 64 68.9 | 69.0, 96^3 92.8 | 91.1; slabs of a chunk of 2^20 points 512 x 256 x 64 530 | 508, 512 x 512 x 64 929 | 902, 448 x 448 x 64 859 |
+// 822; 200^3 in a box of a tenth 306 | 293, 304 x 256 x 128 627 | 609, 256^3 904 | 915, 512^3 the same; of 2^22 128^3 152 | 155, 400 x 80 x 240 330 | 323.  (Seven: 512 x 256 x 64 3 % and 200^3 3 % faster, 256^3 and 512^3 1 % slower.)
+static inline uint32_t n2_lattice_fine_waves(uint32_t runs, uint32_t nz) { return (uint64_t)runs * nz <= 10240u ? 5u : 6u; }
 // The walk, `per_simd` of whose waves a SIMD holds: the 1024 SIMDs take the waves in rounds, of which each costs a wave's planes and a start as long
 // as two of them.  (By eye, up to 16 planes where there are many | by this count: 96^3 101 | 97, 128^3 174 | 171, 320^3 1547 | 1524, 512 x 64 x 512 623 | 600; with up to
 // 30 planes 96^3 to 320^3 lose up to 1.5 %.)

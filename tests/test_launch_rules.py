@@ -18,6 +18,7 @@ extern "C" uint64_t lattice_slab_points(uint64_t rest, uint64_t words, uint32_t 
 }
 extern "C" int lattice_large_slabs(uint64_t all, uint64_t words, uint32_t n_fine) { return n2_lattice_large_slabs(all, words, n_fine); }
 extern "C" uint32_t lattice_fine_walk(uint32_t runs, uint32_t nz) { return n2_lattice_fine_walk(runs, nz); }
+extern "C" uint32_t lattice_fine_waves(uint32_t runs, uint32_t nz) { return n2_lattice_fine_waves(runs, nz); }
 extern "C" uint32_t lattice_walk(uint32_t runs, uint32_t nz, uint32_t per_simd) { return n2_lattice_walk(runs, nz, per_simd); }
 extern "C" int gather_visits(uint32_t by_xcd_max, uint32_t n, uint32_t n_levels, uint32_t points_per_block, uint32_t* visits, uint32_t* grid) {
 	const N2GatherGrid g = n2_gather_grid(by_xcd_max, n, n_levels, points_per_block);
@@ -126,6 +127,12 @@ def test_planes_of_a_wave_are_equal_shares_of_the_slab(rules, runs, nz, per_simd
         assert 1 <= walk <= min(most, nz)
         parts = -(-nz // walk)
         assert walk == -(-nz // parts)  # no shorter waves for as many of them
+
+
+# 64^3, both sides of the line along either number, the smallest, more runs than 32 bits count
+@pytest.mark.parametrize("runs,nz,waves", [(64, 64, 5), (1, 1, 5), (160, 64, 5), (161, 64, 6), (1, 10240, 5), (1, 10241, 6), (4096, 29, 6), (1 << 22, 1 << 10, 6)])
+def test_waves_of_the_fine_levels(rules, runs, nz, waves):
+    assert rules.lattice_fine_waves(runs, nz) == waves
 
 
 # parameters of the field with tables of 2^14 to 2^22 entries a level (18 bytes of optimiser state each), batch, streamed
