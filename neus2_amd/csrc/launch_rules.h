@@ -39,6 +39,24 @@ static inline bool n2_optimiser_streams(uint64_t state_bytes, uint64_t batch, bo
 	return listed ? n2_moments_stream(state_bytes, 8u * batch) : n2_moments_stream(state_bytes + (96ull << 20), 2u * batch);
 }
 
+// The encoding's Jacobian (384 bytes per point of sixteen levels) is streamed from 64 MiB on.  Forward, scatter and input gradient in
+// us with nothing | the loads | the stores | both streamed: 2^18 uniform points (96 MiB) 219 | 203 | 204 | 195, along rays 169 | 165 | 163 | 157;
+// 2^19 434 | 430 | 430 | 423; 2^17 (48 MiB) 108 in all four, along rays 92.  The SDF network with the eikonal term, 2^18: uniform 283 | 285 | 288 | 287,
+// along rays 244 | 236 | 241 | 235; 2^17 155 | 154 | 155 | 153.
+static inline bool n2_jacobian_streams(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (64ull << 20); }
+// Whether n elements to a row leave every row at the start of a line of 128 bytes (of an array that starts there).
+static inline bool n2_rows_of_whole_lines(uint32_t n, uint32_t bytes) { return (uint64_t)n * bytes % 128u == 0u; }
+// In the SDF network's step it is read once, by the launch right behind the one that writes it (n2_fused_sdf_eikonal): the stores stay in the last-level cache up to where
+// that is full, and the loads, which nothing follows, are streamed much earlier.  Step in us, by the rule above | this one: 32 768 uniform 68.3 | 66.3, 65 536 along rays 83.2 | 81.8, 2^17
+// 124.7 | 124.1 (uniform 144.4 | 145.0), 180 000 159.0 | 154.4, 2^18 209.6 | 204.6 (uniform 257.2 | 253.2), 393 216 uniform 377.4 | 364.5; with the stores cached beyond 2^19 along rays
+// 380.6 | 385.0 (uniform 489.9 | 479.2), 2^20 752.9 | 771.8; with the loads streamed 8192 37.6 | 37.9.
+static inline bool n2_step_jacobian_stores_stream(uint32_t n_points, uint32_t rows) { return 12ull * n_points * rows >= (160ull << 20); }
+// Rows that do not start lines are streamed from 64 MiB on as above: where two waves share a line, the first one's streamed load costs the second one the line.  Along rays, streamed earlier all
+// the same | not: 72 008 97.2 | 96.3, 100 008 115.2 | 112.4, 150 008 149.9 | 147.3; streamed | not at all: 262 136 217.0 | 219.9.
+static inline bool n2_step_jacobian_loads_stream(uint32_t n_points, uint32_t rows) {
+	return n2_rows_of_whole_lines(n_points, 12u) ? 12ull * n_points * rows >= (12ull << 20) : n2_jacobian_streams(n_points, rows);
+}
+
 // Points per thread of the scatter's sorting kernel.  Three of its workgroups share a CU, 768 run at a time.  One point per thread where all workgroups
 // (levels x tiles) then start together: the launch takes one workgroup's chain of round trips, which is shorter for one point.  Beyond, a
 // workgroup of two points per thread takes less than two of one, and the summing kernel finds half as many runs.  Both kernels in us, one | two:

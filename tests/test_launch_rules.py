@@ -59,6 +59,12 @@ extern "C" uint32_t run_tile(uint32_t group, uint32_t groups, uint32_t run, uint
 extern "C" uint64_t run_base(uint32_t first_tile, uint32_t tile_records) { return n2_run_base(first_tile, tile_records); }
 extern "C" uint32_t run_place(uint32_t first_tile, uint32_t tile, uint32_t tile_records) { return n2_run_place(first_tile, tile, tile_records); }
 extern "C" int sdf_one_pass(uint32_t n) { return n2_sdf_one_pass(n); }
+extern "C" int adam_lists(uint64_t n_params, uint32_t n_levels, uint64_t batch) { return n2_adam_lists(n_params, n_levels, batch); }
+extern "C" int optimiser_streams(uint64_t state_bytes, uint64_t batch, int listed) { return n2_optimiser_streams(state_bytes, batch, listed); }
+extern "C" int jacobian_streams(uint32_t n, uint32_t rows) { return n2_jacobian_streams(n, rows); }
+extern "C" int whole_lines(uint32_t n, uint32_t bytes) { return n2_rows_of_whole_lines(n, bytes); }
+extern "C" int step_stores_stream(uint32_t n, uint32_t rows) { return n2_step_jacobian_stores_stream(n, rows); }
+extern "C" int step_loads_stream(uint32_t n, uint32_t rows) { return n2_step_jacobian_loads_stream(n, rows); }
 extern "C" int moments_stream(uint64_t state_bytes, uint64_t batch) { return n2_moments_stream(state_bytes, batch); }
 """
 
@@ -135,12 +141,36 @@ def test_waves_of_the_fine_levels(rules, runs, nz, waves):
     assert rules.lattice_fine_waves(runs, nz) == waves
 
 
-# parameters of the field with tables of 2^14 to 2^22 entries a level (18 bytes of optimiser state each), batch, streamed
+# What the two rules below are made of.  Parameters of the field with tables of 2^14 to 2^22 entries a level (18 bytes of optimiser state each), batch, streamed
 @pytest.mark.parametrize("n_params,batch,streams", [
     (506884, 1 << 14, 0), (506884, 1 << 16, 0), (506884, 1 << 18, 1), (3507780, 1 << 16, 0), (3507780, 1 << 18, 1), (12612212, 1 << 12, 0),
     (12612212, 20480, 0), (12612212, 28672, 1), (12612212, 1 << 18, 1), (24146548, 1 << 12, 1), (85050820, 1 << 12, 1), (1 << 31, 1 << 31, 1)])
 def test_moments_are_streamed_where_state_and_samples_exceed_the_cache(rules, n_params, batch, streams):
     assert rules.moments_stream(C.c_uint64(18 * n_params), C.c_uint64(batch)) == streams
+
+
+# The optimiser of a training step: the field with tables of 2^14 to 2^22 entries a level, 18 bytes of state per parameter (24 with the average).  Both sides of each line: a sixth of the
+# parameters met (8192 | 8320 samples at the default table, fewer levels meet fewer), the smallest table and the largest batch that are listed, and where lists and whole pieces are streamed
+@pytest.mark.parametrize("n_params,n_levels,state,batch,listed,streams", [
+    (12612212, 16, 18, 128, 1, 0), (12612212, 16, 18, 3072, 1, 0), (12612212, 16, 18, 3328, 1, 1), (12612212, 16, 18, 8192, 1, 1), (12612212, 16, 18, 8320, 0, 1), (12612212, 16, 18, 20480, 0, 1),
+    (12612212, 16, 18, 1 << 18, 0, 1), (12612212, 16, 24, 512, 1, 1), (12612212, 8, 18, 16384, 1, 1), (12612212, 8, 18, 16512, 0, 1), (506884, 16, 18, 128, 0, 0), (506884, 16, 18, 48896, 0, 0),
+    (506884, 16, 18, 50048, 0, 1), ((1 << 21) - 4, 16, 18, 1024, 0, 0), (1 << 21, 16, 18, 1280, 1, 0), (1 << 21, 16, 18, 1408, 0, 0), (3507780, 16, 18, 2176, 1, 0), (3507780, 16, 18, 2304, 0, 0),
+    (24146548, 16, 18, 15616, 1, 1), (24146548, 16, 18, 16384, 0, 1), (85050820, 16, 18, 40960, 1, 1), (85050820, 16, 18, 41088, 0, 1), (1 << 32, 16, 18, 41088, 0, 1), (1 << 32, 16, 18, 128, 1, 1)])
+def test_which_optimiser_a_batch_takes(rules, n_params, n_levels, state, batch, listed, streams):
+    assert rules.adam_lists(C.c_uint64(n_params), n_levels, C.c_uint64(batch)) == listed
+    assert rules.optimiser_streams(C.c_uint64(state * n_params), C.c_uint64(batch), listed) == streams
+
+
+# 32 rows of 12 bytes a point: 12 MiB, 64 MiB and 160 MiB from both sides, rows that start lines (a multiple of 32 points) and that do not, the most points
+@pytest.mark.parametrize("n,stores,loads,alone", [(8, 0, 0, 0), (32736, 0, 0, 0), (32768, 0, 1, 0), (32776, 0, 0, 0), (174752, 0, 1, 0), (174760, 0, 0, 0), (174768, 0, 1, 1),
+                                                  (174784, 0, 1, 1), (174792, 0, 1, 1), (436896, 0, 1, 1), (436928, 1, 1, 1), (436936, 1, 1, 1), (0xFFFFFFF8, 1, 1, 1)])
+def test_where_the_jacobian_is_streamed(rules, n, stores, loads, alone):
+    assert (rules.step_stores_stream(C.c_uint32(n), 32), rules.step_loads_stream(C.c_uint32(n), 32), rules.jacobian_streams(C.c_uint32(n), 32)) == (stores, loads, alone)
+
+
+@pytest.mark.parametrize("n,bytes,whole", [(0, 2, 1), (64, 2, 1), (63, 2, 0), (32, 2, 0), (32, 4, 1), (31, 4, 0), (32, 12, 1), (8, 12, 0), (1 << 31, 12, 1), ((1 << 32) - 32, 12, 1), ((1 << 32) - 8, 12, 0)])
+def test_rows_that_start_lines(rules, n, bytes, whole):
+    assert rules.whole_lines(C.c_uint32(n), bytes) == whole
 
 
 # one level, fewer levels than XCDs, a last round that is not full, the most levels; one tile, tiles that the XCDs cannot share
