@@ -69,9 +69,11 @@ def test_small_batches_of_the_trainer_match_oracle(oracle, batch, beta2, ema):
     tr.set_scene(pack_cameras(cams), len(cams), dev(scene.render_sphere_images(cams)), dev(scene.sphere_bitfield()))
     tr.initialize_params(seed=5, sdf_mlp_weights=None)
     w, m1, m2, steps = host(tr.master).copy(), np.zeros(tr.n_params, np.float32), np.zeros(tr.n_params, np.float32), np.zeros(tr.n_params, np.uint32)
+    size1 = np.zeros(tr.n_params)  # what the first moment would be if all its terms had one sign
     for seed in (3, 4):
         tr.step(n_rays=max(16, batch // 40), n_inference=1 << 17, seed=seed)
         g = host(tr.grads)
+        size1 = np.where((g != 0) | (np.arange(tr.n_params) < tr.offsets[2]), 0.9 * size1 + 0.1 * (np.abs(g / 128.0) + 1e-6 * np.abs(w)), size1)
         oracle.adam_step(w, g, m1, m2, steps, n_matrix_params=tr.offsets[2], beta2=beta2)
     s = tr.optimizer_state()
     assert s.param_steps_bits == (16 if beta2 == 0.99 else 32)
@@ -79,8 +81,10 @@ def test_small_batches_of_the_trainer_match_oracle(oracle, batch, beta2, ema):
     met = 2 * batch * 16 * 8 * 2 + tr.offsets[2] + tr.n_params - tr.offsets[3]  # two steps, eight entries of two parameters on 16 levels; the networks and the variance
     assert tr.offsets[2] < (steps > 0).sum() <= met and np.array_equal(got, steps.astype(got.dtype))
     np.testing.assert_allclose(host(tr.master), w, rtol=1e-5, atol=1e-6)
-    np.testing.assert_allclose(host(tr._view(s.first_moments, tr.n_params, torch.float32)), m1, rtol=1e-5, atol=1e-7)
-    np.testing.assert_allclose(host(tr._view(s.second_moments, tr.n_params, torch.float32)), m2, rtol=1e-5, atol=1e-9)
+    # Moments of a table's entries are 1e-11 and less, so each is measured by its own size: a few roundings of 2^-24, and what weights that agree to 1e-5 (above) add
+    # through the networks' decay.  A moment that the last step did not store is off by about half of it, or by all.
+    assert (np.abs(host(tr._view(s.first_moments, tr.n_params, torch.float32)).astype(np.float64) - m1) <= 1e-5 * size1).all()
+    np.testing.assert_allclose(host(tr._view(s.second_moments, tr.n_params, torch.float32)), m2, rtol=3e-5, atol=0)
     np.testing.assert_array_equal(host(tr.params), q16(host(tr.master)))
 
 

@@ -289,7 +289,7 @@ def test_lattices_walked_by_rows_equal_the_same_points_queried(side, res, part, 
 
 
 # The finest level's row that a run of 64 points meets, in chunks of four entries: each number of words a lane takes, and both sides of where it becomes one
-# more, wide loads begin and the points gather for themselves; by waves of two planes, whose loads are wide always, and of five.
+# more, wide loads begin and the points gather for themselves; by waves of three planes, whose loads are wide always, and of five.
 @pytest.mark.parametrize("rows", [(6, 9), (160, 130)])
 @pytest.mark.parametrize("chunks", [2, 16, 32, 33, 48, 49, 64, 65, 96, 97, 128, 129])
 def test_fine_rows_of_every_length(chunks, rows):
