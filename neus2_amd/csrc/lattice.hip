@@ -13,15 +13,16 @@
 //    missed, 1.4 GB per 2^22 points through the fabric.)
 // The walk hands its 64 points to the SDF network as two MFMA tiles: v_permlane32_swap_b32 turns "lane = point, register =
 // level" into the operand layout "lane = (point, level group)" without touching LDS.
-// 512^3 lattice 4.00 ms in ten slabs: 2.43 ms for six fine levels and 1.81 ms for the walk under the profiler.  The fine levels are held by lines (one of 128 bytes into an L1 in every
-// 3.0 clocks; 2.3 at best) beside vector issue (79 %), the walk by vector instructions, waits of three waves per SIMD and
-// the features, which come from beyond the L2 (28 % hits).  (4.30 ms with 2.57 and 2.06, before what stands at the two kernels; 4.80 in 18 slabs, when a walk's start waited for its planes one after
-// the other and then for the fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch for a slab's
-// walk and the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
-// Features and SDF are written, and features read, as streams that pass by the caches: each is met once, and the tables stay where they are (us: 512^3 3905 -> 3840, the walk's alone 3815;
-// 464^3 3628 -> 3546, 400^3 2367 -> 2315, 192^3 399 -> 392, 128^3 160.9 -> 159.6; 448 x 512 x 96 1026 -> 1024, with the walk's alone 1035).
-// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before the features were streams, before | now, us: 64^3 59.7 | 57.7, 80^3 73 | 72, 96^3 96 | 96, 128^3 171 | 166, 208^3 611 | 571, 256^3 935 | 890,
-// 320^3 1600 | 1480, 400^3 2720 | 2500, 464^3 4047 | 3656, 512 x 64 x 512 690 | 630, 64 x 512 x 512 1575 | 1423; with a chunk of 2^20 points 256^3 1045 | 981, 512^3 4550 | 4263.
+// 512^3 lattice in ten slabs: 3.86 to 3.98 ms on four cards; under the profiler 2.30 ms for six fine levels and 1.75 ms for the walk.  The fine levels are held by lines (one of 128 bytes into an L1
+// in every 2.8 clocks; 2.3 at best) beside vector issue (83 %), the walk by vector instructions (69 %), waits of three waves per SIMD and
+// the features, which come from beyond the L2 (37 % hits).  (On the same cards 4.25 to 4.32 ms with 2.46 and 1.98, before what stands at the two kernels; 4.80 in 18 slabs, when a walk's start waited
+// for its planes one after the other and then for the fine features; 5.76 before that, with vertices picked out of LDS row by row, and four gathers per point and plane by two waves per SIMD.  One launch
+// for a slab's walk and the next one's fine levels, in any mixture, or the two on two streams: 5.3 ms and more, the two hold each other up.)
+// Features and SDF are written, and features read, as streams that pass by the caches: each is met once, and the tables stay where they are (by that alone 512^3 takes 1.7 % less, with the walk's
+// alone 2.3; 464^3 2.3 %, 400^3 2.2, 192^3 1.8, 128^3 0.8; 448 x 512 x 96 0.2 %, with the walk's alone 0.9 more).
+// Rows that are no multiple of 64 leave lanes idle in their last run.  Other lattices, before what stands at the two kernels | now, us: 64^3 59.2 | 54.3, 80^3 72.8 | 69.5, 96^3 96.0 | 91.3, 128^3 168.6 | 156.4,
+// 208^3 563 | 509, 256^3 843 | 775, 320^3 1484 | 1348, 400^3 2634 | 2383, 464^3 4049 | 3605, 512 x 64 x 512 583 | 535, 64 x 512 x 512 1555 | 1425; with a chunk of 2^20 points 128^3 189 | 176, 256^3 971 | 918,
+// 400^3 2839 | 2561, 512^3 4557 | 4203.
 #include "n2_common.h"
 
 #include "grid_device.h"
@@ -114,15 +115,15 @@ __global__ void __launch_bounds__(LT_BLOCK) lattice_frags_kernel(const LatticeAr
 // group of four lanes at least, and up to four where the lanes' spacing makes their banks collide (spacing 8, the finest level of a 512^3 lattice: 65 clocks).  So the wave
 // loads the rows as a whole and weighs the four rows against each other where they are, in
 // registers; what remains is one row, which goes through LDS (in fp32, a slot left out after every 32 entries so that lanes any
-// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 32 % of the
+// number of entries apart meet different banks), and every point picks its two neighbours (LDS active in 34 % of the
 // clocks; 73 % when the eight vertices were picked there).  Runs longer than that (coarse lattices) and dense levels gather from memory.
 //  * Rows of up to 384 entries come a word per lane (walk_words).  64 words of which sixteen lanes each meet aligned 64 bytes, in any order, take an L1 4.4 clocks; a load of 8
 //    or 16 bytes per lane takes it 16.5 however few lanes take part, and a row seldom fills the last of those.
 //  * Longer ones, 16 bytes per lane (walk_wide): eight words a lane and row would be as many clocks and four times the instructions.
 //  * The waves of a small lattice, of four planes at most, take 8 or 16 bytes per lane always: there the number of a plane's loads counts and not what an L1 makes of them (64^3
 //    60 us with wide loads, 65 with words).
-// The kernel's launches for 512^3, wide loads alone | this: 2.57 | 2.44 ms; lattices 256^3 935 | 910 us, 320^3 1605 | 1534, 400^3 2706 | 2624, 464^3 4047 | 3850, 512 x 64 x 512 680 | 655.
-// It takes a line of 128 bytes in every 3.0 clocks (3.2 before; 2.3 at best, 216 lines for 64 points on six levels), beside vector issue (79 % of the clocks).  Each point taking the
+// The kernel's launches for 512^3, wide loads alone | this, five waves per SIMD: 2.57 | 2.44 ms; lattices 256^3 935 | 910 us, 320^3 1605 | 1534, 400^3 2706 | 2624, 464^3 4047 | 3850, 512 x 64 x 512 680 | 655.
+// It takes a line of 128 bytes in every 2.8 clocks (3.1 with wide loads alone; 2.3 at best, 216 lines for 64 points on six levels), beside vector issue (83 % of the clocks).  Each point taking the
 // aligned 8 bytes round its corners by itself, without LDS, is slower where rows are of 64 entries and more (finest levels of 512^3 527 -> 575 and 690 -> 750 us).
 constexpr uint32_t FINE_CHUNKS = 128;  // chunks of four entries a row may have
 constexpr uint32_t FINE_SLOTS = FINE_CHUNKS * 4u + FINE_CHUNKS / 8u;
@@ -422,7 +423,7 @@ __device__ __forceinline__ hf lattice_network(const hf* F, uint32_t lane, uint32
 // The walk.  NM levels are interpolated here, the others come from a.features.  A row of a walked level's vertices that a run of 64
 // points meets fits the wave's lanes (n2_lattice_row_levels): lane v holds vertex v of the run, the two rows of a plane are loaded
 // as consecutive words and interpolated in y there, and the points pick their two neighbours through LDS.
-// Three waves per SIMD (157 registers), whose vector instructions and waits fill the time.  What took instructions away, the walk of 512^3 in ms: masks kept as they are (below) and rows'
+// Three waves per SIMD (157 registers for ten levels, 22 scalars spilled to vector lanes), whose vector instructions and waits fill the time.  What took instructions away, the walk of 512^3 in ms: masks kept as they are (below) and rows'
 // offsets by one product instead of five 2.06 -> 1.92, the coordinates in registers of their own 1.91, features loaded one step ahead instead of two, without twelve moves a
 // step, 1.87, the second layer by small matrix products 1.81.
 template <int NM>
@@ -663,7 +664,7 @@ __global__ void __launch_bounds__(LT_BLOCK, lattice_gather_waves(NM)) lattice_ga
 	for (int l = 0; l < NM; ++l) wy[l] = lane_f32(my_wy, l);
 	// the plane of vertices at `row0`, `row1` (byte offsets of its rows y, y + 1): four gathers, and their interpolation in x and y
 	// What depends on x is worked out at each plane, from an opaque copy of the position: kept across the loop, cell and weight of
-	// every level take 40 registers more than the 225 that two waves per SIMD leave room for.
+	// every level would come on top of the 168 registers of six levels, which are all that three waves per SIMD have, the 183 of eight and the 197 of ten.
 	auto place = [&](int l, float& w, uint32_t& c) {
 		float p = px;
 		asm volatile("" : "+v"(p));

@@ -276,8 +276,10 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES) mlp_wgrad_kernel(const 
 		stage_order();
 		uint4 sl[Tail::active ? 8 : 1];
 		if constexpr (Tail::active) {
-			// the slopes of this lane's 8 levels (level 4 (j / 2) + 2 g + j % 2): their last use, past the caches (training step of 2^18 samples 338.7 -> 335.8 us, 2^16 184.6 -> 183.3,
-			// trained 492.2 -> 491.8; the field's forward and backward 2^18 242.8 -> 240.6, 52 344 88.5 -> 87.7)
+			// the slopes of this lane's 8 levels (level 4 (j / 2) + 2 g + j % 2): their last use, past the caches.  At any size: a row of a batch, which is a multiple of 8 samples of 16
+			// bytes, starts a line, and so does a tile's part of it; where a selection picks the columns two tiles may meet a line, which shows in no time.  In us, cached | streamed: the field's
+			// forward and backward 2^18 245.4 | 239.2, 262 136 245.3 | 243.6, 150 008 165.2 | 164.8, 100 008 125.3 | 125.4, 52 344 88.9 | 87.7; training step 2^18 339.3 | 336.5, 100 096 216.0 | 216.4;
+			// with columns picked (trained) 2^18 494.2 | 491.8, 100 096 289.3 | 289.5, 59 904 225.3 | 224.5, 29 952 170.6 | 170.1.
 			const uint4* const at = reinterpret_cast<const uint4*>(tail.a.slopes) + (size_t)(4u * g < tail.a.enc_w ? 2u * g : 0u) * tail.a.n_src + col_src;
 #pragma unroll
 			for (int j = 0; j < 8; ++j) {
